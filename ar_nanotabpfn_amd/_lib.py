@@ -78,6 +78,23 @@ class ArtabSampleEmbedArgs(ctypes.Structure):
     ]
 
 
+class ArtabTrajectoryArgs(ctypes.Structure):
+    """``artab_trajectory_args`` of include/artab_attention.h, field for field."""
+
+    _fields_ = [
+        ("tape", _p), ("vecs", _p), ("kv", _p), ("n_layers", _i),
+        ("n_ctx", _i), ("ctx_rows", _i), ("own_base", _i), ("own_rows", _i), ("park_target", _i),
+        ("eps1", _f), ("eps2", _f), ("eps3", _f),
+        ("norm_gamma", _p), ("norm_beta", _p), ("eps", _f),
+        ("b_h1", _p), ("b_h2", _p), ("mix", _p), ("K", _i), ("std_min", _f), ("std_max", _f),
+        ("rand_u", _p), ("rand_n", _p), ("rand_n_f32", _i), ("x_mean", _p),
+        ("w_x", _p), ("b_x", _p), ("w_y", _p), ("b_y", _p), ("markers", _p), ("ar_tokens", _p), ("bs", _i),
+        ("preds", _p), ("B", _i), ("Nt", _i), ("group", _i), ("D", _i), ("F", _i),
+    ]
+
+
+TAPE_FO, TAPE_QKV, TAPE_O, TAPE_1, TAPE_2, TAPE_H1, TAPE_H2, TAPE_CLOSE = range(8)
+
 # name -> (restype, argtypes); every symbol declared in include/artab_attention.h
 SIGNATURES = {
     "artab_version": (_i, []),
@@ -139,6 +156,10 @@ SIGNATURES = {
         [ctypes.POINTER(ArtabAttentionPartials), _p, _i64, _p, _i64, _p, _p, _p, _f, _p, _p, _p, _p, _p, _p, _f,
          ctypes.POINTER(ArtabSampleEmbedArgs), _p, _p, _p, _f, _p, _p, _p, _i, _i, _p],
     ),
+    "artab_trajectory_group": (_i, [_i, _i, _i, _i, _i, _i, _i, _i]),
+    "artab_trajectory_tape_bytes": (_sz, [_i, _i, _i, _i]),
+    "artab_trajectory_pack": (_i, [_p, _p, _i, _i, _i, _i, _i, _i, _i, _p]),
+    "artab_trajectory_decode": (_i, [ctypes.POINTER(ArtabTrajectoryArgs), _i, _p]),
     "artab_layer_post": (_i, [_p, _i64, _p, _i64, _p, _p, _p, _f, _p, _p, _p, _p, _p, _p, _f, _p, _i64, _i, _i, _i, _p]),
 }
 
@@ -153,7 +174,7 @@ BENCH_SIGNATURES = {
 
 TUNING_KEYS = ("ARTAB_BM", "ARTAB_SPLIT", "ARTAB_SMALL", "ARTAB_STREAM", "ARTAB_STREAM_PER_CU", "ARTAB_STREAM_PRIO",
                "ARTAB_STREAM_SHORT", "ARTAB_STREAM_CALM", "ARTAB_DENSE_BELOW", "ARTAB_CTX_YIELD", "ARTAB_ORDER_GATE_LAUNCH", "ARTAB_BN", "ARTAB_LEAN",
-               "ARTAB_LEAN_OCC", "ARTAB_NW", "ARTAB_TILE_ROWS", "ARTAB_LAYER_FETCHERS")
+               "ARTAB_LEAN_OCC", "ARTAB_NW", "ARTAB_TILE_ROWS", "ARTAB_LAYER_FETCHERS", "ARTAB_TRAJECTORY")
 
 _lib: Optional[ctypes.CDLL] = None
 _product_lib: Optional[ctypes.CDLL] = None

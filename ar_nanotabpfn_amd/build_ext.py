@@ -57,6 +57,10 @@ for _bf16 in (1, 0):
                       f"layer_launch_{'bf16' if _bf16 else 'f16'}_{_group}.o"))
 
 
+for _type, _name in enumerate(("bf16", "f16", "f32")):
+    UNITS.append(("trajectory_launch.hip", [f"-DARTAB_TRAJ_TYPE={_type}"], f"trajectory_launch_{_name}.o"))
+
+
 def find_hipcc() -> str:
     for cand in (shutil.which("hipcc"), "/opt/rocm/bin/hipcc"):
         if cand and os.path.exists(cand):

@@ -40,6 +40,7 @@ static TuneSlot g_tune[kTuneCount] = {
     {"ARTAB_CTX_YIELD", false, 0},    {"ARTAB_ORDER_GATE_LAUNCH", false, 0},
     {"ARTAB_BN", false, 0},          {"ARTAB_LEAN", false, 0},         {"ARTAB_LEAN_OCC", false, 0},
     {"ARTAB_NW", false, 0},          {"ARTAB_TILE_ROWS", false, 0},    {"ARTAB_LAYER_FETCHERS", false, 0},
+    {"ARTAB_TRAJECTORY", false, 0},
 };
 static const bool g_tune_loaded = [] {
     for (TuneSlot &t : g_tune) {
@@ -1472,6 +1473,117 @@ int artab_decode_step_boundary(const artab_attention_partials *parts, const void
     if (B == 0) return ARTAB_OK;
     hipError_t e = launch_step_boundary(P, S, N, D, F, dtype == ARTAB_BF16, st);
     return launch_status(e, "decode_step_boundary");
+}
+
+static TrajectoryTapeLayout trajectory_layout(int D, int F, int n_layers, int dtype) {
+    if (dtype == ARTAB_BF16) return trajectory_tape_layout_bf16(D, F, n_layers);
+    if (dtype == ARTAB_F16) return trajectory_tape_layout_f16(D, F, n_layers);
+    if (dtype == ARTAB_F32) return trajectory_tape_layout_f32(D, F, n_layers);
+    return TrajectoryTapeLayout{};
+}
+
+// The rule for the whole-run kernel.  Per layer and step one of its workgroups streams the layer's
+// weights, the context and its trajectories' rows through one compute unit (64 B per clock), and
+// pays about 3 us for nine barriers; the launches of the other route take 27 us (45 us at d_model 512,
+// whose layer kernel streams 3 MB of weights per workgroup as well) unless their context pass, which
+// has the matrix cores of the whole chip, takes longer.  A trajectory with a context of its own has
+// no recorded alternative: it always comes here.
+int artab_trajectory_group(int B, int Nc, int Nt, int H, int D, int F, int own_context, int dtype) {
+    if (B < 1 || Nt < 1 || Nc < 1 || H * 32 != D || trajectory_layout(D, F, 1, dtype).stride == 0) return 0;
+    static const int cus = [] {
+        int dev = 0, n = 0;
+        if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
+            n = 256;
+        return n;
+    }();
+    const int group = B <= cus ? 1 : (B + cus - 1) / cus < kTrajMax ? (B + cus - 1) / cus : kTrajMax;
+    const int force = tune(kTuneTrajectory, -1);
+    if (force >= 0) return force == 0 ? 0 : force < kTrajMax ? force : kTrajMax;
+    if (own_context) return group;
+    const double esz = elem_size(dtype), rounds = std::ceil(std::ceil(static_cast<double>(B) / group) / cus);
+    const double bytes = esz * (5.0 * D * D + 2.0 * D * F) + 2 * esz * D * (Nc + 0.5 * Nt * group);
+    const double here = rounds * (3.0 + bytes / 150e3);
+    const double flops = 8.0 * B * Nc * D;
+    const double there = (D == 512 ? 45.0 : 27.0) + (dtype == ARTAB_F32 ? 30.0 + flops / 5e6 : flops / 1200e6);
+    return here < there ? group : 0;
+}
+
+size_t artab_trajectory_tape_bytes(int D, int F, int n_layers, int dtype) {
+    return n_layers < 1 ? 0 : static_cast<size_t>(kTrajWaves) * trajectory_layout(D, F, n_layers, dtype).stride;
+}
+
+int artab_trajectory_pack(void *tape, const void *w, int which, int layer, int rows, int D, int F, int n_layers,
+                          int dtype, void *stream) {
+    const TrajectoryTapeLayout t = trajectory_layout(D, F, n_layers, dtype);
+    if (t.stride == 0 || n_layers < 1)
+        return fail(ARTAB_ERR_UNSUPPORTED, "no whole-run decode kernel for D=%d F=%d layers=%d dtype code %d", D, F, n_layers, dtype);
+    if (!tape || (!w && which != ARTAB_TAPE_CLOSE)) return fail(ARTAB_ERR_NULL_POINTER, "trajectory_pack: tape or w is NULL");
+    if (misaligned16(tape) || misaligned16(w)) return fail(ARTAB_ERR_BAD_STRIDE, "tape and w must be 16-byte aligned");
+    if (layer < 0 || layer >= n_layers) return fail(ARTAB_ERR_BAD_SHAPE, "layer %d outside [0, %d)", layer, n_layers);
+    if (which == ARTAB_TAPE_H2 && (rows < 1 || rows > kTrajHeadOut))
+        return fail(ARTAB_ERR_BAD_SHAPE, "the head has %d outputs, at most %d are supported", rows, kTrajHeadOut);
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    char *to = static_cast<char *>(tape);
+    auto put = [&](const void *src, int N, int K, const TrajectoryTapeLayout::Matrix &m, int section) {
+        hipError_t e = dtype == ARTAB_BF16 ? launch_trajectory_tape_bf16(src, to, t.stride, N, K, m, section, st)
+                       : dtype == ARTAB_F16 ? launch_trajectory_tape_f16(src, to, t.stride, N, K, m, section, st)
+                                            : launch_trajectory_tape_f32(src, to, t.stride, N, K, m, section, st);
+        return launch_status(e, "trajectory_pack");
+    };
+    const int at = layer * t.layer, head = n_layers * t.layer;
+    switch (which) {
+        case ARTAB_TAPE_FO: return put(w, D, D, t.fo, at);
+        case ARTAB_TAPE_QKV:
+            for (int p = 0; p < 3; ++p)
+                ARTAB_TRY(put(static_cast<const char *>(w) + static_cast<size_t>(p) * D * D * elem_size(dtype), D, D, t.qkv[p], at));
+            return ARTAB_OK;
+        case ARTAB_TAPE_O: return put(w, D, D, t.o, at);
+        case ARTAB_TAPE_1: return put(w, F, D, t.w1, at);
+        case ARTAB_TAPE_2: return put(w, D, F, t.w2, at);
+        case ARTAB_TAPE_H1: return put(w, F, D, t.h1, head);
+        case ARTAB_TAPE_H2: return put(w, rows, F, t.h2, head);
+        case ARTAB_TAPE_CLOSE:
+            return launch_status(launch_trajectory_tape_wrap(to, t.stride, static_cast<long>(t.ring) * 1024, st), "trajectory_pack");
+        default: return fail(ARTAB_ERR_UNSUPPORTED, "trajectory_pack: unknown matrix %d", which);
+    }
+}
+
+int artab_trajectory_decode(const artab_trajectory_args *a, int dtype, void *stream) {
+    if (!a) return fail(ARTAB_ERR_NULL_POINTER, "args is NULL");
+    const TrajectoryTapeLayout t = trajectory_layout(a->D, a->F, a->n_layers, dtype);
+    if (t.stride == 0 || a->n_layers < 1)
+        return fail(ARTAB_ERR_UNSUPPORTED, "no whole-run decode kernel for D=%d F=%d layers=%d dtype code %d", a->D, a->F, a->n_layers, dtype);
+    if (a->B < 0 || a->Nt < 1 || a->K < 1 || a->K > kTrajMaxMix || a->bs < 1 || a->group < 1 || a->group > kTrajMax)
+        return fail(ARTAB_ERR_BAD_SHAPE, "trajectory_decode: bad sizes B=%d Nt=%d K=%d bs=%d group=%d", a->B, a->Nt, a->K, a->bs, a->group);
+    if (a->n_ctx < 0 || a->own_base < 0 || (a->n_ctx == 0) == (a->own_base == 0) || a->n_ctx > a->ctx_rows)
+        return fail(ARTAB_ERR_BAD_SHAPE, "trajectory_decode: one of a shared context (%d of %d rows) and own contexts (%d rows)", a->n_ctx,
+                    a->ctx_rows, a->own_base);
+    // committed rows: the values of steps 0 .. Nt - 2; behind them the target row if it is kept
+    if (a->own_base + a->Nt - 1 + (a->park_target ? 1 : 0) > a->own_rows)
+        return fail(ARTAB_ERR_CAPACITY, "trajectory_decode: %d rows do not fit a cache of %d", a->own_base + a->Nt - 1 + (a->park_target ? 1 : 0),
+                    a->own_rows);
+    if (a->B == 0) return ARTAB_OK;
+    if (!a->tape || !a->vecs || !a->kv || !a->norm_gamma || !a->norm_beta || !a->b_h1 || !a->b_h2 || !a->mix || !a->rand_u || !a->rand_n ||
+        !a->x_mean || !a->w_x || !a->b_x || !a->w_y || !a->b_y || !a->markers || !a->ar_tokens || !a->preds)
+        return fail(ARTAB_ERR_NULL_POINTER, "trajectory_decode: no pointer may be NULL");
+    if (misaligned16(a->tape) || misaligned16(a->vecs))
+        return fail(ARTAB_ERR_BAD_STRIDE, "trajectory_decode: tape and vecs must be 16-byte aligned");
+    TrajectoryParams P{};
+    P.tape = static_cast<const char *>(a->tape); P.tape_stride = t.stride; P.vecs = a->vecs;
+    P.kv = reinterpret_cast<const unsigned long long *>(a->kv); P.n_layers = a->n_layers;
+    P.n_ctx = a->n_ctx; P.ctx_rows = a->ctx_rows; P.own_base = a->own_base; P.own_rows = a->own_rows; P.park_target = a->park_target;
+    P.qscale = resolve_scale(0.f, 32) * kLog2e;
+    P.eps1 = a->eps1; P.eps2 = a->eps2; P.eps3 = a->eps3;
+    P.norm_g = a->norm_gamma; P.norm_b = a->norm_beta; P.eps_out = a->eps;
+    P.b_h1 = a->b_h1; P.b_h2 = a->b_h2; P.mix = a->mix; P.K = a->K; P.std_min = a->std_min; P.std_max = a->std_max;
+    P.rand_u = a->rand_u; P.rand_n = a->rand_n; P.rand_n_f32 = a->rand_n_f32 || dtype == ARTAB_F32; P.x_mean = a->x_mean;
+    P.w_x = a->w_x; P.b_x = a->b_x; P.w_y = a->w_y; P.b_y = a->b_y; P.markers = a->markers; P.ar_tokens = a->ar_tokens; P.bs = a->bs;
+    P.preds = a->preds; P.B = a->B; P.Nt = a->Nt; P.G = a->group;
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    hipError_t e = dtype == ARTAB_BF16 ? launch_trajectory_decode_bf16(P, a->D, a->F, st)
+                   : dtype == ARTAB_F16 ? launch_trajectory_decode_f16(P, a->D, a->F, st)
+                                        : launch_trajectory_decode_f32(P, a->D, a->F, st);
+    return launch_status(e, "trajectory_decode");
 }
 
 }  // extern "C"

@@ -11,6 +11,7 @@
 #include "attention_backward.h"
 #include "fused_layer.h"
 #include "mfma_flash.h"
+#include "trajectory_decode.h"
 
 namespace artab {
 
@@ -35,6 +36,7 @@ enum Tune : int {
     kTuneNW,              // ARTAB_NW: 2 = two wavefronts of two query blocks for 128-row tiles
     kTuneTileRows,        // ARTAB_TILE_ROWS: token rows per workgroup of the layer kernels (16/32)
     kTuneLayerFetchers,   // ARTAB_LAYER_FETCHERS: weight-fetching workgroups per XCD of a layer-boundary launch (0..32)
+    kTuneTrajectory,      // ARTAB_TRAJECTORY: 0 keeps sampling runs off the whole-run kernel, 1..8 trajectories per workgroup
     kTuneCount
 };
 // The override of `key` if one is set, else `fallback` (artab_api.hip).
@@ -94,5 +96,29 @@ hipError_t launch_layer_post_pre(const FusedPostParams &P, const FusedPreParams 
 hipError_t launch_sample_embed(const SampleEmbedParams &P, int D, int F, bool is_bf16, hipStream_t st);
 hipError_t launch_step_boundary(const FusedPostParams &P, const SampleEmbedParams &S, const FusedPreParams &N, int D,
                                 int F, bool is_bf16, hipStream_t st);
+
+
+// trajectory_launch.hip (one object per element type): the whole-run decode kernel and its weight
+// tapes.  A layout of zeros (stride 0) says that no kernel is built for the widths.
+struct TrajectoryTapeLayout {
+    // fragment (contraction step k, block b) of a wavefront at first + k * step + offset + b
+    struct Matrix {
+        int first, step, offset, per_wave;
+    };
+    long stride;            // bytes of one wavefront's tape
+    int layer, head, ring;  // fragments of a layer, of the head, of the register ring
+    Matrix fo, qkv[3], o, w1, w2, h1, h2;
+};
+#define ARTAB_TRAJ_DECLARE(suffix)                                                                       \
+    TrajectoryTapeLayout trajectory_tape_layout_##suffix(int D, int F, int n_layers);                    \
+    hipError_t launch_trajectory_tape_##suffix(const void *w, char *tape, long stride, int N, int K,     \
+                                               const TrajectoryTapeLayout::Matrix &m, int section,       \
+                                               hipStream_t st);                                          \
+    hipError_t launch_trajectory_decode_##suffix(const TrajectoryParams &P, int D, int F, hipStream_t st);
+ARTAB_TRAJ_DECLARE(bf16)
+ARTAB_TRAJ_DECLARE(f16)
+ARTAB_TRAJ_DECLARE(f32)
+#undef ARTAB_TRAJ_DECLARE
+hipError_t launch_trajectory_tape_wrap(char *tape, long stride, long bytes, hipStream_t st);
 
 }  // namespace artab

@@ -19,7 +19,8 @@ from torch import Tensor, nn
 
 from . import _lib
 
-__all__ = ["add_layer_norm", "bias_gelu", "layer_fusable", "pack_weight", "layer_pre", "layer_post", "layer_post_pre", "SampleEmbedStep", "DecodeStepBoundary"]
+__all__ = ["add_layer_norm", "bias_gelu", "layer_fusable", "pack_weight", "layer_pre", "layer_post", "layer_post_pre", "SampleEmbedStep", "DecodeStepBoundary",
+           "TrajectoryDecoder"]
 
 
 def _rows2d(t: Tensor) -> Tensor:
@@ -339,3 +340,110 @@ class DecodeStepBoundary:
                 _lib.current_stream(self.tail.device),
             )
         )
+
+
+class TrajectoryDecoder:
+    """A whole sampling run as one launch (``artab_trajectory_decode``): every workgroup takes a few
+    trajectories through all steps and all layers.  Holds what the launch reads of a model — its
+    weights in the order the kernel consumes them, the small vectors packed — and is built once per
+    model state; ``__call__`` only launches."""
+
+    MAX_COMPONENTS = 21  # 3 K outputs in 64 columns
+
+    @staticmethod
+    def supported(embedder, backbone, head, x: Tensor) -> bool:
+        """Whether the kernel is built for this model: equal layers of head dim 32 and widths it has
+        tiles for (``artab_trajectory_tape_bytes``), a scalar mixture head of the same hidden width."""
+        layers = list(backbone.layers)
+        if not (x.is_cuda and x.dtype in _lib._DTYPE_CODE and layers):
+            return False
+        lin1, lin2 = head.head[0], head.head[2]
+        D, F_ = lin1.in_features, lin1.out_features
+        first = layers[0]
+
+        def same(layer):
+            lf = layer.ff
+            return (layer.attn_rows.n_heads * 32 == D and lf[0].in_features == D and lf[0].out_features == F_
+                    and lf[2].out_features == D and lf[0].bias is not None and lf[2].bias is not None
+                    and all(getattr(layer, n).eps == getattr(first, n).eps for n in ("norm1", "norm2", "norm3"))
+                    and layer.norm1.weight.dtype == x.dtype)
+
+        return (head.dim_y == 1 and head.num_components <= TrajectoryDecoder.MAX_COMPONENTS
+                and lin2.out_features == 3 * head.num_components and lin1.bias is not None and lin2.bias is not None
+                and all(same(layer) for layer in layers)
+                and _lib.load().artab_trajectory_tape_bytes(D, F_, len(layers), _lib.dtype_code(x.dtype)) > 0)
+
+    def __init__(self, embedder, backbone, head, ar_tokens: Tensor):
+        lib = _lib.load()
+        layers = list(backbone.layers)
+        lin1, lin2 = head.head[0], head.head[2]
+        D, F_, L = lin1.in_features, lin1.out_features, len(layers)
+        dt, dev = lin1.weight.dtype, lin1.weight.device
+        code, stream = _lib.dtype_code(dt), _lib.current_stream(dev)
+        self.dtype_code, self.device = code, dev
+        self.D, self.F, self.L, self.H = D, F_, L, layers[0].attn_rows.n_heads
+        tape = torch.empty(lib.artab_trajectory_tape_bytes(D, F_, L, code), device=dev, dtype=torch.uint8)
+
+        def pack(w, which, layer=0, rows=0):
+            w = w.detach().contiguous() if w is not None else None
+            _lib.check(lib.artab_trajectory_pack(_ptr(tape), _ptr(w), which, layer, rows, D, F_, L, code, stream))
+
+        vecs = torch.zeros((L, 8, max(D, F_)), device=dev, dtype=dt)
+        for i, layer in enumerate(layers):
+            w_fo, w_qkv = layer.fused_weights()
+            pack(w_fo, _lib.TAPE_FO, i)
+            pack(w_qkv, _lib.TAPE_QKV, i)
+            pack(layer.attn_rows.out_proj.weight, _lib.TAPE_O, i)
+            pack(layer.ff[0].weight, _lib.TAPE_1, i)
+            pack(layer.ff[2].weight, _lib.TAPE_2, i)
+            for j, v in enumerate((layer.norm1.weight, layer.norm1.bias, layer.norm2.weight, layer.norm2.bias,
+                                   layer.ff[0].bias, layer.norm3.weight, layer.norm3.bias, layer.ff[2].bias)):
+                vecs[i, j, : v.numel()] = v.detach()
+        pack(lin1.weight, _lib.TAPE_H1)
+        pack(lin2.weight, _lib.TAPE_H2, rows=lin2.out_features)
+        pack(None, _lib.TAPE_CLOSE)
+        b_h2 = torch.zeros(64, device=dev, dtype=dt)
+        b_h2[: lin2.out_features] = lin2.bias.detach()
+        vec = lambda p: p.detach().reshape(-1).contiguous()  # noqa: E731
+        # everything the launch points at is kept alive here
+        self._keep = k = dict(
+            tape=tape, vecs=vecs, b_h1=vec(lin1.bias), b_h2=b_h2,
+            mix=torch.cat([vec(head.mean_bias), vec(head.std_bias), vec(head.weight_bias)]).to(dt),
+            w_x=vec(embedder.x_embed.weight), b_x=vec(embedder.x_embed.bias),
+            w_y=vec(embedder.y_embed.weight), b_y=vec(embedder.y_embed.bias),
+            markers=embedder.marker_embed.weight.detach().contiguous(), ar_tokens=ar_tokens.detach().contiguous(),
+            norm_g=vec(backbone.norm.weight), norm_b=vec(backbone.norm.bias),
+        )
+        a = self.args = _lib.ArtabTrajectoryArgs()
+        a.tape, a.vecs, a.n_layers = tape.data_ptr(), vecs.data_ptr(), L
+        a.eps1, a.eps2, a.eps3 = layers[0].norm1.eps, layers[0].norm2.eps, layers[0].norm3.eps
+        a.norm_gamma, a.norm_beta, a.eps = k["norm_g"].data_ptr(), k["norm_b"].data_ptr(), backbone.norm.eps
+        a.b_h1, a.b_h2, a.mix = k["b_h1"].data_ptr(), b_h2.data_ptr(), k["mix"].data_ptr()
+        a.K, a.std_min, a.std_max = head.num_components, float(head.std_min), 2.0
+        a.w_x, a.b_x, a.w_y, a.b_y = (k[n].data_ptr() for n in ("w_x", "b_x", "w_y", "b_y"))
+        a.markers, a.ar_tokens, a.bs = k["markers"].data_ptr(), k["ar_tokens"].data_ptr(), ar_tokens.shape[0]
+        a.D, a.F = D, F_
+        self._kv_key = None
+
+    def group(self, B: int, Nc: int, Nt: int, own_context: bool) -> int:
+        """Trajectories per workgroup, or 0 where the step-by-step launches are the faster route."""
+        return _lib.load().artab_trajectory_group(B, Nc, Nt, self.H, self.D, self.F, int(own_context), self.dtype_code)
+
+    def __call__(self, caches, n_ctx: int, own_base: int, x_mean: Tensor, rand_u: Tensor, rand_n: Tensor, group: int) -> Tensor:
+        """``caches``: per layer ``(context K, context V, trajectory K, trajectory V)``, contiguous; with
+        ``n_ctx == 0`` every trajectory's own context fills the first ``own_base`` rows of its cache and
+        the context tensors are not read.  ``x_mean [B,Nt]``; ``rand_u`` / ``rand_n`` ``[>=Nt,B]``.  Returns
+        the drawn values ``[B,Nt]``."""
+        key = tuple(t.data_ptr() for layer in caches for t in layer)
+        if key != self._kv_key:
+            self._kv = torch.tensor(key, dtype=torch.int64, device=self.device)
+            self._kv_key = key
+        B, Nt = x_mean.shape
+        preds = torch.empty((B, Nt), device=self.device, dtype=x_mean.dtype)
+        a = self.args
+        a.kv, a.n_ctx, a.ctx_rows, a.own_base = self._kv.data_ptr(), n_ctx, caches[0][0].shape[-2], own_base
+        a.own_rows, a.park_target = caches[0][2].shape[2], int(n_ctx == 0)
+        a.rand_u, a.rand_n, a.rand_n_f32 = rand_u.data_ptr(), rand_n.data_ptr(), int(rand_n.dtype == torch.float32)
+        a.x_mean, a.preds, a.B, a.Nt, a.group = x_mean.data_ptr(), preds.data_ptr(), B, Nt, group
+        _lib.check(_lib.load().artab_trajectory_decode(ctypes.byref(a), self.dtype_code, _lib.current_stream(self.device)))
+        return preds

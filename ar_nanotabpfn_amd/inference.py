@@ -26,7 +26,7 @@ from torch import Tensor
 from . import attention_kernels as ak
 from .attention import DecodeMask, TeacherForcingMask
 from . import _lib
-from .glue import SampleEmbedStep, DecodeStepBoundary, add_layer_norm
+from .glue import SampleEmbedStep, DecodeStepBoundary, TrajectoryDecoder, add_layer_norm
 
 __all__ = ["ARTabPFNPredictor"]
 
@@ -90,6 +90,10 @@ class ARTabPFNPredictor:
         # In the sampling loop the last layer finishes the target row only: the buffer row's output
         # of that layer is read by nobody (its K/V were cached before the attention call).
         self.target_only_last_layer = True
+        # Take a whole sampling run through one launch where that is the faster route (the library's
+        # rule, ``artab_trajectory_group``) and the sampling switches above are at their defaults.
+        self.whole_run_decode = True
+        self._trajectory = None      # (key of the model state, TrajectoryDecoder or None)
         self._side_streams = {}
         self._graph_state = None
         self._graph_params = None    # the tensors a recorded step points at (collected at first use)
@@ -373,6 +377,9 @@ class ARTabPFNPredictor:
         """The decode loop of ``sample_sequence`` (inference.py:353-366) on caches that
         are already initialised and prefilled: samples ``x_target [B,Nt,F]`` in order."""
         Nt = x_target.shape[1]
+        values = self._sample_whole_run(x_target)
+        if values is not None:
+            return values
         if (self.use_hip_graph and self.backend == _SHARED and x_target.is_cuda and Nt >= 3
                 and self.buffer_len == 0 and Nt <= self.max_buffer_len):
             return self._sample_sequence_graph(x_target)
@@ -384,6 +391,60 @@ class ARTabPFNPredictor:
             preds.append(y_t)
             prev_x, prev_y = x_t, y_t
         return torch.cat(preds, dim=1)
+
+    def _model_key(self):
+        """What identifies the state of the model's weights, and the tensors it was taken from."""
+        # (walking the module tree costs a millisecond of host time with the GPU idle: done once; a
+        # weight that is updated or moved changes its version or address and is seen through the key)
+        if self._graph_params is None:
+            self._graph_params = (list(self.backbone.parameters()) + list(self.embedder.parameters()) +
+                                  list(self.head.parameters()) + [self.ar_tokens])
+        return tuple((p.data_ptr(), p._version) for p in self._graph_params)
+
+    def _sample_whole_run(self, x_target: Tensor) -> Optional[Tensor]:
+        """The sampling run as one launch (``TrajectoryDecoder``), or None where it does not apply.  The
+        variates are drawn from torch's generator in the order in which the other routes draw them, so
+        that a seed gives the same values on every route."""
+        B, Nt, _ = x_target.shape
+        shared = self.backend == _SHARED
+        layers = self.backbone.layers
+        if not (self.whole_run_decode and self.use_hip_graph and self.fuse_step_tail and not self.launch_live
+                and int(self.decode_chains) == 1 and x_target.is_cuda and Nt >= 1):
+            return None
+        if shared:
+            caches = [(l.k_ctx_cache, l.v_ctx_cache, l.k_buf_cache, l.v_buf_cache) for l in layers]
+            n_ctx, own_base, fits = self.context_len, 0, self.buffer_len == 0 and Nt <= self.max_buffer_len
+        else:
+            caches = [(l.k_cache, l.v_cache, l.k_cache, l.v_cache) for l in layers]
+            n_ctx, own_base, fits = 0, self.seq_len, self.seq_len + Nt <= layers[0].k_cache.shape[2]
+        if not (fits and n_ctx + own_base > 0 and caches[0][2].shape[0] == B
+                and all(t.dtype == x_target.dtype and t.is_contiguous() for c in caches for t in c)):
+            return None
+        key = (x_target.dtype, self._model_key())
+        if self._trajectory is None or self._trajectory[0] != key:
+            ok = TrajectoryDecoder.supported(self.embedder, self.backbone, self.head, x_target)
+            self._trajectory = (key, TrajectoryDecoder(self.embedder, self.backbone, self.head, self.ar_tokens) if ok else None)
+        run = self._trajectory[1]
+        group = run.group(B, n_ctx + own_base, Nt, not shared) if run is not None else 0
+        if group == 0:
+            return None
+        device, dtype = x_target.device, x_target.dtype
+        if shared and Nt >= 3 and SampleEmbedStep.supported(self.embedder, self.backbone, self.head, x_target):
+            rand_u, rand_n = torch.empty((2, self.max_buffer_len, B), device=device, dtype=torch.float32).unbind(0)
+            self._draw_step_variates(rand_u, rand_n)
+        else:
+            rand_u = torch.empty((Nt, B), device=device, dtype=torch.float32)
+            rand_n = torch.empty((Nt, B), device=device, dtype=dtype)
+            for u, n in zip(rand_u.unbind(0), rand_n.unbind(0)):  # as head.sample does, step by step
+                u.uniform_()
+                n.normal_()
+        values = run(caches, n_ctx, own_base, x_target.mean(dim=-1).contiguous(), rand_u, rand_n, group)
+        if shared:
+            self.buffer_len = Nt - 1
+            self.seq_len = self.context_len + self.buffer_len
+        else:
+            self.seq_len += Nt - 1
+        return values
 
     def _graph_step(self, st) -> None:
         """One ``[buffer, target]`` decode step driven entirely by device-side state
@@ -452,12 +513,6 @@ class ARTabPFNPredictor:
         B, Nt, F_ = x_target.shape
         device, dtype = x_target.device, x_target.dtype
         layer0 = self.backbone.layers[0]
-        # (walking the module tree costs a millisecond of host time with the GPU idle: done once; a
-        # weight that is updated or moved changes its version or address and is seen through the key)
-        if self._graph_params is None:
-            self._graph_params = (list(self.backbone.parameters()) + list(self.embedder.parameters()) +
-                                  list(self.head.parameters()) + [self.ar_tokens])
-        params = self._graph_params
         chain_rows = self._chain_rows(B)
         # The recorded step depends on the capacity of the buffer cache, not on how many steps are
         # replayed: loop state is sized for the capacity, so runs of any length share one recording.
@@ -465,7 +520,7 @@ class ARTabPFNPredictor:
         key = (B, cap, F_, self.context_len, dtype, str(device), layer0.k_ctx_cache.data_ptr(),
                layer0.k_buf_cache.data_ptr(), self.fuse_step_tail, self.overlap_buffer_pass, self.merge_in_layer,
                len(chain_rows), int(self.steps_per_graph), bool(self.counter_ordering),
-               bool(self.target_only_last_layer), bool(self.fuse_step_boundary), tuple((p.data_ptr(), p._version) for p in params))
+               bool(self.target_only_last_layer), bool(self.fuse_step_boundary), self._model_key())
         gs = self._graph_state
         if gs is None or gs.key != key:
             gs = _GraphState()

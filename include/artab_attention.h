@@ -85,7 +85,8 @@ const char *artab_last_error(void);
  * environment of the host process cannot change a kernel route between two calls.  Keys:
  * ARTAB_BM, ARTAB_SPLIT, ARTAB_SMALL, ARTAB_STREAM, ARTAB_STREAM_PER_CU, ARTAB_STREAM_PRIO,
  * ARTAB_STREAM_SHORT, ARTAB_STREAM_CALM, ARTAB_DENSE_BELOW, ARTAB_CTX_YIELD, ARTAB_ORDER_GATE_LAUNCH,
- * ARTAB_BN, ARTAB_LEAN, ARTAB_LEAN_OCC, ARTAB_NW, ARTAB_TILE_ROWS, ARTAB_LAYER_FETCHERS (what each
+ * ARTAB_BN, ARTAB_LEAN, ARTAB_LEAN_OCC, ARTAB_NW, ARTAB_TILE_ROWS, ARTAB_LAYER_FETCHERS,
+ * ARTAB_TRAJECTORY (what each
  * selects: csrc/launchers.h).
  *   artab_tuning_set: enable != 0 sets the override to `value`, enable == 0 removes it (the
  *                     library's own choice applies again).  Not thread-safe against running calls.
@@ -494,6 +495,60 @@ typedef struct artab_sample_embed_args {
 } artab_sample_embed_args;
 
 int artab_decode_sample_embed(const artab_sample_embed_args *args, int dtype, void *stream);
+
+/*
+ * A whole sampling run in one launch: every workgroup takes a few trajectories through all Nt steps
+ * and all layers of the model (inference.py:278-320, :353-366 with the layers of :687-744 or
+ * :746-833).  Contexts are in the caches; the buffer rows are appended there as the run goes.
+ *
+ * artab_trajectory_group says how many trajectories a workgroup should take, or 0: no kernel for
+ * these widths (head_dim 32; D in {128, 256, 512}, F = 256; D 512 in 16-bit types only), or the step-by-step
+ * launches, which spread one layer over the whole chip, are the faster route for this problem.
+ * own_context: every trajectory has its own context rows in front of its buffer rows.
+ *
+ * The weights are kept a second time as `tape`, artab_trajectory_tape_bytes of device memory (16-byte aligned),
+ * written by artab_trajectory_pack: once per layer for ARTAB_TAPE_FO (w = W_out W_v of the feature attention,
+ * [D, D]), _QKV ([3D, D]), _O, _1 ([F, D]), _2 ([D, F]), once with layer = 0 for _H1 ([F, D]) and _H2
+ * ([n, F], n <= 64 given as `rows`), and at the very end ARTAB_TAPE_CLOSE (w = NULL).
+ */
+#define ARTAB_TAPE_FO 0
+#define ARTAB_TAPE_QKV 1
+#define ARTAB_TAPE_O 2
+#define ARTAB_TAPE_1 3
+#define ARTAB_TAPE_2 4
+#define ARTAB_TAPE_H1 5
+#define ARTAB_TAPE_H2 6
+#define ARTAB_TAPE_CLOSE 7
+typedef struct artab_trajectory_args {
+    const void *tape;
+    const void *vecs;        /* [n_layers][8][max(D, F)]: norm1 g, b, norm2 g, b, ff bias 1, norm3 g, b, ff bias 2 */
+    const uint64_t *kv;      /* device: [n_layers][4] addresses of context K, V and trajectory K, V */
+    int n_layers;
+    int n_ctx, ctx_rows;     /* shared context: rows used of [H, ctx_rows, 32]; 0: own contexts */
+    int own_base, own_rows;  /* own context rows in front; rows of [B, H, own_rows, 32] */
+    int park_target;         /* store the last target row's K, V behind the last committed row */
+    float eps1, eps2, eps3;
+    const void *norm_gamma, *norm_beta; /* backbone.norm */
+    float eps;
+    const void *b_h1, *b_h2; /* head biases [F], [64] (zeros behind 3 K) */
+    const void *mix;         /* [3][K]: mean, std and weight biases */
+    int K;                   /* <= 21 */
+    float std_min, std_max;
+    const float *rand_u;     /* [Nt, B] uniform in [0, 1) */
+    const void *rand_n;      /* [Nt, B] standard normal, float32 or (rand_n_f32 = 0) of the model's type */
+    int rand_n_f32;
+    const void *x_mean;      /* [B, Nt] */
+    const void *w_x, *b_x, *w_y, *b_y, *markers, *ar_tokens; /* as in artab_sample_embed_args */
+    int bs;
+    void *preds;             /* [B, Nt] */
+    int B, Nt, group, D, F;
+} artab_trajectory_args;
+
+int artab_trajectory_group(int B, int Nc, int Nt, int H, int D, int F, int own_context, int dtype);
+size_t artab_trajectory_tape_bytes(int D, int F, int n_layers, int dtype);
+int artab_trajectory_pack(void *tape, const void *w, int which, int layer, int rows, int D, int F, int n_layers,
+                          int dtype, void *stream);
+int artab_trajectory_decode(const artab_trajectory_args *args, int dtype, void *stream);
 
 /*
  * The boundary between two decode steps in one launch: artab_layer_post (or
