@@ -1483,28 +1483,34 @@ static TrajectoryTapeLayout trajectory_layout(int D, int F, int n_layers, int dt
 }
 
 // The rule for the whole-run kernel.  Per layer and step one of its workgroups streams the layer's
-// weights, the context and its trajectories' rows through one compute unit (64 B per clock), and
-// pays about 3 us for nine barriers; the launches of the other route take 27 us (45 us at d_model 512,
-// whose layer kernel streams 3 MB of weights per workgroup as well) unless their context pass, which
-// has the matrix cores of the whole chip, takes longer.  A trajectory with a context of its own has
-// no recorded alternative: it always comes here.
+// weights, the context and its trajectories' rows through one compute unit: 3 us and 85 GB/s of those
+// bytes (float32, bound by its products as well: 52 GB/s), whatever the batch.  The launches of the
+// other route take 26 / 29 / 50 us at d_model 128 / 256 / 512, more beyond 1024 trajectories, and
+// their context pass has the matrix cores of the whole chip (float32: neither fused nor on the matrix
+// cores).  Measured on 48 shapes (4 layers, 24 steps; us per layer and step, whole run against launches):
+// d_model 128, 256 trajectories: 8.6 / 24.9 at 64 context rows, 14.8 / 27.1 at 1024, 35.6 / 27.5 at 4096;
+// d_model 256: 15.3 / 28.9, 21.1 / 31.0 at 512, 39.6 / 31.0 at 2048; d_model 512: 38.6 / 49.7, 49.3 / 52.1
+// at 512, 87.7 / 53.8 at 2048; float32 at d_model 256: 37.5 / 186, 71.0 / 443 at 1024.
+// A trajectory with a context of its own has no recorded alternative: it always comes here.
 int artab_trajectory_group(int B, int Nc, int Nt, int H, int D, int F, int own_context, int dtype) {
-    if (B < 1 || Nt < 1 || Nc < 1 || H * 32 != D || trajectory_layout(D, F, 1, dtype).stride == 0) return 0;
+    const TrajectoryTapeLayout layout = trajectory_layout(D, F, 1, dtype);
+    if (B < 1 || Nt < 1 || Nc < 1 || H * 32 != D || layout.stride == 0) return 0;
     static const int cus = [] {
         int dev = 0, n = 0;
         if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
             n = 256;
         return n;
     }();
-    const int group = B <= cus ? 1 : (B + cus - 1) / cus < kTrajMax ? (B + cus - 1) / cus : kTrajMax;
+    const int most = layout.max_group, group = (B + cus - 1) / cus < most ? (B + cus - 1) / cus : most;
     const int force = tune(kTuneTrajectory, -1);
-    if (force >= 0) return force == 0 ? 0 : force < kTrajMax ? force : kTrajMax;
+    if (force >= 0) return force < most ? force : most;
     if (own_context) return group;
     const double esz = elem_size(dtype), rounds = std::ceil(std::ceil(static_cast<double>(B) / group) / cus);
     const double bytes = esz * (5.0 * D * D + 2.0 * D * F) + 2 * esz * D * (Nc + 0.5 * Nt * group);
-    const double here = rounds * (3.0 + bytes / 150e3);
+    const double here = rounds * (3.0 + bytes / (dtype == ARTAB_F32 ? 52e3 : 85e3));
     const double flops = 8.0 * B * Nc * D;
-    const double there = (D == 512 ? 45.0 : 27.0) + (dtype == ARTAB_F32 ? 30.0 + flops / 5e6 : flops / 1200e6);
+    const double there = (D == 512 ? 50.0 : D == 256 ? 29.0 : 26.0) + (B > 1024 ? 4.2e-5 * (B - 1024) * D : 0.0) +
+                         (dtype == ARTAB_F32 ? 70.0 + flops / 5e6 : flops / 1200e6);
     return here < there ? group : 0;
 }
 
@@ -1553,7 +1559,7 @@ int artab_trajectory_decode(const artab_trajectory_args *a, int dtype, void *str
     const TrajectoryTapeLayout t = trajectory_layout(a->D, a->F, a->n_layers, dtype);
     if (t.stride == 0 || a->n_layers < 1)
         return fail(ARTAB_ERR_UNSUPPORTED, "no whole-run decode kernel for D=%d F=%d layers=%d dtype code %d", a->D, a->F, a->n_layers, dtype);
-    if (a->B < 0 || a->Nt < 1 || a->K < 1 || a->K > kTrajMaxMix || a->bs < 1 || a->group < 1 || a->group > kTrajMax)
+    if (a->B < 0 || a->Nt < 1 || a->K < 1 || a->K > kTrajMaxMix || a->bs < 1 || a->group < 1 || a->group > t.max_group)
         return fail(ARTAB_ERR_BAD_SHAPE, "trajectory_decode: bad sizes B=%d Nt=%d K=%d bs=%d group=%d", a->B, a->Nt, a->K, a->bs, a->group);
     if (a->n_ctx < 0 || a->own_base < 0 || (a->n_ctx == 0) == (a->own_base == 0) || a->n_ctx > a->ctx_rows)
         return fail(ARTAB_ERR_BAD_SHAPE, "trajectory_decode: one of a shared context (%d of %d rows) and own contexts (%d rows)", a->n_ctx,

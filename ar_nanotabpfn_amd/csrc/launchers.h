@@ -107,6 +107,7 @@ struct TrajectoryTapeLayout {
     };
     long stride;            // bytes of one wavefront's tape
     int layer, head, ring;  // fragments of a layer, of the head, of the register ring
+    int max_group;          // trajectories a workgroup can take
     Matrix fo, qkv[3], o, w1, w2, h1, h2;
 };
 #define ARTAB_TRAJ_DECLARE(suffix)                                                                       \

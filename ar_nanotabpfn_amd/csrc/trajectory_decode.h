@@ -5,51 +5,54 @@
 // of one trajectory needs from the rest of the chip is the weights and the context's keys and values,
 // both constant.  A step that is cut into launches (context pass, buffer pass, layer boundary, tail)
 // pays 30-40 us per layer for them whatever the size of the problem; here a layer costs what one
-// compute unit needs to stream its weights and keys through (64 B per clock from the L2) plus nine
-// workgroup barriers.  What bounds it: that stream.  Measured per layer at d_model 128 / 256 / 512
-// (short contexts): see trajectory_decode_applies() in trajectory_launch.hip, which holds the rule
-// for when the launches of the other route, which spread one layer over the whole chip, are faster.
+// compute unit needs to stream its weights and keys through (64 B per clock from the L2) plus ten
+// workgroup barriers and the latency chains between them.  The rule for when the launches of the
+// other route, which spread one layer over the whole chip, are faster is artab_trajectory_group().
 //
-// Rows.  A workgroup owns G <= 8 trajectories; token row 2 g is trajectory g's buffer row of the step
-// (the value drawn last), row 2 g + 1 its target row: 16 rows = one MFMA column block.  Products are
-// transposed as in fused_layer.h (C^T[n, m] = sum_k W[n, k] A[m, k] on 16x16 tiles): weights are the
-// A operand, the 16-row activation tile in LDS is the B operand; lane l holds token l % 16 and four
-// consecutive features 4 (l / 16) + r of every 16-feature block.
+// Rows.  A workgroup owns G trajectories; token row 2 g is trajectory g's buffer row of the step (the
+// value drawn last), row 2 g + 1 its target row: at most 16 rows (16-bit types) or 4 (float32, whose
+// matrix rate is an eighth: a 16-row tile with two rows in use would be bound by it).  Products are
+// transposed as in fused_layer.h (C^T[n, m] = sum_k W[n, k] A[m, k]): weights are the A operand, the
+// activation rows in LDS the B operand; a lane holds, for its token row, four consecutive features
+// 4 sub + r of every 16-feature block (TrajOps).
 //
 // Weights.  Each wavefront has a tape: the 1 KiB operand fragments it will consume, in the order it
 // consumes them, layer after layer, then the head's; the first kRing of them are repeated behind the
 // end.  A ring of kRing fragments in registers is always kRing ahead, across products, barriers,
 // layers and steps: after a fragment has been multiplied its registers receive the one kRing further
 // on.  All ring positions are compile-time constants (the fragments of a layer are a multiple of
-// kRing).
+// kRing).  A layer's small vectors travel one layer ahead into the other of two LDS buffers.
 //
 // Attention.  One wavefront owns a head (or half of a head's keys at 4 heads, two heads in turn at
-// 16); the columns of S^T = K Q^T are the 16 token rows.  Keys come in blocks: the shared context
-// serves every column, a trajectory's own rows only its two columns (the others are masked, their
-// state does not change), so no merge of partial results is needed.  The rows of this step that
-// have just been projected are keys too: one last block straight from LDS, masked to (row 2 g,
-// columns 2 g and 2 g + 1).  Softmax is online in float32 with scale * log2(e) folded into the
-// queries and rounded to the model's type, probabilities are rounded to the model's type: the
-// rounding model of the other kernels.
+// 16); the columns of S^T = K Q^T are the token rows.  Keys come in blocks: the shared context serves
+// every column, a trajectory's own rows only its two columns (the others are masked, their state does
+// not change), so no merge of partial results is needed.  The first blocks are requested ahead of the
+// q/k/v product.  The rows of this step that have just been projected are keys too: one last block
+// straight from LDS, masked to (row 2 g, columns 2 g and 2 g + 1).  Softmax in float32 with scale *
+// log2(e) folded into the queries and rounded to the model's type, probabilities rounded to the
+// model's type: the rounding model of the other kernels.  The reference a column's probabilities are
+// taken against follows its maximum only when that has risen by more than kSlack (base 2): the common
+// block has no exchange between lanes and no rescaling.
 #pragma once
+
+#include <type_traits>
 
 #include "common.h"
 #include "mfma_flash.h"
 
 namespace artab {
 
-constexpr int kTrajRows = 16;   // token rows of a workgroup
-constexpr int kTrajMax = 8;     // trajectories of a workgroup
 constexpr int kTrajWaves = 8;
 constexpr int kTrajMaxMix = 21; // 3 K outputs of the head fit 64 columns
 constexpr int kTrajHeadOut = 64;
+constexpr int kTrajMaxLayers = 64;
 
 struct TrajectoryParams {
     const char *tape;        // kTrajWaves tapes of `tape_stride` bytes
     long tape_stride;
     const void *vecs;        // [n_layers][8][max(D, F)]: g1, b1, g2, b2, bias_1, g3, b3, bias_2
     const unsigned long long *kv;  // [n_layers][4] addresses: context K, V; trajectory K, V
-    int n_layers;
+    int n_layers;            // <= kTrajMaxLayers
     // shared context: rows [0, n_ctx) of [H, ctx_rows, 32]; own_base = 0.  Per-trajectory context:
     // n_ctx = 0 and the trajectory's cache holds its context in rows [0, own_base).
     int n_ctx, ctx_rows, own_base;
@@ -73,24 +76,75 @@ struct TrajectoryParams {
     int B, Nt, G;
 };
 
-// One 1 KiB fragment of each operand: 16-bit types one 16x16x32 product, float32 four 16x16x4 ones
-// (element j of every lane's four makes the contraction indices 4 s + j of both operands).
+// Exchanges between the four rows of 16 lanes (gfx950 swaps: vector instructions, no LDS).  (Elements
+// of a vector are copied to scalars before they are reinterpreted: __builtin_bit_cast of a vector's
+// element reads element 0.)
+template <typename Op>
+__device__ __forceinline__ float over_rows(float x, Op op) {
+    const unsigned a = __builtin_bit_cast(unsigned, x);
+    auto s = __builtin_amdgcn_permlane32_swap(a, a, false, false);
+    unsigned lo = s[0], hi = s[1];
+    const unsigned b = __builtin_bit_cast(unsigned, op(__builtin_bit_cast(float, lo), __builtin_bit_cast(float, hi)));
+    s = __builtin_amdgcn_permlane16_swap(b, b, false, false);
+    lo = s[0];
+    hi = s[1];
+    return op(__builtin_bit_cast(float, lo), __builtin_bit_cast(float, hi));
+}
+__device__ __forceinline__ float row_sum(float x) {
+    return over_rows(x, [](float a, float b) { return a + b; });
+}
+__device__ __forceinline__ float row_max(float x) {
+    return over_rows(x, [](float a, float b) { return fmaxf(a, b); });
+}
+// x of the lane `N` further on in the row of 16 (row_ror)
+template <int N>
+__device__ __forceinline__ float row_rotate(float x) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0x120 | N, 0xf, 0xf, true));
+}
+
+// One 1 KiB fragment per operand and product.  Both types read the A operand as row lane % 16 of a
+// 16-row block, kPer consecutive contraction elements at kPer (lane / 16).
+//   16-bit: one 16x16x32 product; token lane % 16, features 4 sub + r with sub = lane / 16.
+//   float32: four 4x4x1 products of 16 independent 4x4 blocks: block (lane / 16, lane / 4 % 4) holds
+//   the partial sums of features 4 (lane / 4 % 4) + r over the contraction elements of lane / 16;
+//   finish() adds the four of them, every row of 16 lanes then holds the same values.
 template <typename T>
 struct TrajOps {
-    static constexpr int kStep = 32, kPer = 8;
+    static constexpr int kRows = 16, kMax = 8, kStep = 32, kPer = 8;
+    static constexpr float kSlack = std::is_same<T, f16_t>::value ? 8.f : 16.f;
+    static __device__ __forceinline__ int tok(int lane) { return lane & 15; }
+    static __device__ __forceinline__ int sub(int lane) { return lane >> 4; }
     static __device__ __forceinline__ f32x4 mma(u32x4 a, u32x4 b, f32x4 c) {
         typedef typename MfmaOps<T>::vec vec;
         return MfmaOps<T>::mma16(__builtin_bit_cast(vec, a), __builtin_bit_cast(vec, b), c);
     }
+    static __device__ __forceinline__ void finish(f32x4 &) {}
+    static __device__ __forceinline__ float sum(float x) { return row_sum(x); }  // over a token's four subs
+    static __device__ __forceinline__ float max(float x) { return row_max(x); }
 };
 template <>
 struct TrajOps<float> {
-    static constexpr int kStep = 16, kPer = 4;
+    static constexpr int kRows = 4, kMax = 2, kStep = 16, kPer = 4;
+    static constexpr float kSlack = 16.f;
+    static __device__ __forceinline__ int tok(int lane) { return lane & 3; }
+    static __device__ __forceinline__ int sub(int lane) { return (lane >> 2) & 3; }
     static __device__ __forceinline__ f32x4 mma(u32x4 a, u32x4 b, f32x4 c) {
         const f32x4 fa = __builtin_bit_cast(f32x4, a), fb = __builtin_bit_cast(f32x4, b);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) c = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[j], fb[j], c, 0, 0, 0);
+        for (int j = 0; j < 4; ++j) c = __builtin_amdgcn_mfma_f32_4x4x1f32(fa[j], fb[j], c, 0, 0, 0);
         return c;
+    }
+    static __device__ __forceinline__ void finish(f32x4 &c) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) c[r] = row_sum(c[r]);
+    }
+    static __device__ __forceinline__ float sum(float x) {
+        x += row_rotate<8>(x);
+        return x + row_rotate<4>(x);
+    }
+    static __device__ __forceinline__ float max(float x) {
+        x = fmaxf(x, row_rotate<8>(x));
+        return fmaxf(x, row_rotate<4>(x));
     }
 };
 
@@ -116,26 +170,16 @@ __device__ __forceinline__ void traj_store4(T *p, const float (&f)[4]) {
     }
 }
 
-// A lane's entries of NB parameter vectors' 16-feature blocks, as they come from memory (converted where
-// they are used, so that nothing waits for them where they are requested).
-template <typename T, int NB>
-struct TrajCols {
-    typedef typename std::conditional<sizeof(T) == 2, u32x2, f32x4>::type raw_t;
-    raw_t raw[NB];
-    __device__ __forceinline__ void load(const T *vec, int wave, int s4) {
-#pragma unroll
-        for (int b = 0; b < NB; ++b) raw[b] = *reinterpret_cast<const raw_t *>(vec + 16 * (wave + kTrajWaves * b) + 4 * s4);
-    }
-    __device__ __forceinline__ void get(int b, float (&f)[4]) const {
-        if constexpr (sizeof(T) == 2) {
-            f[0] = unpack_lo<T>(raw[b][0]); f[1] = unpack_hi<T>(raw[b][0]);
-            f[2] = unpack_lo<T>(raw[b][1]); f[3] = unpack_hi<T>(raw[b][1]);
-        } else {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) f[e] = raw[b][e];
-        }
-    }
-};
+// gelu for results that are rounded to 16 bits: erf by the rational form 7.1.26 of Abramowitz and Stegun
+// (absolute error below 1.5e-7, a thousandth of the rounding that follows) in 14 instructions
+// instead of some 60; at two token rows in use the activation of all 16 was a quarter of its product.
+__device__ __forceinline__ float traj_gelu16(float x) {
+    const float z = fabsf(x) * 0.70710678118654752f;
+    const float t = __builtin_amdgcn_rcpf(fmaf(0.3275911f, z, 1.f));
+    const float poly = t * fmaf(t, fmaf(t, fmaf(t, fmaf(t, 1.061405429f, -1.453152027f), 1.421413741f), -0.284496736f), 0.254829592f);
+    const float erf = fmaf(-poly, fast_exp2(-z * z * kLog2e), 1.f);
+    return 0.5f * x * (1.f + copysignf(erf, x));
+}
 
 // Sizes shared by the kernel and the host code that writes the tapes.
 template <typename T, int D, int F>
@@ -178,26 +222,33 @@ template <typename T, int D, int F>
 __global__ __launch_bounds__(kTrajWaves * 64) void trajectory_decode_kernel(TrajectoryParams P) {
     typedef TrajOps<T> Ops;
     typedef TrajShape<T, D, F> S;
-    constexpr int NW = kTrajWaves, NT = NW * 64, DH = 32, H = D / DH;
+    constexpr int NW = kTrajWaves, NT = NW * 64, DH = 32, H = D / DH, ROWS = Ops::kRows;
     constexpr bool k16 = sizeof(T) == 2;
     constexpr int LD = D + (k16 ? 8 : 4), LF = F + (k16 ? 8 : 4);  // row strides: 16 bytes off a multiple of 128
     constexpr int VW = D > F ? D : F;
-    constexpr int BK = k16 ? 32 : 16;      // keys per block
-    constexpr int NP = NW > H ? NW / H : 1;  // wavefronts per head
-    constexpr int HPW = H > NW ? H / NW : 1; // heads per wavefront, in turn
+    // keys per block: one step of the second product's contraction.  (Two steps per block, which give the
+    // chains between the two products company, lose 12 % at 200 context rows: they round the
+    // requests up further, and a request costs the compute unit's address unit 16 clocks whatever it
+    // brings.)
+    constexpr int BK = k16 ? 32 : 16;
+    constexpr int NP = NW > H ? NW / H : 1;         // wavefronts per head
+    constexpr int HPW = H > NW ? H / NW : 1;        // heads per wavefront, in turn
     constexpr int VPAD = DH + 16;
 
-    __shared__ __attribute__((aligned(16))) T xs[kTrajRows * LD];   // layer input; attention output
-    __shared__ __attribute__((aligned(16))) T ys[kTrajRows * LD];   // normed feature stage, then x1; z of the head
-    constexpr int QKV = 3 * kTrajRows * LD, HID = kTrajRows * LF;
+    __shared__ __attribute__((aligned(16))) T xs[ROWS * LD];   // layer input; attention output
+    __shared__ __attribute__((aligned(16))) T ys[ROWS * LD];   // normed feature stage, then x1; z of the head
+    constexpr int QKV = 3 * ROWS * LD, HID = ROWS * LF;
     __shared__ __attribute__((aligned(16))) T qkv[QKV > HID ? QKV : HID];  // q, k, v of the step; hidden layer
-    T *const qs = qkv, *const kn = qkv + kTrajRows * LD, *const vn = qkv + 2 * kTrajRows * LD, *const hs = qkv;
+    T *const qs = qkv, *const kn = qkv + ROWS * LD, *const vn = qkv + 2 * ROWS * LD, *const hs = qkv;
     __shared__ __attribute__((aligned(16))) T v_lds[k16 ? NW * BK * VPAD : 8];
-    __shared__ float red_a[NW * kTrajRows], red_b[NW * kTrajRows];
-    __shared__ float part_o[NP > 1 ? NW * kTrajRows * DH : 1];
-    __shared__ float part_m[NP > 1 ? NW * kTrajRows : 1], part_l[NP > 1 ? NW * kTrajRows : 1];
-    __shared__ float raw_s[kTrajRows][kTrajHeadOut + 1];
-    __shared__ float y_s[kTrajMax], x_s[2 * kTrajMax];
+    __shared__ float red_a[NW * ROWS], red_b[NW * ROWS];
+    __shared__ __attribute__((aligned(16))) float part_o[NP > 1 ? NW * ROWS * DH : 4];
+    __shared__ float part_m[NP > 1 ? NW * ROWS : 1], part_l[NP > 1 ? NW * ROWS : 1];
+    __shared__ float raw_s[ROWS][kTrajHeadOut + 1];
+    __shared__ float y_s[Ops::kMax], x_s[2 * Ops::kMax];
+    // the parameter vectors of this layer and of the next; cache addresses of every layer
+    __shared__ __attribute__((aligned(16))) T pbuf[2][8 * VW];
+    __shared__ unsigned long long kv_s[4 * kTrajMaxLayers];
     // what the end of every step needs: norm g and b, x and y embedding w and b, markers target and
     // buffer; the head's biases; the position token of the coming step
     __shared__ __attribute__((aligned(16))) T cst[8 * D + F + kTrajHeadOut + 3 * kTrajMaxMix + 1], tok_s[D];
@@ -206,7 +257,8 @@ __global__ __launch_bounds__(kTrajWaves * 64) void trajectory_decode_kernel(Traj
              *const c_b2 = c_b1 + F, *const c_mix = c_b2 + kTrajHeadOut;
 
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-    const int tok = lane & 15, s4 = lane >> 4;
+    const int tok = Ops::tok(lane), sub = Ops::sub(lane);  // output layout of the products
+    const int row16 = lane & 15, quad = lane >> 4;         // operand layout
     const long b0 = static_cast<long>(blockIdx.x) * P.G;
     const int valid = static_cast<int>(min(static_cast<long>(P.G), P.B - b0));
 
@@ -218,38 +270,43 @@ __global__ __launch_bounds__(kTrajWaves * 64) void trajectory_decode_kernel(Traj
         ring[i] = *reinterpret_cast<const u32x4 *>(next);
         next += 1024;
     }
-    // acc[b] += W_b A^T over KS steps of NB blocks; fragments pos .. pos + KS * NB - 1 of the tape section
+    // acc[b] += W_b A^T over KS steps of NB blocks; fragments POS .. POS + KS * NB - 1 of the tape section
     auto product = [&](auto pos_, auto ks_, auto &acc, const T *act, int ld) {
         constexpr int POS = decltype(pos_)::value, KS = decltype(ks_)::value;
         constexpr int NB = sizeof(acc) / sizeof(acc[0]);
+        constexpr int KC = KS < 8 ? KS : 8;  // activation operands are read KC steps at a time
+        const T *const a = act + (k16 ? row16 : tok) * ld + Ops::kPer * quad;
 #pragma unroll
         for (int b = 0; b < NB; ++b) acc[b] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            const u32x4 bf = *reinterpret_cast<const u32x4 *>(act + tok * ld + Ops::kStep * ks + Ops::kPer * s4);
+        for (int k0 = 0; k0 < KS; k0 += KC) {
+            u32x4 bf[KC];
 #pragma unroll
-            for (int b = 0; b < NB; ++b) {
-                constexpr int R = S::kRing;
-                const int slot = (POS + ks * NB + b) % R;
-                acc[b] = Ops::mma(ring[slot], bf, acc[b]);
-                ring[slot] = *reinterpret_cast<const u32x4 *>(next);
-                next += 1024;
-            }
+            for (int k = 0; k < KC; ++k) bf[k] = *reinterpret_cast<const u32x4 *>(a + Ops::kStep * (k0 + k));
+#pragma unroll
+            for (int k = 0; k < KC; ++k)
+#pragma unroll
+                for (int b = 0; b < NB; ++b) {
+                    constexpr int R = S::kRing;
+                    const int slot = (POS + (k0 + k) * NB + b) % R;
+                    acc[b] = Ops::mma(ring[slot], bf[k], acc[b]);
+                    ring[slot] = *reinterpret_cast<const u32x4 *>(next);
+                    next += 1024;
+                }
             __builtin_amdgcn_sched_barrier(0);
         }
+#pragma unroll
+        for (int b = 0; b < NB; ++b) Ops::finish(acc[b]);
     };
     // LayerNorm of v (this lane's features of its token row) into dst
-    auto norm_store = [&](auto &v, const auto &gam, const auto &bet, float eps, T *dst) {
+    auto norm_store = [&](auto &v, const T *gam, const T *bet, float eps, T *dst) {
         constexpr int NB = sizeof(v) / sizeof(v[0]);
         constexpr float kLocal = NB * 16;
-        float sum = 0.f;
+        float s = 0.f;
 #pragma unroll
-        for (int b = 0; b < NB; ++b)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) sum += v[b][e];
-        sum += __shfl_xor(sum, 16, 64);
-        sum += __shfl_xor(sum, 32, 64);
-        const float lmean = sum * (1.f / kLocal);
+        for (int b = 0; b < NB; ++b) s += (v[b][0] + v[b][1]) + (v[b][2] + v[b][3]);
+        s = Ops::sum(s);
+        const float lmean = s * (1.f / kLocal);
         float q = 0.f;
 #pragma unroll
         for (int b = 0; b < NB; ++b)
@@ -258,283 +315,301 @@ __global__ __launch_bounds__(kTrajWaves * 64) void trajectory_decode_kernel(Traj
                 const float d = v[b][e] - lmean;
                 q += d * d;
             }
-        q += __shfl_xor(q, 16, 64);
-        q += __shfl_xor(q, 32, 64);
-        if (s4 == 0) {
-            red_a[wave * kTrajRows + tok] = lmean;
-            red_b[wave * kTrajRows + tok] = q;
+        q = Ops::sum(q);
+        if (lane < ROWS * (k16 ? 1 : 4) && sub == 0) {
+            red_a[wave * ROWS + tok] = lmean;
+            red_b[wave * ROWS + tok] = q;
+        }
+        float g[NB][4], be[NB][4];
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            traj_load4<T>(gam + 16 * (wave + NW * b) + 4 * sub, g[b]);
+            traj_load4<T>(bet + 16 * (wave + NW * b) + 4 * sub, be[b]);
         }
         __syncthreads();
-        float lm[NW], tot = 0.f;
+        float lm[NW], lq[NW], sum8[NW];
 #pragma unroll
         for (int w = 0; w < NW; ++w) {
-            lm[w] = red_a[w * kTrajRows + tok];
-            tot += lm[w];
+            lm[w] = red_a[w * ROWS + tok];
+            lq[w] = red_b[w * ROWS + tok];
         }
-        const float mean = tot * (1.f / NW);
-        float m2 = 0.f;
+        auto tree = [&](const float (&x)[NW]) { return ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7])); };
+        const float mean = tree(lm) * (1.f / NW);
 #pragma unroll
         for (int w = 0; w < NW; ++w) {
             const float d = lm[w] - mean;
-            m2 += red_b[w * kTrajRows + tok] + kLocal * d * d;
+            sum8[w] = fmaf(kLocal * d, d, lq[w]);
         }
-        const float rstd = rsqrtf(m2 / D + eps);
+        const float rstd = __builtin_amdgcn_rsqf(fmaf(tree(sum8), 1.f / D, eps));
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
-            float o[4], g[4], be[4];
-            gam.get(b, g);
-            bet.get(b, be);
+            float o[4];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) o[e] = (v[b][e] - mean) * rstd * g[e] + be[e];
-            traj_store4<T>(dst + tok * LD + 16 * (wave + NW * b) + 4 * s4, o);
+            for (int e = 0; e < 4; ++e) o[e] = (v[b][e] - mean) * rstd * g[b][e] + be[b][e];
+            traj_store4<T>(dst + tok * LD + 16 * (wave + NW * b) + 4 * sub, o);
         }
         __syncthreads();
     };
-    auto gelu = [](float t) { return 0.5f * t * (1.f + erff(t * 0.70710678118654752f)); };
-
-    // ---- attention of this wavefront's head(s): committed rows, then the rows of this step
-    const int part = wave / H;  // (only with NP > 1)
-    T *const vt = v_lds + (k16 ? wave * BK * VPAD : 0);
-    auto attention = [&](const T *kc, const T *vc, const T *ko, const T *vo, int t) {
-        const int n_own = P.own_base + (t > 0 ? t - 1 : 0);  // rows of a trajectory's cache
-        const int nb_ctx = (P.n_ctx + BK - 1) / BK, nb_own = (n_own + BK - 1) / BK;
-        const int n_blocks = nb_ctx + valid * nb_own;
-        for (int hh = 0; hh < HPW; ++hh) {
-            const int h = NP > 1 ? wave % H : wave + NW * hh;
-            u32x4 qf[k16 ? 1 : 2];
+    // gelu of this lane's 4 values of every block, stored to the hidden tile
+    auto gelu_store = [&](auto &acc, const T *bias) {
+        constexpr int NB = sizeof(acc) / sizeof(acc[0]);
 #pragma unroll
-            for (int x = 0; x < (k16 ? 1 : 2); ++x)
-                qf[x] = *reinterpret_cast<const u32x4 *>(qs + tok * LD + DH * h + Ops::kStep * x + Ops::kPer * s4);
-            f32x4 o_acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
-            float m_run = -1e30f, l_run = 0.f;
-            // one block of keys as it comes from memory: K in operand order; V as 16-byte pieces of the
-            // row-major tile (16-bit) or as the operand of the second product (float32)
-            struct Block {
-                u32x4 k[2];
-                u32x4 v[2];
-            };
-            // keys [row0, row0 + BK) of block i: where they start, how many there are, whose they are
-            auto locate = [&](int i, const T *&kp, const T *&vp, int &row0, int &n, int &g) {
-                if (i < nb_ctx) {
-                    g = -1;
-                    row0 = i * BK;
-                    n = P.n_ctx;
-                    const long at = static_cast<long>(h) * P.ctx_rows * DH;
-                    kp = kc + at;
-                    vp = vc + at;
-                } else {
-                    int j = i - nb_ctx;
-                    g = 0;
-                    while (j >= nb_own) {
-                        j -= nb_own;
-                        ++g;
-                    }
-                    row0 = j * BK;
-                    n = n_own;
-                    const long at = ((b0 + g) * H + h) * P.own_rows * DH;
-                    kp = ko + at;
-                    vp = vo + at;
-                }
-            };
-            auto fetch = [&](int i, Block &r) {
-                const T *kp, *vp;
-                int row0, n, g;
-                locate(i, kp, vp, row0, n, g);
-                if constexpr (k16) {
+        for (int b = 0; b < NB; ++b) {
+            const int col = 16 * (wave + NW * b) + 4 * sub;
+            float bi[4];
+            traj_load4<T>(bias + col, bi);
+            if constexpr (k16) {
+                float o[4];
 #pragma unroll
-                    for (int x = 0; x < 2; ++x)
-                        r.k[x] = *reinterpret_cast<const u32x4 *>(kp + static_cast<long>(min(row0 + 16 * x + tok, n - 1)) * DH + 8 * s4);
-#pragma unroll
-                    for (int x = 0; x < 2; ++x) {
-                        const int p = lane + 64 * x;
-                        r.v[x] = *reinterpret_cast<const u32x4 *>(vp + static_cast<long>(min(row0 + p / 4, n - 1)) * DH + 8 * (p % 4));
-                    }
-                } else {
-                    const T *kr = kp + static_cast<long>(min(row0 + tok, n - 1)) * DH + 4 * s4;
-#pragma unroll
-                    for (int x = 0; x < 2; ++x) r.k[x] = *reinterpret_cast<const u32x4 *>(kr + 16 * x);
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        const T *vr = vp + static_cast<long>(min(row0 + 4 * s4 + j, n - 1)) * DH + tok;
-                        r.v[0][j] = __builtin_bit_cast(unsigned, vr[0]);
-                        r.v[1][j] = __builtin_bit_cast(unsigned, vr[16]);
-                    }
-                }
-            };
-            // softmax bookkeeping of a block of scores (lane: keys 4 s + r of each 16-key half, its token)
-            auto fold = [&](auto &sc, auto &pb) {
-                constexpr int NX = sizeof(sc) / sizeof(sc[0]);
-                float tmax = sc[0][0];
-#pragma unroll
-                for (int x = 0; x < NX; ++x)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) tmax = fmaxf(tmax, sc[x][r]);
-                tmax = fmaxf(tmax, __shfl_xor(tmax, 16, 64));
-                tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
-                const float m_new = fmaxf(m_run, tmax);
-                const float alpha = fast_exp2(m_run - m_new);
-                if (__any(alpha != 1.f)) {
-                    l_run *= alpha;
-#pragma unroll
-                    for (int db = 0; db < 2; ++db)
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) o_acc[db][r] *= alpha;
-                }
-                m_run = m_new;
-#pragma unroll
-                for (int x = 0; x < NX; ++x)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const float p = fast_exp2(sc[x][r] - m_new);
-                        l_run += p;
-                        pb[x][r] = p;
-                    }
-            };
-            auto compute = [&](int i, const Block &r) {
-                const T *kp, *vp;
-                int row0, n, g;
-                locate(i, kp, vp, row0, n, g);
-                constexpr int NX = BK / 16;
-                f32x4 sc[NX];
-                if constexpr (k16) {
-#pragma unroll
-                    for (int x = 0; x < 2; ++x) {
-                        const int p = lane + 64 * x;
-                        *reinterpret_cast<u32x4 *>(vt + (p / 4) * VPAD + 8 * (p % 4)) = r.v[x];
-                    }
-#pragma unroll
-                    for (int x = 0; x < 2; ++x) sc[x] = Ops::mma(r.k[x], qf[0], f32x4{0.f, 0.f, 0.f, 0.f});
-                } else {
-                    sc[0] = Ops::mma(r.k[0], qf[0], f32x4{0.f, 0.f, 0.f, 0.f});
-                    sc[0] = Ops::mma(r.k[1], qf[1], sc[0]);
-                }
-                if (row0 + BK > n || g >= 0) {
-                    const bool mine = g < 0 || (tok >> 1) == g;
-#pragma unroll
-                    for (int x = 0; x < NX; ++x)
-#pragma unroll
-                        for (int e = 0; e < 4; ++e)
-                            if (!mine || row0 + 16 * x + 4 * s4 + e >= n) sc[x][e] = -INFINITY;
-                }
-                float pb[NX][4];
-                fold(sc, pb);
-                if constexpr (k16) {
-                    const u32x4 pv = {pack2<T>(pb[0][0], pb[0][1]), pack2<T>(pb[0][2], pb[0][3]),
-                                      pack2<T>(pb[1][0], pb[1][1]), pack2<T>(pb[1][2], pb[1][3])};
-                    __builtin_amdgcn_wave_barrier();
-#pragma unroll
-                    for (int db = 0; db < 2; ++db) {
-                        const T *a = vt + (4 * s4 + (tok >> 2)) * VPAD + 16 * db + 4 * (tok & 3);
-                        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4 *)(a));
-                        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4 *)(a + 16 * VPAD));
-                        typedef short s16x8 __attribute__((ext_vector_type(8)));
-                        const s16x8 both = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-                        o_acc[db] = Ops::mma(__builtin_bit_cast(u32x4, both), pv, o_acc[db]);
-                    }
-                    __builtin_amdgcn_wave_barrier();
-                } else {
-                    const u32x4 pv = {__builtin_bit_cast(unsigned, pb[0][0]), __builtin_bit_cast(unsigned, pb[0][1]),
-                                      __builtin_bit_cast(unsigned, pb[0][2]), __builtin_bit_cast(unsigned, pb[0][3])};
-#pragma unroll
-                    for (int db = 0; db < 2; ++db) o_acc[db] = Ops::mma(r.v[db], pv, o_acc[db]);
-                }
-            };
-            Block r0, r1, r2;
-            const int first = NP > 1 ? part : 0;
-            if (first < n_blocks) fetch(first, r0);
-            if (first + NP < n_blocks) fetch(first + NP, r1);
-            for (int i = first; i < n_blocks;) {
-                if (i + 2 * NP < n_blocks) fetch(i + 2 * NP, r2);
-                compute(i, r0);
-                if ((i += NP) >= n_blocks) break;
-                if (i + 2 * NP < n_blocks) fetch(i + 2 * NP, r0);
-                compute(i, r1);
-                if ((i += NP) >= n_blocks) break;
-                if (i + 2 * NP < n_blocks) fetch(i + 2 * NP, r1);
-                compute(i, r2);
-                i += NP;
-            }
-            if (t > 0 && (NP == 1 || part == 0)) {  // the buffer rows of this step
-                f32x4 sc[1];
-                if constexpr (k16) {
-                    const u32x4 kf = *reinterpret_cast<const u32x4 *>(kn + tok * LD + DH * h + 8 * s4);
-                    sc[0] = Ops::mma(kf, qf[0], f32x4{0.f, 0.f, 0.f, 0.f});
-                } else {
-                    const T *kr = kn + tok * LD + DH * h + 4 * s4;
-                    sc[0] = Ops::mma(*reinterpret_cast<const u32x4 *>(kr), qf[0], f32x4{0.f, 0.f, 0.f, 0.f});
-                    sc[0] = Ops::mma(*reinterpret_cast<const u32x4 *>(kr + 16), qf[1], sc[0]);
-                }
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    if (4 * s4 + e != (tok & ~1)) sc[0][e] = -INFINITY;
-                float pb[1][4];
-                fold(sc, pb);
-                if constexpr (k16) {
-                    const u32x4 pv = {pack2<T>(pb[0][0], pb[0][1]), pack2<T>(pb[0][2], pb[0][3]), 0u, 0u};
-#pragma unroll
-                    for (int db = 0; db < 2; ++db) {
-                        const T *a = vn + (4 * s4 + (tok >> 2)) * LD + DH * h + 16 * db + 4 * (tok & 3);
-                        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4 *)(a));
-                        typedef short s16x8 __attribute__((ext_vector_type(8)));
-                        const s16x8 both = {lo[0], lo[1], lo[2], lo[3], 0, 0, 0, 0};
-                        o_acc[db] = Ops::mma(__builtin_bit_cast(u32x4, both), pv, o_acc[db]);
-                    }
-                } else {
-#pragma unroll
-                    for (int db = 0; db < 2; ++db) {
-                        u32x4 vf, pv;
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) {
-                            vf[j] = __builtin_bit_cast(unsigned, vn[(4 * s4 + j) * LD + DH * h + 16 * db + tok]);
-                            pv[j] = __builtin_bit_cast(unsigned, pb[0][j]);
-                        }
-                        o_acc[db] = Ops::mma(vf, pv, o_acc[db]);
-                    }
-                }
-            }
-            float l_tot = l_run + __shfl_xor(l_run, 16, 64);
-            l_tot += __shfl_xor(l_tot, 32, 64);
-            if constexpr (NP > 1) {  // the other wavefronts' keys of this head
-                if (part > 0) {
-                    if (s4 == 0) {
-                        part_m[wave * kTrajRows + tok] = m_run;
-                        part_l[wave * kTrajRows + tok] = l_tot;
-                    }
-#pragma unroll
-                    for (int db = 0; db < 2; ++db)
-                        *reinterpret_cast<f32x4 *>(part_o + (wave * kTrajRows + tok) * DH + 16 * db + 4 * s4) = o_acc[db];
-                }
-                __syncthreads();
-                if (part == 0) {
-#pragma unroll
-                    for (int p = 1; p < NP; ++p) {
-                        const int w = wave + p * H;
-                        const float m2 = part_m[w * kTrajRows + tok], l2 = part_l[w * kTrajRows + tok];
-                        const float m_new = fmaxf(m_run, m2);
-                        const float a1 = fast_exp2(m_run - m_new), a2 = fast_exp2(m2 - m_new);
-#pragma unroll
-                        for (int db = 0; db < 2; ++db) {
-                            const f32x4 o2 = *reinterpret_cast<const f32x4 *>(part_o + (w * kTrajRows + tok) * DH + 16 * db + 4 * s4);
-#pragma unroll
-                            for (int e = 0; e < 4; ++e) o_acc[db][e] = o_acc[db][e] * a1 + o2[e] * a2;
-                        }
-                        l_tot = l_tot * a1 + l2 * a2;
-                        m_run = m_new;
-                    }
-                }
-            }
-            if (NP == 1 || part == 0) {
-                const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-#pragma unroll
-                for (int db = 0; db < 2; ++db) {
-                    const float o[4] = {o_acc[db][0] * inv, o_acc[db][1] * inv, o_acc[db][2] * inv, o_acc[db][3] * inv};
-                    traj_store4<T>(xs + tok * LD + DH * h + 16 * db + 4 * s4, o);
-                }
+                for (int e = 0; e < 4; ++e) o[e] = traj_gelu16(acc[b][e] + bi[e]);
+                traj_store4<T>(hs + tok * LF + col, o);
+            } else {  // the four rows of lanes hold the same values: each does one of them
+                const float a = acc[b][0] + bi[0], c = acc[b][1] + bi[1], d = acc[b][2] + bi[2], f = acc[b][3] + bi[3];
+                const float x = quad == 0 ? a : quad == 1 ? c : quad == 2 ? d : f;
+                hs[tok * LF + col + quad] = 0.5f * x * (1.f + erff(x * 0.70710678118654752f));
             }
         }
     };
 
-    // ---- embedding of step 0: target rows; every other row is zero
+    // ---- attention of this wavefront's head(s): committed rows, then the rows of this step
+    const int part = wave / H;  // (only with NP > 1)
+    const int head0 = NP > 1 ? wave % H : wave;
+    T *const vt = v_lds + (k16 ? wave * BK * VPAD : 0);
+    // One block of keys as it comes from memory: K in operand order; V as 16-byte pieces of the
+    // row-major tile (16-bit) or as the operand of the second product (float32); which rows they are.
+    struct Block {
+        u32x4 k[2], v[2];
+        int row0, n, g;
+    };
+    // The layer's caches, as addresses in global memory: made from integers, plain pointers would be
+    // generic ones, whose loads count as LDS accesses too — every wait for LDS would wait for the keys.
+    typedef __attribute__((address_space(1))) char *Global;
+    Global kv[4];
+    // Blocks by number: the context's, then trajectory 0's, 1's, ... (the division of the number by
+    // the blocks of a trajectory as a multiplication: a loop here costs more than the block's loads)
+    int n_own = 0, nb_ctx = (P.n_ctx + BK - 1) / BK, nb_own = 0, n_blocks = 0;
+    unsigned own_inv = 0;
+    auto set_step = [&](int t) {
+        n_own = P.own_base + (t > 0 ? t - 1 : 0);
+        nb_own = (n_own + BK - 1) / BK;
+        own_inv = nb_own > 1 ? 0xffffffffu / static_cast<unsigned>(nb_own) + 1 : 0;
+        n_blocks = nb_ctx + valid * nb_own;
+    };
+    // (rows past a segment's end re-read its last one)
+    auto fetch = [&](int h, int i, Block &r) {
+        if (i >= n_blocks) return;
+        const int j = i - nb_ctx;
+        const int of = nb_own > 1 ? static_cast<int>(__umulhi(static_cast<unsigned>(j), own_inv)) : j;
+        const int g = j < 0 ? -1 : of, row0 = BK * (j < 0 ? i : j - of * nb_own);
+        r.row0 = row0;
+        r.n = g < 0 ? P.n_ctx : n_own;
+        r.g = g;
+        const int last = r.n - 1;
+        const long at = (g < 0 ? static_cast<long>(h) * P.ctx_rows : ((b0 + g) * H + h) * P.own_rows) * DH;
+        const Global kp = kv[g < 0 ? 0 : 2] + at * static_cast<long>(sizeof(T)), vp = kv[g < 0 ? 1 : 3] + at * static_cast<long>(sizeof(T));
+        typedef const __attribute__((address_space(1))) u32x4 *Global16;
+        constexpr unsigned RB = DH * sizeof(T);  // bytes of a row
+        if constexpr (k16) {
+#pragma unroll
+            for (int x = 0; x < 2; ++x)
+                r.k[x] = *(Global16)(kp + (static_cast<unsigned>(min(row0 + 16 * x + row16, last)) * RB + 16 * quad));
+#pragma unroll
+            for (int x = 0; x < 2; ++x)
+                r.v[x] = *(Global16)(vp + (static_cast<unsigned>(min(row0 + 16 * x + lane / 4, last)) * RB + 16 * (lane % 4)));
+        } else {
+            const Global kr = kp + (static_cast<unsigned>(min(row0 + row16, last)) * RB + 16 * quad);
+            r.k[0] = *(Global16)kr;
+            r.k[1] = *(Global16)(kr + 64);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const __attribute__((address_space(1))) unsigned *vr =
+                    (const __attribute__((address_space(1))) unsigned *)(vp + (static_cast<unsigned>(min(row0 + 4 * quad + j, last)) * RB + 4 * row16));
+                r.v[0][j] = vr[0];
+                r.v[1][j] = vr[16];
+            }
+        }
+    };
+    Block r0, r1;
+    const int first_block = NP > 1 ? part : 0;  // the wavefront's blocks: this one and every NP-th
+    auto first_blocks = [&](int h) {
+        fetch(h, first_block, r0);
+        fetch(h, first_block + NP, r1);
+    };
+    auto attention = [&](int h, int t) {
+        u32x4 qf[k16 ? 1 : 2];
+#pragma unroll
+        for (int x = 0; x < (k16 ? 1 : 2); ++x)
+            qf[x] = *reinterpret_cast<const u32x4 *>(qs + (k16 ? row16 : tok) * LD + DH * h + Ops::kStep * x + Ops::kPer * quad);
+        f32x4 o_acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+        float m_run = -1e30f, l_run = 0.f;
+        // Scores (lane: keys 4 sub + r of each 16-key part, its token) to probabilities.
+        auto fold = [&](auto &sc) {
+            constexpr int NX = sizeof(sc) / sizeof(sc[0]);
+            float tmax = sc[0][0];
+#pragma unroll
+            for (int x = 0; x < NX; ++x)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) tmax = fmaxf(tmax, sc[x][r]);
+            if (__any(tmax > m_run + Ops::kSlack)) {
+                const float m_new = fmaxf(m_run, Ops::max(tmax));
+                const float alpha = fast_exp2(m_run - m_new);
+                l_run *= alpha;
+#pragma unroll
+                for (int db = 0; db < 2; ++db)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) o_acc[db][r] *= alpha;
+                m_run = m_new;
+            }
+#pragma unroll
+            for (int x = 0; x < NX; ++x) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) sc[x][r] = fast_exp2(sc[x][r] - m_run);
+                l_run += (sc[x][0] + sc[x][1]) + (sc[x][2] + sc[x][3]);
+            }
+        };
+        typedef short s16x8 __attribute__((ext_vector_type(8)));
+        auto tr_read = [](const T *a) {
+            return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4 *)(a));
+        };
+        // float32: the probabilities of keys 4 (lane / 16) + j for this lane's token
+        const int p_from = ((lane & 48) | (quad << 2) | (lane & 3)) << 2;
+        auto p_operand = [&](const f32x4 &p) {
+            u32x4 r;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const float pj = p[j];
+                r[j] = __builtin_amdgcn_ds_bpermute(p_from, __builtin_bit_cast(int, pj));
+            }
+            return r;
+        };
+        auto compute = [&](Block &r, int i) {  // block i; the wavefront's block after next goes where this one was
+            constexpr int NX = BK / 16;
+            const int row0 = r.row0, n = r.n, g = r.g;
+            f32x4 sc[NX];
+            if constexpr (k16) {
+#pragma unroll
+                for (int x = 0; x < 2; ++x)
+                    *reinterpret_cast<u32x4 *>(vt + (16 * x + lane / 4) * VPAD + 8 * (lane % 4)) = r.v[x];
+#pragma unroll
+                for (int x = 0; x < NX; ++x) sc[x] = Ops::mma(r.k[x], qf[0], f32x4{0.f, 0.f, 0.f, 0.f});
+                fetch(h, i + 2 * NP, r);
+            } else {
+                sc[0] = Ops::mma(r.k[0], qf[0], f32x4{0.f, 0.f, 0.f, 0.f});
+                sc[0] = Ops::mma(r.k[1], qf[1], sc[0]);
+                Ops::finish(sc[0]);
+            }
+            if (row0 + BK > n || (g >= 0 && valid > 1)) {
+                // (with one trajectory the other columns are nobody's)
+                const bool mine = g < 0 || valid == 1 || (tok >> 1) == g;
+#pragma unroll
+                for (int x = 0; x < NX; ++x)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        if (!mine || row0 + 16 * x + 4 * sub + e >= n) sc[x][e] = -INFINITY;
+            }
+            fold(sc);
+            if constexpr (k16) {
+                __builtin_amdgcn_wave_barrier();
+                const u32x4 pv = {pack2<T>(sc[0][0], sc[0][1]), pack2<T>(sc[0][2], sc[0][3]),
+                                  pack2<T>(sc[1][0], sc[1][1]), pack2<T>(sc[1][2], sc[1][3])};
+#pragma unroll
+                for (int db = 0; db < 2; ++db) {
+                    const T *a = vt + (4 * quad + (row16 >> 2)) * VPAD + 16 * db + 4 * (lane & 3);
+                    const s16x4 lo = tr_read(a), hi = tr_read(a + 16 * VPAD);
+                    const s16x8 both = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+                    o_acc[db] = Ops::mma(__builtin_bit_cast(u32x4, both), pv, o_acc[db]);
+                }
+                __builtin_amdgcn_wave_barrier();
+            } else {
+                const u32x4 pv = p_operand(sc[0]);
+#pragma unroll
+                for (int db = 0; db < 2; ++db) o_acc[db] = Ops::mma(r.v[db], pv, o_acc[db]);
+                fetch(h, i + 2 * NP, r);
+            }
+        };
+        for (int i = first_block; i < n_blocks; i += 2 * NP) {
+            compute(r0, i);
+            if (i + NP < n_blocks) compute(r1, i + NP);
+        }
+        if (t > 0 && (NP == 1 || part == 0)) {  // the buffer rows of this step
+            f32x4 sc[1];
+            const T *const kr = kn + (k16 ? row16 : lane & 3) * LD + DH * h + Ops::kPer * quad;
+            sc[0] = Ops::mma(*reinterpret_cast<const u32x4 *>(kr), qf[0], f32x4{0.f, 0.f, 0.f, 0.f});
+            if constexpr (!k16) {
+                sc[0] = Ops::mma(*reinterpret_cast<const u32x4 *>(kr + 16), qf[1], sc[0]);
+                Ops::finish(sc[0]);
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (4 * sub + e != (tok & ~1)) sc[0][e] = -INFINITY;
+            fold(sc);
+            if constexpr (k16) {
+                const u32x4 pv = {pack2<T>(sc[0][0], sc[0][1]), pack2<T>(sc[0][2], sc[0][3]), 0u, 0u};
+#pragma unroll
+                for (int db = 0; db < 2; ++db) {
+                    const s16x4 lo = tr_read(vn + (4 * quad + (row16 >> 2)) * LD + DH * h + 16 * db + 4 * (lane & 3));
+                    const s16x8 both = {lo[0], lo[1], lo[2], lo[3], 0, 0, 0, 0};
+                    o_acc[db] = Ops::mma(__builtin_bit_cast(u32x4, both), pv, o_acc[db]);
+                }
+            } else {
+                const u32x4 pv = p_operand(sc[0]);
+#pragma unroll
+                for (int db = 0; db < 2; ++db) {
+                    u32x4 vf;  // (rows past the fourth do not exist: their probabilities are zero)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) vf[j] = __builtin_bit_cast(unsigned, vn[j * LD + DH * h + 16 * db + row16]);
+                    o_acc[db] = Ops::mma(vf, pv, o_acc[db]);
+                }
+            }
+        }
+        float l_tot = Ops::sum(l_run);
+#pragma unroll
+        for (int db = 0; db < 2; ++db) Ops::finish(o_acc[db]);
+        if constexpr (NP > 1) {  // the other wavefronts' keys of this head
+            if (part > 0) {
+                if (sub == 0) {
+                    part_m[wave * ROWS + tok] = m_run;
+                    part_l[wave * ROWS + tok] = l_tot;
+                }
+#pragma unroll
+                for (int db = 0; db < 2; ++db)
+                    *reinterpret_cast<f32x4 *>(part_o + (wave * ROWS + tok) * DH + 16 * db + 4 * sub) = o_acc[db];
+            }
+            __syncthreads();
+            if (part == 0) {
+#pragma unroll
+                for (int p = 1; p < NP; ++p) {
+                    const int w = wave + p * H;
+                    const float m2 = part_m[w * ROWS + tok], l2 = part_l[w * ROWS + tok];
+                    const float m_new = fmaxf(m_run, m2);
+                    const float a1 = fast_exp2(m_run - m_new), a2 = fast_exp2(m2 - m_new);
+#pragma unroll
+                    for (int db = 0; db < 2; ++db) {
+                        const f32x4 o2 = *reinterpret_cast<const f32x4 *>(part_o + (w * ROWS + tok) * DH + 16 * db + 4 * sub);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) o_acc[db][e] = o_acc[db][e] * a1 + o2[e] * a2;
+                    }
+                    l_tot = l_tot * a1 + l2 * a2;
+                    m_run = m_new;
+                }
+            }
+        }
+        if (NP == 1 || part == 0) {
+            const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
+#pragma unroll
+            for (int db = 0; db < 2; ++db) {
+                const float o[4] = {o_acc[db][0] * inv, o_acc[db][1] * inv, o_acc[db][2] * inv, o_acc[db][3] * inv};
+                traj_store4<T>(xs + tok * LD + DH * h + 16 * db + 4 * sub, o);
+            }
+        }
+    };
+
+    // ---- constants, the first layer's vectors, the embedding of step 0: target rows; every other row is zero
+    constexpr int kPieces = 8 * VW * static_cast<int>(sizeof(T)) / 16;  // of a layer's vectors
+    static_assert(kPieces <= NT, "one piece per thread");
+    const u32x4 *const vec_src = static_cast<const u32x4 *>(P.vecs);
+    if (tid < kPieces) reinterpret_cast<u32x4 *>(pbuf[0])[tid] = vec_src[tid];
+    for (int i = tid; i < 4 * P.n_layers; i += NT) kv_s[i] = P.kv[i];
     const T *const xm = static_cast<const T *>(P.x_mean);
     for (int d = tid; d < D; d += NT) {
         c_ng[d] = static_cast<const T *>(P.norm_g)[d];
@@ -550,7 +625,7 @@ __global__ __launch_bounds__(kTrajWaves * 64) void trajectory_decode_kernel(Traj
     if (tid < kTrajHeadOut) c_b2[tid] = static_cast<const T *>(P.b_h2)[tid];
     if (tid < 3 * P.K) c_mix[tid] = static_cast<const T *>(P.mix)[tid];
     __syncthreads();
-    for (int i = tid; i < kTrajRows * D; i += NT) {
+    for (int i = tid; i < ROWS * D; i += NT) {
         const int r = i / D, d = i % D, g = r >> 1;
         float v = 0.f;
         if ((r & 1) && g < valid) v = to_f32(xm[(b0 + g) * P.Nt]) * to_f32(c_wx[d]) + to_f32(c_bx[d]) + to_f32(c_mt[d]);
@@ -559,8 +634,10 @@ __global__ __launch_bounds__(kTrajWaves * 64) void trajectory_decode_kernel(Traj
     __syncthreads();
 
     using std::integral_constant;
+    int pp = 0;  // which of the two vector buffers holds this layer's
     for (int t = 0; t < P.Nt; ++t) {
         const bool last_step = t + 1 == P.Nt;
+        set_step(t);
         // the variates and feature means of the step's draw, long before they are needed
         float my_u = 0.f, my_n = 0.f;
         T my_x = from_f32<T>(0.f), my_tok = my_x;
@@ -572,21 +649,16 @@ __global__ __launch_bounds__(kTrajWaves * 64) void trajectory_decode_kernel(Traj
         if (tid < 2 * valid && !last_step) my_x = xm[(b0 + (tid >> 1)) * P.Nt + t + (tid & 1)];
         if (tid < D) my_tok = static_cast<const T *>(P.ar_tokens)[static_cast<long>((t + 1) % P.bs) * D + tid];
         for (int l = 0; l < P.n_layers; ++l) {
-            // the layer's parameter vectors and cache addresses are requested ahead of everything
-            const T *vec = static_cast<const T *>(P.vecs) + static_cast<long>(l) * 8 * VW;
-            TrajCols<T, S::ND> g1, be1, g2, be2, g3, be3, bias2;
-            TrajCols<T, S::NF> bias1;
-            g1.load(vec, wave, s4);
-            be1.load(vec + VW, wave, s4);
-            g2.load(vec + 2 * VW, wave, s4);
-            be2.load(vec + 3 * VW, wave, s4);
-            bias1.load(vec + 4 * VW, wave, s4);
-            g3.load(vec + 5 * VW, wave, s4);
-            be3.load(vec + 6 * VW, wave, s4);
-            bias2.load(vec + 7 * VW, wave, s4);
-            unsigned long long kv_raw[4];
+            const T *const vec = pbuf[pp];
+            u32x4 next_vec = {0u, 0u, 0u, 0u};
+            if (tid < kPieces) next_vec = vec_src[(l + 1 < P.n_layers ? l + 1 : 0) * kPieces + tid];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) kv_raw[i] = P.kv[4 * l + i];
+            for (int i = 0; i < 4; ++i) {
+                const unsigned long long raw = kv_s[4 * l + i];
+                const unsigned lo = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(raw)),
+                               hi = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(raw >> 32));
+                kv[i] = (Global)(static_cast<unsigned long long>(hi) << 32 | lo);
+            }
             {   // y = LN1(x + x W_fo^T)
                 f32x4 acc[S::ND];
                 product(integral_constant<int, 0>{}, integral_constant<int, S::KD>{}, acc, xs, LD);
@@ -594,12 +666,13 @@ __global__ __launch_bounds__(kTrajWaves * 64) void trajectory_decode_kernel(Traj
 #pragma unroll
                 for (int b = 0; b < S::ND; ++b) {
                     float r[4];
-                    traj_load4<T>(xs + tok * LD + 16 * (wave + NW * b) + 4 * s4, r);
+                    traj_load4<T>(xs + tok * LD + 16 * (wave + NW * b) + 4 * sub, r);
 #pragma unroll
                     for (int e = 0; e < 4; ++e) v[b][e] = acc[b][e] + r[e];
                 }
-                norm_store(v, g1, be1, P.eps1, ys);
+                norm_store(v, vec, vec + VW, P.eps1, ys);
             }
+            first_blocks(head0);
             {   // q, k, v
                 f32x4 acc[3 * S::ND];
                 product(integral_constant<int, S::kFo>{}, integral_constant<int, S::KD>{}, acc, ys, LD);
@@ -613,31 +686,31 @@ __global__ __launch_bounds__(kTrajWaves * 64) void trajectory_decode_kernel(Traj
                             o[e] = acc[p * S::ND + b][e];
                             if (p == 0) o[e] = to_f32(from_f32<T>(o[e])) * P.qscale;
                         }
-                        traj_store4<T>(qkv + p * kTrajRows * LD + tok * LD + 16 * (wave + NW * b) + 4 * s4, o);
+                        traj_store4<T>(qkv + p * ROWS * LD + tok * LD + 16 * (wave + NW * b) + 4 * sub, o);
                     }
                 __syncthreads();
             }
-            T *kv[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const unsigned lo = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(kv_raw[i])),
-                               hi = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(kv_raw[i] >> 32));
-                kv[i] = reinterpret_cast<T *>(static_cast<unsigned long long>(hi) << 32 | lo);
-            }
-            // the caches: row 2 g is committed at slot t - 1 of trajectory g (its first read is a step away)
+            // the caches: row 2 g is committed at slot t - 1 of trajectory g (its first read is a step
+            // away); behind the last one the target row, where the caller keeps it
             {
                 constexpr int CPR = DH * sizeof(T) / 16, PER = H * CPR;  // 16-byte pieces of a head's row, of a row
-                const int rows = P.park_target && last_step ? 2 : 1;
-                for (int i = tid; i < valid * rows * 2 * PER; i += NT) {
-                    const int c = i % PER, which = i / PER & 1, rr = i / (2 * PER), g = rr / rows, target = rr % rows;
-                    const int slot = P.own_base + t - 1 + target;
-                    if (!target && t == 0) continue;
-                    T *dst = (which ? kv[3] : kv[2]) + (((b0 + g) * H + c / CPR) * P.own_rows + slot) * DH + (c % CPR) * (16 / sizeof(T));
-                    const T *src = (which ? vn : kn) + (2 * g + target) * LD + c * (16 / sizeof(T));
-                    *reinterpret_cast<u32x4 *>(dst) = *reinterpret_cast<const u32x4 *>(src);
-                }
+                auto commit = [&](int from, int slot) {
+                    for (int i = tid; i < valid * 2 * PER; i += NT) {
+                        const int c = i % PER, which = i / PER & 1, g = i / (2 * PER);
+                        const Global dst = (which ? kv[3] : kv[2]) + (((b0 + g) * H + c / CPR) * P.own_rows + slot) * static_cast<long>(DH * sizeof(T)) + 16 * (c % CPR);
+                        *(__attribute__((address_space(1))) u32x4 *)dst =
+                            *reinterpret_cast<const u32x4 *>((which ? vn : kn) + (2 * g + from) * LD + c * (16 / sizeof(T)));
+                    }
+                };
+                if (t > 0) commit(0, P.own_base + t - 1);
+                if (P.park_target && last_step) commit(1, P.own_base + t);
             }
-            attention(kv[0], kv[1], kv[2], kv[3], t);
+            attention(head0, t);
+#pragma unroll
+            for (int hh = 1; hh < HPW; ++hh) {
+                first_blocks(head0 + NW * hh);
+                attention(head0 + NW * hh, t);
+            }
             __syncthreads();
             {   // x1 = LN2(y + attn W_o^T)
                 f32x4 acc[S::ND];
@@ -646,23 +719,17 @@ __global__ __launch_bounds__(kTrajWaves * 64) void trajectory_decode_kernel(Traj
 #pragma unroll
                 for (int b = 0; b < S::ND; ++b) {
                     float r[4];
-                    traj_load4<T>(ys + tok * LD + 16 * (wave + NW * b) + 4 * s4, r);
+                    traj_load4<T>(ys + tok * LD + 16 * (wave + NW * b) + 4 * sub, r);
 #pragma unroll
                     for (int e = 0; e < 4; ++e) v[b][e] = acc[b][e] + r[e];
                 }
-                norm_store(v, g2, be2, P.eps2, ys);
+                norm_store(v, vec + 2 * VW, vec + 3 * VW, P.eps2, ys);
             }
             {   // h = gelu(x1 W_1^T + b_1)
                 f32x4 acc[S::NF];
                 product(integral_constant<int, S::kFo + S::kQkv + S::kO>{}, integral_constant<int, S::KD>{}, acc, ys, LD);
-#pragma unroll
-                for (int b = 0; b < S::NF; ++b) {
-                    float o[4], bias[4];
-                    bias1.get(b, bias);
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) o[e] = gelu(acc[b][e] + bias[e]);
-                    traj_store4<T>(hs + tok * LF + 16 * (wave + NW * b) + 4 * s4, o);
-                }
+                gelu_store(acc, vec + 4 * VW);
+                if (tid < kPieces) reinterpret_cast<u32x4 *>(pbuf[pp ^ 1])[tid] = next_vec;
                 __syncthreads();
             }
             {   // x = LN3(x1 + h W_2^T + b_2)
@@ -672,25 +739,20 @@ __global__ __launch_bounds__(kTrajWaves * 64) void trajectory_decode_kernel(Traj
 #pragma unroll
                 for (int b = 0; b < S::ND; ++b) {
                     float r[4], bias[4];
-                    bias2.get(b, bias);
-                    traj_load4<T>(ys + tok * LD + 16 * (wave + NW * b) + 4 * s4, r);
+                    traj_load4<T>(vec + 7 * VW + 16 * (wave + NW * b) + 4 * sub, bias);
+                    traj_load4<T>(ys + tok * LD + 16 * (wave + NW * b) + 4 * sub, r);
 #pragma unroll
                     for (int e = 0; e < 4; ++e) v[b][e] = acc[b][e] + r[e] + bias[e];
                 }
-                norm_store(v, g3, be3, P.eps3, xs);
+                norm_store(v, vec + 5 * VW, vec + 6 * VW, P.eps3, xs);
             }
+            pp ^= 1;
         }
 
         // ---- the head on the target rows, one draw per trajectory, the rows of the next step
         {
             constexpr int EPL = D / 64;
-            float gam[EPL], bet[EPL];
-#pragma unroll
-            for (int e = 0; e < EPL; ++e) {
-                gam[e] = to_f32(c_ng[lane * EPL + e]);
-                bet[e] = to_f32(c_nb[lane * EPL + e]);
-            }
-            for (int r = wave; r < kTrajRows; r += NW) {
+            for (int r = wave; r < ROWS; r += NW) {
                 const T *row = xs + r * LD + lane * EPL;
                 float x[EPL], sum = 0.f;
 #pragma unroll
@@ -704,21 +766,16 @@ __global__ __launch_bounds__(kTrajWaves * 64) void trajectory_decode_kernel(Traj
                 for (int e = 0; e < EPL; ++e) q += (x[e] - mean) * (x[e] - mean);
                 const float rstd = rsqrtf(wave_sum(q) / D + P.eps_out);
 #pragma unroll
-                for (int e = 0; e < EPL; ++e) ys[r * LD + lane * EPL + e] = from_f32<T>((x[e] - mean) * rstd * gam[e] + bet[e]);
+                for (int e = 0; e < EPL; ++e)
+                    ys[r * LD + lane * EPL + e] =
+                        from_f32<T>((x[e] - mean) * rstd * to_f32(c_ng[lane * EPL + e]) + to_f32(c_nb[lane * EPL + e]));
             }
             __syncthreads();
         }
         {
             f32x4 acc[S::NF];
             product(integral_constant<int, 0>{}, integral_constant<int, S::KD>{}, acc, ys, LD);
-#pragma unroll
-            for (int b = 0; b < S::NF; ++b) {
-                float o[4], bias[4];
-                traj_load4<T>(c_b1 + 16 * (wave + NW * b) + 4 * s4, bias);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) o[e] = gelu(acc[b][e] + bias[e]);
-                traj_store4<T>(hs + tok * LF + 16 * (wave + NW * b) + 4 * s4, o);
-            }
+            gelu_store(acc, c_b1);
             __syncthreads();
         }
         {
@@ -726,9 +783,9 @@ __global__ __launch_bounds__(kTrajWaves * 64) void trajectory_decode_kernel(Traj
             product(integral_constant<int, S::kH1>{}, integral_constant<int, S::KF>{}, acc, hs, LF);
             if (16 * wave < kTrajHeadOut) {
                 float bias[4];
-                traj_load4<T>(c_b2 + 16 * wave + 4 * s4, bias);
+                traj_load4<T>(c_b2 + 16 * wave + 4 * sub, bias);
 #pragma unroll
-                for (int e = 0; e < 4; ++e) raw_s[tok][16 * wave + 4 * s4 + e] = acc[0][e] + bias[e];
+                for (int e = 0; e < 4; ++e) raw_s[tok][16 * wave + 4 * sub + e] = acc[0][e] + bias[e];
             }
             // fragments that only fill the head's part of the tape up to a whole number of rings
 #pragma unroll

@@ -41,11 +41,13 @@ bool with_shape(int D, int F, Fn f) {
 template <typename T>
 TrajectoryTapeLayout tape_layout(int D, int F, int n_layers) {
     TrajectoryTapeLayout t{};
+    if (n_layers > kTrajMaxLayers) return t;
     with_shape<T>(D, F, [&](auto d, auto f) {
         typedef TrajShape<T, decltype(d)::value, decltype(f)::value> S;
         t.layer = S::kLayer;
         t.head = S::kHead;
         t.ring = S::kRing;
+        t.max_group = TrajOps<T>::kMax;
         t.stride = (static_cast<long>(n_layers) * S::kLayer + S::kHead + S::kRing) * 1024;
         // first fragment, fragments per contraction step, blocks per wavefront of every matrix
         t.fo = {0, S::ND, 0, S::ND};
