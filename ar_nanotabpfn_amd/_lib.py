@@ -93,6 +93,27 @@ class ArtabTrajectoryArgs(ctypes.Structure):
     ]
 
 
+class ArtabTrainArgs(ctypes.Structure):
+    """``artab_train_args`` of include/artab_attention.h, field for field."""
+
+    _fields_ = [
+        *((n, _i) for n in ("B", "R", "H", "D", "F", "n_layers", "context_len", "buffer_len", "attending_chunks", "first_row")),
+        ("eps1", _f), ("eps2", _f), ("eps3", _f), ("eps_out", _f),
+        ("x", _p), ("params", _p), ("norm_gamma", _p), ("norm_beta", _p), ("saved", _p), ("z", _p),
+        ("dz", _p), ("dx", _p), ("grads", _p), ("scratch", _p),
+    ]
+
+
+class ArtabTrainEmbedArgs(ctypes.Structure):
+    """``artab_train_embed_args`` of include/artab_attention.h, field for field."""
+
+    _fields_ = [
+        *((n, _i) for n in ("B", "n_context", "n_buffer", "n_target", "feat", "D")),
+        *((n, _p) for n in ("x_context", "y_context", "x_buffer", "y_buffer", "x_target", "w_x", "b_x", "w_y", "b_y", "markers",
+                            "tokens", "out", "xy", "grads", "scratch")),
+    ]
+
+
 TAPE_FO, TAPE_QKV, TAPE_O, TAPE_1, TAPE_2, TAPE_H1, TAPE_H2, TAPE_CLOSE = range(8)
 
 # name -> (restype, argtypes); every symbol declared in include/artab_attention.h
@@ -156,6 +177,13 @@ SIGNATURES = {
         [ctypes.POINTER(ArtabAttentionPartials), _p, _i64, _p, _i64, _p, _p, _p, _f, _p, _p, _p, _p, _p, _p, _f,
          ctypes.POINTER(ArtabSampleEmbedArgs), _p, _p, _p, _f, _p, _p, _p, _i, _i, _p],
     ),
+    "artab_train_saved_bytes": (_sz, [ctypes.POINTER(ArtabTrainArgs)]),
+    "artab_train_scratch_bytes": (_sz, [ctypes.POINTER(ArtabTrainArgs)]),
+    "artab_train_forward": (_i, [ctypes.POINTER(ArtabTrainArgs), _p]),
+    "artab_train_backward": (_i, [ctypes.POINTER(ArtabTrainArgs), _p]),
+    "artab_train_embed_scratch_bytes": (_sz, [ctypes.POINTER(ArtabTrainEmbedArgs)]),
+    "artab_train_embed": (_i, [ctypes.POINTER(ArtabTrainEmbedArgs), _p]),
+    "artab_train_embed_backward": (_i, [ctypes.POINTER(ArtabTrainEmbedArgs), _p]),
     "artab_trajectory_group": (_i, [_i, _i, _i, _i, _i, _i, _i, _i]),
     "artab_trajectory_tape_bytes": (_sz, [_i, _i, _i, _i]),
     "artab_trajectory_pack": (_i, [_p, _p, _i, _i, _i, _i, _i, _i, _i, _p]),

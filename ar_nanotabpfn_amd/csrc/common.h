@@ -113,6 +113,32 @@ __device__ __forceinline__ float wave_sum(float x) {
     return x;
 }
 
+// Exchanges between the four rows of 16 lanes (gfx950 swaps: vector instructions, no LDS).  (Elements
+// of a vector are copied to scalars before they are reinterpreted: __builtin_bit_cast of a vector's
+// element reads element 0.)
+template <typename Op>
+__device__ __forceinline__ float over_rows(float x, Op op) {
+    const unsigned a = __builtin_bit_cast(unsigned, x);
+    auto s = __builtin_amdgcn_permlane32_swap(a, a, false, false);
+    unsigned lo = s[0], hi = s[1];
+    const unsigned b = __builtin_bit_cast(unsigned, op(__builtin_bit_cast(float, lo), __builtin_bit_cast(float, hi)));
+    s = __builtin_amdgcn_permlane16_swap(b, b, false, false);
+    lo = s[0];
+    hi = s[1];
+    return op(__builtin_bit_cast(float, lo), __builtin_bit_cast(float, hi));
+}
+__device__ __forceinline__ float row_sum(float x) {
+    return over_rows(x, [](float a, float b) { return a + b; });
+}
+__device__ __forceinline__ float row_max(float x) {
+    return over_rows(x, [](float a, float b) { return fmaxf(a, b); });
+}
+// x of the lane `N` further on in the row of 16 (row_ror)
+template <int N>
+__device__ __forceinline__ float row_rotate(float x) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0x120 | N, 0xf, 0xf, true));
+}
+
 // s_waitcnt immediate that waits for vmcnt <= n only (gfx9 encoding).
 constexpr int vmcnt_imm(int n) { return (n & 15) | (7 << 4) | (15 << 8) | ((n >> 4) << 14); }
 

@@ -1,0 +1,371 @@
+// The layer stack of a training step: buffers and launches of the kernels of train_layers.h around the row
+// attention (include/artab_attention.h, artab_train_*).
+#include "../../include/artab_attention.h"
+#include "launchers.h"
+#include "train_layers.h"
+
+namespace artab {
+namespace {
+
+constexpr int kParams = 16;  // per layer, in the order of artab_train_args.params
+enum ParamIndex : int { kPFeatV, kPFeatOut, kPQ, kPK, kPV, kPO, kPW1, kPBias1, kPW2, kPBias2, kPG1, kPB1, kPG2, kPB2, kPG3, kPB3 };
+
+struct Arena {  // deals out 256-byte aligned pieces of one allocation (or only counts them)
+    char *base;
+    size_t used = 0;
+    explicit Arena(void *p) : base(static_cast<char *>(p)) {}
+    template <typename T>
+    T *take(size_t n) {
+        T *r = base ? reinterpret_cast<T *>(base + used) : nullptr;
+        used += (n * sizeof(T) + 255) / 256 * 256;
+        return r;
+    }
+};
+
+struct SavedLayer {
+    float *r1, *r2, *r3, *lse;
+    float2 *stats1, *stats2, *stats3;
+    bf16_t *qkv, *attn;
+};
+struct Saved {
+    bf16_t *packed;
+    float *fo;
+    char *layers;
+    size_t layer_bytes, bytes;
+    SavedLayer layer(const artab_train_args &a, int l) const {
+        const size_t M = static_cast<size_t>(a.B) * a.R;
+        Arena s(layers ? layers + l * layer_bytes : nullptr);
+        return take(a, M, s);
+    }
+    static SavedLayer take(const artab_train_args &a, size_t M, Arena &s) {
+        SavedLayer v;
+        v.r1 = s.take<float>(M * a.D);
+        v.r2 = s.take<float>(M * a.D);
+        v.r3 = s.take<float>(M * a.D);
+        v.lse = s.take<float>(M * a.H);
+        v.stats1 = s.take<float2>(M);
+        v.stats2 = s.take<float2>(M);
+        v.stats3 = s.take<float2>(M);
+        v.qkv = s.take<bf16_t>(M * 3 * a.D);
+        v.attn = s.take<bf16_t>(M * a.D);
+        return v;
+    }
+};
+size_t packed_elems(int D, int F) { return 2 * (5 * static_cast<size_t>(D) * D + 2 * static_cast<size_t>(D) * F); }
+
+Saved saved_layout(const artab_train_args &a) {
+    Saved v;
+    Arena s(a.saved);
+    v.packed = s.take<bf16_t>(a.n_layers * packed_elems(a.D, a.F));
+    v.fo = s.take<float>(static_cast<size_t>(a.n_layers) * a.D * a.D);
+    v.layers = a.saved ? s.base + s.used : nullptr;
+    Arena one(nullptr);
+    Saved::take(a, static_cast<size_t>(a.B) * a.R, one);
+    v.layer_bytes = one.used;
+    v.bytes = s.used + v.layer_bytes * a.n_layers;
+    return v;
+}
+
+// offsets (floats) inside a layer's gradients
+struct GradLayout {
+    long qkv, fo, o, w1, w2, vec_b, vec_a, out, v, total;
+    GradLayout(int D, int F) {
+        const long dd = static_cast<long>(D) * D, df = static_cast<long>(D) * F;
+        qkv = 0; fo = 3 * dd; o = 4 * dd; w1 = 5 * dd; w2 = w1 + df;
+        vec_b = w2 + df;           // g3, b3, bias2, g2, b2, bias1
+        vec_a = vec_b + 5 * D + F; // g1, b1
+        out = vec_a + 2 * D; v = out + dd;
+        total = v + dd;
+    }
+};
+
+// Workgroups of a backward kernel: about two per compute unit, every one with the same number of tiles.
+int backward_groups(long M) {
+    const long tiles = (M + kTrainRows - 1) / kTrainRows, rounds = (tiles + 511) / 512;
+    return static_cast<int>((tiles + rounds - 1) / rounds);
+}
+int grad_jobs(int D, int F) { return (5 * D * D + 2 * D * F) / (128 * 128); }
+// Row slices of the weight-gradient products: enough that pieces times slices give every compute unit a
+// workgroup, none shorter than 256 rows.
+int grad_slices(long M, int jobs) {
+    const long most = (M + 255) / 256, want = (256 + jobs - 1) / jobs;
+    return static_cast<int>(want < most ? want : most);
+}
+constexpr int kFinalGroups = 512;
+
+struct Scratch {
+    float *dx, *dr2, *delta, *part_w, *part_b, *part_a, *part_f;
+    bf16_t *d3, *x2, *h, *du, *d2, *dattn, *dqkv, *x1, *d1, *x;
+    size_t bytes;
+};
+Scratch scratch_layout(const artab_train_args &a) {
+    const size_t M = static_cast<size_t>(a.B) * a.R, D = a.D, F = a.F;
+    const int groups = backward_groups(M), jobs = grad_jobs(a.D, a.F);
+    Scratch v;
+    Arena s(a.scratch);
+    v.dx = s.take<float>(M * D);
+    v.dr2 = s.take<float>(M * D);
+    v.delta = s.take<float>(M * a.H);
+    v.part_w = s.take<float>(static_cast<size_t>(grad_slices(M, jobs)) * jobs * 16384);
+    v.part_b = s.take<float>(groups * (5 * D + F));
+    v.part_a = s.take<float>(groups * 2 * D);
+    v.part_f = s.take<float>(kFinalGroups * 2 * D);
+    v.d3 = s.take<bf16_t>(M * D);
+    v.x2 = s.take<bf16_t>(M * D);
+    v.h = s.take<bf16_t>(M * F);
+    v.du = s.take<bf16_t>(M * F);
+    v.d2 = s.take<bf16_t>(M * D);
+    v.dattn = s.take<bf16_t>(M * D);
+    v.dqkv = s.take<bf16_t>(M * 3 * D);
+    v.x1 = s.take<bf16_t>(M * D);
+    v.d1 = s.take<bf16_t>(M * D);
+    v.x = s.take<bf16_t>(M * D);
+    v.bytes = s.used;
+    return v;
+}
+
+TrainWeights weights(const artab_train_args &a, int first) {
+    TrainWeights w{};
+    for (int i = 0; i < kTrainPackLayers && first + i < a.n_layers; ++i) {
+        const float *const *p = a.params + static_cast<size_t>(first + i) * kParams;
+        w.v[i] = p[kPFeatV]; w.out[i] = p[kPFeatOut];
+        w.q[i] = p[kPQ]; w.k[i] = p[kPK]; w.vr[i] = p[kPV]; w.o[i] = p[kPO];
+        w.w1[i] = p[kPW1]; w.w2[i] = p[kPW2];
+    }
+    return w;
+}
+
+struct HeadViews {
+    artab_view q, k, v, out;
+};
+HeadViews head_views(const artab_train_args &a, bf16_t *qkv, bf16_t *out) {
+    const int64_t D = a.D, Dh = a.D / a.H;
+    auto part = [&](int i) { return artab_view{qkv + i * D, a.R * 3 * D, Dh, 3 * D}; };
+    return {part(0), part(1), part(2), artab_view{out, a.R * D, Dh, D}};
+}
+
+#define TRAIN_TRY(expr)             \
+    do {                            \
+        const int rc_ = (expr);     \
+        if (rc_ != ARTAB_OK) return rc_; \
+    } while (0)
+
+template <int D, int F>
+int forward(const artab_train_args &a, hipStream_t st) {
+    const Saved S = saved_layout(a);
+    const long M = static_cast<long>(a.B) * a.R;
+    for (int l0 = 0; l0 < a.n_layers; l0 += kTrainPackLayers) {
+        const TrainWeights W = weights(a, l0);
+        const unsigned n = static_cast<unsigned>(a.n_layers - l0 < kTrainPackLayers ? a.n_layers - l0 : kTrainPackLayers);
+        float *fo = S.fo + static_cast<long>(l0) * D * D;
+        hipLaunchKernelGGL((train_fold_kernel<D>), dim3(D / 16, n), dim3(D), 0, st, W, fo);
+        hipLaunchKernelGGL((train_pack_kernel<D, F>), dim3(static_cast<unsigned>((train_packed_elems<D, F>() / 8 + 255) / 256), n), dim3(256),
+                           0, st, W, fo, S.packed + l0 * train_packed_elems<D, F>());
+    }
+    const dim3 grid(static_cast<unsigned>((M + kTrainRows - 1) / kTrainRows)), block(kTrainWaves * 64);
+    for (int l = 0; l < a.n_layers; ++l) {
+        const float *const *p = a.params + static_cast<size_t>(l) * kParams;
+        const SavedLayer v = S.layer(a, l);
+        const bf16_t *packed = S.packed + l * train_packed_elems<D, F>();
+        TrainForwardA A{};
+        A.r_prev = a.x;
+        if (l > 0) {
+            const SavedLayer b = S.layer(a, l - 1);
+            A.r_prev = b.r3; A.stats_prev = b.stats3; A.g_prev = p[kPG3 - kParams]; A.b_prev = p[kPB3 - kParams];
+        }
+        A.packed = packed; A.g1 = p[kPG1]; A.b1 = p[kPB1]; A.eps1 = a.eps1;
+        A.r1 = v.r1; A.stats1 = v.stats1; A.qkv = v.qkv; A.M = M;
+        hipLaunchKernelGGL((train_forward_a_kernel<D, F>), grid, block, 0, st, A);
+        const HeadViews h = head_views(a, v.qkv, v.attn);
+        TRAIN_TRY(artab_row_mask_attention(&h.q, &h.k, &h.v, &h.out, v.lse, a.B, a.H, a.R, a.context_len, a.buffer_len, a.attending_chunks,
+                                           D / a.H, 0.f, ARTAB_BF16, ARTAB_IMPL_AUTO, st));
+        TrainForwardB B{};
+        B.attn = v.attn; B.r1 = v.r1; B.stats1 = v.stats1; B.g1 = p[kPG1]; B.b1 = p[kPB1]; B.packed = packed;
+        B.g2 = p[kPG2]; B.b2 = p[kPB2]; B.bias1 = p[kPBias1]; B.bias2 = p[kPBias2]; B.eps2 = a.eps2; B.eps3 = a.eps3;
+        B.r2 = v.r2; B.stats2 = v.stats2; B.r3 = v.r3; B.stats3 = v.stats3; B.M = M;
+        hipLaunchKernelGGL((train_forward_b_kernel<D, F>), grid, block, 0, st, B);
+    }
+    const float *const *p = a.params + static_cast<size_t>(a.n_layers - 1) * kParams;
+    const SavedLayer v = S.layer(a, a.n_layers - 1);
+    TrainFinal Z{};
+    Z.r3 = v.r3; Z.stats3 = v.stats3; Z.g3 = p[kPG3]; Z.b3 = p[kPB3]; Z.g = a.norm_gamma; Z.b = a.norm_beta; Z.eps = a.eps_out;
+    Z.z = a.z; Z.B = a.B; Z.R = a.R; Z.first = a.first_row;
+    const long rows = static_cast<long>(a.B) * (a.R - a.first_row);
+    hipLaunchKernelGGL((train_final_kernel<D, false>), dim3(static_cast<unsigned>((rows + 3) / 4 < 2048 ? (rows + 3) / 4 : 2048)), dim3(256), 0, st, Z);
+    return hipGetLastError() == hipSuccess ? ARTAB_OK : ARTAB_ERR_LAUNCH;
+}
+
+template <int D, int F>
+int backward(const artab_train_args &a, hipStream_t st) {
+    const Saved S = saved_layout(a);
+    const Scratch X = scratch_layout(a);
+    const GradLayout G(D, F);
+    const long M = static_cast<long>(a.B) * a.R;
+    const int groups = backward_groups(M), jobs = grad_jobs(D, F), slices = grad_slices(M, jobs);
+    const dim3 block(kTrainWaves * 64);
+    {
+        const float *const *p = a.params + static_cast<size_t>(a.n_layers - 1) * kParams;
+        const SavedLayer v = S.layer(a, a.n_layers - 1);
+        TrainFinal Z{};
+        Z.r3 = v.r3; Z.stats3 = v.stats3; Z.g3 = p[kPG3]; Z.b3 = p[kPB3]; Z.g = a.norm_gamma; Z.b = a.norm_beta; Z.eps = a.eps_out;
+        Z.dz = a.dz; Z.dx = X.dx; Z.part = X.part_f; Z.B = a.B; Z.R = a.R; Z.first = a.first_row;
+        hipLaunchKernelGGL((train_final_kernel<D, true>), dim3(kFinalGroups), dim3(256), 0, st, Z);
+        TrainReduce T{};
+        T.cols[0] = {X.part_f, a.grads + a.n_layers * G.total, kFinalGroups, 2 * D};
+        T.n_cols = 1;
+        hipLaunchKernelGGL(train_reduce_kernel, dim3(2 * D / 64), dim3(256), 0, st, T);
+    }
+    for (int l = a.n_layers - 1; l >= 0; --l) {
+        const float *const *p = a.params + static_cast<size_t>(l) * kParams;
+        const SavedLayer v = S.layer(a, l);
+        const bf16_t *packed = S.packed + l * train_packed_elems<D, F>();
+        float *g = a.grads + l * G.total;
+        TrainBackwardB B{};
+        B.dx = X.dx; B.r3 = v.r3; B.stats3 = v.stats3; B.g3 = p[kPG3]; B.r2 = v.r2; B.stats2 = v.stats2; B.g2 = p[kPG2]; B.b2 = p[kPB2];
+        B.bias1 = p[kPBias1]; B.packed = packed; B.dr2 = X.dr2; B.d3 = X.d3; B.x2 = X.x2; B.h = X.h; B.du = X.du; B.d2 = X.d2;
+        B.dattn = X.dattn; B.part = X.part_b; B.M = M;
+        hipLaunchKernelGGL((train_backward_b_kernel<D, F>), dim3(groups), block, 0, st, B);
+        const HeadViews h = head_views(a, v.qkv, v.attn), d = head_views(a, X.dqkv, X.dattn);
+        TRAIN_TRY(artab_row_mask_attention_backward(&h.q, &h.k, &h.v, &h.out, &d.out, v.lse, X.delta, &d.q, &d.k, &d.v, a.B, a.H, a.R, a.context_len,
+                                                    a.buffer_len, a.attending_chunks, D / a.H, 0.f, ARTAB_BF16, ARTAB_IMPL_AUTO, st));
+        TrainBackwardA A{};
+        A.dqkv = X.dqkv; A.dr2 = X.dr2; A.r1 = v.r1; A.stats1 = v.stats1; A.g1 = p[kPG1]; A.b1 = p[kPB1];
+        A.r_prev = a.x;
+        if (l > 0) {
+            const SavedLayer b = S.layer(a, l - 1);
+            A.r_prev = b.r3; A.stats_prev = b.stats3; A.g_prev = p[kPG3 - kParams]; A.b_prev = p[kPB3 - kParams];
+        }
+        A.packed = packed; A.dx = l > 0 ? X.dx : a.dx; A.x1 = X.x1; A.d1 = X.d1; A.x = X.x; A.part = X.part_a; A.M = M;
+        hipLaunchKernelGGL((train_backward_a_kernel<D, F>), dim3(groups), block, 0, st, A);
+
+        TrainGradJobs J{};
+        TrainReduce T{};
+        auto add = [&](const bf16_t *P, int ldp, const bf16_t *Q, int ldq, int N, int K, float *out) {
+            for (int n = 0; n < N; n += 128)
+                for (int k = 0; k < K; k += 128) {
+                    J.p[J.jobs] = P + n; J.q[J.jobs] = Q + k; J.ldp[J.jobs] = ldp; J.ldq[J.jobs] = ldq;
+                    T.out[J.jobs] = out + static_cast<long>(n) * K + k; T.ld[J.jobs] = K;
+                    ++J.jobs;
+                }
+        };
+        add(X.dqkv, 3 * D, X.x1, D, 3 * D, D, g + G.qkv);
+        add(X.d1, D, X.x, D, D, D, g + G.fo);
+        add(X.d2, D, v.attn, D, D, D, g + G.o);
+        add(X.du, F, X.x2, D, F, D, g + G.w1);
+        add(X.d3, D, X.h, F, D, F, g + G.w2);
+        J.part = X.part_w; J.M = M; J.rows_per_slice = ((M + slices - 1) / slices + 63) / 64 * 64;
+        hipLaunchKernelGGL(train_weight_grad_kernel, dim3(jobs, slices), dim3(512), 0, st, J);
+        T.part = X.part_w; T.jobs = jobs; T.slices = slices;
+        T.cols[0] = {X.part_b, g + G.vec_b, groups, 5 * D + F};
+        T.cols[1] = {X.part_a, g + G.vec_a, groups, 2 * D};
+        T.n_cols = 2;
+        hipLaunchKernelGGL(train_reduce_kernel, dim3(jobs * 16 + (7 * D + F) / 64), dim3(256), 0, st, T);
+    }
+    for (int l0 = 0; l0 < a.n_layers; l0 += kTrainPackLayers) {
+        const unsigned n = static_cast<unsigned>(a.n_layers - l0 < kTrainPackLayers ? a.n_layers - l0 : kTrainPackLayers);
+        hipLaunchKernelGGL((train_unfold_kernel<D>), dim3(2 * (D / 16), n), dim3(D), 0, st, weights(a, l0), a.grads + l0 * G.total, G.total,
+                           G.fo, G.out, G.v);
+    }
+    return hipGetLastError() == hipSuccess ? ARTAB_OK : ARTAB_ERR_LAUNCH;
+}
+
+bool supported(const artab_train_args *a) {
+    if (!a || a->B < 1 || a->R < 1 || a->H < 1 || a->n_layers < 1) return false;
+    if ((a->D != 128 && a->D != 256) || a->F != 256 || a->D % a->H) return false;
+    const int Dh = a->D / a->H;
+    if (Dh != 32 && Dh != 64) return false;
+    return a->context_len >= 1 && a->buffer_len >= 0 && a->context_len + a->buffer_len <= a->R && a->attending_chunks >= 0 &&
+           a->first_row >= 0 && a->first_row < a->R && static_cast<int64_t>(a->B) * a->R < (1 << 30);
+}
+
+constexpr int kEmbedSlices = 8;
+
+bool embed_supported(const artab_train_embed_args *a) {
+    return a && a->B >= 1 && (a->D == 128 || a->D == 256) && a->feat >= 1 && a->n_context >= 1 && a->n_buffer >= 0 && a->n_target >= 1 &&
+           static_cast<int64_t>(a->B) * (a->n_context + a->n_buffer + a->n_target) < (1 << 30);
+}
+
+template <int D>
+int embed(const artab_train_embed_args &a, hipStream_t st) {
+    TrainEmbed P{};
+    P.x[0] = a.x_context; P.x[1] = a.x_buffer; P.x[2] = a.x_target; P.y[0] = a.y_context; P.y[1] = a.y_buffer;
+    P.n[0] = a.n_context; P.n[1] = a.n_buffer; P.n[2] = a.n_target; P.feat = a.feat;
+    P.w_x = a.w_x; P.b_x = a.b_x; P.w_y = a.w_y; P.b_y = a.b_y; P.markers = a.markers; P.tokens = a.tokens;
+    P.out = a.out; P.xy = reinterpret_cast<float2 *>(a.xy); P.B = a.B; P.R = a.n_context + a.n_buffer + a.n_target;
+    const long n = static_cast<long>(P.B) * P.R * (D / 4);
+    hipLaunchKernelGGL((train_embed_kernel<D>), dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, st, P);
+    return hipGetLastError() == hipSuccess ? ARTAB_OK : ARTAB_ERR_LAUNCH;
+}
+
+template <int D>
+int embed_backward(const artab_train_embed_args &a, hipStream_t st) {
+    TrainEmbedBackward P{};
+    P.dx = a.out; P.xy = reinterpret_cast<const float2 *>(a.xy); P.B = a.B; P.R = a.n_context + a.n_buffer + a.n_target;
+    P.n_ctx = a.n_context; P.n_buf = a.n_buffer; P.slices = kEmbedSlices;
+    Arena s(a.scratch);
+    P.part = s.take<float>(static_cast<size_t>(a.B) * kEmbedSlices * 5 * D);
+    float *sums = s.take<float>(5 * D);
+    P.d_tokens = a.grads + 7 * D;
+    hipLaunchKernelGGL((train_embed_backward_kernel<D>), dim3(a.B > a.n_buffer ? a.B : a.n_buffer, kEmbedSlices + 1), dim3(D), 0, st, P);
+    TrainReduce T{};
+    T.cols[0] = {P.part, sums, a.B * kEmbedSlices, 5 * D};
+    T.n_cols = 1;
+    hipLaunchKernelGGL(train_reduce_kernel, dim3(5 * D / 64), dim3(256), 0, st, T);
+    hipLaunchKernelGGL(train_embed_finish_kernel, dim3(1), dim3(D), 0, st, sums, a.grads, D);
+    return hipGetLastError() == hipSuccess ? ARTAB_OK : ARTAB_ERR_LAUNCH;
+}
+
+}  // namespace
+}  // namespace artab
+
+extern "C" {
+
+size_t artab_train_embed_scratch_bytes(const artab_train_embed_args *a) {
+    if (!artab::embed_supported(a)) return 0;
+    artab::Arena s(nullptr);
+    s.take<float>(static_cast<size_t>(a->B) * artab::kEmbedSlices * 5 * a->D);
+    s.take<float>(5 * a->D);
+    return s.used;
+}
+int artab_train_embed(const artab_train_embed_args *a, void *stream) {
+    if (!artab::embed_supported(a)) return ARTAB_ERR_UNSUPPORTED;
+    if (!a->x_context || !a->y_context || (a->n_buffer && (!a->x_buffer || !a->y_buffer || !a->tokens)) || !a->x_target || !a->w_x || !a->b_x ||
+        !a->w_y || !a->b_y || !a->markers || !a->out || !a->xy)
+        return ARTAB_ERR_NULL_POINTER;
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    return a->D == 128 ? artab::embed<128>(*a, st) : artab::embed<256>(*a, st);
+}
+int artab_train_embed_backward(const artab_train_embed_args *a, void *stream) {
+    if (!artab::embed_supported(a)) return ARTAB_ERR_UNSUPPORTED;
+    if (!a->out || !a->xy || !a->grads || !a->scratch) return ARTAB_ERR_NULL_POINTER;
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    return a->D == 128 ? artab::embed_backward<128>(*a, st) : artab::embed_backward<256>(*a, st);
+}
+
+size_t artab_train_saved_bytes(const artab_train_args *a) {
+    if (!artab::supported(a)) return 0;
+    artab_train_args b = *a;
+    b.saved = nullptr;
+    return artab::saved_layout(b).bytes;
+}
+size_t artab_train_scratch_bytes(const artab_train_args *a) {
+    if (!artab::supported(a)) return 0;
+    artab_train_args b = *a;
+    b.scratch = nullptr;
+    return artab::scratch_layout(b).bytes;
+}
+int artab_train_forward(const artab_train_args *a, void *stream) {
+    if (!artab::supported(a)) return ARTAB_ERR_UNSUPPORTED;
+    if (!a->x || !a->params || !a->saved || !a->z || !a->norm_gamma || !a->norm_beta) return ARTAB_ERR_NULL_POINTER;
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    return a->D == 128 ? artab::forward<128, 256>(*a, st) : artab::forward<256, 256>(*a, st);
+}
+int artab_train_backward(const artab_train_args *a, void *stream) {
+    if (!artab::supported(a)) return ARTAB_ERR_UNSUPPORTED;
+    if (!a->x || !a->params || !a->saved || !a->dz || !a->dx || !a->grads || !a->scratch || !a->norm_gamma || !a->norm_beta)
+        return ARTAB_ERR_NULL_POINTER;
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    return a->D == 128 ? artab::backward<128, 256>(*a, st) : artab::backward<256, 256>(*a, st);
+}
+
+}  // extern "C"

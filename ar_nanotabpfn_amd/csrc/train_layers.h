@@ -1,0 +1,984 @@
+// The transformer layers of a training step around the row attention, forward and backward (gfx950;
+// float32 parameters and residual stream, bfloat16 products with float32 sums: what autocast computes).
+//
+// A step of the reference's training configuration touches 38912 rows of width 128 twelve times over; every
+// layer is five small products per row.  As library calls that is 1300 launches with a cast, a bias, a norm
+// or a copy of 20 MB between any two products, and weight gradients whose 128 x 128 outputs leave most of
+// the chip idle.  Here a layer is: forward two kernels around the attention call, backward two kernels
+// around its backward call, one split product for all weight gradients, one reduction.  They are bound by
+// memory: each reads and writes the residual stream and what the weight gradients need once.
+//
+//   forward    a: x = LN3(r3 of the layer in front); r1 = x + x W_fo^T; x1 = LN1(r1); qkv = x1 W_qkv^T
+//              b: r2 = x1 + attn W_o^T; x2 = LN2(r2); u = x2 W_1^T + b_1; r3 = x2 + gelu(u) W_2^T + b_2
+//   backward   b: d(x of the next layer) -> dr3, du (u is recomputed), dr2, d(attn)
+//              a: d(qkv) -> dr1, dx
+// with W_fo = out_proj v_proj of the single-column feature attention (one key per query: the softmax weight
+// is 1); dW_out = dW_fo W_v^T and dW_v = W_out^T dW_fo follow from its gradient.  Of every LayerNorm the sum
+// in front of it and (mean, 1/std) are kept; its output is recomputed where it is read.
+//
+// Tiles.  A workgroup of four wavefronts owns 32 rows and all columns; products are transposed as in
+// fused_layer.h (C^T[n, m] = sum_k W[n, k] A[m, k], v_mfma_f32_16x16x32): a lane holds, for two token rows
+// (lane % 16 and + 16), four consecutive features 4 (lane / 16) + r of every 16-feature block.  Small
+// workgroups, four or five to a compute unit, so that the loads of one run under the products of others.
+#pragma once
+
+#include "common.h"
+#include "fused_layer.h"
+#include "mfma_flash.h"
+
+namespace artab {
+
+constexpr int kTrainWaves = 4, kTrainRows = 32;
+constexpr int kTrainPackLayers = 16;   // layers per launch of the weight kernels
+constexpr int kTrainMaxJobs = 32;      // 128 x 128 pieces of a layer's weight gradients
+
+// packed bf16 matrices of a layer, in this order; T: the transposed matrix
+enum TrainMatrix : int { kTmFo, kTmFoT, kTmQkv, kTmQkvT, kTmO, kTmOT, kTm1, kTm1T, kTm2, kTm2T, kTmCount };
+template <int D, int F>
+__host__ __device__ constexpr long train_matrix_at(int m) {  // element offset inside a layer's packed weights
+    constexpr long size[kTmCount] = {D * D, D * D, 3 * D * D, 3 * D * D, D * D, D * D, D * F, D * F, D * F, D * F};
+    long at = 0;
+    for (int i = 0; i < m; ++i) at += size[i];
+    return at;
+}
+template <int D, int F>
+constexpr long train_packed_elems() { return train_matrix_at<D, F>(kTmCount); }
+
+struct TrainWeights {  // float32 masters of up to kTrainPackLayers layers, row-major
+    const float *v[kTrainPackLayers], *out[kTrainPackLayers];              // feature attention [D, D]
+    const float *q[kTrainPackLayers], *k[kTrainPackLayers], *vr[kTrainPackLayers], *o[kTrainPackLayers];
+    const float *w1[kTrainPackLayers], *w2[kTrainPackLayers];              // [F, D], [D, F]
+};
+
+// fo[layer] = out v: 16 rows of one layer per workgroup
+template <int D>
+__global__ __launch_bounds__(D) void train_fold_kernel(TrainWeights W, float *fo) {
+    __shared__ float out_s[16][D];
+    const int layer = blockIdx.y, n0 = 16 * blockIdx.x, k = threadIdx.x;
+    const float *out = W.out[layer], *v = W.v[layer];
+#pragma unroll
+    for (int n = 0; n < 16; ++n) out_s[n][k] = out[(n0 + n) * D + k];
+    __syncthreads();
+    float acc[16];
+#pragma unroll
+    for (int n = 0; n < 16; ++n) acc[n] = 0.f;
+    for (int j = 0; j < D; ++j) {
+        const float x = v[j * D + k];
+#pragma unroll
+        for (int n = 0; n < 16; ++n) acc[n] = fmaf(out_s[n][j], x, acc[n]);
+    }
+#pragma unroll
+    for (int n = 0; n < 16; ++n) fo[(static_cast<long>(layer) * D + n0 + n) * D + k] = acc[n];
+}
+
+// dout[n][j] = sum_k dfo[n][k] v[j][k];  dv[j][k] = sum_n out[n][j] dfo[n][k].  16 rows per workgroup.
+template <int D>
+__global__ __launch_bounds__(D) void train_unfold_kernel(TrainWeights W, float *grads, long layer_stride, long at_fo, long at_out,
+                                                         long at_v) {
+    __shared__ float a_s[16][D + 1];
+    const int layer = blockIdx.y, r0 = 16 * (blockIdx.x % (D / 16)), c = threadIdx.x;
+    const bool for_v = blockIdx.x >= D / 16;
+    float *g = grads + layer * layer_stride;
+    const float *dfo = g + at_fo;
+    float acc[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+    if (!for_v) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) a_s[i][c] = dfo[(r0 + i) * D + c];
+        __syncthreads();
+        const f32x4 *row = reinterpret_cast<const f32x4 *>(W.v[layer] + static_cast<long>(c) * D);
+        for (int k = 0; k < D / 4; ++k) {
+            const f32x4 x = row[k];
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) acc[i] = fmaf(a_s[i][4 * k + e], x[e], acc[i]);
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) a_s[i][c] = W.out[layer][static_cast<long>(c) * D + r0 + i];
+        __syncthreads();
+        for (int n = 0; n < D; ++n) {
+            const float x = dfo[n * D + c];
+#pragma unroll
+            for (int i = 0; i < 16; ++i) acc[i] = fmaf(a_s[i][n], x, acc[i]);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) g[(for_v ? at_v : at_out) + (r0 + i) * D + c] = acc[i];
+}
+
+// Every matrix of a layer as bf16 operand fragments: fragment (nb, ks) of W [N, K] is 1 KiB, lane l holds
+// W[16 nb + l % 16][32 ks + 8 (l / 16) ..].  One 16-byte piece per thread.
+template <int D, int F>
+__global__ __launch_bounds__(256) void train_pack_kernel(TrainWeights W, const float *fo, bf16_t *packed) {
+    const int layer = blockIdx.y;
+    const long piece = static_cast<long>(blockIdx.x) * 256 + threadIdx.x;
+    if (piece * 8 >= train_packed_elems<D, F>()) return;
+    int m = 0;
+    while (m + 1 < kTmCount && piece * 8 >= train_matrix_at<D, F>(m + 1)) ++m;
+    const long in = piece - train_matrix_at<D, F>(m) / 8;
+    const bool t = m & 1;
+    int N, K;  // of the matrix as it is packed
+    switch (m & ~1) {
+        case kTmQkv: N = 3 * D; K = D; break;
+        case kTm1: N = F; K = D; break;
+        case kTm2: N = D; K = F; break;
+        default: N = K = D; break;
+    }
+    if (t) { const int x = N; N = K; K = x; }
+    const int lane = static_cast<int>(in & 63), frag = static_cast<int>(in >> 6), ks = frag % (K / 32), nb = frag / (K / 32);
+    const int n = 16 * nb + (lane & 15), k0 = 32 * ks + 8 * (lane >> 4);
+    const float *src;
+    switch (m & ~1) {
+        case kTmFo: src = fo + static_cast<long>(layer) * D * D; break;
+        case kTmQkv: src = nullptr; break;
+        case kTmO: src = W.o[layer]; break;
+        case kTm1: src = W.w1[layer]; break;
+        default: src = W.w2[layer]; break;
+    }
+    float f[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const int row = t ? k0 + e : n, col = t ? n : k0 + e, width = t ? N : K;  // element [row][col] of the master
+        if ((m & ~1) == kTmQkv) {
+            const float *part = row < D ? W.q[layer] : row < 2 * D ? W.k[layer] : W.vr[layer];
+            f[e] = part[static_cast<long>(row % D) * D + col];
+        } else {
+            f[e] = src[static_cast<long>(row) * width + col];
+        }
+    }
+    const u32x4 v = {pack2<bf16_t>(f[0], f[1]), pack2<bf16_t>(f[2], f[3]), pack2<bf16_t>(f[4], f[5]), pack2<bf16_t>(f[6], f[7])};
+    reinterpret_cast<u32x4 *>(packed + static_cast<long>(layer) * train_packed_elems<D, F>())[piece] = v;
+}
+
+// ---- tiles
+
+template <int NB>
+using TrainAcc = f32x4[NB][2];  // [16-feature block][token half]
+
+// A pointer again, as one the compiler cannot trace: in a loop over tiles it would otherwise take the weights,
+// which are the same for every tile, as something to keep in registers.
+__device__ __forceinline__ const bf16_t *train_opaque(const bf16_t *p) {
+    asm volatile("" : "+s"(p));
+    return p;
+}
+
+struct TrainLane {
+    int wave, lane, tok, quad;
+    long row0, M;
+    __device__ __forceinline__ TrainLane(long tile, long M_) : M(M_) {
+        wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        lane = threadIdx.x & 63;
+        tok = lane & 15;
+        quad = lane >> 4;
+        row0 = tile * kTrainRows;
+    }
+    __device__ __forceinline__ long row(int tb) const { return min(row0 + 16 * tb + tok, M - 1); }
+    __device__ __forceinline__ bool live(int tb) const { return row0 + 16 * tb + tok < M; }
+    __device__ __forceinline__ int col(int b) const { return 16 * (wave + kTrainWaves * b) + 4 * quad; }
+};
+
+template <int D, int NB>
+__device__ __forceinline__ void train_load(f32x4 (&v)[NB][2], const float *src, const TrainLane &L) {
+#pragma unroll
+    for (int tb = 0; tb < 2; ++tb)
+#pragma unroll
+        for (int b = 0; b < NB; ++b) v[b][tb] = *reinterpret_cast<const f32x4 *>(src + L.row(tb) * D + L.col(b));
+}
+template <int D, int NB>
+__device__ __forceinline__ void train_store(float *dst, const f32x4 (&v)[NB][2], const TrainLane &L) {
+#pragma unroll
+    for (int tb = 0; tb < 2; ++tb)
+        if (L.live(tb)) {
+#pragma unroll
+            for (int b = 0; b < NB; ++b) *reinterpret_cast<f32x4 *>(dst + L.row(tb) * D + L.col(b)) = v[b][tb];
+        }
+}
+template <int NB>
+__device__ __forceinline__ void train_store16(bf16_t *dst, long ld, int col0, const f32x4 (&v)[NB][2], const TrainLane &L) {
+#pragma unroll
+    for (int tb = 0; tb < 2; ++tb)
+        if (L.live(tb)) {
+#pragma unroll
+            for (int b = 0; b < NB; ++b) store4f<bf16_t>(dst + L.row(tb) * ld + col0 + L.col(b), v[b][tb][0], v[b][tb][1], v[b][tb][2], v[b][tb][3]);
+        }
+}
+template <int NB>
+__device__ __forceinline__ void train_to_lds(bf16_t *tile, int ld, const f32x4 (&v)[NB][2], const TrainLane &L) {
+#pragma unroll
+    for (int tb = 0; tb < 2; ++tb)
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+            store4f<bf16_t>(tile + (16 * tb + L.tok) * ld + L.col(b), v[b][tb][0], v[b][tb][1], v[b][tb][2], v[b][tb][3]);
+}
+// [32, W] bf16 between global memory (row stride ld) and an LDS tile (row stride lds_ld), 16 bytes a lane
+template <int W>
+__device__ __forceinline__ void train_stage(bf16_t *tile, int lds_ld, const bf16_t *src, long ld, long row0, long M) {
+    constexpr int CPR = W / 8;
+#pragma unroll
+    for (int i = threadIdx.x; i < kTrainRows * CPR; i += kTrainWaves * 64) {
+        const int r = i / CPR, c = i % CPR;
+        *reinterpret_cast<u32x4 *>(tile + r * lds_ld + 8 * c) = *reinterpret_cast<const u32x4 *>(src + min(row0 + r, M - 1) * ld + 8 * c);
+    }
+}
+template <int W>
+__device__ __forceinline__ void train_unstage(bf16_t *dst, long ld, const bf16_t *tile, int lds_ld, long row0, long M) {
+    constexpr int CPR = W / 8;
+#pragma unroll
+    for (int i = threadIdx.x; i < kTrainRows * CPR; i += kTrainWaves * 64) {
+        const int r = i / CPR, c = i % CPR;
+        if (row0 + r < M) *reinterpret_cast<u32x4 *>(dst + (row0 + r) * ld + 8 * c) = *reinterpret_cast<const u32x4 *>(tile + r * lds_ld + 8 * c);
+    }
+}
+
+// acc[b][tb] = sum_k W[16 (nb0 + wave + 4 b) ..][k] A[16 tb + tok][k]; a few contraction steps of the
+// weights are on their way ahead of the one being multiplied
+template <int NB, int KS>
+__device__ __forceinline__ void train_product(f32x4 (&acc)[NB][2], const bf16_t *tile, int ld, const bf16_t *w, int nb0, const TrainLane &L) {
+    typedef MfmaOps<bf16_t> Ops;
+    constexpr int PF = NB <= 2 ? (KS < 4 ? KS : 4) : 2;
+    const char *const base = reinterpret_cast<const char *>(w) + (static_cast<long>(nb0 + L.wave) * KS) * 1024 + 16 * L.lane;
+    auto frag = [&](int b, int ks) { return *reinterpret_cast<const u32x4 *>(base + (static_cast<long>(kTrainWaves) * b * KS + ks) * 1024); };
+    u32x4 ring[PF][NB];
+#pragma unroll
+    for (int p = 0; p < PF; ++p)
+#pragma unroll
+        for (int b = 0; b < NB; ++b) ring[p][b] = frag(b, p);
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int tb = 0; tb < 2; ++tb) acc[b][tb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const bf16_t *const a = tile + L.tok * ld + 8 * L.quad;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+        const bf16x8 a0 = *reinterpret_cast<const bf16x8 *>(a + 32 * ks), a1 = *reinterpret_cast<const bf16x8 *>(a + 16 * ld + 32 * ks);
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            const bf16x8 wv = __builtin_bit_cast(bf16x8, ring[ks % PF][b]);
+            acc[b][0] = Ops::mma16(wv, a0, acc[b][0]);
+            acc[b][1] = Ops::mma16(wv, a1, acc[b][1]);
+            if (ks + PF < KS) ring[ks % PF][b] = frag(b, ks + PF);
+        }
+    }
+}
+
+// Sums of two per-row values over all features: lanes, then wavefronts.  red: [4][32] float2.
+struct TrainPair {
+    float a, b;
+};
+__device__ __forceinline__ void train_row_sums(TrainPair (&s)[2], float2 *red, const TrainLane &L) {
+#pragma unroll
+    for (int tb = 0; tb < 2; ++tb) {
+        s[tb].a = row_sum(s[tb].a);
+        s[tb].b = row_sum(s[tb].b);
+        if (L.quad == 0) red[L.wave * kTrainRows + 16 * tb + L.tok] = make_float2(s[tb].a, s[tb].b);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int tb = 0; tb < 2; ++tb) {
+        float2 p[kTrainWaves];
+#pragma unroll
+        for (int w = 0; w < kTrainWaves; ++w) p[w] = red[w * kTrainRows + 16 * tb + L.tok];
+        s[tb].a = (p[0].x + p[1].x) + (p[2].x + p[3].x);
+        s[tb].b = (p[0].y + p[1].y) + (p[2].y + p[3].y);
+    }
+}
+
+// (mean, 1/std) of the rows of v, kept in `stats`; one barrier inside.  The wavefronts' means and squared
+// deviations are combined pairwise (Chan et al.).
+template <int D, int NB>
+__device__ __forceinline__ void train_stats(const f32x4 (&v)[NB][2], float2 *red, float eps, float2 *stats, float2 (&st)[2], const TrainLane &L) {
+    constexpr float kLocal = NB * 16;
+#pragma unroll
+    for (int tb = 0; tb < 2; ++tb) {
+        float s = 0.f;
+#pragma unroll
+        for (int b = 0; b < NB; ++b) s += (v[b][tb][0] + v[b][tb][1]) + (v[b][tb][2] + v[b][tb][3]);
+        const float mean = row_sum(s) * (1.f / kLocal);
+        float q = 0.f;
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float d = v[b][tb][e] - mean;
+                q = fmaf(d, d, q);
+            }
+        q = row_sum(q);
+        if (L.quad == 0) red[L.wave * kTrainRows + 16 * tb + L.tok] = make_float2(mean, q);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int tb = 0; tb < 2; ++tb) {
+        float2 p[kTrainWaves];
+#pragma unroll
+        for (int w = 0; w < kTrainWaves; ++w) p[w] = red[w * kTrainRows + 16 * tb + L.tok];
+        const float mean = ((p[0].x + p[1].x) + (p[2].x + p[3].x)) * (1.f / kTrainWaves);
+        float m2 = 0.f;
+#pragma unroll
+        for (int w = 0; w < kTrainWaves; ++w) {
+            const float d = p[w].x - mean;
+            m2 += fmaf(kLocal * d, d, p[w].y);
+        }
+        st[tb] = make_float2(mean, rsqrtf(m2 / D + eps));
+        if (L.wave == 0 && L.quad == 0 && L.live(tb)) stats[L.row(tb)] = st[tb];
+    }
+}
+__device__ __forceinline__ void train_get_stats(float2 (&st)[2], const float2 *stats, const TrainLane &L) {
+#pragma unroll
+    for (int tb = 0; tb < 2; ++tb) st[tb] = stats[L.row(tb)];
+}
+// x = (r - mean) / std * g + b
+template <int NB>
+__device__ __forceinline__ void train_norm(f32x4 (&x)[NB][2], const f32x4 (&r)[NB][2], const float2 (&st)[2], const float *g, const float *be, const TrainLane &L) {
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        const f32x4 gv = *reinterpret_cast<const f32x4 *>(g + L.col(b)), bv = *reinterpret_cast<const f32x4 *>(be + L.col(b));
+#pragma unroll
+        for (int tb = 0; tb < 2; ++tb)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[b][tb][e] = fmaf((r[b][tb][e] - st[tb].x) * st[tb].y, gv[e], bv[e]);
+    }
+}
+
+struct TrainForwardA {
+    const float *r_prev;       // [M, D]: x itself (layer 0) or the sum in front of the last norm of the layer before
+    const float2 *stats_prev;  // its statistics, or nullptr (layer 0)
+    const float *g_prev, *b_prev;
+    const bf16_t *packed;
+    const float *g1, *b1;
+    float eps1;
+    float *r1; float2 *stats1;
+    bf16_t *qkv;               // [M, 3 D]
+    long M;
+};
+
+template <int D, int F>
+__global__ __launch_bounds__(kTrainWaves * 64) void train_forward_a_kernel(TrainForwardA P) {
+    constexpr int NB = D / 64, KS = D / 32, LD = D + 8;
+    __shared__ __attribute__((aligned(16))) bf16_t xs[kTrainRows * LD], ys[kTrainRows * LD];
+    __shared__ float2 red[kTrainWaves * kTrainRows];
+    const TrainLane L(blockIdx.x, P.M);
+    f32x4 x[NB][2], acc[NB][2];
+    train_load<D>(x, P.r_prev, L);
+    if (P.stats_prev) {
+        float2 st[2];
+        train_get_stats(st, P.stats_prev, L);
+        train_norm(x, x, st, P.g_prev, P.b_prev, L);
+    }
+    train_to_lds(xs, LD, x, L);
+    __syncthreads();
+    train_product<NB, KS>(acc, xs, LD, P.packed + train_matrix_at<D, F>(kTmFo), 0, L);
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int tb = 0; tb < 2; ++tb) acc[b][tb] += x[b][tb];
+    train_store<D>(P.r1, acc, L);
+    float2 st[2];
+    train_stats<D>(acc, red, P.eps1, P.stats1, st, L);
+    train_norm(acc, acc, st, P.g1, P.b1, L);
+    train_to_lds(ys, LD, acc, L);
+    __syncthreads();
+#pragma unroll
+    for (int part = 0; part < 3; ++part) {
+        train_product<NB, KS>(acc, ys, LD, P.packed + train_matrix_at<D, F>(kTmQkv), part * (D / 16), L);
+        train_store16(P.qkv, 3 * D, part * D, acc, L);
+    }
+}
+
+struct TrainForwardB {
+    const bf16_t *attn;        // [M, D]
+    const float *r1; const float2 *stats1;
+    const float *g1, *b1;
+    const bf16_t *packed;
+    const float *g2, *b2, *bias1, *bias2;
+    float eps2, eps3;
+    float *r2; float2 *stats2;
+    float *r3; float2 *stats3;
+    long M;
+};
+
+// h = gelu(u) and its derivative, in float32: erf by the rational form 7.1.26 of Abramowitz and Stegun (absolute
+// error below 1.5e-7; both results are rounded to bf16), which shares its exponential with the derivative
+__device__ __forceinline__ void train_gelu(float u, float &h, float &dh) {
+    const float z = fabsf(u) * 0.70710678118654752f, e = fast_exp2(-z * z * kLog2e);
+    const float t = __builtin_amdgcn_rcpf(fmaf(0.3275911f, z, 1.f));
+    const float poly = t * fmaf(t, fmaf(t, fmaf(t, fmaf(t, 1.061405429f, -1.453152027f), 1.421413741f), -0.284496736f), 0.254829592f);
+    const float cdf = fmaf(0.5f, copysignf(fmaf(-poly, e, 1.f), u), 0.5f);
+    h = u * cdf;
+    dh = fmaf(u * 0.39894228040143268f, e, cdf);
+}
+
+template <int D, int F>
+__global__ __launch_bounds__(kTrainWaves * 64) void train_forward_b_kernel(TrainForwardB P) {
+    constexpr int NB = D / 64, NF = F / 64, LD = D + 8, LF = F + 8;
+    __shared__ __attribute__((aligned(16))) bf16_t as[kTrainRows * (LD > LF ? LD : LF)], ys[kTrainRows * LD];
+    __shared__ float2 red[kTrainWaves * kTrainRows];
+    const TrainLane L(blockIdx.x, P.M);
+    f32x4 x[NB][2], acc[NB][2];
+    train_stage<D>(as, LD, P.attn, D, L.row0, P.M);
+    train_load<D>(x, P.r1, L);
+    {
+        float2 st[2];
+        train_get_stats(st, P.stats1, L);
+        train_norm(x, x, st, P.g1, P.b1, L);
+    }
+    __syncthreads();
+    train_product<NB, D / 32>(acc, as, LD, P.packed + train_matrix_at<D, F>(kTmO), 0, L);
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int tb = 0; tb < 2; ++tb) x[b][tb] += acc[b][tb];
+    train_store<D>(P.r2, x, L);
+    float2 st[2];
+    train_stats<D>(x, red, P.eps2, P.stats2, st, L);
+    train_norm(x, x, st, P.g2, P.b2, L);
+    train_to_lds(ys, LD, x, L);
+    __syncthreads();
+    {
+        f32x4 u[NF][2];
+        train_product<NF, D / 32>(u, ys, LD, P.packed + train_matrix_at<D, F>(kTm1), 0, L);
+#pragma unroll
+        for (int b = 0; b < NF; ++b) {
+            const f32x4 bias = *reinterpret_cast<const f32x4 *>(P.bias1 + L.col(b));
+#pragma unroll
+            for (int tb = 0; tb < 2; ++tb)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    float h, dh;
+                    train_gelu(u[b][tb][e] + bias[e], h, dh);
+                    u[b][tb][e] = h;
+                }
+        }
+        train_to_lds(as, LF, u, L);
+    }
+    __syncthreads();
+    train_product<NB, F / 32>(acc, as, LF, P.packed + train_matrix_at<D, F>(kTm2), 0, L);
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        const f32x4 bias = *reinterpret_cast<const f32x4 *>(P.bias2 + L.col(b));
+#pragma unroll
+        for (int tb = 0; tb < 2; ++tb) x[b][tb] += acc[b][tb] + bias;
+    }
+    train_store<D>(P.r3, x, L);
+    train_stats<D>(x, red, P.eps3, P.stats3, st, L);
+}
+
+// ---- backward
+
+// Column sums over the token rows of this workgroup's tiles, in LDS: every column belongs to one lane group.
+__device__ __forceinline__ void train_col_add(float *sums, const f32x4 &s, int col, const TrainLane &L) {
+    f32x4 t = s;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        float x = t[e];
+        x += row_rotate<8>(x);
+        x += row_rotate<4>(x);
+        x += row_rotate<2>(x);
+        x += row_rotate<1>(x);
+        t[e] = x;
+    }
+    if (L.tok == 0) *reinterpret_cast<f32x4 *>(sums + col) += t;
+}
+
+// d(sum in front of a norm) from d(its output); column sums of the parameters' gradients.  Rows past the end
+// contribute nothing.  One barrier inside.
+template <int D, int NB>
+__device__ __forceinline__ void train_norm_backward(f32x4 (&d)[NB][2], const f32x4 (&r)[NB][2], const float2 (&st)[2], const float *g,
+                                                    float *sum_g, float *sum_b, float2 *red, const TrainLane &L) {
+    TrainPair s[2] = {{0.f, 0.f}, {0.f, 0.f}};
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        const f32x4 gv = *reinterpret_cast<const f32x4 *>(g + L.col(b));
+        f32x4 cg = {0.f, 0.f, 0.f, 0.f}, cb = cg;
+#pragma unroll
+        for (int tb = 0; tb < 2; ++tb) {
+            if (!L.live(tb)) d[b][tb] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float xh = (r[b][tb][e] - st[tb].x) * st[tb].y, dy = d[b][tb][e];
+                cg[e] = fmaf(dy, xh, cg[e]);
+                cb[e] += dy;
+                const float gy = dy * gv[e];
+                s[tb].a += gy;
+                s[tb].b = fmaf(gy, xh, s[tb].b);
+                d[b][tb][e] = gy;
+            }
+        }
+        train_col_add(sum_g, cg, L.col(b), L);
+        train_col_add(sum_b, cb, L.col(b), L);
+    }
+    train_row_sums(s, red, L);
+#pragma unroll
+    for (int tb = 0; tb < 2; ++tb) {
+        const float m1 = s[tb].a * (1.f / D), m2 = s[tb].b * (1.f / D);
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float xh = (r[b][tb][e] - st[tb].x) * st[tb].y;
+                d[b][tb][e] = st[tb].y * (d[b][tb][e] - m1 - xh * m2);
+            }
+    }
+}
+
+struct TrainBackwardB {
+    const float *dx;           // [M, D] gradient of the layer's output
+    const float *r3; const float2 *stats3; const float *g3;
+    const float *r2; const float2 *stats2; const float *g2, *b2;
+    const float *bias1;
+    const bf16_t *packed;
+    float *dr2;                // [M, D]: gradient of x1 along the residual
+    bf16_t *d3, *x2, *h, *du, *d2, *dattn;  // [M, D], [M, D], [M, F], [M, F], [M, D], [M, D]
+    float *part;               // [gridDim.x][5 D + F]: column sums g3, b3, bias2, g2, b2 (D each), bias1
+    long M;
+};
+
+template <int D, int F>
+__global__ __launch_bounds__(kTrainWaves * 64, 2) void train_backward_b_kernel(TrainBackwardB P) {
+    constexpr int NB = D / 64, NF = F / 64, LD = D + 8, LF = F + 8, NS = 5 * D + F;
+    __shared__ __attribute__((aligned(16))) bf16_t ds[kTrainRows * LD], xs[kTrainRows * LD], us[kTrainRows * LF];
+    __shared__ float2 red[kTrainWaves * kTrainRows];
+    __shared__ __attribute__((aligned(16))) float sums[NS];
+    for (int i = threadIdx.x; i < NS; i += kTrainWaves * 64) sums[i] = 0.f;
+    __syncthreads();
+    const long tiles = (P.M + kTrainRows - 1) / kTrainRows;
+    for (long tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+        const TrainLane L(tile, P.M);
+        const bf16_t *const packed = train_opaque(P.packed);
+        f32x4 d[NB][2], r[NB][2], acc[NB][2];
+        float2 st[2], st2[2];
+        train_load<D>(d, P.dx, L);
+        train_load<D>(r, P.r3, L);
+        train_get_stats(st, P.stats3, L);
+        train_norm_backward<D>(d, r, st, P.g3, sums, sums + D, red, L);
+#pragma unroll
+        for (int b = 0; b < NB; ++b) train_col_add(sums + 2 * D, d[b][0] + d[b][1], L.col(b), L);  // (rows past the end are zero)
+        train_to_lds(ds, LD, d, L);
+        train_load<D>(r, P.r2, L);
+        train_get_stats(st2, P.stats2, L);
+        train_norm(acc, r, st2, P.g2, P.b2, L);
+        train_to_lds(xs, LD, acc, L);
+        __syncthreads();
+        train_unstage<D>(P.d3, D, ds, LD, L.row0, P.M);
+        train_unstage<D>(P.x2, D, xs, LD, L.row0, P.M);
+        {
+            f32x4 u[NF][2], dh[NF][2];
+            train_product<NF, D / 32>(u, xs, LD, packed + train_matrix_at<D, F>(kTm1), 0, L);
+#pragma unroll
+            for (int b = 0; b < NF; ++b) {
+                const f32x4 bias = *reinterpret_cast<const f32x4 *>(P.bias1 + L.col(b));
+#pragma unroll
+                for (int tb = 0; tb < 2; ++tb)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        float hv, dv;
+                        train_gelu(u[b][tb][e] + bias[e], hv, dv);
+                        dh[b][tb][e] = hv;
+                        u[b][tb][e] = dv;
+                    }
+            }
+            train_store16(P.h, F, 0, dh, L);
+            train_product<NF, D / 32>(dh, ds, LD, packed + train_matrix_at<D, F>(kTm2T), 0, L);
+#pragma unroll
+            for (int b = 0; b < NF; ++b) {
+#pragma unroll
+                for (int tb = 0; tb < 2; ++tb) u[b][tb] *= dh[b][tb];
+                train_col_add(sums + 5 * D, u[b][0] + u[b][1], L.col(b), L);
+            }
+            train_to_lds(us, LF, u, L);
+        }
+        __syncthreads();
+        train_unstage<F>(P.du, F, us, LF, L.row0, P.M);
+        train_product<NB, F / 32>(acc, us, LF, packed + train_matrix_at<D, F>(kTm1T), 0, L);
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int tb = 0; tb < 2; ++tb) d[b][tb] += acc[b][tb];
+        train_norm_backward<D>(d, r, st2, P.g2, sums + 3 * D, sums + 4 * D, red, L);
+        train_store<D>(P.dr2, d, L);
+        train_to_lds(ds, LD, d, L);  // (its readers are behind the barrier inside the norm)
+        __syncthreads();
+        train_unstage<D>(P.d2, D, ds, LD, L.row0, P.M);
+        train_product<NB, D / 32>(acc, ds, LD, packed + train_matrix_at<D, F>(kTmOT), 0, L);
+        train_store16(P.dattn, D, 0, acc, L);
+        __syncthreads();
+    }
+    for (int i = threadIdx.x; i < NS; i += kTrainWaves * 64) P.part[static_cast<long>(blockIdx.x) * NS + i] = sums[i];
+}
+
+struct TrainBackwardA {
+    const bf16_t *dqkv;        // [M, 3 D]
+    const float *dr2;
+    const float *r1; const float2 *stats1; const float *g1, *b1;
+    const float *r_prev; const float2 *stats_prev; const float *g_prev, *b_prev;  // as in TrainForwardA
+    const bf16_t *packed;
+    float *dx;                 // [M, D] gradient of the layer's input
+    bf16_t *x1, *d1, *x;       // [M, D] each
+    float *part;               // [gridDim.x][2 D]: column sums g1, b1
+    long M;
+};
+
+template <int D, int F>
+__global__ __launch_bounds__(kTrainWaves * 64, 2) void train_backward_a_kernel(TrainBackwardA P) {
+    constexpr int NB = D / 64, LD = D + 8, LQ = 3 * D + 8, NS = 2 * D;
+    __shared__ __attribute__((aligned(16))) bf16_t qs[kTrainRows * LQ], ds[kTrainRows * LD];
+    __shared__ float2 red[kTrainWaves * kTrainRows];
+    __shared__ __attribute__((aligned(16))) float sums[NS];
+    for (int i = threadIdx.x; i < NS; i += kTrainWaves * 64) sums[i] = 0.f;
+    const long tiles = (P.M + kTrainRows - 1) / kTrainRows;
+    for (long tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+        const TrainLane L(tile, P.M);
+        const bf16_t *const packed = train_opaque(P.packed);
+        f32x4 d[NB][2], r[NB][2], acc[NB][2];
+        float2 st[2];
+        train_stage<3 * D>(qs, LQ, P.dqkv, 3 * D, L.row0, P.M);
+        train_load<D>(d, P.dr2, L);
+        train_load<D>(r, P.r1, L);
+        train_get_stats(st, P.stats1, L);
+        train_norm(acc, r, st, P.g1, P.b1, L);
+        train_store16(P.x1, D, 0, acc, L);
+        __syncthreads();
+        train_product<NB, 3 * D / 32>(acc, qs, LQ, packed + train_matrix_at<D, F>(kTmQkvT), 0, L);
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int tb = 0; tb < 2; ++tb) d[b][tb] += acc[b][tb];
+        train_norm_backward<D>(d, r, st, P.g1, sums, sums + D, red, L);
+        train_to_lds(ds, LD, d, L);
+        train_load<D>(r, P.r_prev, L);
+        if (P.stats_prev) {
+            train_get_stats(st, P.stats_prev, L);
+            train_norm(r, r, st, P.g_prev, P.b_prev, L);
+        }
+        train_store16(P.x, D, 0, r, L);
+        __syncthreads();
+        train_unstage<D>(P.d1, D, ds, LD, L.row0, P.M);
+        train_product<NB, D / 32>(acc, ds, LD, packed + train_matrix_at<D, F>(kTmFoT), 0, L);
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int tb = 0; tb < 2; ++tb) d[b][tb] += acc[b][tb];
+        train_store<D>(P.dx, d, L);
+        __syncthreads();
+    }
+    for (int i = threadIdx.x; i < NS; i += kTrainWaves * 64) P.part[static_cast<long>(blockIdx.x) * NS + i] = sums[i];
+}
+
+// ---- the norm behind the stack, on the rows the head reads (rows first .. R - 1 of every batch entry)
+
+struct TrainFinal {
+    const float *r3; const float2 *stats3; const float *g3, *b3;  // of the last layer
+    const float *g, *b; float eps;                                 // backbone.norm
+    float *z;                  // [B, R - first, D]
+    const float *dz;
+    float *dx;                 // [M, D] gradient of the last layer's output: zero where the head does not read
+    float *part;               // [gridDim.x][2 D]
+    int B, R, first;
+};
+
+// one wavefront per row; lane l holds elements l D/64 ..
+template <int D, bool BACKWARD>
+__global__ __launch_bounds__(256) void train_final_kernel(TrainFinal P) {
+    constexpr int E = D / 64;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    __shared__ float sums[4][2 * D];
+    float cg[E], cb[E], g3[E], b3[E], g[E], be[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        cg[e] = cb[e] = 0.f;
+        g3[e] = P.g3[lane * E + e];
+        b3[e] = P.b3[lane * E + e];
+        g[e] = P.g[lane * E + e];
+        be[e] = P.b[lane * E + e];
+    }
+    const int per = BACKWARD ? P.R : P.R - P.first;
+    const long rows = static_cast<long>(P.B) * per;
+    for (long i = static_cast<long>(blockIdx.x) * 4 + wave; i < rows; i += static_cast<long>(gridDim.x) * 4) {
+        const long b = i / per;
+        const int in = static_cast<int>(i % per), at = BACKWARD ? in : in + P.first;
+        const long m = b * P.R + at;
+        if (BACKWARD && at < P.first) {
+#pragma unroll
+            for (int e = 0; e < E; ++e) P.dx[m * D + lane * E + e] = 0.f;
+            continue;
+        }
+        const float2 st = P.stats3[m];
+        float x[E], s = 0.f;
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            x[e] = fmaf((P.r3[m * D + lane * E + e] - st.x) * st.y, g3[e], b3[e]);
+            s += x[e];
+        }
+        const float mean = wave_sum(s) * (1.f / D);
+        float q = 0.f;
+#pragma unroll
+        for (int e = 0; e < E; ++e) q = fmaf(x[e] - mean, x[e] - mean, q);
+        const float rstd = rsqrtf(wave_sum(q) * (1.f / D) + P.eps);
+        const long zi = (b * (P.R - P.first) + (at - P.first)) * D + lane * E;
+        if (!BACKWARD) {
+#pragma unroll
+            for (int e = 0; e < E; ++e) P.z[zi + e] = fmaf((x[e] - mean) * rstd, g[e], be[e]);
+        } else {
+            float xh[E], gy[E], s1 = 0.f, s2 = 0.f;
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                const float dy = P.dz[zi + e];
+                xh[e] = (x[e] - mean) * rstd;
+                cg[e] = fmaf(dy, xh[e], cg[e]);
+                cb[e] += dy;
+                gy[e] = dy * g[e];
+                s1 += gy[e];
+                s2 = fmaf(gy[e], xh[e], s2);
+            }
+            const float m1 = wave_sum(s1) * (1.f / D), m2 = wave_sum(s2) * (1.f / D);
+#pragma unroll
+            for (int e = 0; e < E; ++e) P.dx[m * D + lane * E + e] = rstd * (gy[e] - m1 - xh[e] * m2);
+        }
+    }
+    if (BACKWARD) {
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            sums[wave][lane * E + e] = cg[e];
+            sums[wave][D + lane * E + e] = cb[e];
+        }
+        __syncthreads();
+        for (int i = threadIdx.x; i < 2 * D; i += 256)
+            P.part[static_cast<long>(blockIdx.x) * 2 * D + i] = (sums[0][i] + sums[1][i]) + (sums[2][i] + sums[3][i]);
+    }
+}
+
+// ---- weight gradients: C[n][k] = sum_m P[m][n] Q[m][k] in pieces of 128 x 128, each over `slices` runs of
+// rows.  Both operands want the contraction (rows) consecutive in a lane: transposing reads of row-major LDS
+// tiles.  Eight wavefronts: two groups take half of a tile's 64 rows each, a group's four hold 64 x 64.
+struct TrainGradJobs {
+    const bf16_t *p[kTrainMaxJobs], *q[kTrainMaxJobs];
+    int ldp[kTrainMaxJobs], ldq[kTrainMaxJobs];
+    float *part;               // [slices][jobs][128 * 128]
+    long M, rows_per_slice;    // a multiple of 64
+    int jobs;
+};
+
+static __global__ __launch_bounds__(512) void train_weight_grad_kernel(TrainGradJobs J) {
+    typedef MfmaOps<bf16_t> Ops;
+    constexpr int TR = 64, LD = 128 + 16;  // 288 bytes: 32 mod 128, what the transposing reads want
+    __shared__ __attribute__((aligned(16))) bf16_t lds[2][2][TR * LD];
+    const int job = blockIdx.x, slice = blockIdx.y;
+    const bf16_t *const p = J.p[job], *const q = J.q[job];
+    const int ldp = J.ldp[job], ldq = J.ldq[job];
+    const long m0 = slice * J.rows_per_slice, m1 = min(J.M, m0 + J.rows_per_slice);
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const int half = wave >> 2, wn = wave & 1, wk = (wave >> 1) & 1;
+    f32x16 acc[2][2];
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) acc[a][c][v] = 0.f;
+    u32x4 rp[2], rq[2];
+    auto fetch = [&](long m) {
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+            const int i = tid + 512 * x, r = i / 16, c = i % 16;
+            const long row = min(m + r, J.M - 1);
+            rp[x] = *reinterpret_cast<const u32x4 *>(p + row * ldp + 8 * c);
+            rq[x] = *reinterpret_cast<const u32x4 *>(q + row * ldq + 8 * c);
+        }
+    };
+    auto put = [&](int buf, long m) {
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+            const int i = tid + 512 * x, r = i / 16, c = i % 16;
+            const u32x4 zero = {0u, 0u, 0u, 0u};
+            *reinterpret_cast<u32x4 *>(&lds[buf][0][r * LD + 8 * c]) = m + r < m1 ? rp[x] : zero;  // rows past the end: no product
+            *reinterpret_cast<u32x4 *>(&lds[buf][1][r * LD + 8 * c]) = rq[x];
+        }
+    };
+    typedef short s16x8 __attribute__((ext_vector_type(8)));
+    // rows m .. m + 15, columns n .. n + 31 as an operand: lane column n + lane % 32, rows m + 8 (lane / 32) + e
+    auto operand = [&](const bf16_t *t, int m, int n) {
+        const bf16_t *a = t + (m + 8 * (lane >> 5) + ((lane & 15) >> 2)) * LD + n + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4 *)(a));
+        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4 *)(a + 4 * LD));
+        const s16x8 both = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+        return __builtin_bit_cast(bf16x8, both);
+    };
+    if (m0 < m1) {
+        fetch(m0);
+        put(0, m0);
+        int buf = 0;
+        for (long m = m0; m < m1; m += TR, buf ^= 1) {
+            const bool more = m + TR < m1;
+            if (more) fetch(m + TR);
+            __syncthreads();
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks) {
+                bf16x8 a[2], c[2];
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    a[i] = operand(lds[buf][0], 32 * half + 16 * ks, 64 * wn + 32 * i);
+                    c[i] = operand(lds[buf][1], 32 * half + 16 * ks, 64 * wk + 32 * i);
+                }
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int j = 0; j < 2; ++j) acc[i][j] = Ops::mma(a[i], c[j], acc[i][j]);
+            }
+            if (more) put(buf ^ 1, m + TR);  // the other buffer's readers passed the barrier above
+        }
+    }
+    // the second group's sums through LDS (64 x 64 floats per wavefront pair would fill it: one quarter at a time)
+    float *const x = reinterpret_cast<float *>(lds);
+    float *const out = J.part + (static_cast<long>(slice) * J.jobs + job) * (128 * 128);
+    const int c32 = lane & 31, hb = lane >> 5;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            __syncthreads();
+            if (half == 1) {
+#pragma unroll
+                for (int v = 0; v < 16; ++v) x[(wave & 3) * 1024 + v * 64 + lane] = acc[i][j][v];
+            }
+            __syncthreads();
+            if (half == 0) {
+#pragma unroll
+                for (int v = 0; v < 16; ++v) {
+                    const int n = 64 * wn + 32 * i + 8 * (v >> 2) + 4 * hb + (v & 3), k = 64 * wk + 32 * j + c32;
+                    out[n * 128 + k] = acc[i][j][v] + x[(wave & 3) * 1024 + v * 64 + lane];
+                }
+            }
+        }
+}
+
+// Adds up the slices of the weight gradients (where each piece goes: `out`, row stride `ld`) and the workgroups'
+// column sums.
+struct TrainReduce {
+    const float *part; int jobs, slices;
+    float *out[kTrainMaxJobs]; int ld[kTrainMaxJobs];
+    struct Cols {
+        const float *part;     // [groups][n]
+        float *out;
+        int groups, n;
+    } cols[2];
+    int n_cols;
+};
+static __global__ __launch_bounds__(256) void train_reduce_kernel(TrainReduce P) {
+    const int tid = threadIdx.x;
+    const int piece_groups = P.jobs * 16;  // 16 workgroups of 1024 elements per piece
+    if (static_cast<int>(blockIdx.x) < piece_groups) {
+        const int job = blockIdx.x / 16, e = (blockIdx.x % 16) * 1024 + 4 * tid;
+        f32x4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
+        for (int i = 0; i < P.slices; ++i) s += *reinterpret_cast<const f32x4 *>(P.part + (static_cast<long>(i) * P.jobs + job) * 16384 + e);
+        *reinterpret_cast<f32x4 *>(P.out[job] + static_cast<long>(e / 128) * P.ld[job] + e % 128) = s;
+        return;
+    }
+    // 64 columns per workgroup, four wavefronts deal the rows
+    __shared__ float acc[4][64];
+    int at = (static_cast<int>(blockIdx.x) - piece_groups) * 64;
+    int which = 0;
+    while (which + 1 < P.n_cols && at >= P.cols[which].n) {
+        at -= P.cols[which].n;
+        ++which;
+    }
+    const TrainReduce::Cols C = P.cols[which];
+    const int wave = tid >> 6, lane = tid & 63;
+    float part[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};  // eight rows on their way at a time
+    const float *col = C.part + at + lane;
+    int i = wave;
+    for (; i + 28 < C.groups; i += 32)
+#pragma unroll
+        for (int u = 0; u < 8; ++u) part[u] += col[static_cast<long>(i + 4 * u) * C.n];
+    for (; i < C.groups; i += 4) part[0] += col[static_cast<long>(i) * C.n];
+    const float s = ((part[0] + part[1]) + (part[2] + part[3])) + ((part[4] + part[5]) + (part[6] + part[7]));
+    acc[wave][lane] = s;
+    __syncthreads();
+    if (wave == 0) C.out[at + lane] = (acc[0][lane] + acc[1][lane]) + (acc[2][lane] + acc[3][lane]);
+}
+
+// ---- row embeddings (model.py:23-76, :323-333): x = mean(features) w_x + b_x + marker, context and buffer rows
+// with y w_y + b_y, buffer rows with their position token
+
+struct TrainEmbed {
+    const float *x[3], *y[2];  // context, buffer, target rows: [B, n, feat] and [B, n]
+    int n[3], feat;
+    const float *w_x, *b_x, *w_y, *b_y, *markers, *tokens;  // markers [3, D]: target, context, buffer; tokens [>= n[1], D]
+    float *out;                // [B, R, D]
+    float2 *xy;                // [B, R] (feature mean, y): what the backward pass needs of the data
+    int B, R;
+};
+template <int D>
+__global__ __launch_bounds__(256) void train_embed_kernel(TrainEmbed P) {
+    constexpr int PER = D / 4;  // threads per row
+    const long i = static_cast<long>(blockIdx.x) * 256 + threadIdx.x, m = i / PER;
+    const int d = 4 * static_cast<int>(i % PER);
+    if (m >= static_cast<long>(P.B) * P.R) return;
+    const long b = m / P.R;
+    int r = static_cast<int>(m % P.R), kind = 0;
+    while (kind < 2 && r >= P.n[kind]) r -= P.n[kind++];
+    const long at = b * P.n[kind] + r;
+    float mean = 0.f;
+    for (int f = 0; f < P.feat; ++f) mean += P.x[kind][at * P.feat + f];
+    mean /= P.feat;
+    const float y = kind < 2 ? P.y[kind][at] : 0.f;
+    f32x4 v = *reinterpret_cast<const f32x4 *>(P.w_x + d) * mean + *reinterpret_cast<const f32x4 *>(P.b_x + d) +
+              *reinterpret_cast<const f32x4 *>(P.markers + (kind == 2 ? 0 : kind + 1) * D + d);
+    if (kind < 2) v += *reinterpret_cast<const f32x4 *>(P.w_y + d) * y + *reinterpret_cast<const f32x4 *>(P.b_y + d);
+    if (kind == 1) v += *reinterpret_cast<const f32x4 *>(P.tokens + static_cast<long>(r) * D + d);
+    *reinterpret_cast<f32x4 *>(P.out + m * D + d) = v;
+    if (d == 0) P.xy[m] = make_float2(mean, y);
+}
+
+// Column sums of dx [B, R, D]: over context rows, buffer rows, target rows, weighted by the feature mean, by y.
+// blockIdx.y < slices: a share of one batch entry's rows -> part[block][5][D];
+// blockIdx.y == slices: the gradient of token blockIdx.x, summed over the batch (blockIdx.x < n_tokens).
+struct TrainEmbedBackward {
+    const float *dx;
+    const float2 *xy;
+    int B, R, n_ctx, n_buf, slices;
+    float *part, *d_tokens;
+};
+template <int D>
+__global__ __launch_bounds__(D) void train_embed_backward_kernel(TrainEmbedBackward P) {
+    const int d = threadIdx.x;
+    if (static_cast<int>(blockIdx.y) == P.slices) {
+        const int j = blockIdx.x;
+        if (j >= P.n_buf) return;
+        float s = 0.f;
+        for (int b = 0; b < P.B; ++b) s += P.dx[(static_cast<long>(b) * P.R + P.n_ctx + j) * D + d];
+        P.d_tokens[static_cast<long>(j) * D + d] = s;
+        return;
+    }
+    const long b = blockIdx.x;
+    if (b >= P.B) return;
+    float s[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+    for (int r = blockIdx.y; r < P.R; r += P.slices) {
+        const float v = P.dx[(b * P.R + r) * D + d];
+        const float2 xy = P.xy[b * P.R + r];
+        const int kind = r < P.n_ctx ? 0 : r < P.n_ctx + P.n_buf ? 1 : 2;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) s[k] += k == kind ? v : 0.f;
+        s[3] = fmaf(v, xy.x, s[3]);
+        s[4] = fmaf(v, xy.y, s[4]);
+    }
+#pragma unroll
+    for (int k = 0; k < 5; ++k) P.part[((b * P.slices + blockIdx.y) * 5 + k) * D + d] = s[k];
+}
+// sums [5][D] -> d(w_x), d(b_x), d(w_y), d(b_y) [D] each, d(markers) [3, D]
+static __global__ void train_embed_finish_kernel(const float *sums, float *grads, int D) {
+    const int d = threadIdx.x;
+    const float ctx = sums[d], buf = sums[D + d], tgt = sums[2 * D + d];
+    grads[d] = sums[3 * D + d];
+    grads[D + d] = ctx + buf + tgt;
+    grads[2 * D + d] = sums[4 * D + d];
+    grads[3 * D + d] = ctx + buf;
+    grads[4 * D + d] = tgt;
+    grads[5 * D + d] = ctx;
+    grads[6 * D + d] = buf;
+}
+
+}  // namespace artab

@@ -26,9 +26,25 @@ from torch import Tensor, nn
 from .attention import DenseMask, MultiheadAttention, RowMask
 from .glue import add_layer_norm, bias_gelu, layer_fusable, layer_post, layer_post_pre, layer_pre, pack_weight
 
+from .training import embed_rows, layer_stack, layer_stack_supported
+
 __all__ = ["Embedder", "TwoStageTransformerLayer", "TwoStageTransformer", "MixtureGaussianHead", "ARTabPFN"]
 
 _MARKERS = {"target": 0, "context": 1, "buffer": 2}  # model.py:36-38
+
+
+class _ZeroGradients(torch.autograd.Function):
+    """``z`` unchanged; the parameters given with it get gradients of zero."""
+
+    @staticmethod
+    def forward(ctx, z, *params):
+        ctx.shapes = [(p.shape, p.dtype, p.device) for p in params]
+        return z.view_as(z)
+
+    @staticmethod
+    def backward(ctx, grad):
+        flat = torch.zeros(sum(s.numel() for s, _, _ in ctx.shapes), dtype=ctx.shapes[0][1], device=ctx.shapes[0][2])
+        return (grad, *(t.view(s) for t, (s, _, _) in zip(flat.split([s.numel() for s, _, _ in ctx.shapes]), ctx.shapes)))
 
 
 class Embedder(nn.Module):
@@ -328,13 +344,22 @@ class ARTabPFN(nn.Module):
         directions: ``loss.backward()`` gives every parameter its gradient, as in the reference's
         training step (train.py:289-300).  Under ``torch.no_grad()`` the layers take the fused
         inference kernels instead."""
-        ctx_emb = self.embedder.embed_context(x_context, y_context)
-        buf_emb = self.embedder.embed_buffer(x_buffer, y_buffer) + self.ar_tokens[: x_buffer.size(1)]
-        tgt_emb = self.embedder.embed_target(x_target)
-        Nc, Nb = ctx_emb.size(1), buf_emb.size(1)
-        embeddings = torch.cat([ctx_emb, buf_emb, tgt_emb], dim=1).unsqueeze(2)
-        z, _ = self.backbone(embeddings, mask_features, mask_rows)
-        z_target = z[:, Nc + Nb:, 0, :]
+        Nc, Nb = x_context.size(1), x_buffer.size(1)
+        embeddings = embed_rows(self, x_context, y_context, x_buffer, y_buffer, x_target) if torch.is_grad_enabled() else None
+        if embeddings is None:
+            ctx_emb = self.embedder.embed_context(x_context, y_context)
+            buf_emb = self.embedder.embed_buffer(x_buffer, y_buffer) + self.ar_tokens[:Nb]
+            embeddings = torch.cat([ctx_emb, buf_emb, self.embedder.embed_target(x_target)], dim=1)
+        if layer_stack_supported(self.backbone, embeddings, mask_rows, Nc + Nb):
+            z_target = layer_stack(self.backbone, embeddings, mask_rows, Nc + Nb)
+            # q_proj and k_proj of the feature attention do not enter (one key per query); they get the exact
+            # zero gradients autograd gives them in the reference
+            unused = [p for layer in self.backbone.layers
+                      for p in (layer.attn_features.q_proj.weight, layer.attn_features.k_proj.weight)]
+            z_target = _ZeroGradients.apply(z_target, *unused)
+        else:
+            z, _ = self.backbone(embeddings.unsqueeze(2), mask_features, mask_rows)
+            z_target = z[:, Nc + Nb:, 0, :]
         if y_target is not None and y_target.dim() == 2:
             y_target = y_target.unsqueeze(-1)
         loss, _, _, _ = self.head(z_target, y_target)

@@ -1,0 +1,166 @@
+"""The layer stack of a training step on the device kernels (``artab_train_forward`` / ``_backward``): what
+``TwoStageTransformer.forward`` and the final norm record under bfloat16 autocast (model.py:100-147, :317-369;
+train.py:289-300), as one differentiable call.
+
+The residual stream, the norms and every sum stay float32; products take bfloat16 operands, as autocast's do.
+"""
+
+from __future__ import annotations
+
+import ctypes
+
+import torch
+from torch import Tensor
+
+from . import _lib
+from . import attention_kernels as ak
+from .attention import RowMask
+
+__all__ = ["embed_rows", "layer_stack_supported", "layer_stack"]
+
+# A program that has put callables of its own in their place gets the modules, which call them.
+_attention_calls = (ak.row_mask_attention, ak.row_mask_attention_backward)
+
+
+def _layer_params(layer):
+    """The parameters of a layer in the order of ``artab_train_args.params``."""
+    af, ar = layer.attn_features, layer.attn_rows
+    return (af.v_proj.weight, af.out_proj.weight, ar.q_proj.weight, ar.k_proj.weight, ar.v_proj.weight, ar.out_proj.weight,
+            layer.ff[0].weight, layer.ff[0].bias, layer.ff[2].weight, layer.ff[2].bias, layer.norm1.weight, layer.norm1.bias,
+            layer.norm2.weight, layer.norm2.bias, layer.norm3.weight, layer.norm3.bias)
+
+
+def _args(backbone, B: int, R: int, mask: RowMask, first_row: int) -> "_lib.ArtabTrainArgs":
+    layer = backbone.layers[0]
+    a = _lib.ArtabTrainArgs()
+    a.B, a.R, a.H, a.D, a.F = B, R, layer.attn_rows.n_heads, backbone.d_model, layer.ff[0].out_features
+    a.n_layers, a.first_row = len(backbone.layers), first_row
+    a.context_len, a.buffer_len, a.attending_chunks = mask.context_len, mask.buffer_len, mask.attending_chunks
+    a.eps1, a.eps2, a.eps3, a.eps_out = layer.norm1.eps, layer.norm2.eps, layer.norm3.eps, backbone.norm.eps
+    return a
+
+
+def layer_stack_supported(backbone, x: Tensor, mask, first_row: int) -> bool:
+    """True when ``layer_stack`` computes what the modules would: gradients are being recorded under bfloat16
+    autocast, float32 parameters, widths the kernels are built for, equal layers."""
+    if not (x.is_cuda and x.dtype == torch.float32 and torch.is_grad_enabled() and isinstance(mask, RowMask)
+            and torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") == torch.bfloat16
+            and (ak.row_mask_attention, ak.row_mask_attention_backward) == _attention_calls):
+        return False
+    layers = list(backbone.layers)
+    if not layers or x.shape[1] != mask.num_rows:
+        return False
+    first = layers[0]
+
+    def same(layer):
+        return (layer.attn_rows.n_heads == first.attn_rows.n_heads and layer.ff[0].out_features == first.ff[0].out_features
+                and all(getattr(layer, n).eps == getattr(first, n).eps for n in ("norm1", "norm2", "norm3"))
+                and all(p is not None and p.dtype == torch.float32 and p.device == x.device and p.is_contiguous()
+                        and p.data_ptr() % 16 == 0 for p in _layer_params(layer)))
+
+    return (all(same(layer) for layer in layers)
+            and _lib.load().artab_train_saved_bytes(ctypes.byref(_args(backbone, x.shape[0], x.shape[1], mask, first_row))) > 0)
+
+
+def _f32(*tensors) -> bool:
+    return all(t is not None and t.is_cuda and t.dtype == torch.float32 and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in tensors)
+
+
+class _Embed(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, xc, yc, xb, yb, xt, w_x, b_x, w_y, b_y, markers, tokens):
+        a = _lib.ArtabTrainEmbedArgs()
+        B, a.feat, a.D = xc.shape[0], xc.shape[2], markers.shape[1]
+        a.B, a.n_context, a.n_buffer, a.n_target = B, xc.shape[1], xb.shape[1], xt.shape[1]
+        R = a.n_context + a.n_buffer + a.n_target
+        out = torch.empty((B, R, a.D), device=xc.device, dtype=torch.float32)
+        xy = torch.empty((B, R, 2), device=xc.device, dtype=torch.float32)
+        for name, t in zip(("x_context", "y_context", "x_buffer", "y_buffer", "x_target", "w_x", "b_x", "w_y", "b_y", "markers",
+                            "tokens", "out", "xy"), (xc, yc, xb, yb, xt, w_x, b_x, w_y, b_y, markers, tokens, out, xy)):
+            setattr(a, name, t.data_ptr())
+        _lib.check(_lib.load().artab_train_embed(ctypes.byref(a), _lib.current_stream(xc.device)))
+        ctx.args, ctx.xy, ctx.shapes = a, xy, (w_x.shape, w_y.shape, tokens.shape)
+        return out
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, dx):
+        lib, a = _lib.load(), ctx.args
+        dx = dx.contiguous()
+        D, n = a.D, ctx.shapes[2][0]
+        grads = torch.empty((7 + n) * D, device=dx.device, dtype=torch.float32)
+        if n > a.n_buffer:  # tokens behind the buffer rows take no part
+            grads[(7 + a.n_buffer) * D :].zero_()
+        scratch = torch.empty(lib.artab_train_embed_scratch_bytes(ctypes.byref(a)), device=dx.device, dtype=torch.uint8)
+        a.out, a.grads, a.scratch = dx.data_ptr(), grads.data_ptr(), scratch.data_ptr()
+        _lib.check(lib.artab_train_embed_backward(ctypes.byref(a), _lib.current_stream(dx.device)))
+        w_x, b_x, w_y, b_y, markers, tokens = grads.split((D, D, D, D, 3 * D, n * D))
+        return (None,) * 5 + (w_x.view(ctx.shapes[0]), b_x, w_y.view(ctx.shapes[1]), b_y, markers.view(3, D), tokens.view(n, D))
+
+
+def embed_rows(model, x_context, y_context, x_buffer, y_buffer, x_target):
+    """The embedded rows ``[B,R,D]`` of ``ARTabPFN.forward``, or None where the kernel does not apply (the data
+    itself wants gradients, types or widths it is not built for)."""
+    e = model.embedder
+    params = (e.x_embed.weight, e.x_embed.bias, e.y_embed.weight, e.y_embed.bias, e.marker_embed.weight, model.ar_tokens)
+    data = [t.contiguous() for t in (x_context, y_context, x_buffer, y_buffer, x_target)]
+    xs, ys = data[0::2], data[1::2]
+    if not (_f32(*data, *params) and not any(t.requires_grad for t in data) and model.d_model in (128, 256)
+            and torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") == torch.bfloat16
+            and all(t.dim() == 3 and t.shape[2] == xs[0].shape[2] and t.shape[0] == xs[0].shape[0] for t in xs)
+            and all(y.numel() == x.shape[0] * x.shape[1] for x, y in zip(xs, ys))
+            and xs[0].shape[1] >= 1 and xs[2].shape[1] >= 1 and xs[1].shape[1] <= model.ar_tokens.shape[0]):
+        return None
+    return _Embed.apply(*data, *params)
+
+
+class _LayerStack(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, x, backbone, mask, first_row, *params):
+        lib = _lib.load()
+        B, R, D = x.shape
+        x = x.contiguous()
+        a = _args(backbone, B, R, mask, first_row)
+        n = 16 * a.n_layers
+        pointers = (ctypes.c_void_p * n)(*(p.data_ptr() for p in params[:n]))
+        saved = torch.empty(lib.artab_train_saved_bytes(ctypes.byref(a)), device=x.device, dtype=torch.uint8)
+        z = torch.empty((B, R - first_row, D), device=x.device, dtype=torch.float32)
+        a.x, a.params = x.data_ptr(), ctypes.cast(pointers, ctypes.c_void_p)
+        a.norm_gamma, a.norm_beta = params[n].data_ptr(), params[n + 1].data_ptr()
+        a.saved, a.z = saved.data_ptr(), z.data_ptr()
+        _lib.check(lib.artab_train_forward(ctypes.byref(a), _lib.current_stream(x.device)))
+        ctx.args, ctx.pointers, ctx.saved = a, pointers, saved
+        ctx.save_for_backward(x, *params)
+        return z
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, dz):
+        lib = _lib.load()
+        x, *params = ctx.saved_tensors  # (raises if one of them was changed in place since)
+        a = ctx.args
+        D, F, L = a.D, a.F, a.n_layers
+        dz = dz.contiguous().float()
+        scratch = torch.empty(lib.artab_train_scratch_bytes(ctypes.byref(a)), device=x.device, dtype=torch.uint8)
+        dx = torch.empty_like(x)
+        sizes = (D * D,) * 5 + (F * D, D * F) + (D,) * 5 + (F,) + (D,) * 2 + (D * D,) * 2
+        total = sum(sizes)
+        grads = torch.empty(L * total + 2 * D, device=x.device, dtype=torch.float32)
+        a.dz, a.dx, a.grads, a.scratch = dz.data_ptr(), dx.data_ptr(), grads.data_ptr(), scratch.data_ptr()
+        _lib.check(lib.artab_train_backward(ctypes.byref(a), _lib.current_stream(x.device)))
+        out = []
+        for i in range(L):
+            q, k, v, _, o, w1, w2, g3, b3, bias2, g2, b2, bias1, g1, b1, f_out, f_v = grads[i * total : (i + 1) * total].split(sizes)
+            square = lambda t: t.view(D, D)  # noqa: E731
+            out += [square(f_v), square(f_out), square(q), square(k), square(v), square(o), w1.view(F, D), bias1, w2.view(D, F), bias2,
+                    g1, b1, g2, b2, g3, b3]
+        out += [grads[L * total : L * total + D], grads[L * total + D :]]
+        return (dx, None, None, None, *out)
+
+
+def layer_stack(backbone, x: Tensor, mask: RowMask, first_row: int) -> Tensor:
+    """``backbone`` on the rows ``x [B,R,D]`` under the training row mask: the final norm's output of rows
+    ``first_row`` and on, ``[B, R - first_row, D]``, differentiable in ``x`` and every parameter that takes part.
+    The feature attention's q and k projections do not (one key per query: the softmax weight is 1)."""
+    params = [p for layer in backbone.layers for p in _layer_params(layer)]
+    return _LayerStack.apply(x, backbone, mask, first_row, *params, backbone.norm.weight, backbone.norm.bias)

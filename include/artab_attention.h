@@ -497,6 +497,57 @@ typedef struct artab_sample_embed_args {
 int artab_decode_sample_embed(const artab_sample_embed_args *args, int dtype, void *stream);
 
 /*
+ * The layer stack of a training step around the row attention (model.py:100-126, :317-369 under the bf16
+ * autocast of train.py:289-300), forward and backward: B x R rows [context | buffer | target], float32
+ * parameters and residual stream, bf16 products with float32 sums.  D in {128, 256}, F = 256, head_dim 32
+ * or 64; anything else: artab_train_saved_bytes returns 0.
+ *   forward:  x [B R, D] -> z [B, R - first_row, D] = norm(output of the last layer) of rows first_row ..;
+ *             fills `saved` (artab_train_saved_bytes, kept by the caller for the backward call).
+ *   backward: dz -> dx [B R, D] and `grads` (float32): per layer dW_qkv [3D, D], dW_fo [D, D] (scratch),
+ *             dW_o [D, D], dW_1 [F, D], dW_2 [D, F], d(norm3 g, b, ff bias 2, norm2 g, b) [D] each,
+ *             d(ff bias 1) [F], d(norm1 g, b) [D] each, dW_out [D, D], dW_v [D, D] of the feature
+ *             attention; behind the layers d(norm g, b) [D] each.
+ * `params` is a HOST array of n_layers x 16 device pointers: feature attention W_v, W_out; row attention
+ * W_q, W_k, W_v, W_o; ff W_1, b_1, W_2, b_2; norm1 g, b; norm2 g, b; norm3 g, b.  16-byte aligned, contiguous.
+ */
+typedef struct artab_train_args {
+    int B, R, H, D, F, n_layers, context_len, buffer_len, attending_chunks, first_row;
+    float eps1, eps2, eps3, eps_out;
+    const float *x;
+    const float *const *params;
+    const float *norm_gamma, *norm_beta;
+    void *saved;
+    float *z;
+    const float *dz;
+    float *dx, *grads;
+    void *scratch;           /* artab_train_scratch_bytes, backward only */
+} artab_train_args;
+
+size_t artab_train_saved_bytes(const artab_train_args *args);
+size_t artab_train_scratch_bytes(const artab_train_args *args);
+int artab_train_forward(const artab_train_args *args, void *stream);
+int artab_train_backward(const artab_train_args *args, void *stream);
+
+/*
+ * The row embeddings in front of that stack (model.py:23-76, :323-333), float32, D in {128, 256}:
+ * mean(features) w_x + b_x + marker, context and buffer rows with y w_y + b_y, buffer rows with tokens[j].
+ *   forward:  out [B, n_context + n_buffer + n_target, D]; xy (two floats per row) is kept for the backward call
+ *   backward: `out` holds d(out); grads: d(w_x), d(b_x), d(w_y), d(b_y) [D] each, d(markers) [3, D],
+ *             d(tokens) [n_buffer, D]
+ */
+typedef struct artab_train_embed_args {
+    int B, n_context, n_buffer, n_target, feat, D;
+    const float *x_context, *y_context, *x_buffer, *y_buffer, *x_target; /* [B, n, feat], [B, n], contiguous */
+    const float *w_x, *b_x, *w_y, *b_y, *markers, *tokens;
+    float *out, *xy;
+    float *grads;
+    void *scratch;           /* artab_train_embed_scratch_bytes, backward only */
+} artab_train_embed_args;
+size_t artab_train_embed_scratch_bytes(const artab_train_embed_args *args);
+int artab_train_embed(const artab_train_embed_args *args, void *stream);
+int artab_train_embed_backward(const artab_train_embed_args *args, void *stream);
+
+/*
  * A whole sampling run in one launch: every workgroup takes a few trajectories through all Nt steps
  * and all layers of the model (inference.py:278-320, :353-366 with the layers of :687-744 or
  * :746-833).  Contexts are in the caches; the buffer rows are appended there as the run goes.

@@ -1,0 +1,52 @@
+"""``ARTabPFN.forward`` under bfloat16 autocast on the fused training kernels (embedding, layer stack) against the
+same model as PyTorch modules around the device row attention: loss and every parameter gradient."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+# edges: one row tile and one row past it, no whole 64-row piece for the weight gradients, one layer, one buffer row,
+# one feature, both widths and head dims, tokens that take no part, more tiles than workgroups of a backward kernel
+@pytest.mark.parametrize("D,H,L,B,Nc,Nb,Nt,feat,tokens", [
+    (128, 4, 1, 1, 16, 1, 15, 1, 1), (128, 4, 2, 3, 17, 4, 12, 2, 6), (128, 2, 2, 5, 40, 8, 100, 3, 8),
+    (256, 8, 2, 2, 33, 5, 61, 10, 32), (256, 4, 1, 7, 64, 16, 129, 2, 16), (128, 4, 1, 33, 300, 32, 512, 2, 32)])
+def test_fused_training_equals_modules(device, monkeypatch, D, H, L, B, Nc, Nb, Nt, feat, tokens):
+    import ar_nanotabpfn_amd.model as model_mod
+    from ar_nanotabpfn_amd.attention import create_dense_mask, create_row_mask
+
+    torch.manual_seed(1)
+    model = model_mod.ARTabPFN(d_model=D, n_heads=H, n_layers=L, d_ff=256, num_features=feat, buffer_size=tokens, num_components=5)
+    with torch.no_grad():
+        for name, p in model.named_parameters():
+            if "norm" in name or name.endswith("bias"):
+                p.add_(0.1 * torch.randn_like(p))
+    model = model.to(device)
+    g = torch.Generator().manual_seed(2)
+    mk = lambda *s: torch.randn(*s, generator=g).to(device)  # noqa: E731
+    data = (mk(B, Nc, feat), mk(B, Nc), mk(B, Nb, feat), mk(B, Nb), mk(B, Nt, feat))
+    y = mk(B, Nt)
+    masks = (create_dense_mask(1), create_row_mask(Nc + Nb + Nt, Nc, Nb))
+
+    def step():
+        model.zero_grad(set_to_none=True)
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            loss = model(*data, *masks, y_target=y)
+        loss.backward()
+        return loss.item(), {n: p.grad for n, p in model.named_parameters()}
+
+    calls = []
+    monkeypatch.setattr(model_mod, "layer_stack", lambda *a, f=model_mod.layer_stack: calls.append(1) or f(*a))
+    loss, grads = step()
+    assert calls, "the fused route was not taken"
+    loss2, grads2 = step()
+    assert loss == loss2 and all(torch.equal(grads[n], grads2[n]) for n in grads if "head" not in n)
+    monkeypatch.setattr(model_mod, "layer_stack_supported", lambda *a: False)
+    monkeypatch.setattr(model_mod, "embed_rows", lambda *a: None)
+    ref_loss, ref = step()
+    assert abs(loss - ref_loss) <= 5e-3 * abs(ref_loss)
+    for n, r in ref.items():
+        assert grads[n].shape == r.shape and torch.isfinite(grads[n]).all()
+        # (both sides round every product operand to eight bits: a per cent or two for the smallest gradients)
+        assert float((grads[n] - r).norm()) <= 4e-2 * float(r.norm()) + 1e-6, n
