@@ -12,11 +12,13 @@ the duration of a ``with`` block.  Only ``bench.py`` does that.
 from __future__ import annotations
 
 import ctypes
+import importlib
 import os
 from typing import Optional
 
 import torch
 
+native = None  # the module _native.so, once the library is loaded
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libartab_attention.so")
 BENCH_LIB_PATH = os.path.join(_HERE, "libartab_bench.so")
@@ -237,7 +239,21 @@ def load() -> ctypes.CDLL:
         return _lib
     _product_lib = _open(LIB_PATH, SIGNATURES)
     _lib = _product_lib
+    _bind_native(_lib)
     return _lib
+
+
+def _bind_native(lib: ctypes.CDLL) -> None:
+    """The native call module works through the library that is in use."""
+    global native
+    if native is None:
+        try:
+            native = importlib.import_module("._native", __package__)
+        except ImportError as err:
+            raise RuntimeError(f"ar_nanotabpfn_amd/_native.so cannot be loaded ({err}); "
+                               "build it with `python -m ar_nanotabpfn_amd.build_ext`") from err
+    native.bind({name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in SIGNATURES},
+                lambda index, nbytes: workspace(torch.device("cuda", index), nbytes))
 
 
 class benchmark_library:
@@ -252,11 +268,13 @@ class benchmark_library:
         if _bench_lib is None:
             _bench_lib = _open(BENCH_LIB_PATH, {**SIGNATURES, **BENCH_SIGNATURES})
         _lib = _bench_lib
+        _bind_native(_lib)
         return _bench_lib
 
     def __exit__(self, *exc):
         global _lib
         _lib = _product_lib
+        _bind_native(_lib)
         return False
 
 

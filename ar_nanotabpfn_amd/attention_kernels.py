@@ -61,6 +61,13 @@ def _impl(use_triton: bool) -> int:
     return _lib.IMPL_AUTO if use_triton else _lib.IMPL_PORTABLE
 
 
+def _call(name: str, *args):
+    """The native form of a call, or None where it leaves the call to the path below it."""
+    if _lib._lib is None:
+        _lib.load()
+    return getattr(_lib.native, name)(*args)
+
+
 def _alloc_out(q: Tensor) -> Tensor:
     """Output ``[B,H,Lq,Dh]`` backed by ``[B,Lq,H,Dh]`` storage, so the caller's
     ``out.transpose(1, 2).reshape(B, Lq, H*Dh)`` (inference.py:825) is a free view."""
@@ -93,6 +100,9 @@ def context_attention(
     :532-567) or ``[B,H,Nc,D]`` per dataset.  Returns ``out [B,H,Lq,D]`` (q's dtype)
     and ``lse [B,H,Lq]`` float32.
     """
+    done = _call("context_attention", q, k_ctx, v_ctx, scale, _impl(use_triton))
+    if done is not None:
+        return done
     dev = _lib.require_device(q, k_ctx, v_ctx)
     lib = _lib.load()
     B, H, Lq, Dh = q.shape
@@ -254,6 +264,10 @@ def decode_attention(
     and returns an ``AttentionPartials`` for ``glue.layer_post`` / ``layer_post_pre`` to merge
     while they load their input; where it does not, the merged tensor is returned as usual.
     """
+    if side_stream is None and not leave_partials and order is None and n_buf_device is None:
+        done = _call("decode_attention", q, k_ctx, v_ctx, k_buf_cache, v_buf_cache, n_buf, k_new, v_new, _impl(use_triton))
+        if done is not None:
+            return done
     dev = _lib.require_device(q, k_ctx, v_ctx, k_buf_cache, v_buf_cache, k_new, v_new)
     lib = _lib.load()
     B, H, Lq, Dh = q.shape

@@ -24,6 +24,7 @@ CSRC = os.path.join(HERE, "csrc")
 OBJ_DIR = os.path.join(CSRC, "build")
 OUT = os.path.join(HERE, "libartab_attention.so")
 OUT_BENCH = os.path.join(HERE, "libartab_bench.so")
+OUT_NATIVE = os.path.join(HERE, "_native.so")  # Python module: host side of the most frequent calls
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",
@@ -79,6 +80,22 @@ def _run(cmd, verbose):
         print(log)
 
 
+def native_command():
+    """The host-only extension module (C++, no device code) that calls the C ABI with torch tensors."""
+    import sysconfig
+
+    import torch
+
+    base = os.path.dirname(torch.__file__)
+    inc = [os.path.join(base, "include"), os.path.join(base, "include", "torch", "csrc", "api", "include"), "/opt/rocm/include",
+           sysconfig.get_paths()["include"]]
+    libdir = os.path.join(base, "lib")
+    return ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-w", *[f"-I{i}" for i in inc],
+            os.path.join(CSRC, "native_calls.cpp"), "-o", OUT_NATIVE + ".tmp", f"-L{libdir}", f"-Wl,-rpath,{libdir}",
+            "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip"]
+
+
 def build(verbose: bool = True, jobs: int = 0) -> str:
     """Compile every translation unit from source (every time it is called) and link the two
     libraries; returns the path of the drop-in library."""
@@ -93,7 +110,8 @@ def build(verbose: bool = True, jobs: int = 0) -> str:
     cmds = [[hipcc, *HIPCC_FLAGS, *defs, "-c", os.path.join(CSRC, src), "-o", os.path.join(OBJ_DIR, o)]
             for src, defs, o in units]
     with ThreadPoolExecutor(max_workers=jobs) as pool:
-        list(pool.map(lambda c: _run(c, verbose), cmds))
+        list(pool.map(lambda c: _run(c, verbose), [native_command(), *cmds]))
+    os.replace(OUT_NATIVE + ".tmp", OUT_NATIVE)
     exports = os.path.join(OBJ_DIR, "exports.map")
     with open(exports, "w") as f:
         f.write(EXPORTS)
