@@ -47,7 +47,7 @@ HIPCC_FLAGS = [
 EXPORTS = "{ global: artab_*; local: *; };\n"
 
 # (source, extra defines, object name)
-UNITS = [("artab_api.hip", [], "artab_api.o"), ("flash_launch.hip", [], "flash_launch.o"),
+UNITS = [("artab_api.hip", [], "artab_api.o"), ("flash_launch.hip", [], "flash_launch.o"), ("f32_launch.hip", [], "f32_launch.o"),
          ("backward_launch.hip", [], "backward_launch.o"), ("train_launch.hip", [], "train_launch.o")]
 # objects that differ between the two libraries
 PRODUCT_ONLY = [("launch_observer_none.hip", [], "launch_observer_none.o")]

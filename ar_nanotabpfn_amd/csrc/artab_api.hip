@@ -124,6 +124,8 @@ static inline bool mfma_shape_ok(int dtype, int Dh) {
     return (dtype == ARTAB_BF16 || dtype == ARTAB_F16) && (Dh == 32 || Dh == 64 || Dh == 128);
 }
 
+static inline bool f32_shape_ok(int dtype, int Dh) { return dtype == ARTAB_F32 && (Dh == 32 || Dh == 64 || Dh == 128); }
+
 // ---------------------------------------------------------------------------------------------
 // Flash (MFMA) launch planning
 // ---------------------------------------------------------------------------------------------
@@ -286,6 +288,19 @@ static hipError_t launch_portable_dtype(const PortableParams &P, int dtype, hipS
     }
 }
 
+// Float32 calls that the matrix-core kernel takes go there, everything else to the portable kernel.  The
+// kernel addresses a run of rows with 32-bit byte offsets and stores new rows as 16-byte pieces.
+static hipError_t launch_portable_or_f32(const PortableParams &P, int dtype, int impl, bool stacked, hipStream_t stream,
+                                         void *workspace = nullptr, size_t workspace_bytes = 0) {
+    const auto fits = [](int64_t stride, int64_t rows) { return stride >= 0 && stride * rows < (1LL << 29); };
+    const long buf_rows = P.nbuf_dev ? P.capacity : P.Nb;
+    if (impl != ARTAB_IMPL_PORTABLE && f32_shape_ok(dtype, P.Dh) && P.vec_ok && P.mode != kModeMasked && fits(P.kc.sn, P.Nc) &&
+        fits(P.vc.sn, P.Nc) && fits(P.kb.sn, buf_rows) && fits(P.vb.sn, buf_rows) && (P.new_row < 0 || !stacked || (fits(P.knew.sb, 64) && fits(P.vnew.sb, 64))) &&
+        static_cast<long>(P.B) * P.Lq < (1L << 30))
+        return launch_f32_attention(P, stacked, workspace, workspace_bytes, stream);
+    return launch_portable_dtype(P, dtype, stream);
+}
+
 // Combine split-context partials of arbitrary Lq into the final output: one thread
 // per (row, 4 output elements).
 struct CombineParams {
@@ -420,7 +435,12 @@ int artab_tuning_get(const char *name, int *value) {
 }
 
 size_t artab_workspace_bytes(int B, int H, int Lq, int Nc, int Dh, int dtype) {
-    if (B <= 0 || H <= 0 || Lq <= 0 || Nc <= 0 || !mfma_shape_ok(dtype, Dh)) return 0;
+    if (B <= 0 || H <= 0 || Lq <= 0 || Nc <= 0) return 0;
+    if (f32_shape_ok(dtype, Dh)) {  // (optional: without it the keys are not split)
+        const int n = plan_f32(H, Nc, Dh, B * Lq, 1).n_split, m = plan_f32(H, Nc, Dh, Lq, B).n_split;
+        return n > 1 || m > 1 ? f32_workspace_bytes(static_cast<long>(B) * H * Lq, Dh, n > m ? n : m) : 0;
+    }
+    if (!mfma_shape_ok(dtype, Dh)) return 0;
     // Upper bound over the two schedules (queries stacked over a shared context, or
     // grouped per batch entry over per-dataset contexts).
     FlashPlan a = plan_flash(B, H, Lq, Nc, Dh, /*stacked=*/true, /*allow_split=*/true);
@@ -457,7 +477,7 @@ int artab_context_attention(const artab_view *q, const artab_view *k_ctx, const 
         P.B = B; P.H = H; P.Lq = Lq; P.Nc = Nc; P.Nb = 0;
         P.new_row = -1; P.mode = kModePlain; P.Dh = Dh; P.scale = scale;
         P.vec_ok = aligned ? 1 : 0;
-        return launch_status(launch_portable_dtype(P, dtype, st), "context attention (portable)");
+        return launch_status(launch_portable_or_f32(P, dtype, impl, (k_ctx->stride_b == 0 && v_ctx->stride_b == 0) || B == 1, st, workspace, workspace_bytes), "context attention");
     }
 
     const bool stacked = (k_ctx->stride_b == 0 && v_ctx->stride_b == 0) || B == 1;
@@ -651,7 +671,7 @@ static int decode_impl(const artab_view *q, const artab_view *k_ctx, const artab
         P.capacity = buf_capacity;
         P.mode = kModePlain; P.Dh = Dh; P.scale = scale;
         P.vec_ok = aligned ? 1 : 0;
-        return launch_status(launch_portable_dtype(P, dtype, st), "decode attention (portable)");
+        return launch_status(launch_portable_or_f32(P, dtype, impl, shared_ctx, st, workspace, workspace_bytes), "decode attention");
     }
 
     FlashParams F;
@@ -876,7 +896,7 @@ int artab_decode_attention_static(const artab_view *q, const artab_view *k_ctx, 
                                   int dtype, int impl, void *stream) {
     // the bound that artab_workspace_bytes gives callers of artab_decode_attention
     const size_t need = artab_workspace_bytes(B, H, Lq, Nc, Dh, dtype);
-    if (need > static_cast<size_t>(ARTAB_STATIC_SCRATCH_BYTES))
+    if (need > static_cast<size_t>(ARTAB_STATIC_SCRATCH_BYTES) && dtype != ARTAB_F32)  // (optional for float32)
         return fail(ARTAB_ERR_WORKSPACE,
                     "artab_decode_attention_static: this problem needs %zu bytes of scratch, the built-in array holds "
                     "%zu; use artab_decode_attention with a workspace of your own",
@@ -956,7 +976,7 @@ int artab_teacher_forcing_attention(const artab_view *q, const artab_view *k_ctx
         P.B = B; P.H = H; P.Lq = Lq; P.Nc = Nc; P.Nb = Nt; P.Nt = Nt;
         P.new_row = -1; P.mode = kModeTeacher; P.Dh = Dh; P.scale = scale;
         P.vec_ok = aligned ? 1 : 0;
-        return launch_status(launch_portable_dtype(P, dtype, st), "teacher forcing (portable)");
+        return launch_status(launch_portable_or_f32(P, dtype, impl, false, st), "teacher forcing");
     }
     FlashPlan pl = plan_flash(B, H, Lq, Nc, Dh, /*stacked=*/false, /*allow_split=*/false);
     FlashParams F;
@@ -1010,7 +1030,7 @@ int artab_row_mask_attention(const artab_view *q, const artab_view *k, const art
         P.rm_nc = Nc; P.rm_attend = attending_chunks; P.lse = lse;
         P.new_row = -1; P.mode = kModeRowMask; P.Dh = Dh; P.scale = scale;
         P.vec_ok = aligned ? 1 : 0;
-        return launch_status(launch_portable_dtype(P, dtype, st), "row-mask attention (portable)");
+        return launch_status(launch_portable_or_f32(P, dtype, impl, false, st), "row-mask attention");
     }
     FlashPlan pl = plan_flash(B, H, R, Nc, Dh, /*stacked=*/false, /*allow_split=*/false);
     FlashParams F;
@@ -1093,7 +1113,7 @@ int artab_prefill_attention(const artab_view *q, const artab_view *k, const arta
         P.B = B; P.H = H; P.Lq = Nc; P.Nc = Nc; P.Nb = 0;
         P.new_row = -1; P.mode = kModePlain; P.Dh = Dh; P.scale = scale;
         P.vec_ok = aligned ? 1 : 0;
-        return launch_status(launch_portable_dtype(P, dtype, st), "prefill (portable)");
+        return launch_status(launch_portable_or_f32(P, dtype, impl, false, st), "prefill");
     }
     FlashPlan pl = plan_flash(B, H, Nc, Nc, Dh, /*stacked=*/false, /*allow_split=*/false);
     FlashParams F;

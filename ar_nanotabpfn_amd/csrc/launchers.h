@@ -83,6 +83,16 @@ inline void launch_observed(int kind, Kernel kernel, dim3 grid, dim3 block, size
 // flash_launch.hip: BM = query rows per workgroup (256, 128 or 64), as planned by the caller
 hipError_t launch_flash_dtype(const FlashParams &P, bool is_bf16, int Dh, int BM, hipStream_t stream);
 
+// f32_launch.hip: float32 attention on the matrix cores, for head_dim 32 / 64 / 128 (see f32_attention.h)
+struct F32Shape {
+    int qb;       // 16-row query blocks of a tile
+    bool split;   // a tile's keys are dealt over the wavefronts of a workgroup
+    int n_split;  // ... and over this many workgroups
+};
+F32Shape plan_f32(int H, int Nc, int Dh, int G, int n_groups);
+inline size_t f32_workspace_bytes(long rows, int Dh, int n_split) { return static_cast<size_t>(rows) * (Dh + 1) * n_split * 4; }
+hipError_t launch_f32_attention(PortableParams P, bool stacked, void *workspace, size_t workspace_bytes, hipStream_t stream);
+
 // backward_launch.hip: dQ launch, then dK/dV launch, of the training row attention.  `elem` is
 // the element type of every tensor; the matrix-core kernels take bf16 / f16 with head_dim 32 / 64.
 enum BackwardElem : int { kElemF32 = 0, kElemBf16 = 1, kElemF16 = 2 };
