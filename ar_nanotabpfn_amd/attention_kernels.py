@@ -456,10 +456,15 @@ def prefill_attention(
         kcv, vcv = _lib.view4(k_cache, shared_batch=shared), _lib.view4(v_cache, shared_batch=shared)
         cache_batches = 1 if shared else k_cache.shape[0]
     qv, kv, vv, ov = _lib.view4(q), _lib.view4(k), _lib.view4(v), _lib.view4(out)
+    code = _lib.dtype_code(q.dtype)
+    # memory of this call's own, from the caching allocator: prefills on several streams do not share it
+    nbytes = lib.artab_prefill_workspace_bytes(B, H, Nc, Dh, code)
+    ws = torch.empty(nbytes, device=q.device, dtype=torch.uint8) if nbytes else None
     _lib.check(
-        lib.artab_prefill_attention(
+        lib.artab_prefill_attention_sliced(
             _lib.ref(qv), _lib.ref(kv), _lib.ref(vv), _lib.ref(ov), _lib.ref(kcv), _lib.ref(vcv), cache_batches,
-            B, H, Nc, Dh, 0.0, _lib.dtype_code(q.dtype), _impl(use_triton), _lib.current_stream(dev),
+            B, H, Nc, Dh, 0.0, code, ws.data_ptr() if nbytes else None, nbytes, _impl(use_triton),
+            _lib.current_stream(dev),
         )
     )
     return out

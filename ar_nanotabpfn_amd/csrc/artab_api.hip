@@ -185,6 +185,37 @@ static FlashPlan plan_flash(int B, int H, int Lq, int Nc, int Dh, bool stacked, 
     return pl;
 }
 
+// Key slices of a prefill.  One context has few query tiles: 5001 rows of 8 heads are 160 workgroups of
+// 256 rows, and cutting the tiles to 64 rows leaves wavefronts that wait for their own tiles (1.2 of
+// them per SIMD, 295 TFLOP/s).  Whole tiles with the keys dealt over workgroups, float32 partials and a
+// merge are faster from about 1000 rows on.  The choice weighs estimates in microseconds, fitted to
+// launches of 200 to 16384 rows, 4 to 16 heads, 1 to 16 tables (bf16; f16 gains more everywhere): a
+// compute unit takes 12 ns per key for one tile, 17 for a pair, a slice costs 5 to start, the merge 5 and
+// its traffic at 3.5 TB/s; unsliced launches of small tiles take 12.5 to 21 ns per key, the more wavefronts
+// share a SIMD.  Unsliced -> sliced: 1 x 8 x 1024 17.1 -> 15.5, 4096 67 -> 36, 5001 81 -> 47, 9000 174 -> 122,
+// 12000 256 -> 185, 1 x 16 x 9000 246 -> 225; 700 rows 13.4 against 14.1, 8 x 8 x 512 14.2 against 17.8: not sliced.
+static int prefill_slices(int B, int H, int Nc, int Dh) {
+    if (Dh != 32) return 1;
+    const int forced = tune(kTuneSplit, 0);
+    if (forced > 0) return forced;
+    const long pairs = static_cast<long>(B) * H, tiles = (Nc + 255) / 256 * pairs;
+    if (tiles > 1024) return 1;
+    const auto wide = [&](int keys, long wgs) {  // workgroups of 256 queries, `keys` keys each
+        const long q = (wgs + 255) / 256;
+        return static_cast<double>((q + 1) / 2) * 5.0 + keys * (17e-3 * (q / 2) + 12e-3 * (q % 2));
+    };
+    int bm = 256;
+    while (bm > 64 && (Nc + bm - 1) / bm * pairs < 512) bm /= 2;  // as plan_flash cuts the unsliced tiles
+    double best = bm == 256 ? wide(Nc, tiles)
+                            : 4.5 + Nc * (12.5e-3 + 3e-3 * ((Nc + bm - 1) / bm * pairs * (bm / 32) / 1024.0));
+    int slices = 1;
+    for (int s = 2; s <= 16 && Nc >= 256 * s; ++s) {
+        const double t = wide((Nc + s - 1) / s, tiles * s) + 5.0 + s * (pairs * Nc * (Dh * 8.0)) / 3.5e6;
+        if (t < best) best = t, slices = s;
+    }
+    return slices;
+}
+
 template <typename T, int LQ>
 static hipError_t launch_decode_lq(const DecodeParams &P, int Dh, hipStream_t stream) {
     const long pairs = static_cast<long>(P.B) * P.H;
@@ -305,14 +336,14 @@ static hipError_t launch_portable_or_f32(const PortableParams &P, int dtype, int
 // per (row, 4 output elements).
 struct CombineParams {
     View out;
-    const void *part_o;  // input type
+    const void *part_o;  // input type, float32 for a prefill
     const float *part_lse;
     float *lse;
     long rows;
     int H, Lq, Dh, n_split;
 };
 
-template <typename T>
+template <typename T, typename PT = T>  // PT: element type of the partials
 __global__ __launch_bounds__(256) void combine_kernel(CombineParams P) {
     const int per_row = P.Dh / 4;
     long idx = static_cast<long>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -324,10 +355,16 @@ __global__ __launch_bounds__(256) void combine_kernel(CombineParams P) {
     float wsum = 0.f, acc[4] = {0.f, 0.f, 0.f, 0.f};
     for (int s = 0; s < P.n_split; ++s) {
         float w = merge_weight(P.part_lse[s * P.rows + row], mx);
-        const T *o = static_cast<const T *>(P.part_o) + (s * P.rows + row) * P.Dh + d0;
+        const PT *o = static_cast<const PT *>(P.part_o) + (s * P.rows + row) * P.Dh + d0;
         wsum += w;
+        if constexpr (sizeof(PT) == 4) {
+            const f32x4 v = *reinterpret_cast<const f32x4 *>(o);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) acc[e] = fmaf(w, to_f32(o[e]), acc[e]);
+            for (int e = 0; e < 4; ++e) acc[e] = fmaf(w, v[e], acc[e]);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[e] = fmaf(w, to_f32(o[e]), acc[e]);
+        }
     }
     int i = static_cast<int>(row % P.Lq);
     int h = static_cast<int>((row / P.Lq) % P.H);
@@ -1081,9 +1118,10 @@ int artab_row_mask_attention_backward(const artab_view *q, const artab_view *k, 
                          use_mfma ? "row-mask attention backward (mfma)" : "row-mask attention backward (portable)");
 }
 
-int artab_prefill_attention(const artab_view *q, const artab_view *k, const artab_view *v, const artab_view *out,
+static int prefill_impl(const artab_view *q, const artab_view *k, const artab_view *v, const artab_view *out,
                             const artab_view *k_cache, const artab_view *v_cache, int cache_batches, int B, int H,
-                            int Nc, int Dh, float scale, int dtype, int impl, void *stream) {
+                            int Nc, int Dh, float scale, int dtype, void *workspace, size_t workspace_bytes, int impl,
+                            void *stream) {
     ARTAB_TRY(check_common(B, H, Nc, Dh, dtype));
     if (B == 0 || Nc == 0) return ARTAB_OK;
     ARTAB_TRY(check_view(q, "q", dtype, true));
@@ -1115,7 +1153,16 @@ int artab_prefill_attention(const artab_view *q, const artab_view *k, const arta
         P.vec_ok = aligned ? 1 : 0;
         return launch_status(launch_portable_or_f32(P, dtype, impl, false, st), "prefill");
     }
+    const long rows = static_cast<long>(B) * H * Nc;
+    const int slices = prefill_slices(B, H, Nc, Dh);
     FlashPlan pl = plan_flash(B, H, Nc, Nc, Dh, /*stacked=*/false, /*allow_split=*/false);
+    if (slices > 1 && workspace && workspace_bytes >= f32_workspace_bytes(rows, Dh, slices) &&
+        reinterpret_cast<uintptr_t>(workspace) % 16 == 0) {
+        pl.BM = 256;
+        pl.tiles_per_group = (Nc + 255) / 256;
+        pl.kv_per_split = ((Nc + slices - 1) / slices + 127) / 128 * 128;
+        pl.n_split = (Nc + pl.kv_per_split - 1) / pl.kv_per_split;
+    }
     FlashParams F;
     memset(&F, 0, sizeof(F));
     F.q = dv(q); F.kc = dv(k); F.vc = dv(v); F.out = dv(out);
@@ -1123,11 +1170,47 @@ int artab_prefill_attention(const artab_view *q, const artab_view *k, const arta
     F.cache_batches = kc_given ? cache_batches : 0;
     F.B = B; F.H = H; F.Lq = Nc; F.Nc = Nc;
     F.G = pl.G; F.tiles_per_group = pl.tiles_per_group; F.n_groups = pl.n_groups;
-    F.n_split = 1; F.kv_per_split = pl.kv_per_split;
+    F.n_split = pl.n_split; F.kv_per_split = pl.kv_per_split;
     F.qscale = scale * kLog2e;
     F.mode = kFlashPrefill;
-    return launch_status(launch_flash_dtype(F, dtype == ARTAB_BF16, Dh, pl.BM, st), "prefill (mfma)");
+    if (pl.n_split > 1) {
+        F.part_o = workspace;
+        F.part_f32 = 1;
+        F.part_lse = static_cast<float *>(workspace) + rows * Dh * pl.n_split;
+    }
+    ARTAB_TRY(launch_status(launch_flash_dtype(F, dtype == ARTAB_BF16, Dh, pl.BM, st), "prefill (mfma)"));
+    if (pl.n_split == 1) return ARTAB_OK;
+    CombineParams C;
+    C.out = dv(out); C.part_o = F.part_o; C.part_lse = F.part_lse; C.lse = nullptr;
+    C.rows = rows; C.H = H; C.Lq = Nc; C.Dh = Dh; C.n_split = pl.n_split;
+    const unsigned grid = static_cast<unsigned>((rows * (Dh / 4) + 255) / 256);
+    if (dtype == ARTAB_BF16)
+        hipLaunchKernelGGL((combine_kernel<bf16_t, float>), dim3(grid), dim3(256), 0, st, C);
+    else
+        hipLaunchKernelGGL((combine_kernel<f16_t, float>), dim3(grid), dim3(256), 0, st, C);
+    return launch_status(hipGetLastError(), "prefill combine");
 }
+
+size_t artab_prefill_workspace_bytes(int B, int H, int Nc, int Dh, int dtype) {
+    if (B <= 0 || H <= 0 || Nc <= 0 || !mfma_shape_ok(dtype, Dh)) return 0;
+    const int slices = prefill_slices(B, H, Nc, Dh);
+    return slices > 1 ? f32_workspace_bytes(static_cast<long>(B) * H * Nc, Dh, slices) : 0;
+}
+
+int artab_prefill_attention(const artab_view *q, const artab_view *k, const artab_view *v, const artab_view *out,
+                            const artab_view *k_cache, const artab_view *v_cache, int cache_batches, int B, int H,
+                            int Nc, int Dh, float scale, int dtype, int impl, void *stream) {
+    return prefill_impl(q, k, v, out, k_cache, v_cache, cache_batches, B, H, Nc, Dh, scale, dtype, nullptr, 0, impl, stream);
+}
+
+int artab_prefill_attention_sliced(const artab_view *q, const artab_view *k, const artab_view *v, const artab_view *out,
+                                   const artab_view *k_cache, const artab_view *v_cache, int cache_batches, int B, int H,
+                                   int Nc, int Dh, float scale, int dtype, void *workspace, size_t workspace_bytes,
+                                   int impl, void *stream) {
+    return prefill_impl(q, k, v, out, k_cache, v_cache, cache_batches, B, H, Nc, Dh, scale, dtype, workspace,
+                        workspace_bytes, impl, stream);
+}
+
 
 int artab_buffer_attention(const artab_view *q, const artab_view *k_buf, const artab_view *v_buf,
                            const uint8_t *mask, int64_t mask_sb, int64_t mask_sh, int64_t mask_sq,

@@ -102,6 +102,7 @@ struct FlashParams {
     void *part_o;     // split partials: [n_split][B*H*Lq][DH] normalised, in the input type (the
                       // reference merges partial outputs of the input type too, triton_kernels.py:478-524)
     float *part_lse;  // [n_split][B*H*Lq] natural log
+    int part_f32;     // the partials are float32 (prefill: its sums were float32 throughout before it was split)
     int B, H, Lq;
     int Nc, Nb, Nt;
     int G;                // query rows per group (B*Lq stacked, or Lq per batch entry)
@@ -430,7 +431,7 @@ void flash_kernel(const char *early_k, const char *early_v, int early_sh, int ea
     };
 
     // ---- prefill: this tile's own K/V rows go to the cache.
-    if (!PLAIN && P.mode == kFlashPrefill && P.kcache.p && g < P.cache_batches) {
+    if (!PLAIN && P.mode == kFlashPrefill && P.kcache.p && g < P.cache_batches && split == 0) {
         int nrows = min(BM, P.G - row0_wg);
         for (int idx = tid; idx < nrows * CPR; idx += NT) {
             int rr = row0_wg + idx / CPR, ch = idx % CPR;
@@ -1314,7 +1315,19 @@ void flash_kernel(const char *early_k, const char *early_v, int early_sh, int ea
         const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
         const float m_fin = m_run[j] == -INFINITY ? 0.f : m_run[j];
         const float lse = l_tot > 0.f ? (m_fin + fast_log2(l_tot)) * kLn2 : -INFINITY;
-        if (P.part_o) {
+        if (!PLAIN && P.part_o && P.part_f32) {
+            float *po = static_cast<float *>(P.part_o) + (static_cast<long>(split) * total_rows + orow_idx) * DH;
+#pragma unroll
+            for (int db = 0; db < DB; ++db)
+#pragma unroll
+                for (int gq = 0; gq < 4; ++gq) {
+                    f32x4 val;
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) val[r] = o_acc[j][db][4 * gq + r] * inv;
+                    *reinterpret_cast<f32x4 *>(po + 32 * db + 8 * gq + 4 * hb_e) = val;
+                }
+            if (hb_e == 0) P.part_lse[static_cast<long>(split) * total_rows + orow_idx] = lse;
+        } else if (P.part_o) {
             T *po = static_cast<T *>(P.part_o) + (static_cast<long>(split) * total_rows + orow_idx) * DH;
 #pragma unroll
             for (int db = 0; db < DB; ++db)

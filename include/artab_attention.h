@@ -329,6 +329,19 @@ int artab_prefill_attention(const artab_view *q, const artab_view *k, const arta
                             int impl, void *stream);
 
 /*
+ * The same with scratch memory (16-byte aligned, artab_prefill_workspace_bytes of it, the caller's own
+ * until the call's work on `stream` is done).  A prefill with too few query tiles for the chip then deals
+ * the keys over several workgroups and merges their float32 partials; without the memory, or where the
+ * size asked for is 0, it runs as artab_prefill_attention.
+ */
+size_t artab_prefill_workspace_bytes(int B, int H, int Nc, int Dh, int dtype);
+int artab_prefill_attention_sliced(const artab_view *q, const artab_view *k, const artab_view *v,
+                                   const artab_view *out,
+                                   const artab_view *k_cache, const artab_view *v_cache, int cache_batches,
+                                   int B, int H, int Nc, int Dh, float scale, int dtype,
+                                   void *workspace, size_t workspace_bytes, int impl, void *stream);
+
+/*
  * Row attention of the training forward under the context / buffer / target mask.
  * Replaces flex_attention under create_row_mask (ar_tabpfn/model/attention.py:86-175), as called
  * by the training forward (ar_tabpfn/model/model.py:317-369 through :95-126).  Rows are
