@@ -95,6 +95,25 @@ class ArtabTrajectoryArgs(ctypes.Structure):
     ]
 
 
+class ArtabStackLayer(ctypes.Structure):
+    """``artab_stack_layer`` of include/artab_attention.h, field for field."""
+
+    _fields_ = [
+        *((n, _p) for n in ("w_fo", "w_qkv", "w_o", "w_1", "b_1", "w_2", "b_2", "gamma1", "beta1", "gamma2", "beta2", "gamma3",
+                            "beta3", "k_cache", "v_cache")),
+        ("eps1", _f), ("eps2", _f), ("eps3", _f),
+    ]
+
+
+class ArtabStackArgs(ctypes.Structure):
+    """``artab_stack_args`` of include/artab_attention.h, field for field."""
+
+    _fields_ = [
+        ("layers", _p), *((n, _i) for n in ("n_layers", "B", "N", "H", "D", "F", "num_targets", "Nc", "own_caches", "cache_rows")),
+        ("x", _p), ("out", _p), ("scratch", _p),
+    ]
+
+
 class ArtabTrainArgs(ctypes.Structure):
     """``artab_train_args`` of include/artab_attention.h, field for field."""
 
@@ -156,6 +175,8 @@ SIGNATURES = {
     "artab_row_mask_attention_backward": (
         _i, [_VP, _VP, _VP, _VP, _VP, _p, _p, _VP, _VP, _VP, _i, _i, _i, _i, _i, _i, _i, _f, _i, _i, _p]),
     "artab_prefill_attention": (_i, [_VP, _VP, _VP, _VP, _VP, _VP, _i, _i, _i, _i, _i, _f, _i, _i, _p]),
+    "artab_layer_stack_scratch_bytes": (_sz, [_p, _i]),
+    "artab_layer_stack": (_i, [_p, _i, _p]),
     "artab_prefill_workspace_bytes": (_sz, [_i, _i, _i, _i, _i]),
     "artab_prefill_attention_sliced": (_i, [_VP, _VP, _VP, _VP, _VP, _VP, _i, _i, _i, _i, _i, _f, _i, _p, _sz, _i, _p]),
     "artab_buffer_attention": (_i, [_VP, _VP, _VP, _p, _i64, _i64, _i64, _VP, _p, _i, _i, _i, _i, _i, _f, _i, _p]),

@@ -1578,6 +1578,112 @@ int artab_decode_step_boundary(const artab_attention_partials *parts, const void
     return launch_status(e, "decode_step_boundary");
 }
 
+// Rows of the fresh K and V projections into the caches of their own, one launch for both (16-byte pieces).
+struct CacheRowsParams {
+    const char *k, *v;          // [B, N] rows of row_bytes, `ld` bytes apart; head h in piece h * head_pieces ..
+    char *k_cache, *v_cache;    // [B, H, cache_rows] rows of head_pieces * 16 bytes, rows `first` on
+    long ld;
+    int B, N, H, head_pieces, cache_rows, first;
+};
+__global__ __launch_bounds__(256) void cache_rows_kernel(CacheRowsParams P) {
+    const long per_batch = static_cast<long>(P.H) * P.N * P.head_pieces;
+    const long idx = static_cast<long>(blockIdx.x) * 256 + threadIdx.x;
+    if (idx >= P.B * per_batch) return;
+    const long b = idx / per_batch;
+    const int piece = static_cast<int>(idx % P.head_pieces);
+    const int n = static_cast<int>(idx / P.head_pieces % P.N), h = static_cast<int>(idx / P.head_pieces / P.N % P.H);
+    const long src = (b * P.N + n) * P.ld + (static_cast<long>(h) * P.head_pieces + piece) * 16;
+    const long dst = (((b * P.H + h) * P.cache_rows + P.first + n) * P.head_pieces + piece) * 16;
+    *reinterpret_cast<u32x4 *>(P.k_cache + dst) = *reinterpret_cast<const u32x4 *>(P.k + src);
+    *reinterpret_cast<u32x4 *>(P.v_cache + dst) = *reinterpret_cast<const u32x4 *>(P.v + src);
+}
+
+namespace {
+struct StackScratch {
+    size_t y[2], qkv, attn, prefill, total;
+};
+StackScratch stack_scratch(const artab_stack_args *a, int dtype) {
+    const size_t rows = static_cast<size_t>(a->B) * a->N, e = elem_size(dtype);
+    StackScratch s;
+    size_t used = 0;
+    const auto take = [&](size_t bytes) { const size_t at = used; used += (bytes + 255) / 256 * 256; return at; };
+    s.y[0] = take(rows * a->D * e);
+    s.y[1] = take(rows * a->D * e);
+    s.qkv = take(rows * 3 * a->D * e);
+    s.attn = take(rows * a->D * e);
+    s.prefill = used;
+    s.total = used + (a->num_targets ? 0 : artab_prefill_workspace_bytes(a->B, a->H, a->N, a->D / a->H, dtype));
+    return s;
+}
+int check_stack(const artab_stack_args *a) {
+    if (!a || !a->layers) return fail(ARTAB_ERR_NULL_POINTER, "layer stack without arguments or layers");
+    if (a->n_layers < 1 || a->B < 1 || a->N < 1 || a->H < 1 || a->D < 1 || a->D % a->H || a->num_targets < 0 ||
+        (a->num_targets && a->N != 2L * a->num_targets))
+        return fail(ARTAB_ERR_BAD_SHAPE, "layer stack: n_layers=%d B=%d N=%d H=%d D=%d num_targets=%d",
+                    a->n_layers, a->B, a->N, a->H, a->D, a->num_targets);
+    const long need = a->num_targets == 0 ? a->N : a->Nc + (a->own_caches ? static_cast<long>(a->N) : 0);
+    if (a->cache_rows < need || a->Nc < 0)
+        return fail(ARTAB_ERR_BAD_SHAPE, "layer stack: caches of %d rows, %ld needed", a->cache_rows, need);
+    return ARTAB_OK;
+}
+}  // namespace
+
+size_t artab_layer_stack_scratch_bytes(const artab_stack_args *args, int dtype) {
+    if (check_stack(args) != ARTAB_OK) return 0;
+    return stack_scratch(args, dtype).total;
+}
+
+int artab_layer_stack(const artab_stack_args *a, int dtype, void *stream) {
+    ARTAB_TRY(check_stack(a));
+    ARTAB_TRY(check_layer_dtype_rows("layer_stack", dtype, static_cast<int64_t>(a->B) * a->N));
+    if (!a->x || !a->out || !a->scratch) return fail(ARTAB_ERR_NULL_POINTER, "layer stack: x, out and scratch are required");
+    const int Dh = a->D / a->H, e = elem_size(dtype);
+    if (misaligned16(a->scratch) || Dh * e % 16)
+        return fail(ARTAB_ERR_BAD_STRIDE, "layer stack: scratch and heads must be whole 16-byte pieces");
+    const StackScratch s = stack_scratch(a, dtype);
+    char *base = static_cast<char *>(a->scratch);
+    char *qkv = base + s.qkv, *attn = base + s.attn;
+    const int64_t rows = static_cast<int64_t>(a->B) * a->N, D = a->D;
+    const auto head_view = [&](int which) {
+        return artab_view{qkv + which * D * e, a->N * 3 * D, Dh, 3 * D};
+    };
+    const artab_view q = head_view(0), k = head_view(1), v = head_view(2), out = {attn, a->N * D, Dh, D};
+    const int64_t cache_h = static_cast<int64_t>(a->cache_rows) * Dh, cache_b = a->own_caches ? a->H * cache_h : 0;
+    const artab_stack_layer *L = a->layers;
+    ARTAB_TRY(artab_layer_pre(a->x, D, L->w_fo, L->gamma1, L->beta1, L->eps1, L->w_qkv, base + s.y[0], qkv, rows, a->D, dtype, stream));
+    for (int l = 0; l < a->n_layers; ++l, ++L) {
+        if (!L->k_cache || !L->v_cache || misaligned16(L->k_cache) || misaligned16(L->v_cache))
+            return fail(ARTAB_ERR_NULL_POINTER, "layer stack: layer %d needs 16-byte aligned caches", l);
+        const artab_view kc = {L->k_cache, cache_b, cache_h, Dh}, vc = {L->v_cache, cache_b, cache_h, Dh};
+        if (a->num_targets == 0) {
+            ARTAB_TRY(artab_prefill_attention_sliced(&q, &k, &v, &out, &kc, &vc, a->own_caches ? a->B : 1, a->B, a->H, a->N, Dh, 0.f,
+                                                     dtype, base + s.prefill, s.total - s.prefill, ARTAB_IMPL_AUTO, stream));
+        } else {
+            if (a->own_caches) {
+                CacheRowsParams C = {static_cast<const char *>(k.data), static_cast<const char *>(v.data),
+                                     static_cast<char *>(L->k_cache), static_cast<char *>(L->v_cache), 3 * D * e,
+                                     a->B, a->N, a->H, Dh * e / 16, a->cache_rows, a->Nc};
+                const long pieces = rows * a->H * C.head_pieces;
+                if ((pieces + 255) / 256 > 0x7fffffffL) return fail(ARTAB_ERR_BAD_SHAPE, "layer stack: too many rows");
+                hipLaunchKernelGGL(cache_rows_kernel, dim3(static_cast<unsigned>((pieces + 255) / 256)), dim3(256), 0,
+                                   static_cast<hipStream_t>(stream), C);
+                ARTAB_TRY(launch_status(hipGetLastError(), "cache rows"));
+            }
+            ARTAB_TRY(artab_teacher_forcing_attention(&q, &kc, &vc, &k, &v, &out, nullptr, a->B, a->H, a->num_targets, a->Nc, Dh,
+                                                      0.f, dtype, ARTAB_IMPL_AUTO, stream));
+        }
+        const char *y = base + s.y[l & 1];
+        if (l + 1 == a->n_layers)
+            return artab_layer_post(attn, D, y, D, L->w_o, L->gamma2, L->beta2, L->eps2, L->w_1, L->b_1, L->w_2, L->b_2, L->gamma3,
+                                    L->beta3, L->eps3, a->out, rows, a->D, a->F, dtype, stream);
+        const artab_stack_layer *n = L + 1;
+        ARTAB_TRY(artab_layer_post_pre(attn, D, y, D, L->w_o, L->gamma2, L->beta2, L->eps2, L->w_1, L->b_1, L->w_2, L->b_2, L->gamma3,
+                                       L->beta3, L->eps3, n->w_fo, n->gamma1, n->beta1, n->eps1, n->w_qkv, base + s.y[1 - (l & 1)], qkv,
+                                       rows, a->D, a->F, dtype, stream));
+    }
+    return ARTAB_OK;
+}
+
 static TrajectoryTapeLayout trajectory_layout(int D, int F, int n_layers, int dtype) {
     if (dtype == ARTAB_BF16) return trajectory_tape_layout_bf16(D, F, n_layers);
     if (dtype == ARTAB_F16) return trajectory_tape_layout_f16(D, F, n_layers);

@@ -26,9 +26,13 @@ from torch import Tensor
 from . import attention_kernels as ak
 from .attention import DecodeMask, TeacherForcingMask
 from . import _lib
+from .stack import LayerStack
 from .glue import SampleEmbedStep, DecodeStepBoundary, TrajectoryDecoder, add_layer_norm
 
 __all__ = ["ARTabPFNPredictor"]
+
+
+_attention_module = ak
 
 
 class _GraphState:
@@ -93,6 +97,7 @@ class ARTabPFNPredictor:
         # Take a whole sampling run through one launch where that is the faster route (the library's
         # rule, ``artab_trajectory_group``) and the sampling switches above are at their defaults.
         self.whole_run_decode = True
+        self._stack = LayerStack()
         self._trajectory = None      # (key of the model state, TrajectoryDecoder or None)
         self._side_streams = {}
         self._graph_state = None
@@ -115,13 +120,15 @@ class ARTabPFNPredictor:
             dtype = dtype or param.dtype
         self._device, self._dtype = device, dtype
         self.seq_len = self.context_len = self.buffer_len = 0
+        kept = []
+
         def zeros(layer, name, shape):
             # same contents as a fresh torch.zeros; memory (and its address, which recorded
             # HIP graphs refer to) is kept when the shape, dtype and device are unchanged
             old = getattr(layer, name, None)
             if (isinstance(old, torch.Tensor) and tuple(old.shape) == tuple(shape) and old.dtype == dtype
                     and old.device == torch.device(device) and old.is_contiguous()):
-                old.zero_()
+                kept.append(old)
             else:
                 setattr(layer, name, torch.zeros(shape, device=device, dtype=dtype))
 
@@ -136,12 +143,16 @@ class ARTabPFNPredictor:
                     layer.v_ctx_cache = torch.empty_like(layer.k_ctx_cache)
                 zeros(layer, "k_buf_cache", (batch_size, H, max_seq_len, Dh))
                 zeros(layer, "v_buf_cache", (batch_size, H, max_seq_len, Dh))
+            if kept:
+                torch._foreach_zero_(kept)
             return
         self.max_buffer_len = 0
         for layer in self.backbone.layers:
             H, Dh = layer.attn_rows.n_heads, layer.attn_rows.head_dim
             zeros(layer, "k_cache", (batch_size, H, max_seq_len, Dh))
             zeros(layer, "v_cache", (batch_size, H, max_seq_len, Dh))
+        if kept:
+            torch._foreach_zero_(kept)
 
     def _side_stream(self, device, tag=0):
         if device.type != "cuda":
@@ -199,6 +210,12 @@ class ARTabPFNPredictor:
                 return finish(y, attn) if finish is not None else layer.finish(y, attn)
             state = layer.finish_then_pre(y, attend(layer, q, k, v), layers[idx + 1])
 
+    def _stack_pass(self, x_row: Tensor, caches, num_targets: int = 0, context_len: int = 0) -> Optional[Tensor]:
+        """The whole stack as one call, or None where the layers have to be run one by one."""
+        if ak is not _attention_module:  # calls of a program's own in the place of this package's
+            return None
+        return self._stack(list(self.backbone.layers), x_row, caches, num_targets, context_len)
+
     # ------------------------------------------------------------------ prefill
 
     @torch.no_grad()
@@ -213,7 +230,9 @@ class ARTabPFNPredictor:
         for layer in self.backbone.layers:
             if layer.k_cache.shape[2] < Nc:
                 raise ValueError("KV cache too small for the context; call init_kv_cache with a larger max_seq_len.")
-        self._run_layers(x_row, lambda layer, q, k, v: ak.prefill_attention(q, k, v, layer.k_cache, layer.v_cache))
+        layers = list(self.backbone.layers)
+        if self._stack_pass(x_row, [(l.k_cache, l.v_cache) for l in layers]) is None:
+            self._run_layers(x_row, lambda layer, q, k, v: ak.prefill_attention(q, k, v, layer.k_cache, layer.v_cache))
         self.seq_len = Nc
 
     @torch.no_grad()
@@ -227,8 +246,9 @@ class ARTabPFNPredictor:
             if layer.k_ctx_cache.shape[1] != Nc or layer.k_ctx_cache.shape[0] != H:
                 layer.k_ctx_cache = torch.zeros(H, Nc, Dh, device=x_row.device, dtype=x_row.dtype)
                 layer.v_ctx_cache = torch.zeros_like(layer.k_ctx_cache)
-        self._run_layers(
-            x_row, lambda layer, q, k, v: ak.prefill_attention(q, k, v, layer.k_ctx_cache, layer.v_ctx_cache))
+        if self._stack_pass(x_row, [(l.k_ctx_cache, l.v_ctx_cache) for l in self.backbone.layers]) is None:
+            self._run_layers(
+                x_row, lambda layer, q, k, v: ak.prefill_attention(q, k, v, layer.k_ctx_cache, layer.v_ctx_cache))
         self.context_len = Nc
         self.buffer_len = 0
         self.seq_len = Nc
@@ -781,15 +801,20 @@ class ARTabPFNPredictor:
             raise ValueError("Expected N == 2*num_targets for teacher forcing.")
         mask = TeacherForcingMask(num_cached=self.seq_len, num_targets=num_targets)
         start = self.seq_len
-        x_row = self._run_layers(embedding, lambda layer, q, k, v: self._attend_with_cache(layer, q, k, v, mask, start))
+        x_row = self._stack_pass(embedding, [(l.k_cache, l.v_cache) for l in self.backbone.layers], num_targets, start)
+        if x_row is None:
+            x_row = self._run_layers(embedding, lambda layer, q, k, v: self._attend_with_cache(layer, q, k, v, mask, start))
         return add_layer_norm(x_row, None, None, self.backbone.norm)
 
     @torch.no_grad()
     def _teacher_forcing_decode_shared(self, embedding: Tensor, num_targets: int) -> Tensor:
         if embedding.shape[1] != 2 * num_targets:
             raise ValueError("Expected N == 2*num_targets for teacher forcing.")
-        x_row = self._run_layers(
-            embedding, lambda layer, q, k, v: self._attend_teacher_forcing_shared(layer, q, k, v, num_targets))
+        x_row = self._stack_pass(embedding, [(l.k_ctx_cache, l.v_ctx_cache) for l in self.backbone.layers], num_targets,
+                                 self.context_len)
+        if x_row is None:
+            x_row = self._run_layers(
+                embedding, lambda layer, q, k, v: self._attend_teacher_forcing_shared(layer, q, k, v, num_targets))
         return add_layer_norm(x_row, None, None, self.backbone.norm)
 
     def _layer_teacher_forcing_shared(self, layer, x_row: Tensor, num_targets: int) -> Tensor:

@@ -1,0 +1,102 @@
+"""A prefill or teacher-forced pass through the layer stack as one call of the library (``artab_layer_stack``).
+
+A layer is two launches of 15 to 70 us; issued one by one from Python they cost about 100 us of host time, which
+is what such passes waited for (12 layers against 5001 rows: 1.2 ms of host time, 0.9 ms of kernels)."""
+
+from __future__ import annotations
+
+import ctypes
+from typing import Optional
+
+import torch
+from torch import Tensor
+
+from . import _lib
+from . import attention_kernels as ak
+
+__all__ = ["LayerStack"]
+
+# A program that has put callables of its own in their place gets the layer-by-layer form, which calls them.
+_attention_calls = (ak.prefill_attention, ak.teacher_forcing_attention, ak.hybrid_teacher_forcing_attention)
+
+
+def _small_vectors(layer):
+    """Parameters that enter unpacked, in the order of ``artab_stack_layer``, and the weights that are packed."""
+    mods = layer._modules
+    feat, rows, ff = mods["attn_features"]._modules, mods["attn_rows"]._modules, mods["ff"]._modules
+    p1, p2 = ff["0"]._parameters, ff["2"]._parameters
+    n1, n2, n3 = (mods[n]._parameters for n in ("norm1", "norm2", "norm3"))
+    return ((p1["bias"], p2["bias"], n1["weight"], n1["bias"], n2["weight"], n2["bias"], n3["weight"], n3["bias"]),
+            (feat["v_proj"]._parameters["weight"], feat["out_proj"]._parameters["weight"], rows["q_proj"]._parameters["weight"],
+             rows["k_proj"]._parameters["weight"], rows["v_proj"]._parameters["weight"], rows["out_proj"]._parameters["weight"],
+             p1["weight"], p2["weight"]))
+
+
+class LayerStack:
+    """What a pass reads of the layers, collected again whenever a parameter is another tensor or has been
+    written to; each call looks at all of them."""
+
+    def __init__(self):
+        self._key = self._layers = self._keep = None
+
+    def _collect(self, layers, x: Tensor) -> bool:
+        """Bring ``self._layers`` up to date; False where the layers are not of the form the call takes."""
+        try:
+            params = [_small_vectors(layer) for layer in layers]
+        except KeyError:
+            return False
+        key = (x.dtype, x.device, *[(p.data_ptr(), p._version) if p is not None else None for two in params for ps in two for p in ps])
+        if key == self._key:
+            return self._layers is not None
+        self._key, self._layers, self._keep = key, None, None
+        first = layers[0]
+        D, F = x.shape[-1], first.ff[0].out_features
+        for layer, (vectors, weights) in zip(layers, params):
+            sizes = ((F,), (D,)) + ((D,),) * 6 + ((D, D),) * 6 + ((F, D), (D, F))
+            if not (type(layer) is type(first) and layer.attn_rows.n_heads == first.attn_rows.n_heads
+                    and all(p is not None and p.dtype == x.dtype and p.device == x.device and p.is_contiguous() and tuple(p.shape) == s
+                            for p, s in zip(vectors + weights, sizes))
+                    and all(p.data_ptr() % 16 == 0 for p in vectors)):
+                return False
+        array, keep = (_lib.ArtabStackLayer * len(layers))(), []
+        for a, layer, (v, w) in zip(array, layers, params):
+            packed = layer.packed_weights()
+            a.w_fo, a.w_qkv, a.w_o, a.w_1, a.w_2 = (t.data_ptr() for t in packed)
+            a.b_1, a.b_2, a.gamma1, a.beta1, a.gamma2, a.beta2, a.gamma3, a.beta3 = (t.data_ptr() for t in v)
+            a.eps1, a.eps2, a.eps3 = layer.norm1.eps, layer.norm2.eps, layer.norm3.eps
+            keep += [*packed, *v]
+        self._layers, self._keep = array, keep
+        return True
+
+    def __call__(self, layers, x: Tensor, caches, num_targets: int = 0, context_len: int = 0) -> Optional[Tensor]:
+        """``x [B,N,D]`` through ``layers``; ``caches``: ``(k, v)`` of every layer, ``[H,R,Dh]`` or ``[B,H,R,Dh]``.
+        ``num_targets`` 0: prefill; else teacher forcing against the first ``context_len`` cached rows.  None, with
+        nothing done, where the call does not apply."""
+        if not (x.is_cuda and layers and x.numel() and (ak.prefill_attention, ak.teacher_forcing_attention,
+                                                       ak.hybrid_teacher_forcing_attention) == _attention_calls):
+            return None
+        first = layers[0]
+        B, N, D = x.shape
+        k0 = caches[0][0]
+        own = k0.dim() == 4
+        H, Dh, rows = first.attn_rows.n_heads, first.attn_rows.head_dim, k0.shape[-2]
+        shape = (B, H, rows, Dh) if own else (H, rows, Dh)
+        if not (Dh in (32, 64, 128) and first.fused_for(x) and rows >= (N if num_targets == 0 else context_len + (N if own else 0))
+                and (num_targets == 0 or context_len > 0)
+                and all(t.shape == shape and t.dtype == x.dtype and t.device == x.device and t.is_contiguous() and t.data_ptr() % 16 == 0
+                        for c in caches for t in c)
+                and self._collect(layers, x)):
+            return None
+        x = x.contiguous()
+        if x.data_ptr() % 16:
+            x = x.clone()
+        lib, code = _lib.load(), _lib.dtype_code(x.dtype)
+        for a, (k, v) in zip(self._layers, caches):
+            a.k_cache, a.v_cache = k.data_ptr(), v.data_ptr()
+        out = torch.empty_like(x)
+        args = _lib.ArtabStackArgs(ctypes.addressof(self._layers), len(layers), B, N, H, D, first.ff[0].out_features, num_targets,
+                                   context_len, int(own), rows, x.data_ptr(), out.data_ptr(), None)
+        scratch = torch.empty(lib.artab_layer_stack_scratch_bytes(ctypes.byref(args), code), device=x.device, dtype=torch.uint8)
+        args.scratch = scratch.data_ptr()
+        _lib.check(lib.artab_layer_stack(ctypes.byref(args), code, _lib.current_stream(x.device)))
+        return out

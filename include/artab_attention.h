@@ -561,6 +561,33 @@ int artab_train_embed(const artab_train_embed_args *args, void *stream);
 int artab_train_embed_backward(const artab_train_embed_args *args, void *stream);
 
 /*
+ * A pass through the whole layer stack, issued by one call: the first layer's artab_layer_pre, then per layer
+ * the row attention and artab_layer_post_pre (artab_layer_post behind the last), with the results those give.
+ *   num_targets == 0  prefill (inference.py:143-223): dense attention over the N rows, whose K and V go to rows
+ *                     [0, N) of the caches
+ *   num_targets > 0   teacher forcing (inference.py:455-471, :835-890): N = 2 num_targets rows against rows
+ *                     [0, Nc) of the caches; caches of their own per batch entry get the N rows' K and V behind
+ * Caches: contiguous, [B, H, cache_rows, D / H] with own_caches, else [H, cache_rows, D / H] shared by all batch
+ * entries (a prefill stores batch entry 0).  x and out: [B, N, D] contiguous.  The struct is read before the call returns.
+ */
+typedef struct artab_stack_layer {
+    const void *w_fo, *w_qkv, *w_o, *w_1, *b_1, *w_2, *b_2; /* weights packed, as for artab_layer_pre / _post */
+    const void *gamma1, *beta1, *gamma2, *beta2, *gamma3, *beta3;
+    void *k_cache, *v_cache;
+    float eps1, eps2, eps3;
+} artab_stack_layer;
+typedef struct artab_stack_args {
+    const artab_stack_layer *layers;
+    int n_layers, B, N, H, D, F;
+    int num_targets, Nc, own_caches, cache_rows;
+    const void *x;
+    void *out;
+    void *scratch;           /* artab_layer_stack_scratch_bytes, 16-byte aligned, the call's own while it runs */
+} artab_stack_args;
+size_t artab_layer_stack_scratch_bytes(const artab_stack_args *args, int dtype);
+int artab_layer_stack(const artab_stack_args *args, int dtype, void *stream);
+
+/*
  * A whole sampling run in one launch: every workgroup takes a few trajectories through all Nt steps
  * and all layers of the model (inference.py:278-320, :353-366 with the layers of :687-744 or
  * :746-833).  Contexts are in the caches; the buffer rows are appended there as the run goes.

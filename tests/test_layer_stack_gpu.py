@@ -1,0 +1,45 @@
+"""The layer stack as one call against the layer-by-layer form: the same launches, the same bits."""
+
+import pytest
+import torch
+
+from ar_nanotabpfn_amd.inference import ARTabPFNPredictor
+from ar_nanotabpfn_amd.model import ARTabPFN
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("backend", ["shared_context", "per_dataset"])
+# one row, odd counts around a 16-row tile, a prefill whose keys are sliced, three head sizes
+@pytest.mark.parametrize("B,Nc,Nt,D,H", [(1, 1, 1, 128, 4), (3, 17, 5, 128, 2), (2, 333, 45, 256, 8), (1, 1100, 16, 512, 4)])
+def test_one_call_equals_layer_by_layer(device, monkeypatch, dtype, backend, B, Nc, Nt, D, H):
+    torch.manual_seed(Nc)
+    model = ARTabPFN(d_model=D, n_heads=H, n_layers=3, d_ff=256, num_features=2).to(device, dtype).eval()
+    g = torch.Generator().manual_seed(Nt)
+    xc, xt = (torch.randn(B, n, 2, generator=g).to(device, dtype) for n in (Nc, Nt))
+    yc, yt = (torch.randn(B, n, generator=g).to(device, dtype) for n in (Nc, Nt))
+    names = ("k_ctx_cache", "v_ctx_cache") if backend == "shared_context" else ("k_cache", "v_cache")
+
+    def run(one_call):
+        p = ARTabPFNPredictor.from_trained_model(model, backend=backend)
+        taken = []
+        stack = p._stack_pass
+        monkeypatch.setattr(p, "_stack_pass", lambda *a: taken.append(stack(*a) if one_call else None) or taken[-1])
+        out = p.evaluate_joint_density(xc, yc, xt, yt)
+        assert len(taken) == 2 and all((t is not None) == one_call for t in taken)
+        again = p.evaluate_joint_density(xc, yc, xt, yt)
+        assert torch.equal(out, again)
+        return [out] + [getattr(layer, n).clone() for layer in model.backbone.layers for n in names]
+
+    for a, b in zip(run(True), run(False)):
+        assert torch.equal(a, b)
+    # a weight written to in place is seen by the next call
+    before = run(True)[0]
+    with torch.no_grad():
+        model.backbone.layers[1].ff[0].weight.mul_(1.5)
+        model.backbone.layers[2].norm2.bias.add_(0.5)
+    after = run(True)
+    assert not torch.equal(after[0], before)
+    for a, b in zip(after, run(False)):
+        assert torch.equal(a, b)
