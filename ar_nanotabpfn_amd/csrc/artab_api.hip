@@ -20,6 +20,7 @@
 #include "mfma_flash.h"
 #include "portable_kernels.h"
 #include "queue_order.h"
+#include "f32_layer.h"
 #include "launchers.h"
 
 namespace artab {
@@ -1615,6 +1616,21 @@ StackScratch stack_scratch(const artab_stack_args *a, int dtype) {
     s.total = used + (a->num_targets ? 0 : artab_prefill_workspace_bytes(a->B, a->H, a->N, a->D / a->H, dtype));
     return s;
 }
+F32LayerParams &f32_head(F32LayerParams &P, const artab_stack_layer &n, void *y, void *qkv, int64_t rows) {
+    const auto in = [](const void *p) { return static_cast<const float *>(p); };
+    P.w_fo = in(n.w_fo); P.gamma1 = in(n.gamma1); P.beta1 = in(n.beta1); P.w_qkv = in(n.w_qkv); P.eps1 = n.eps1;
+    P.y_next = static_cast<float *>(y); P.qkv = static_cast<float *>(qkv);
+    P.rows = rows; P.pre = 1;
+    return P;
+}
+void f32_tail(F32LayerParams &P, const artab_stack_layer &n, const void *attn, const void *y, void *out, int64_t rows) {
+    const auto in = [](const void *p) { return static_cast<const float *>(p); };
+    P.attn = in(attn); P.y = in(y); P.w_o = in(n.w_o); P.gamma2 = in(n.gamma2); P.beta2 = in(n.beta2); P.eps2 = n.eps2;
+    P.w_1 = in(n.w_1); P.b_1 = in(n.b_1); P.w_2 = in(n.w_2); P.b_2 = in(n.b_2);
+    P.gamma3 = in(n.gamma3); P.beta3 = in(n.beta3); P.eps3 = n.eps3;
+    P.out = static_cast<float *>(out);
+    P.rows = rows; P.post = 1;
+}
 int check_stack(const artab_stack_args *a) {
     if (!a || !a->layers) return fail(ARTAB_ERR_NULL_POINTER, "layer stack without arguments or layers");
     if (a->n_layers < 1 || a->B < 1 || a->N < 1 || a->H < 1 || a->D < 1 || a->D % a->H || a->num_targets < 0 ||
@@ -1628,6 +1644,14 @@ int check_stack(const artab_stack_args *a) {
 }
 }  // namespace
 
+int artab_pack_stack_weight_f32(const void *w, void *packed, int N, int K, void *stream) {
+    if (N <= 0 || K <= 0 || N % 16 || K % 16) return fail(ARTAB_ERR_BAD_SHAPE, "pack: N and K must be multiples of 16 (got %d, %d)", N, K);
+    if (!w || !packed) return fail(ARTAB_ERR_NULL_POINTER, "pack: null pointer");
+    if (misaligned16(w) || misaligned16(packed)) return fail(ARTAB_ERR_BAD_STRIDE, "pack: pointers must be 16-byte aligned");
+    return launch_status(launch_f32_pack(static_cast<const float *>(w), static_cast<float *>(packed), N, K,
+                                         static_cast<hipStream_t>(stream)), "pack (float32)");
+}
+
 size_t artab_layer_stack_scratch_bytes(const artab_stack_args *args, int dtype) {
     if (check_stack(args) != ARTAB_OK) return 0;
     return stack_scratch(args, dtype).total;
@@ -1635,7 +1659,10 @@ size_t artab_layer_stack_scratch_bytes(const artab_stack_args *args, int dtype) 
 
 int artab_layer_stack(const artab_stack_args *a, int dtype, void *stream) {
     ARTAB_TRY(check_stack(a));
-    ARTAB_TRY(check_layer_dtype_rows("layer_stack", dtype, static_cast<int64_t>(a->B) * a->N));
+    const bool f32 = dtype == ARTAB_F32;
+    if (!f32) ARTAB_TRY(check_layer_dtype_rows("layer_stack", dtype, static_cast<int64_t>(a->B) * a->N));
+    if (f32 && !f32_layer_width_ok(a->D, a->F))
+        return fail(ARTAB_ERR_UNSUPPORTED, "layer stack in float32: D in {128, 256, 512} and F = 256 (got %d, %d)", a->D, a->F);
     if (!a->x || !a->out || !a->scratch) return fail(ARTAB_ERR_NULL_POINTER, "layer stack: x, out and scratch are required");
     const int Dh = a->D / a->H, e = elem_size(dtype);
     if (misaligned16(a->scratch) || Dh * e % 16)
@@ -1650,7 +1677,14 @@ int artab_layer_stack(const artab_stack_args *a, int dtype, void *stream) {
     const artab_view q = head_view(0), k = head_view(1), v = head_view(2), out = {attn, a->N * D, Dh, D};
     const int64_t cache_h = static_cast<int64_t>(a->cache_rows) * Dh, cache_b = a->own_caches ? a->H * cache_h : 0;
     const artab_stack_layer *L = a->layers;
-    ARTAB_TRY(artab_layer_pre(a->x, D, L->w_fo, L->gamma1, L->beta1, L->eps1, L->w_qkv, base + s.y[0], qkv, rows, a->D, dtype, stream));
+    if (f32) {
+        F32LayerParams P{};
+        P.x = static_cast<const float *>(a->x);
+        ARTAB_TRY(launch_status(launch_f32_layer(f32_head(P, *L, base + s.y[0], qkv, rows), a->D, static_cast<hipStream_t>(stream)), "layer (float32)"));
+    } else {
+        ARTAB_TRY(artab_layer_pre(a->x, D, L->w_fo, L->gamma1, L->beta1, L->eps1, L->w_qkv, base + s.y[0], qkv, rows, a->D, dtype,
+                                  stream));
+    }
     for (int l = 0; l < a->n_layers; ++l, ++L) {
         if (!L->k_cache || !L->v_cache || misaligned16(L->k_cache) || misaligned16(L->v_cache))
             return fail(ARTAB_ERR_NULL_POINTER, "layer stack: layer %d needs 16-byte aligned caches", l);
@@ -1673,6 +1707,13 @@ int artab_layer_stack(const artab_stack_args *a, int dtype, void *stream) {
                                                       0.f, dtype, ARTAB_IMPL_AUTO, stream));
         }
         const char *y = base + s.y[l & 1];
+        if (f32) {
+            F32LayerParams P{};
+            f32_tail(P, *L, attn, y, a->out, rows);
+            if (l + 1 < a->n_layers) f32_head(P, L[1], base + s.y[1 - (l & 1)], qkv, rows);
+            ARTAB_TRY(launch_status(launch_f32_layer(P, a->D, static_cast<hipStream_t>(stream)), "layer (float32)"));
+            continue;
+        }
         if (l + 1 == a->n_layers)
             return artab_layer_post(attn, D, y, D, L->w_o, L->gamma2, L->beta2, L->eps2, L->w_1, L->b_1, L->w_2, L->b_2, L->gamma3,
                                     L->beta3, L->eps3, a->out, rows, a->D, a->F, dtype, stream);

@@ -93,6 +93,12 @@ F32Shape plan_f32(int H, int Nc, int Dh, int G, int n_groups);
 inline size_t f32_workspace_bytes(long rows, int Dh, int n_split) { return static_cast<size_t>(rows) * (Dh + 1) * n_split * 4; }
 hipError_t launch_f32_attention(PortableParams P, bool stacked, void *workspace, size_t workspace_bytes, hipStream_t stream);
 
+// f32_layer_launch.hip: float32 layers around the row attention (f32_layer.h), weights packed by launch_f32_pack
+struct F32LayerParams;
+bool f32_layer_width_ok(int D, int F);
+hipError_t launch_f32_layer(const F32LayerParams &P, int D, hipStream_t st);
+hipError_t launch_f32_pack(const float *w, float *packed, int N, int K, hipStream_t st);
+
 // backward_launch.hip: dQ launch, then dK/dV launch, of the training row attention.  `elem` is
 // the element type of every tensor; the matrix-core kernels take bf16 / f16 with head_dim 32 / 64.
 enum BackwardElem : int { kElemF32 = 0, kElemBf16 = 1, kElemF16 = 2 };

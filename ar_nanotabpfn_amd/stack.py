@@ -32,6 +32,22 @@ def _small_vectors(layer):
              p1["weight"], p2["weight"]))
 
 
+def _pack_f32(w: Tensor) -> Tensor:
+    w = w.detach().contiguous()
+    if w.data_ptr() % 16:
+        w = w.clone()
+    packed = torch.empty_like(w)
+    _lib.check(_lib.load().artab_pack_stack_weight_f32(w.data_ptr(), packed.data_ptr(), *w.shape, _lib.current_stream(w.device)))
+    return packed
+
+
+def _covered(layer, x: Tensor) -> bool:
+    """Whether the call has kernels for this layer's widths and type (``artab_layer_stack``)."""
+    if x.dtype == torch.float32:
+        return x.shape[-1] in (128, 256, 512) and layer.ff[0].out_features == 256
+    return layer.fused_for(x)
+
+
 class LayerStack:
     """What a pass reads of the layers, collected again whenever a parameter is another tensor or has been
     written to; each call looks at all of them."""
@@ -60,7 +76,10 @@ class LayerStack:
                 return False
         array, keep = (_lib.ArtabStackLayer * len(layers))(), []
         for a, layer, (v, w) in zip(array, layers, params):
-            packed = layer.packed_weights()
+            if x.dtype == torch.float32:
+                packed = tuple(_pack_f32(p) for p in (*layer.fused_weights(), *w[5:]))
+            else:
+                packed = layer.packed_weights()
             a.w_fo, a.w_qkv, a.w_o, a.w_1, a.w_2 = (t.data_ptr() for t in packed)
             a.b_1, a.b_2, a.gamma1, a.beta1, a.gamma2, a.beta2, a.gamma3, a.beta3 = (t.data_ptr() for t in v)
             a.eps1, a.eps2, a.eps3 = layer.norm1.eps, layer.norm2.eps, layer.norm3.eps
@@ -81,7 +100,7 @@ class LayerStack:
         own = k0.dim() == 4
         H, Dh, rows = first.attn_rows.n_heads, first.attn_rows.head_dim, k0.shape[-2]
         shape = (B, H, rows, Dh) if own else (H, rows, Dh)
-        if not (Dh in (32, 64, 128) and first.fused_for(x) and rows >= (N if num_targets == 0 else context_len + (N if own else 0))
+        if not (Dh in (32, 64, 128) and _covered(first, x) and rows >= (N if num_targets == 0 else context_len + (N if own else 0))
                 and (num_targets == 0 or context_len > 0)
                 and all(t.shape == shape and t.dtype == x.dtype and t.device == x.device and t.is_contiguous() and t.data_ptr() % 16 == 0
                         for c in caches for t in c)

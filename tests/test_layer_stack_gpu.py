@@ -43,3 +43,32 @@ def test_one_call_equals_layer_by_layer(device, monkeypatch, dtype, backend, B, 
     assert not torch.equal(after[0], before)
     for a, b in zip(after, run(False)):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("backend", ["shared_context", "per_dataset"])
+# one row, odd counts around the 16-row tile, more tiles than compute units
+@pytest.mark.parametrize("B,Nc,Nt,D,H", [(1, 1, 1, 128, 4), (3, 17, 5, 256, 8), (2, 333, 45, 512, 16), (64, 129, 65, 128, 2),
+                                         (41, 201, 103, 256, 4)])
+def test_float32_layers(device, monkeypatch, backend, B, Nc, Nt, D, H):
+    """The float32 layer kernels against the library's products around the same attention."""
+    torch.manual_seed(Nc)
+    model = ARTabPFN(d_model=D, n_heads=H, n_layers=3, d_ff=256, num_features=2).to(device).eval()
+    g = torch.Generator().manual_seed(Nt)
+    xc, xt = (torch.randn(B, n, 2, generator=g).to(device) for n in (Nc, Nt))
+    yc, yt = (torch.randn(B, n, generator=g).to(device) for n in (Nc, Nt))
+    names = ("k_ctx_cache", "v_ctx_cache") if backend == "shared_context" else ("k_cache", "v_cache")
+
+    def run(one_call):
+        p = ARTabPFNPredictor.from_trained_model(model, backend=backend)
+        stack = p._stack_pass
+        taken = []
+        monkeypatch.setattr(p, "_stack_pass", lambda *a: taken.append(stack(*a) if one_call else None) or taken[-1])
+        out = p.evaluate_joint_density(xc, yc, xt, yt)
+        assert len(taken) == 2 and all((t is not None) == one_call for t in taken)
+        return [out] + [getattr(layer, n).clone() for layer in model.backbone.layers for n in names]
+
+    # Sums of up to 512 float32 products in another order: each rounds at 2^-24 of its terms; three layers of five
+    # products and three norms, whose gain is of order one, stay under 1e-5 of the result's size.
+    for a, b in zip(run(True), run(False)):
+        assert ((a - b).double().norm() / b.double().norm().clamp(min=1e-30)).item() < 1e-5
+        assert torch.isfinite(a).all()
