@@ -20,6 +20,7 @@
 #include "mfma_flash.h"
 #include "portable_kernels.h"
 #include "queue_order.h"
+#include "context_small.h"
 #include "f32_layer.h"
 #include "launchers.h"
 
@@ -189,12 +190,12 @@ static FlashPlan plan_flash(int B, int H, int Lq, int Nc, int Dh, bool stacked, 
 // Key slices of a prefill.  One context has few query tiles: 5001 rows of 8 heads are 160 workgroups of
 // 256 rows, and cutting the tiles to 64 rows leaves wavefronts that wait for their own tiles (1.2 of
 // them per SIMD, 295 TFLOP/s).  Whole tiles with the keys dealt over workgroups, float32 partials and a
-// merge are faster from about 1000 rows on.  The choice weighs estimates in microseconds, fitted to
+// merge are faster from about 1000 rows on (shorter ones go to context_small_kernel, on one compute unit each).  The choice weighs estimates in microseconds, fitted to
 // launches of 200 to 16384 rows, 4 to 16 heads, 1 to 16 tables (bf16; f16 gains more everywhere): a
 // compute unit takes 12 ns per key for one tile, 17 for a pair, a slice costs 5 to start, the merge 5 and
 // its traffic at 3.5 TB/s; unsliced launches of small tiles take 12.5 to 21 ns per key, the more wavefronts
-// share a SIMD.  Unsliced -> sliced: 1 x 8 x 1024 17.1 -> 15.5, 4096 67 -> 36, 5001 81 -> 47, 9000 174 -> 122,
-// 12000 256 -> 185, 1 x 16 x 9000 246 -> 225; 700 rows 13.4 against 14.1, 8 x 8 x 512 14.2 against 17.8: not sliced.
+// share a SIMD.  Unsliced -> sliced: 1 x 16 x 2048 37.7 -> 26.4, 1 x 8 x 4096 67 -> 36, 5001 81 -> 47, 9000 174 -> 122,
+// 12000 256 -> 185, 1 x 16 x 9000 246 -> 225; 4 x 8 x 1024 20.9 against 20.5, 8 x 8 x 512 14.2 against 17.8: not sliced.
 static int prefill_slices(int B, int H, int Nc, int Dh) {
     if (Dh != 32) return 1;
     const int forced = tune(kTuneSplit, 0);
@@ -273,6 +274,28 @@ static hipError_t launch_small_t(const DecodeParams &P, const View &kc, const Vi
             launch_observed(kLaunchSmallDecode, decode_small_kernel<T, 64, 2>, grid, block, 0, stream, kp, vp, ksh, ksn, vsh,
                             vsn, P.H, Nc, P);
     }
+    return hipGetLastError();
+}
+
+// Calls that context_small_kernel takes (context attention and prefill): as long as its workgroups of 32 query
+// rows fit the chip at one per compute unit, and the context is neither so short that there is nothing to deal
+// out nor so long that every workgroup reading all of it costs more than the launch it saves.  us, mfma_flash.h (with
+// its merge) -> here: 8 rows, H 8, bf16: head_dim 64, 77 keys 5.7 -> 5.8, 512 11.1 -> 8.4, 2048 15.3 -> 15.8; head_dim 32,
+// 77 keys 5.1 -> 4.5, 512 9.0 -> 5.6, 2048 13.0 -> 9.6, 4096 14.9 -> 14.7; f16, whose other route is the online
+// softmax: 2048 x 64 18.8 -> 15.8.  1024 rows x 512 x 64: 17.2 -> 9.4; twice the rows 18.1 -> 18.0, four times 18.5 -> 32.8.
+// Prefill: 512 rows 10.9 -> 7.0, 1 x 8 x 1024 15.4 -> 9.0, 1500 rows (376 workgroups) 18.6 -> 18.3.
+static bool context_small_applies(int H, int Nc, int Dh, long tiles, int dtype) {
+    if (tune(kTuneSmall, 1) == 0 || tune(kTuneBM, 0) != 0 || tune(kTuneSplit, 0) != 0 || (Dh != 32 && Dh != 64)) return false;
+    return tiles * H <= 256 && Nc >= 64 && static_cast<long>(Nc) * Dh <= (dtype == ARTAB_F16 ? 2048L : 1536L) * 64;
+}
+
+template <typename T>
+static hipError_t launch_context_small(const ContextSmallParams &P, int Dh, int n_groups, hipStream_t st) {
+    const dim3 grid(static_cast<unsigned>(static_cast<long>(P.tiles) * n_groups * P.H)), block(kContextSmallWaves * 64);
+    if (Dh == 32)
+        hipLaunchKernelGGL((context_small_kernel<T, 32>), grid, block, 0, st, P);
+    else
+        hipLaunchKernelGGL((context_small_kernel<T, 64>), grid, block, 0, st, P);
     return hipGetLastError();
 }
 
@@ -520,6 +543,17 @@ int artab_context_attention(const artab_view *q, const artab_view *k_ctx, const 
 
     const bool stacked = (k_ctx->stride_b == 0 && v_ctx->stride_b == 0) || B == 1;
     const long rows = static_cast<long>(B) * H * Lq;
+    {
+        const long G = stacked ? static_cast<long>(B) * Lq : Lq, tiles = (G + kContextSmallRows - 1) / kContextSmallRows;
+        const int n_groups = stacked ? 1 : B;
+        if (impl == ARTAB_IMPL_AUTO && context_small_applies(H, Nc, Dh, tiles * n_groups, dtype)) {
+            const ContextSmallParams S = {dv(q), dv(k_ctx), dv(v_ctx), dv(out), lse, H, Lq, Nc, static_cast<int>(G),
+                                          static_cast<int>(tiles), stacked ? 1 : 0, scale * kLog2e, {}, {}, 0};
+            const hipError_t e = dtype == ARTAB_BF16 ? launch_context_small<bf16_t>(S, Dh, n_groups, st)
+                                                     : launch_context_small<f16_t>(S, Dh, n_groups, st);
+            return launch_status(e, "context attention (small)");
+        }
+    }
     FlashPlan pl = plan_flash(B, H, Lq, Nc, Dh, stacked, /*allow_split=*/true);
     if (pl.n_split > 1) {
         size_t need = split_workspace_bytes(rows, Dh, pl.n_split);
@@ -1155,6 +1189,14 @@ static int prefill_impl(const artab_view *q, const artab_view *k, const artab_vi
         return launch_status(launch_portable_or_f32(P, dtype, impl, false, st), "prefill");
     }
     const long rows = static_cast<long>(B) * H * Nc;
+    const long small_tiles = (Nc + kContextSmallRows - 1) / kContextSmallRows;
+    if (impl == ARTAB_IMPL_AUTO && context_small_applies(H, Nc, Dh, small_tiles * B, dtype)) {
+        const ContextSmallParams S = {dv(q), dv(k), dv(v), dv(out), nullptr, H, Nc, Nc, Nc, static_cast<int>(small_tiles), 0,
+                                      scale * kLog2e, dv(kc_given ? k_cache : nullptr), dv(kc_given ? v_cache : nullptr),
+                                      kc_given ? cache_batches : 0};
+        const hipError_t e = dtype == ARTAB_BF16 ? launch_context_small<bf16_t>(S, Dh, B, st) : launch_context_small<f16_t>(S, Dh, B, st);
+        return launch_status(e, "prefill (small)");
+    }
     const int slices = prefill_slices(B, H, Nc, Dh);
     FlashPlan pl = plan_flash(B, H, Nc, Nc, Dh, /*stacked=*/false, /*allow_split=*/false);
     if (slices > 1 && workspace && workspace_bytes >= f32_workspace_bytes(rows, Dh, slices) &&
@@ -1194,6 +1236,7 @@ static int prefill_impl(const artab_view *q, const artab_view *k, const artab_vi
 
 size_t artab_prefill_workspace_bytes(int B, int H, int Nc, int Dh, int dtype) {
     if (B <= 0 || H <= 0 || Nc <= 0 || !mfma_shape_ok(dtype, Dh)) return 0;
+    if (context_small_applies(H, Nc, Dh, static_cast<long>((Nc + kContextSmallRows - 1) / kContextSmallRows) * B, dtype)) return 0;
     const int slices = prefill_slices(B, H, Nc, Dh);
     return slices > 1 ? f32_workspace_bytes(static_cast<long>(B) * H * Nc, Dh, slices) : 0;
 }
