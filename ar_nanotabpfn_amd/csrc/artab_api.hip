@@ -1430,7 +1430,7 @@ static int fill_post(FusedPostParams &P, const void *attn, int64_t lda, const vo
 // Ordering that a partial descriptor asks of its consumer.  The wait goes into the kernel when its grid leaves half of the compute units
 // free — a waiting workgroup must not keep the buffer pass it waits for off the chip — and into a
 // launch of its own otherwise.
-static int apply_partials_order(const artab_attention_partials *parts, FusedPostParams &P, int64_t rows,
+static int apply_partials_order(const artab_attention_partials *parts, FusedPostParams &P, int64_t rows, int D,
                                 hipStream_t st, int64_t grid_of_launch = -1) {
     if (!parts || !(parts->order_flags & ARTAB_ORDER_WAIT)) return ARTAB_OK;
     ARTAB_TRY(check_order_args(parts->order_state, ARTAB_ORDER_MAIN));
@@ -1440,8 +1440,9 @@ static int apply_partials_order(const artab_attention_partials *parts, FusedPost
         if (hipGetDevice(&dev) != hipSuccess ||
             hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
             cus = 0;
+        const int tile_rows = fused_tile_rows(rows, fused_small_max_rows(D));
         const int64_t grid =
-            grid_of_launch >= 0 ? grid_of_launch : (rows + fused_tile_rows(rows) - 1) / fused_tile_rows(rows);
+            grid_of_launch >= 0 ? grid_of_launch : (rows + tile_rows - 1) / tile_rows;
         const uint64_t us = parts->order_timeout_us ? parts->order_timeout_us : 2000000;
         if (grid * 2 <= cus && tune(kTuneOrderGateLaunch, 0) == 0) {
             P.order_wait = parts->order_state;
@@ -1501,7 +1502,7 @@ static int layer_post_pre_impl(const artab_attention_partials *parts, const void
     ARTAB_TRY(fill_pre(N, nullptr, 0, next_w_fo, next_ln1_gamma, next_ln1_beta, next_eps1, next_w_qkv, next_y,
                        next_qkv, rows, D, false));
     hipStream_t st = static_cast<hipStream_t>(stream);
-    ARTAB_TRY(apply_partials_order(parts, P, rows, st));
+    ARTAB_TRY(apply_partials_order(parts, P, rows, D, st));
     if (rows == 0) return ARTAB_OK;
     hipError_t e = launch_layer_post_pre(P, N, D, F, dtype == ARTAB_BF16, st);
     return launch_status(e, "layer_post_pre");
@@ -1543,7 +1544,7 @@ int artab_layer_post_from_partials(const artab_attention_partials *parts, const 
     ARTAB_TRY(fill_post(P, nullptr, 0, y, ldy, w_o, ln2_gamma, ln2_beta, eps2, w_1, b_1, w_2, b_2, ln3_gamma,
                         ln3_beta, eps3, out, rows, D, F, true, parts));
     hipStream_t st = static_cast<hipStream_t>(stream);
-    ARTAB_TRY(apply_partials_order(parts, P, rows, st));
+    ARTAB_TRY(apply_partials_order(parts, P, rows, D, st));
     if (rows == 0) return ARTAB_OK;
     hipError_t e = launch_layer_post(P, D, F, dtype == ARTAB_BF16, st);
     return launch_status(e, "layer_post");
@@ -1605,9 +1606,9 @@ int artab_decode_step_boundary(const artab_attention_partials *parts, const void
     if (F != tail->F)
         return fail(ARTAB_ERR_UNSUPPORTED, "decode_step_boundary: head width %d differs from the layers' feed-forward width %d",
                     tail->F, F);
-    if (fused_tile_rows(2 * B) != kFusedRowsSmall || fused_tile_rows(B) != kFusedRowsSmall)
+    if (fused_tile_rows(2 * B, kFusedTailMaxRows) != kFusedRowsSmall || fused_tile_rows(B, kFusedTailMaxRows) != kFusedRowsSmall)
         return fail(ARTAB_ERR_UNSUPPORTED, "decode_step_boundary covers up to %ld trajectories on %d-row tiles",
-                    kFusedSmallMaxRows / 2, kFusedRowsSmall);
+                    kFusedTailMaxRows / 2, kFusedRowsSmall);
     if (parts && parts->n_slots == 0) parts = nullptr;  // the call that made them wrote `attn` instead
     FusedPostParams P{};
     FusedPreParams N{};
@@ -1616,7 +1617,7 @@ int artab_decode_step_boundary(const artab_attention_partials *parts, const void
     ARTAB_TRY(fill_pre(N, nullptr, 0, next_w_fo, next_ln1_gamma, next_ln1_beta, next_eps1, next_w_qkv, next_y, next_qkv,
                        2 * B, D, false));
     hipStream_t st = static_cast<hipStream_t>(stream);
-    ARTAB_TRY(apply_partials_order(parts, P, B, st, (B + kFusedRowsSmall / 2 - 1) / (kFusedRowsSmall / 2)));
+    ARTAB_TRY(apply_partials_order(parts, P, B, D, st, (B + kFusedRowsSmall / 2 - 1) / (kFusedRowsSmall / 2)));
     if (B == 0) return ARTAB_OK;
     hipError_t e = launch_step_boundary(P, S, N, D, F, dtype == ARTAB_BF16, st);
     return launch_status(e, "decode_step_boundary");

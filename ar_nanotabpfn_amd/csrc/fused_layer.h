@@ -31,7 +31,12 @@ constexpr int kFusedRowsSmall = 16;  // ... or, when that leaves most of the chi
                                      // 2048 rows = 64 workgroups of 32, and everything a workgroup does
                                      // per row (merge, LayerNorm, epilogues) is bound by its one CU's
                                      // instruction issue
-constexpr long kFusedSmallMaxRows = 8192;  // up to here the 16-row tiles are used
+// Up to here the 16-row tiles are used.  At d_model 256 and 512 a compute unit's second tile costs as much as its first
+// (all of it waits for the weight stream), so the line is where 256 of them are used up: one layer boundary at d_model
+// 256, 16- against 32-row tiles, 4096 rows 14.6 / 17.4 us, 4200 24.9 / 17.4, 8192 26.0 / 19.2; d_model 512 37.7 / 47.9,
+// 69.6 / 47.6, 70.2 / 52.7.  At 128 two tiles share one: 8192 rows 12.8 / 14.2, 9000 19.1 / 16.7.
+constexpr long fused_small_max_rows(int D) { return D == 128 ? 8192 : 4096; }
+constexpr long kFusedTailMaxRows = 8192;  // of the step tail and the step boundary
 
 // Stands in for an absent bias vector (1024 16-bit zeros; widths go up to 512).
 static __device__ const unsigned int kZeroVector[512] = {0u};

@@ -44,11 +44,11 @@ int tune(Tune key, int fallback);
 
 // Token rows per workgroup of the layer kernels: 16 while that still leaves the launch within a
 // few workgroups per CU (everything a workgroup does per row is bound by its one CU), else 32
-// (half the weight traffic per row).
-inline int fused_tile_rows(long rows) {
+// (half the weight traffic per row).  small_max: fused_small_max_rows of the layer, or kFusedTailMaxRows.
+inline int fused_tile_rows(long rows, long small_max) {
     const int v = tune(kTuneTileRows, 0);
     if (v == kFusedRows || v == kFusedRowsSmall) return v;
-    return rows <= kFusedSmallMaxRows ? kFusedRowsSmall : kFusedRows;
+    return rows <= small_max ? kFusedRowsSmall : kFusedRows;
 }
 
 // What a benchmark build of the library hangs on a kernel launch: a pair of events that receive

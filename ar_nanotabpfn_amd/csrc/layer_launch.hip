@@ -29,7 +29,7 @@ hipError_t launch_pre_r(const FusedPreParams &P, int D, hipStream_t st) {
 }
 template <typename T>
 hipError_t launch_pre(const FusedPreParams &P, int D, hipStream_t st) {
-    return fused_tile_rows(P.rows) == kFusedRowsSmall ? launch_pre_r<T, kFusedRowsSmall>(P, D, st)
+    return fused_tile_rows(P.rows, fused_small_max_rows(D)) == kFusedRowsSmall ? launch_pre_r<T, kFusedRowsSmall>(P, D, st)
                                                       : launch_pre_r<T, kFusedRows>(P, D, st);
 }
 
@@ -83,7 +83,7 @@ hipError_t launch_post_pre_r(const FusedPostParams &P, const FusedPreParams &N, 
 }
 template <typename T>
 hipError_t launch_post_pre(const FusedPostParams &P, const FusedPreParams &N, int D, int F, hipStream_t st) {
-    return fused_tile_rows(P.rows) == kFusedRowsSmall ? launch_post_pre_r<T, kFusedRowsSmall>(P, N, D, F, st)
+    return fused_tile_rows(P.rows, fused_small_max_rows(D)) == kFusedRowsSmall ? launch_post_pre_r<T, kFusedRowsSmall>(P, N, D, F, st)
                                                       : launch_post_pre_r<T, kFusedRows>(P, N, D, F, st);
 }
 
@@ -97,7 +97,7 @@ hipError_t launch_post_r(const FusedPostParams &P, int D, int F, hipStream_t st)
 }
 template <typename T>
 hipError_t launch_post(const FusedPostParams &P, int D, int F, hipStream_t st) {
-    return fused_tile_rows(P.rows) == kFusedRowsSmall ? launch_post_r<T, kFusedRowsSmall>(P, D, F, st)
+    return fused_tile_rows(P.rows, fused_small_max_rows(D)) == kFusedRowsSmall ? launch_post_r<T, kFusedRowsSmall>(P, D, F, st)
                                                       : launch_post_r<T, kFusedRows>(P, D, F, st);
 }
 
@@ -122,7 +122,7 @@ hipError_t launch_sample_r(const SampleEmbedParams &P, int D, int F, hipStream_t
 }
 template <typename T>
 hipError_t launch_sample(const SampleEmbedParams &P, int D, int F, hipStream_t st) {
-    return fused_tile_rows(P.B) == kFusedRowsSmall ? launch_sample_r<T, kFusedRowsSmall>(P, D, F, st)
+    return fused_tile_rows(P.B, kFusedTailMaxRows) == kFusedRowsSmall ? launch_sample_r<T, kFusedRowsSmall>(P, D, F, st)
                                                    : launch_sample_r<T, kFusedRows>(P, D, F, st);
 }
 

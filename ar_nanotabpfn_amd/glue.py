@@ -282,7 +282,7 @@ class DecodeStepBoundary:
     ``TwoStageTransformerLayer.pre_attention`` returns.
     """
 
-    MAX_TRAJECTORIES = 4096  # twice as many rows still take the 16-row tiles of the layer kernels
+    MAX_TRAJECTORIES = 4096  # the launch is built for 16-row tiles of both parts
     # At d_model 512 a workgroup streams 3 MB of weights and is bound by that; eight trajectories
     # per workgroup instead of sixteen rows then double the traffic of the first two parts for
     # nothing (measured at B=2048, d_model 512: 457 against 462 target-steps/s with three launches).
