@@ -175,7 +175,7 @@ SIGNATURES = {
     "artab_row_mask_attention_backward": (
         _i, [_VP, _VP, _VP, _VP, _VP, _p, _p, _VP, _VP, _VP, _i, _i, _i, _i, _i, _i, _i, _f, _i, _i, _p]),
     "artab_prefill_attention": (_i, [_VP, _VP, _VP, _VP, _VP, _VP, _i, _i, _i, _i, _i, _f, _i, _i, _p]),
-    "artab_pack_stack_weight_f32": (_i, [_p, _p, _i, _i, _p]),
+    "artab_pack_stack_weight_float": (_i, [_p, _p, _i, _i, _p]),
     "artab_layer_stack_scratch_bytes": (_sz, [_p, _i]),
     "artab_layer_stack": (_i, [_p, _i, _p]),
     "artab_prefill_workspace_bytes": (_sz, [_i, _i, _i, _i, _i]),

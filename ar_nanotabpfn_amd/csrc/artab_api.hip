@@ -1688,7 +1688,7 @@ int check_stack(const artab_stack_args *a) {
 }
 }  // namespace
 
-int artab_pack_stack_weight_f32(const void *w, void *packed, int N, int K, void *stream) {
+int artab_pack_stack_weight_float(const void *w, void *packed, int N, int K, void *stream) {
     if (N <= 0 || K <= 0 || N % 16 || K % 16) return fail(ARTAB_ERR_BAD_SHAPE, "pack: N and K must be multiples of 16 (got %d, %d)", N, K);
     if (!w || !packed) return fail(ARTAB_ERR_NULL_POINTER, "pack: null pointer");
     if (misaligned16(w) || misaligned16(packed)) return fail(ARTAB_ERR_BAD_STRIDE, "pack: pointers must be 16-byte aligned");

@@ -37,7 +37,7 @@ def _pack_f32(w: Tensor) -> Tensor:
     if w.data_ptr() % 16:
         w = w.clone()
     packed = torch.empty_like(w)
-    _lib.check(_lib.load().artab_pack_stack_weight_f32(w.data_ptr(), packed.data_ptr(), *w.shape, _lib.current_stream(w.device)))
+    _lib.check(_lib.load().artab_pack_stack_weight_float(w.data_ptr(), packed.data_ptr(), *w.shape, _lib.current_stream(w.device)))
     return packed
 
 

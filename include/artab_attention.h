@@ -585,7 +585,7 @@ typedef struct artab_stack_args {
     void *scratch;           /* artab_layer_stack_scratch_bytes, 16-byte aligned, the call's own while it runs */
 } artab_stack_args;
 /* float32 (D in {128, 256, 512}, F = 256): the weights [N, K] packed by this, N K floats each, 16-byte aligned */
-int artab_pack_stack_weight_f32(const void *w, void *packed, int N, int K, void *stream);
+int artab_pack_stack_weight_float(const void *w, void *packed, int N, int K, void *stream);
 size_t artab_layer_stack_scratch_bytes(const artab_stack_args *args, int dtype);
 int artab_layer_stack(const artab_stack_args *args, int dtype, void *stream);
 
