@@ -28,7 +28,8 @@
 // every column, a trajectory's own rows only its two columns (the others are masked, their state does
 // not change), so no merge of partial results is needed.  The first blocks are requested ahead of the
 // q/k/v product.  The rows of this step that have just been projected are keys too: one last block
-// straight from LDS, masked to (row 2 g, columns 2 g and 2 g + 1).  Softmax in float32 with scale *
+// straight from LDS, masked to (row 2 g, columns 2 g and 2 g + 1).  A value that is not finite stays with
+// the columns that see it: products of keys that only some columns see reach those columns only.  Softmax in float32 with scale *
 // log2(e) folded into the queries and rounded to the model's type, probabilities rounded to the
 // model's type: the rounding model of the other kernels.  The reference a column's probabilities are
 // taken against follows its maximum only when that has risen by more than kSlack (base 2): the common
@@ -192,7 +193,8 @@ __global__ void trajectory_tape_kernel(const T *w, char *tape, long tape_stride,
     *reinterpret_cast<u32x4 *>(tape + wave * tape_stride + (static_cast<long>(first) + ks * stride + offset + b) * 1024 +
                                16 * lane) = v;
 }
-template <typename T, int D, int F>
+// SEVERAL: G > 1.  (One trajectory has no columns to keep apart: doing it all the same costs 3 % of a run.)
+template <typename T, int D, int F, bool SEVERAL>
 __global__ __launch_bounds__(kTrajWaves * 64) void trajectory_decode_kernel(TrajectoryParams P) {
     typedef TrajOps<T> Ops;
     typedef TrajShape<T, D, F> S;
@@ -456,7 +458,10 @@ __global__ __launch_bounds__(kTrajWaves * 64) void trajectory_decode_kernel(Traj
             }
             return r;
         };
-        auto compute = [&](Block &r, int i) {  // block i; the wavefront's block after next goes where this one was
+        // Block i; the wavefront's block after next goes where this one was.  With SEVERAL, a trajectory's block
+        // is masked for the columns of the others, and they keep what they have: their probabilities are
+        // zeros, but a zero times a value that is not finite is not zero.
+        auto compute = [&](Block &r, int i) {
             constexpr int NX = BK / 16;
             const int row0 = r.row0, n = r.n, g = r.g;
             f32x4 sc[NX];
@@ -472,9 +477,14 @@ __global__ __launch_bounds__(kTrajWaves * 64) void trajectory_decode_kernel(Traj
                 sc[0] = Ops::mma(r.k[1], qf[1], sc[0]);
                 Ops::finish(sc[0]);
             }
-            if (row0 + BK > n || (g >= 0 && valid > 1)) {
-                // (with one trajectory the other columns are nobody's)
-                const bool mine = g < 0 || valid == 1 || (tok >> 1) == g;
+            // (with one trajectory the other columns are nobody's)
+            const bool mine = !SEVERAL || g < 0 || (tok >> 1) == g;
+            auto add = [&](f32x4 &o, const u32x4 &v, const u32x4 &pv) {
+                const f32x4 sum = Ops::mma(v, pv, o);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o[e] = mine ? sum[e] : o[e];
+            };
+            if (row0 + BK > n || (SEVERAL && g >= 0)) {
 #pragma unroll
                 for (int x = 0; x < NX; ++x)
 #pragma unroll
@@ -491,13 +501,13 @@ __global__ __launch_bounds__(kTrajWaves * 64) void trajectory_decode_kernel(Traj
                     const T *a = vt + (4 * quad + (row16 >> 2)) * VPAD + 16 * db + 4 * (lane & 3);
                     const s16x4 lo = tr_read(a), hi = tr_read(a + 16 * VPAD);
                     const s16x8 both = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-                    o_acc[db] = Ops::mma(__builtin_bit_cast(u32x4, both), pv, o_acc[db]);
+                    add(o_acc[db], __builtin_bit_cast(u32x4, both), pv);
                 }
                 __builtin_amdgcn_wave_barrier();
             } else {
                 const u32x4 pv = p_operand(sc[0]);
 #pragma unroll
-                for (int db = 0; db < 2; ++db) o_acc[db] = Ops::mma(r.v[db], pv, o_acc[db]);
+                for (int db = 0; db < 2; ++db) add(o_acc[db], r.v[db], pv);
                 fetch(h, i + 2 * NP, r);
             }
         };
@@ -516,24 +526,19 @@ __global__ __launch_bounds__(kTrajWaves * 64) void trajectory_decode_kernel(Traj
 #pragma unroll
             for (int e = 0; e < 4; ++e)
                 if (4 * sub + e != (tok & ~1)) sc[0][e] = -INFINITY;
+            // One key per column: its probability to every lane of the column, and the products of the column's
+            // own row (a matrix product over the rows of all trajectories would multiply each by all of them).
+            float vr[2][4];
+#pragma unroll
+            for (int db = 0; db < 2; ++db) traj_load4<T>(vn + (tok & ~1) * LD + DH * h + 16 * db + 4 * sub, vr[db]);
             fold(sc);
-            if constexpr (k16) {
-                const u32x4 pv = {pack2<T>(sc[0][0], sc[0][1]), pack2<T>(sc[0][2], sc[0][3]), 0u, 0u};
+            float p = Ops::sum((sc[0][0] + sc[0][1]) + (sc[0][2] + sc[0][3]));
+            if constexpr (k16) p = to_f32(from_f32<T>(p));
+            if (k16 || quad == 0) {  // (float32: the four rows of lanes are partial sums)
 #pragma unroll
-                for (int db = 0; db < 2; ++db) {
-                    const s16x4 lo = tr_read(vn + (4 * quad + (row16 >> 2)) * LD + DH * h + 16 * db + 4 * (lane & 3));
-                    const s16x8 both = {lo[0], lo[1], lo[2], lo[3], 0, 0, 0, 0};
-                    o_acc[db] = Ops::mma(__builtin_bit_cast(u32x4, both), pv, o_acc[db]);
-                }
-            } else {
-                const u32x4 pv = p_operand(sc[0]);
+                for (int db = 0; db < 2; ++db)
 #pragma unroll
-                for (int db = 0; db < 2; ++db) {
-                    u32x4 vf;  // (rows past the fourth do not exist: their probabilities are zero)
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) vf[j] = __builtin_bit_cast(unsigned, vn[j * LD + DH * h + 16 * db + row16]);
-                    o_acc[db] = Ops::mma(vf, pv, o_acc[db]);
-                }
+                    for (int e = 0; e < 4; ++e) o_acc[db][e] = fmaf(p, vr[db][e], o_acc[db][e]);
             }
         }
         float l_tot = Ops::sum(l_run);

@@ -74,8 +74,11 @@ template <typename T>
 hipError_t decode(const TrajectoryParams &P, int D, int F, hipStream_t st) {
     hipError_t e = hipErrorInvalidValue;
     with_shape<T>(D, F, [&](auto d, auto f) {
-        hipLaunchKernelGGL((trajectory_decode_kernel<T, decltype(d)::value, decltype(f)::value>),
-                           dim3(static_cast<unsigned>((P.B + P.G - 1) / P.G)), dim3(kTrajWaves * 64), 0, st, P);
+        const dim3 grid(static_cast<unsigned>((P.B + P.G - 1) / P.G)), block(kTrajWaves * 64);
+        if (P.G > 1)
+            hipLaunchKernelGGL((trajectory_decode_kernel<T, decltype(d)::value, decltype(f)::value, true>), grid, block, 0, st, P);
+        else
+            hipLaunchKernelGGL((trajectory_decode_kernel<T, decltype(d)::value, decltype(f)::value, false>), grid, block, 0, st, P);
         e = hipGetLastError();
     });
     return e;
