@@ -29,6 +29,8 @@
 // otherwise every wavefront has its own tile.
 #pragma once
 
+#include <type_traits>
+
 #include "common.h"
 #include "portable_kernels.h"
 
@@ -129,13 +131,13 @@ __global__ __launch_bounds__(NW * 64) void f32_attention_kernel(PortableParams P
     const int n_ctx_t = (P.Nc + 31) / 32, per_traj = (buf_max + 31) / 32;
     const int n_buf_t = n_traj * per_traj, n_new_t = has_new ? (n_traj + 31) / 32 : 0;
     const int n_tasks = n_ctx_t + n_buf_t + n_new_t;
-    int t_now, t_end, t_step;
+    int t_first, t_end, t_step;
     if (SPLIT) {
-        t_now = static_cast<int>(static_cast<long>(n_tasks) * slice / L.n_split) + wave;
+        t_first = static_cast<int>(static_cast<long>(n_tasks) * slice / L.n_split) + wave;
         t_end = static_cast<int>(static_cast<long>(n_tasks) * (slice + 1) / L.n_split);
         t_step = NW;
     } else {
-        t_now = 0;
+        t_first = 0;
         t_end = n_tasks;
         t_step = 1;
     }
@@ -176,33 +178,45 @@ __global__ __launch_bounds__(NW * 64) void f32_attention_kernel(PortableParams P
                 kf[sb][t] = *reinterpret_cast<const f32x4 __attribute__((address_space(1))) *>(B.k + (row + 64 * t));
         }
     };
+    auto load_v = [&](const Block &B, int key, fvec (&v)[VN]) {  // this lane's piece of a value row
+        const unsigned row = min(key * B.v_sn, B.last * B.v_sn) + 4 * KT * c;
+#pragma unroll
+        for (int n = 0; n < VN; ++n) v[n] = *reinterpret_cast<const fvec __attribute__((address_space(1))) *>(B.v + (row + 16 * n));
+    };
     auto request_v = [&](const Block &B) {
 #pragma unroll
         for (int sb = 0; sb < 2; ++sb)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const unsigned row = min((B.key0 + 16 * sb + 4 * g + r) * B.v_sn, B.last * B.v_sn) + 4 * KT * c;
-#pragma unroll
-                for (int n = 0; n < VN; ++n)
-                    vf[sb][r][n] = *reinterpret_cast<const fvec __attribute__((address_space(1))) *>(B.v + (row + 16 * n));
-            }
+            for (int r = 0; r < 4; ++r) load_v(B, B.key0 + 16 * sb + 4 * g + r, vf[sb][r]);
     };
 
+    // The wavefront's tasks.  A key that is hidden from a column has probability 0 there, and 0 times a value that
+    // is not finite is NaN: the pass that multiplies every value of a block by every column watches for
+    // such values in blocks that are hidden from somebody (the context is hidden from nobody; its last
+    // block repeats a row that everybody sees) and, if there were any, is followed by a second one,
+    // CAREFUL: column after column, with zeros for the values that the column does not see, and with
+    // nothing requested ahead, so that it needs no registers that the common pass does not.
     f32x4 o[QB][KT];
     float m[QB], l[QB];
+    auto pass = [&](auto careful) {
+        constexpr bool CAREFUL = decltype(careful)::value;
+        float watch = 0.f;  // NaN: values that are not finite
 #pragma unroll
-    for (int j = 0; j < QB; ++j) {
-        m[j] = -INFINITY;
-        l[j] = 0.f;
+        for (int j = 0; j < QB; ++j) {
+            m[j] = -INFINITY;
+            l[j] = 0.f;
 #pragma unroll
-        for (int n = 0; n < KT; ++n) o[j][n] = f32x4{0.f, 0.f, 0.f, 0.f};
-    }
-
-    if (t_now < t_end) {
+            for (int n = 0; n < KT; ++n) o[j][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+        int t_now = t_first;
+        if (t_now >= t_end) return false;
         Block cur = block_of(t_now);
-        request_k(cur);
-        request_v(cur);
+        if (!CAREFUL) {
+            request_k(cur);
+            request_v(cur);
+        }
         for (; t_now < t_end; t_now += t_step) {
+            if (CAREFUL) request_k(cur);
             const int t_next = t_now + t_step < t_end ? t_now + t_step : t_now;
             const Block next = block_of(t_next);
             // (a trajectory's columns are within one block of 16: other blocks sit its buffer out)
@@ -222,7 +236,7 @@ __global__ __launch_bounds__(NW * 64) void f32_attention_kernel(PortableParams P
                         for (int e = 0; e < 4; ++e)
                             s[j][sb] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[sb][t][e], q[j][4 * t + e], s[j][sb], 0, 0, 0);
             }
-            request_k(next);
+            if (!CAREFUL) request_k(next);
 #pragma unroll
             for (int j = 0; j < QB; ++j) {
                 if (one && only != j) continue;
@@ -235,7 +249,8 @@ __global__ __launch_bounds__(NW * 64) void f32_attention_kernel(PortableParams P
                     lo = traj[j];
                     hi = traj[j] + 1;
                 }
-                if (__any(hi < cur.key0 + 32 || lo > cur.key0)) {
+                const bool hidden = __any(hi < cur.key0 + 32 || lo > cur.key0);
+                if (hidden) {
 #pragma unroll
                     for (int sb = 0; sb < 2; ++sb)
 #pragma unroll
@@ -264,22 +279,58 @@ __global__ __launch_bounds__(NW * 64) void f32_attention_kernel(PortableParams P
                         s[j][sb][r] = fast_exp2(s[j][sb][r] - m_use);
                         l[j] += s[j][sb][r];
                     }
+                const bool masked = hidden && cur.kind != 0;
+                auto value = [&](const fvec (&v)[VN], int n) {
+                    if constexpr (KT < 4) return v[0][n];
+                    else return v[n / 4][n % 4];
+                };
+                if constexpr (CAREFUL) {
+                    const int n_cols = masked ? 16 : 1;
+#pragma unroll 1
+                    for (int col = 0; col < n_cols; ++col) {
+                        const int lo_c = masked ? __builtin_amdgcn_readlane(lo, col) : 0;
+                        const int hi_c = masked ? __builtin_amdgcn_readlane(hi, col) : 0x7fffffff;
+                        f32x4 sum[KT];
 #pragma unroll
-                for (int sb = 0; sb < 2; ++sb)
+                        for (int n = 0; n < KT; ++n) sum[n] = o[j][n];
 #pragma unroll
-                    for (int r = 0; r < 4; ++r)
+                        for (int x = 0; x < 8; ++x) {
+                            __builtin_amdgcn_sched_barrier(0);
+                            const int key = cur.key0 + 16 * (x >> 2) + 4 * g + (x & 3);
+                            fvec v[VN];
+                            load_v(cur, key, v);
 #pragma unroll
-                        for (int n = 0; n < KT; ++n) {
-                            float a;
-                            if constexpr (KT < 4) a = vf[sb][r][0][n];
-                            else a = vf[sb][r][n / 4][n % 4];
-                            o[j][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, s[j][sb][r], o[j][n], 0, 0, 0);
+                            for (int n = 0; n < KT; ++n)
+                                sum[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(key >= lo_c && key < hi_c ? value(v, n) : 0.f,
+                                                                              s[j][x >> 2][x & 3], sum[n], 0, 0, 0);
                         }
+#pragma unroll
+                        for (int n = 0; n < KT; ++n)
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) o[j][n][e] = !masked || c == col ? sum[n][e] : o[j][n][e];
+                    }
+                } else {
+                    if (masked) {
+#pragma unroll
+                        for (int x = 0; x < 8; ++x)
+#pragma unroll
+                            for (int n = 0; n < KT; ++n) watch = fmaf(value(vf[x >> 2][x & 3], n), 0.f, watch);
+                    }
+#pragma unroll
+                    for (int sb = 0; sb < 2; ++sb)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r)
+#pragma unroll
+                            for (int n = 0; n < KT; ++n)
+                                o[j][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(value(vf[sb][r], n), s[j][sb][r], o[j][n], 0, 0, 0);
+                }
             }
-            request_v(next);
+            if (!CAREFUL) request_v(next);
             cur = next;
         }
-    }
+        return __any(watch != 0.f) != 0;
+    };
+    if (pass(std::false_type{})) pass(std::true_type{});
 #pragma unroll
     for (int j = 0; j < QB; ++j) l[j] = row_sum(l[j]);
 
