@@ -26,6 +26,7 @@ from torch import Tensor
 from . import attention_kernels as ak
 from .attention import DecodeMask, TeacherForcingMask
 from . import _lib
+from .live import ModelState
 from .stack import LayerStack
 from .glue import SampleEmbedStep, DecodeStepBoundary, TrajectoryDecoder, add_layer_norm
 
@@ -101,7 +102,7 @@ class ARTabPFNPredictor:
         self._trajectory = None      # (key of the model state, TrajectoryDecoder or None)
         self._side_streams = {}
         self._graph_state = None
-        self._graph_params = None    # the tensors a recorded step points at (collected at first use)
+        self._model_state = ModelState()  # (what a recorded step points at is held by it)
         self.graph_recordings = 0    # HIP graphs recorded so far (a run that only replays leaves it unchanged)
 
     @classmethod
@@ -413,13 +414,9 @@ class ARTabPFNPredictor:
         return torch.cat(preds, dim=1)
 
     def _model_key(self):
-        """What identifies the state of the model's weights, and the tensors it was taken from."""
-        # (walking the module tree costs a millisecond of host time with the GPU idle: done once; a
-        # weight that is updated or moved changes its version or address and is seen through the key)
-        if self._graph_params is None:
-            self._graph_params = (list(self.backbone.parameters()) + list(self.embedder.parameters()) +
-                                  list(self.head.parameters()) + [self.ar_tokens])
-        return tuple((p.data_ptr(), p._version) for p in self._graph_params)
+        """What identifies the state of the model: another number when any module, parameter or constant of it
+        is another one or has been written to."""
+        return self._model_state.look((self.backbone, self.embedder, self.head), self.ar_tokens)
 
     def _sample_whole_run(self, x_target: Tensor) -> Optional[Tensor]:
         """The sampling run as one launch (``TrajectoryDecoder``), or None where it does not apply.  The

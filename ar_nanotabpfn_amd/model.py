@@ -26,6 +26,7 @@ from torch import Tensor, nn
 from .attention import DenseMask, MultiheadAttention, RowMask
 from .glue import add_layer_norm, bias_gelu, layer_fusable, layer_post, layer_post_pre, layer_pre, pack_weight
 
+from .live import Sources
 from .training import embed_rows, layer_stack, layer_stack_supported
 
 __all__ = ["Embedder", "TwoStageTransformerLayer", "TwoStageTransformer", "MixtureGaussianHead", "ARTabPFN"]
@@ -103,13 +104,12 @@ class TwoStageTransformerLayer(nn.Module):
         """
         af, ar = self.attn_features, self.attn_rows
         srcs = (af.v_proj.weight, af.out_proj.weight, ar.q_proj.weight, ar.k_proj.weight, ar.v_proj.weight)
-        key = tuple((p.data_ptr(), p._version, p.dtype, p.device) for p in srcs)
-        cached = getattr(self, "_fused_cache", None)
-        if cached is None or cached[0] != key:
+        cached = self.__dict__.get("_fused_cache")
+        if cached is None or not cached[0].unchanged(srcs):
             with torch.no_grad():
                 w_fo = (af.out_proj.weight.float() @ af.v_proj.weight.float()).to(af.v_proj.weight.dtype)
                 w_qkv = torch.cat([ar.q_proj.weight, ar.k_proj.weight, ar.v_proj.weight], dim=0).contiguous()
-            cached = (key, w_fo, w_qkv)
+            cached = (Sources(srcs), w_fo, w_qkv)
             self._fused_cache = cached
         return cached[1], cached[2]
 
@@ -138,10 +138,9 @@ class TwoStageTransformerLayer(nn.Module):
         ``(w_fo, w_qkv, out_proj, ff[0], ff[2])``."""
         w_fo, w_qkv = self.fused_weights()
         srcs = (w_fo, w_qkv, self.attn_rows.out_proj.weight, self.ff[0].weight, self.ff[2].weight)
-        key = tuple((p.data_ptr(), p._version, p.dtype, p.device) for p in srcs)
-        cached = getattr(self, "_packed_cache", None)
-        if cached is None or cached[0] != key:
-            cached = (key, tuple(pack_weight(p) for p in srcs))
+        cached = self.__dict__.get("_packed_cache")
+        if cached is None or not cached[0].unchanged(srcs):
+            cached = (Sources(srcs), tuple(pack_weight(p) for p in srcs))
             self._packed_cache = cached
         return cached[1]
 

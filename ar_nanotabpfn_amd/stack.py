@@ -13,6 +13,7 @@ from torch import Tensor
 
 from . import _lib
 from . import attention_kernels as ak
+from .live import Sources
 
 __all__ = ["LayerStack"]
 
@@ -21,15 +22,18 @@ _attention_calls = (ak.prefill_attention, ak.teacher_forcing_attention, ak.hybri
 
 
 def _small_vectors(layer):
-    """Parameters that enter unpacked, in the order of ``artab_stack_layer``, and the weights that are packed."""
+    """Parameters that enter unpacked, in the order of ``artab_stack_layer``, the weights that are packed, and the
+    constants."""
     mods = layer._modules
     feat, rows, ff = mods["attn_features"]._modules, mods["attn_rows"]._modules, mods["ff"]._modules
     p1, p2 = ff["0"]._parameters, ff["2"]._parameters
-    n1, n2, n3 = (mods[n]._parameters for n in ("norm1", "norm2", "norm3"))
+    norms = mods["norm1"], mods["norm2"], mods["norm3"]
+    n1, n2, n3 = (n._parameters for n in norms)
     return ((p1["bias"], p2["bias"], n1["weight"], n1["bias"], n2["weight"], n2["bias"], n3["weight"], n3["bias"]),
             (feat["v_proj"]._parameters["weight"], feat["out_proj"]._parameters["weight"], rows["q_proj"]._parameters["weight"],
              rows["k_proj"]._parameters["weight"], rows["v_proj"]._parameters["weight"], rows["out_proj"]._parameters["weight"],
-             p1["weight"], p2["weight"]))
+             p1["weight"], p2["weight"]),
+            (*(n.eps for n in norms), mods["attn_rows"].n_heads))
 
 
 def _pack_f32(w: Tensor) -> Tensor:
@@ -50,39 +54,42 @@ def _covered(layer, x: Tensor) -> bool:
 
 class LayerStack:
     """What a pass reads of the layers, collected again whenever a parameter is another tensor or has been
-    written to; each call looks at all of them."""
+    written to, or a constant is another number; each call looks at all of them."""
 
     def __init__(self):
-        self._key = self._layers = self._keep = None
+        self._sources = self._key = self._layers = self._keep = None
 
     def _collect(self, layers, x: Tensor) -> bool:
         """Bring ``self._layers`` up to date; False where the layers are not of the form the call takes."""
         try:
             params = [_small_vectors(layer) for layer in layers]
-        except KeyError:
+        except (AttributeError, KeyError):
             return False
-        key = (x.dtype, x.device, *[(p.data_ptr(), p._version) if p is not None else None for two in params for ps in two for p in ps])
-        if key == self._key:
+        tensors = [p for vectors, weights, _ in params for ps in (vectors, weights) for p in ps]
+        if any(p is None for p in tensors):
+            return False
+        key = (x.dtype, x.device, *[constants for _, _, constants in params])
+        if key == self._key and self._sources.unchanged(tensors):
             return self._layers is not None
-        self._key, self._layers, self._keep = key, None, None
+        self._key, self._sources, self._layers, self._keep = key, Sources(tensors), None, None
         first = layers[0]
         D, F = x.shape[-1], first.ff[0].out_features
-        for layer, (vectors, weights) in zip(layers, params):
+        for layer, (vectors, weights, _) in zip(layers, params):
             sizes = ((F,), (D,)) + ((D,),) * 6 + ((D, D),) * 6 + ((F, D), (D, F))
             if not (type(layer) is type(first) and layer.attn_rows.n_heads == first.attn_rows.n_heads
-                    and all(p is not None and p.dtype == x.dtype and p.device == x.device and p.is_contiguous() and tuple(p.shape) == s
+                    and all(p.dtype == x.dtype and p.device == x.device and p.is_contiguous() and tuple(p.shape) == s
                             for p, s in zip(vectors + weights, sizes))
                     and all(p.data_ptr() % 16 == 0 for p in vectors)):
                 return False
         array, keep = (_lib.ArtabStackLayer * len(layers))(), []
-        for a, layer, (v, w) in zip(array, layers, params):
+        for a, layer, (v, w, constants) in zip(array, layers, params):
             if x.dtype == torch.float32:
                 packed = tuple(_pack_f32(p) for p in (*layer.fused_weights(), *w[5:]))
             else:
                 packed = layer.packed_weights()
             a.w_fo, a.w_qkv, a.w_o, a.w_1, a.w_2 = (t.data_ptr() for t in packed)
             a.b_1, a.b_2, a.gamma1, a.beta1, a.gamma2, a.beta2, a.gamma3, a.beta3 = (t.data_ptr() for t in v)
-            a.eps1, a.eps2, a.eps3 = layer.norm1.eps, layer.norm2.eps, layer.norm3.eps
+            a.eps1, a.eps2, a.eps3 = constants[:3]
             keep += [*packed, *v]
         self._layers, self._keep = array, keep
         return True
