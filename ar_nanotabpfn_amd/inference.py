@@ -21,19 +21,22 @@ from __future__ import annotations
 from typing import Optional
 
 import torch
-from torch import Tensor
+from torch import Tensor, nn
 
 from . import attention_kernels as ak
 from .attention import DecodeMask, TeacherForcingMask
 from . import _lib
-from .live import ModelState
-from .stack import LayerStack
+from .live import Methods, ModelState, plain_modules
+from .model import Embedder, MixtureGaussianHead
+from .stack import LAYER_METHODS, LayerStack
 from .glue import SampleEmbedStep, DecodeStepBoundary, TrajectoryDecoder, add_layer_norm
 
 __all__ = ["ARTabPFNPredictor"]
 
 
-_attention_module = ak
+_attention_module, _decode_attention = ak, ak.decode_attention
+_EMBEDDER_METHODS = Methods(Embedder, "_x", "_y", "_marker", "embed_buffer", "embed_target")
+_HEAD_METHODS = Methods(MixtureGaussianHead, "_parameterize", "sample")
 
 
 class _GraphState:
@@ -213,7 +216,8 @@ class ARTabPFNPredictor:
 
     def _stack_pass(self, x_row: Tensor, caches, num_targets: int = 0, context_len: int = 0) -> Optional[Tensor]:
         """The whole stack as one call, or None where the layers have to be run one by one."""
-        if ak is not _attention_module:  # calls of a program's own in the place of this package's
+        # calls of a program's own in the place of this package's are called
+        if ak is not _attention_module or not _STACK_METHODS.of(self):
             return None
         return self._stack(list(self.backbone.layers), x_row, caches, num_targets, context_len)
 
@@ -418,6 +422,18 @@ class ARTabPFNPredictor:
         is another one or has been written to."""
         return self._model_state.look((self.backbone, self.embedder, self.head), self.ar_tokens)
 
+    def _run_as_defined(self) -> bool:
+        """Whether the methods and modules that the step-by-step routes call are this package's own, so that the
+        whole-run launch computes the same."""
+        if not (ak is _attention_module and ak.decode_attention is _decode_attention and _RUN_METHODS.of(self)
+                and LAYER_METHODS.of(*self.backbone.layers) and _EMBEDDER_METHODS.of(self.embedder) and _HEAD_METHODS.of(self.head)):
+            return False
+        try:
+            modules = [self.embedder.x_embed, self.embedder.y_embed, self.head.head, *self.head.head._modules.values()]
+        except AttributeError:
+            return False
+        return plain_modules(modules, (nn.Linear, nn.Linear, nn.Sequential, nn.Linear, nn.GELU, nn.Linear))
+
     def _sample_whole_run(self, x_target: Tensor) -> Optional[Tensor]:
         """The sampling run as one launch (``TrajectoryDecoder``), or None where it does not apply.  The
         variates are drawn from torch's generator in the order in which the other routes draw them, so
@@ -435,7 +451,7 @@ class ARTabPFNPredictor:
             caches = [(l.k_cache, l.v_cache, l.k_cache, l.v_cache) for l in layers]
             n_ctx, own_base, fits = 0, self.seq_len, self.seq_len + Nt <= layers[0].k_cache.shape[2]
         if not (fits and n_ctx + own_base > 0 and caches[0][2].shape[0] == B
-                and all(t.dtype == x_target.dtype and t.is_contiguous() for c in caches for t in c)):
+                and all(t.dtype == x_target.dtype and t.is_contiguous() for c in caches for t in c) and self._run_as_defined()):
             return None
         key = (x_target.dtype, self._model_key())
         if self._trajectory is None or self._trajectory[0] != key:
@@ -828,3 +844,9 @@ class ARTabPFNPredictor:
             q, layer.k_ctx_cache[:, : self.context_len], layer.v_ctx_cache[:, : self.context_len],
             k[:, :, :num_targets], v[:, :, :num_targets], num_targets,
         )
+
+
+# what the one-launch forms stand for: a subclass that overrides one of these gets the routes that call it
+_RUN_METHODS = Methods(ARTabPFNPredictor, "autoregressive_decode", "transformer_decode", "_run_layers", "_attend_decode_shared",
+                       "_attend_with_cache", "_graph_step", "_first_step", "_sample_sequence_graph")
+_STACK_METHODS = Methods(ARTabPFNPredictor, "_run_layers", "_attend_with_cache", "_attend_teacher_forcing_shared")

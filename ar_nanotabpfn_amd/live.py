@@ -1,4 +1,5 @@
-"""The state of a model's modules as it is now, for calls that read parameters past ``nn.Module.__call__``.
+"""The state of a model's modules as it is now, for calls that read parameters past ``nn.Module.__call__`` and compute
+what the methods of the package's classes would.
 
 A program may exchange any parameter or module between two calls (``load_state_dict(assign=True)``, a new
 ``nn.Parameter``, another head).  What a call has prepared from the modules is used again only while
@@ -6,11 +7,36 @@ A program may exchange any parameter or module between two calls (``load_state_d
 
 from __future__ import annotations
 
-from operator import is_
+from operator import attrgetter, is_
 
 import torch
+from torch import nn
 
-__all__ = ["ModelState", "Sources"]
+__all__ = ["Methods", "ModelState", "Sources", "plain_modules"]
+
+_hooks_of = attrgetter("_forward_hooks", "_forward_pre_hooks", "_backward_hooks", "_backward_pre_hooks")
+_global_hooks = tuple(getattr(nn.modules.module, f"_global_{n}_hooks") for n in ("forward", "forward_pre", "backward", "backward_pre"))
+_forwards = tuple((c, c.forward) for c in (nn.Linear, nn.LayerNorm, nn.GELU, nn.Sequential, nn.Embedding))
+
+
+def plain_modules(modules, classes) -> bool:
+    """Whether calling these modules is nothing but the forward of these classes: no subclass, no hook, no function of
+    a program's own in the place of a method."""
+    return (list(map(type, modules)) == list(classes) and not any(map(any, map(_hooks_of, modules))) and not any(_global_hooks)
+            and not any("forward" in m.__dict__ for m in modules) and all(c.forward is f for c, f in _forwards)
+            and all(m.approximate == "none" for m in modules if type(m) is nn.GELU))
+
+
+class Methods:
+    """The methods of a class that a prepared call stands for, as they are at import: ``of(obj)`` while nothing
+    has taken the place of one of them, in a subclass, in the class or in the object."""
+
+    def __init__(self, cls, *names):
+        self._functions, self._names = [(n, getattr(cls, n)) for n in names], frozenset(names)
+
+    def of(self, *objects) -> bool:
+        return (all(getattr(t, n, None) is f for t in set(map(type, objects)) for n, f in self._functions)
+                and all(self._names.isdisjoint(o.__dict__) for o in objects))
 
 
 def _walk(roots):

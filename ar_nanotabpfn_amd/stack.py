@@ -13,11 +13,14 @@ from torch import Tensor
 
 from . import _lib
 from . import attention_kernels as ak
-from .live import Sources
+from .live import Methods, Sources
+from .model import TwoStageTransformerLayer
 
-__all__ = ["LayerStack"]
+__all__ = ["LAYER_METHODS", "LayerStack"]
 
 # A program that has put callables of its own in their place gets the layer-by-layer form, which calls them.
+LAYER_METHODS = Methods(TwoStageTransformerLayer, "fused_weights", "feature_stage", "qkv_heads", "packed_weights", "_fusable", "fused_for",
+                        "pre_attention", "finish", "finish_then_pre", "feed_forward")
 _attention_calls = (ak.prefill_attention, ak.teacher_forcing_attention, ak.hybrid_teacher_forcing_attention)
 
 
@@ -76,7 +79,7 @@ class LayerStack:
         D, F = x.shape[-1], first.ff[0].out_features
         for layer, (vectors, weights, _) in zip(layers, params):
             sizes = ((F,), (D,)) + ((D,),) * 6 + ((D, D),) * 6 + ((F, D), (D, F))
-            if not (type(layer) is type(first) and layer.attn_rows.n_heads == first.attn_rows.n_heads
+            if not (layer.attn_rows.n_heads == first.attn_rows.n_heads
                     and all(p.dtype == x.dtype and p.device == x.device and p.is_contiguous() and tuple(p.shape) == s
                             for p, s in zip(vectors + weights, sizes))
                     and all(p.data_ptr() % 16 == 0 for p in vectors)):
@@ -99,7 +102,8 @@ class LayerStack:
         ``num_targets`` 0: prefill; else teacher forcing against the first ``context_len`` cached rows.  None, with
         nothing done, where the call does not apply."""
         if not (x.is_cuda and layers and x.numel() and (ak.prefill_attention, ak.teacher_forcing_attention,
-                                                       ak.hybrid_teacher_forcing_attention) == _attention_calls):
+                                                       ak.hybrid_teacher_forcing_attention) == _attention_calls
+                and LAYER_METHODS.of(*layers)):
             return None
         first = layers[0]
         B, N, D = x.shape
