@@ -12,7 +12,7 @@ from operator import attrgetter, is_
 import torch
 from torch import nn
 
-__all__ = ["Methods", "ModelState", "Sources", "plain_modules"]
+__all__ = ["Methods", "ModelState", "Sources", "plain_modules", "walk"]
 
 _hooks_of = attrgetter("_forward_hooks", "_forward_pre_hooks", "_backward_hooks", "_backward_pre_hooks")
 _global_hooks = tuple(getattr(nn.modules.module, f"_global_{n}_hooks") for n in ("forward", "forward_pre", "backward", "backward_pre"))
@@ -39,7 +39,7 @@ class Methods:
                 and all(self._names.isdisjoint(o.__dict__) for o in objects))
 
 
-def _walk(roots):
+def walk(roots):
     """The modules of the trees below ``roots`` at the moment, and the entries of their parameter tables."""
     modules, parameters = list(roots), []
     for m in modules:  # (grows while it is walked)
@@ -87,7 +87,7 @@ class ModelState:
         self._modules = self._types = self._parameters = self._sources = self._constants = self._values = None
 
     def look(self, roots, *tensors) -> int:
-        modules, parameters = _walk(roots)
+        modules, parameters = walk(roots)
         parameters += tensors
         types = list(map(type, modules))
         if not (_same(self._modules, modules) and types == self._types and _same(self._parameters, parameters)

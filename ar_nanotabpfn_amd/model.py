@@ -26,7 +26,7 @@ from torch import Tensor, nn
 from .attention import DenseMask, MultiheadAttention, RowMask
 from .glue import add_layer_norm, bias_gelu, layer_fusable, layer_post, layer_post_pre, layer_pre, pack_weight
 
-from .live import Sources
+from .live import Methods, Sources, plain_modules, walk
 from .training import embed_rows, layer_stack, layer_stack_supported
 
 __all__ = ["Embedder", "TwoStageTransformerLayer", "TwoStageTransformer", "MixtureGaussianHead", "ARTabPFN"]
@@ -344,12 +344,14 @@ class ARTabPFN(nn.Module):
         training step (train.py:289-300).  Under ``torch.no_grad()`` the layers take the fused
         inference kernels instead."""
         Nc, Nb = x_context.size(1), x_buffer.size(1)
-        embeddings = embed_rows(self, x_context, y_context, x_buffer, y_buffer, x_target) if torch.is_grad_enabled() else None
+        embeddings = None
+        if torch.is_grad_enabled() and _embedder_as_defined(self.embedder):
+            embeddings = embed_rows(self, x_context, y_context, x_buffer, y_buffer, x_target)
         if embeddings is None:
             ctx_emb = self.embedder.embed_context(x_context, y_context)
             buf_emb = self.embedder.embed_buffer(x_buffer, y_buffer) + self.ar_tokens[:Nb]
             embeddings = torch.cat([ctx_emb, buf_emb, self.embedder.embed_target(x_target)], dim=1)
-        if layer_stack_supported(self.backbone, embeddings, mask_rows, Nc + Nb):
+        if torch.is_grad_enabled() and _backbone_as_defined(self.backbone) and layer_stack_supported(self.backbone, embeddings, mask_rows, Nc + Nb):
             z_target = layer_stack(self.backbone, embeddings, mask_rows, Nc + Nb)
             # q_proj and k_proj of the feature attention do not enter (one key per query); they get the exact
             # zero gradients autograd gives them in the reference
@@ -400,3 +402,27 @@ class ARTabPFN(nn.Module):
                     buffer_size=buffer_size, num_components=num_components)
         model.load_state_dict(sd, strict=True)
         return model, step
+
+
+# What the fused kernels of a training step (training.py) stand for: these methods of these classes in their places.
+# Subclasses, exchanged modules, hooks and functions of a program's own are run as modules.
+_EMBEDDER_METHODS = Methods(Embedder, "_x", "_y", "_marker", "embed_context", "embed_buffer", "embed_target")
+_BACKBONE_METHODS = Methods(TwoStageTransformer, "forward")
+_LAYER_METHODS = Methods(TwoStageTransformerLayer, "forward", "_forward_recording")
+_ATTENTION_METHODS = Methods(MultiheadAttention, "forward", "split_heads")
+
+
+def _embedder_as_defined(embedder) -> bool:
+    modules, _ = walk((embedder,))
+    return plain_modules(modules, (Embedder, nn.Linear, nn.Linear, nn.Embedding)) and _EMBEDDER_METHODS.of(embedder)
+
+
+def _backbone_as_defined(backbone) -> bool:
+    """Whether the modules below ``backbone``, level by level, are those of ``TwoStageTransformer.__init__``."""
+    modules, _ = walk((backbone,))
+    L = len(backbone.layers)
+    classes = (TwoStageTransformer, nn.ModuleList, nn.LayerNorm) + (TwoStageTransformerLayer,) * L
+    classes += (MultiheadAttention, MultiheadAttention, nn.Sequential, nn.LayerNorm, nn.LayerNorm, nn.LayerNorm) * L
+    classes += ((nn.Linear,) * 9 + (nn.GELU, nn.Linear)) * L  # the projections of both attentions, the feed-forward
+    return (plain_modules(modules, classes) and _BACKBONE_METHODS.of(backbone) and _LAYER_METHODS.of(*modules[3:3 + L])
+            and _ATTENTION_METHODS.of(*(m for m in modules[3 + L:3 + 7 * L] if type(m) is MultiheadAttention)))

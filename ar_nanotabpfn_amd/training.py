@@ -10,7 +10,7 @@ from __future__ import annotations
 import ctypes
 
 import torch
-from torch import Tensor
+from torch import Tensor, nn
 
 from . import _lib
 from . import attention_kernels as ak
@@ -24,10 +24,19 @@ _attention_calls = (ak.row_mask_attention, ak.row_mask_attention_backward)
 
 def _layer_params(layer):
     """The parameters of a layer in the order of ``artab_train_args.params``."""
-    af, ar = layer.attn_features, layer.attn_rows
-    return (af.v_proj.weight, af.out_proj.weight, ar.q_proj.weight, ar.k_proj.weight, ar.v_proj.weight, ar.out_proj.weight,
-            layer.ff[0].weight, layer.ff[0].bias, layer.ff[2].weight, layer.ff[2].bias, layer.norm1.weight, layer.norm1.bias,
-            layer.norm2.weight, layer.norm2.bias, layer.norm3.weight, layer.norm3.bias)
+    mods = layer._modules
+    af, ar, ff = mods["attn_features"]._modules, mods["attn_rows"]._modules, mods["ff"]._modules
+    one, two = ff["0"]._parameters, ff["2"]._parameters
+    n1, n2, n3 = mods["norm1"]._parameters, mods["norm2"]._parameters, mods["norm3"]._parameters
+    return (af["v_proj"]._parameters["weight"], af["out_proj"]._parameters["weight"], ar["q_proj"]._parameters["weight"],
+            ar["k_proj"]._parameters["weight"], ar["v_proj"]._parameters["weight"], ar["out_proj"]._parameters["weight"],
+            one["weight"], one["bias"], two["weight"], two["bias"], n1["weight"], n1["bias"], n2["weight"], n2["bias"],
+            n3["weight"], n3["bias"])
+
+
+def _shapes(D: int, F: int):
+    """Their sizes."""
+    return ((D, D),) * 6 + ((F, D), (F,), (D, F), (D,)) + ((D,),) * 6
 
 
 def _args(backbone, B: int, R: int, mask: RowMask, first_row: int) -> "_lib.ArtabTrainArgs":
@@ -48,22 +57,30 @@ def layer_stack_supported(backbone, x: Tensor, mask, first_row: int) -> bool:
             and (ak.row_mask_attention, ak.row_mask_attention_backward) == _attention_calls):
         return False
     layers = list(backbone.layers)
-    if not layers or x.shape[1] != mask.num_rows:
+    if not layers or x.shape[1] != mask.num_rows or x.shape[2] != backbone.d_model:
         return False
     first = layers[0]
+    D, F, norm = x.shape[2], first.ff[0].out_features, backbone.norm
+    shapes, heads = _shapes(D, F), first.attn_rows.n_heads
+    constants = [getattr(first, n).eps for n in ("norm1", "norm2", "norm3")]
 
     def same(layer):
-        return (layer.attn_rows.n_heads == first.attn_rows.n_heads and layer.ff[0].out_features == first.ff[0].out_features
-                and all(getattr(layer, n).eps == getattr(first, n).eps for n in ("norm1", "norm2", "norm3"))
-                and all(p is not None and p.dtype == torch.float32 and p.device == x.device and p.is_contiguous()
-                        and p.data_ptr() % 16 == 0 for p in _layer_params(layer)))
+        af, ar = layer._modules["attn_features"], layer._modules["attn_rows"]
+        projections = [*af._modules.values(), *ar._modules.values()]
+        unused = (af._modules["q_proj"]._parameters["weight"], af._modules["k_proj"]._parameters["weight"])
+        return (ar.n_heads == heads and ar.head_dim * heads == D and [layer._modules[n].eps for n in ("norm1", "norm2", "norm3")] == constants
+                and _f32(x.device, _layer_params(layer), shapes) and all(m._parameters["bias"] is None for m in projections)
+                and all(p.dtype == torch.float32 and p.device == x.device for p in unused))
 
-    return (all(same(layer) for layer in layers)
+    return (all(same(layer) for layer in layers) and _f32(x.device, (norm.weight, norm.bias), ((D,), (D,)))
+            and (x.requires_grad or any(p.requires_grad for p in backbone.parameters()))
             and _lib.load().artab_train_saved_bytes(ctypes.byref(_args(backbone, x.shape[0], x.shape[1], mask, first_row))) > 0)
 
 
-def _f32(*tensors) -> bool:
-    return all(t is not None and t.is_cuda and t.dtype == torch.float32 and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in tensors)
+def _f32(device, tensors, shapes) -> bool:
+    """Float32 tensors of these sizes, as the kernels read them (16-byte pieces, no strides)."""
+    return all(t is not None and type(t) in (Tensor, nn.Parameter) and t.dtype == torch.float32 and t.device == device and t.shape == s
+               and t.is_contiguous() and t.data_ptr() % 16 == 0 for t, s in zip(tensors, shapes))
 
 
 class _Embed(torch.autograd.Function):
@@ -105,11 +122,15 @@ def embed_rows(model, x_context, y_context, x_buffer, y_buffer, x_target):
     params = (e.x_embed.weight, e.x_embed.bias, e.y_embed.weight, e.y_embed.bias, e.marker_embed.weight, model.ar_tokens)
     data = [t.contiguous() for t in (x_context, y_context, x_buffer, y_buffer, x_target)]
     xs, ys = data[0::2], data[1::2]
-    if not (_f32(*data, *params) and not any(t.requires_grad for t in data) and model.d_model in (128, 256)
-            and torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") == torch.bfloat16
-            and all(t.dim() == 3 and t.shape[2] == xs[0].shape[2] and t.shape[0] == xs[0].shape[0] for t in xs)
-            and all(y.numel() == x.shape[0] * x.shape[1] for x, y in zip(xs, ys))
-            and xs[0].shape[1] >= 1 and xs[2].shape[1] >= 1 and xs[1].shape[1] <= model.ar_tokens.shape[0]):
+    D, (B, feat) = model.d_model, (xs[0].shape[0], xs[0].shape[-1])
+    if not (torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") == torch.bfloat16 and D in (128, 256)
+            and xs[0].is_cuda and all(t.dim() == 3 and t.shape[0] == B and t.shape[2] == feat for t in xs)
+            and all(tuple(y.shape) in ((B, x.shape[1]), (B, x.shape[1], 1)) for x, y in zip(xs, ys))
+            and not any(t.requires_grad for t in data) and any(p.requires_grad for p in params)
+            and xs[0].shape[1] >= 1 and xs[2].shape[1] >= 1 and xs[1].shape[1] <= model.ar_tokens.shape[0]
+            and _f32(xs[0].device, data, [t.shape for t in data])
+            and _f32(xs[0].device, params, ((D, 1), (D,), (D, 1), (D,), (3, D), (model.ar_tokens.shape[0], D)))
+            and B >= 1 and feat >= 1 and B * sum(x.shape[1] for x in xs) < 2 ** 30):
         return None
     return _Embed.apply(*data, *params)
 
