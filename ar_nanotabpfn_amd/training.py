@@ -83,6 +83,12 @@ def _f32(device, tensors, shapes) -> bool:
                and t.is_contiguous() and t.data_ptr() % 16 == 0 for t, s in zip(tensors, shapes))
 
 
+def _pieces(t: Tensor) -> Tensor:
+    """``t`` without strides, at an address that 16-byte loads can take."""
+    t = t.contiguous()
+    return t.clone() if t.data_ptr() % 16 else t
+
+
 class _Embed(torch.autograd.Function):
     @staticmethod
     def forward(ctx, xc, yc, xb, yb, xt, w_x, b_x, w_y, b_y, markers, tokens):
@@ -96,20 +102,23 @@ class _Embed(torch.autograd.Function):
                             "tokens", "out", "xy"), (xc, yc, xb, yb, xt, w_x, b_x, w_y, b_y, markers, tokens, out, xy)):
             setattr(a, name, t.data_ptr())
         _lib.check(_lib.load().artab_train_embed(ctypes.byref(a), _lib.current_stream(xc.device)))
-        ctx.args, ctx.xy, ctx.shapes = a, xy, (w_x.shape, w_y.shape, tokens.shape)
+        # (through save_for_backward: freed when the backward pass is done, seen by saved-tensor hooks)
+        ctx.save_for_backward(xy)
+        ctx.args, ctx.shapes = a, (w_x.shape, w_y.shape, tokens.shape)
         return out
 
     @staticmethod
     @torch.autograd.function.once_differentiable
     def backward(ctx, dx):
-        lib, a = _lib.load(), ctx.args
-        dx = dx.contiguous()
+        lib, a = _lib.load(), _lib.ArtabTrainEmbedArgs.from_buffer_copy(ctx.args)
+        (xy,) = ctx.saved_tensors
+        dx, xy = _pieces(dx), _pieces(xy)
         D, n = a.D, ctx.shapes[2][0]
         grads = torch.empty((7 + n) * D, device=dx.device, dtype=torch.float32)
         if n > a.n_buffer:  # tokens behind the buffer rows take no part
             grads[(7 + a.n_buffer) * D :].zero_()
         scratch = torch.empty(lib.artab_train_embed_scratch_bytes(ctypes.byref(a)), device=dx.device, dtype=torch.uint8)
-        a.out, a.grads, a.scratch = dx.data_ptr(), grads.data_ptr(), scratch.data_ptr()
+        a.out, a.xy, a.grads, a.scratch = dx.data_ptr(), xy.data_ptr(), grads.data_ptr(), scratch.data_ptr()
         _lib.check(lib.artab_train_embed_backward(ctypes.byref(a), _lib.current_stream(dx.device)))
         w_x, b_x, w_y, b_y, markers, tokens = grads.split((D, D, D, D, 3 * D, n * D))
         return (None,) * 5 + (w_x.view(ctx.shapes[0]), b_x, w_y.view(ctx.shapes[1]), b_y, markers.view(3, D), tokens.view(n, D))
@@ -135,33 +144,44 @@ def embed_rows(model, x_context, y_context, x_buffer, y_buffer, x_target):
     return _Embed.apply(*data, *params)
 
 
+def _set_pointers(a, x: Tensor, params, saved: Tensor):
+    """The tensors of a call into its arguments; returns what the arguments point at."""
+    n = 16 * a.n_layers
+    pointers = (ctypes.c_void_p * n)(*(p.data_ptr() for p in params[:n]))
+    a.x, a.params, a.saved = x.data_ptr(), ctypes.cast(pointers, ctypes.c_void_p), saved.data_ptr()
+    a.norm_gamma, a.norm_beta = params[n].data_ptr(), params[n + 1].data_ptr()
+    return pointers
+
+
 class _LayerStack(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, backbone, mask, first_row, *params):
         lib = _lib.load()
         B, R, D = x.shape
-        x = x.contiguous()
+        x = _pieces(x)
         a = _args(backbone, B, R, mask, first_row)
-        n = 16 * a.n_layers
-        pointers = (ctypes.c_void_p * n)(*(p.data_ptr() for p in params[:n]))
         saved = torch.empty(lib.artab_train_saved_bytes(ctypes.byref(a)), device=x.device, dtype=torch.uint8)
         z = torch.empty((B, R - first_row, D), device=x.device, dtype=torch.float32)
-        a.x, a.params = x.data_ptr(), ctypes.cast(pointers, ctypes.c_void_p)
-        a.norm_gamma, a.norm_beta = params[n].data_ptr(), params[n + 1].data_ptr()
-        a.saved, a.z = saved.data_ptr(), z.data_ptr()
+        ctx.args = _lib.ArtabTrainArgs.from_buffer_copy(a)  # (sizes and constants only)
+        pointers = _set_pointers(a, x, params, saved)  # noqa: F841  (alive until the call)
+        a.z = z.data_ptr()
         _lib.check(lib.artab_train_forward(ctypes.byref(a), _lib.current_stream(x.device)))
-        ctx.args, ctx.pointers, ctx.saved = a, pointers, saved
-        ctx.save_for_backward(x, *params)
+        ctx.save_for_backward(x, saved, *params)
         return z
 
     @staticmethod
     @torch.autograd.function.once_differentiable
     def backward(ctx, dz):
         lib = _lib.load()
-        x, *params = ctx.saved_tensors  # (raises if one of them was changed in place since)
-        a = ctx.args
+        x, saved, *params = ctx.saved_tensors  # (raises if one of them was changed in place since)
+        a = _lib.ArtabTrainArgs.from_buffer_copy(ctx.args)
         D, F, L = a.D, a.F, a.n_layers
-        dz = dz.contiguous().float()
+        # parameters whose data was exchanged since are read where they now are: they have to be of the same form
+        if not (_f32(x.device, (x,), ((a.B, a.R, D),)) and saved.data_ptr() % 16 == 0
+                and _f32(x.device, params, _shapes(D, F) * L + ((D,), (D,)))):
+            raise RuntimeError("a parameter of the layer stack has another size or type than in the forward pass")
+        dz = _pieces(dz.float())
+        pointers = _set_pointers(a, x, params, saved)  # noqa: F841  (alive until the call)
         scratch = torch.empty(lib.artab_train_scratch_bytes(ctypes.byref(a)), device=x.device, dtype=torch.uint8)
         dx = torch.empty_like(x)
         sizes = (D * D,) * 5 + (F * D, D * F) + (D,) * 5 + (F,) + (D,) * 2 + (D * D,) * 2
