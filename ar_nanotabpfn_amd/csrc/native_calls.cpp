@@ -4,12 +4,14 @@
 // attention_kernels.py spends about 16 us on describing eight tensors, allocating the results and converting
 // nineteen arguments.  These functions do the same from C++ in about 3.  Each returns None where anything
 // about its arguments is not the plain case (another device or type, shapes that do not match, a status other
-// than OK); the Python wrapper then takes its own path, which raises what has to be raised.
+// than OK); the Python wrapper then takes its own path, which raises what has to be raised.  C++ exceptions (no
+// memory for a result, a tensor without storage) become Python's in every entry.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
 #include <ATen/ATen.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <cstdint>
@@ -72,8 +74,15 @@ bool workspace(int device, size_t bytes, void **ptr, size_t *have) {
 
 PyObject *none() { Py_RETURN_NONE; }
 
+// A number that does not convert: left to the Python path
+PyObject *not_plain() {
+    PyErr_Clear();
+    return none();
+}
+
 // context_attention(q, k_ctx, v_ctx, scale, impl) -> (out, lse) or None
 PyObject *context_attention(PyObject *, PyObject *const *args, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
     if (n != 5 || !lib.context_attention) return none();
     for (int i = 0; i < 3; ++i)
         if (!THPVariable_Check(args[i])) return none();
@@ -88,9 +97,10 @@ PyObject *context_attention(PyObject *, PyObject *const *args, Py_ssize_t n) {
     double scale = 0.;
     if (args[3] != Py_None) {
         scale = PyFloat_AsDouble(args[3]);
-        if (PyErr_Occurred()) return nullptr;
+        if (PyErr_Occurred()) return not_plain();
     }
     const int impl = static_cast<int>(PyLong_AsLong(args[4]));
+    if (PyErr_Occurred()) return not_plain();
     at::AutoDispatchBelowAutograd guard;
     void *ws;
     size_t have;
@@ -101,13 +111,16 @@ PyObject *context_attention(PyObject *, PyObject *const *args, Py_ssize_t n) {
                               c.stream()) != ARTAB_OK)
         return none();
     PyObject *r = PyTuple_New(2);
+    if (!r) return nullptr;
     PyTuple_SET_ITEM(r, 0, THPVariable_Wrap(std::move(out)));
     PyTuple_SET_ITEM(r, 1, THPVariable_Wrap(std::move(lse)));
     return r;
+    END_HANDLE_TH_ERRORS
 }
 
 // decode_attention(q, k_ctx, v_ctx, k_buf, v_buf, n_buf, k_new, v_new, impl) -> out or None
 PyObject *decode_attention(PyObject *, PyObject *const *args, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
     if (n != 9 || !lib.decode_attention) return none();
     const int tensors[] = {0, 1, 2, 3, 4, 6, 7};
     if (!THPVariable_Check(args[0])) return none();
@@ -129,8 +142,9 @@ PyObject *decode_attention(PyObject *, PyObject *const *args, Py_ssize_t n) {
         kb.sizes() != vb.sizes() || kb.size(0) != B || kb.size(1) != H || kb.size(3) != Dh || has_new != (args[7] != Py_None) || !PyLong_Check(args[5]))
         return none();
     const long n_buf = PyLong_AsLong(args[5]);
-    if (n_buf < 0 || n_buf > cap) return none();
     const int impl = static_cast<int>(PyLong_AsLong(args[8]));
+    if (PyErr_Occurred()) return not_plain();
+    if (n_buf < 0 || n_buf > cap) return none();
     artab_view knv{}, vnv{};
     if (has_new) {
         const at::Tensor &kn = THPVariable_Unpack(args[6]), &vn = THPVariable_Unpack(args[7]);
@@ -148,6 +162,7 @@ PyObject *decode_attention(PyObject *, PyObject *const *args, Py_ssize_t n) {
                              static_cast<int>(n_buf), nullptr, cap, Dh, 0.f, c.dtype, ws, have, impl, c.stream()) != ARTAB_OK)
         return none();
     return THPVariable_Wrap(std::move(out));
+    END_HANDLE_TH_ERRORS
 }
 
 // bind(addresses: dict, workspace: callable)
