@@ -14,11 +14,13 @@ from __future__ import annotations
 import ctypes
 import importlib
 import os
+import warnings
 from typing import Optional
 
 import torch
 
-native = None  # the module _native.so, once the library is loaded
+native = None  # the module _native.so, once the library is loaded; None where it cannot be
+_native_missing = False
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libartab_attention.so")
 BENCH_LIB_PATH = os.path.join(_HERE, "libartab_bench.so")
@@ -268,16 +270,24 @@ def load() -> ctypes.CDLL:
 
 
 def _bind_native(lib: ctypes.CDLL) -> None:
-    """The native call module works through the library that is in use."""
-    global native
-    if native is None:
+    """The native call module works through the library that is in use.  It speaks the C++ interface of the torch it
+    was built with; under another one (or without it) the calls take their Python form, which needs the C
+    ABI only."""
+    global native, _native_missing
+    if native is None and not _native_missing:
         try:
-            native = importlib.import_module("._native", __package__)
+            module = importlib.import_module("._native", __package__)
+            built_with = getattr(module, "torch_version", "of another version")
+            if built_with != torch.__version__.split("+")[0]:
+                raise ImportError(f"built with torch {built_with}")
+            native = module
         except ImportError as err:
-            raise RuntimeError(f"ar_nanotabpfn_amd/_native.so cannot be loaded ({err}); "
-                               "build it with `python -m ar_nanotabpfn_amd.build_ext`") from err
-    native.bind({name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in SIGNATURES},
-                lambda index, nbytes: workspace(torch.device("cuda", index), nbytes))
+            _native_missing = True
+            warnings.warn(f"ar_nanotabpfn_amd/_native.so is not used ({err}): small attention calls take about 10 us more of "
+                          "host time; build it with `python -m ar_nanotabpfn_amd.build_ext`", RuntimeWarning, stacklevel=3)
+    if native is not None:
+        native.bind({name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in SIGNATURES},
+                    lambda index, nbytes: workspace(torch.device("cuda", index), nbytes))
 
 
 class benchmark_library:

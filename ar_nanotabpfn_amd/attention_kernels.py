@@ -65,7 +65,7 @@ def _call(name: str, *args):
     """The native form of a call, or None where it leaves the call to the path below it."""
     if _lib._lib is None:
         _lib.load()
-    return getattr(_lib.native, name)(*args)
+    return getattr(_lib.native, name)(*args) if _lib.native is not None else None
 
 
 def _alloc_out(q: Tensor) -> Tensor:

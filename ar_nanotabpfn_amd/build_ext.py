@@ -92,7 +92,8 @@ def native_command():
            sysconfig.get_paths()["include"]]
     libdir = os.path.join(base, "lib")
     return ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM",
-            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-w", *[f"-I{i}" for i in inc],
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-Wall", "-Wextra",
+            *[f"-isystem{i}" for i in inc],
             os.path.join(CSRC, "native_calls.cpp"), "-o", OUT_NATIVE + ".tmp", f"-L{libdir}", f"-Wl,-rpath,{libdir}",
             "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip"]
 
