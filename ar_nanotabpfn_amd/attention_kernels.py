@@ -82,13 +82,19 @@ def _ctx_views(k_ctx: Tensor, v_ctx: Tensor):
 
 
 def _workspace_for(q: Tensor, Nc: int):
+    """Scratch memory of a context or decode call: the tensor, its address and bytes.  The 16-bit types use the
+    device's scratch tensor (``workspace_tag``), where partial results may stay for the call behind; float32
+    calls leave nothing there and have memory of their own, so that calls on several streams do not share it."""
     B, H, Lq, Dh = q.shape
     lib = _lib.load()
     nbytes = lib.artab_workspace_bytes(B, H, Lq, Nc, Dh, _lib.dtype_code(q.dtype))
-    ws = _lib.workspace(q.device, nbytes)
+    if q.dtype == torch.float32:
+        ws = torch.empty(nbytes, device=q.device, dtype=torch.uint8) if nbytes else None
+    else:
+        ws = _lib.workspace(q.device, nbytes)
     if ws is None:
-        return None, 0
-    return ctypes.c_void_p(ws.data_ptr()), ws.numel() * 4
+        return None, None, 0
+    return ws, ctypes.c_void_p(ws.data_ptr()), ws.numel() * ws.element_size()
 
 
 def context_attention(
@@ -113,7 +119,7 @@ def context_attention(
         raise ValueError("q, k_ctx and v_ctx must share one dtype")
     out = _alloc_out(q)
     lse = torch.empty((B, H, Lq), device=dev, dtype=torch.float32)
-    ws_ptr, ws_bytes = _workspace_for(q, Nc)
+    ws, ws_ptr, ws_bytes = _workspace_for(q, Nc)  # (ws: alive until the launch)
     qv, ov = _lib.view4(q), _lib.view4(out)
     _lib.check(
         lib.artab_context_attention(
@@ -280,7 +286,7 @@ def decode_attention(
     if n_buf_device is not None and (n_buf_device.dtype != torch.int32 or not n_buf_device.is_cuda):
         raise ValueError("n_buf_device must be an int32 tensor on the device")
     out = _alloc_out(q)
-    ws_ptr, ws_bytes = _workspace_for(q, Nc)
+    ws, ws_ptr, ws_bytes = _workspace_for(q, Nc)  # (ws: alive until the launch)
     qv, ov = _lib.view4(q), _lib.view4(out)
     kbv, vbv = _lib.view4(k_buf_cache), _lib.view4(v_buf_cache)
     knv, vnv = _lib.view4(k_new), _lib.view4(v_new)

@@ -57,12 +57,19 @@ at::Tensor heads_out(const at::Tensor &q) {
     return at::empty_strided({B, H, L, D}, {L * H * D, D, H * D, 1}, q.options().requires_grad(false));
 }
 
-// The device's scratch tensor for `bytes` (null for none); false: the Python side failed
-bool workspace(int device, size_t bytes, void **ptr, size_t *have) {
+// Scratch memory for `bytes` (null for none): the device's scratch tensor, or for float32 calls memory of the
+// call's own, which `own` keeps until the launch; false: the Python side failed
+bool workspace(const Call &c, const at::Tensor &q, size_t bytes, at::Tensor &own, void **ptr, size_t *have) {
     *ptr = nullptr;
     *have = 0;
     if (bytes == 0) return true;
-    PyObject *t = PyObject_CallFunction(workspace_of, "in", device, static_cast<Py_ssize_t>(bytes));
+    if (c.type == at::kFloat) {
+        own = at::empty({static_cast<int64_t>(bytes)}, q.options().dtype(at::kByte).requires_grad(false));
+        *ptr = own.data_ptr();
+        *have = bytes;
+        return true;
+    }
+    PyObject *t = PyObject_CallFunction(workspace_of, "in", c.device, static_cast<Py_ssize_t>(bytes));
     if (!t) return false;
     if (THPVariable_Check(t)) {
         const at::Tensor &w = THPVariable_Unpack(t);
@@ -103,9 +110,10 @@ PyObject *context_attention(PyObject *, PyObject *const *args, Py_ssize_t n) {
     const int impl = static_cast<int>(PyLong_AsLong(args[4]));
     if (PyErr_Occurred()) return not_plain();
     at::AutoDispatchBelowAutograd guard;
+    at::Tensor own;
     void *ws;
     size_t have;
-    if (!workspace(c.device, lib.workspace_bytes(B, H, Lq, Nc, Dh, c.dtype), &ws, &have)) return nullptr;
+    if (!workspace(c, q, lib.workspace_bytes(B, H, Lq, Nc, Dh, c.dtype), own, &ws, &have)) return nullptr;
     at::Tensor out = heads_out(q), lse = at::empty({B, H, Lq}, q.options().dtype(at::kFloat).requires_grad(false));
     const artab_view qv = view(q), kv = view(k), vv = view(v), ov = view(out);
     if (lib.context_attention(&qv, &kv, &vv, &ov, lse.data_ptr<float>(), B, H, Lq, Nc, Dh, static_cast<float>(scale), c.dtype, ws, have, impl,
@@ -154,9 +162,10 @@ PyObject *decode_attention(PyObject *, PyObject *const *args, Py_ssize_t n) {
         vnv = view(vn);
     }
     at::AutoDispatchBelowAutograd guard;
+    at::Tensor own;
     void *ws;
     size_t have;
-    if (!workspace(c.device, lib.workspace_bytes(B, H, Lq, Nc, Dh, c.dtype), &ws, &have)) return nullptr;
+    if (!workspace(c, q, lib.workspace_bytes(B, H, Lq, Nc, Dh, c.dtype), own, &ws, &have)) return nullptr;
     at::Tensor out = heads_out(q);
     const artab_view qv = view(q), kv = view(kc), vv = view(vc), kbv = view(kb), vbv = view(vb), ov = view(out);
     if (lib.decode_attention(&qv, &kv, &vv, &kbv, &vbv, has_new ? &knv : nullptr, has_new ? &vnv : nullptr, &ov, B, H, Lq, Nc,
