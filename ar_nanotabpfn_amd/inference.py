@@ -108,6 +108,17 @@ class ARTabPFNPredictor:
         self._model_state = ModelState()  # (what a recorded step points at is held by it)
         self.graph_recordings = 0    # HIP graphs recorded so far (a run that only replays leaves it unchanged)
 
+    # Copies and pickles take the modules, the caches' state and the switches; what calls have prepared (recorded
+    # graphs, packed weights, streams) is made again by the copy's first call.
+    _PREPARED = ("_stack", "_trajectory", "_model_state", "_graph_state", "_side_streams")
+
+    def __getstate__(self):
+        return {k: v for k, v in self.__dict__.items() if k not in self._PREPARED}
+
+    def __setstate__(self, state):
+        ARTabPFNPredictor.__init__(self, state["embedder"], state["backbone"], state["head"], state["ar_tokens"], state["backend"])
+        self.__dict__.update((k, v) for k, v in state.items() if k not in self._PREPARED)
+
     @classmethod
     def from_trained_model(cls, model, backend: str = "flex_attention") -> "ARTabPFNPredictor":
         return cls(model.embedder, model.backbone, model.head, model.ar_tokens, backend=backend)

@@ -93,6 +93,10 @@ class TwoStageTransformerLayer(nn.Module):
         self.norm2 = nn.LayerNorm(d_model)
         self.norm3 = nn.LayerNorm(d_model)
 
+    def __getstate__(self):
+        """Copies and pickles leave out what is prepared from the weights."""
+        return {k: v for k, v in self.__dict__.items() if k not in ("_fused", "_packed")}
+
     def fused_weights(self):
         """Weights of the fused inference GEMMs, rebuilt when a source weight changes.
 
@@ -104,13 +108,13 @@ class TwoStageTransformerLayer(nn.Module):
         """
         af, ar = self.attn_features, self.attn_rows
         srcs = (af.v_proj.weight, af.out_proj.weight, ar.q_proj.weight, ar.k_proj.weight, ar.v_proj.weight)
-        cached = self.__dict__.get("_fused_cache")
+        cached = self.__dict__.get("_fused")
         if cached is None or not cached[0].unchanged(srcs):
             with torch.no_grad():
                 w_fo = (af.out_proj.weight.float() @ af.v_proj.weight.float()).to(af.v_proj.weight.dtype)
                 w_qkv = torch.cat([ar.q_proj.weight, ar.k_proj.weight, ar.v_proj.weight], dim=0).contiguous()
             cached = (Sources(srcs), w_fo, w_qkv)
-            self._fused_cache = cached
+            self._fused = cached
         return cached[1], cached[2]
 
     def feature_stage(self, x_row: Tensor) -> Tensor:
@@ -138,10 +142,10 @@ class TwoStageTransformerLayer(nn.Module):
         ``(w_fo, w_qkv, out_proj, ff[0], ff[2])``."""
         w_fo, w_qkv = self.fused_weights()
         srcs = (w_fo, w_qkv, self.attn_rows.out_proj.weight, self.ff[0].weight, self.ff[2].weight)
-        cached = self.__dict__.get("_packed_cache")
+        cached = self.__dict__.get("_packed")
         if cached is None or not cached[0].unchanged(srcs):
             cached = (Sources(srcs), tuple(pack_weight(p) for p in srcs))
-            self._packed_cache = cached
+            self._packed = cached
         return cached[1]
 
     def _fusable(self, x_row: Tensor) -> bool:
