@@ -18,6 +18,7 @@ import torch.nn.functional as F
 from torch import Tensor, nn
 
 from . import _lib
+from .live import Prepared
 
 __all__ = ["add_layer_norm", "bias_gelu", "layer_fusable", "pack_weight", "layer_pre", "layer_post", "layer_post_pre", "SampleEmbedStep", "DecodeStepBoundary",
            "TrajectoryDecoder"]
@@ -405,8 +406,7 @@ class TrajectoryDecoder:
         b_h2 = torch.zeros(64, device=dev, dtype=dt)
         b_h2[: lin2.out_features] = lin2.bias.detach()
         vec = lambda p: p.detach().reshape(-1).contiguous()  # noqa: E731
-        # everything the launch points at is kept alive here
-        self._keep = k = dict(
+        k = dict(
             tape=tape, vecs=vecs, b_h1=vec(lin1.bias), b_h2=b_h2,
             mix=torch.cat([vec(head.mean_bias), vec(head.std_bias), vec(head.weight_bias)]).to(dt),
             w_x=vec(embedder.x_embed.weight), b_x=vec(embedder.x_embed.bias),
@@ -414,6 +414,8 @@ class TrajectoryDecoder:
             markers=embedder.marker_embed.weight.detach().contiguous(), ar_tokens=ar_tokens.detach().contiguous(),
             norm_g=vec(backbone.norm.weight), norm_b=vec(backbone.norm.bias),
         )
+        # everything the launch points at is kept alive here
+        self._prepared = Prepared(k.values())
         a = self.args = _lib.ArtabTrajectoryArgs()
         a.tape, a.vecs, a.n_layers = tape.data_ptr(), vecs.data_ptr(), L
         a.eps1, a.eps2, a.eps3 = layers[0].norm1.eps, layers[0].norm2.eps, layers[0].norm3.eps
@@ -423,7 +425,11 @@ class TrajectoryDecoder:
         a.w_x, a.b_x, a.w_y, a.b_y = (k[n].data_ptr() for n in ("w_x", "b_x", "w_y", "b_y"))
         a.markers, a.ar_tokens, a.bs = k["markers"].data_ptr(), k["ar_tokens"].data_ptr(), ar_tokens.shape[0]
         a.D, a.F = D, F_
-        self._kv_key = None
+        self._kv_key = self._kv = None
+
+    def tables_made(self, caches) -> bool:
+        """Whether a call on these caches launches only (and can be recorded)."""
+        return tuple(t.data_ptr() for layer in caches for t in layer) == self._kv_key
 
     def group(self, B: int, Nc: int, Nt: int, own_context: bool) -> int:
         """Trajectories per workgroup, or 0 where the step-by-step launches are the faster route."""
@@ -436,12 +442,14 @@ class TrajectoryDecoder:
         the drawn values ``[B,Nt]``."""
         key = tuple(t.data_ptr() for layer in caches for t in layer)
         if key != self._kv_key:
-            self._kv = torch.tensor(key, dtype=torch.int64, device=self.device)
+            self._kv = Prepared([torch.tensor(key, dtype=torch.int64, device=self.device)])
             self._kv_key = key
+        self._prepared.use()
+        (kv,) = self._kv.use()
         B, Nt = x_mean.shape
         preds = torch.empty((B, Nt), device=self.device, dtype=x_mean.dtype)
         a = self.args
-        a.kv, a.n_ctx, a.ctx_rows, a.own_base = self._kv.data_ptr(), n_ctx, caches[0][0].shape[-2], own_base
+        a.kv, a.n_ctx, a.ctx_rows, a.own_base = kv.data_ptr(), n_ctx, caches[0][0].shape[-2], own_base
         a.own_rows, a.park_target = caches[0][2].shape[2], int(n_ctx == 0)
         a.rand_u, a.rand_n, a.rand_n_f32 = rand_u.data_ptr(), rand_n.data_ptr(), int(rand_n.dtype == torch.float32)
         a.x_mean, a.preds, a.B, a.Nt, a.group = x_mean.data_ptr(), preds.data_ptr(), B, Nt, group

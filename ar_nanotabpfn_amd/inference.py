@@ -26,7 +26,7 @@ from torch import Tensor, nn
 from . import attention_kernels as ak
 from .attention import DecodeMask, TeacherForcingMask
 from . import _lib
-from .live import Methods, ModelState, plain_modules
+from .live import Methods, ModelState, capturing, plain_modules
 from .model import Embedder, MixtureGaussianHead
 from .stack import LAYER_METHODS, LayerStack
 from .glue import SampleEmbedStep, DecodeStepBoundary, TrajectoryDecoder, add_layer_norm
@@ -466,9 +466,13 @@ class ARTabPFNPredictor:
             return None
         key = (x_target.dtype, self._model_key())
         if self._trajectory is None or self._trajectory[0] != key:
+            if capturing(x_target.device):  # (what a recording packs exists when it is replayed)
+                return None
             ok = TrajectoryDecoder.supported(self.embedder, self.backbone, self.head, x_target)
             self._trajectory = (key, TrajectoryDecoder(self.embedder, self.backbone, self.head, self.ar_tokens) if ok else None)
         run = self._trajectory[1]
+        if run is not None and capturing(x_target.device) and not run.tables_made(caches):
+            return None
         group = run.group(B, n_ctx + own_base, Nt, not shared) if run is not None else 0
         if group == 0:
             return None

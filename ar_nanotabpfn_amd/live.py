@@ -12,7 +12,7 @@ from operator import attrgetter, is_
 import torch
 from torch import nn
 
-__all__ = ["Methods", "ModelState", "Sources", "plain_modules", "walk"]
+__all__ = ["Methods", "ModelState", "Prepared", "Sources", "plain_modules", "walk"]
 
 _hooks_of = attrgetter("_forward_hooks", "_forward_pre_hooks", "_backward_hooks", "_backward_pre_hooks")
 _global_hooks = tuple(getattr(nn.modules.module, f"_global_{n}_hooks") for n in ("forward", "forward_pre", "backward", "backward_pre"))
@@ -71,6 +71,38 @@ class Sources:
 
     def unchanged(self, tensors) -> bool:
         return _same(self._tensors, tensors) and _values_at(tensors) == self._facts
+
+
+def capturing(device) -> bool:
+    return device.type == "cuda" and torch.cuda.is_current_stream_capturing()
+
+
+class Prepared:
+    """Tensors that are made once, on the current stream, and read by calls on any: ``use()`` in front of every call
+    on the current stream orders it behind the making, and keeps the memory from being given away under it
+    when the tensors are dropped."""
+
+    def __init__(self, tensors):
+        self.tensors = tuple(tensors)
+        self._device = next((t.device for t in self.tensors if t.is_cuda), None)
+        if self._device is not None and not capturing(self._device):
+            stream = torch.cuda.current_stream(self._device)
+            self._made, self._home, self._others = torch.cuda.Event(), stream.cuda_stream, set()
+            self._made.record(stream)
+
+    def use(self) -> tuple:
+        # (a recording cannot wait for what lies outside of it; it begins with everything in front of it done)
+        if self._device is None or capturing(self._device):
+            return self.tensors
+        stream = torch.cuda.current_stream(self._device)
+        if stream.cuda_stream != self._home:
+            stream.wait_event(self._made)
+            if stream.cuda_stream not in self._others:
+                for t in self.tensors:
+                    if t.is_cuda:
+                        t.record_stream(stream)
+                self._others.add(stream.cuda_stream)
+        return self.tensors
 
 
 class ModelState:

@@ -26,7 +26,7 @@ from torch import Tensor, nn
 from .attention import DenseMask, MultiheadAttention, RowMask
 from .glue import add_layer_norm, bias_gelu, layer_fusable, layer_post, layer_post_pre, layer_pre, pack_weight
 
-from .live import Methods, Sources, plain_modules, walk
+from .live import Methods, Prepared, Sources, capturing, plain_modules, walk
 from .training import embed_rows, layer_stack, layer_stack_supported
 
 __all__ = ["Embedder", "TwoStageTransformerLayer", "TwoStageTransformer", "MixtureGaussianHead", "ARTabPFN"]
@@ -113,9 +113,10 @@ class TwoStageTransformerLayer(nn.Module):
             with torch.no_grad():
                 w_fo = (af.out_proj.weight.float() @ af.v_proj.weight.float()).to(af.v_proj.weight.dtype)
                 w_qkv = torch.cat([ar.q_proj.weight, ar.k_proj.weight, ar.v_proj.weight], dim=0).contiguous()
-            cached = (Sources(srcs), w_fo, w_qkv)
-            self._fused = cached
-        return cached[1], cached[2]
+            cached = (Sources(srcs), Prepared((w_fo, w_qkv)))
+            if not capturing(w_fo.device):  # (what a recording makes exists when it is replayed)
+                self._fused = cached
+        return cached[1].use()
 
     def feature_stage(self, x_row: Tensor) -> Tensor:
         """Feature attention for the single-column case (C = 1) followed by norm1.
@@ -144,9 +145,10 @@ class TwoStageTransformerLayer(nn.Module):
         srcs = (w_fo, w_qkv, self.attn_rows.out_proj.weight, self.ff[0].weight, self.ff[2].weight)
         cached = self.__dict__.get("_packed")
         if cached is None or not cached[0].unchanged(srcs):
-            cached = (Sources(srcs), tuple(pack_weight(p) for p in srcs))
-            self._packed = cached
-        return cached[1]
+            cached = (Sources(srcs), Prepared(pack_weight(p) for p in srcs))
+            if not capturing(w_fo.device):
+                self._packed = cached
+        return cached[1].use()
 
     def _fusable(self, x_row: Tensor) -> bool:
         return layer_fusable(x_row, x_row.shape[-1], self.ff[0].out_features)

@@ -13,7 +13,7 @@ from torch import Tensor
 
 from . import _lib
 from . import attention_kernels as ak
-from .live import Methods, Sources
+from .live import Methods, Prepared, Sources, capturing
 from .model import TwoStageTransformerLayer
 
 __all__ = ["LAYER_METHODS", "LayerStack"]
@@ -60,7 +60,7 @@ class LayerStack:
     written to, or a constant is another number; each call looks at all of them."""
 
     def __init__(self):
-        self._sources = self._key = self._layers = self._keep = None
+        self._sources = self._key = self._layers = self._prepared = None
 
     def _collect(self, layers, x: Tensor) -> bool:
         """Bring ``self._layers`` up to date; False where the layers are not of the form the call takes."""
@@ -74,7 +74,9 @@ class LayerStack:
         key = (x.dtype, x.device, *[constants for _, _, constants in params])
         if key == self._key and self._sources.unchanged(tensors):
             return self._layers is not None
-        self._key, self._sources, self._layers, self._keep = key, Sources(tensors), None, None
+        if capturing(x.device):  # (what a recording packs exists when it is replayed)
+            return False
+        self._key, self._sources, self._layers, self._prepared = key, Sources(tensors), None, None
         first = layers[0]
         D, F = x.shape[-1], first.ff[0].out_features
         for layer, (vectors, weights, _) in zip(layers, params):
@@ -94,7 +96,7 @@ class LayerStack:
             a.b_1, a.b_2, a.gamma1, a.beta1, a.gamma2, a.beta2, a.gamma3, a.beta3 = (t.data_ptr() for t in v)
             a.eps1, a.eps2, a.eps3 = constants[:3]
             keep += [*packed, *v]
-        self._layers, self._keep = array, keep
+        self._layers, self._prepared = array, Prepared(keep)
         return True
 
     def __call__(self, layers, x: Tensor, caches, num_targets: int = 0, context_len: int = 0) -> Optional[Tensor]:
@@ -120,6 +122,7 @@ class LayerStack:
         x = x.contiguous()
         if x.data_ptr() % 16:
             x = x.clone()
+        self._prepared.use()
         lib, code = _lib.load(), _lib.dtype_code(x.dtype)
         for a, (k, v) in zip(self._layers, caches):
             a.k_cache, a.v_cache = k.data_ptr(), v.data_ptr()

@@ -1,0 +1,122 @@
+"""Weights that are prepared once are read on other streams behind their making, are not given away under a launch
+that reads them, and are not taken from a recording that has not been replayed."""
+
+import pytest
+import torch
+
+from ar_nanotabpfn_amd.glue import TrajectoryDecoder
+from ar_nanotabpfn_amd.model import ARTabPFN
+from ar_nanotabpfn_amd.stack import LayerStack
+
+pytestmark = pytest.mark.gpu
+
+CYCLES = 400_000_000  # some tenths of a second: the host is through with everything long before
+DTYPES = pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "f32"])
+
+
+def _model(device, dtype):
+    torch.manual_seed(1)
+    return ARTabPFN(d_model=128, n_heads=4, n_layers=2, d_ff=256, num_features=2, buffer_size=6, num_components=4).eval().to(device, dtype)
+
+
+def _caches(device, dtype, *shape):
+    return [tuple(torch.zeros(*shape, device=device, dtype=dtype) for _ in range(2)) for _ in range(2)]
+
+
+def _run_args(device, dtype):
+    B, Nc, Nt, g = 6, 20, 7, torch.Generator().manual_seed(3)
+    caches = [tuple(0.3 * torch.randn(*s, generator=g) for s in ((4, Nc, 32), (4, Nc, 32), (B, 4, Nt, 32), (B, 4, Nt, 32)))
+              for _ in range(2)]
+    return ([tuple(t.to(device, dtype) for t in c) for c in caches], Nc, 0, torch.randn(B, Nt, generator=g).to(device, dtype),
+            torch.rand(Nt, B, generator=g).to(device), torch.randn(Nt, B, generator=g).to(device, dtype), 1)
+
+
+def _decoder(m):
+    return TrajectoryDecoder(m.embedder, m.backbone, m.head, m.ar_tokens)
+
+
+@DTYPES
+@torch.no_grad()
+def test_another_stream_waits_for_the_packing(device, dtype):
+    x = torch.randn(1, 40, 128, device=device).to(dtype)
+    want = LayerStack()(list(_model(device, dtype).backbone.layers), x, _caches(device, dtype, 4, 40, 32))
+    run = _run_args(device, dtype)
+    want_run = _decoder(_model(device, dtype))(*run)
+    m, stack = _model(device, dtype), LayerStack()
+    layers, mine, other = list(m.backbone.layers), _caches(device, dtype, 4, 40, 32), _caches(device, dtype, 4, 40, 32)
+    torch.cuda.synchronize()
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    with torch.cuda.stream(a):
+        torch.cuda._sleep(CYCLES)
+        stack(layers, x, mine)
+        decoder = _decoder(m)
+    with torch.cuda.stream(b):
+        got = stack(layers, x, other)
+        got_run = decoder(*run)
+        got_layer = layers[0].packed_weights()[0].clone() if dtype != torch.float32 else layers[0].fused_weights()[0].clone()
+    torch.cuda.synchronize()
+    assert torch.equal(got, want) and torch.equal(got_run, want_run)
+    fresh = _model(device, dtype).backbone.layers[0]
+    assert torch.equal(got_layer, (fresh.packed_weights() if dtype != torch.float32 else fresh.fused_weights())[0])
+
+
+@DTYPES
+@torch.no_grad()
+def test_dropped_weights_stay_while_another_stream_reads_them(device, dtype):
+    run = _run_args(device, dtype)
+    m = _model(device, dtype)
+    want = _decoder(m)(*run)
+    decoder = _decoder(m)
+    decoder(*run)
+    sizes = [t.nbytes for t in decoder._prepared.tensors] if hasattr(decoder, "_prepared") else [t.nbytes for t in decoder._keep.values()]
+    torch.cuda.synchronize()
+    b = torch.cuda.Stream()
+    with torch.cuda.stream(b):
+        torch.cuda._sleep(CYCLES)
+        got = decoder(*run)
+    del decoder
+    others = [torch.full((n,), 255, device=device, dtype=torch.uint8) for n in sizes for _ in range(3)]
+    torch.cuda.synchronize()
+    assert torch.equal(got, want) and others
+
+
+@DTYPES
+@torch.no_grad()
+def test_a_recording_prepares_nothing_for_eager_calls(device, dtype):
+    from ar_nanotabpfn_amd.inference import ARTabPFNPredictor
+
+    Nc = 40
+    g = torch.Generator().manual_seed(4)
+    xc, yc = torch.randn(1, Nc, 2, generator=g).to(device, dtype), torch.randn(1, Nc, generator=g).to(device, dtype)
+
+    def prefill(p):
+        p.prefill_context(xc, yc)
+        return [t for l in p.backbone.layers for t in (l.k_ctx_cache, l.v_ctx_cache)]
+
+    def predictor():
+        p = ARTabPFNPredictor.from_trained_model(_model(device, dtype), backend="triton_shared_context")
+        p.init_kv_cache(1, 4, device, dtype)
+        for l in p.backbone.layers:
+            l.k_ctx_cache, l.v_ctx_cache = (torch.zeros(4, Nc, 32, device=device, dtype=dtype) for _ in range(2))
+        return p
+
+    want = [t.clone() for t in prefill(predictor())]  # (library workspaces are made here)
+    p = predictor()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        recorded = prefill(p)
+
+    def check(caches):
+        for a, b in zip(caches, want):  # (a recording takes the layers one by one: other roundings)
+            a, b = a.float(), b.float()
+            assert float((a - b).norm() / b.norm()) <= (1e-5 if dtype == torch.float32 else 1e-2)
+        for t in caches:
+            t.zero_()
+
+    check(prefill(p))  # before any replay
+    for _ in range(3):
+        graph.replay()
+        check(recorded)
+        check(prefill(p))
