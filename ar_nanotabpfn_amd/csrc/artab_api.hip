@@ -1686,6 +1686,22 @@ int check_stack(const artab_stack_args *a) {
         return fail(ARTAB_ERR_BAD_SHAPE, "layer stack: caches of %d rows, %ld needed", a->cache_rows, need);
     return ARTAB_OK;
 }
+// Every pointer of every layer, before anything is launched.  b_2 may be NULL, and b_1 in 16 bits.
+int check_stack_pointers(const artab_stack_args *a, bool f32) {
+    if (misaligned16(a->x) || misaligned16(a->out)) return fail(ARTAB_ERR_BAD_STRIDE, "layer stack: x and out must be 16-byte aligned");
+    for (int l = 0; l < a->n_layers; ++l) {
+        const artab_stack_layer &L = a->layers[l];
+        const void *required[] = {L.w_fo, L.w_qkv, L.w_o, L.w_1, L.w_2, L.gamma1, L.beta1, L.gamma2, L.beta2, L.gamma3, L.beta3,
+                                  L.k_cache, L.v_cache};
+        for (const void *p : required)
+            if (!p) return fail(ARTAB_ERR_NULL_POINTER, "layer stack: layer %d: only the biases may be NULL", l);
+        if (f32 && !L.b_1) return fail(ARTAB_ERR_NULL_POINTER, "layer stack: layer %d: b_1 is required in float32", l);
+        bool off = misaligned16(L.b_1) || misaligned16(L.b_2);
+        for (const void *p : required) off = off || misaligned16(p);
+        if (off) return fail(ARTAB_ERR_BAD_STRIDE, "layer stack: layer %d: weights, vectors and caches must be 16-byte aligned", l);
+    }
+    return ARTAB_OK;
+}
 }  // namespace
 
 int artab_pack_stack_weight_float(const void *w, void *packed, int N, int K, void *stream) {
@@ -1711,6 +1727,7 @@ int artab_layer_stack(const artab_stack_args *a, int dtype, void *stream) {
     const int Dh = a->D / a->H, e = elem_size(dtype);
     if (misaligned16(a->scratch) || Dh * e % 16)
         return fail(ARTAB_ERR_BAD_STRIDE, "layer stack: scratch and heads must be whole 16-byte pieces");
+    ARTAB_TRY(check_stack_pointers(a, f32));
     const StackScratch s = stack_scratch(a, dtype);
     char *base = static_cast<char *>(a->scratch);
     char *qkv = base + s.qkv, *attn = base + s.attn;
@@ -1730,8 +1747,6 @@ int artab_layer_stack(const artab_stack_args *a, int dtype, void *stream) {
                                   stream));
     }
     for (int l = 0; l < a->n_layers; ++l, ++L) {
-        if (!L->k_cache || !L->v_cache || misaligned16(L->k_cache) || misaligned16(L->v_cache))
-            return fail(ARTAB_ERR_NULL_POINTER, "layer stack: layer %d needs 16-byte aligned caches", l);
         const artab_view kc = {L->k_cache, cache_b, cache_h, Dh}, vc = {L->v_cache, cache_b, cache_h, Dh};
         if (a->num_targets == 0) {
             ARTAB_TRY(artab_prefill_attention_sliced(&q, &k, &v, &out, &kc, &vc, a->own_caches ? a->B : 1, a->B, a->H, a->N, Dh, 0.f,

@@ -278,6 +278,20 @@ bool supported(const artab_train_args *a) {
            a->first_row >= 0 && a->first_row < a->R && static_cast<int64_t>(a->B) * a->R < (1 << 30);
 }
 
+// The kernels read and write 16-byte pieces.
+template <typename... P>
+bool off_16(P... p) {
+    return ((reinterpret_cast<uintptr_t>(p) % 16 != 0) || ...);
+}
+int check_parameters(const artab_train_args *a) {
+    const void *const *p = reinterpret_cast<const void *const *>(a->params);
+    for (int i = 0; i < 16 * a->n_layers; ++i) {
+        if (!p[i]) return ARTAB_ERR_NULL_POINTER;
+        if (off_16(p[i])) return ARTAB_ERR_BAD_STRIDE;
+    }
+    return off_16(a->x, a->saved, a->norm_gamma, a->norm_beta) ? ARTAB_ERR_BAD_STRIDE : ARTAB_OK;
+}
+
 constexpr int kEmbedSlices = 8;
 
 bool embed_supported(const artab_train_embed_args *a) {
@@ -332,12 +346,14 @@ int artab_train_embed(const artab_train_embed_args *a, void *stream) {
     if (!a->x_context || !a->y_context || (a->n_buffer && (!a->x_buffer || !a->y_buffer || !a->tokens)) || !a->x_target || !a->w_x || !a->b_x ||
         !a->w_y || !a->b_y || !a->markers || !a->out || !a->xy)
         return ARTAB_ERR_NULL_POINTER;
+    if (artab::off_16(a->w_x, a->b_x, a->w_y, a->b_y, a->markers, a->tokens, a->out, a->xy)) return ARTAB_ERR_BAD_STRIDE;
     hipStream_t st = static_cast<hipStream_t>(stream);
     return a->D == 128 ? artab::embed<128>(*a, st) : artab::embed<256>(*a, st);
 }
 int artab_train_embed_backward(const artab_train_embed_args *a, void *stream) {
     if (!artab::embed_supported(a)) return ARTAB_ERR_UNSUPPORTED;
     if (!a->out || !a->xy || !a->grads || !a->scratch) return ARTAB_ERR_NULL_POINTER;
+    if (artab::off_16(a->out, a->xy, a->grads, a->scratch)) return ARTAB_ERR_BAD_STRIDE;
     hipStream_t st = static_cast<hipStream_t>(stream);
     return a->D == 128 ? artab::embed_backward<128>(*a, st) : artab::embed_backward<256>(*a, st);
 }
@@ -357,6 +373,8 @@ size_t artab_train_scratch_bytes(const artab_train_args *a) {
 int artab_train_forward(const artab_train_args *a, void *stream) {
     if (!artab::supported(a)) return ARTAB_ERR_UNSUPPORTED;
     if (!a->x || !a->params || !a->saved || !a->z || !a->norm_gamma || !a->norm_beta) return ARTAB_ERR_NULL_POINTER;
+    const int rc = artab::off_16(a->z) ? ARTAB_ERR_BAD_STRIDE : artab::check_parameters(a);
+    if (rc != ARTAB_OK) return rc;
     hipStream_t st = static_cast<hipStream_t>(stream);
     return a->D == 128 ? artab::forward<128, 256>(*a, st) : artab::forward<256, 256>(*a, st);
 }
@@ -364,6 +382,8 @@ int artab_train_backward(const artab_train_args *a, void *stream) {
     if (!artab::supported(a)) return ARTAB_ERR_UNSUPPORTED;
     if (!a->x || !a->params || !a->saved || !a->dz || !a->dx || !a->grads || !a->scratch || !a->norm_gamma || !a->norm_beta)
         return ARTAB_ERR_NULL_POINTER;
+    const int rc = artab::off_16(a->dz, a->dx, a->grads, a->scratch) ? ARTAB_ERR_BAD_STRIDE : artab::check_parameters(a);
+    if (rc != ARTAB_OK) return rc;
     hipStream_t st = static_cast<hipStream_t>(stream);
     return a->D == 128 ? artab::backward<128, 256>(*a, st) : artab::backward<256, 256>(*a, st);
 }

@@ -568,7 +568,8 @@ int artab_train_embed_backward(const artab_train_embed_args *args, void *stream)
  *   num_targets > 0   teacher forcing (inference.py:455-471, :835-890): N = 2 num_targets rows against rows
  *                     [0, Nc) of the caches; caches of their own per batch entry get the N rows' K and V behind
  * Caches: contiguous, [B, H, cache_rows, D / H] with own_caches, else [H, cache_rows, D / H] shared by all batch
- * entries (a prefill stores batch entry 0).  x and out: [B, N, D] contiguous.  The struct is read before the call returns.
+ * entries (a prefill stores batch entry 0).  x and out: [B, N, D] contiguous.  Every pointer 16-byte aligned, checked before the
+ * first launch; b_2 may be NULL, b_1 in 16 bits only.  The struct is read before the call returns.
  */
 typedef struct artab_stack_layer {
     const void *w_fo, *w_qkv, *w_o, *w_1, *b_1, *w_2, *b_2; /* weights packed, as for artab_layer_pre / _post */
