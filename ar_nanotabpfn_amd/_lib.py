@@ -213,6 +213,7 @@ SIGNATURES = {
     "artab_train_embed": (_i, [ctypes.POINTER(ArtabTrainEmbedArgs), _p]),
     "artab_train_embed_backward": (_i, [ctypes.POINTER(ArtabTrainEmbedArgs), _p]),
     "artab_trajectory_group": (_i, [_i, _i, _i, _i, _i, _i, _i, _i]),
+    "artab_trajectory_group_layers": (_i, [_i, _i, _i, _i, _i, _i, _i, _i, _i]),
     "artab_trajectory_tape_bytes": (_sz, [_i, _i, _i, _i]),
     "artab_trajectory_pack": (_i, [_p, _p, _i, _i, _i, _i, _i, _i, _i, _p]),
     "artab_trajectory_decode": (_i, [ctypes.POINTER(ArtabTrajectoryArgs), _i, _p]),

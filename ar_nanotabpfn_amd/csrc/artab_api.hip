@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -1795,32 +1796,52 @@ static TrajectoryTapeLayout trajectory_layout(int D, int F, int n_layers, int dt
 // weights, the context and its trajectories' rows through one compute unit: 3 us and 85 GB/s of those
 // bytes (float32, bound by its products as well: 52 GB/s), whatever the batch.  The launches of the
 // other route take 26 / 29 / 50 us at d_model 128 / 256 / 512, more beyond 1024 trajectories, and
-// their context pass has the matrix cores of the whole chip (float32: neither fused nor on the matrix
-// cores).  Measured on 48 shapes (4 layers, 24 steps; us per layer and step, whole run against launches):
+// their context pass has the matrix cores of the whole chip.  In float32 their layers are not fused: 135 us at
+// d_model 128, 170 at 256, and 40 and 80 TFLOP/s over the context.  Measured on 48 shapes (4 layers, 24 steps; us per layer and step, whole run against launches):
 // d_model 128, 256 trajectories: 8.6 / 24.9 at 64 context rows, 14.8 / 27.1 at 1024, 35.6 / 27.5 at 4096;
 // d_model 256: 15.3 / 28.9, 21.1 / 31.0 at 512, 39.6 / 31.0 at 2048; d_model 512: 38.6 / 49.7, 49.3 / 52.1
-// at 512, 87.7 / 53.8 at 2048; float32 at d_model 256: 37.5 / 186, 71.0 / 443 at 1024.
-// A trajectory with a context of its own has no recorded alternative: it always comes here.
-int artab_trajectory_group(int B, int Nc, int Nt, int H, int D, int F, int own_context, int dtype) {
-    const TrajectoryTapeLayout layout = trajectory_layout(D, F, 1, dtype);
-    if (B < 1 || Nt < 1 || Nc < 1 || H * 32 != D || layout.stride == 0) return 0;
-    static const int cus = [] {
-        int dev = 0, n = 0;
-        if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
-            n = 256;
-        return n;
-    }();
+// at 512, 87.7 / 53.8 at 2048.  float32 (12 steps), d_model 128: 18 / 136 at 64, 55 / 156 at 2048, 167 / 189 at 8192,
+// 64 trajectories: 170 / 165, 1024: 348 / 262; d_model 256: 38 / 176 at 64, 112 / 189 at 2048, 337 / 221 at 8192,
+// 1024 trajectories: 107 / 145 at 512, 226 / 169 at 2048.
+//
+// A trajectory with a context of its own has no recorded alternative: its steps are issued from the host,
+// 100 us per layer and 480 per step (float32: 240), or what their kernels take: one wavefront per
+// trajectory and head at 6.5 GB/s (16-bit types, more than one trajectory), 5 TB/s in all.  Here a workgroup
+// reads the context once per step, 77 GB/s with few of them, 55 with many (float32: 50, 40), 5.6 TB/s in all.
+// Measured at 12 layers, us per layer and step, here / step by step: d_model 512, one trajectory: 91 / 140 at 2048 rows, 146 / 143 at 4096, 255 / 145 at 8192; 64 of
+// them: 127 / 141 at 2048, 207 / 153 at 4096; d_model 256: 123 / 142 at 8192, 176 / 143 at 12288, 16 of
+// them: 167 / 184 at 8192, 64: 100 / 140 at 4096; d_model 128: 118 / 143 at 16384; float32 at d_model 256:
+// 200 / 281 at 4096, 380 / 280 at 8192 (2 layers: 480).
+int artab_trajectory_group_layers(int B, int Nc, int Nt, int H, int D, int F, int n_layers, int own_context, int dtype) {
+    const TrajectoryTapeLayout layout = trajectory_layout(D, F, n_layers, dtype);
+    if (B < 1 || Nt < 1 || Nc < 1 || n_layers < 1 || H * 32 != D || layout.stride == 0) return 0;
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+        cus = 256;
     const int most = layout.max_group, group = (B + cus - 1) / cus < most ? (B + cus - 1) / cus : most;
     const int force = tune(kTuneTrajectory, -1);
     if (force >= 0) return force < most ? force : most;
-    if (own_context) return group;
+    const bool f32 = dtype == ARTAB_F32;
     const double esz = elem_size(dtype), rounds = std::ceil(std::ceil(static_cast<double>(B) / group) / cus);
-    const double bytes = esz * (5.0 * D * D + 2.0 * D * F) + 2 * esz * D * (Nc + 0.5 * Nt * group);
-    const double here = rounds * (3.0 + bytes / (dtype == ARTAB_F32 ? 52e3 : 85e3));
+    const double weights = esz * (5.0 * D * D + 2.0 * D * F), row = 2 * esz * D, l2_rate = f32 ? 52e3 : 85e3;
+    if (own_context) {
+        const double one = row * (Nc + 0.5 * Nt), all = one * B;
+        const double rate = B <= 8 ? (f32 ? 50e3 : 77e3) : (f32 ? 40e3 : 55e3), total = 5.6e6 / std::min(B, cus);
+        const double here = rounds * (3.0 + weights / l2_rate + group * one / std::min(rate, total));
+        const double issued = (f32 ? 240.0 : 100.0) + 480.0 / n_layers;
+        const double wavefront = f32 || B == 1 ? 0.0 : one / H / 6.5e3;
+        const double there = std::max(issued, 20.0 + std::max(wavefront, all / 5e6));
+        return here < there ? group : 0;
+    }
+    const double here = rounds * (3.0 + (weights + row * (Nc + 0.5 * Nt * group)) / l2_rate);
     const double flops = 8.0 * B * Nc * D;
-    const double there = (D == 512 ? 50.0 : D == 256 ? 29.0 : 26.0) + (B > 1024 ? 4.2e-5 * (B - 1024) * D : 0.0) +
-                         (dtype == ARTAB_F32 ? 70.0 + flops / 5e6 : flops / 1200e6);
+    const double there = f32 ? (D == 128 ? 135.0 + flops / 40e6 : 170.0 + flops / 80e6)
+                             : (D == 512 ? 50.0 : D == 256 ? 29.0 : 26.0) + (B > 1024 ? 4.2e-5 * (B - 1024) * D : 0.0) + flops / 1200e6;
     return here < there ? group : 0;
+}
+
+int artab_trajectory_group(int B, int Nc, int Nt, int H, int D, int F, int own_context, int dtype) {
+    return artab_trajectory_group_layers(B, Nc, Nt, H, D, F, 12, own_context, dtype);
 }
 
 size_t artab_trajectory_tape_bytes(int D, int F, int n_layers, int dtype) {

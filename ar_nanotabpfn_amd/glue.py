@@ -433,7 +433,7 @@ class TrajectoryDecoder:
 
     def group(self, B: int, Nc: int, Nt: int, own_context: bool) -> int:
         """Trajectories per workgroup, or 0 where the step-by-step launches are the faster route."""
-        return _lib.load().artab_trajectory_group(B, Nc, Nt, self.H, self.D, self.F, int(own_context), self.dtype_code)
+        return _lib.load().artab_trajectory_group_layers(B, Nc, Nt, self.H, self.D, self.F, self.L, int(own_context), self.dtype_code)
 
     def __call__(self, caches, n_ctx: int, own_base: int, x_mean: Tensor, rand_u: Tensor, rand_n: Tensor, group: int) -> Tensor:
         """``caches``: per layer ``(context K, context V, trajectory K, trajectory V)``, contiguous; with

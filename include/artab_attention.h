@@ -598,7 +598,8 @@ int artab_layer_stack(const artab_stack_args *args, int dtype, void *stream);
  * artab_trajectory_group says how many trajectories a workgroup should take, or 0: no kernel for
  * these widths (head_dim 32; D in {128, 256, 512}, F = 256; D 512 in 16-bit types only), or the step-by-step
  * launches, which spread one layer over the whole chip, are the faster route for this problem.
- * own_context: every trajectory has its own context rows in front of its buffer rows.
+ * own_context: every trajectory has its own context rows in front of its buffer rows.  _layers: of a model of n_layers
+ * (the other route has a cost per step beside that per layer); without it, of 12.
  *
  * The weights are kept a second time as `tape`, artab_trajectory_tape_bytes of device memory (16-byte aligned),
  * written by artab_trajectory_pack: once per layer for ARTAB_TAPE_FO (w = W_out W_v of the feature attention,
@@ -639,6 +640,7 @@ typedef struct artab_trajectory_args {
 } artab_trajectory_args;
 
 int artab_trajectory_group(int B, int Nc, int Nt, int H, int D, int F, int own_context, int dtype);
+int artab_trajectory_group_layers(int B, int Nc, int Nt, int H, int D, int F, int n_layers, int own_context, int dtype);
 size_t artab_trajectory_tape_bytes(int D, int F, int n_layers, int dtype);
 int artab_trajectory_pack(void *tape, const void *w, int which, int layer, int rows, int D, int F, int n_layers,
                           int dtype, void *stream);
