@@ -399,8 +399,11 @@ struct TrainForwardB {
     long M;
 };
 
-// h = gelu(u) and its derivative, in float32: erf by the rational form 7.1.26 of Abramowitz and Stegun (absolute
-// error below 1.5e-7; both results are rounded to bf16), which shares its exponential with the derivative
+// h = gelu(u) and its derivative, in float32: erf by the rational form 7.1.26 of Abramowitz and Stegun, which shares
+// its exponential with the derivative.  Its absolute error is below 1.5e-7; both results are rounded to bf16, of
+// whose unit in the last place that is a hundredth for u above -3 and a quarter at -4.5, where h is 1.5e-5.  On
+// normal u the rounded results are as far from float64 as with erff (1.66620e-3 and 1.91314e-3 of their norms).  With
+// normal_tail() instead a training step of 38912 rows and 12 layers takes 4.23 ms, 4.19 with this.
 __device__ __forceinline__ void train_gelu(float u, float &h, float &dh) {
     const float z = fabsf(u) * 0.70710678118654752f, e = fast_exp2(-z * z * kLog2e);
     const float t = __builtin_amdgcn_rcpf(fmaf(0.3275911f, z, 1.f));
