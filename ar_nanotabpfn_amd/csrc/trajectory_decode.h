@@ -31,7 +31,7 @@
 // straight from LDS, masked to (row 2 g, columns 2 g and 2 g + 1).  A value that is not finite stays with
 // the columns that see it: products of keys that only some columns see reach those columns only.  Softmax in float32 with scale *
 // log2(e) folded into the queries and rounded to the model's type, probabilities rounded to the
-// model's type: the rounding model of the other kernels.  The reference a column's probabilities are
+// model's type and summed as rounded: the rounding model of the context pass (mfma_flash.h).  The reference a column's probabilities are
 // taken against follows its maximum only when that has risen by more than kSlack (base 2): the common
 // block has no exchange between lanes and no rescaling.
 #pragma once
@@ -414,6 +414,12 @@ __global__ __launch_bounds__(kTrajWaves * 64) void trajectory_decode_kernel(Traj
             qf[x] = *reinterpret_cast<const u32x4 *>(qs + (k16 ? row16 : tok) * LD + DH * h + Ops::kStep * x + Ops::kPer * quad);
         f32x4 o_acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
         float m_run = -1e30f, l_run = 0.f;
+        // 16 bits: the sum of the probabilities as the second product takes them, rounded, from one more product
+        // with a row of ones (of the unrounded ones, their rounding would not cancel in the division)
+        f32x4 l_acc = {0.f, 0.f, 0.f, 0.f};
+        unsigned one2 = 0u;
+        if constexpr (k16) one2 = pack2<T>(1.f, 1.f);
+        const u32x4 ones = {one2, one2, one2, one2};
         // Scores (lane: keys 4 sub + r of each 16-key part, its token) to probabilities.
         auto fold = [&](auto &sc) {
             constexpr int NX = sizeof(sc) / sizeof(sc[0]);
@@ -425,7 +431,8 @@ __global__ __launch_bounds__(kTrajWaves * 64) void trajectory_decode_kernel(Traj
             if (__any(tmax > m_run + Ops::kSlack)) {
                 const float m_new = fmaxf(m_run, Ops::max(tmax));
                 const float alpha = fast_exp2(m_run - m_new);
-                l_run *= alpha;
+                if constexpr (k16) l_acc[0] *= alpha;
+                else l_run *= alpha;
 #pragma unroll
                 for (int db = 0; db < 2; ++db)
 #pragma unroll
@@ -436,7 +443,7 @@ __global__ __launch_bounds__(kTrajWaves * 64) void trajectory_decode_kernel(Traj
             for (int x = 0; x < NX; ++x) {
 #pragma unroll
                 for (int r = 0; r < 4; ++r) sc[x][r] = fast_exp2(sc[x][r] - m_run);
-                l_run += (sc[x][0] + sc[x][1]) + (sc[x][2] + sc[x][3]);
+                if constexpr (!k16) l_run += (sc[x][0] + sc[x][1]) + (sc[x][2] + sc[x][3]);
             }
         };
         typedef short s16x8 __attribute__((ext_vector_type(8)));
@@ -492,6 +499,7 @@ __global__ __launch_bounds__(kTrajWaves * 64) void trajectory_decode_kernel(Traj
                 __builtin_amdgcn_wave_barrier();
                 const u32x4 pv = {pack2<T>(sc[0][0], sc[0][1]), pack2<T>(sc[0][2], sc[0][3]),
                                   pack2<T>(sc[1][0], sc[1][1]), pack2<T>(sc[1][2], sc[1][3])};
+                l_acc = Ops::mma(ones, pv, l_acc);
 #pragma unroll
                 for (int db = 0; db < 2; ++db) {
                     const T *a = vt + (4 * quad + (row16 >> 2)) * VPAD + 16 * db + 4 * (lane & 3);
@@ -529,7 +537,10 @@ __global__ __launch_bounds__(kTrajWaves * 64) void trajectory_decode_kernel(Traj
             for (int db = 0; db < 2; ++db) traj_load4<T>(vn + (tok & ~1) * LD + DH * h + 16 * db + 4 * sub, vr[db]);
             fold(sc);
             float p = Ops::sum((sc[0][0] + sc[0][1]) + (sc[0][2] + sc[0][3]));
-            if constexpr (k16) p = to_f32(from_f32<T>(p));
+            if constexpr (k16) {
+                p = to_f32(from_f32<T>(p));
+                l_acc[0] += p;
+            }
             if (k16 || quad == 0) {  // (float32: the four rows of lanes are partial sums)
 #pragma unroll
                 for (int db = 0; db < 2; ++db)
@@ -537,7 +548,7 @@ __global__ __launch_bounds__(kTrajWaves * 64) void trajectory_decode_kernel(Traj
                     for (int e = 0; e < 4; ++e) o_acc[db][e] = fmaf(p, vr[db][e], o_acc[db][e]);
             }
         }
-        float l_tot = Ops::sum(l_run);
+        float l_tot = k16 ? l_acc[0] : Ops::sum(l_run);
 #pragma unroll
         for (int db = 0; db < 2; ++db) Ops::finish(o_acc[db]);
         if constexpr (NP > 1) {  // the other wavefronts' keys of this head
