@@ -36,14 +36,27 @@ def test_native_calls_equal_the_python_path(device, monkeypatch, dtype, own_cont
         assert torch.equal(a, b) and a.stride() == b.stride()
 
 
-def test_what_is_not_plain_raises_as_before(device):
+def test_what_is_not_plain_raises_as_before(device, monkeypatch):
     q, k = _randn(device, torch.float16, 2, 4, 1, 32), _randn(device, torch.float16, 4, 16, 32)
     buf = _randn(device, torch.float16, 2, 4, 3, 32)
-    with pytest.raises(Exception):
-        ak.context_attention(q, k[:3], k[:3])
-    with pytest.raises(Exception):
-        ak.context_attention(q.cpu(), k, k)
-    with pytest.raises(Exception):
-        ak.decode_attention(q, k, k, buf, buf, 4)
-    with pytest.raises(Exception):
-        ak.decode_attention(q, k, k, buf, buf, 3, q, q)  # no room for the new row
+    cases = [
+        (ValueError, "do not match q", lambda: ak.context_attention(q, k[:3], k[:3])),
+        (ValueError, "do not match q", lambda: ak.context_attention(q, k[:, :, :16], k[:, :, :16])),
+        (ValueError, "one dtype", lambda: ak.context_attention(q, k.float(), k.float())),
+        (ValueError, "needs Nc >= 1", lambda: ak.context_attention(q, k[:, :0], k[:, :0])),
+        (ValueError, "head_dim axis must be contiguous", lambda: ak.context_attention(q, k.transpose(1, 2).contiguous().transpose(1, 2), k)),
+        (ValueError, "unsupported dtype", lambda: ak.context_attention(q.double(), k.double(), k.double())),
+        (RuntimeError, "HIP device only", lambda: ak.context_attention(q.cpu(), k, k)),
+        (ValueError, "capacity", lambda: ak.decode_attention(q, k, k, buf, buf, 4)),
+        (ValueError, "capacity", lambda: ak.decode_attention(q, k, k, buf, buf, 3, q, q)),  # no room for the new row
+        (ValueError, "must be given together", lambda: ak.decode_attention(q, k, k, buf, buf, 1, q)),
+        (ValueError, "N=1 .target. or N=2", lambda: ak.decode_attention(q.expand(-1, -1, 3, -1), k, k, buf, buf, 1)),
+        (ValueError, "negative buffer length", lambda: ak.decode_attention(q, k, k, buf, buf, -1)),
+    ]
+    for error, message, call in cases:
+        with pytest.raises(error, match=message) as with_native:
+            call()
+        with monkeypatch.context() as m, pytest.raises(error, match=message) as without:
+            m.setattr(ak, "_call", lambda *a: None)
+            call()
+        assert type(with_native.value) is type(without.value) is error and str(with_native.value) == str(without.value)

@@ -50,3 +50,42 @@ def test_fused_training_equals_modules(device, monkeypatch, D, H, L, B, Nc, Nb, 
         assert grads[n].shape == r.shape and torch.isfinite(grads[n]).all()
         # (both sides round every product operand to eight bits: a per cent or two for the smallest gradients)
         assert float((grads[n] - r).norm()) <= 4e-2 * float(r.norm()) + 1e-6, n
+
+
+@pytest.mark.parametrize("D,H,L,B,Nc,Nb,Nt", [(128, 4, 4, 8, 40, 8, 64), (256, 8, 2, 5, 33, 5, 61)])
+def test_both_routes_against_float32(device, monkeypatch, D, H, L, B, Nc, Nb, Nt):
+    """The gradients of both routes under autocast against those of the modules in float32: the fused kernels, which keep
+    the residual stream and the norms in float32, are not further off than the modules."""
+    import ar_nanotabpfn_amd.model as model_mod
+    from ar_nanotabpfn_amd.attention import create_dense_mask, create_row_mask
+
+    torch.manual_seed(1)
+    model = model_mod.ARTabPFN(d_model=D, n_heads=H, n_layers=L, d_ff=256, num_features=2, buffer_size=Nb, num_components=5).to(device)
+    g = torch.Generator().manual_seed(2)
+    mk = lambda *s: torch.randn(*s, generator=g).to(device)  # noqa: E731
+    data, y = (mk(B, Nc, 2), mk(B, Nc), mk(B, Nb, 2), mk(B, Nb), mk(B, Nt, 2)), mk(B, Nt)
+    masks = (create_dense_mask(1), create_row_mask(Nc + Nb + Nt, Nc, Nb))
+
+    def step(autocast):
+        model.zero_grad(set_to_none=True)
+        with torch.autocast("cuda", dtype=torch.bfloat16, enabled=autocast):
+            loss = model(*data, *masks, y_target=y)
+        loss.backward()
+        return loss.double(), {n: p.grad.double() for n, p in model.named_parameters()}
+
+    fused_loss, fused = step(True)
+    monkeypatch.setattr(model_mod, "layer_stack_supported", lambda *a: False)
+    monkeypatch.setattr(model_mod, "embed_rows", lambda *a: None)
+    module_loss, modules = step(True)
+    true_loss, true = step(False)
+
+    def error(a, names):
+        return float(torch.stack([(a[n] - true[n]).norm() ** 2 for n in names]).sum().sqrt()
+                     / torch.stack([true[n].norm() ** 2 for n in names]).sum().sqrt())
+
+    groups = {"all": list(true), "layers": [n for n in true if "layers" in n], "embedding": [n for n in true if "embed" in n or n == "ar_tokens"]}
+    report = {g: (error(fused, names), error(modules, names)) for g, names in groups.items()}
+    print(report, float(abs(fused_loss - true_loss) / true_loss), float(abs(module_loss - true_loss) / true_loss))
+    # products of bf16 operands on both sides: 2^-9 each, some tens of them
+    assert all(f <= m and f <= 2e-2 for f, m in report.values()), report
+    assert abs(fused_loss - true_loss) <= 2e-3 * abs(true_loss)
