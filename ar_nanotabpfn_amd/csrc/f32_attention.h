@@ -45,7 +45,8 @@ struct F32Plan {
     long rows;            // B * H * Lq
 };
 
-template <int DH, int QB, bool SPLIT, int NW>
+// HIDES: there are keys that some column may not see (buffers, new rows); without them there is one pass and no watch.
+template <int DH, int QB, bool SPLIT, int NW, bool HIDES>
 __global__ __launch_bounds__(NW * 64) void f32_attention_kernel(PortableParams P, F32Plan L) {
     constexpr int KT = DH / 16;   // 16-byte pieces per lane and K row; output blocks
     constexpr int COLS = 16 * QB;
@@ -198,16 +199,17 @@ __global__ __launch_bounds__(NW * 64) void f32_attention_kernel(PortableParams P
     // nothing requested ahead, so that it needs no registers that the common pass does not.
     f32x4 o[QB][KT];
     float m[QB], l[QB];
+    // (here and below: set inside the lambda, they cost the common kernels up to 30 registers)
+#pragma unroll
+    for (int j = 0; j < QB; ++j) {
+        m[j] = -INFINITY;
+        l[j] = 0.f;
+#pragma unroll
+        for (int n = 0; n < KT; ++n) o[j][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
     auto pass = [&](auto careful) {
         constexpr bool CAREFUL = decltype(careful)::value;
         float watch = 0.f;  // NaN: values that are not finite
-#pragma unroll
-        for (int j = 0; j < QB; ++j) {
-            m[j] = -INFINITY;
-            l[j] = 0.f;
-#pragma unroll
-            for (int n = 0; n < KT; ++n) o[j][n] = f32x4{0.f, 0.f, 0.f, 0.f};
-        }
         int t_now = t_first;
         if (t_now >= t_end) return false;
         Block cur = block_of(t_now);
@@ -279,7 +281,7 @@ __global__ __launch_bounds__(NW * 64) void f32_attention_kernel(PortableParams P
                         s[j][sb][r] = fast_exp2(s[j][sb][r] - m_use);
                         l[j] += s[j][sb][r];
                     }
-                const bool masked = hidden && cur.kind != 0;
+                const bool masked = HIDES && hidden && cur.kind != 0;
                 auto value = [&](const fvec (&v)[VN], int n) {
                     if constexpr (KT < 4) return v[0][n];
                     else return v[n / 4][n % 4];
@@ -330,7 +332,19 @@ __global__ __launch_bounds__(NW * 64) void f32_attention_kernel(PortableParams P
         }
         return __any(watch != 0.f) != 0;
     };
-    if (pass(std::false_type{})) pass(std::true_type{});
+    const bool again = pass(std::false_type{});
+    if constexpr (HIDES) {
+        if (again) {
+#pragma unroll
+            for (int j = 0; j < QB; ++j) {
+                m[j] = -INFINITY;
+                l[j] = 0.f;
+#pragma unroll
+                for (int n = 0; n < KT; ++n) o[j][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+            }
+            pass(std::true_type{});
+        }
+    }
 #pragma unroll
     for (int j = 0; j < QB; ++j) l[j] = row_sum(l[j]);
 

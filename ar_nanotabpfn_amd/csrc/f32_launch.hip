@@ -28,19 +28,26 @@ F32Shape plan_f32(int H, int Nc, int Dh, int G, int n_groups) {
     return s;
 }
 
-template <int DH, int QB>
-static hipError_t launch(const PortableParams &P, const F32Plan &L, bool split, hipStream_t st) {
+template <int DH, int QB, bool HIDES>
+static hipError_t launch_hides(const PortableParams &P, const F32Plan &L, bool split, hipStream_t st) {
     const long kvg8 = (static_cast<long>(P.H) * L.n_groups + 7) / 8;
     if (split) {
         const unsigned grid = static_cast<unsigned>(8 * kvg8 * L.tiles * L.n_split);
-        hipLaunchKernelGGL((f32_attention_kernel<DH, QB, true, 8>), dim3(grid), dim3(512), 0, st, P, L);
+        hipLaunchKernelGGL((f32_attention_kernel<DH, QB, true, 8, HIDES>), dim3(grid), dim3(512), 0, st, P, L);
         if (L.n_split > 1)
             hipLaunchKernelGGL(f32_combine_kernel<DH>, dim3(static_cast<unsigned>((L.rows * (DH / 4) + 255) / 256)), dim3(256), 0, st, P, L);
     } else {
         const unsigned grid = static_cast<unsigned>(8 * kvg8 * ((L.tiles + 3) / 4));
-        hipLaunchKernelGGL((f32_attention_kernel<DH, QB, false, 4>), dim3(grid), dim3(256), 0, st, P, L);
+        hipLaunchKernelGGL((f32_attention_kernel<DH, QB, false, 4, HIDES>), dim3(grid), dim3(256), 0, st, P, L);
     }
     return hipGetLastError();
+}
+
+// A context alone is seen by every column: its calls go without the watch for values that have to be kept apart
+// (one query on 4000 rows 13.5 -> 13.1 us).
+template <int DH, int QB>
+static hipError_t launch(const PortableParams &P, const F32Plan &L, bool split, hipStream_t st) {
+    return P.Nb > 0 || P.new_row >= 0 || P.nbuf_dev ? launch_hides<DH, QB, true>(P, L, split, st) : launch_hides<DH, QB, false>(P, L, split, st);
 }
 
 hipError_t launch_f32_attention(PortableParams P, bool stacked, void *workspace, size_t workspace_bytes, hipStream_t st) {

@@ -67,7 +67,7 @@ class Sources:
 
     def __init__(self, tensors):
         self._tensors, self._facts = list(tensors), _values_at(tensors)
-        self._storages = [t.detach() for t in tensors]
+        self._storages = [t.untyped_storage() for t in self._tensors]
 
     def unchanged(self, tensors) -> bool:
         return _same(self._tensors, tensors) and _values_at(tensors) == self._facts
@@ -75,6 +75,11 @@ class Sources:
 
 def capturing(device) -> bool:
     return device.type == "cuda" and torch.cuda.is_current_stream_capturing()
+
+
+def _current_stream(device) -> int:
+    """The current stream's handle (a ``torch.cuda.Stream`` object costs 3 us; a first call asks some 50 times)."""
+    return torch._C._cuda_getCurrentRawStream(device.index if device.index is not None else torch.cuda.current_device())
 
 
 class Prepared:
@@ -85,23 +90,23 @@ class Prepared:
     def __init__(self, tensors):
         self.tensors = tuple(tensors)
         self._device = next((t.device for t in self.tensors if t.is_cuda), None)
-        if self._device is not None and not capturing(self._device):
-            stream = torch.cuda.current_stream(self._device)
-            self._made, self._home, self._others = torch.cuda.Event(), stream.cuda_stream, set()
-            self._made.record(stream)
+        if self._device is not None:
+            self._home = _current_stream(self._device)
+            self._streams = {self._home}
 
     def use(self) -> tuple:
         # (a recording cannot wait for what lies outside of it; it begins with everything in front of it done)
-        if self._device is None or capturing(self._device):
-            return self.tensors
-        stream = torch.cuda.current_stream(self._device)
-        if stream.cuda_stream != self._home:
-            stream.wait_event(self._made)
-            if stream.cuda_stream not in self._others:
-                for t in self.tensors:
-                    if t.is_cuda:
-                        t.record_stream(stream)
-                self._others.add(stream.cuda_stream)
+        if (self._device is not None and _current_stream(self._device) not in self._streams
+                and not torch.cuda.is_current_stream_capturing()):
+            stream = torch.cuda.current_stream(self._device)
+            home = (torch.cuda.ExternalStream(self._home, device=self._device) if self._home
+                    else torch.cuda.default_stream(self._device))
+            # behind what the making stream has been given so far: no event has to be kept for calls that stay on it
+            stream.wait_event(home.record_event())
+            for t in self.tensors:
+                if t.is_cuda:
+                    t.record_stream(stream)
+            self._streams.add(stream.cuda_stream)
         return self.tensors
 
 
