@@ -1,7 +1,7 @@
 // Portable attention kernels: one wavefront per query row, float32 arithmetic,
 // any dtype, any head_dim <= 256.  They implement every entry point of the C ABI
 // (context / decode / teacher forcing / prefill / masked buffer attention / merge)
-// and serve the float32 path and the shapes the MFMA kernels do not cover.
+// and serve the shapes, views and masks that the matrix-core kernels do not cover.
 #pragma once
 
 #include "common.h"

@@ -19,7 +19,8 @@
 // Tiles.  A workgroup of four wavefronts owns 32 rows and all columns; products are transposed as in
 // fused_layer.h (C^T[n, m] = sum_k W[n, k] A[m, k], v_mfma_f32_16x16x32): a lane holds, for two token rows
 // (lane % 16 and + 16), four consecutive features 4 (lane / 16) + r of every 16-feature block.  Small
-// workgroups, four or five to a compute unit, so that the loads of one run under the products of others.
+// workgroups, so that the loads of one run under the products of others: forward four or five to a compute unit at
+// d_model 128, three or four at 256; backward two or three, where registers (256 in backward b) are the limit.
 #pragma once
 
 #include "common.h"

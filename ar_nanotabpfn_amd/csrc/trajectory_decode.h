@@ -7,7 +7,7 @@
 // pays 30-40 us per layer for them whatever the size of the problem; here a layer costs what one
 // compute unit needs to stream its weights and keys through (64 B per clock from the L2) plus ten
 // workgroup barriers and the latency chains between them.  The rule for when the launches of the
-// other route, which spread one layer over the whole chip, are faster is artab_trajectory_group().
+// other route, which spread one layer over the whole chip, are faster is artab_trajectory_group_layers().
 //
 // Rows.  A workgroup owns G trajectories; token row 2 g is trajectory g's buffer row of the step (the
 // value drawn last), row 2 g + 1 its target row: at most 16 rows (16-bit types) or 4 (float32, whose

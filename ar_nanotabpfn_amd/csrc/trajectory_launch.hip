@@ -18,8 +18,10 @@ typedef float TrajT;
 
 namespace {
 
-// Runs `f` with the shape of (D, F) as a compile-time type; false where none is built.  The widths
-// are those whose activation tiles fit the LDS of one compute unit.
+// Runs `f` with the shape of (D, F) as a compile-time type; false where none is built.  The widths D are those
+// whose activation tiles fit the LDS of one compute unit; F is the feed-forward width that the model's default
+// and the training configuration have, others would be further instances (a model with one of them takes
+// the step-by-step launches).
 template <typename T, typename Fn>
 bool with_shape(int D, int F, Fn f) {
     if (F == 256) {

@@ -99,7 +99,7 @@ class ARTabPFNPredictor:
         # of that layer is read by nobody (its K/V were cached before the attention call).
         self.target_only_last_layer = True
         # Take a whole sampling run through one launch where that is the faster route (the library's
-        # rule, ``artab_trajectory_group``) and the sampling switches above are at their defaults.
+        # rule, ``artab_trajectory_group_layers``) and the sampling switches above are at their defaults.
         self.whole_run_decode = True
         self._stack = LayerStack()
         self._trajectory = None      # (key of the model state, TrajectoryDecoder or None)
