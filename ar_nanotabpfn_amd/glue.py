@@ -102,12 +102,34 @@ def pack_weight(w: Tensor) -> Tensor:
     return packed
 
 
+def _check_sizes(D: int, packed, vectors) -> None:
+    """Sizes that the layer launches take for granted: ``packed`` are (packed weight, N, K), ``vectors`` (vector or None,
+    length).  As a product of matrices that do not fit, anything else is a ``RuntimeError``."""
+    for w, n, k in packed:
+        if w.shape[0] * 32 != n or w.shape[1] * 16 != k:
+            raise RuntimeError(f"a weight of {w.shape[0] * 32} x {w.shape[1] * 16} in a layer of width {D} that needs {n} x {k}")
+    for v, n in vectors:
+        if v is not None and v.numel() != n:
+            raise RuntimeError(f"a vector of {v.numel()} in a layer of width {D} that needs {n}")
+
+
+def _check_pre(D: int, w_fo: Tensor, norm1: nn.LayerNorm, w_qkv: Tensor) -> None:
+    _check_sizes(D, ((w_fo, D, D), (w_qkv, 3 * D, D)), ((norm1.weight, D), (norm1.bias, D)))
+
+
+def _check_post(D: int, w_o: Tensor, norm2: nn.LayerNorm, w_1: Tensor, b_1, w_2: Tensor, b_2, norm3: nn.LayerNorm) -> None:
+    F_ = w_1.shape[0] * 32
+    _check_sizes(D, ((w_o, D, D), (w_1, F_, D), (w_2, D, F_)),
+                 ((norm2.weight, D), (norm2.bias, D), (b_1, F_), (b_2, D), (norm3.weight, D), (norm3.bias, D)))
+
+
 def layer_pre(x: Tensor, w_fo: Tensor, norm1: nn.LayerNorm, w_qkv: Tensor):
     """``y = norm1(x + x @ W_fo.T)``, ``qkv = y @ W_qkv.T`` in one launch; ``w_fo`` and
     ``w_qkv`` are the packed forms (``pack_weight``) of ``W_fo [D, D]`` and ``W_qkv [3D, D]``.
 
     Returns ``(y [rows, D], qkv [rows, 3D])``."""
     D = x.shape[-1]
+    _check_pre(D, w_fo, norm1, w_qkv)
     x2 = _rows16(x)
     rows = x2.shape[0]
     y = torch.empty((rows, D), device=x.device, dtype=x.dtype)
@@ -128,6 +150,7 @@ def layer_post(attn: Tensor, y: Tensor, w_o: Tensor, norm2: nn.LayerNorm, w_1: T
 
     ``attn`` and ``y`` are ``[rows, D]``-shaped (any leading dims); returns ``[rows, D]``."""
     D = y.shape[-1]
+    _check_post(D, w_o, norm2, w_1, b_1, w_2, b_2, norm3)
     y2 = _rows16(y)
     rows = y2.shape[0]
     out = torch.empty((rows, D), device=y.device, dtype=y.dtype)
@@ -159,6 +182,8 @@ def layer_post_pre(attn: Tensor, y: Tensor, w_o: Tensor, norm2: nn.LayerNorm, w_
     """``layer_post`` of one layer and ``layer_pre`` of the next in one launch; the layer output
     between them is not materialised.  Returns the next layer's ``(y [rows, D], qkv [rows, 3D])``."""
     D = y.shape[-1]
+    _check_post(D, w_o, norm2, w_1, b_1, w_2, b_2, norm3)
+    _check_pre(D, next_w_fo, next_norm1, next_w_qkv)
     y2 = _rows16(y)
     rows = y2.shape[0]
     y_next = torch.empty((rows, D), device=y.device, dtype=y.dtype)
@@ -326,6 +351,8 @@ class DecodeStepBoundary:
             y2 = y2.contiguous()
         p_o, p_1, p_2 = last.packed_weights()[2:]
         n_fo, n_qkv = first.packed_weights()[:2]
+        _check_post(D, p_o, last.norm2, p_1, last.ff[0].bias, p_2, last.ff[2].bias, last.norm3)
+        _check_pre(D, n_fo, first.norm1, n_qkv)
         if hasattr(attn, "desc"):
             parts, a_ptr, lda = ctypes.byref(attn.desc), None, 0
         else:
