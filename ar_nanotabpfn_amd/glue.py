@@ -379,26 +379,36 @@ class TrajectoryDecoder:
     MAX_COMPONENTS = 21  # 3 K outputs in 64 columns
 
     @staticmethod
-    def supported(embedder, backbone, head, x: Tensor) -> bool:
+    def supported(embedder, backbone, head, ar_tokens: Tensor, x: Tensor) -> bool:
         """Whether the kernel is built for this model: equal layers of head dim 32 and widths it has
-        tiles for (``artab_trajectory_tape_bytes``), a scalar mixture head of the same hidden width."""
+        tiles for (``artab_trajectory_tape_bytes``), a scalar mixture head of the same hidden width, every
+        parameter of the type, on the device and of the size that the launch reads it with."""
         layers = list(backbone.layers)
         if not (x.is_cuda and x.dtype in _lib._DTYPE_CODE and layers):
             return False
         lin1, lin2 = head.head[0], head.head[2]
-        D, F_ = lin1.in_features, lin1.out_features
+        D, F_, K = lin1.in_features, lin1.out_features, head.num_components
         first = layers[0]
 
-        def same(layer):
-            lf = layer.ff
-            return (layer.attn_rows.n_heads * 32 == D and lf[0].in_features == D and lf[0].out_features == F_
-                    and lf[2].out_features == D and lf[0].bias is not None and lf[2].bias is not None
-                    and all(getattr(layer, n).eps == getattr(first, n).eps for n in ("norm1", "norm2", "norm3"))
-                    and layer.norm1.weight.dtype == x.dtype)
+        def fits(*tensors_and_shapes):
+            return all(t is not None and t.dtype == x.dtype and t.device == x.device and tuple(t.shape) == shape
+                       for t, shape in zip(tensors_and_shapes[0::2], tensors_and_shapes[1::2]))
 
-        return (head.dim_y == 1 and head.num_components <= TrajectoryDecoder.MAX_COMPONENTS
-                and lin2.out_features == 3 * head.num_components and lin1.bias is not None and lin2.bias is not None
-                and all(same(layer) for layer in layers)
+        def same(layer):
+            af, ar, ff = layer.attn_features, layer.attn_rows, layer.ff
+            norms = [layer.norm1, layer.norm2, layer.norm3]
+            return (ar.n_heads * 32 == D and [n.eps for n in norms] == [getattr(first, n).eps for n in ("norm1", "norm2", "norm3")]
+                    and fits(af.v_proj.weight, (D, D), af.out_proj.weight, (D, D), ar.q_proj.weight, (D, D), ar.k_proj.weight, (D, D),
+                             ar.v_proj.weight, (D, D), ar.out_proj.weight, (D, D), ff[0].weight, (F_, D), ff[0].bias, (F_,),
+                             ff[2].weight, (D, F_), ff[2].bias, (D,))
+                    and all(fits(n.weight, (D,), n.bias, (D,)) for n in norms))
+
+        return (head.dim_y == 1 and K <= TrajectoryDecoder.MAX_COMPONENTS and all(same(layer) for layer in layers)
+                and fits(lin1.weight, (F_, D), lin1.bias, (F_,), lin2.weight, (3 * K, F_), lin2.bias, (3 * K,), head.mean_bias, (K,),
+                         head.std_bias, (K,), head.weight_bias, (K,), backbone.norm.weight, (D,), backbone.norm.bias, (D,),
+                         embedder.x_embed.weight, (D, 1), embedder.x_embed.bias, (D,), embedder.y_embed.weight, (D, 1),
+                         embedder.y_embed.bias, (D,), embedder.marker_embed.weight, (3, D), ar_tokens, (ar_tokens.shape[0], D))
+                and ar_tokens.shape[0] >= 1
                 and _lib.load().artab_trajectory_tape_bytes(D, F_, len(layers), _lib.dtype_code(x.dtype)) > 0)
 
     def __init__(self, embedder, backbone, head, ar_tokens: Tensor):

@@ -461,14 +461,19 @@ class ARTabPFNPredictor:
         else:
             caches = [(l.k_cache, l.v_cache, l.k_cache, l.v_cache) for l in layers]
             n_ctx, own_base, fits = 0, self.seq_len, self.seq_len + Nt <= layers[0].k_cache.shape[2]
-        if not (fits and n_ctx + own_base > 0 and caches[0][2].shape[0] == B
-                and all(t.dtype == x_target.dtype and t.is_contiguous() for c in caches for t in c) and self._run_as_defined()):
+        # (one description of the caches serves all layers)
+        H = layers[0].attn_rows.n_heads
+        shapes = [(H, caches[0][0].shape[-2], 32)] * 2 if shared else [caches[0][0].shape] * 2
+        shapes += [(B, H, caches[0][2].shape[2], 32)] * 2
+        if not (fits and n_ctx + own_base > 0
+                and all(t.dtype == x_target.dtype and t.device == x_target.device and t.shape == s and t.is_contiguous()
+                        for c in caches for t, s in zip(c, shapes)) and self._run_as_defined()):
             return None
         key = (x_target.dtype, self._model_key())
         if self._trajectory is None or self._trajectory[0] != key:
             if capturing(x_target.device):  # (what a recording packs exists when it is replayed)
                 return None
-            ok = TrajectoryDecoder.supported(self.embedder, self.backbone, self.head, x_target)
+            ok = TrajectoryDecoder.supported(self.embedder, self.backbone, self.head, self.ar_tokens, x_target)
             self._trajectory = (key, TrajectoryDecoder(self.embedder, self.backbone, self.head, self.ar_tokens) if ok else None)
         run = self._trajectory[1]
         if run is not None and capturing(x_target.device) and not run.tables_made(caches):

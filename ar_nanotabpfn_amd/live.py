@@ -99,10 +99,13 @@ class Prepared:
         if (self._device is not None and _current_stream(self._device) not in self._streams
                 and not torch.cuda.is_current_stream_capturing()):
             stream = torch.cuda.current_stream(self._device)
-            home = (torch.cuda.ExternalStream(self._home, device=self._device) if self._home
-                    else torch.cuda.default_stream(self._device))
             # behind what the making stream has been given so far: no event has to be kept for calls that stay on it
-            stream.wait_event(home.record_event())
+            try:
+                home = (torch.cuda.ExternalStream(self._home, device=self._device) if self._home
+                        else torch.cuda.default_stream(self._device))
+                stream.wait_event(home.record_event())
+            except RuntimeError:  # a stream of somebody else's making, gone since
+                torch.cuda.synchronize(self._device)
             for t in self.tensors:
                 if t.is_cuda:
                     t.record_stream(stream)
