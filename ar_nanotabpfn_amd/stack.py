@@ -113,7 +113,7 @@ class LayerStack:
         own = k0.dim() == 4
         H, Dh, rows = first.attn_rows.n_heads, first.attn_rows.head_dim, k0.shape[-2]
         shape = (B, H, rows, Dh) if own else (H, rows, Dh)
-        if not (Dh in (32, 64, 128) and _covered(first, x) and rows >= (N if num_targets == 0 else context_len + (N if own else 0))
+        if not (Dh in (32, 64, 128) and H * Dh == D and _covered(first, x) and rows >= (N if num_targets == 0 else context_len + (N if own else 0))
                 and (num_targets == 0 or context_len > 0)
                 and all(t.shape == shape and t.dtype == x.dtype and t.device == x.device and t.is_contiguous() and t.data_ptr() % 16 == 0
                         for c in caches for t in c)
