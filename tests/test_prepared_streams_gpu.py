@@ -68,8 +68,9 @@ def test_dropped_weights_stay_while_another_stream_reads_them(device, dtype):
     want = _decoder(m)(*run)
     decoder = _decoder(m)
     decoder(*run)
-    # (weights and vectors only: nothing that holds addresses)
-    sizes = [t.nbytes for t in decoder._prepared.tensors if t.nbytes >= 1 << 14]
+    # (weights and vectors only: the table of addresses stays)
+    table = decoder._kv
+    sizes = [t.nbytes for t in decoder._prepared.tensors if t.nbytes >= 1 << 12]
     assert len(sizes) >= 2
     torch.cuda.synchronize()
     b = torch.cuda.Stream()
@@ -79,7 +80,7 @@ def test_dropped_weights_stay_while_another_stream_reads_them(device, dtype):
     del decoder
     others = [torch.full((n,), 255, device=device, dtype=torch.uint8) for n in sizes for _ in range(3)]
     torch.cuda.synchronize()
-    assert torch.equal(got, want) and others
+    assert torch.equal(got, want) and others and table
 
 
 @DTYPES
