@@ -423,7 +423,10 @@ class TrajectoryDecoder:
         tape = torch.empty(lib.artab_trajectory_tape_bytes(D, F_, L, code), device=dev, dtype=torch.uint8)
 
         def pack(w, which, layer=0, rows=0):
-            w = w.detach().contiguous() if w is not None else None
+            if w is not None:
+                w = w.detach().contiguous()
+                if w.data_ptr() % 16:  # (a view into a vector of all parameters)
+                    w = w.clone()
             _lib.check(lib.artab_trajectory_pack(_ptr(tape), _ptr(w), which, layer, rows, D, F_, L, code, stream))
 
         vecs = torch.zeros((L, 8, max(D, F_)), device=dev, dtype=dt)
