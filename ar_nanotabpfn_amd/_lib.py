@@ -398,8 +398,13 @@ def ref(v: Optional[ArtabView]):
     return ctypes.byref(v) if v is not None else None
 
 
+def raw_stream(device: torch.device) -> int:
+    """The current stream's handle (a ``torch.cuda.Stream`` object costs 4 us more; a model's first call asks some 80 times)."""
+    return torch._C._cuda_getCurrentRawStream(device.index if device.index is not None else torch.cuda.current_device())
+
+
 def current_stream(device: torch.device) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    return ctypes.c_void_p(raw_stream(device))
 
 
 def check(status: int) -> None:

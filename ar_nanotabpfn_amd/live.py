@@ -12,6 +12,8 @@ from operator import attrgetter, is_
 import torch
 from torch import nn
 
+from ._lib import raw_stream
+
 __all__ = ["Methods", "ModelState", "Prepared", "Sources", "plain_modules", "walk"]
 
 _hooks_of = attrgetter("_forward_hooks", "_forward_pre_hooks", "_backward_hooks", "_backward_pre_hooks")
@@ -77,11 +79,6 @@ def capturing(device) -> bool:
     return device.type == "cuda" and torch.cuda.is_current_stream_capturing()
 
 
-def _current_stream(device) -> int:
-    """The current stream's handle (a ``torch.cuda.Stream`` object costs 3 us; a first call asks some 50 times)."""
-    return torch._C._cuda_getCurrentRawStream(device.index if device.index is not None else torch.cuda.current_device())
-
-
 class Prepared:
     """Tensors that are made once, on the current stream, and read by calls on any: ``use()`` in front of every call
     on the current stream orders it behind the making, and keeps the memory from being given away under it
@@ -91,12 +88,12 @@ class Prepared:
         self.tensors = tuple(tensors)
         self._device = next((t.device for t in self.tensors if t.is_cuda), None)
         if self._device is not None:
-            self._home = _current_stream(self._device)
+            self._home = raw_stream(self._device)
             self._streams = {self._home}
 
     def use(self) -> tuple:
         # (a recording cannot wait for what lies outside of it; it begins with everything in front of it done)
-        if (self._device is not None and _current_stream(self._device) not in self._streams
+        if (self._device is not None and raw_stream(self._device) not in self._streams
                 and not torch.cuda.is_current_stream_capturing()):
             stream = torch.cuda.current_stream(self._device)
             # behind what the making stream has been given so far: no event has to be kept for calls that stay on it
