@@ -7,7 +7,8 @@
 // pays 30-40 us per layer for them whatever the size of the problem; here a layer costs what one
 // compute unit needs to stream its weights and keys through (64 B per clock from the L2) plus ten
 // workgroup barriers and the latency chains between them.  The rule for when the launches of the
-// other route, which spread one layer over the whole chip, are faster is artab_trajectory_group_layers().
+// other route, which spread one layer over the whole chip, are faster is artab_trajectory_group_layers().  One
+// trajectory per workgroup on a context that is not long: trajectory_crews.h.
 //
 // Rows.  A workgroup owns G trajectories; token row 2 g is trajectory g's buffer row of the step (the
 // value drawn last), row 2 g + 1 its target row: at most 16 rows (16-bit types) or 4 (float32, whose
@@ -159,7 +160,8 @@ struct TrajShape {
     static constexpr int KD = D / TrajOps<T>::kStep, KF = F / TrajOps<T>::kStep;  // contraction steps
     static constexpr int ND = D / 16 / NW, NF = F / 16 / NW;                      // 16-feature blocks per wavefront
     static constexpr int kFo = ND * KD, kQkv = 3 * ND * KD, kO = ND * KD, k1 = NF * KD, k2 = ND * KF;
-    static constexpr int kLayer = kFo + kQkv + kO + k1 + k2;
+    static constexpr int pFo = 0, pQkv = kFo, pO = pQkv + kQkv, p1 = pO + kO, p2 = p1 + k1;  // in a layer's part of the tape
+    static constexpr int kLayer = p2 + k2;
     static constexpr int ring() {
         for (int r = 16; r > 1; --r)
             if (kLayer % r == 0) return r;

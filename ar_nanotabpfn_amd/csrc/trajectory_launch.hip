@@ -1,6 +1,7 @@
 // Launches of the whole-run decode kernel (trajectory_decode.h), one object per element type:
 // -DARTAB_TRAJ_TYPE=0 (bf16, with the type-dispatching entry points) | 1 (f16) | 2 (float32).
 #include "launchers.h"
+#include "trajectory_crews.h"
 
 #ifndef ARTAB_TRAJ_TYPE
 #error "define ARTAB_TRAJ_TYPE (0, 1 or 2)"
@@ -77,6 +78,13 @@ hipError_t decode(const TrajectoryParams &P, int D, int F, hipStream_t st) {
     hipError_t e = hipErrorInvalidValue;
     with_shape<T>(D, F, [&](auto d, auto f) {
         const dim3 grid(static_cast<unsigned>((P.B + P.G - 1) / P.G)), block(kTrajWaves * 64);
+        if constexpr (decltype(d)::value <= 256) {
+            if (crews_serve(P, D, sizeof(T) == 4)) {
+                hipLaunchKernelGGL((trajectory_crews_kernel<T, decltype(d)::value, decltype(f)::value>), grid, dim3(2 * kTrajWaves * 64), 0, st, P);
+                e = hipGetLastError();
+                return;
+            }
+        }
         if (P.G > 1)
             hipLaunchKernelGGL((trajectory_decode_kernel<T, decltype(d)::value, decltype(f)::value, true>), grid, block, 0, st, P);
         else
