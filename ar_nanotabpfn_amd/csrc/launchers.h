@@ -34,7 +34,7 @@ enum Tune : int {
     kTuneLean,            // ARTAB_LEAN: 0 selects the software-pipelined pass at head_dim 32
     kTuneLeanOcc,         // ARTAB_LEAN_OCC: 4 gives the lean pass 128 registers
     kTuneNW,              // ARTAB_NW: 2 = two wavefronts of two query blocks for 128-row tiles
-    kTuneTileRows,        // ARTAB_TILE_ROWS: token rows per workgroup of the layer kernels (16/32)
+    kTuneTileRows,        // ARTAB_TILE_ROWS: layer kernels with 16 or 32 token rows per workgroup; 33, 64: layer_wide.h's with 32, 64
     kTuneLayerFetchers,   // ARTAB_LAYER_FETCHERS: weight-fetching workgroups per XCD of a layer-boundary launch (0..32)
     kTuneTrajectory,      // ARTAB_TRAJECTORY: 0 keeps sampling runs off the whole-run kernel, 1..8 trajectories per workgroup
     kTuneCount

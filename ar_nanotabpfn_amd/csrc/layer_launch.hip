@@ -2,6 +2,7 @@
 // group: -DARTAB_LAYER_BF16=0|1 and -DARTAB_LAYER_GROUP=0 (pre, post) | 1 (post+pre) | 2 (step tail) | 3 (step boundary);
 // the type-dispatching entry points live in the bf16 object of each group.
 #include "launchers.h"
+#include "layer_wide.h"
 
 #ifndef ARTAB_LAYER_BF16
 #error "define ARTAB_LAYER_BF16 (0 or 1) and ARTAB_LAYER_GROUP (0 .. 3)"
@@ -27,8 +28,48 @@ hipError_t launch_pre_r(const FusedPreParams &P, int D, hipStream_t st) {
     }
     return hipGetLastError();
 }
+// Runs f with the row blocks per workgroup of layer_wide.h's kernels for `rows` token rows as a compile-time number;
+// false: the kernels of fused_layer.h.
+template <int D, typename Fn>
+bool with_wide(long rows, Fn f) {
+    const int v = tune(kTuneTileRows, 0);
+    int blocks = v == kFusedRows || v == kFusedRowsSmall ? 0 : v == 33 ? 1 : v == 64 ? 2 : wide_blocks(D, rows);
+    if (D != 256 && blocks) blocks = 1;  // (two blocks lose at d_model 128 up to 50000 rows, and do not fit twice at 512)
+    if (blocks == 1) f(std::integral_constant<int, 1>{});
+    if constexpr (D == 256) {
+        if (blocks == 2) f(std::integral_constant<int, 2>{});
+    }
+    return blocks > 0;
+}
+template <typename T, int D>
+bool launch_wide_pre(const FusedPreParams &P, hipStream_t st) {
+    return with_wide<D>(P.rows, [&](auto rb) {
+        typedef WideTile<T, D, kWideFeedForward, decltype(rb)::value> W;
+        launch_observed(kLaunchLayer, wide_pre_kernel<T, D, kWideFeedForward, decltype(rb)::value>,
+                        dim3(static_cast<unsigned>((P.rows + W::TR - 1) / W::TR)), dim3(W::NT), 0, st, P);
+    });
+}
+template <typename T, int D>
+bool launch_wide_post(const FusedPostParams &P, int F, hipStream_t st) {
+    return F == kWideFeedForward && !P.part_o && with_wide<D>(P.rows, [&](auto rb) {
+        typedef WideTile<T, D, kWideFeedForward, decltype(rb)::value> W;
+        launch_observed(kLaunchLayer, wide_post_kernel<T, D, kWideFeedForward, decltype(rb)::value>,
+                        dim3(static_cast<unsigned>((P.rows + W::TR - 1) / W::TR)), dim3(W::NT), 0, st, P);
+    });
+}
+template <typename T, int D>
+bool launch_wide_post_pre(const FusedPostParams &P, const FusedPreParams &N, int F, hipStream_t st) {
+    return F == kWideFeedForward && !P.part_o && with_wide<D>(P.rows, [&](auto rb) {
+        typedef WideTile<T, D, kWideFeedForward, decltype(rb)::value> W;
+        launch_observed(kLaunchLayer, wide_post_pre_kernel<T, D, kWideFeedForward, decltype(rb)::value>,
+                        dim3(static_cast<unsigned>((P.rows + W::TR - 1) / W::TR)), dim3(W::NT), 0, st, P, N);
+    });
+}
+
 template <typename T>
 hipError_t launch_pre(const FusedPreParams &P, int D, hipStream_t st) {
+    if (D == 128 ? launch_wide_pre<T, 128>(P, st) : D == 256 ? launch_wide_pre<T, 256>(P, st) : launch_wide_pre<T, 512>(P, st))
+        return hipGetLastError();
     return fused_tile_rows(P.rows, fused_small_max_rows(D)) == kFusedRowsSmall ? launch_pre_r<T, kFusedRowsSmall>(P, D, st)
                                                       : launch_pre_r<T, kFusedRows>(P, D, st);
 }
@@ -83,6 +124,10 @@ hipError_t launch_post_pre_r(const FusedPostParams &P, const FusedPreParams &N, 
 }
 template <typename T>
 hipError_t launch_post_pre(const FusedPostParams &P, const FusedPreParams &N, int D, int F, hipStream_t st) {
+    if (D == 128   ? launch_wide_post_pre<T, 128>(P, N, F, st)
+        : D == 256 ? launch_wide_post_pre<T, 256>(P, N, F, st)
+                   : launch_wide_post_pre<T, 512>(P, N, F, st))
+        return hipGetLastError();
     return fused_tile_rows(P.rows, fused_small_max_rows(D)) == kFusedRowsSmall ? launch_post_pre_r<T, kFusedRowsSmall>(P, N, D, F, st)
                                                       : launch_post_pre_r<T, kFusedRows>(P, N, D, F, st);
 }
@@ -97,6 +142,10 @@ hipError_t launch_post_r(const FusedPostParams &P, int D, int F, hipStream_t st)
 }
 template <typename T>
 hipError_t launch_post(const FusedPostParams &P, int D, int F, hipStream_t st) {
+    if (D == 128   ? launch_wide_post<T, 128>(P, F, st)
+        : D == 256 ? launch_wide_post<T, 256>(P, F, st)
+                   : launch_wide_post<T, 512>(P, F, st))
+        return hipGetLastError();
     return fused_tile_rows(P.rows, fused_small_max_rows(D)) == kFusedRowsSmall ? launch_post_r<T, kFusedRowsSmall>(P, D, F, st)
                                                       : launch_post_r<T, kFusedRows>(P, D, F, st);
 }
