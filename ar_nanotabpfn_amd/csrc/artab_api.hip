@@ -1462,16 +1462,22 @@ static int check_layer_dtype_rows(const char *what, int dtype, int64_t rows) {
     return ARTAB_OK;
 }
 
-int artab_layer_pre(const void *x, int64_t ldx, const void *w_fo, const void *ln1_gamma, const void *ln1_beta,
-                    float eps1, const void *w_qkv, void *y, void *qkv, int64_t rows, int D, int dtype,
-                    void *stream) {
+static int layer_pre_impl(const KeyValueRows &kv, const void *x, int64_t ldx, const void *w_fo, const void *ln1_gamma,
+                          const void *ln1_beta, float eps1, const void *w_qkv, void *y, void *qkv, int64_t rows, int D, int dtype,
+                          void *stream) {
     ARTAB_TRY(check_layer_dtype_rows("layer_pre", dtype, rows));
     FusedPreParams P{};
     ARTAB_TRY(fill_pre(P, x, ldx, w_fo, ln1_gamma, ln1_beta, eps1, w_qkv, y, qkv, rows, D, true));
     if (rows == 0) return ARTAB_OK;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    hipError_t e = launch_layer_pre(P, D, dtype == ARTAB_BF16, st);
+    hipError_t e = launch_layer_pre(P, kv, D, dtype == ARTAB_BF16, st);
     return launch_status(e, "layer_pre");
+}
+
+int artab_layer_pre(const void *x, int64_t ldx, const void *w_fo, const void *ln1_gamma, const void *ln1_beta,
+                    float eps1, const void *w_qkv, void *y, void *qkv, int64_t rows, int D, int dtype,
+                    void *stream) {
+    return layer_pre_impl(KeyValueRows{}, x, ldx, w_fo, ln1_gamma, ln1_beta, eps1, w_qkv, y, qkv, rows, D, dtype, stream);
 }
 
 int artab_layer_post(const void *attn, int64_t lda, const void *y, int64_t ldy, const void *w_o,
@@ -1488,7 +1494,7 @@ int artab_layer_post(const void *attn, int64_t lda, const void *y, int64_t ldy, 
     return launch_status(e, "layer_post");
 }
 
-static int layer_post_pre_impl(const artab_attention_partials *parts, const void *attn, int64_t lda, const void *y,
+static int layer_post_pre_impl(const KeyValueRows &kv, const artab_attention_partials *parts, const void *attn, int64_t lda, const void *y,
                                int64_t ldy, const void *w_o, const void *ln2_gamma, const void *ln2_beta, float eps2,
                                const void *w_1, const void *b_1, const void *w_2, const void *b_2,
                                const void *ln3_gamma, const void *ln3_beta, float eps3, const void *next_w_fo,
@@ -1505,7 +1511,7 @@ static int layer_post_pre_impl(const artab_attention_partials *parts, const void
     hipStream_t st = static_cast<hipStream_t>(stream);
     ARTAB_TRY(apply_partials_order(parts, P, rows, D, st));
     if (rows == 0) return ARTAB_OK;
-    hipError_t e = launch_layer_post_pre(P, N, D, F, dtype == ARTAB_BF16, st);
+    hipError_t e = launch_layer_post_pre(P, N, kv, D, F, dtype == ARTAB_BF16, st);
     return launch_status(e, "layer_post_pre");
 }
 
@@ -1515,7 +1521,7 @@ int artab_layer_post_pre(const void *attn, int64_t lda, const void *y, int64_t l
                          const void *next_w_fo, const void *next_ln1_gamma, const void *next_ln1_beta,
                          float next_eps1, const void *next_w_qkv, void *next_y, void *next_qkv, int64_t rows, int D,
                          int F, int dtype, void *stream) {
-    return layer_post_pre_impl(nullptr, attn, lda, y, ldy, w_o, ln2_gamma, ln2_beta, eps2, w_1, b_1, w_2, b_2,
+    return layer_post_pre_impl(KeyValueRows{}, nullptr, attn, lda, y, ldy, w_o, ln2_gamma, ln2_beta, eps2, w_1, b_1, w_2, b_2,
                                ln3_gamma, ln3_beta, eps3, next_w_fo, next_ln1_gamma, next_ln1_beta, next_eps1,
                                next_w_qkv, next_y, next_qkv, rows, D, F, dtype, stream);
 }
@@ -1529,7 +1535,7 @@ int artab_layer_post_pre_from_partials(const artab_attention_partials *parts, co
                                        void *next_y, void *next_qkv, int64_t rows, int D, int F, int dtype,
                                        void *stream) {
     if (!parts) return fail(ARTAB_ERR_NULL_POINTER, "partials descriptor is NULL");
-    return layer_post_pre_impl(parts, nullptr, 0, y, ldy, w_o, ln2_gamma, ln2_beta, eps2, w_1, b_1, w_2, b_2,
+    return layer_post_pre_impl(KeyValueRows{}, parts, nullptr, 0, y, ldy, w_o, ln2_gamma, ln2_beta, eps2, w_1, b_1, w_2, b_2,
                                ln3_gamma, ln3_beta, eps3, next_w_fo, next_ln1_gamma, next_ln1_beta, next_eps1,
                                next_w_qkv, next_y, next_qkv, rows, D, F, dtype, stream);
 }
@@ -1739,17 +1745,36 @@ int artab_layer_stack(const artab_stack_args *a, int dtype, void *stream) {
     const artab_view q = head_view(0), k = head_view(1), v = head_view(2), out = {attn, a->N * D, Dh, D};
     const int64_t cache_h = static_cast<int64_t>(a->cache_rows) * Dh, cache_b = a->own_caches ? a->H * cache_h : 0;
     const artab_stack_layer *L = a->layers;
+    // Where the layer kernels can, they put keys and values where they belong, and the attention reads them there: no copy
+    // of them, and rows of a head that follow each other (in the q/k/v matrix a head's 64 bytes share a line with its
+    // neighbour's).  A prefill of several entries with one cache keeps entry 0's and cannot.
+    const bool direct = !f32 && (a->own_caches || (a->num_targets == 0 && a->B == 1)) && rows <= 0x7fffffffL &&
+                        layer_takes_key_value_rows(rows, a->D, a->F);
+    const size_t behind = a->num_targets ? static_cast<size_t>(a->Nc) * Dh * e : 0;
+    const auto rows_of = [&](const artab_stack_layer &n) {
+        if (!direct) return KeyValueRows{};
+        return KeyValueRows{static_cast<char *>(n.k_cache) + behind, static_cast<char *>(n.v_cache) + behind, cache_b, cache_h, a->N, Dh};
+    };
     if (f32) {
         F32LayerParams P{};
         P.x = static_cast<const float *>(a->x);
         ARTAB_TRY(launch_status(launch_f32_layer(f32_head(P, *L, base + s.y[0], qkv, rows), a->D, static_cast<hipStream_t>(stream)), "layer (float32)"));
     } else {
-        ARTAB_TRY(artab_layer_pre(a->x, D, L->w_fo, L->gamma1, L->beta1, L->eps1, L->w_qkv, base + s.y[0], qkv, rows, a->D, dtype,
-                                  stream));
+        ARTAB_TRY(layer_pre_impl(rows_of(*L), a->x, D, L->w_fo, L->gamma1, L->beta1, L->eps1, L->w_qkv, base + s.y[0], qkv, rows, a->D,
+                                 dtype, stream));
     }
     for (int l = 0; l < a->n_layers; ++l, ++L) {
         const artab_view kc = {L->k_cache, cache_b, cache_h, Dh}, vc = {L->v_cache, cache_b, cache_h, Dh};
-        if (a->num_targets == 0) {
+        if (direct) {
+            const KeyValueRows r = rows_of(*L);
+            const artab_view kd = {r.k, cache_b, cache_h, Dh}, vd = {r.v, cache_b, cache_h, Dh};
+            if (a->num_targets == 0)
+                ARTAB_TRY(artab_prefill_attention_sliced(&q, &kd, &vd, &out, nullptr, nullptr, 0, a->B, a->H, a->N, Dh, 0.f, dtype,
+                                                         base + s.prefill, s.total - s.prefill, ARTAB_IMPL_AUTO, stream));
+            else
+                ARTAB_TRY(artab_teacher_forcing_attention(&q, &kc, &vc, &kd, &vd, &out, nullptr, a->B, a->H, a->num_targets, a->Nc, Dh,
+                                                          0.f, dtype, ARTAB_IMPL_AUTO, stream));
+        } else if (a->num_targets == 0) {
             ARTAB_TRY(artab_prefill_attention_sliced(&q, &k, &v, &out, &kc, &vc, a->own_caches ? a->B : 1, a->B, a->H, a->N, Dh, 0.f,
                                                      dtype, base + s.prefill, s.total - s.prefill, ARTAB_IMPL_AUTO, stream));
         } else {
@@ -1778,9 +1803,9 @@ int artab_layer_stack(const artab_stack_args *a, int dtype, void *stream) {
             return artab_layer_post(attn, D, y, D, L->w_o, L->gamma2, L->beta2, L->eps2, L->w_1, L->b_1, L->w_2, L->b_2, L->gamma3,
                                     L->beta3, L->eps3, a->out, rows, a->D, a->F, dtype, stream);
         const artab_stack_layer *n = L + 1;
-        ARTAB_TRY(artab_layer_post_pre(attn, D, y, D, L->w_o, L->gamma2, L->beta2, L->eps2, L->w_1, L->b_1, L->w_2, L->b_2, L->gamma3,
-                                       L->beta3, L->eps3, n->w_fo, n->gamma1, n->beta1, n->eps1, n->w_qkv, base + s.y[1 - (l & 1)], qkv,
-                                       rows, a->D, a->F, dtype, stream));
+        ARTAB_TRY(layer_post_pre_impl(rows_of(*n), nullptr, attn, D, y, D, L->w_o, L->gamma2, L->beta2, L->eps2, L->w_1, L->b_1, L->w_2,
+                                      L->b_2, L->gamma3, L->beta3, L->eps3, n->w_fo, n->gamma1, n->beta1, n->eps1, n->w_qkv,
+                                      base + s.y[1 - (l & 1)], qkv, rows, a->D, a->F, dtype, stream));
     }
     return ARTAB_OK;
 }

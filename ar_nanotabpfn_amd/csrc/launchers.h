@@ -10,6 +10,7 @@
 
 #include "attention_backward.h"
 #include "fused_layer.h"
+#include "layer_wide.h"
 #include "mfma_flash.h"
 #include "trajectory_decode.h"
 
@@ -105,10 +106,12 @@ enum BackwardElem : int { kElemF32 = 0, kElemBf16 = 1, kElemF16 = 2 };
 hipError_t launch_row_mask_backward(const BackwardParams &P, int elem, bool use_mfma, hipStream_t stream);
 
 // layer_launch.hip (one object per element type and kernel group)
-hipError_t launch_layer_pre(const FusedPreParams &P, int D, bool is_bf16, hipStream_t st);
+// kv.k set: the keys and values go there and not into the q/k/v matrix, where layer_takes_key_value_rows()
+bool layer_takes_key_value_rows(long rows, int D, int F);
+hipError_t launch_layer_pre(const FusedPreParams &P, const KeyValueRows &kv, int D, bool is_bf16, hipStream_t st);
 hipError_t launch_layer_post(const FusedPostParams &P, int D, int F, bool is_bf16, hipStream_t st);
-hipError_t launch_layer_post_pre(const FusedPostParams &P, const FusedPreParams &N, int D, int F, bool is_bf16,
-                                 hipStream_t st);
+hipError_t launch_layer_post_pre(const FusedPostParams &P, const FusedPreParams &N, const KeyValueRows &kv, int D, int F,
+                                 bool is_bf16, hipStream_t st);
 hipError_t launch_sample_embed(const SampleEmbedParams &P, int D, int F, bool is_bf16, hipStream_t st);
 hipError_t launch_step_boundary(const FusedPostParams &P, const SampleEmbedParams &S, const FusedPreParams &N, int D,
                                 int F, bool is_bf16, hipStream_t st);

@@ -2,7 +2,6 @@
 // group: -DARTAB_LAYER_BF16=0|1 and -DARTAB_LAYER_GROUP=0 (pre, post) | 1 (post+pre) | 2 (step tail) | 3 (step boundary);
 // the type-dispatching entry points live in the bf16 object of each group.
 #include "launchers.h"
-#include "layer_wide.h"
 
 #ifndef ARTAB_LAYER_BF16
 #error "define ARTAB_LAYER_BF16 (0 or 1) and ARTAB_LAYER_GROUP (0 .. 3)"
@@ -42,11 +41,11 @@ bool with_wide(long rows, Fn f) {
     return blocks > 0;
 }
 template <typename T, int D>
-bool launch_wide_pre(const FusedPreParams &P, hipStream_t st) {
+bool launch_wide_pre(const FusedPreParams &P, const KeyValueRows &kv, hipStream_t st) {
     return with_wide<D>(P.rows, [&](auto rb) {
         typedef WideTile<T, D, kWideFeedForward, decltype(rb)::value> W;
         launch_observed(kLaunchLayer, wide_pre_kernel<T, D, kWideFeedForward, decltype(rb)::value>,
-                        dim3(static_cast<unsigned>((P.rows + W::TR - 1) / W::TR)), dim3(W::NT), 0, st, P);
+                        dim3(static_cast<unsigned>((P.rows + W::TR - 1) / W::TR)), dim3(W::NT), 0, st, P, kv);
     });
 }
 template <typename T, int D>
@@ -58,17 +57,17 @@ bool launch_wide_post(const FusedPostParams &P, int F, hipStream_t st) {
     });
 }
 template <typename T, int D>
-bool launch_wide_post_pre(const FusedPostParams &P, const FusedPreParams &N, int F, hipStream_t st) {
+bool launch_wide_post_pre(const FusedPostParams &P, const FusedPreParams &N, const KeyValueRows &kv, int F, hipStream_t st) {
     return F == kWideFeedForward && !P.part_o && with_wide<D>(P.rows, [&](auto rb) {
         typedef WideTile<T, D, kWideFeedForward, decltype(rb)::value> W;
         launch_observed(kLaunchLayer, wide_post_pre_kernel<T, D, kWideFeedForward, decltype(rb)::value>,
-                        dim3(static_cast<unsigned>((P.rows + W::TR - 1) / W::TR)), dim3(W::NT), 0, st, P, N);
+                        dim3(static_cast<unsigned>((P.rows + W::TR - 1) / W::TR)), dim3(W::NT), 0, st, P, N, kv);
     });
 }
 
 template <typename T>
-hipError_t launch_pre(const FusedPreParams &P, int D, hipStream_t st) {
-    if (D == 128 ? launch_wide_pre<T, 128>(P, st) : D == 256 ? launch_wide_pre<T, 256>(P, st) : launch_wide_pre<T, 512>(P, st))
+hipError_t launch_pre(const FusedPreParams &P, const KeyValueRows &kv, int D, hipStream_t st) {
+    if (D == 128 ? launch_wide_pre<T, 128>(P, kv, st) : D == 256 ? launch_wide_pre<T, 256>(P, kv, st) : launch_wide_pre<T, 512>(P, kv, st))
         return hipGetLastError();
     return fused_tile_rows(P.rows, fused_small_max_rows(D)) == kFusedRowsSmall ? launch_pre_r<T, kFusedRowsSmall>(P, D, st)
                                                       : launch_pre_r<T, kFusedRows>(P, D, st);
@@ -123,10 +122,10 @@ hipError_t launch_post_pre_r(const FusedPostParams &P, const FusedPreParams &N, 
     }
 }
 template <typename T>
-hipError_t launch_post_pre(const FusedPostParams &P, const FusedPreParams &N, int D, int F, hipStream_t st) {
-    if (D == 128   ? launch_wide_post_pre<T, 128>(P, N, F, st)
-        : D == 256 ? launch_wide_post_pre<T, 256>(P, N, F, st)
-                   : launch_wide_post_pre<T, 512>(P, N, F, st))
+hipError_t launch_post_pre(const FusedPostParams &P, const FusedPreParams &N, const KeyValueRows &kv, int D, int F, hipStream_t st) {
+    if (D == 128   ? launch_wide_post_pre<T, 128>(P, N, kv, F, st)
+        : D == 256 ? launch_wide_post_pre<T, 256>(P, N, kv, F, st)
+                   : launch_wide_post_pre<T, 512>(P, N, kv, F, st))
         return hipGetLastError();
     return fused_tile_rows(P.rows, fused_small_max_rows(D)) == kFusedRowsSmall ? launch_post_pre_r<T, kFusedRowsSmall>(P, N, D, F, st)
                                                       : launch_post_pre_r<T, kFusedRows>(P, N, D, F, st);
@@ -202,34 +201,44 @@ hipError_t launch_boundary(const FusedPostParams &P, const SampleEmbedParams &S,
 // fp16 forms, defined in the fp16 objects
 hipError_t launch_step_boundary_f16(const FusedPostParams &P, const SampleEmbedParams &S, const FusedPreParams &N,
                                     int D, int F, hipStream_t st);
-hipError_t launch_layer_pre_f16(const FusedPreParams &P, int D, hipStream_t st);
+hipError_t launch_layer_pre_f16(const FusedPreParams &P, const KeyValueRows &kv, int D, hipStream_t st);
 hipError_t launch_layer_post_f16(const FusedPostParams &P, int D, int F, hipStream_t st);
-hipError_t launch_layer_post_pre_f16(const FusedPostParams &P, const FusedPreParams &N, int D, int F, hipStream_t st);
+hipError_t launch_layer_post_pre_f16(const FusedPostParams &P, const FusedPreParams &N, const KeyValueRows &kv, int D, int F,
+                                     hipStream_t st);
 hipError_t launch_sample_embed_f16(const SampleEmbedParams &P, int D, int F, hipStream_t st);
 
 #if ARTAB_LAYER_GROUP == 0
 #if ARTAB_LAYER_BF16
-hipError_t launch_layer_pre(const FusedPreParams &P, int D, bool is_bf16, hipStream_t st) {
-    return is_bf16 ? launch_pre<LayerT>(P, D, st) : launch_layer_pre_f16(P, D, st);
+hipError_t launch_layer_pre(const FusedPreParams &P, const KeyValueRows &kv, int D, bool is_bf16, hipStream_t st) {
+    return is_bf16 ? launch_pre<LayerT>(P, kv, D, st) : launch_layer_pre_f16(P, kv, D, st);
+}
+bool layer_takes_key_value_rows(long rows, int D, int F) {
+    return F == kWideFeedForward && (D == 128   ? with_wide<128>(rows, [](auto) {})
+                                     : D == 256 ? with_wide<256>(rows, [](auto) {})
+                                     : D == 512 ? with_wide<512>(rows, [](auto) {})
+                                                : false);
 }
 hipError_t launch_layer_post(const FusedPostParams &P, int D, int F, bool is_bf16, hipStream_t st) {
     return is_bf16 ? launch_post<LayerT>(P, D, F, st) : launch_layer_post_f16(P, D, F, st);
 }
 #else
-hipError_t launch_layer_pre_f16(const FusedPreParams &P, int D, hipStream_t st) { return launch_pre<LayerT>(P, D, st); }
+hipError_t launch_layer_pre_f16(const FusedPreParams &P, const KeyValueRows &kv, int D, hipStream_t st) {
+    return launch_pre<LayerT>(P, kv, D, st);
+}
 hipError_t launch_layer_post_f16(const FusedPostParams &P, int D, int F, hipStream_t st) {
     return launch_post<LayerT>(P, D, F, st);
 }
 #endif
 #elif ARTAB_LAYER_GROUP == 1
 #if ARTAB_LAYER_BF16
-hipError_t launch_layer_post_pre(const FusedPostParams &P, const FusedPreParams &N, int D, int F, bool is_bf16,
-                                 hipStream_t st) {
-    return is_bf16 ? launch_post_pre<LayerT>(P, N, D, F, st) : launch_layer_post_pre_f16(P, N, D, F, st);
+hipError_t launch_layer_post_pre(const FusedPostParams &P, const FusedPreParams &N, const KeyValueRows &kv, int D, int F,
+                                 bool is_bf16, hipStream_t st) {
+    return is_bf16 ? launch_post_pre<LayerT>(P, N, kv, D, F, st) : launch_layer_post_pre_f16(P, N, kv, D, F, st);
 }
 #else
-hipError_t launch_layer_post_pre_f16(const FusedPostParams &P, const FusedPreParams &N, int D, int F, hipStream_t st) {
-    return launch_post_pre<LayerT>(P, N, D, F, st);
+hipError_t launch_layer_post_pre_f16(const FusedPostParams &P, const FusedPreParams &N, const KeyValueRows &kv, int D, int F,
+                                     hipStream_t st) {
+    return launch_post_pre<LayerT>(P, N, kv, D, F, st);
 }
 #endif
 #elif ARTAB_LAYER_GROUP == 3

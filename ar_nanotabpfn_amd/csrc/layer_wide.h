@@ -30,6 +30,14 @@ constexpr int wide_blocks(int D, long rows) { return rows <= 8192 ? 0 : D == 256
 constexpr int kWideRing = 8;
 constexpr int kWideFeedForward = 256;  // the feed-forward width these are built for (others: fused_layer.h)
 
+// Where the projected keys and values go instead of the q/k/v matrix: row r of the launch is row r % N of batch entry
+// r / N, head h starts h * sh elements into its entry.
+struct KeyValueRows {
+    void *k, *v;  // null: the matrix
+    long sb, sh;  // elements
+    int N, Dh;    // head_dim: 32, 64 or 128, rows of a head contiguous
+};
+
 __device__ __forceinline__ float wide_over_token(float x) {  // the lanes that hold the same token: l and l ^ 32
     const unsigned a = __builtin_bit_cast(unsigned, x);
     auto s = __builtin_amdgcn_permlane32_swap(a, a, false, false);
@@ -198,8 +206,10 @@ struct WideTile {
             }
         __syncthreads();
     }
-    // The wavefront's columns of a tile in registers to memory, through its own columns of `tile` (row stride LDD).
-    __device__ __forceinline__ void store_columns(const f32x16 (&acc)[NBD][RB], T *tile, T *dst, long ld, int valid) {
+    // The wavefront's columns of a tile in registers to memory, through its own columns of `tile` (row stride LDD):
+    // `at(row)` is where the tile's row begins, `head(col0)` how much further 32 columns from col0 on do.
+    template <typename Row, typename Head>
+    __device__ __forceinline__ void store_columns(const f32x16 (&acc)[NBD][RB], T *tile, int valid, Row at, Head head) {
 #pragma unroll
         for (int b = 0; b < NBD; ++b) {
             const int col0 = 32 * (wave + NW * b);
@@ -214,7 +224,7 @@ struct WideTile {
             for (int i = 0; i < TR / 16; ++i) {  // 16 rows of 64 bytes at a time
                 const int row = 16 * i + (lane >> 2), col = col0 + 8 * (lane & 3);
                 const u32x4 v = *reinterpret_cast<const u32x4 *>(tile + row * LDD + col);
-                if (row < valid) *reinterpret_cast<u32x4 *>(dst + static_cast<long>(row) * ld + col) = v;
+                if (row < valid) *reinterpret_cast<u32x4 *>(at(row) + head(col0) + 8 * (lane & 3)) = v;
             }
             __builtin_amdgcn_wave_barrier();
         }
@@ -239,7 +249,7 @@ struct WideTile {
         norm(acc, a1, vecs + kVecBias2 * VW, vecs + kVecG3 * VW, vecs + kVecB3 * VW, a0, P.eps3);
     }
     // y = LN1(x + x W_fo^T) and q, k, v = y W^T from the tile in a0.  The ring holds W_fo's first fragments.
-    __device__ __forceinline__ void pre(const FusedPreParams &P, long row0, int valid) {
+    __device__ __forceinline__ void pre(const FusedPreParams &P, const KeyValueRows &kv, long row0, int valid) {
         const T *w_fo = static_cast<const T *>(P.w_fo), *w_qkv = static_cast<const T *>(P.w_qkv);
         f32x16 acc[NBD][RB];
         product<D, NBD, D, NBD>(acc, w_fo, a0, LDD, w_qkv);
@@ -249,7 +259,20 @@ struct WideTile {
         for (int p = 0; p < 3; ++p) {
             const T *w = w_qkv + static_cast<long>(p) * D * D;
             product<D, NBD, D, NBD>(acc, w, a1, LDD, p < 2 ? w + static_cast<long>(D) * D : nullptr);
-            store_columns(acc, a0, static_cast<T *>(P.qkv) + row0 * (3 * D) + p * D, 3 * D, valid);
+            if (p == 0 || !kv.k) {
+                T *const dst = static_cast<T *>(P.qkv) + row0 * (3 * D) + p * D;
+                store_columns(acc, a0, valid, [&](int row) { return dst + row * (3L * D); }, [](int col0) { return col0; });
+            } else {
+                T *const dst = static_cast<T *>(p == 1 ? kv.k : kv.v);
+                const unsigned first = static_cast<unsigned>(row0), n_rows = static_cast<unsigned>(kv.N);
+                store_columns(
+                    acc, a0, valid,
+                    [&](int row) {
+                        const unsigned r = first + row, entry = r / n_rows;
+                        return dst + entry * kv.sb + static_cast<long>(r - entry * n_rows) * kv.Dh;
+                    },
+                    [&](int col0) { return col0 / kv.Dh * kv.sh + col0 % kv.Dh; });
+            }
         }
     }
 };
@@ -269,7 +292,7 @@ __device__ __forceinline__ void wide_stage_post(WideTile<T, D, F, RB> &tile, con
 }
 
 template <typename T, int D, int F, int RB>
-__global__ __launch_bounds__(fused_waves(D) * 64, 4) void wide_pre_kernel(FusedPreParams P) {
+__global__ __launch_bounds__(fused_waves(D) * 64, 4) void wide_pre_kernel(FusedPreParams P, KeyValueRows kv) {
     typedef WideTile<T, D, F, RB> W;
     __shared__ __attribute__((aligned(16))) unsigned char lds[W::kLds];
     W tile(lds);
@@ -280,7 +303,7 @@ __global__ __launch_bounds__(fused_waves(D) * 64, 4) void wide_pre_kernel(FusedP
     stage_pre_vectors<T, D, W::NT>(P, tile.vecs, W::VW, threadIdx.x);
     wait_all_loads();
     __syncthreads();
-    tile.pre(P, row0, valid);
+    tile.pre(P, kv, row0, valid);
 }
 
 template <typename T, int D, int F, int RB>
@@ -299,7 +322,7 @@ __global__ __launch_bounds__(fused_waves(D) * 64, 4) void wide_post_kernel(Fused
 }
 
 template <typename T, int D, int F, int RB>
-__global__ __launch_bounds__(fused_waves(D) * 64, 4) void wide_post_pre_kernel(FusedPostParams P, FusedPreParams N) {
+__global__ __launch_bounds__(fused_waves(D) * 64, 4) void wide_post_pre_kernel(FusedPostParams P, FusedPreParams N, KeyValueRows kv) {
     typedef WideTile<T, D, F, RB> W;
     __shared__ __attribute__((aligned(16))) unsigned char lds[W::kLds];
     W tile(lds);
@@ -311,7 +334,7 @@ __global__ __launch_bounds__(fused_waves(D) * 64, 4) void wide_post_pre_kernel(F
     wait_all_loads();
     __syncthreads();
     tile.post(P, static_cast<const T *>(N.w_fo));
-    tile.pre(N, row0, valid);
+    tile.pre(N, kv, row0, valid);
 }
 
 }  // namespace artab

@@ -85,3 +85,33 @@ def test_rule(device, tuning, rows, tile):
         results[t] = layer_post(attn, y, p_o, n2, p_1, None, p_2, None, n3)
     for t in (16, 32, 33, 64):
         assert torch.equal(results[None], results[t]) == (t == tile)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("backend", ["shared_context", "per_dataset"])
+# batch entries that end inside a tile and inside its 16-row stores; one row per entry; head sizes 32, 64 and 128
+@pytest.mark.parametrize("B,Nc,Nt,D,H,tile", [(1, 77, 5, 128, 4, 33), (3, 17, 5, 256, 8, 64), (5, 33, 1, 256, 4, 33), (2, 65, 31, 512, 4, 33),
+                                              (41, 3, 2, 128, 4, 33)])
+def test_keys_and_values_go_to_the_caches(device, tuning, monkeypatch, dtype, backend, B, Nc, Nt, D, H, tile):
+    """Prefill and teacher forcing as one call, where the layer kernels write keys and values into the caches and the
+    attention reads them there, against the layer-by-layer form, which copies them: the same bits."""
+    from ar_nanotabpfn_amd.inference import ARTabPFNPredictor
+    from ar_nanotabpfn_amd.model import ARTabPFN
+
+    tuning(ARTAB_TILE_ROWS=tile)
+    torch.manual_seed(Nc)
+    model = ARTabPFN(d_model=D, n_heads=H, n_layers=3, d_ff=256, num_features=2).to(device, dtype).eval()
+    g = torch.Generator().manual_seed(Nt)
+    xc, xt = (torch.randn(B, n, 2, generator=g).to(device, dtype) for n in (Nc, Nt))
+    yc, yt = (torch.randn(B, n, generator=g).to(device, dtype) for n in (Nc, Nt))
+    names = ("k_ctx_cache", "v_ctx_cache") if backend == "shared_context" else ("k_cache", "v_cache")
+
+    def run(one_call):
+        p = ARTabPFNPredictor.from_trained_model(model, backend=backend)
+        stack = p._stack_pass
+        monkeypatch.setattr(p, "_stack_pass", lambda *a: stack(*a) if one_call else None)
+        out = p.evaluate_joint_density(xc, yc, xt, yt)
+        return [out] + [getattr(layer, n).clone() for layer in model.backbone.layers for n in names]
+
+    for a, b in zip(run(True), run(False)):
+        assert torch.equal(a, b)
