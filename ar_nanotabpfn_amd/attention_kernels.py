@@ -529,7 +529,7 @@ def row_mask_attention_backward(q: Tensor, k: Tensor, v: Tensor, out: Tensor, do
 
 
 class _RowMaskAttention(torch.autograd.Function):
-    """``row_mask_attention`` with its device backward pass (two launches: dQ, then dK and dV)."""
+    """``row_mask_attention`` with its device backward pass (one launch, or two: dQ, then dK and dV)."""
 
     @staticmethod
     def forward(ctx, q, k, v, context_len, buffer_len, attending_chunks, use_triton):

@@ -1,5 +1,6 @@
 // Launches of the backward kernels of the training row attention (attention_backward.h):
 // template selection by element type and head_dim.
+#include "attention_backward_pair.h"
 #include "launchers.h"
 
 namespace artab {
@@ -22,8 +23,30 @@ static hipError_t launch_backward_portable(const BackwardParams &P, hipStream_t 
     return hipGetLastError();
 }
 
+template <typename T, int DH, int W, int G>
+static hipError_t launch_backward_pair(const BackwardParams &P, hipStream_t stream) {
+    hipLaunchKernelGGL((backward_pair_kernel<T, DH, W, G>), dim3(static_cast<unsigned>(P.H) * P.B), dim3(64 * W * G), 0, stream, P);
+    return hipGetLastError();
+}
+
 template <typename T>
 static hipError_t launch_backward_mfma(const BackwardParams &P, hipStream_t stream) {
+    // One workgroup per pair (backward_pair_kernel) while the keys that anybody sees fit it.  It stays on one compute
+    // unit: with up to 128 keys it is the faster form at any number of pairs (head_dim 32, 96 keys, 608 rows: 22.6 ->
+    // 18.5 us for 4 pairs, 49 -> 24 for 256); with more, the two kernels' many workgroups win while pairs are few (256
+    // keys, 768 rows: 29.8 against 31.9 at 32 pairs, 33.5 at 64, 41.6 against 35.2 at 128; 512 keys, 1024 rows: 52
+    // against 70 at 64, 91 -> 73 at 128, 283 -> 171 at 512; head_dim 64, 256 keys: 46 against 58 at 64, 63 -> 60 at 128).
+    // More pairs than compute units: two workgroups of half the groups to a unit (300 pairs, 96 keys: 53 -> 33).
+    const long pairs = static_cast<long>(P.H) * P.B;
+    const int keys = P.Nc + P.Nb;
+    if (P.Dh == 32) {
+        if (keys <= 128) return pairs <= 256 ? launch_backward_pair<T, 32, 4, 4>(P, stream) : launch_backward_pair<T, 32, 4, 2>(P, stream);
+        if (keys <= 256 && pairs >= 64) return launch_backward_pair<T, 32, 8, 2>(P, stream);
+        if (keys <= 512 && pairs >= 128) return launch_backward_pair<T, 32, 16, 1>(P, stream);
+    } else {
+        if (keys <= 128) return launch_backward_pair<T, 64, 4, 2>(P, stream);
+        if (keys <= 256 && pairs >= 128) return launch_backward_pair<T, 64, 8, 1>(P, stream);
+    }
     const long blocks = (P.R + kBackwardRows - 1) / kBackwardRows;
     const dim3 grid(static_cast<unsigned>(blocks * P.H * P.B)), block(kBackwardWaves * 64);
     if (P.Dh == 32) {

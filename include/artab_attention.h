@@ -362,11 +362,10 @@ int artab_row_mask_attention(const artab_view *q, const artab_view *k, const art
  * (ar_tabpfn/model/attention.py:52-61 under the mask of :86-175; ar_tabpfn/train.py:289-300).
  *   q, k, v, out, dout [B,H,R,Dh]: the forward's inputs, its output and the output's gradient;
  *   lse float32 [B,H,R]: the forward's log-sum-exp;
- *   delta float32 [B,H,R]: workspace (row sums of dout * out; written by the first launch, read by
- *                          the second);
+ *   delta float32 [B,H,R]: workspace (row sums of dout * out, where two launches pass them on);
  *   grad_q, grad_k, grad_v [B,H,R,Dh]: results, every element written (target keys get zeros).
  * With P the masked softmax: grad_v = P^T dout, dS = P o (dout v^T - delta),
- * grad_q = scale dS k, grad_k = scale dS^T q.  Two launches on `stream`, no atomics: the
+ * grad_q = scale dS k, grad_k = scale dS^T q.  One or two launches on `stream`, no atomics: the
  * result does not depend on the schedule.  The matrix-core kernels take bf16 / f16 with head_dim
  * 32 or 64; everything else runs the float32-arithmetic kernels.
  */
