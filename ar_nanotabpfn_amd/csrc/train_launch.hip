@@ -79,10 +79,12 @@ struct GradLayout {
     }
 };
 
-// Workgroups of a backward kernel: about two per compute unit, every one with the same number of tiles.
-int backward_groups(long M) {
-    const long tiles = (M + kTrainRows - 1) / kTrainRows, rounds = (tiles + 511) / 512;
-    return static_cast<int>((tiles + rounds - 1) / rounds);
+// Workgroups of the backward kernel: as many as are resident, three to a compute unit at d_model 128, two at 256.
+// (Of 1216 tiles some then have two, some one; 608 workgroups of two each: 83 us instead of 74, some compute units
+// with six tiles, some with four.)
+int backward_groups(long M, int D) {
+    const long resident = D == 128 ? 768 : 512, tiles = (M + kTrainRows - 1) / kTrainRows;
+    return static_cast<int>(tiles < resident ? tiles : resident);
 }
 int grad_jobs(int D, int F) { return (5 * D * D + 2 * D * F) / (128 * 128); }
 // Row slices of the weight-gradient products: enough that pieces times slices give every compute unit a
@@ -94,21 +96,20 @@ int grad_slices(long M, int jobs) {
 constexpr int kFinalGroups = 512;
 
 struct Scratch {
-    float *dx, *dr2, *delta, *part_w, *part_b, *part_a, *part_f;
+    float *dx, *dr2, *delta, *part_w, *part_c, *part_f;
     bf16_t *d3, *x2, *h, *du, *d2, *dattn, *dqkv, *x1, *d1, *x;
     size_t bytes;
 };
 Scratch scratch_layout(const artab_train_args &a) {
     const size_t M = static_cast<size_t>(a.B) * a.R, D = a.D, F = a.F;
-    const int groups = backward_groups(M), jobs = grad_jobs(a.D, a.F);
+    const int groups = backward_groups(M, a.D), jobs = grad_jobs(a.D, a.F);
     Scratch v;
     Arena s(a.scratch);
     v.dx = s.take<float>(M * D);
     v.dr2 = s.take<float>(M * D);
     v.delta = s.take<float>(M * a.H);
     v.part_w = s.take<float>(static_cast<size_t>(grad_slices(M, jobs)) * jobs * 16384);
-    v.part_b = s.take<float>(groups * (5 * D + F));
-    v.part_a = s.take<float>(groups * 2 * D);
+    v.part_c = s.take<float>(groups * (7 * D + F));
     v.part_f = s.take<float>(kFinalGroups * 2 * D);
     v.d3 = s.take<bf16_t>(M * D);
     v.x2 = s.take<bf16_t>(M * D);
@@ -163,27 +164,33 @@ int forward(const artab_train_args &a, hipStream_t st) {
                            0, st, W, fo, S.packed + l0 * train_packed_elems<D, F>());
     }
     const dim3 grid(static_cast<unsigned>((M + kTrainRows - 1) / kTrainRows)), block(kTrainWaves * 64);
-    for (int l = 0; l < a.n_layers; ++l) {
+    for (int l = 0; l <= a.n_layers; ++l) {  // launch l: behind the attention of layer l - 1, in front of that of layer l
+        TrainForward A{};
+        A.M = M;
+        if (l == 0) {
+            A.x = a.x;
+        } else {
+            const float *const *p = a.params + static_cast<size_t>(l - 1) * kParams;
+            const SavedLayer v = S.layer(a, l - 1);
+            A.attn = v.attn; A.r1 = v.r1; A.stats1 = v.stats1; A.g1 = p[kPG1]; A.b1 = p[kPB1]; A.packed = S.packed + (l - 1) * train_packed_elems<D, F>();
+            A.g2 = p[kPG2]; A.b2 = p[kPB2]; A.bias1 = p[kPBias1]; A.bias2 = p[kPBias2]; A.eps2 = a.eps2; A.eps3 = a.eps3;
+            A.r2 = v.r2; A.stats2 = v.stats2; A.r3 = v.r3; A.stats3 = v.stats3; A.g3 = p[kPG3]; A.b3 = p[kPB3];
+        }
+        if (l == a.n_layers) {
+            hipLaunchKernelGGL((train_forward_kernel<D, F, true, false>), grid, block, 0, st, A);
+            break;
+        }
         const float *const *p = a.params + static_cast<size_t>(l) * kParams;
         const SavedLayer v = S.layer(a, l);
-        const bf16_t *packed = S.packed + l * train_packed_elems<D, F>();
-        TrainForwardA A{};
-        A.r_prev = a.x;
-        if (l > 0) {
-            const SavedLayer b = S.layer(a, l - 1);
-            A.r_prev = b.r3; A.stats_prev = b.stats3; A.g_prev = p[kPG3 - kParams]; A.b_prev = p[kPB3 - kParams];
-        }
-        A.packed = packed; A.g1 = p[kPG1]; A.b1 = p[kPB1]; A.eps1 = a.eps1;
-        A.r1 = v.r1; A.stats1 = v.stats1; A.qkv = v.qkv; A.M = M;
-        hipLaunchKernelGGL((train_forward_a_kernel<D, F>), grid, block, 0, st, A);
+        A.next_packed = S.packed + l * train_packed_elems<D, F>(); A.next_g1 = p[kPG1]; A.next_b1 = p[kPB1]; A.next_eps1 = a.eps1;
+        A.next_r1 = v.r1; A.next_stats1 = v.stats1; A.next_qkv = v.qkv;
+        if (l == 0)
+            hipLaunchKernelGGL((train_forward_kernel<D, F, false, true>), grid, block, 0, st, A);
+        else
+            hipLaunchKernelGGL((train_forward_kernel<D, F, true, true>), grid, block, 0, st, A);
         const HeadViews h = head_views(a, v.qkv, v.attn);
         TRAIN_TRY(artab_row_mask_attention(&h.q, &h.k, &h.v, &h.out, v.lse, a.B, a.H, a.R, a.context_len, a.buffer_len, a.attending_chunks,
                                            D / a.H, 0.f, ARTAB_BF16, ARTAB_IMPL_AUTO, st));
-        TrainForwardB B{};
-        B.attn = v.attn; B.r1 = v.r1; B.stats1 = v.stats1; B.g1 = p[kPG1]; B.b1 = p[kPB1]; B.packed = packed;
-        B.g2 = p[kPG2]; B.b2 = p[kPB2]; B.bias1 = p[kPBias1]; B.bias2 = p[kPBias2]; B.eps2 = a.eps2; B.eps3 = a.eps3;
-        B.r2 = v.r2; B.stats2 = v.stats2; B.r3 = v.r3; B.stats3 = v.stats3; B.M = M;
-        hipLaunchKernelGGL((train_forward_b_kernel<D, F>), grid, block, 0, st, B);
     }
     const float *const *p = a.params + static_cast<size_t>(a.n_layers - 1) * kParams;
     const SavedLayer v = S.layer(a, a.n_layers - 1);
@@ -201,7 +208,7 @@ int backward(const artab_train_args &a, hipStream_t st) {
     const Scratch X = scratch_layout(a);
     const GradLayout G(D, F);
     const long M = static_cast<long>(a.B) * a.R;
-    const int groups = backward_groups(M), jobs = grad_jobs(D, F), slices = grad_slices(M, jobs);
+    const int groups = backward_groups(M, a.D), jobs = grad_jobs(D, F), slices = grad_slices(M, jobs);
     const dim3 block(kTrainWaves * 64);
     {
         const float *const *p = a.params + static_cast<size_t>(a.n_layers - 1) * kParams;
@@ -211,33 +218,12 @@ int backward(const artab_train_args &a, hipStream_t st) {
         Z.dz = a.dz; Z.dx = X.dx; Z.part = X.part_f; Z.B = a.B; Z.R = a.R; Z.first = a.first_row;
         hipLaunchKernelGGL((train_final_kernel<D, true>), dim3(kFinalGroups), dim3(256), 0, st, Z);
         TrainReduce T{};
-        T.cols[0] = {X.part_f, a.grads + a.n_layers * G.total, kFinalGroups, 2 * D};
+        T.cols[0] = {X.part_f, a.grads + a.n_layers * G.total, kFinalGroups, 2 * D, 2 * D};
         T.n_cols = 1;
         hipLaunchKernelGGL(train_reduce_kernel, dim3(2 * D / 64), dim3(256), 0, st, T);
     }
-    for (int l = a.n_layers - 1; l >= 0; --l) {
-        const float *const *p = a.params + static_cast<size_t>(l) * kParams;
-        const SavedLayer v = S.layer(a, l);
-        const bf16_t *packed = S.packed + l * train_packed_elems<D, F>();
-        float *g = a.grads + l * G.total;
-        TrainBackwardB B{};
-        B.dx = X.dx; B.r3 = v.r3; B.stats3 = v.stats3; B.g3 = p[kPG3]; B.r2 = v.r2; B.stats2 = v.stats2; B.g2 = p[kPG2]; B.b2 = p[kPB2];
-        B.bias1 = p[kPBias1]; B.packed = packed; B.dr2 = X.dr2; B.d3 = X.d3; B.x2 = X.x2; B.h = X.h; B.du = X.du; B.d2 = X.d2;
-        B.dattn = X.dattn; B.part = X.part_b; B.M = M;
-        hipLaunchKernelGGL((train_backward_b_kernel<D, F>), dim3(groups), block, 0, st, B);
-        const HeadViews h = head_views(a, v.qkv, v.attn), d = head_views(a, X.dqkv, X.dattn);
-        TRAIN_TRY(artab_row_mask_attention_backward(&h.q, &h.k, &h.v, &h.out, &d.out, v.lse, X.delta, &d.q, &d.k, &d.v, a.B, a.H, a.R, a.context_len,
-                                                    a.buffer_len, a.attending_chunks, D / a.H, 0.f, ARTAB_BF16, ARTAB_IMPL_AUTO, st));
-        TrainBackwardA A{};
-        A.dqkv = X.dqkv; A.dr2 = X.dr2; A.r1 = v.r1; A.stats1 = v.stats1; A.g1 = p[kPG1]; A.b1 = p[kPB1];
-        A.r_prev = a.x;
-        if (l > 0) {
-            const SavedLayer b = S.layer(a, l - 1);
-            A.r_prev = b.r3; A.stats_prev = b.stats3; A.g_prev = p[kPG3 - kParams]; A.b_prev = p[kPB3 - kParams];
-        }
-        A.packed = packed; A.dx = l > 0 ? X.dx : a.dx; A.x1 = X.x1; A.d1 = X.d1; A.x = X.x; A.part = X.part_a; A.M = M;
-        hipLaunchKernelGGL((train_backward_a_kernel<D, F>), dim3(groups), block, 0, st, A);
-
+    for (int l = a.n_layers; l >= 0; --l) {  // launch l: the front of layer l, then the back of layer l - 1
+        TrainBackward A{};
         TrainGradJobs J{};
         TrainReduce T{};
         auto add = [&](const bf16_t *P, int ldp, const bf16_t *Q, int ldq, int N, int K, float *out) {
@@ -248,18 +234,44 @@ int backward(const artab_train_args &a, hipStream_t st) {
                     ++J.jobs;
                 }
         };
-        add(X.dqkv, 3 * D, X.x1, D, 3 * D, D, g + G.qkv);
-        add(X.d1, D, X.x, D, D, D, g + G.fo);
-        add(X.d2, D, v.attn, D, D, D, g + G.o);
-        add(X.du, F, X.x2, D, F, D, g + G.w1);
-        add(X.d3, D, X.h, F, D, F, g + G.w2);
+        A.M = M; A.dr2 = X.dr2; A.part = X.part_c; A.dx = l > 0 ? X.dx : a.dx;
+        if (l < a.n_layers) {
+            const float *const *p = a.params + static_cast<size_t>(l) * kParams;
+            const SavedLayer v = S.layer(a, l);
+            const HeadViews h = head_views(a, v.qkv, v.attn), d = head_views(a, X.dqkv, X.dattn);
+            TRAIN_TRY(artab_row_mask_attention_backward(&h.q, &h.k, &h.v, &h.out, &d.out, v.lse, X.delta, &d.q, &d.k, &d.v, a.B, a.H, a.R,
+                                                        a.context_len, a.buffer_len, a.attending_chunks, D / a.H, 0.f, ARTAB_BF16, ARTAB_IMPL_AUTO, st));
+            A.dqkv = X.dqkv; A.r1 = v.r1; A.stats1 = v.stats1; A.g1 = p[kPG1]; A.b1 = p[kPB1]; A.packed = S.packed + l * train_packed_elems<D, F>();
+            A.x1 = X.x1; A.d1 = X.d1; A.x = X.x; A.r3 = a.x;
+            float *g = a.grads + l * G.total;
+            add(X.dqkv, 3 * D, X.x1, D, 3 * D, D, g + G.qkv);
+            add(X.d1, D, X.x, D, D, D, g + G.fo);
+            T.cols[T.n_cols++] = {X.part_c + 5 * D + F, g + G.vec_a, groups, 7 * D + F, 2 * D};
+        }
+        if (l > 0) {
+            const float *const *p = a.params + static_cast<size_t>(l - 1) * kParams;
+            const SavedLayer v = S.layer(a, l - 1);
+            A.r3 = v.r3; A.stats3 = v.stats3; A.g3 = p[kPG3]; A.b3 = p[kPB3]; A.r2 = v.r2; A.stats2 = v.stats2; A.g2 = p[kPG2]; A.b2 = p[kPB2];
+            A.bias1 = p[kPBias1]; A.back_packed = S.packed + (l - 1) * train_packed_elems<D, F>();
+            A.d3 = X.d3; A.x2 = X.x2; A.h = X.h; A.du = X.du; A.d2 = X.d2; A.dattn = X.dattn;
+            float *g = a.grads + (l - 1) * G.total;
+            add(X.d2, D, v.attn, D, D, D, g + G.o);
+            add(X.du, F, X.x2, D, F, D, g + G.w1);
+            add(X.d3, D, X.h, F, D, F, g + G.w2);
+            T.cols[T.n_cols++] = {X.part_c, g + G.vec_b, groups, 7 * D + F, 5 * D + F};
+        }
+        if (l == a.n_layers)
+            hipLaunchKernelGGL((train_backward_kernel<D, F, false, true>), dim3(groups), block, 0, st, A);
+        else if (l == 0)
+            hipLaunchKernelGGL((train_backward_kernel<D, F, true, false>), dim3(groups), block, 0, st, A);
+        else
+            hipLaunchKernelGGL((train_backward_kernel<D, F, true, true>), dim3(groups), block, 0, st, A);
         J.part = X.part_w; J.M = M; J.rows_per_slice = ((M + slices - 1) / slices + 63) / 64 * 64;
-        hipLaunchKernelGGL(train_weight_grad_kernel, dim3(jobs, slices), dim3(512), 0, st, J);
-        T.part = X.part_w; T.jobs = jobs; T.slices = slices;
-        T.cols[0] = {X.part_b, g + G.vec_b, groups, 5 * D + F};
-        T.cols[1] = {X.part_a, g + G.vec_a, groups, 2 * D};
-        T.n_cols = 2;
-        hipLaunchKernelGGL(train_reduce_kernel, dim3(jobs * 16 + (7 * D + F) / 64), dim3(256), 0, st, T);
+        hipLaunchKernelGGL(train_weight_grad_kernel, dim3(J.jobs, slices), dim3(512), 0, st, J);
+        T.part = X.part_w; T.jobs = J.jobs; T.slices = slices;
+        int columns = 0;
+        for (int i = 0; i < T.n_cols; ++i) columns += T.cols[i].n;
+        hipLaunchKernelGGL(train_reduce_kernel, dim3(J.jobs * 16 + columns / 64), dim3(256), 0, st, T);
     }
     for (int l0 = 0; l0 < a.n_layers; l0 += kTrainPackLayers) {
         const unsigned n = static_cast<unsigned>(a.n_layers - l0 < kTrainPackLayers ? a.n_layers - l0 : kTrainPackLayers);
@@ -322,7 +334,7 @@ int embed_backward(const artab_train_embed_args &a, hipStream_t st) {
     P.d_tokens = a.grads + 7 * D;
     hipLaunchKernelGGL((train_embed_backward_kernel<D>), dim3(a.B > a.n_buffer ? a.B : a.n_buffer, kEmbedSlices + 1), dim3(D), 0, st, P);
     TrainReduce T{};
-    T.cols[0] = {P.part, sums, a.B * kEmbedSlices, 5 * D};
+    T.cols[0] = {P.part, sums, a.B * kEmbedSlices, 5 * D, 5 * D};
     T.n_cols = 1;
     hipLaunchKernelGGL(train_reduce_kernel, dim3(5 * D / 64), dim3(256), 0, st, T);
     hipLaunchKernelGGL(train_embed_finish_kernel, dim3(1), dim3(D), 0, st, sums, a.grads, D);

@@ -4,14 +4,13 @@
 // A step of the reference's training configuration touches 38912 rows of width 128 twelve times over; every
 // layer is five small products per row.  As library calls that is 1300 launches with a cast, a bias, a norm
 // or a copy of 20 MB between any two products, and weight gradients whose 128 x 128 outputs leave most of
-// the chip idle.  Here a layer is: forward two kernels around the attention call, backward two kernels
-// around its backward call, one split product for all weight gradients, one reduction.  They are bound by
+// the chip idle.  Here a layer is: forward one kernel and the attention call, backward one kernel and the
+// attention's backward call, one split product for all weight gradients, one reduction.  They are bound by
 // memory: each reads and writes the residual stream and what the weight gradients need once.
 //
-//   forward    a: x = LN3(r3 of the layer in front); r1 = x + x W_fo^T; x1 = LN1(r1); qkv = x1 W_qkv^T
-//              b: r2 = x1 + attn W_o^T; x2 = LN2(r2); u = x2 W_1^T + b_1; r3 = x2 + gelu(u) W_2^T + b_2
-//   backward   b: d(x of the next layer) -> dr3, du (u is recomputed), dr2, d(attn)
-//              a: d(qkv) -> dr1, dx
+//   forward    behind the attention   r2 = x1 + attn W_o^T; x2 = LN2(r2); u = x2 W_1^T + b_1; r3 = x2 + gelu(u) W_2^T + b_2
+//              in front of the next   x = LN3(r3); r1 = x + x W_fo^T; x1 = LN1(r1); qkv = x1 W_qkv^T
+//   backward   d(qkv) -> dr1, d(x) | d(x) of the layer before -> dr3, du (u is recomputed), dr2, d(attn)
 // with W_fo = out_proj v_proj of the single-column feature attention (one key per query: the softmax weight
 // is 1); dW_out = dW_fo W_v^T and dW_v = W_out^T dW_fo follow from its gradient.  Of every LayerNorm the sum
 // in front of it and (mean, 1/std) are kept; its output is recomputed where it is read.
@@ -19,8 +18,13 @@
 // Tiles.  A workgroup of four wavefronts owns 32 rows and all columns; products are transposed as in
 // fused_layer.h (C^T[n, m] = sum_k W[n, k] A[m, k], v_mfma_f32_16x16x32): a lane holds, for two token rows
 // (lane % 16 and + 16), four consecutive features 4 (lane / 16) + r of every 16-feature block.  Small
-// workgroups, so that the loads of one run under the products of others: forward four or five to a compute unit at
-// d_model 128, three or four at 256; backward two or three, where registers (256 in backward b) are the limit.
+// workgroups, so that the loads of one run under the products of others: four to a compute unit forward, three backward
+// at d_model 128; three and two at 256.
+//
+// 38912 rows of 128: forward 51 us a layer (as two kernels, with r3 written and read back between them, 56; its bytes
+// at the rate of a copy 25), backward 74 us (two kernels 107; 50).  The rest is the weights, 295 and 360 KB a tile from
+// L2, and that the few tiles of a compute unit (4.75) load, multiply and store nearly in step.  Measured and not kept
+// (forward): weights requested ahead of the barriers (50), five workgroups to a compute unit (53, spills).
 #pragma once
 
 #include "common.h"
@@ -171,7 +175,7 @@ struct TrainLane {
     long row0, M;
     __device__ __forceinline__ TrainLane(long tile, long M_) : M(M_) {
         wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-        lane = threadIdx.x & 63;
+        lane = opaque(threadIdx.x & 63);
         tok = lane & 15;
         quad = lane >> 4;
         row0 = tile * kTrainRows;
@@ -218,18 +222,22 @@ __device__ __forceinline__ void train_to_lds(bf16_t *tile, int ld, const f32x4 (
 template <int W>
 __device__ __forceinline__ void train_stage(bf16_t *tile, int lds_ld, const bf16_t *src, long ld, long row0, long M) {
     constexpr int CPR = W / 8;
+    static_assert(kTrainRows * CPR % (kTrainWaves * 64) == 0, "whole passes");
+    const int tid = opaque(threadIdx.x);
 #pragma unroll
-    for (int i = threadIdx.x; i < kTrainRows * CPR; i += kTrainWaves * 64) {
-        const int r = i / CPR, c = i % CPR;
+    for (int x = 0; x < kTrainRows * CPR / (kTrainWaves * 64); ++x) {
+        const int i = tid + kTrainWaves * 64 * x, r = i / CPR, c = i % CPR;
         *reinterpret_cast<u32x4 *>(tile + r * lds_ld + 8 * c) = *reinterpret_cast<const u32x4 *>(src + min(row0 + r, M - 1) * ld + 8 * c);
     }
 }
 template <int W>
 __device__ __forceinline__ void train_unstage(bf16_t *dst, long ld, const bf16_t *tile, int lds_ld, long row0, long M) {
     constexpr int CPR = W / 8;
+    static_assert(kTrainRows * CPR % (kTrainWaves * 64) == 0, "whole passes");
+    const int tid = opaque(threadIdx.x);
 #pragma unroll
-    for (int i = threadIdx.x; i < kTrainRows * CPR; i += kTrainWaves * 64) {
-        const int r = i / CPR, c = i % CPR;
+    for (int x = 0; x < kTrainRows * CPR / (kTrainWaves * 64); ++x) {
+        const int i = tid + kTrainWaves * 64 * x, r = i / CPR, c = i % CPR;
         if (row0 + r < M) *reinterpret_cast<u32x4 *>(dst + (row0 + r) * ld + 8 * c) = *reinterpret_cast<const u32x4 *>(tile + r * lds_ld + 8 * c);
     }
 }
@@ -343,63 +351,6 @@ __device__ __forceinline__ void train_norm(f32x4 (&x)[NB][2], const f32x4 (&r)[N
     }
 }
 
-struct TrainForwardA {
-    const float *r_prev;       // [M, D]: x itself (layer 0) or the sum in front of the last norm of the layer before
-    const float2 *stats_prev;  // its statistics, or nullptr (layer 0)
-    const float *g_prev, *b_prev;
-    const bf16_t *packed;
-    const float *g1, *b1;
-    float eps1;
-    float *r1; float2 *stats1;
-    bf16_t *qkv;               // [M, 3 D]
-    long M;
-};
-
-template <int D, int F>
-__global__ __launch_bounds__(kTrainWaves * 64) void train_forward_a_kernel(TrainForwardA P) {
-    constexpr int NB = D / 64, KS = D / 32, LD = D + 8;
-    __shared__ __attribute__((aligned(16))) bf16_t xs[kTrainRows * LD], ys[kTrainRows * LD];
-    __shared__ float2 red[kTrainWaves * kTrainRows];
-    const TrainLane L(blockIdx.x, P.M);
-    f32x4 x[NB][2], acc[NB][2];
-    train_load<D>(x, P.r_prev, L);
-    if (P.stats_prev) {
-        float2 st[2];
-        train_get_stats(st, P.stats_prev, L);
-        train_norm(x, x, st, P.g_prev, P.b_prev, L);
-    }
-    train_to_lds(xs, LD, x, L);
-    __syncthreads();
-    train_product<NB, KS>(acc, xs, LD, P.packed + train_matrix_at<D, F>(kTmFo), 0, L);
-#pragma unroll
-    for (int b = 0; b < NB; ++b)
-#pragma unroll
-        for (int tb = 0; tb < 2; ++tb) acc[b][tb] += x[b][tb];
-    train_store<D>(P.r1, acc, L);
-    float2 st[2];
-    train_stats<D>(acc, red, P.eps1, P.stats1, st, L);
-    train_norm(acc, acc, st, P.g1, P.b1, L);
-    train_to_lds(ys, LD, acc, L);
-    __syncthreads();
-#pragma unroll
-    for (int part = 0; part < 3; ++part) {
-        train_product<NB, KS>(acc, ys, LD, P.packed + train_matrix_at<D, F>(kTmQkv), part * (D / 16), L);
-        train_store16(P.qkv, 3 * D, part * D, acc, L);
-    }
-}
-
-struct TrainForwardB {
-    const bf16_t *attn;        // [M, D]
-    const float *r1; const float2 *stats1;
-    const float *g1, *b1;
-    const bf16_t *packed;
-    const float *g2, *b2, *bias1, *bias2;
-    float eps2, eps3;
-    float *r2; float2 *stats2;
-    float *r3; float2 *stats3;
-    long M;
-};
-
 // h = gelu(u) and its derivative, in float32: erf by the rational form 7.1.26 of Abramowitz and Stegun, which shares
 // its exponential with the derivative.  Its absolute error is below 1.5e-7; both results are rounded to bf16, of
 // whose unit in the last place that is a hundredth for u above -3 and a quarter at -4.5, where h is 1.5e-5.  On
@@ -414,59 +365,104 @@ __device__ __forceinline__ void train_gelu(float u, float &h, float &dh) {
     dh = fmaf(u * 0.39894228040143268f, e, cdf);
 }
 
-template <int D, int F>
-__global__ __launch_bounds__(kTrainWaves * 64) void train_forward_b_kernel(TrainForwardB P) {
+// What follows the attention of a layer, and what leads to the attention of the next: the stream between the two
+// stays in registers.
+struct TrainForward {
+    // behind the attention (BACK)
+    const bf16_t *attn;        // [M, D]
+    const float *r1; const float2 *stats1;
+    const float *g1, *b1;
+    const float *g2, *b2, *bias1, *bias2;
+    float eps2, eps3;
+    float *r2; float2 *stats2;
+    float *r3; float2 *stats3;
+    const bf16_t *packed;
+    // in front of the next (FRONT)
+    const float *x;            // without BACK: its input
+    const float *g3, *b3;      // with BACK: the norm between the two
+    const float *next_g1, *next_b1;
+    float next_eps1;
+    float *next_r1; float2 *next_stats1;
+    bf16_t *next_qkv;          // [M, 3 D]
+    const bf16_t *next_packed;
+    long M;
+};
+
+template <int D, int F, bool BACK, bool FRONT>
+__global__ __launch_bounds__(kTrainWaves * 64) void train_forward_kernel(TrainForward P) {
     constexpr int NB = D / 64, NF = F / 64, LD = D + 8, LF = F + 8;
-    __shared__ __attribute__((aligned(16))) bf16_t as[kTrainRows * (LD > LF ? LD : LF)], ys[kTrainRows * LD];
+    __shared__ __attribute__((aligned(16))) bf16_t as[kTrainRows * (LD > LF || !BACK ? LD : LF)], ys[kTrainRows * LD];
     __shared__ float2 red[kTrainWaves * kTrainRows];
     const TrainLane L(blockIdx.x, P.M);
     f32x4 x[NB][2], acc[NB][2];
-    train_stage<D>(as, LD, P.attn, D, L.row0, P.M);
-    train_load<D>(x, P.r1, L);
-    {
-        float2 st[2];
+    float2 st[2];
+    if constexpr (BACK) {
+        train_stage<D>(as, LD, P.attn, D, L.row0, P.M);
+        train_load<D>(x, P.r1, L);
         train_get_stats(st, P.stats1, L);
         train_norm(x, x, st, P.g1, P.b1, L);
-    }
-    __syncthreads();
-    train_product<NB, D / 32>(acc, as, LD, P.packed + train_matrix_at<D, F>(kTmO), 0, L);
+        __syncthreads();
+        train_product<NB, D / 32>(acc, as, LD, P.packed + train_matrix_at<D, F>(kTmO), 0, L);
 #pragma unroll
-    for (int b = 0; b < NB; ++b)
+        for (int b = 0; b < NB; ++b)
 #pragma unroll
-        for (int tb = 0; tb < 2; ++tb) x[b][tb] += acc[b][tb];
-    train_store<D>(P.r2, x, L);
-    float2 st[2];
-    train_stats<D>(x, red, P.eps2, P.stats2, st, L);
-    train_norm(x, x, st, P.g2, P.b2, L);
-    train_to_lds(ys, LD, x, L);
-    __syncthreads();
-    {
-        f32x4 u[NF][2];
-        train_product<NF, D / 32>(u, ys, LD, P.packed + train_matrix_at<D, F>(kTm1), 0, L);
+            for (int tb = 0; tb < 2; ++tb) x[b][tb] += acc[b][tb];
+        train_store<D>(P.r2, x, L);
+        train_stats<D>(x, red, P.eps2, P.stats2, st, L);
+        train_norm(x, x, st, P.g2, P.b2, L);
+        train_to_lds(ys, LD, x, L);
+        __syncthreads();
+        {
+            f32x4 u[NF][2];
+            train_product<NF, D / 32>(u, ys, LD, P.packed + train_matrix_at<D, F>(kTm1), 0, L);
 #pragma unroll
-        for (int b = 0; b < NF; ++b) {
-            const f32x4 bias = *reinterpret_cast<const f32x4 *>(P.bias1 + L.col(b));
+            for (int b = 0; b < NF; ++b) {
+                const f32x4 bias = *reinterpret_cast<const f32x4 *>(P.bias1 + L.col(b));
 #pragma unroll
-            for (int tb = 0; tb < 2; ++tb)
+                for (int tb = 0; tb < 2; ++tb)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    float h, dh;
-                    train_gelu(u[b][tb][e] + bias[e], h, dh);
-                    u[b][tb][e] = h;
-                }
+                    for (int e = 0; e < 4; ++e) {
+                        float h, dh;
+                        train_gelu(u[b][tb][e] + bias[e], h, dh);
+                        u[b][tb][e] = h;
+                    }
+            }
+            train_to_lds(as, LF, u, L);
         }
-        train_to_lds(as, LF, u, L);
-    }
-    __syncthreads();
-    train_product<NB, F / 32>(acc, as, LF, P.packed + train_matrix_at<D, F>(kTm2), 0, L);
+        __syncthreads();
+        train_product<NB, F / 32>(acc, as, LF, P.packed + train_matrix_at<D, F>(kTm2), 0, L);
 #pragma unroll
-    for (int b = 0; b < NB; ++b) {
-        const f32x4 bias = *reinterpret_cast<const f32x4 *>(P.bias2 + L.col(b));
+        for (int b = 0; b < NB; ++b) {
+            const f32x4 bias = *reinterpret_cast<const f32x4 *>(P.bias2 + L.col(b));
 #pragma unroll
-        for (int tb = 0; tb < 2; ++tb) x[b][tb] += acc[b][tb] + bias;
+            for (int tb = 0; tb < 2; ++tb) x[b][tb] += acc[b][tb] + bias;
+        }
+        train_store<D>(P.r3, x, L);
+        train_stats<D>(x, red, P.eps3, P.stats3, st, L);  // (its barrier: nobody reads the tiles any more)
+        if constexpr (FRONT) train_norm(x, x, st, P.g3, P.b3, L);
+    } else {
+        train_load<D>(x, P.x, L);
     }
-    train_store<D>(P.r3, x, L);
-    train_stats<D>(x, red, P.eps3, P.stats3, st, L);
+    if constexpr (FRONT) {
+        const TrainLane L(blockIdx.x, P.M);
+        train_to_lds(as, LD, x, L);
+        __syncthreads();
+        train_product<NB, D / 32>(acc, as, LD, P.next_packed + train_matrix_at<D, F>(kTmFo), 0, L);
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int tb = 0; tb < 2; ++tb) acc[b][tb] += x[b][tb];
+        train_store<D>(P.next_r1, acc, L);
+        train_stats<D>(acc, red, P.next_eps1, P.next_stats1, st, L);
+        train_norm(acc, acc, st, P.next_g1, P.next_b1, L);
+        train_to_lds(ys, LD, acc, L);
+        __syncthreads();
+#pragma unroll
+        for (int part = 0; part < 3; ++part) {
+            train_product<NB, D / 32>(acc, ys, LD, P.next_packed + train_matrix_at<D, F>(kTmQkv), part * (D / 16), L);
+            train_store16(P.next_qkv, 3 * D, part * D, acc, L);
+        }
+    }
 }
 
 // ---- backward
@@ -527,146 +523,145 @@ __device__ __forceinline__ void train_norm_backward(f32x4 (&d)[NB][2], const f32
     }
 }
 
-struct TrainBackwardB {
-    const float *dx;           // [M, D] gradient of the layer's output
-    const float *r3; const float2 *stats3; const float *g3;
+// The front of a layer backward (FRONT), then the back of the layer before it (BACK): the gradient between the two
+// stays in registers, and the sum in front of the norm between them is read once.
+struct TrainBackward {
+    // the layer whose d(qkv) is known
+    const bf16_t *dqkv;        // [M, 3 D]
+    const float *r1; const float2 *stats1; const float *g1, *b1;
+    const bf16_t *packed;
+    bf16_t *x1, *d1, *x;       // [M, D] each
+    // between the two: the sum in front of the norm of the layer before (its output is this layer's input), or,
+    // without BACK, the input itself
+    const float *r3; const float2 *stats3; const float *g3, *b3;
+    float *dx;                 // [M, D]: without FRONT the gradient of the layer's output, without BACK that of the input
+    // the layer before
     const float *r2; const float2 *stats2; const float *g2, *b2;
     const float *bias1;
-    const bf16_t *packed;
-    float *dr2;                // [M, D]: gradient of x1 along the residual
+    const bf16_t *back_packed;
     bf16_t *d3, *x2, *h, *du, *d2, *dattn;  // [M, D], [M, D], [M, F], [M, F], [M, D], [M, D]
-    float *part;               // [gridDim.x][5 D + F]: column sums g3, b3, bias2, g2, b2 (D each), bias1
+    float *dr2;                // [M, D]: gradient of x1 along the residual: of the later layer, then of the one before
+    float *part;               // [gridDim.x][7 D + F]: column sums g3, b3, bias2, g2, b2 (D each), bias1 (F); g1, b1
     long M;
 };
 
-template <int D, int F>
-__global__ __launch_bounds__(kTrainWaves * 64, 2) void train_backward_b_kernel(TrainBackwardB P) {
-    constexpr int NB = D / 64, NF = F / 64, LD = D + 8, LF = F + 8, NS = 5 * D + F;
-    __shared__ __attribute__((aligned(16))) bf16_t ds[kTrainRows * LD], xs[kTrainRows * LD], us[kTrainRows * LF];
+// (d_model 128: held to 168 registers, three workgroups to a compute unit.  For that the feed-forward goes in two halves
+// and lane indices are taken anew in each part, or some 40 addresses would be kept over the loop: two workgroups
+// of 256 registers took 90 us, three of them 83, every resident one started 74.)
+template <int D, int F, bool FRONT, bool BACK>
+__global__ __launch_bounds__(kTrainWaves * 64, D == 128 ? 3 : 2) void train_backward_kernel(TrainBackward P) {
+    constexpr int NB = D / 64, LD = D + 8, LQ = 3 * D + 8, LF = F + 8, NS = 7 * D + F;
+    constexpr int kWide = FRONT && LQ > LD + LF ? LQ : LD + LF;  // d(qkv) lies where x2 and d(u) do later
+    __shared__ __attribute__((aligned(16))) bf16_t ds[kTrainRows * LD], wide[kTrainRows * kWide];
     __shared__ float2 red[kTrainWaves * kTrainRows];
     __shared__ __attribute__((aligned(16))) float sums[NS];
+    bf16_t *const qs = wide, *const xs = wide, *const us = wide + kTrainRows * LD;
     for (int i = threadIdx.x; i < NS; i += kTrainWaves * 64) sums[i] = 0.f;
     __syncthreads();
     const long tiles = (P.M + kTrainRows - 1) / kTrainRows;
     for (long tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
         const TrainLane L(tile, P.M);
-        const bf16_t *const packed = train_opaque(P.packed);
-        f32x4 d[NB][2], r[NB][2], acc[NB][2];
-        float2 st[2], st2[2];
-        train_load<D>(d, P.dx, L);
-        train_load<D>(r, P.r3, L);
-        train_get_stats(st, P.stats3, L);
-        train_norm_backward<D>(d, r, st, P.g3, sums, sums + D, red, L);
-#pragma unroll
-        for (int b = 0; b < NB; ++b) train_col_add(sums + 2 * D, d[b][0] + d[b][1], L.col(b), L);  // (rows past the end are zero)
-        train_to_lds(ds, LD, d, L);
-        train_load<D>(r, P.r2, L);
-        train_get_stats(st2, P.stats2, L);
-        train_norm(acc, r, st2, P.g2, P.b2, L);
-        train_to_lds(xs, LD, acc, L);
-        __syncthreads();
-        train_unstage<D>(P.d3, D, ds, LD, L.row0, P.M);
-        train_unstage<D>(P.x2, D, xs, LD, L.row0, P.M);
-        {
-            f32x4 u[NF][2], dh[NF][2];
-            train_product<NF, D / 32>(u, xs, LD, packed + train_matrix_at<D, F>(kTm1), 0, L);
-#pragma unroll
-            for (int b = 0; b < NF; ++b) {
-                const f32x4 bias = *reinterpret_cast<const f32x4 *>(P.bias1 + L.col(b));
-#pragma unroll
-                for (int tb = 0; tb < 2; ++tb)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        float hv, dv;
-                        train_gelu(u[b][tb][e] + bias[e], hv, dv);
-                        dh[b][tb][e] = hv;
-                        u[b][tb][e] = dv;
-                    }
-            }
-            train_store16(P.h, F, 0, dh, L);
-            train_product<NF, D / 32>(dh, ds, LD, packed + train_matrix_at<D, F>(kTm2T), 0, L);
-#pragma unroll
-            for (int b = 0; b < NF; ++b) {
-#pragma unroll
-                for (int tb = 0; tb < 2; ++tb) u[b][tb] *= dh[b][tb];
-                train_col_add(sums + 5 * D, u[b][0] + u[b][1], L.col(b), L);
-            }
-            train_to_lds(us, LF, u, L);
-        }
-        __syncthreads();
-        train_unstage<F>(P.du, F, us, LF, L.row0, P.M);
-        train_product<NB, F / 32>(acc, us, LF, packed + train_matrix_at<D, F>(kTm1T), 0, L);
-#pragma unroll
-        for (int b = 0; b < NB; ++b)
-#pragma unroll
-            for (int tb = 0; tb < 2; ++tb) d[b][tb] += acc[b][tb];
-        train_norm_backward<D>(d, r, st2, P.g2, sums + 3 * D, sums + 4 * D, red, L);
-        train_store<D>(P.dr2, d, L);
-        train_to_lds(ds, LD, d, L);  // (its readers are behind the barrier inside the norm)
-        __syncthreads();
-        train_unstage<D>(P.d2, D, ds, LD, L.row0, P.M);
-        train_product<NB, D / 32>(acc, ds, LD, packed + train_matrix_at<D, F>(kTmOT), 0, L);
-        train_store16(P.dattn, D, 0, acc, L);
-        __syncthreads();
-    }
-    for (int i = threadIdx.x; i < NS; i += kTrainWaves * 64) P.part[static_cast<long>(blockIdx.x) * NS + i] = sums[i];
-}
-
-struct TrainBackwardA {
-    const bf16_t *dqkv;        // [M, 3 D]
-    const float *dr2;
-    const float *r1; const float2 *stats1; const float *g1, *b1;
-    const float *r_prev; const float2 *stats_prev; const float *g_prev, *b_prev;  // as in TrainForwardA
-    const bf16_t *packed;
-    float *dx;                 // [M, D] gradient of the layer's input
-    bf16_t *x1, *d1, *x;       // [M, D] each
-    float *part;               // [gridDim.x][2 D]: column sums g1, b1
-    long M;
-};
-
-template <int D, int F>
-__global__ __launch_bounds__(kTrainWaves * 64, 2) void train_backward_a_kernel(TrainBackwardA P) {
-    constexpr int NB = D / 64, LD = D + 8, LQ = 3 * D + 8, NS = 2 * D;
-    __shared__ __attribute__((aligned(16))) bf16_t qs[kTrainRows * LQ], ds[kTrainRows * LD];
-    __shared__ float2 red[kTrainWaves * kTrainRows];
-    __shared__ __attribute__((aligned(16))) float sums[NS];
-    for (int i = threadIdx.x; i < NS; i += kTrainWaves * 64) sums[i] = 0.f;
-    const long tiles = (P.M + kTrainRows - 1) / kTrainRows;
-    for (long tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
-        const TrainLane L(tile, P.M);
-        const bf16_t *const packed = train_opaque(P.packed);
+        const bf16_t *const packed = train_opaque(P.packed), *const back_packed = train_opaque(P.back_packed);
         f32x4 d[NB][2], r[NB][2], acc[NB][2];
         float2 st[2];
-        train_stage<3 * D>(qs, LQ, P.dqkv, 3 * D, L.row0, P.M);
-        train_load<D>(d, P.dr2, L);
-        train_load<D>(r, P.r1, L);
-        train_get_stats(st, P.stats1, L);
-        train_norm(acc, r, st, P.g1, P.b1, L);
-        train_store16(P.x1, D, 0, acc, L);
-        __syncthreads();
-        train_product<NB, 3 * D / 32>(acc, qs, LQ, packed + train_matrix_at<D, F>(kTmQkvT), 0, L);
+        if constexpr (FRONT) {
+            train_stage<3 * D>(qs, LQ, P.dqkv, 3 * D, L.row0, P.M);
+            train_load<D>(d, P.dr2, L);
+            train_load<D>(r, P.r1, L);
+            train_get_stats(st, P.stats1, L);
+            train_norm(acc, r, st, P.g1, P.b1, L);
+            train_store16(P.x1, D, 0, acc, L);
+            __syncthreads();
+            train_product<NB, 3 * D / 32>(acc, qs, LQ, packed + train_matrix_at<D, F>(kTmQkvT), 0, L);
 #pragma unroll
-        for (int b = 0; b < NB; ++b)
+            for (int b = 0; b < NB; ++b)
 #pragma unroll
-            for (int tb = 0; tb < 2; ++tb) d[b][tb] += acc[b][tb];
-        train_norm_backward<D>(d, r, st, P.g1, sums, sums + D, red, L);
-        train_to_lds(ds, LD, d, L);
-        train_load<D>(r, P.r_prev, L);
-        if (P.stats_prev) {
-            train_get_stats(st, P.stats_prev, L);
-            train_norm(r, r, st, P.g_prev, P.b_prev, L);
+                for (int tb = 0; tb < 2; ++tb) d[b][tb] += acc[b][tb];
+            train_norm_backward<D>(d, r, st, P.g1, sums + 5 * D + F, sums + 6 * D + F, red, L);
+            train_to_lds(ds, LD, d, L);
+            train_load<D>(r, P.r3, L);
+            if (BACK || P.stats3) {
+                train_get_stats(st, P.stats3, L);
+                train_norm(acc, r, st, P.g3, P.b3, L);
+                train_store16(P.x, D, 0, acc, L);
+            } else {
+                train_store16(P.x, D, 0, r, L);
+            }
+            __syncthreads();
+            train_unstage<D>(P.d1, D, ds, LD, L.row0, P.M);
+            train_product<NB, D / 32>(acc, ds, LD, packed + train_matrix_at<D, F>(kTmFoT), 0, L);
+#pragma unroll
+            for (int b = 0; b < NB; ++b)
+#pragma unroll
+                for (int tb = 0; tb < 2; ++tb) d[b][tb] += acc[b][tb];
+            if constexpr (!BACK) train_store<D>(P.dx, d, L);
+        } else {
+            train_load<D>(d, P.dx, L);
+            train_load<D>(r, P.r3, L);
+            train_get_stats(st, P.stats3, L);
         }
-        train_store16(P.x, D, 0, r, L);
-        __syncthreads();
-        train_unstage<D>(P.d1, D, ds, LD, L.row0, P.M);
-        train_product<NB, D / 32>(acc, ds, LD, packed + train_matrix_at<D, F>(kTmFoT), 0, L);
+        if constexpr (BACK) {
+            const TrainLane L(tile, P.M);
+            train_norm_backward<D>(d, r, st, P.g3, sums, sums + D, red, L);  // (its barrier: nobody reads ds or the wide tile any more)
 #pragma unroll
-        for (int b = 0; b < NB; ++b)
+            for (int b = 0; b < NB; ++b) train_col_add(sums + 2 * D, d[b][0] + d[b][1], L.col(b), L);  // (rows past the end are zero)
+            train_to_lds(ds, LD, d, L);
+            train_load<D>(r, P.r2, L);
+            train_get_stats(st, P.stats2, L);
+            train_norm(acc, r, st, P.g2, P.b2, L);
+            train_to_lds(xs, LD, acc, L);
+            __syncthreads();
+            train_unstage<D>(P.d3, D, ds, LD, L.row0, P.M);
+            train_unstage<D>(P.x2, D, xs, LD, L.row0, P.M);
+            // the feed-forward in two halves of its width
+            constexpr int HF = F / 2, NH = HF / 64;
+#pragma unroll 1
+            for (int half = 0; half < 2; ++half) {
+                const int f0 = half * HF;
+                const TrainLane L(tile, P.M);
+                f32x4 u[NH][2], dh[NH][2];
+                train_product<NH, D / 32>(u, xs, LD, back_packed + train_matrix_at<D, F>(kTm1), f0 / 16, L);
 #pragma unroll
-            for (int tb = 0; tb < 2; ++tb) d[b][tb] += acc[b][tb];
-        train_store<D>(P.dx, d, L);
+                for (int b = 0; b < NH; ++b) {
+                    const f32x4 bias = *reinterpret_cast<const f32x4 *>(P.bias1 + f0 + L.col(b));
+#pragma unroll
+                    for (int tb = 0; tb < 2; ++tb)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            float hv, dv;
+                            train_gelu(u[b][tb][e] + bias[e], hv, dv);
+                            dh[b][tb][e] = hv;
+                            u[b][tb][e] = dv;
+                        }
+                }
+                train_store16(P.h, F, f0, dh, L);
+                train_product<NH, D / 32>(dh, ds, LD, back_packed + train_matrix_at<D, F>(kTm2T), f0 / 16, L);
+#pragma unroll
+                for (int b = 0; b < NH; ++b) {
+#pragma unroll
+                    for (int tb = 0; tb < 2; ++tb) u[b][tb] *= dh[b][tb];
+                    train_col_add(sums + 5 * D + f0, u[b][0] + u[b][1], L.col(b), L);
+                }
+                train_to_lds(us + f0, LF, u, L);
+            }
+            __syncthreads();
+            train_unstage<F>(P.du, F, us, LF, L.row0, P.M);
+            train_product<NB, F / 32>(acc, us, LF, back_packed + train_matrix_at<D, F>(kTm1T), 0, L);
+#pragma unroll
+            for (int b = 0; b < NB; ++b)
+#pragma unroll
+                for (int tb = 0; tb < 2; ++tb) d[b][tb] += acc[b][tb];
+            train_norm_backward<D>(d, r, st, P.g2, sums + 3 * D, sums + 4 * D, red, L);
+            train_store<D>(P.dr2, d, L);
+            train_to_lds(ds, LD, d, L);  // (its readers are behind the barrier inside the norm)
+            __syncthreads();
+            train_unstage<D>(P.d2, D, ds, LD, L.row0, P.M);
+            train_product<NB, D / 32>(acc, ds, LD, back_packed + train_matrix_at<D, F>(kTmOT), 0, L);
+            train_store16(P.dattn, D, 0, acc, L);
+        }
         __syncthreads();
     }
+    // (without the other half its columns are zero and belong to nobody)
     for (int i = threadIdx.x; i < NS; i += kTrainWaves * 64) P.part[static_cast<long>(blockIdx.x) * NS + i] = sums[i];
 }
 
@@ -863,9 +858,9 @@ struct TrainReduce {
     const float *part; int jobs, slices;
     float *out[kTrainMaxJobs]; int ld[kTrainMaxJobs];
     struct Cols {
-        const float *part;     // [groups][n]
+        const float *part;     // [groups][ld], n columns of it
         float *out;
-        int groups, n;
+        int groups, ld, n;
     } cols[2];
     int n_cols;
 };
@@ -895,8 +890,8 @@ static __global__ __launch_bounds__(256) void train_reduce_kernel(TrainReduce P)
     int i = wave;
     for (; i + 28 < C.groups; i += 32)
 #pragma unroll
-        for (int u = 0; u < 8; ++u) part[u] += col[static_cast<long>(i + 4 * u) * C.n];
-    for (; i < C.groups; i += 4) part[0] += col[static_cast<long>(i) * C.n];
+        for (int u = 0; u < 8; ++u) part[u] += col[static_cast<long>(i + 4 * u) * C.ld];
+    for (; i < C.groups; i += 4) part[0] += col[static_cast<long>(i) * C.ld];
     const float s = ((part[0] + part[1]) + (part[2] + part[3])) + ((part[4] + part[5]) + (part[6] + part[7]));
     acc[wave][lane] = s;
     __syncthreads();

@@ -1,0 +1,16 @@
+"""The training kernels that reach from one layer into the next, where a workgroup of the backward kernel has several
+tiles and others have fewer, with a ragged last one; against the modules."""
+
+import pytest
+
+from tests.test_training_stack_gpu import test_fused_training_equals_modules as equals_modules
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("D,H,L,B,Nc,Nb,Nt,feat,tokens", [
+    (128, 4, 3, 61, 70, 9, 324, 2, 9),     # 769 tiles of 32 rows, the last of 7 rows: one workgroup with two
+    (256, 8, 2, 37, 100, 8, 337, 2, 8),    # 515 tiles on 512 workgroups
+])
+def test_stack_of_many_tiles_equals_modules(device, monkeypatch, D, H, L, B, Nc, Nb, Nt, feat, tokens):
+    equals_modules(device, monkeypatch, D, H, L, B, Nc, Nb, Nt, feat, tokens)
