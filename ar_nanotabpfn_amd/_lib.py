@@ -137,6 +137,17 @@ class ArtabTrainEmbedArgs(ctypes.Structure):
     ]
 
 
+class ArtabTrainHeadArgs(ctypes.Structure):
+    """``artab_train_head_args`` of include/artab_attention.h, field for field."""
+
+    _fields_ = [
+        *((n, _i) for n in ("rows", "D", "F", "K")),
+        ("std_min", _f),
+        *((n, _p) for n in ("z", "y", "w1", "b1", "w2", "b2", "mean_bias", "std_bias", "weight_bias", "saved", "loss", "dloss", "dz",
+                            "grads", "scratch")),
+    ]
+
+
 TAPE_FO, TAPE_QKV, TAPE_O, TAPE_1, TAPE_2, TAPE_H1, TAPE_H2, TAPE_CLOSE = range(8)
 
 # name -> (restype, argtypes); every symbol declared in include/artab_attention.h
@@ -212,6 +223,10 @@ SIGNATURES = {
     "artab_train_embed_scratch_bytes": (_sz, [ctypes.POINTER(ArtabTrainEmbedArgs)]),
     "artab_train_embed": (_i, [ctypes.POINTER(ArtabTrainEmbedArgs), _p]),
     "artab_train_embed_backward": (_i, [ctypes.POINTER(ArtabTrainEmbedArgs), _p]),
+    "artab_train_head_saved_bytes": (_sz, [ctypes.POINTER(ArtabTrainHeadArgs)]),
+    "artab_train_head_scratch_bytes": (_sz, [ctypes.POINTER(ArtabTrainHeadArgs)]),
+    "artab_train_head_forward": (_i, [ctypes.POINTER(ArtabTrainHeadArgs), _p]),
+    "artab_train_head_backward": (_i, [ctypes.POINTER(ArtabTrainHeadArgs), _p]),
     "artab_trajectory_group": (_i, [_i, _i, _i, _i, _i, _i, _i, _i]),
     "artab_trajectory_group_layers": (_i, [_i, _i, _i, _i, _i, _i, _i, _i, _i]),
     "artab_trajectory_tape_bytes": (_sz, [_i, _i, _i, _i]),

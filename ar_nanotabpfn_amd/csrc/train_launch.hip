@@ -2,6 +2,7 @@
 // attention (include/artab_attention.h, artab_train_*).
 #include "../../include/artab_attention.h"
 #include "launchers.h"
+#include "train_head.h"
 #include "train_layers.h"
 
 namespace artab {
@@ -202,6 +203,31 @@ int forward(const artab_train_args &a, hipStream_t st) {
     return hipGetLastError() == hipSuccess ? ARTAB_OK : ARTAB_ERR_LAUNCH;
 }
 
+// Weight gradients of a launch: C[n][k] = sum_m P[m][n] Q[m][k] in pieces, and the workgroups' column sums.
+struct GradProducts {
+    TrainGradJobs jobs{};
+    TrainReduce reduce{};
+    GradProducts(long M, int slices, float *part) {
+        jobs.part = part; jobs.M = M; jobs.rows_per_slice = ((M + slices - 1) / slices + 63) / 64 * 64;
+        reduce.part = part; reduce.slices = slices;
+    }
+    void add(const bf16_t *P, int ldp, const bf16_t *Q, int ldq, int N, int K, float *out) {
+        for (int n = 0; n < N; n += 128)
+            for (int k = 0; k < K; k += 128) {
+                const int i = jobs.jobs++;
+                jobs.p[i] = P + n; jobs.q[i] = Q + k; jobs.ldp[i] = ldp; jobs.ldq[i] = ldq;
+                reduce.out[i] = out + static_cast<long>(n) * K + k; reduce.ld[i] = K;
+            }
+    }
+    void launch(hipStream_t st) {
+        reduce.jobs = jobs.jobs;
+        int columns = 0;
+        for (int i = 0; i < reduce.n_cols; ++i) columns += reduce.cols[i].n;
+        hipLaunchKernelGGL(train_weight_grad_kernel, dim3(jobs.jobs, reduce.slices), dim3(512), 0, st, jobs);
+        hipLaunchKernelGGL(train_reduce_kernel, dim3(jobs.jobs * 16 + columns / 64), dim3(256), 0, st, reduce);
+    }
+};
+
 template <int D, int F>
 int backward(const artab_train_args &a, hipStream_t st) {
     const Saved S = saved_layout(a);
@@ -224,16 +250,7 @@ int backward(const artab_train_args &a, hipStream_t st) {
     }
     for (int l = a.n_layers; l >= 0; --l) {  // launch l: the front of layer l, then the back of layer l - 1
         TrainBackward A{};
-        TrainGradJobs J{};
-        TrainReduce T{};
-        auto add = [&](const bf16_t *P, int ldp, const bf16_t *Q, int ldq, int N, int K, float *out) {
-            for (int n = 0; n < N; n += 128)
-                for (int k = 0; k < K; k += 128) {
-                    J.p[J.jobs] = P + n; J.q[J.jobs] = Q + k; J.ldp[J.jobs] = ldp; J.ldq[J.jobs] = ldq;
-                    T.out[J.jobs] = out + static_cast<long>(n) * K + k; T.ld[J.jobs] = K;
-                    ++J.jobs;
-                }
-        };
+        GradProducts products(M, slices, X.part_w);
         A.M = M; A.dr2 = X.dr2; A.part = X.part_c; A.dx = l > 0 ? X.dx : a.dx;
         if (l < a.n_layers) {
             const float *const *p = a.params + static_cast<size_t>(l) * kParams;
@@ -244,9 +261,9 @@ int backward(const artab_train_args &a, hipStream_t st) {
             A.dqkv = X.dqkv; A.r1 = v.r1; A.stats1 = v.stats1; A.g1 = p[kPG1]; A.b1 = p[kPB1]; A.packed = S.packed + l * train_packed_elems<D, F>();
             A.x1 = X.x1; A.d1 = X.d1; A.x = X.x; A.r3 = a.x;
             float *g = a.grads + l * G.total;
-            add(X.dqkv, 3 * D, X.x1, D, 3 * D, D, g + G.qkv);
-            add(X.d1, D, X.x, D, D, D, g + G.fo);
-            T.cols[T.n_cols++] = {X.part_c + 5 * D + F, g + G.vec_a, groups, 7 * D + F, 2 * D};
+            products.add(X.dqkv, 3 * D, X.x1, D, 3 * D, D, g + G.qkv);
+            products.add(X.d1, D, X.x, D, D, D, g + G.fo);
+            products.reduce.cols[products.reduce.n_cols++] = {X.part_c + 5 * D + F, g + G.vec_a, groups, 7 * D + F, 2 * D};
         }
         if (l > 0) {
             const float *const *p = a.params + static_cast<size_t>(l - 1) * kParams;
@@ -255,10 +272,10 @@ int backward(const artab_train_args &a, hipStream_t st) {
             A.bias1 = p[kPBias1]; A.back_packed = S.packed + (l - 1) * train_packed_elems<D, F>();
             A.d3 = X.d3; A.x2 = X.x2; A.h = X.h; A.du = X.du; A.d2 = X.d2; A.dattn = X.dattn;
             float *g = a.grads + (l - 1) * G.total;
-            add(X.d2, D, v.attn, D, D, D, g + G.o);
-            add(X.du, F, X.x2, D, F, D, g + G.w1);
-            add(X.d3, D, X.h, F, D, F, g + G.w2);
-            T.cols[T.n_cols++] = {X.part_c, g + G.vec_b, groups, 7 * D + F, 5 * D + F};
+            products.add(X.d2, D, v.attn, D, D, D, g + G.o);
+            products.add(X.du, F, X.x2, D, F, D, g + G.w1);
+            products.add(X.d3, D, X.h, F, D, F, g + G.w2);
+            products.reduce.cols[products.reduce.n_cols++] = {X.part_c, g + G.vec_b, groups, 7 * D + F, 5 * D + F};
         }
         if (l == a.n_layers)
             hipLaunchKernelGGL((train_backward_kernel<D, F, false, true>), dim3(groups), block, 0, st, A);
@@ -266,12 +283,7 @@ int backward(const artab_train_args &a, hipStream_t st) {
             hipLaunchKernelGGL((train_backward_kernel<D, F, true, false>), dim3(groups), block, 0, st, A);
         else
             hipLaunchKernelGGL((train_backward_kernel<D, F, true, true>), dim3(groups), block, 0, st, A);
-        J.part = X.part_w; J.M = M; J.rows_per_slice = ((M + slices - 1) / slices + 63) / 64 * 64;
-        hipLaunchKernelGGL(train_weight_grad_kernel, dim3(J.jobs, slices), dim3(512), 0, st, J);
-        T.part = X.part_w; T.jobs = J.jobs; T.slices = slices;
-        int columns = 0;
-        for (int i = 0; i < T.n_cols; ++i) columns += T.cols[i].n;
-        hipLaunchKernelGGL(train_reduce_kernel, dim3(J.jobs * 16 + columns / 64), dim3(256), 0, st, T);
+        products.launch(st);
     }
     for (int l0 = 0; l0 < a.n_layers; l0 += kTrainPackLayers) {
         const unsigned n = static_cast<unsigned>(a.n_layers - l0 < kTrainPackLayers ? a.n_layers - l0 : kTrainPackLayers);
@@ -332,12 +344,93 @@ int embed_backward(const artab_train_embed_args &a, hipStream_t st) {
     P.part = s.take<float>(static_cast<size_t>(a.B) * kEmbedSlices * 5 * D);
     float *sums = s.take<float>(5 * D);
     P.d_tokens = a.grads + 7 * D;
-    hipLaunchKernelGGL((train_embed_backward_kernel<D>), dim3(a.B > a.n_buffer ? a.B : a.n_buffer, kEmbedSlices + 1), dim3(D), 0, st, P);
+    hipLaunchKernelGGL((train_embed_backward_kernel<D>), dim3(a.B > a.n_buffer ? a.B : a.n_buffer, kEmbedSlices + 1), dim3(256), 0, st, P);
     TrainReduce T{};
     T.cols[0] = {P.part, sums, a.B * kEmbedSlices, 5 * D, 5 * D};
     T.n_cols = 1;
     hipLaunchKernelGGL(train_reduce_kernel, dim3(5 * D / 64), dim3(256), 0, st, T);
     hipLaunchKernelGGL(train_embed_finish_kernel, dim3(1), dim3(D), 0, st, sums, a.grads, D);
+    return hipGetLastError() == hipSuccess ? ARTAB_OK : ARTAB_ERR_LAUNCH;
+}
+
+// ---- the head
+
+bool head_supported(const artab_train_head_args *a) {
+    return a && a->rows >= 1 && a->rows < (1 << 30) && (a->D == 128 || a->D == 256) && a->F == 256 && a->K >= 1 && 3 * a->K <= kHeadCols;
+}
+int head_cols(const artab_train_head_args &a) { return 3 * a.K <= 64 ? 64 : 128; }
+int head_groups(long M) {  // as many workgroups as are resident (three to a compute unit), or fewer
+    const long tiles = (M + kTrainRows - 1) / kTrainRows;
+    return static_cast<int>(tiles < 768 ? tiles : 768);
+}
+int head_jobs(const artab_train_head_args &a) { return (a.F / 128) * (a.D / 128) + a.F / 128; }
+
+struct HeadSaved {
+    bf16_t *packed;
+    float *part_loss;
+    size_t bytes;
+};
+HeadSaved head_saved(const artab_train_head_args &a) {
+    Arena s(a.saved);
+    HeadSaved v;
+    v.packed = s.take<bf16_t>(2 * static_cast<size_t>(a.F) * (a.D + head_cols(a)));
+    v.part_loss = s.take<float>(head_groups(a.rows));
+    v.bytes = s.used;
+    return v;
+}
+struct HeadScratch {
+    bf16_t *zb, *h, *du, *draw;
+    float *part, *part_w;
+    size_t bytes;
+};
+HeadScratch head_scratch(const artab_train_head_args &a) {
+    Arena s(a.scratch);
+    HeadScratch v;
+    const size_t M = a.rows;
+    const int jobs = head_jobs(a);
+    v.zb = s.take<bf16_t>(M * a.D);
+    v.h = s.take<bf16_t>(M * a.F);
+    v.du = s.take<bf16_t>(M * a.F);
+    v.draw = s.take<bf16_t>(M * kHeadCols);
+    v.part = s.take<float>(static_cast<size_t>(head_groups(a.rows)) * (a.F + kHeadCols));
+    v.part_w = s.take<float>(static_cast<size_t>(grad_slices(M, jobs)) * jobs * 16384);
+    v.bytes = s.used;
+    return v;
+}
+
+TrainHead head_params(const artab_train_head_args &a) {
+    TrainHead P{};
+    P.z = a.z; P.y = a.y; P.w1 = a.w1; P.b1 = a.b1; P.w2 = a.w2; P.b2 = a.b2;
+    P.mean_bias = a.mean_bias; P.std_bias = a.std_bias; P.weight_bias = a.weight_bias; P.std_min = a.std_min; P.K = a.K; P.M = a.rows;
+    const HeadSaved S = head_saved(a);
+    P.packed = S.packed; P.part_loss = S.part_loss;
+    return P;
+}
+
+template <int D, int NP>
+int head_forward(const artab_train_head_args &a, hipStream_t st) {
+    constexpr int F = 256;
+    const TrainHead P = head_params(a);
+    const int groups = head_groups(a.rows);
+    hipLaunchKernelGGL((train_head_pack_kernel<D, F, NP>), dim3(static_cast<unsigned>((train_head_packed_elems<D, F, NP>() / 8 + 255) / 256)),
+                       dim3(256), 0, st, P);
+    hipLaunchKernelGGL((train_head_kernel<D, F, NP, false>), dim3(groups), dim3(kTrainWaves * 64), 0, st, P);
+    hipLaunchKernelGGL(train_head_loss_kernel, dim3(1), dim3(256), 0, st, P.part_loss, groups, P.M, a.loss);
+    return hipGetLastError() == hipSuccess ? ARTAB_OK : ARTAB_ERR_LAUNCH;
+}
+template <int D, int NP>
+int head_backward(const artab_train_head_args &a, hipStream_t st) {
+    constexpr int F = 256;
+    TrainHead P = head_params(a);
+    const HeadScratch X = head_scratch(a);
+    const int groups = head_groups(a.rows), jobs = head_jobs(a), slices = grad_slices(P.M, jobs);
+    P.dloss = a.dloss; P.dz = a.dz; P.zb = X.zb; P.h = X.h; P.du = X.du; P.draw = X.draw; P.part = X.part;
+    hipLaunchKernelGGL((train_head_kernel<D, F, NP, true>), dim3(groups), dim3(kTrainWaves * 64), 0, st, P);
+    GradProducts products(P.M, slices, X.part_w);
+    products.add(X.du, F, X.zb, D, F, D, a.grads);
+    products.add(X.draw, kHeadCols, X.h, F, kHeadCols, F, a.grads + static_cast<long>(F) * D);
+    products.reduce.cols[products.reduce.n_cols++] = {X.part, a.grads + static_cast<long>(F) * (D + kHeadCols), groups, F + kHeadCols, F + kHeadCols};
+    products.launch(st);
     return hipGetLastError() == hipSuccess ? ARTAB_OK : ARTAB_ERR_LAUNCH;
 }
 
@@ -368,6 +461,40 @@ int artab_train_embed_backward(const artab_train_embed_args *a, void *stream) {
     if (artab::off_16(a->out, a->xy, a->grads, a->scratch)) return ARTAB_ERR_BAD_STRIDE;
     hipStream_t st = static_cast<hipStream_t>(stream);
     return a->D == 128 ? artab::embed_backward<128>(*a, st) : artab::embed_backward<256>(*a, st);
+}
+
+size_t artab_train_head_saved_bytes(const artab_train_head_args *a) {
+    if (!artab::head_supported(a)) return 0;
+    artab_train_head_args b = *a;
+    b.saved = nullptr;
+    return artab::head_saved(b).bytes;
+}
+size_t artab_train_head_scratch_bytes(const artab_train_head_args *a) {
+    if (!artab::head_supported(a)) return 0;
+    artab_train_head_args b = *a;
+    b.scratch = nullptr;
+    return artab::head_scratch(b).bytes;
+}
+int artab_train_head_forward(const artab_train_head_args *a, void *stream) {
+    if (!artab::head_supported(a)) return ARTAB_ERR_UNSUPPORTED;
+    if (!a->z || !a->y || !a->w1 || !a->b1 || !a->w2 || !a->b2 || !a->mean_bias || !a->std_bias || !a->weight_bias || !a->saved || !a->loss)
+        return ARTAB_ERR_NULL_POINTER;
+    if (artab::off_16(a->z, a->w1, a->b1, a->w2, a->saved)) return ARTAB_ERR_BAD_STRIDE;
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    const bool narrow = artab::head_cols(*a) == 64;
+    if (a->D == 128) return narrow ? artab::head_forward<128, 64>(*a, st) : artab::head_forward<128, 128>(*a, st);
+    return narrow ? artab::head_forward<256, 64>(*a, st) : artab::head_forward<256, 128>(*a, st);
+}
+int artab_train_head_backward(const artab_train_head_args *a, void *stream) {
+    if (!artab::head_supported(a)) return ARTAB_ERR_UNSUPPORTED;
+    if (!a->z || !a->y || !a->w1 || !a->b1 || !a->w2 || !a->b2 || !a->mean_bias || !a->std_bias || !a->weight_bias || !a->saved || !a->dloss ||
+        !a->dz || !a->grads || !a->scratch)
+        return ARTAB_ERR_NULL_POINTER;
+    if (artab::off_16(a->z, a->w1, a->b1, a->w2, a->saved, a->dz, a->grads, a->scratch)) return ARTAB_ERR_BAD_STRIDE;
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    const bool narrow = artab::head_cols(*a) == 64;
+    if (a->D == 128) return narrow ? artab::head_backward<128, 64>(*a, st) : artab::head_backward<128, 128>(*a, st);
+    return narrow ? artab::head_backward<256, 64>(*a, st) : artab::head_backward<256, 128>(*a, st);
 }
 
 size_t artab_train_saved_bytes(const artab_train_args *a) {

@@ -27,7 +27,7 @@ from .attention import DenseMask, MultiheadAttention, RowMask
 from .glue import add_layer_norm, bias_gelu, layer_fusable, layer_post, layer_post_pre, layer_pre, pack_weight
 
 from .live import Methods, Prepared, Sources, capturing, plain_modules, walk
-from .training import embed_rows, layer_stack, layer_stack_supported
+from .training import embed_rows, head_loss, layer_stack, layer_stack_supported
 
 __all__ = ["Embedder", "TwoStageTransformerLayer", "TwoStageTransformer", "MixtureGaussianHead", "ARTabPFN"]
 
@@ -369,6 +369,10 @@ class ARTabPFN(nn.Module):
             z_target = z[:, Nc + Nb:, 0, :]
         if y_target is not None and y_target.dim() == 2:
             y_target = y_target.unsqueeze(-1)
+        if y_target is not None and torch.is_grad_enabled() and _head_as_defined(self.head):
+            loss = head_loss(self.head, z_target, y_target)
+            if loss is not None:
+                return loss
         loss, _, _, _ = self.head(z_target, y_target)
         return loss
 
@@ -415,12 +419,18 @@ class ARTabPFN(nn.Module):
 _EMBEDDER_METHODS = Methods(Embedder, "_x", "_y", "_marker", "embed_context", "embed_buffer", "embed_target")
 _BACKBONE_METHODS = Methods(TwoStageTransformer, "forward")
 _LAYER_METHODS = Methods(TwoStageTransformerLayer, "forward", "_forward_recording")
+_HEAD_METHODS = Methods(MixtureGaussianHead, "forward", "_parameterize", "_log_likelihood")
 _ATTENTION_METHODS = Methods(MultiheadAttention, "forward", "split_heads")
 
 
 def _embedder_as_defined(embedder) -> bool:
     modules, _ = walk((embedder,))
     return plain_modules(modules, (Embedder, nn.Linear, nn.Linear, nn.Embedding)) and _EMBEDDER_METHODS.of(embedder)
+
+
+def _head_as_defined(head) -> bool:
+    modules, _ = walk((head,))
+    return plain_modules(modules, (MixtureGaussianHead, nn.Sequential, nn.Linear, nn.GELU, nn.Linear)) and _HEAD_METHODS.of(head)
 
 
 def _backbone_as_defined(backbone) -> bool:

@@ -1,6 +1,7 @@
 """The layer stack of a training step on the device kernels (``artab_train_forward`` / ``_backward``): what
 ``TwoStageTransformer.forward`` and the final norm record under bfloat16 autocast (model.py:100-147, :317-369;
-train.py:289-300), as one differentiable call.
+train.py:289-300), as one differentiable call; the row embeddings in front of it and the mixture head with its loss
+behind it as one each.
 
 The residual stream, the norms and every sum stay float32; products take bfloat16 operands, as autocast's do.
 """
@@ -16,7 +17,7 @@ from . import _lib
 from . import attention_kernels as ak
 from .attention import RowMask
 
-__all__ = ["embed_rows", "layer_stack_supported", "layer_stack"]
+__all__ = ["embed_rows", "layer_stack_supported", "layer_stack", "head_loss"]
 
 # A program that has put callables of its own in their place gets the modules, which call them.
 _attention_calls = (ak.row_mask_attention, ak.row_mask_attention_backward)
@@ -205,3 +206,77 @@ def layer_stack(backbone, x: Tensor, mask: RowMask, first_row: int) -> Tensor:
     The feature attention's q and k projections do not (one key per query: the softmax weight is 1)."""
     params = [p for layer in backbone.layers for p in _layer_params(layer)]
     return _LayerStack.apply(x, backbone, mask, first_row, *params, backbone.norm.weight, backbone.norm.bias)
+
+
+class _HeadLoss(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, z, y, head, *params):
+        lib = _lib.load()
+        a = _lib.ArtabTrainHeadArgs()
+        a.rows, a.D, a.F, a.K, a.std_min = z.shape[0] * z.shape[1], z.shape[2], params[0].shape[0], params[4].shape[0], head.std_min
+        saved = torch.empty(lib.artab_train_head_saved_bytes(ctypes.byref(a)), device=z.device, dtype=torch.uint8)
+        loss = torch.empty((), device=z.device, dtype=torch.float32)
+        ctx.args, ctx.head = _lib.ArtabTrainHeadArgs.from_buffer_copy(a), head  # (sizes and constants only)
+        _head_pointers(a, z, y, params, saved)
+        a.loss = loss.data_ptr()
+        _lib.check(lib.artab_train_head_forward(ctypes.byref(a), _lib.current_stream(z.device)))
+        ctx.save_for_backward(z, y, saved, *params)
+        return loss
+
+    @staticmethod
+    def backward(ctx, dloss):
+        lib = _lib.load()
+        z, y, saved, *params = ctx.saved_tensors  # (raises if one of them was changed in place since)
+        if torch.is_grad_enabled():  # (create_graph: gradients that can be differentiated again)
+            wanted = [t for t in (z, *params) if t.requires_grad]
+            with torch.autocast("cuda", torch.bfloat16):
+                loss = torch.func.functional_call(ctx.head, dict(zip(_HEAD_PARAMETERS, params)), (z, y))[0]
+            grads = iter(torch.autograd.grad(loss, wanted, dloss, create_graph=True))
+            dz, *dparams = (next(grads) if t.requires_grad else None for t in (z, *params))
+            return (dz, None, None, *dparams)
+        a = _lib.ArtabTrainHeadArgs.from_buffer_copy(ctx.args)
+        D, F, K = a.D, a.F, a.K
+        if not (_f32(z.device, (z, y), (z.shape, y.shape)) and z.numel() == a.rows * D and y.numel() == a.rows
+                and saved.data_ptr() % 16 == 0 and _f32(z.device, params, _head_shapes(D, F, K))):
+            raise RuntimeError("a parameter of the head has another size or type than in the forward pass")
+        dloss = dloss.float().contiguous()
+        _head_pointers(a, z, y, params, saved)
+        scratch = torch.empty(lib.artab_train_head_scratch_bytes(ctypes.byref(a)), device=z.device, dtype=torch.uint8)
+        dz = torch.empty_like(z)
+        grads = torch.empty(F * D + 128 * F + F + 128, device=z.device, dtype=torch.float32)
+        a.dloss, a.dz, a.grads, a.scratch = dloss.data_ptr(), dz.data_ptr(), grads.data_ptr(), scratch.data_ptr()
+        _lib.check(lib.artab_train_head_backward(ctypes.byref(a), _lib.current_stream(z.device)))
+        w1, w2, b1, raw = grads.split((F * D, 128 * F, F, 128))
+        per_component = raw[: 3 * K].view(K, 3).t().contiguous()  # a bias added behind b_2 has b_2's gradient
+        return (dz, None, None, w1.view(F, D), b1, w2[: 3 * K * F].view(3 * K, F), raw[: 3 * K], *per_component)
+
+
+_HEAD_PARAMETERS = ("head.0.weight", "head.0.bias", "head.2.weight", "head.2.bias", "mean_bias", "std_bias", "weight_bias")
+
+
+def _head_shapes(D: int, F: int, K: int):
+    return ((F, D), (F,), (3 * K, F), (3 * K,), (K,), (K,), (K,))
+
+
+def _head_pointers(a, z: Tensor, y: Tensor, params, saved: Tensor):
+    for name, t in zip(("z", "y", "w1", "b1", "w2", "b2", "mean_bias", "std_bias", "weight_bias", "saved"), (z, y, *params, saved)):
+        setattr(a, name, t.data_ptr())
+
+
+def head_loss(head, z: Tensor, y: Tensor):
+    """The loss of ``MixtureGaussianHead.forward(z, y)`` for ``z [B,T,D]``, ``y [B,T,1]`` under bfloat16 autocast,
+    differentiable in ``z`` and the head's parameters, or None where the kernels do not apply (the data itself wants
+    gradients, types or sizes they are not built for)."""
+    one, two = head.head[0], head.head[2]
+    params = (one.weight, one.bias, two.weight, two.bias, head.mean_bias, head.std_bias, head.weight_bias)
+    F, K = one.out_features, head.num_components
+    if not (torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") == torch.bfloat16 and torch.is_grad_enabled()
+            and z.is_cuda and z.dtype == torch.float32 and z.dim() == 3 and tuple(y.shape) == (z.shape[0], z.shape[1], 1)
+            and not y.requires_grad and head.dim_y == 1 and isinstance(K, int) and isinstance(head.std_min, float)
+            and z.shape[2] in (128, 256) and F == 256 and 1 <= 3 * K <= 128 and 1 <= z.shape[0] * z.shape[1] < 2 ** 30
+            and (z.requires_grad or any(p.requires_grad for p in params))):
+        return None
+    y = y.contiguous()
+    if not (type(z) is Tensor and z.is_contiguous() and z.data_ptr() % 16 == 0 and type(y) is Tensor and y.dtype == torch.float32 and y.device == z.device and _f32(z.device, params, _head_shapes(z.shape[2], F, K))):
+        return None
+    return _HeadLoss.apply(z, y, head, *params)

@@ -560,6 +560,30 @@ int artab_train_embed(const artab_train_embed_args *args, void *stream);
 int artab_train_embed_backward(const artab_train_embed_args *args, void *stream);
 
 /*
+ * The mixture head behind that stack and its loss (model.py:150-246), for `rows` rows: gelu(z W_1^T + b_1) W_2^T + b_2
+ * as K x (mean, deviation, weight); loss = the mean negative log-likelihood of y.  D in {128, 256}, F = 256,
+ * 3 K <= 128; anything else: artab_train_head_saved_bytes returns 0.
+ *   forward:  z [rows, D], y [rows] -> loss (one float); fills `saved`, kept by the caller for the backward call.
+ *   backward: dloss (one float) -> dz [rows, D] and `grads` (float32): dW_1 [F, D], dW_2 [128, F] (zero past row 3 K),
+ *             db_1 [F], db_2 [128] (entries 3 k + 0, 1, 2 are also those of the three biases of component k).
+ */
+typedef struct artab_train_head_args {
+    int rows, D, F, K;
+    float std_min;
+    const float *z, *y;
+    const float *w1, *b1, *w2, *b2, *mean_bias, *std_bias, *weight_bias;
+    void *saved;             /* artab_train_head_saved_bytes */
+    float *loss;
+    const float *dloss;
+    float *dz, *grads;
+    void *scratch;           /* artab_train_head_scratch_bytes, backward only */
+} artab_train_head_args;
+size_t artab_train_head_saved_bytes(const artab_train_head_args *args);
+size_t artab_train_head_scratch_bytes(const artab_train_head_args *args);
+int artab_train_head_forward(const artab_train_head_args *args, void *stream);
+int artab_train_head_backward(const artab_train_head_args *args, void *stream);
+
+/*
  * A pass through the whole layer stack, issued by one call: the first layer's artab_layer_pre, then per layer
  * the row attention and artab_layer_post_pre (artab_layer_post behind the last), with the results those give.
  *   num_targets == 0  prefill (inference.py:143-223): dense attention over the N rows, whose K and V go to rows
