@@ -208,13 +208,6 @@ struct BackwardTile {
     static constexpr int BLOCK = 32 * 8 + 32;  // elements from one 8-column block to the next
     static constexpr int SIZE = CPR * BLOCK;
     static_assert(SIZE <= 32 * PAD, "a tile fits the array of the padded form");
-    // (every thread loads, without a lane mask: threads beyond the tile's pieces re-read one of
-    // them and never store it.  A masked load merged with zeros makes the compiler wait for the
-    // load where it is issued, and the prefetch of the next tile would hide nothing.)
-    static __device__ __forceinline__ u32x4 fetch(const View &src, long b, long h, int row0, int R, int tid) {
-        const int piece = tid % PIECES;
-        return *reinterpret_cast<const u32x4 *>(view_row<T>(src, b, h, min(row0 + piece / CPR, R - 1)) + 8 * (piece % CPR));
-    }
     static __device__ __forceinline__ void stash(T *tile, int tid, const u32x4 &raw) {
         const int row = tid / CPR, piece = tid % CPR;
         if (tid < PIECES) *reinterpret_cast<u32x4 *>(tile + piece * BLOCK + row * 8) = raw;
@@ -237,6 +230,45 @@ struct BackwardTile {
         typedef short s16x8 __attribute__((ext_vector_type(8)));
         s16x8 both = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
         return __builtin_bit_cast(typename MfmaOps<T>::vec, both);
+    }
+};
+
+// The two tensors whose tiles a workgroup walks, as its threads fetch and stash them: at head_dim 32 half of the threads
+// take each tensor's pieces, at 64 every thread one of either.
+template <typename T, int DH>
+struct BackwardStager {
+    typedef BackwardTile<T, DH> Tile;
+    static constexpr int THREADS = 64 * kBackwardWaves, LOADS = 2 * Tile::PIECES / THREADS;
+    static_assert(LOADS == 1 || LOADS == 2, "pieces of two tiles over the workgroup");
+    static constexpr int SIZE = 32 * Tile::PAD;  // from tile to tile in LDS: [slot][tensor]
+    const T *next[LOADS];  // this thread's piece of the next tile
+    T *at[LOADS];          // and its place in slot 0
+    long stride[LOADS];    // from row to row
+    u32x4 raw[LOADS];
+    // (wave: a scalar, so that which tensor a wavefront reads is one too)
+    __device__ __forceinline__ BackwardStager(const View &first, const View &second, long b, long h, int tile, T *lds, int wave, int lane) {
+#pragma unroll
+        for (int x = 0; x < LOADS; ++x) {
+            const int i = 64 * wave + THREADS * x, piece = i % Tile::PIECES + lane;
+            const View src = i < Tile::PIECES ? first : second;
+            next[x] = view_row<T>(src, b, h, 32 * tile + piece / Tile::CPR) + 8 * (piece % Tile::CPR);
+            at[x] = lds + (i < Tile::PIECES ? 0 : SIZE) + (piece % Tile::CPR) * Tile::BLOCK + (piece / Tile::CPR) * 8;
+            stride[x] = src.sn;
+        }
+    }
+    // tile t, one further than the call before; rows past the end re-read the last one
+    __device__ __forceinline__ void fetch(int t, int R, int wave, int lane) {
+#pragma unroll
+        for (int x = 0; x < LOADS; ++x) {
+            const T *p = next[x];
+            if (32 * t + 32 > R) p -= max(0, 32 * t + ((64 * wave + THREADS * x) % Tile::PIECES + opaque(lane)) / Tile::CPR - (R - 1)) * stride[x];
+            raw[x] = *reinterpret_cast<const u32x4 *>(p);
+            next[x] += 32 * stride[x];
+        }
+    }
+    __device__ __forceinline__ void stash(int slot) const {
+#pragma unroll
+        for (int x = 0; x < LOADS; ++x) *reinterpret_cast<u32x4 *>(at[x] + slot * (2 * SIZE)) = raw[x];
     }
 };
 
@@ -274,17 +306,20 @@ __device__ __forceinline__ void backward_store_rows(T *tile, const f32x16 (&acc)
     __builtin_amdgcn_wave_barrier();
 }
 
-// (head_dim 32 is held to 128 registers, four wavefronts per SIMD: measured 6 % faster than the
-// 130 the compiler takes unconstrained; the dK/dV kernel loses 12 % when held to the same)
+// Bound by vector instructions and a serial chain per tile.  Loops by two tiles, so that the LDS slot is a constant and
+// the operands' addresses are the lane's with an offset in the instruction; half of the threads stage each tensor; the
+// products start at -lse and -delta.  64 x 4 pairs of 1544 rows, 1032 keys: dQ 136 -> 117 us, dK/dV 211 -> 172
+// (with the clock of one sitting), head_dim 64, 512 x 1028 rows, 516 keys: 186 -> 180, 298 -> 272.
+// (head_dim 32 is held to 128 registers, four wavefronts per SIMD: 122 us with three)
 template <typename T, int DH>
-__global__ __launch_bounds__(kBackwardWaves * 64) __attribute__((amdgpu_waves_per_eu(DH == 32 ? 4 : 2)))
+__global__ __launch_bounds__(kBackwardWaves * 64) __attribute__((amdgpu_waves_per_eu(DH == 32 ? 4 : 3)))
 void backward_dq_mfma_kernel(BackwardParams P) {
     typedef MfmaOps<T> Ops;
     typedef typename Ops::vec vec;
     typedef BackwardTile<T, DH> Tile;
     constexpr int KS = DH / 16, DB = DH / 32;
-    __shared__ __attribute__((aligned(16))) T k_tiles[2][32 * Tile::PAD];  // two tiles in turn: one barrier per tile
-    __shared__ __attribute__((aligned(16))) T v_tiles[2][32 * Tile::PAD];
+    constexpr int SIZE = BackwardStager<T, DH>::SIZE;
+    __shared__ __attribute__((aligned(16))) T lds[4 * SIZE];  // K and V tiles, two of each in turn: one barrier per tile
 
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, c = lane & 31, hb = lane >> 5;
     const int blocks = (P.R + kBackwardRows - 1) / kBackwardRows;
@@ -321,41 +356,38 @@ void backward_dq_mfma_kernel(BackwardParams P) {
     const int vis_end = backward_vis_end(P, qi);
     if (qi < P.R && hb == 0) P.delta[stat] = delta;
 
-    f32x16 acc[DB];
+    // where the products start, so that they leave log2 P and dP - delta: at head_dim 32 kept as they are over the walk
+    // (at 64 those 32 registers are a wavefront less per SIMD: 182 us -> 195 at 64 x 8 pairs of 1028 rows)
+    constexpr bool KEPT = DH == 32;
+    f32x16 acc[DB], minus_lse2, minus_delta;
 #pragma unroll
-    for (int db = 0; db < DB; ++db)
+    for (int v = 0; v < 16; ++v) {
 #pragma unroll
-        for (int v = 0; v < 16; ++v) acc[db][v] = 0.f;
+        for (int db = 0; db < DB; ++db) acc[db][v] = 0.f;
+        minus_lse2[v] = KEPT ? -lse2 : 0.f;
+        minus_delta[v] = -delta;
+    }
+    if constexpr (KEPT) asm volatile("" : "+v"(minus_lse2), "+v"(minus_delta));
+    const float left = KEPT ? 0.f : lse2;
 
     // every workgroup walks the keys anybody can see; what its own rows do not see is masked
     const int n_tiles = (P.Nc + P.Nb + 31) / 32;
     // tile kt + 1 goes to LDS at the start of iteration kt (it was requested one iteration earlier), tile
     // kt + 2 is requested then: one barrier per tile, a whole iteration to cover the memory round trip
-    u32x4 k_raw = Tile::fetch(P.k, b, h, 0, P.R, tid), v_raw = Tile::fetch(P.v, b, h, 0, P.R, tid);
-    Tile::stash(k_tiles[0], tid, k_raw);
-    Tile::stash(v_tiles[0], tid, v_raw);
-    if (n_tiles > 1) {
-        k_raw = Tile::fetch(P.k, b, h, 32, P.R, tid);
-        v_raw = Tile::fetch(P.v, b, h, 32, P.R, tid);
-    }
-    for (int kt = 0; kt < n_tiles; ++kt) {
+    BackwardStager<T, DH> tiles(P.k, P.v, b, h, 0, lds, wave, lane);
+    tiles.fetch(0, P.R, wave, lane);
+    tiles.stash(0);
+    if (n_tiles > 1) tiles.fetch(1, P.R, wave, lane);
+    // (the slot a constant: LDS addresses are then the lane's and an offset in the instruction)
+    auto walk = [&](auto slot_tag, int kt) {
+        constexpr int slot = decltype(slot_tag)::value;
         __syncthreads();  // tile kt is complete; everyone has finished reading the other one
-        const T *k_tile = k_tiles[kt & 1], *v_tile = v_tiles[kt & 1];
+        const T *const k_tile = lds + slot * (2 * SIZE), *const v_tile = k_tile + SIZE;
         if (kt + 1 < n_tiles) {
-            Tile::stash(k_tiles[(kt + 1) & 1], tid, k_raw);
-            Tile::stash(v_tiles[(kt + 1) & 1], tid, v_raw);
-            if (kt + 2 < n_tiles) {
-                k_raw = Tile::fetch(P.k, b, h, 32 * (kt + 2), P.R, tid);
-                v_raw = Tile::fetch(P.v, b, h, 32 * (kt + 2), P.R, tid);
-            }
+            tiles.stash(slot ^ 1);
+            if (kt + 2 < n_tiles) tiles.fetch(kt + 2, P.R, wave, lane);
         }
-        f32x16 s, dp;  // dp starts at -delta: the product leaves dP - delta.  (Starting s at -lse2
-                       // as well costs 16 more registers than four wavefronts per SIMD leave: measured slower.)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-            s[v] = 0.f;
-            dp[v] = -delta;
-        }
+        f32x16 s = minus_lse2, dp = minus_delta;
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
             s = Ops::mma(Tile::row_operand(k_tile, c, hb, ks), qf[ks], s);
@@ -369,9 +401,10 @@ void backward_dq_mfma_kernel(BackwardParams P) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     const int v = 8 * t + 2 * e;
-                    dsb[t][e] = pack2<T>(fast_exp2(s[v] - lse2) * dp[v], fast_exp2(s[v + 1] - lse2) * dp[v + 1]);
+                    dsb[t][e] = pack2<T>(fast_exp2(KEPT ? s[v] : s[v] - left) * dp[v], fast_exp2(KEPT ? s[v + 1] : s[v + 1] - left) * dp[v + 1]);
                 }
         } else {
+            const int end = vis_end - 32 * kt;
 #pragma unroll
             for (int t = 0; t < 2; ++t)
 #pragma unroll
@@ -380,8 +413,8 @@ void backward_dq_mfma_kernel(BackwardParams P) {
 #pragma unroll
                     for (int x = 0; x < 2; ++x) {
                         const int v = 8 * t + 2 * e + x;
-                        const bool vis = 32 * kt + 8 * (v >> 2) + 4 * hb + (v & 3) < vis_end;
-                        ds[x] = vis ? fast_exp2(s[v] - lse2) * dp[v] : 0.f;
+                        const bool vis = 8 * (v >> 2) + 4 * hb + (v & 3) < end;
+                        ds[x] = vis ? fast_exp2(KEPT ? s[v] : s[v] - left) * dp[v] : 0.f;
                     }
                     dsb[t][e] = pack2<T>(ds[0], ds[1]);
                 }
@@ -391,11 +424,14 @@ void backward_dq_mfma_kernel(BackwardParams P) {
 #pragma unroll
             for (int t = 0; t < 2; ++t)
                 acc[db] = Ops::mma(Tile::col_operand(k_tile, lane, t, db), __builtin_bit_cast(vec, dsb[t]), acc[db]);
+    };
+    for (int kt = 0; kt < n_tiles; kt += 2) {
+        walk(std::integral_constant<int, 0>{}, kt);
+        if (kt + 1 < n_tiles) walk(std::integral_constant<int, 1>{}, kt + 1);
     }
 
     __syncthreads();  // the tiles are free: one per wavefront stages its rows
-    T *stage = wave < 2 ? k_tiles[wave] : v_tiles[wave - 2];
-    backward_store_rows<T, DH>(stage, acc, P.scale, P.dq, b, h, blk * kBackwardRows + 32 * wave, P.R, lane);
+    backward_store_rows<T, DH>(lds + wave * SIZE, acc, P.scale, P.dq, b, h, blk * kBackwardRows + 32 * wave, P.R, lane);
 }
 
 template <typename T, int DH>
@@ -404,8 +440,8 @@ __global__ __launch_bounds__(kBackwardWaves * 64) void backward_dkv_mfma_kernel(
     typedef typename Ops::vec vec;
     typedef BackwardTile<T, DH> Tile;
     constexpr int KS = DH / 16, DB = DH / 32;
-    __shared__ __attribute__((aligned(16))) T q_tiles[2][32 * Tile::PAD];  // two tiles in turn: one barrier per tile
-    __shared__ __attribute__((aligned(16))) T g_tiles[2][32 * Tile::PAD];
+    constexpr int SIZE = BackwardStager<T, DH>::SIZE;
+    __shared__ __attribute__((aligned(16))) T lds[4 * SIZE];  // Q and dO tiles, two of each in turn: one barrier per tile
     __shared__ __attribute__((aligned(16))) float lse2_t[2][32];
     __shared__ __attribute__((aligned(16))) float delta_t[2][32];
     __shared__ __attribute__((aligned(16))) int end_t[2][32];
@@ -463,44 +499,48 @@ __global__ __launch_bounds__(kBackwardWaves * 64) void backward_dkv_mfma_kernel(
     // rows from the first buffer row on otherwise.
     const int t_end = (P.R + 31) / 32;
     const int t_begin = key0 < P.Nc ? 0 : P.Nc / 32;
-    u32x4 q_raw = {0u, 0u, 0u, 0u}, g_raw = {0u, 0u, 0u, 0u};
+    BackwardStager<T, DH> tiles(P.q, P.dout, b, h, t_begin, lds, wave, lane);
+    // the rows' statistics: by the first wavefront
     float st_lse2 = 0.f, st_delta = 0.f;
-    int st_end = 0;
     auto fetch = [&](int qt) {
-        q_raw = Tile::fetch(P.q, b, h, 32 * qt, P.R, tid);
-        g_raw = Tile::fetch(P.dout, b, h, 32 * qt, P.R, tid);
-        {   // (all threads, as above; threads 32.. hold copies that are never stored)
-            const int i = 32 * qt + (tid & 31);
+        tiles.fetch(qt, P.R, wave, lane);
+        if (wave == 0) {
+            const long i = stat0 + min(32 * qt + (lane & 31), P.R - 1);
             // (as loaded: any arithmetic on them here would wait for the loads, and with them for
             // the tile requested just before; they are negated and scaled when they go to LDS)
-            st_lse2 = P.lse[stat0 + min(i, P.R - 1)];
-            st_delta = P.delta[stat0 + min(i, P.R - 1)];
-            st_end = backward_vis_end(P, i);
+            st_lse2 = P.lse[i];
+            st_delta = P.delta[i];
         }
     };
-    auto stash = [&](int slot) {
-        Tile::stash(q_tiles[slot], tid, q_raw);
-        Tile::stash(g_tiles[slot], tid, g_raw);
-        if (tid < 32) {
-            lse2_t[slot][tid] = -st_lse2 * kLog2e;  // negated: the accumulators start from them
-            delta_t[slot][tid] = -st_delta;
-            end_t[slot][tid] = st_end;
+    auto stash = [&](int slot, int qt) {
+        tiles.stash(slot);
+        if (wave == 0) {
+            if (lane < 32) {
+                lse2_t[slot][lane] = -st_lse2 * kLog2e;  // negated: the accumulators start from them
+                delta_t[slot][lane] = -st_delta;
+            }
+            // (the key limit takes a division: not for rows of which every one sees the context alone)
+            if (32 * qt + 32 <= P.Nc) {
+                if (lane < 32) end_t[slot][lane] = P.Nc;
+            } else if (lane < 32) {
+                end_t[slot][lane] = backward_vis_end(P, 32 * qt + lane);
+            }
         }
     };
     // as in the dQ kernel: tile qt + 1 goes to LDS at the start of iteration qt, tile qt + 2 is requested then
     if (t_begin < t_end) {
         fetch(t_begin);
-        stash(0);
+        stash(0, t_begin);
         if (t_begin + 1 < t_end) fetch(t_begin + 1);
     }
-    for (int qt = t_begin; qt < t_end; ++qt) {
+    auto walk = [&](auto slot_tag, int qt) {  // (the slot a constant, as in the dQ kernel)
+        constexpr int slot = decltype(slot_tag)::value;
         __syncthreads();
-        const int slot = (qt - t_begin) & 1;
-        const T *q_tile = q_tiles[slot], *g_tile = g_tiles[slot];
+        const T *const q_tile = lds + slot * (2 * SIZE), *const g_tile = q_tile + SIZE;
         const float *lse2_s = lse2_t[slot], *delta_s = delta_t[slot];
         const int *end_s = end_t[slot];
         if (qt + 1 < t_end) {
-            stash(slot ^ 1);
+            stash(slot ^ 1, qt + 1);
             if (qt + 2 < t_end) fetch(qt + 2);
         }
         // rows of the accumulators are queries 8g + 4hb + r of the tile: the accumulators start at
@@ -567,10 +607,14 @@ __global__ __launch_bounds__(kBackwardWaves * 64) void backward_dkv_mfma_kernel(
                 acc_v[db] = Ops::mma(Tile::col_operand(g_tile, lane, t, db), __builtin_bit_cast(vec, pb[t]), acc_v[db]);
                 acc_k[db] = Ops::mma(Tile::col_operand(q_tile, lane, t, db), __builtin_bit_cast(vec, dsb[t]), acc_k[db]);
             }
+    };
+    for (int qt = t_begin; qt < t_end; qt += 2) {
+        walk(std::integral_constant<int, 0>{}, qt);
+        if (qt + 1 < t_end) walk(std::integral_constant<int, 1>{}, qt + 1);
     }
 
     __syncthreads();  // the tiles are free: one per wavefront stages its rows
-    T *stage = wave < 2 ? q_tiles[wave] : g_tiles[wave - 2];
+    T *const stage = lds + wave * SIZE;
     backward_store_rows<T, DH>(stage, acc_k, P.scale, P.dk, b, h, key0 + 32 * wave, P.R, lane);
     backward_store_rows<T, DH>(stage, acc_v, 1.f, P.dv, b, h, key0 + 32 * wave, P.R, lane);
 }

@@ -32,20 +32,22 @@ static hipError_t launch_backward_pair(const BackwardParams &P, hipStream_t stre
 template <typename T>
 static hipError_t launch_backward_mfma(const BackwardParams &P, hipStream_t stream) {
     // One workgroup per pair (backward_pair_kernel) while the keys that anybody sees fit it.  It stays on one compute
-    // unit: with up to 128 keys it is the faster form at any number of pairs (head_dim 32, 96 keys, 608 rows: 22.6 ->
-    // 18.5 us for 4 pairs, 49 -> 24 for 256); with more, the two kernels' many workgroups win while pairs are few (256
-    // keys, 768 rows: 29.8 against 31.9 at 32 pairs, 33.5 at 64, 41.6 against 35.2 at 128; 512 keys, 1024 rows: 52
-    // against 70 at 64, 91 -> 73 at 128, 283 -> 171 at 512; head_dim 64, 256 keys: 46 against 58 at 64, 63 -> 60 at 128).
-    // More pairs than compute units: two workgroups of half the groups to a unit (300 pairs, 96 keys: 53 -> 33).
-    const long pairs = static_cast<long>(P.H) * P.B;
+    // unit: with up to 128 keys it is the faster form at any number of pairs (head_dim 32, 96 keys, 608 rows: 21.5 against
+    // 18.7 us for 16 pairs, 45.7 against 24.3 for 256); with more, the two kernels' many workgroups win while pairs are few
+    // (256 keys, 768 rows: 31.7 against 33.2 at 64 pairs, 36.1 against 34.2 at 96; 512 keys, 1024 rows: 59 against 71 at
+    // 96, 106 against 77 at 192; head_dim 64, 256 keys: 58 against 61 at 128, 71 against 64 at 192).  Where pairs need
+    // one more round of the chip's 256 compute units, that round has to be half full: 300 pairs of 512 keys 156
+    // against 146 us.  Up to 128 keys, two workgroups of half the groups to a unit then (300 pairs, 96 keys: 52 against 32).
+    const long pairs = static_cast<long>(P.H) * P.B, rounds = (pairs + 255) / 256;
     const int keys = P.Nc + P.Nb;
+    const bool filled = pairs >= 150 * rounds;
     if (P.Dh == 32) {
         if (keys <= 128) return pairs <= 256 ? launch_backward_pair<T, 32, 4, 4>(P, stream) : launch_backward_pair<T, 32, 4, 2>(P, stream);
-        if (keys <= 256 && pairs >= 64) return launch_backward_pair<T, 32, 8, 2>(P, stream);
-        if (keys <= 512 && pairs >= 128) return launch_backward_pair<T, 32, 16, 1>(P, stream);
+        if (keys <= 256 && (filled || (pairs >= 80 && rounds == 1))) return launch_backward_pair<T, 32, 8, 2>(P, stream);
+        if (keys <= 512 && filled) return launch_backward_pair<T, 32, 16, 1>(P, stream);
     } else {
         if (keys <= 128) return launch_backward_pair<T, 64, 4, 2>(P, stream);
-        if (keys <= 256 && pairs >= 128) return launch_backward_pair<T, 64, 8, 1>(P, stream);
+        if (keys <= 256 && filled) return launch_backward_pair<T, 64, 8, 1>(P, stream);
     }
     const long blocks = (P.R + kBackwardRows - 1) / kBackwardRows;
     const dim3 grid(static_cast<unsigned>(blocks * P.H * P.B)), block(kBackwardWaves * 64);

@@ -18,14 +18,15 @@ pytestmark = pytest.mark.gpu
         (3, 4, 32, 64, 32, 512, 8),    # the training configuration: targets that attend and targets that do not
         (1, 4, 32, 96, 32, 70, 1),     # all 128 keys, a ragged last tile
         (65, 4, 32, 33, 8, 100, 2),    # more pairs than compute units: two groups
-        (16, 4, 32, 100, 29, 70, 2),   # 129 keys: eight wavefronts, the keys of a dQ piece dealt over two
-        (16, 4, 32, 240, 16, 33, 2),   # all 256
+        (20, 4, 32, 100, 29, 70, 2),   # 129 keys: eight wavefronts, the keys of a dQ piece dealt over two
+        (20, 4, 32, 240, 16, 33, 2),   # all 256
         (8, 4, 32, 240, 16, 33, 2),    # as many keys, fewer pairs: the two launches
-        (32, 4, 32, 230, 27, 90, 1),   # 257 keys: sixteen wavefronts, the keys of a dQ piece dealt over four
-        (32, 4, 32, 500, 12, 20, 1),   # all 512
-        (32, 4, 32, 500, 13, 20, 1),   # one more: the two launches
+        (38, 4, 32, 230, 27, 90, 1),   # 257 keys: sixteen wavefronts, the keys of a dQ piece dealt over four
+        (38, 4, 32, 500, 12, 20, 1),   # all 512
+        (38, 4, 32, 500, 13, 20, 1),   # one more: the two launches
         (2, 3, 64, 65, 16, 65, 2),     # head_dim 64
-        (32, 4, 64, 200, 56, 40, 0),   # all 256, no target attends
+        (38, 4, 64, 200, 56, 40, 0),
+        (65, 4, 32, 240, 16, 33, 2),   # a second round of four pairs: the two launches   # all 256, no target attends
     ],
 )
 def test_gradients_match_the_float32_kernels(device, dtype, B, H, D, Nc, Nb, T, A):
