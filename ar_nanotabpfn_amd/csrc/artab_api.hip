@@ -145,23 +145,44 @@ struct FlashPlan {
     int G;
 };
 
-// Tile planning.  Query tiles of 256 rows (two 32-row blocks per wavefront) give the
-// best MFMA-per-LDS-byte ratio; smaller tiles are used only when a group has fewer
-// rows (no wavefronts of pure padding) or, for the unsplittable phases, when the
-// grid would not cover the chip.  Missing parallelism on long contexts comes from
+// Query rows per workgroup where the keys are not split (prefill, teacher forcing, the training row mask): 256 (head_dim
+// 32: eight wavefronts), 128 or 64.  A long key range takes 10 % less per row with 256 rows, a short one less with 128, and
+// rounding the rows up to whole tiles costs what it adds: weighed as p(256) (N + 100) against p(128) (N + 50) of N keys and
+// p rows, with the measured 1.1 between the two (f16, whose pass keeps a running maximum, 1.06 and less of a start).  Tiles
+// of 64 rows where even they do not fill the chip.  Over 504 calls of 40 to 2000 keys, 40 to 2000 rows, 32 to 512 pairs
+// the choice is within 1 % of the best of the three on average at both head_dims, at most 9 % above it; by rows alone
+// (256 while there are 512 workgroups) it was 4 to 6 % above at head_dim 32 and 6 to 18 at 64.  us: 64 x 4 pairs, 608 rows, 96 keys
+// 22.4 -> 17.1; 616 rows, 316 keys 34 -> 25; 64 x 8, 516 rows, 116 keys of head_dim 64 72 -> 50; 32 x 8, 80 rows, 1040 keys 22 -> 17.
+static int unsliced_tile(long G, long pairs, int Nc, int Dh, bool bf16) {
+    const auto padded = [&](int bm) { return static_cast<double>((G + bm - 1) / bm * bm); };
+    const auto wgs = [&](int bm) { return (G + bm - 1) / bm * pairs; };
+    if (Dh == 32 && wgs(256) >= (bf16 ? 256 : 512) &&
+        padded(256) * (Nc + 100) < padded(128) * (bf16 ? 1.1 * (Nc + 50) : 1.06 * (Nc + 100)))
+        return 256;
+    return (G <= 64 && Nc <= 300) || (wgs(64) <= 256 && Nc <= 256) ? 64 : 128;
+}
+
+// Tile planning.  Over a split context query tiles of 256 rows (head_dim 32: eight wavefronts of the lean pass, and what the
+// streaming buffer pass runs beside) or 128 (head_dim 64: 1024 x 8 rows, 16384 keys 65 -> 59 us with 128 instead of 256, 4096 x 8
+// of 4096 keys 72 -> 60, f16 96 -> 73: two wavefronts per SIMD of one 32-row block instead of one of two); smaller tiles only
+// when a group has fewer rows (no wavefronts of pure padding).  Missing parallelism on long contexts comes from
 // slicing the context (each slice returns a normalised partial + log-sum-exp).
 // kTuneBM / kTuneSplit override the choice.
-static FlashPlan plan_flash(int B, int H, int Lq, int Nc, int Dh, bool stacked, bool allow_split) {
+static FlashPlan plan_flash(int B, int H, int Lq, int Nc, int Dh, bool stacked, bool allow_split, bool bf16 = true) {
     FlashPlan pl;
     pl.n_groups = stacked ? 1 : B;
     pl.G = stacked ? B * Lq : Lq;
     auto wgs = [&](int bm) { return static_cast<long>((pl.G + bm - 1) / bm) * pl.n_groups * H; };
-    int bm = Dh == 128 ? 128 : 256;  // head_dim 128: one 32-row block per wavefront (register budget)
+    int bm = Dh == 32 ? 256 : 128;  // (head_dim 128: one 32-row block per wavefront, for its registers)
     while (bm > 64 && pl.G <= bm / 2) bm /= 2;
-    if (!allow_split)
-        while (bm > 64 && wgs(bm) < 512) bm /= 2;
+    if (!allow_split) {
+        if (Dh == 128)
+            while (bm > 64 && wgs(bm) < 512) bm /= 2;
+        else
+            bm = unsliced_tile(pl.G, static_cast<long>(pl.n_groups) * H, Nc, Dh, bf16);
+    }
     const int bm_env = tune(kTuneBM, 0);
-    if ((bm_env == 64 || bm_env == 128 || (bm_env == 256 && Dh != 128))) bm = bm_env;
+    if (bm_env == 64 || bm_env == 128 || (bm_env == 256 && Dh == 32)) bm = bm_env;
     pl.BM = bm;
     pl.tiles_per_group = (pl.G + bm - 1) / bm;
     const long base = wgs(bm);
@@ -208,7 +229,7 @@ static int prefill_slices(int B, int H, int Nc, int Dh) {
         return static_cast<double>((q + 1) / 2) * 5.0 + keys * (17e-3 * (q / 2) + 12e-3 * (q % 2));
     };
     int bm = 256;
-    while (bm > 64 && (Nc + bm - 1) / bm * pairs < 512) bm /= 2;  // as plan_flash cuts the unsliced tiles
+    while (bm > 64 && (Nc + bm - 1) / bm * pairs < 512) bm /= 2;
     double best = bm == 256 ? wide(Nc, tiles)
                             : 4.5 + Nc * (12.5e-3 + 3e-3 * ((Nc + bm - 1) / bm * pairs * (bm / 32) / 1024.0));
     int slices = 1;
@@ -1051,7 +1072,7 @@ int artab_teacher_forcing_attention(const artab_view *q, const artab_view *k_ctx
         P.vec_ok = aligned ? 1 : 0;
         return launch_status(launch_portable_or_f32(P, dtype, impl, false, st), "teacher forcing");
     }
-    FlashPlan pl = plan_flash(B, H, Lq, Nc, Dh, /*stacked=*/false, /*allow_split=*/false);
+    FlashPlan pl = plan_flash(B, H, Lq, Nc, Dh, /*stacked=*/false, /*allow_split=*/false, dtype == ARTAB_BF16);
     FlashParams F;
     memset(&F, 0, sizeof(F));
     F.q = dv(q); F.kc = dv(k_ctx); F.vc = dv(v_ctx); F.kb = dv(k_buf); F.vb = dv(v_buf); F.out = dv(out);
@@ -1105,7 +1126,7 @@ int artab_row_mask_attention(const artab_view *q, const artab_view *k, const art
         P.vec_ok = aligned ? 1 : 0;
         return launch_status(launch_portable_or_f32(P, dtype, impl, false, st), "row-mask attention");
     }
-    FlashPlan pl = plan_flash(B, H, R, Nc, Dh, /*stacked=*/false, /*allow_split=*/false);
+    FlashPlan pl = plan_flash(B, H, R, Nc, Dh, /*stacked=*/false, /*allow_split=*/false, dtype == ARTAB_BF16);
     FlashParams F;
     memset(&F, 0, sizeof(F));
     F.q = dv(q); F.kc = dv(k); F.vc = dv(v); F.kb = kb; F.vb = vb; F.out = dv(out);
@@ -1199,7 +1220,7 @@ static int prefill_impl(const artab_view *q, const artab_view *k, const artab_vi
         return launch_status(e, "prefill (small)");
     }
     const int slices = prefill_slices(B, H, Nc, Dh);
-    FlashPlan pl = plan_flash(B, H, Nc, Nc, Dh, /*stacked=*/false, /*allow_split=*/false);
+    FlashPlan pl = plan_flash(B, H, Nc, Nc, Dh, /*stacked=*/false, /*allow_split=*/false, dtype == ARTAB_BF16);
     if (slices > 1 && workspace && workspace_bytes >= f32_workspace_bytes(rows, Dh, slices) &&
         reinterpret_cast<uintptr_t>(workspace) % 16 == 0) {
         pl.BM = 256;

@@ -93,9 +93,11 @@ static hipError_t launch_flash_bm(const FlashParams &P, int BM, hipStream_t stre
         }
     }
     if constexpr (DH <= 64) {
-        if (BM == 256) {
-            launch_one(flash_kernel<T, DH, 2, 4, kFlashBN>, grid, 256, stream, P);
-            return hipGetLastError();
+        if constexpr (DH == 32) {
+            if (BM == 256) {
+                launch_one(flash_kernel<T, DH, 2, 4, kFlashBN>, grid, 256, stream, P);
+                return hipGetLastError();
+            }
         }
         if (BM == 128 && tune(kTuneNW, 4) == 2) {  // two wavefronts of two query blocks each
             launch_one(flash_kernel<T, DH, 2, 2, kFlashBN>, grid, 128, stream, P);
