@@ -191,6 +191,8 @@ SIGNATURES = {
     "artab_pack_stack_weight_float": (_i, [_p, _p, _i, _i, _p]),
     "artab_layer_stack_scratch_bytes": (_sz, [_p, _i]),
     "artab_layer_stack": (_i, [_p, _i, _p]),
+    "artab_layer_stack_context_scratch_bytes": (_sz, [_p, _p, _i]),
+    "artab_layer_stack_context": (_i, [_p, _p, _i, _p]),
     "artab_prefill_workspace_bytes": (_sz, [_i, _i, _i, _i, _i]),
     "artab_prefill_attention_sliced": (_i, [_VP, _VP, _VP, _VP, _VP, _VP, _i, _i, _i, _i, _i, _f, _i, _p, _sz, _i, _p]),
     "artab_buffer_attention": (_i, [_VP, _VP, _VP, _p, _i64, _i64, _i64, _VP, _p, _i, _i, _i, _i, _i, _f, _i, _p]),

@@ -1672,11 +1672,21 @@ __global__ __launch_bounds__(256) void cache_rows_kernel(CacheRowsParams P) {
 }
 
 namespace {
+// One pass, or a prefill and the teacher-forced pass that reads its caches, layer by layer side by side: the rows of all
+// parts follow each other, so that a layer boundary is one launch for both.
+struct StackParts {
+    const artab_stack_args *part[2];
+    int n;
+    bool caches_only;  // part 0 is a prefill whose rows nobody reads: it ends with the last layer's K and V
+    int64_t rows(int p) const { return static_cast<int64_t>(part[p]->B) * part[p]->N; }
+    int64_t rows() const { return rows(0) + (n > 1 ? rows(1) : 0); }
+};
 struct StackScratch {
     size_t y[2], qkv, attn, prefill, total;
 };
-StackScratch stack_scratch(const artab_stack_args *a, int dtype) {
-    const size_t rows = static_cast<size_t>(a->B) * a->N, e = elem_size(dtype);
+StackScratch stack_scratch(const StackParts &S, int dtype) {
+    const artab_stack_args *a = S.part[0];
+    const size_t rows = S.rows(), e = elem_size(dtype);
     StackScratch s;
     size_t used = 0;
     const auto take = [&](size_t bytes) { const size_t at = used; used += (bytes + 255) / 256 * 256; return at; };
@@ -1716,7 +1726,7 @@ int check_stack(const artab_stack_args *a) {
 }
 // Every pointer of every layer, before anything is launched.  b_2 may be NULL, and b_1 in 16 bits.
 int check_stack_pointers(const artab_stack_args *a, bool f32) {
-    if (misaligned16(a->x) || misaligned16(a->out)) return fail(ARTAB_ERR_BAD_STRIDE, "layer stack: x and out must be 16-byte aligned");
+    if (misaligned16(a->x) || (a->out && misaligned16(a->out))) return fail(ARTAB_ERR_BAD_STRIDE, "layer stack: x and out must be 16-byte aligned");
     for (int l = 0; l < a->n_layers; ++l) {
         const artab_stack_layer &L = a->layers[l];
         const void *required[] = {L.w_fo, L.w_qkv, L.w_o, L.w_1, L.w_2, L.gamma1, L.beta1, L.gamma2, L.beta2, L.gamma3, L.beta3,
@@ -1742,93 +1752,140 @@ int artab_pack_stack_weight_float(const void *w, void *packed, int N, int K, voi
 
 size_t artab_layer_stack_scratch_bytes(const artab_stack_args *args, int dtype) {
     if (check_stack(args) != ARTAB_OK) return 0;
-    return stack_scratch(args, dtype).total;
+    return stack_scratch({{args, nullptr}, 1, false}, dtype).total;
 }
 
-int artab_layer_stack(const artab_stack_args *a, int dtype, void *stream) {
-    ARTAB_TRY(check_stack(a));
+static int stack_pass(const StackParts &S, int dtype, void *stream) {
+    const artab_stack_args *const a = S.part[0];
     const bool f32 = dtype == ARTAB_F32;
-    if (!f32) ARTAB_TRY(check_layer_dtype_rows("layer_stack", dtype, static_cast<int64_t>(a->B) * a->N));
+    const int64_t rows = S.rows(), D = a->D;
+    if (!f32) ARTAB_TRY(check_layer_dtype_rows("layer_stack", dtype, rows));
     if (f32 && !f32_layer_width_ok(a->D, a->F))
         return fail(ARTAB_ERR_UNSUPPORTED, "layer stack in float32: D in {128, 256, 512} and F = 256 (got %d, %d)", a->D, a->F);
-    if (!a->x || !a->out || !a->scratch) return fail(ARTAB_ERR_NULL_POINTER, "layer stack: x, out and scratch are required");
     const int Dh = a->D / a->H, e = elem_size(dtype);
+    for (int p = 0; p < S.n; ++p)
+        if (!S.part[p]->x || !a->scratch || (!S.part[p]->out && !(p == 0 && S.caches_only)))
+            return fail(ARTAB_ERR_NULL_POINTER, "layer stack: x, out and scratch are required");
     if (misaligned16(a->scratch) || Dh * e % 16)
         return fail(ARTAB_ERR_BAD_STRIDE, "layer stack: scratch and heads must be whole 16-byte pieces");
-    ARTAB_TRY(check_stack_pointers(a, f32));
-    const StackScratch s = stack_scratch(a, dtype);
-    char *base = static_cast<char *>(a->scratch);
-    char *qkv = base + s.qkv, *attn = base + s.attn;
-    const int64_t rows = static_cast<int64_t>(a->B) * a->N, D = a->D;
-    const auto head_view = [&](int which) {
-        return artab_view{qkv + which * D * e, a->N * 3 * D, Dh, 3 * D};
-    };
-    const artab_view q = head_view(0), k = head_view(1), v = head_view(2), out = {attn, a->N * D, Dh, D};
+    for (int p = 0; p < S.n; ++p) ARTAB_TRY(check_stack_pointers(S.part[p], f32));
+    const StackScratch s = stack_scratch(S, dtype);
+    char *const base = static_cast<char *>(a->scratch);
+    hipStream_t st = static_cast<hipStream_t>(stream);
     const int64_t cache_h = static_cast<int64_t>(a->cache_rows) * Dh, cache_b = a->own_caches ? a->H * cache_h : 0;
+    const auto first_row = [&](int p) { return p ? S.rows(0) : int64_t{0}; };
     const artab_stack_layer *L = a->layers;
     // Where the layer kernels can, they put keys and values where they belong, and the attention reads them there: no copy
     // of them, and rows of a head that follow each other (in the q/k/v matrix a head's 64 bytes share a line with its
     // neighbour's).  A prefill of several entries with one cache keeps entry 0's and cannot.
-    const bool direct = !f32 && (a->own_caches || (a->num_targets == 0 && a->B == 1)) && rows <= 0x7fffffffL &&
+    const bool direct = S.n == 1 && !f32 && (a->own_caches || (a->num_targets == 0 && a->B == 1)) && rows <= 0x7fffffffL &&
                         layer_takes_key_value_rows(rows, a->D, a->F);
     const size_t behind = a->num_targets ? static_cast<size_t>(a->Nc) * Dh * e : 0;
     const auto rows_of = [&](const artab_stack_layer &n) {
         if (!direct) return KeyValueRows{};
         return KeyValueRows{static_cast<char *>(n.k_cache) + behind, static_cast<char *>(n.v_cache) + behind, cache_b, cache_h, a->N, Dh};
     };
-    if (f32) {
-        F32LayerParams P{};
-        P.x = static_cast<const float *>(a->x);
-        ARTAB_TRY(launch_status(launch_f32_layer(f32_head(P, *L, base + s.y[0], qkv, rows), a->D, static_cast<hipStream_t>(stream)), "layer (float32)"));
-    } else {
-        ARTAB_TRY(layer_pre_impl(rows_of(*L), a->x, D, L->w_fo, L->gamma1, L->beta1, L->eps1, L->w_qkv, base + s.y[0], qkv, rows, a->D,
-                                 dtype, stream));
+    for (int p = 0; p < S.n; ++p) {
+        const int64_t at = first_row(p), n = S.rows(p);
+        char *const y = base + s.y[0] + at * D * e, *const qkv = base + s.qkv + at * 3 * D * e;
+        if (f32) {
+            F32LayerParams P{};
+            P.x = static_cast<const float *>(S.part[p]->x);
+            ARTAB_TRY(launch_status(launch_f32_layer(f32_head(P, *L, y, qkv, n), a->D, st), "layer (float32)"));
+        } else {
+            ARTAB_TRY(layer_pre_impl(rows_of(*L), S.part[p]->x, D, L->w_fo, L->gamma1, L->beta1, L->eps1, L->w_qkv, y, qkv, n, a->D, dtype,
+                                     stream));
+        }
     }
-    for (int l = 0; l < a->n_layers; ++l, ++L) {
+    const auto cache_rows = [&](const artab_stack_args *t, const artab_view &k, const artab_view &v, int first, int entries) -> int {
+        CacheRowsParams C = {static_cast<const char *>(k.data), static_cast<const char *>(v.data), static_cast<char *>(L->k_cache),
+                             static_cast<char *>(L->v_cache), 3 * D * e, entries, t->N, t->H, Dh * e / 16, t->cache_rows, first};
+        const long pieces = static_cast<long>(entries) * t->N * t->H * C.head_pieces;
+        if ((pieces + 255) / 256 > 0x7fffffffL) return fail(ARTAB_ERR_BAD_SHAPE, "layer stack: too many rows");
+        hipLaunchKernelGGL(cache_rows_kernel, dim3(static_cast<unsigned>((pieces + 255) / 256)), dim3(256), 0, st, C);
+        return launch_status(hipGetLastError(), "cache rows");
+    };
+    const auto attend = [&](int p, bool keys_only) -> int {
+        const artab_stack_args *t = S.part[p];
+        char *const qkv = base + s.qkv + first_row(p) * 3 * D * e, *const attn = base + s.attn + first_row(p) * D * e;
+        const auto head_view = [&](int which) { return artab_view{qkv + which * D * e, t->N * 3 * D, Dh, 3 * D}; };
+        const artab_view q = head_view(0), k = head_view(1), v = head_view(2), out = {attn, t->N * D, Dh, D};
         const artab_view kc = {L->k_cache, cache_b, cache_h, Dh}, vc = {L->v_cache, cache_b, cache_h, Dh};
+        const int entries = t->own_caches ? t->B : 1;
+        if (keys_only) return direct ? ARTAB_OK : cache_rows(t, k, v, 0, entries);
         if (direct) {
             const KeyValueRows r = rows_of(*L);
             const artab_view kd = {r.k, cache_b, cache_h, Dh}, vd = {r.v, cache_b, cache_h, Dh};
-            if (a->num_targets == 0)
-                ARTAB_TRY(artab_prefill_attention_sliced(&q, &kd, &vd, &out, nullptr, nullptr, 0, a->B, a->H, a->N, Dh, 0.f, dtype,
-                                                         base + s.prefill, s.total - s.prefill, ARTAB_IMPL_AUTO, stream));
-            else
-                ARTAB_TRY(artab_teacher_forcing_attention(&q, &kc, &vc, &kd, &vd, &out, nullptr, a->B, a->H, a->num_targets, a->Nc, Dh,
-                                                          0.f, dtype, ARTAB_IMPL_AUTO, stream));
-        } else if (a->num_targets == 0) {
-            ARTAB_TRY(artab_prefill_attention_sliced(&q, &k, &v, &out, &kc, &vc, a->own_caches ? a->B : 1, a->B, a->H, a->N, Dh, 0.f,
-                                                     dtype, base + s.prefill, s.total - s.prefill, ARTAB_IMPL_AUTO, stream));
-        } else {
-            if (a->own_caches) {
-                CacheRowsParams C = {static_cast<const char *>(k.data), static_cast<const char *>(v.data),
-                                     static_cast<char *>(L->k_cache), static_cast<char *>(L->v_cache), 3 * D * e,
-                                     a->B, a->N, a->H, Dh * e / 16, a->cache_rows, a->Nc};
-                const long pieces = rows * a->H * C.head_pieces;
-                if ((pieces + 255) / 256 > 0x7fffffffL) return fail(ARTAB_ERR_BAD_SHAPE, "layer stack: too many rows");
-                hipLaunchKernelGGL(cache_rows_kernel, dim3(static_cast<unsigned>((pieces + 255) / 256)), dim3(256), 0,
-                                   static_cast<hipStream_t>(stream), C);
-                ARTAB_TRY(launch_status(hipGetLastError(), "cache rows"));
-            }
-            ARTAB_TRY(artab_teacher_forcing_attention(&q, &kc, &vc, &k, &v, &out, nullptr, a->B, a->H, a->num_targets, a->Nc, Dh,
-                                                      0.f, dtype, ARTAB_IMPL_AUTO, stream));
+            if (t->num_targets == 0)
+                return artab_prefill_attention_sliced(&q, &kd, &vd, &out, nullptr, nullptr, 0, t->B, t->H, t->N, Dh, 0.f, dtype,
+                                                      base + s.prefill, s.total - s.prefill, ARTAB_IMPL_AUTO, stream);
+            return artab_teacher_forcing_attention(&q, &kc, &vc, &kd, &vd, &out, nullptr, t->B, t->H, t->num_targets, t->Nc, Dh, 0.f,
+                                                   dtype, ARTAB_IMPL_AUTO, stream);
         }
-        const char *y = base + s.y[l & 1];
-        if (f32) {
-            F32LayerParams P{};
-            f32_tail(P, *L, attn, y, a->out, rows);
-            if (l + 1 < a->n_layers) f32_head(P, L[1], base + s.y[1 - (l & 1)], qkv, rows);
-            ARTAB_TRY(launch_status(launch_f32_layer(P, a->D, static_cast<hipStream_t>(stream)), "layer (float32)"));
+        if (t->num_targets == 0)
+            return artab_prefill_attention_sliced(&q, &k, &v, &out, &kc, &vc, entries, t->B, t->H, t->N, Dh, 0.f, dtype,
+                                                  base + s.prefill, s.total - s.prefill, ARTAB_IMPL_AUTO, stream);
+        if (t->own_caches) ARTAB_TRY(cache_rows(t, k, v, t->Nc, t->B));
+        return artab_teacher_forcing_attention(&q, &kc, &vc, &k, &v, &out, nullptr, t->B, t->H, t->num_targets, t->Nc, Dh, 0.f, dtype,
+                                               ARTAB_IMPL_AUTO, stream);
+    };
+    for (int l = 0; l < a->n_layers; ++l, ++L) {
+        const bool last = l + 1 == a->n_layers;
+        for (int p = 0; p < S.n; ++p) ARTAB_TRY(attend(p, last && p == 0 && S.caches_only));
+        const char *const y = base + s.y[l & 1], *const attn = base + s.attn;
+        if (!last) {
+            const artab_stack_layer *n = L + 1;
+            char *const y_next = base + s.y[1 - (l & 1)], *const qkv = base + s.qkv;
+            if (f32) {
+                F32LayerParams P{};
+                f32_tail(P, *L, attn, y, nullptr, rows);
+                ARTAB_TRY(launch_status(launch_f32_layer(f32_head(P, *n, y_next, qkv, rows), a->D, st), "layer (float32)"));
+            } else {
+                ARTAB_TRY(layer_post_pre_impl(rows_of(*n), nullptr, attn, D, y, D, L->w_o, L->gamma2, L->beta2, L->eps2, L->w_1, L->b_1,
+                                              L->w_2, L->b_2, L->gamma3, L->beta3, L->eps3, n->w_fo, n->gamma1, n->beta1, n->eps1, n->w_qkv,
+                                              y_next, qkv, rows, a->D, a->F, dtype, stream));
+            }
             continue;
         }
-        if (l + 1 == a->n_layers)
-            return artab_layer_post(attn, D, y, D, L->w_o, L->gamma2, L->beta2, L->eps2, L->w_1, L->b_1, L->w_2, L->b_2, L->gamma3,
-                                    L->beta3, L->eps3, a->out, rows, a->D, a->F, dtype, stream);
-        const artab_stack_layer *n = L + 1;
-        ARTAB_TRY(layer_post_pre_impl(rows_of(*n), nullptr, attn, D, y, D, L->w_o, L->gamma2, L->beta2, L->eps2, L->w_1, L->b_1, L->w_2,
-                                      L->b_2, L->gamma3, L->beta3, L->eps3, n->w_fo, n->gamma1, n->beta1, n->eps1, n->w_qkv,
-                                      base + s.y[1 - (l & 1)], qkv, rows, a->D, a->F, dtype, stream));
+        for (int p = S.caches_only ? 1 : 0; p < S.n; ++p) {
+            const int64_t at = first_row(p) * D * e;
+            if (f32) {
+                F32LayerParams P{};
+                f32_tail(P, *L, attn + at, y + at, S.part[p]->out, S.rows(p));
+                ARTAB_TRY(launch_status(launch_f32_layer(P, a->D, st), "layer (float32)"));
+            } else {
+                ARTAB_TRY(artab_layer_post(attn + at, D, y + at, D, L->w_o, L->gamma2, L->beta2, L->eps2, L->w_1, L->b_1, L->w_2, L->b_2,
+                                           L->gamma3, L->beta3, L->eps3, S.part[p]->out, S.rows(p), a->D, a->F, dtype, stream));
+            }
+        }
     }
     return ARTAB_OK;
+}
+
+int artab_layer_stack(const artab_stack_args *a, int dtype, void *stream) {
+    ARTAB_TRY(check_stack(a));
+    return stack_pass({{a, nullptr}, 1, false}, dtype, stream);
+}
+
+static int check_stack_pair(const artab_stack_args *c, const artab_stack_args *t) {
+    ARTAB_TRY(check_stack(c));
+    if (c->num_targets) return fail(ARTAB_ERR_BAD_SHAPE, "layer stack: the context is a prefill (num_targets 0)");
+    if (!t) return ARTAB_OK;
+    ARTAB_TRY(check_stack(t));
+    if (!t->num_targets || t->layers != c->layers || t->n_layers != c->n_layers || t->H != c->H || t->D != c->D || t->F != c->F ||
+        t->Nc != c->N || t->own_caches != c->own_caches || t->cache_rows != c->cache_rows || c->B != (c->own_caches ? t->B : 1))
+        return fail(ARTAB_ERR_BAD_SHAPE, "layer stack: the targets' pass is over the context's layers, rows and caches");
+    return ARTAB_OK;
+}
+
+size_t artab_layer_stack_context_scratch_bytes(const artab_stack_args *context, const artab_stack_args *targets, int dtype) {
+    if (check_stack_pair(context, targets) != ARTAB_OK) return 0;
+    return stack_scratch({{context, targets}, targets ? 2 : 1, true}, dtype).total;
+}
+
+int artab_layer_stack_context(const artab_stack_args *context, const artab_stack_args *targets, int dtype, void *stream) {
+    ARTAB_TRY(check_stack_pair(context, targets));
+    return stack_pass({{context, targets}, targets ? 2 : 1, true}, dtype, stream);
 }
 
 static TrajectoryTapeLayout trajectory_layout(int D, int F, int n_layers, int dtype) {

@@ -232,6 +232,13 @@ class ARTabPFNPredictor:
             return None
         return self._stack(list(self.backbone.layers), x_row, caches, num_targets, context_len)
 
+    def _prefill_pass(self, x_row: Tensor, caches, targets: Optional[Tensor] = None):
+        """``_stack_pass`` of a prefill, whose rows nobody reads: the last layer's attention and what follows it are
+        left out.  With ``targets`` the teacher-forced pass beside it; its output, or None."""
+        if ak is not _attention_module or not _STACK_METHODS.of(self):
+            return None
+        return self._stack.context(list(self.backbone.layers), x_row, caches, targets)
+
     # ------------------------------------------------------------------ prefill
 
     @torch.no_grad()
@@ -247,7 +254,7 @@ class ARTabPFNPredictor:
             if layer.k_cache.shape[2] < Nc:
                 raise ValueError("KV cache too small for the context; call init_kv_cache with a larger max_seq_len.")
         layers = list(self.backbone.layers)
-        if self._stack_pass(x_row, [(l.k_cache, l.v_cache) for l in layers]) is None:
+        if self._prefill_pass(x_row, [(l.k_cache, l.v_cache) for l in layers]) is None:
             self._run_layers(x_row, lambda layer, q, k, v: ak.prefill_attention(q, k, v, layer.k_cache, layer.v_cache))
         self.seq_len = Nc
 
@@ -257,18 +264,23 @@ class ARTabPFNPredictor:
         same for every trajectory (inference.py:180-223)."""
         Nc = x_context.shape[1]
         x_row = self.embedder.embed_context(x_context[0:1], y_context[0:1])
-        for layer in self.backbone.layers:
-            H, Dh = layer.attn_rows.n_heads, layer.attn_rows.head_dim
-            if layer.k_ctx_cache.shape[1] != Nc or layer.k_ctx_cache.shape[0] != H:
-                layer.k_ctx_cache = torch.zeros(H, Nc, Dh, device=x_row.device, dtype=x_row.dtype)
-                layer.v_ctx_cache = torch.zeros_like(layer.k_ctx_cache)
-        if self._stack_pass(x_row, [(l.k_ctx_cache, l.v_ctx_cache) for l in self.backbone.layers]) is None:
+        if self._prefill_pass(x_row, self._context_caches(x_row)) is None:
             self._run_layers(
                 x_row, lambda layer, q, k, v: ak.prefill_attention(q, k, v, layer.k_ctx_cache, layer.v_ctx_cache))
         self.context_len = Nc
         self.buffer_len = 0
         self.seq_len = Nc
         self._prefill_batch_size = x_context.shape[0]
+
+    def _context_caches(self, x_row: Tensor):
+        """The shared layout's context caches, of the length of ``x_row``."""
+        Nc = x_row.shape[1]
+        for layer in self.backbone.layers:
+            H, Dh = layer.attn_rows.n_heads, layer.attn_rows.head_dim
+            if layer.k_ctx_cache.shape[1] != Nc or layer.k_ctx_cache.shape[0] != H:
+                layer.k_ctx_cache = torch.zeros(H, Nc, Dh, device=x_row.device, dtype=x_row.dtype)
+                layer.v_ctx_cache = torch.zeros_like(layer.k_ctx_cache)
+        return [(l.k_ctx_cache, l.v_ctx_cache) for l in self.backbone.layers]
 
     # ------------------------------------------------------------------ decode
 
@@ -814,16 +826,46 @@ class ARTabPFNPredictor:
     def _evaluate_joint_density_shared(self, x_context, y_context, x_target, y_target) -> Tensor:
         B, Nt = x_context.shape[0], x_target.shape[1]
         self.init_kv_cache(B, Nt, x_context.device, x_context.dtype)
-        self.prefill_context(x_context, y_context)
-        z = self._teacher_forcing_decode_shared(self._teacher_forcing_embedding(x_target, y_target), Nt)
+        z = self._density_pass(x_context, y_context, x_target, y_target)
+        if z is None:
+            self.prefill_context(x_context, y_context)
+            z = self._teacher_forcing_decode_shared(self._teacher_forcing_embedding(x_target, y_target), Nt)
         return self.head.log_likelihood(z[:, Nt:, :], y_target.unsqueeze(-1))
+
+    # Rows up to which the two passes of a density share their layer boundaries: such a boundary is a launch of few
+    # workgroups that takes as long with twice as many.
+    _DENSITY_ROWS = 8192
+
+    def _density_pass(self, x_context, y_context, x_target, y_target) -> Optional[Tensor]:
+        """Prefill and teacher-forced pass side by side, on caches that have just been made: its normed rows, or None, with
+        nothing done, where they run one after the other."""
+        (B, Nt), shared = x_target.shape[:2], self.backend == _SHARED
+        if not (x_context.is_cuda and _DENSITY_METHODS.of(self) and Nt > 0 and x_context.shape[1] > 0
+                and x_context.shape[1] * (1 if shared else B) + 2 * B * Nt <= self._DENSITY_ROWS):
+            return None
+        n, layers = 1 if shared else x_context.shape[0], list(self.backbone.layers)
+        # (asked before anything is embedded: what does not apply runs as if it had not been asked)
+        if not (ak is _attention_module and _STACK_METHODS.of(self)
+                and self._stack.applies(layers, torch.Size((n, x_context.shape[1], self.backbone.d_model)), x_context.dtype, x_context.device)):
+            return None
+        x_row = self.embedder.embed_context(x_context[:n], y_context[:n])
+        caches = self._context_caches(x_row) if shared else [(l.k_cache, l.v_cache) for l in self.backbone.layers]
+        z = self._prefill_pass(x_row, caches, self._teacher_forcing_embedding(x_target, y_target))
+        if z is None:
+            return None
+        self.seq_len = x_row.shape[1]
+        if shared:
+            self.context_len, self.buffer_len, self._prefill_batch_size = x_row.shape[1], 0, x_context.shape[0]
+        return add_layer_norm(z, None, None, self.backbone.norm)
 
     def _evaluate_joint_density_flex(self, x_context, y_context, x_target, y_target) -> Tensor:
         B, Nc = x_context.shape[0], x_context.shape[1]
         Nt = x_target.shape[1]
         self.init_kv_cache(B, Nc + 2 * Nt, x_context.device, x_context.dtype)
-        self.prefill_context(x_context, y_context)
-        z = self._teacher_forcing_decode(self._teacher_forcing_embedding(x_target, y_target), Nt)
+        z = self._density_pass(x_context, y_context, x_target, y_target)
+        if z is None:
+            self.prefill_context(x_context, y_context)
+            z = self._teacher_forcing_decode(self._teacher_forcing_embedding(x_target, y_target), Nt)
         return self.head.log_likelihood(z[:, Nt:, :], y_target.unsqueeze(-1))
 
     @torch.no_grad()
@@ -870,3 +912,5 @@ class ARTabPFNPredictor:
 _RUN_METHODS = Methods(ARTabPFNPredictor, "autoregressive_decode", "transformer_decode", "_run_layers", "_attend_decode_shared",
                        "_attend_with_cache", "_graph_step", "_first_step", "_sample_sequence_graph")
 _STACK_METHODS = Methods(ARTabPFNPredictor, "_run_layers", "_attend_with_cache", "_attend_teacher_forcing_shared")
+_DENSITY_METHODS = Methods(ARTabPFNPredictor, "prefill_context", "prefill_context_shared", "_teacher_forcing_decode",
+                           "_teacher_forcing_decode_shared", "_stack_pass", "_prefill_pass")

@@ -99,37 +99,83 @@ class LayerStack:
         self._layers, self._prepared = array, Prepared(keep)
         return True
 
+    @staticmethod
+    def applies(layers, shape, dtype, device) -> bool:
+        """Whether passes of such rows ``[B,N,D]`` through these layers have kernels and stand for what the layers do."""
+        if not (device.type == "cuda" and layers and shape.numel() and (ak.prefill_attention, ak.teacher_forcing_attention,
+                                                                        ak.hybrid_teacher_forcing_attention) == _attention_calls
+                and LAYER_METHODS.of(*layers)):
+            return False
+        rows, D = layers[0].attn_rows, shape[-1]
+        return rows.head_dim in (32, 64, 128) and rows.n_heads * rows.head_dim == D and _covered(layers[0], torch.empty((0, D), dtype=dtype, device=device))
+
+    def _ready(self, layers, x: Tensor, caches, need: int) -> bool:
+        """Whether the library takes passes of ``x [B,N,D]`` through ``layers`` with caches of at least ``need`` rows; their
+        weights and caches are then in place."""
+        if not self.applies(layers, x.shape, x.dtype, x.device):
+            return False
+        first = layers[0]
+        k0 = caches[0][0]
+        H, Dh, rows = first.attn_rows.n_heads, first.attn_rows.head_dim, k0.shape[-2]
+        shape = (x.shape[0], H, rows, Dh) if k0.dim() == 4 else (H, rows, Dh)
+        if not (rows >= need
+                and all(t.shape == shape and t.dtype == x.dtype and t.device == x.device and t.is_contiguous() and t.data_ptr() % 16 == 0
+                        for c in caches for t in c)
+                and self._collect(layers, x)):
+            return False
+        for a, (k, v) in zip(self._layers, caches):
+            a.k_cache, a.v_cache = k.data_ptr(), v.data_ptr()
+        return True
+
+    def _args(self, layers, x: Tensor, caches, num_targets: int, context_len: int, out: Optional[Tensor]):
+        first, k0 = layers[0], caches[0][0]
+        B, N, D = x.shape
+        return _lib.ArtabStackArgs(ctypes.addressof(self._layers), len(layers), B, N, first.attn_rows.n_heads, D,
+                                   first.ff[0].out_features, num_targets, context_len, int(k0.dim() == 4), k0.shape[-2], x.data_ptr(),
+                                   None if out is None else out.data_ptr(), None)
+
     def __call__(self, layers, x: Tensor, caches, num_targets: int = 0, context_len: int = 0) -> Optional[Tensor]:
         """``x [B,N,D]`` through ``layers``; ``caches``: ``(k, v)`` of every layer, ``[H,R,Dh]`` or ``[B,H,R,Dh]``.
         ``num_targets`` 0: prefill; else teacher forcing against the first ``context_len`` cached rows.  None, with
         nothing done, where the call does not apply."""
-        if not (x.is_cuda and layers and x.numel() and (ak.prefill_attention, ak.teacher_forcing_attention,
-                                                       ak.hybrid_teacher_forcing_attention) == _attention_calls
-                and LAYER_METHODS.of(*layers)):
+        N, own = x.shape[1], caches[0][0].dim() == 4
+        if (num_targets and context_len <= 0) or not self._ready(layers, x, caches, N if num_targets == 0 else context_len + (N if own else 0)):
             return None
-        first = layers[0]
-        B, N, D = x.shape
-        k0 = caches[0][0]
-        own = k0.dim() == 4
-        H, Dh, rows = first.attn_rows.n_heads, first.attn_rows.head_dim, k0.shape[-2]
-        shape = (B, H, rows, Dh) if own else (H, rows, Dh)
-        if not (Dh in (32, 64, 128) and H * Dh == D and _covered(first, x) and rows >= (N if num_targets == 0 else context_len + (N if own else 0))
-                and (num_targets == 0 or context_len > 0)
-                and all(t.shape == shape and t.dtype == x.dtype and t.device == x.device and t.is_contiguous() and t.data_ptr() % 16 == 0
-                        for c in caches for t in c)
-                and self._collect(layers, x)):
-            return None
-        x = x.contiguous()
-        if x.data_ptr() % 16:
-            x = x.clone()
+        x = _pieces(x)
         self._prepared.use()
         lib, code = _lib.load(), _lib.dtype_code(x.dtype)
-        for a, (k, v) in zip(self._layers, caches):
-            a.k_cache, a.v_cache = k.data_ptr(), v.data_ptr()
         out = torch.empty_like(x)
-        args = _lib.ArtabStackArgs(ctypes.addressof(self._layers), len(layers), B, N, H, D, first.ff[0].out_features, num_targets,
-                                   context_len, int(own), rows, x.data_ptr(), out.data_ptr(), None)
+        args = self._args(layers, x, caches, num_targets, context_len, out)
         scratch = torch.empty(lib.artab_layer_stack_scratch_bytes(ctypes.byref(args), code), device=x.device, dtype=torch.uint8)
         args.scratch = scratch.data_ptr()
         _lib.check(lib.artab_layer_stack(ctypes.byref(args), code, _lib.current_stream(x.device)))
         return out
+
+    def context(self, layers, x: Tensor, caches, targets: Optional[Tensor] = None):
+        """A prefill of ``x [B,Nc,D]`` for the caches alone, and with ``targets [B',2 Nt,D]`` the teacher-forced pass over them
+        beside it.  True or that pass's output; None, with nothing done, where the call does not apply."""
+        N, own = x.shape[1], caches[0][0].dim() == 4
+        both = targets is not None
+        if both and not (targets.dtype == x.dtype and targets.device == x.device and targets.numel() and targets.shape[1] % 2 == 0
+                         and x.shape[0] == (targets.shape[0] if own else 1)):
+            return None
+        if not self._ready(layers, x, caches, N + (targets.shape[1] if both and own else 0)):
+            return None
+        x = _pieces(x)
+        self._prepared.use()
+        lib, code, stream = _lib.load(), _lib.dtype_code(x.dtype), _lib.current_stream(x.device)
+        args, second, out = self._args(layers, x, caches, 0, 0, None), None, True
+        if both:
+            targets = _pieces(targets)
+            out = torch.empty_like(targets)
+            second = ctypes.byref(self._args(layers, targets, caches, targets.shape[1] // 2, N, out))
+        scratch = torch.empty(lib.artab_layer_stack_context_scratch_bytes(ctypes.byref(args), second, code), device=x.device,
+                              dtype=torch.uint8)
+        args.scratch = scratch.data_ptr()
+        _lib.check(lib.artab_layer_stack_context(ctypes.byref(args), second, code, stream))
+        return out
+
+
+def _pieces(x: Tensor) -> Tensor:
+    x = x.contiguous()
+    return x.clone() if x.data_ptr() % 16 else x

@@ -612,6 +612,14 @@ typedef struct artab_stack_args {
 int artab_pack_stack_weight_float(const void *w, void *packed, int N, int K, void *stream);
 size_t artab_layer_stack_scratch_bytes(const artab_stack_args *args, int dtype);
 int artab_layer_stack(const artab_stack_args *args, int dtype, void *stream);
+/*
+ * A prefill of which the caches alone are wanted: nothing behind the last layer's K and V is computed, context->out
+ * is not read.  With `targets` (over the same layers and caches, Nc = context->N) the teacher-forced pass runs beside
+ * it, layer by layer, with one launch per layer boundary for the rows of both: what the two passes one after the
+ * other give.  The scratch memory is context->scratch.
+ */
+size_t artab_layer_stack_context_scratch_bytes(const artab_stack_args *context, const artab_stack_args *targets, int dtype);
+int artab_layer_stack_context(const artab_stack_args *context, const artab_stack_args *targets, int dtype, void *stream);
 
 /*
  * A whole sampling run in one launch: every workgroup takes a few trajectories through all Nt steps
