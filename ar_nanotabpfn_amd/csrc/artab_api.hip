@@ -321,14 +321,17 @@ static hipError_t launch_context_small(const ContextSmallParams &P, int Dh, int 
     return hipGetLastError();
 }
 
-// The streaming buffer pass: one wavefront per workgroup.  Two of them fit on a CU beside the context
-// pass, four or five once it has left (LDS).  The grid holds one workgroup per task up to 32 per CU:
-// which wavefront takes which task is then the dispatcher's decision, made when a slot frees up,
-// not a static deal that leaves the late starters with a full share (measured at B*H = 32768, 256
-// steps: 500 target-steps/s with 4 per CU, 506 with 6, 508 with 16, 512 with 32; at B*H = 8192,
-// where 8 per CU already is one per task, no difference).
+// The streaming buffer pass: one wavefront per workgroup.  Beside the context pass (two workgroups of 33 KiB of LDS to a
+// compute unit) three of them fit, and three per compute unit are started: with more, those that are placed before the
+// context pass's second workgroup keep it off the unit until they are done, and every one of them starts with an empty ring
+// where a persistent one goes on from task to task.  us per layer with its context pass, three against 32 per unit (and against two of
+// 32 KiB each, what fitted while a workgroup held two query regions): B*H = 32768, 4096 context rows, 64 buffer rows 84 / 102 / 107,
+// 128 rows 122 / 137 / 139, 248 rows 199 / 206 / 201; B*H = 8192, 16384 context rows, 128 rows 59 / 67, 248 rows 73 / 91; four
+// per unit 142 and 232, 61 and 77.  With the device to itself (no second stream): one workgroup per task up to 32 per unit; which
+// wavefront takes which task is then the dispatcher's decision, made when a slot frees up (B*H = 32768, 256
+// steps: 500 target-steps/s with 4 per CU, 506 with 6, 508 with 16, 512 with 32).
 template <typename T>
-static hipError_t launch_stream_t(const DecodeParams &P, int Lq, hipStream_t stream) {
+static hipError_t launch_stream_t(const DecodeParams &P, int Lq, bool beside, hipStream_t stream) {
     const long pairs = static_cast<long>(P.B) * P.H;
     if (pairs == 0) return hipSuccess;
     int dev = 0, cus = 0;
@@ -336,7 +339,7 @@ static hipError_t launch_stream_t(const DecodeParams &P, int Lq, hipStream_t str
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
         cus = 256;
     const long tasks = (pairs + 3) / 4;  // of the 4-pair chunk shape; the 16-pair shape leaves the surplus idle
-    long per_cu = 32;
+    long per_cu = beside ? 3 : 32;
     if (const int v = tune(kTuneStreamPerCu, 0); v >= 1 && v <= 32) per_cu = v;
     dim3 grid(static_cast<unsigned>(tasks < per_cu * cus ? tasks : per_cu * cus)), block(64);
     const int prio = tune(kTuneStreamPrio, 3);
@@ -353,8 +356,8 @@ static hipError_t launch_stream_t(const DecodeParams &P, int Lq, hipStream_t str
     return hipGetLastError();
 }
 
-static hipError_t launch_stream(const DecodeParams &P, int dtype, int Lq, hipStream_t stream) {
-    return dtype == ARTAB_BF16 ? launch_stream_t<bf16_t>(P, Lq, stream) : launch_stream_t<f16_t>(P, Lq, stream);
+static hipError_t launch_stream(const DecodeParams &P, int dtype, int Lq, bool beside, hipStream_t stream) {
+    return dtype == ARTAB_BF16 ? launch_stream_t<bf16_t>(P, Lq, beside, stream) : launch_stream_t<f16_t>(P, Lq, beside, stream);
 }
 
 static hipError_t launch_portable_dtype(const PortableParams &P, int dtype, hipStream_t stream) {
@@ -869,7 +872,7 @@ static int decode_impl(const artab_view *q, const artab_view *k_ctx, const artab
         {
             e_ctx = launch_flash_dtype(F, dtype == ARTAB_BF16, Dh, pl.BM, st);
         }
-        e_buf = launch_stream(D, dtype, Lq, side);
+        e_buf = launch_stream(D, dtype, Lq, side != st, side);
         ARTAB_TRY(launch_status(e_ctx, "decode context pass"));
         ARTAB_TRY(launch_status(e_buf, "decode buffer pass (stream)"));
         ARTAB_TRY(order_signal(order_state, ARTAB_ORDER_SIDE, side));    // the buffer pass's partial is ready
@@ -895,7 +898,7 @@ static int decode_impl(const artab_view *q, const artab_view *k_ctx, const artab
     {
         e_ctx = launch_flash_dtype(F, dtype == ARTAB_BF16, Dh, pl.BM, st);
     }
-    e_buf = launch_stream(D, dtype, Lq, side);
+    e_buf = launch_stream(D, dtype, Lq, side != st, side);
     if (side != st) {
         // always rejoin, so that a failed launch does not leave the side stream forked (e.g. inside a capture)
         e_join = hipEventRecord(join, side);

@@ -38,8 +38,9 @@ namespace artab {
 constexpr int kStreamChunks = 3;           // ring depth per wavefront
 constexpr int kStreamShortRows = 32;       // buffers longer than this are read 16 rows x 4 pairs at a time
 constexpr int kStreamChunkBytes = 8192;    // 64 key rows x (64 B of K + 64 B of V)
-constexpr int kStreamQBytes = 4096;        // a region of query slots: 4 x (64 lanes x 16 B)
-constexpr size_t kStreamLdsBytes = kStreamChunks * kStreamChunkBytes + 2 * kStreamQBytes;
+constexpr int kStreamQBytes = 4096;        // the query slots: 4 x (64 lanes x 16 B)
+// 28 KiB: three workgroups beside two of the context pass (2 x 33 KiB of a unit's 160)
+constexpr size_t kStreamLdsBytes = kStreamChunks * kStreamChunkBytes + kStreamQBytes;
 
 // LDS reads of the ring go through inline assembly: the compiler must not see an LDS read that
 // could alias the asynchronous fills, or it would drain every load before each read.
@@ -141,10 +142,10 @@ __device__ __forceinline__ void decode_stream_body(const DecodeParams &P, unsign
     constexpr int S = kStreamChunks;
     constexpr int PP = 64 / KEYS;             // pairs per task
     constexpr int NKG = KEYS / 4;             // lane groups (of four keys each) per pair
-    constexpr int QREG = KEYS == 16 ? 1 : 2;  // 4 KiB query regions in use
-    constexpr int QS = QREG * NKG;            // query slots: lane group k of a region holds one task's queries
+    constexpr int QL = KEYS == 16 ? 4 : 2;    // lanes of a pair that hold one task's queries (of its KEYS in the query region)
+    constexpr int QS = KEYS / QL;             // query slots
     static_assert(KEYS == 4 || KEYS == 16, "chunk shapes: 16 pairs x 4 rows or 4 pairs x 16 rows");
-    static_assert(QS == 2 || QS == 4, "slot index is taken modulo a power of two");
+    static_assert(LQ <= QL && (QS == 2 || QS == 4), "slot index is taken modulo a power of two");
 
     // Every argument the loop needs, as plain values: the inline assembly clobbers memory, and
     // anything still read through the argument block would be re-read after every such statement.
@@ -203,11 +204,12 @@ __device__ __forceinline__ void decode_stream_body(const DecodeParams &P, unsign
         if (first) {
             p_k = view_row<T>(vkb, p_b, p_h, kq);
             p_v = view_row<T>(vvb, p_b, p_h, kq);
-            // the task's queries, fetched by the lanes of one lane group per pair (which group:
-            // the slot); the pieces of lanes that stand for no query stay zero (cleared once, below)
+            // the task's queries, fetched by QL lanes of each pair (which of them: the slot)
             const int qslot = issue_seq & (QS - 1);
-            unsigned char *qd = stream_lds + S * kStreamChunkBytes + (qslot / NKG) * kStreamQBytes;
-            const int j = kq - 4 * (qslot % NKG);
+            int region = S * kStreamChunkBytes;
+            asm volatile("" : "+s"(region));  // (as a constant the code generator makes an illegal instruction of it)
+            unsigned char *qd = stream_lds + region;
+            const int j = kq - QL * qslot;
             if (j >= 0 && j < LQ) load_row64_to_lds(view_row<T>(vq, p_b, p_h, j), qd);
         }
         const T *kr = p_k, *vr = p_v;
@@ -232,11 +234,11 @@ __device__ __forceinline__ void decode_stream_body(const DecodeParams &P, unsign
         }
     };
     // Lanes that stand for no query (index within the lane group >= LQ) contribute zeros to the
-    // score product: their pieces of every query region are cleared once and never written again.
-    if ((lane & 3) >= LQ) {
+    // score product.  Where a slot is a whole lane group, their pieces are cleared once and never written again.
+    if (QL == 4 && (lane & 3) >= LQ) {
         const u32x4 zero = {0u, 0u, 0u, 0u};
 #pragma unroll
-        for (int t = 0; t < 4 * QREG; ++t) lds_write128(q_lds0 + 1024u * t + lane * 16u, zero);
+        for (int t = 0; t < 4; ++t) lds_write128(q_lds0 + 1024u * t + lane * 16u, zero);
     }
     // QS query slots: the producer may be at most QS - 1 tasks ahead of the consumer
     auto may_issue = [&]() { return issued < total_chunks && issue_seq <= seq + (QS - 1); };
@@ -356,11 +358,13 @@ __device__ __forceinline__ void decode_stream_body(const DecodeParams &P, unsign
         const unsigned chunk = lds0 + static_cast<unsigned>(slot) * kStreamChunkBytes;
         const bool more = c + 1 < total_chunks;
         if (g == 0) {
-            // the task's queries: those of the lane's pair and query index, from the lane group
-            // that fetched them for this slot
+            // the task's queries: those of the lane's pair and query index, from where they were put for this slot
             const int ln = opaque(lane), qslot = seq & (QS - 1);
-            const int src = ln - 4 * ((ln % KEYS) >> 2) + 4 * (qslot % NKG);
-            lds_read4x128(qr, q_lds0 + static_cast<unsigned>(qslot / NKG) * kStreamQBytes + src * 16u);
+            const int src = ln - ln % KEYS + QL * qslot + ln % QL;
+            lds_read4x128(qr, q_lds0 + src * 16u);
+            if (QL < 4 && (ln & 3) >= LQ)  // (two slots share a lane group: what such a lane read is another task's query or nothing)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) qr[e] = u32x4{0u, 0u, 0u, 0u};
         }
         u32x2 vop[8];
         wait_chunk(c);

@@ -292,6 +292,17 @@ def test_decode_attention_stream_chunk_shapes(device, stream_chunk_shape, dtype,
     _decode_case(device, dtype, B, H, Lq, Nc, D, n_buf, cap, with_new, True, scale=0.6, overlapped=True)
 
 
+@pytest.mark.parametrize("Lq", [1, 2])
+@pytest.mark.parametrize("n_buf", [0, 3, 4, 13, 31])
+@pytest.mark.parametrize("shape", ["0", "100000"], ids=["16-row-chunks", "4-row-chunks"])
+def test_decode_attention_stream_many_tasks(device, tuning, shape, n_buf, Lq):
+    """Workgroups of the streaming buffer pass that go through two to nine tasks each (one workgroup per compute
+    unit), of one chunk, two, and more than the ring holds: the next task's queries and rows are requested while
+    the last one's are read."""
+    tuning(ARTAB_SMALL=0, ARTAB_STREAM_SHORT=int(shape), ARTAB_STREAM_PER_CU=1)
+    _decode_case(device, torch.bfloat16, 1101, 8, Lq, 64, 32, n_buf, 32, True, True, scale=0.6, overlapped=True)
+
+
 @pytest.mark.parametrize("n_buf", [5, 150])
 def test_decode_attention_wave_priorities_do_not_change_results(device, tuning, n_buf):
     """The two passes of an overlapped call choose their wave priorities from the buffer length
