@@ -235,6 +235,8 @@ class ARTabPFNPredictor:
     def _prefill_pass(self, x_row: Tensor, caches, targets: Optional[Tensor] = None):
         """``_stack_pass`` of a prefill, whose rows nobody reads: the last layer's attention and what follows it are
         left out.  With ``targets`` the teacher-forced pass beside it; its output, or None."""
+        if targets is None and not _STACK_PASS.of(self):  # (one put in its place is asked for prefills too)
+            return self._stack_pass(x_row, caches)
         if ak is not _attention_module or not _STACK_METHODS.of(self):
             return None
         return self._stack.context(list(self.backbone.layers), x_row, caches, targets)
@@ -912,5 +914,6 @@ class ARTabPFNPredictor:
 _RUN_METHODS = Methods(ARTabPFNPredictor, "autoregressive_decode", "transformer_decode", "_run_layers", "_attend_decode_shared",
                        "_attend_with_cache", "_graph_step", "_first_step", "_sample_sequence_graph")
 _STACK_METHODS = Methods(ARTabPFNPredictor, "_run_layers", "_attend_with_cache", "_attend_teacher_forcing_shared")
+_STACK_PASS = Methods(ARTabPFNPredictor, "_stack_pass")
 _DENSITY_METHODS = Methods(ARTabPFNPredictor, "prefill_context", "prefill_context_shared", "_teacher_forcing_decode",
                            "_teacher_forcing_decode_shared", "_stack_pass", "_prefill_pass")
