@@ -218,9 +218,10 @@ def stamped_decode(pred, x_context, y_context, x_target, steps, device, dtype, c
         finally:
             pred._graph_state = None  # later runs record with the drop-in library again
     us = [float(buf[i]) for i in range(n)]
-    if n != L * (steps + 1):
-        sys.exit(f"bench.py: expected {L * (steps + 1)} stamped launches (prefill + {steps} steps), saw {n}")
-    return decode_ms, us[L:]  # the first L launches are the prefill's dense passes
+    first = L - 1  # the prefill's dense passes: it ends with its last layer's keys and values
+    if n != first + L * steps:
+        sys.exit(f"bench.py: expected {first + L * steps} stamped launches (prefill + {steps} steps), saw {n}")
+    return decode_ms, us[first:]
 
 
 def host_info():
@@ -959,7 +960,7 @@ def main():
         pms, pk = (ctypes.c_float * pcap)(), (ctypes.c_int * pcap)()
         pn = bl.artab_profile_end(pms, pk, pcap)
     prefill_kernel_ms = sum(pms[i] for i in range(min(max(pn, 0), pcap)) if pk[i] == KIND_FLASH)
-    prefill_flops = 4.0 * H * NC3 * NC3 * Dh * L
+    prefill_flops = 4.0 * H * NC3 * NC3 * Dh * (L - 1)  # (the last layer's keys and values are all that is wanted of it)
 
     roofline = {
         "kernel": "flash_kernel<bf16,32> context pass of artab_decode_attention",
