@@ -250,7 +250,10 @@ class ARTabPFNPredictor:
         if self.backend == _SHARED:
             self.prefill_context_shared(x_context, y_context)
             return
-        x_row = self.embedder.embed_context(x_context, y_context)
+        self._prefill_own(self.embedder.embed_context(x_context, y_context))
+
+    def _prefill_own(self, x_row: Tensor) -> None:
+        """``prefill_context`` of embedded rows, a cache for each batch entry."""
         Nc = x_row.shape[1]
         for layer in self.backbone.layers:
             if layer.k_cache.shape[2] < Nc:
@@ -264,15 +267,16 @@ class ARTabPFNPredictor:
     def prefill_context_shared(self, x_context: Tensor, y_context: Tensor) -> None:
         """Shared layout: only batch entry 0 is encoded — the context is taken to be the
         same for every trajectory (inference.py:180-223)."""
-        Nc = x_context.shape[1]
-        x_row = self.embedder.embed_context(x_context[0:1], y_context[0:1])
+        self._prefill_shared(self.embedder.embed_context(x_context[0:1], y_context[0:1]), x_context.shape[0])
+
+    def _prefill_shared(self, x_row: Tensor, batch: int) -> None:
+        """``prefill_context_shared`` of embedded rows, for ``batch`` trajectories."""
         if self._prefill_pass(x_row, self._context_caches(x_row)) is None:
             self._run_layers(
                 x_row, lambda layer, q, k, v: ak.prefill_attention(q, k, v, layer.k_ctx_cache, layer.v_ctx_cache))
-        self.context_len = Nc
+        self.context_len = self.seq_len = x_row.shape[1]
         self.buffer_len = 0
-        self.seq_len = Nc
-        self._prefill_batch_size = x_context.shape[0]
+        self._prefill_batch_size = batch
 
     def _context_caches(self, x_row: Tensor):
         """The shared layout's context caches, of the length of ``x_row``."""
@@ -839,22 +843,26 @@ class ARTabPFNPredictor:
     _DENSITY_ROWS = 8192
 
     def _density_pass(self, x_context, y_context, x_target, y_target) -> Optional[Tensor]:
-        """Prefill and teacher-forced pass side by side, on caches that have just been made: its normed rows, or None, with
-        nothing done, where they run one after the other."""
+        """Prefill and teacher-forced pass, side by side where the library takes them so, on caches that have just been
+        made: the second one's normed rows, or None, with nothing done, where they are not even tried so."""
         (B, Nt), shared = x_target.shape[:2], self.backend == _SHARED
         if not (x_context.is_cuda and _DENSITY_METHODS.of(self) and Nt > 0 and x_context.shape[1] > 0
                 and x_context.shape[1] * (1 if shared else B) + 2 * B * Nt <= self._DENSITY_ROWS):
             return None
         n, layers = 1 if shared else x_context.shape[0], list(self.backbone.layers)
-        # (asked before anything is embedded: what does not apply runs as if it had not been asked)
         if not (ak is _attention_module and _STACK_METHODS.of(self)
                 and self._stack.applies(layers, torch.Size((n, x_context.shape[1], self.backbone.d_model)), x_context.dtype, x_context.device)):
             return None
         x_row = self.embedder.embed_context(x_context[:n], y_context[:n])
         caches = self._context_caches(x_row) if shared else [(l.k_cache, l.v_cache) for l in self.backbone.layers]
-        z = self._prefill_pass(x_row, caches, self._teacher_forcing_embedding(x_target, y_target))
-        if z is None:
-            return None
+        targets = self._teacher_forcing_embedding(x_target, y_target)
+        z = self._prefill_pass(x_row, caches, targets)
+        if z is None:  # (layers or caches are not of its form: one after the other, with the rows that are embedded now)
+            if shared:
+                self._prefill_shared(x_row, x_context.shape[0])
+                return self._teacher_forcing_decode_shared(targets, Nt)
+            self._prefill_own(x_row)
+            return self._teacher_forcing_decode(targets, Nt)
         self.seq_len = x_row.shape[1]
         if shared:
             self.context_len, self.buffer_len, self._prefill_batch_size = x_row.shape[1], 0, x_context.shape[0]

@@ -63,3 +63,24 @@ def test_prefill_for_the_caches_alone(device, dtype, own, B, N):
     assert pred._stack.context(layers, x, caches[1]) is True
     for a, b in zip(*caches):
         assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
+
+
+@pytest.mark.parametrize("backend", ["triton_shared_context", "flex_attention"])
+def test_a_refused_pass_embeds_once(device, backend):
+    """Layers that the library refuses only when their parameters are looked at (a weight in column order): hooks on the embedder are
+    called as often as where the two passes are never tried side by side, with the same densities."""
+    pred = _predictor(device, torch.float32, backend, 128)
+    weight = pred.backbone.layers[1].ff[0].weight
+    weight.data = weight.data.t().contiguous().t()
+    g = torch.Generator().manual_seed(1)
+    mk = lambda *s: torch.randn(*s, generator=g).to(device, torch.float32)  # noqa: E731
+    data = (mk(3, 21, 3), mk(3, 21), mk(3, 6, 3), mk(3, 6))
+    calls = []
+    pred.embedder.x_embed.register_forward_hook(lambda m, a, out: calls.append(tuple(out.shape)))
+    got = pred.evaluate_joint_density(*data)
+    seen, state = list(calls), (pred.seq_len, pred.context_len, pred.buffer_len)
+    calls.clear()
+    pred._DENSITY_ROWS = 0
+    ref = pred.evaluate_joint_density(*data)
+    assert seen == calls and state == (pred.seq_len, pred.context_len, pred.buffer_len)
+    assert torch.equal(got, ref)
