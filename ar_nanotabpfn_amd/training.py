@@ -12,6 +12,7 @@ import ctypes
 
 import torch
 from torch import Tensor, nn
+from torch.autograd import forward_ad
 
 from . import _lib
 from . import attention_kernels as ak
@@ -227,11 +228,12 @@ class _HeadLoss(torch.autograd.Function):
     def backward(ctx, dloss):
         lib = _lib.load()
         z, y, saved, *params = ctx.saved_tensors  # (raises if one of them was changed in place since)
-        if torch.is_grad_enabled():  # (create_graph: gradients that can be differentiated again)
+        create_graph = torch.is_grad_enabled()
+        if create_graph or _transformed(dloss, z, *params):  # gradients that can be differentiated again, or many at once
             wanted = [t for t in (z, *params) if t.requires_grad]
-            with torch.autocast("cuda", torch.bfloat16):
+            with torch.enable_grad(), torch.autocast("cuda", torch.bfloat16):
                 loss = torch.func.functional_call(ctx.head, dict(zip(_HEAD_PARAMETERS, params)), (z, y))[0]
-            grads = iter(torch.autograd.grad(loss, wanted, dloss, create_graph=True))
+            grads = iter(torch.autograd.grad(loss, wanted, dloss, create_graph=create_graph))
             dz, *dparams = (next(grads) if t.requires_grad else None for t in (z, *params))
             return (dz, None, None, *dparams)
         a = _lib.ArtabTrainHeadArgs.from_buffer_copy(ctx.args)
@@ -251,6 +253,13 @@ class _HeadLoss(torch.autograd.Function):
         return (dz, None, None, w1.view(F, D), b1, w2[: 3 * K * F].view(3 * K, F), raw[: 3 * K], *per_component)
 
 
+def _transformed(*tensors) -> bool:
+    """Whether a transform is at work (``vmap`` and its kin), or one of the tensors stands for many (batched gradients) or
+    has a tangent."""
+    return torch._C._are_functorch_transforms_active() or any(
+        not torch._C._has_storage(t) or forward_ad.unpack_dual(t).tangent is not None for t in tensors)
+
+
 _HEAD_PARAMETERS = ("head.0.weight", "head.0.bias", "head.2.weight", "head.2.bias", "mean_bias", "std_bias", "weight_bias")
 
 
@@ -266,7 +275,7 @@ def _head_pointers(a, z: Tensor, y: Tensor, params, saved: Tensor):
 def head_loss(head, z: Tensor, y: Tensor):
     """The loss of ``MixtureGaussianHead.forward(z, y)`` for ``z [B,T,D]``, ``y [B,T,1]`` under bfloat16 autocast,
     differentiable in ``z`` and the head's parameters, or None where the kernels do not apply (the data itself wants
-    gradients, types or sizes they are not built for)."""
+    gradients, types or sizes they are not built for, tangents and transforms)."""
     one, two = head.head[0], head.head[2]
     params = (one.weight, one.bias, two.weight, two.bias, head.mean_bias, head.std_bias, head.weight_bias)
     F, K = one.out_features, head.num_components
@@ -274,7 +283,7 @@ def head_loss(head, z: Tensor, y: Tensor):
             and z.is_cuda and z.dtype == torch.float32 and z.dim() == 3 and tuple(y.shape) == (z.shape[0], z.shape[1], 1)
             and not y.requires_grad and head.dim_y == 1 and isinstance(K, int) and isinstance(head.std_min, float)
             and z.shape[2] in (128, 256) and F == 256 and 1 <= 3 * K <= 128 and 1 <= z.shape[0] * z.shape[1] < 2 ** 30
-            and (z.requires_grad or any(p.requires_grad for p in params))):
+            and (z.requires_grad or any(p.requires_grad for p in params)) and not _transformed(z, y, *params)):
         return None
     y = y.contiguous()
     if not (type(z) is Tensor and z.is_contiguous() and z.data_ptr() % 16 == 0 and type(y) is Tensor and y.dtype == torch.float32 and y.device == z.device and _f32(z.device, params, _head_shapes(z.shape[2], F, K))):

@@ -123,3 +123,47 @@ def test_what_the_kernels_are_not_for(device):
         assert head_loss(head, z[:, ::2], y[:, ::2]) is None
         assert head_loss(head, z, y.double()) is None
         assert head_loss(head.half(), z, y) is None
+
+
+def _through_the_model(device):
+    """A training step's loss as a function of nothing, and its head."""
+    import ar_nanotabpfn_amd.model as model_mod
+    from ar_nanotabpfn_amd.attention import create_dense_mask, create_row_mask
+
+    torch.manual_seed(1)
+    model = model_mod.ARTabPFN(d_model=128, n_heads=4, n_layers=1, d_ff=256, num_features=2, buffer_size=4, num_components=5).to(device)
+    mk = lambda *s: torch.randn(*s, generator=torch.Generator().manual_seed(2)).to(device)  # noqa: E731
+    data, y = (mk(3, 17, 2), mk(3, 17), mk(3, 4, 2), mk(3, 4), mk(3, 12, 2)), mk(3, 12)
+    masks = (create_dense_mask(1), create_row_mask(33, 17, 4))
+
+    def loss():
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            return model(*data, *masks, y_target=y)
+    return loss, model.head
+
+
+def test_tangents_of_head_parameters(device):
+    """Forward-mode differentiation in the head's parameters: along a direction, what the gradients give."""
+    import torch.autograd.forward_ad as fwad
+
+    loss, head = _through_the_model(device)
+    bias = head.mean_bias
+    (grad,) = torch.autograd.grad(loss(), bias)
+    direction = torch.linspace(-1.0, 2.0, bias.numel(), device=device)
+    with fwad.dual_level():
+        del head.mean_bias
+        head.mean_bias = fwad.make_dual(bias.detach(), direction)
+        tangent = fwad.unpack_dual(loss()).tangent
+    # (the modules' bf16 products here, the kernels' there: five roundings of at most 2^-9, twice)
+    assert abs(float(tangent) - float(grad @ direction)) <= 2 * 5 * 2.0 ** -9 * float(grad.norm() * direction.norm())
+
+
+def test_batched_gradients_of_head_parameters(device):
+    loss, head = _through_the_model(device)
+    out, params = loss(), list(head.parameters())
+    want = torch.autograd.grad(out, params, retain_graph=True)
+    scales = torch.tensor([1.0, -0.5, 3.0], device=device)
+    got = torch.autograd.grad(out, params, grad_outputs=scales, is_grads_batched=True)
+    for g, w in zip(got, want):  # (the modules' products here, the kernels' there, as above)
+        assert g.shape == (3, *w.shape)
+        assert float((g - scales.view(-1, *[1] * w.dim()) * w).norm()) <= 2 * 2 * 5 * 2.0 ** -9 * float((scales.norm() * w.norm()))
