@@ -20,6 +20,10 @@ pytestmark = pytest.mark.gpu
     (4, 8, 32, 256, 500),    # 64
     (16, 8, 64, 200, 516),   # head_dim 64: 128
     (2, 8, 64, 100, 33),     # 64
+    (1, 8, 32, 1500, 1999),  # 256: 64 workgroups, long keys
+    (2, 4, 32, 900, 1025),   # 128: 40 workgroups of 256 rows, fewer than they are worth there
+    (4, 8, 64, 500, 300),    # head_dim 64, half the chip at 128 rows: 64 in bf16
+    (8, 8, 64, 400, 440),    # 448 rows against 512: 64 in bf16
 ])
 def test_unsplit_calls(device, dtype, B, H, D, Nc, rows):
     import ar_nanotabpfn_amd.attention_kernels as ak
