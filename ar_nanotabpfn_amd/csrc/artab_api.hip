@@ -223,10 +223,12 @@ static FlashPlan plan_flash(int B, int H, int Lq, int Nc, int Dh, bool stacked, 
 // merge are faster from about 1000 rows on (shorter ones go to context_small_kernel, on one compute unit each).  The choice weighs estimates in microseconds, fitted to
 // launches of 200 to 16384 rows, 4 to 16 heads, 1 to 16 tables (bf16; f16 gains more everywhere): a
 // compute unit takes 12 ns per key for one tile, 17 for a pair, a slice costs 5 to start, the merge 5 and
-// its traffic at 3.5 TB/s; unsliced launches of small tiles take 12.5 to 21 ns per key, the more wavefronts
-// share a SIMD.  Unsliced -> sliced: 1 x 16 x 2048 37.7 -> 26.4, 1 x 8 x 4096 67 -> 36, 5001 81 -> 47, 9000 174 -> 122,
+// its traffic at 3.5 TB/s; unsliced launches, in the tiles that unsliced_tile cuts, the same with 256 rows and 12.5 to 21 ns
+// per key with fewer, the more wavefronts share a SIMD.  Over 144 such launches the choice is 0.9 % (f16 2.1) above the best of
+// 1 to 8 slices on average, at most 13 (14); with the unsliced launch taken to be in smaller tiles than it is 2.8 and 34 (4 x 8 x
+// 1600 rows 25 us, sliced in two 33; 2 x 8 x 3300 43 and 48).  Unsliced -> sliced: 1 x 16 x 2048 37.7 -> 26.4, 1 x 8 x 4096 67 -> 36, 5001 81 -> 47, 9000 174 -> 122,
 // 12000 256 -> 185, 1 x 16 x 9000 246 -> 225; 4 x 8 x 1024 20.9 against 20.5, 8 x 8 x 512 14.2 against 17.8: not sliced.
-static int prefill_slices(int B, int H, int Nc, int Dh) {
+static int prefill_slices(int B, int H, int Nc, int Dh, bool bf16) {
     if (Dh != 32) return 1;
     const int forced = tune(kTuneSplit, 0);
     if (forced > 0) return forced;
@@ -236,8 +238,7 @@ static int prefill_slices(int B, int H, int Nc, int Dh) {
         const long q = (wgs + 255) / 256;
         return static_cast<double>((q + 1) / 2) * 5.0 + keys * (17e-3 * (q / 2) + 12e-3 * (q % 2));
     };
-    int bm = 256;
-    while (bm > 64 && (Nc + bm - 1) / bm * pairs < 512) bm /= 2;
+    const int bm = unsliced_tile(Nc, pairs, Nc, Dh, bf16);
     double best = bm == 256 ? wide(Nc, tiles)
                             : 4.5 + Nc * (12.5e-3 + 3e-3 * ((Nc + bm - 1) / bm * pairs * (bm / 32) / 1024.0));
     int slices = 1;
@@ -1230,7 +1231,7 @@ static int prefill_impl(const artab_view *q, const artab_view *k, const artab_vi
         const hipError_t e = dtype == ARTAB_BF16 ? launch_context_small<bf16_t>(S, Dh, B, st) : launch_context_small<f16_t>(S, Dh, B, st);
         return launch_status(e, "prefill (small)");
     }
-    const int slices = prefill_slices(B, H, Nc, Dh);
+    const int slices = prefill_slices(B, H, Nc, Dh, dtype == ARTAB_BF16);
     FlashPlan pl = plan_flash(B, H, Nc, Nc, Dh, /*stacked=*/false, /*allow_split=*/false, dtype == ARTAB_BF16);
     if (slices > 1 && workspace && workspace_bytes >= f32_workspace_bytes(rows, Dh, slices) &&
         reinterpret_cast<uintptr_t>(workspace) % 16 == 0) {
@@ -1270,7 +1271,7 @@ static int prefill_impl(const artab_view *q, const artab_view *k, const artab_vi
 size_t artab_prefill_workspace_bytes(int B, int H, int Nc, int Dh, int dtype) {
     if (B <= 0 || H <= 0 || Nc <= 0 || !mfma_shape_ok(dtype, Dh)) return 0;
     if (context_small_applies(H, Nc, Dh, static_cast<long>((Nc + kContextSmallRows - 1) / kContextSmallRows) * B, dtype)) return 0;
-    const int slices = prefill_slices(B, H, Nc, Dh);
+    const int slices = prefill_slices(B, H, Nc, Dh, dtype == ARTAB_BF16);
     return slices > 1 ? f32_workspace_bytes(static_cast<long>(B) * H * Nc, Dh, slices) : 0;
 }
 
