@@ -336,9 +336,14 @@ static hipError_t launch_context_small(const ContextSmallParams &P, int Dh, int 
 // where a persistent one goes on from task to task.  us per layer with its context pass, three against 32 per unit (and against two of
 // 32 KiB each, what fitted while a workgroup held two query regions): B*H = 32768, 4096 context rows, 64 buffer rows 84 / 102 / 107,
 // 128 rows 122 / 137 / 139, 248 rows 199 / 206 / 201; B*H = 8192, 16384 context rows, 128 rows 59 / 67, 248 rows 73 / 91; four
-// per unit 142 and 232, 61 and 77.  With the device to itself (no second stream): one workgroup per task up to 32 per unit; which
+// per unit 142 and 232, 61 and 77.  Contexts that are over at once: means of 8 to 248 buffer rows, three / four / 32 per unit
+// beside 64 rows: B*H = 32768 110 / 110 / 110, 24576 86 / 87 / 88, 16384 65 / 64 / 64, 12288 50 / 51 / 51, 8192 and 4096 alike.
+// (One stream alone, without fork and join, is shorter beside up to 256 rows: 64 rows 108, 59.5 and 39 at 32768, 16384 and 8192
+// where two take 110, 64 and 41; 512 rows as long.)
+// With the device to itself (no second stream): one workgroup per task up to 32 per unit; which
 // wavefront takes which task is then the dispatcher's decision, made when a slot frees up (B*H = 32768, 256
 // steps: 500 target-steps/s with 4 per CU, 506 with 6, 508 with 16, 512 with 32).
+constexpr int kStreamBeside = 3;
 template <typename T>
 static hipError_t launch_stream_t(const DecodeParams &P, int Lq, bool beside, hipStream_t stream) {
     const long pairs = static_cast<long>(P.B) * P.H;
@@ -348,7 +353,7 @@ static hipError_t launch_stream_t(const DecodeParams &P, int Lq, bool beside, hi
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
         cus = 256;
     const long tasks = (pairs + 3) / 4;  // of the 4-pair chunk shape; the 16-pair shape leaves the surplus idle
-    long per_cu = beside ? 3 : 32;
+    long per_cu = beside ? kStreamBeside : 32;
     if (const int v = tune(kTuneStreamPerCu, 0); v >= 1 && v <= 32) per_cu = v;
     dim3 grid(static_cast<unsigned>(tasks < per_cu * cus ? tasks : per_cu * cus)), block(64);
     const int prio = tune(kTuneStreamPrio, 3);
@@ -840,10 +845,13 @@ static int decode_impl(const artab_view *q, const artab_view *k_ctx, const artab
         // the raised priority it only takes issue slots from that one (measured at B=1024, H=8:
         // base priority +1.0 % target-steps/s over steps 0..63, -3 % over steps 64..95; the buffers
         // hold 64 MiB at the switch).  Only while one round of tasks covers all pairs (16 pairs per
-        // task, two wavefronts per compute unit beside the context pass): with more rounds than
+        // task, kStreamBeside wavefronts per compute unit beside the context pass): with more rounds than
         // that the pass is nearly as long as its neighbour from the first row on (B=2048, H=16:
-        // -0.3 % with a switch at 16 rows, so none there).
-        const long one_round = 16L * 2 * 256;
+        // -0.3 % with a switch at 16 rows, so none there).  Between 8192 pairs, one round of two
+        // wavefronts, and that, means of 8 to 104 buffer rows without a switch and with it: 10240 pairs
+        // beside 4096 context rows 40.1 and 39.8 us a layer, beside 16384 80.1 and 79.5; 12288 pairs 48.1
+        // and 48.0, 94.1 and 93.5.
+        const long one_round = 16L * kStreamBeside * 256;
         const long calm = per_row > 0 && static_cast<long>(B) * H <= one_round ? (64L << 20) / per_row : 0;
         D.stream_calm_rows = tune(kTuneStreamCalm, static_cast<int>(calm < 1 << 20 ? calm : 1 << 20));
     }
@@ -856,7 +864,9 @@ static int decode_impl(const artab_view *q, const artab_view *k_ctx, const artab
         // waits for.  Estimated from the work: buffer bytes at 5 TB/s against context flops at
         // 900 TFLOP/s, switch at 0.8 of the context pass's time (146 rows at B=1024, H=8,
         // N_ctx=16384; 36 at B=2048, H=16, N_ctx=4096).  Measured: +0.9 % target-steps/s over 256
-        // steps at the first shape (switch anywhere in 128..192), +1.0 % at the second.
+        // steps at the first shape (switch anywhere in 128..192), +1.0 % at the second, with two
+        // wavefronts of the buffer pass per unit; with three of them no switch between 24 rows and never
+        // is more than 1 % from another (56.1 us a layer over 8 to 248 rows at the first, 119.3 at the second).
         const double ctx_flops = 4.0 * B * H * Lq * static_cast<double>(Nc) * Dh;
         const double per_row = static_cast<double>(B) * H * 2 * Dh * 2;
         const double yield_rows = per_row > 0 ? ctx_flops * 4.4e-3 / per_row : 0;
