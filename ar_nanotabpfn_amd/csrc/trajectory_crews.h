@@ -14,8 +14,11 @@
 //
 // Measured, us per layer and step, one crew / two, 64 trajectories on a shared context: bf16, d_model 128, 8.6 / 6.9 at
 // 64 rows, 9.6 / 7.4 at 200, 12.1 / 10.7 at 700, 17.5 / 16.6 at 1500, 26.3 / 26.8 at 3000; d_model 256, 15.4 / 13.1 at 64,
-// 17.1 / 15.6 at 200, 22.8 / 22.3 at 700, 32.5 / 32.9 at 1500; float32, d_model 128, 20.2 / 17.5 at 200, 54.2 / 48.9 at 2000;
-// d_model 256, 42.6 / 35.0 and 110.5 / 98.3.  Long contexts in 16 bits are bound by the stream of keys from the L2,
+// 17.1 / 15.6 at 200, 21.1 / 20.2 at 600, 22.6 / 22.8 at 768, 32.5 / 32.9 at 1500; float32, d_model 128, 20.2 / 17.5 at 200,
+// 54.2 / 48.9 at 2000; d_model 256, 42.6 / 35.0 and 110.5 / 98.3.  Contexts of their own, bf16, d_model 128: 64 trajectories 17.9 /
+// 16.6 at 1200, 29.6 / 29.3 at 2000, 35.6 / 35.2 at 2600; 192 of them 26.6 / 25.7 at 1200; 256 13.4 / 11.5 at 300, 17.2 / 17.3 at 500,
+// 21.4 / 21.7 at 700, 37.0 / 37.6 at 1500; d_model 256: 64 30.5 / 29.7 at 768, 38.6 / 38.0 at 1000, 44.4 / 44.9 at 1300; 192 45.1 / 44.4 at
+// 850; 256 39.2 / 37.5 at 500, 45.8 / 45.6 at 700, 47.6 / 48.4 at 768 (f16 alike).  Long contexts in 16 bits are bound by the stream of keys from the L2,
 // which eight wavefronts with twice the registers ask for a little better: crews_serve() draws the line.
 // Not kept: crew 0 taking a share of a long context's keys (its registers do not hold them beside the weights: 9.2
 // instead of 7.0 ms for 64 x 512 own rows); workgroups half a layer apart (no difference: it is not the memory they
@@ -26,10 +29,13 @@
 
 namespace artab {
 
-// Whether these run here (G = 1) and not on one crew: both sides measured above, between 1500 and 3000 rows at d_model
-// 128 and between 700 and 1000 at 256.
+// Whether these run here (G = 1) and not on one crew: both sides measured above.  The lines of 16 bits lie where a shared
+// context crosses; contexts of their own cross later, but for those of nearly every compute unit, which together wait for memory
+// and not for their units.
 inline bool crews_serve(const TrajectoryParams &P, int D, bool f32) {
-    return P.G == 1 && (D == 128 || D == 256) && (f32 || P.n_ctx + P.own_base + P.Nt / 2 <= (D == 128 ? 2048 : 768));
+    const bool memory = P.own_base > 0 && P.B > 192;
+    return P.G == 1 && (D == 128 || D == 256) &&
+           (f32 || P.n_ctx + P.own_base + P.Nt / 2 <= (D == 128 ? (memory ? 448 : 2048) : (memory ? 704 : 768)));
 }
 
 // The first N of a buffer's fragments.
