@@ -1355,12 +1355,11 @@ int artab_add_layernorm(const void *x, int64_t ldx, const void *y, int64_t ldy, 
         return fail(ARTAB_ERR_UNSUPPORTED, "add_layernorm needs D %% 4 == 0 and D <= %d (got %d)", 256 * kGlueMaxPerLane, D);
     if (rows == 0) return ARTAB_OK;
     if (!x || !gamma || !beta || !out) return fail(ARTAB_ERR_NULL_POINTER, "x, gamma, beta and out are required");
-    const int64_t per = 16 / elem_size(dtype) / 2;  // 4-element vectors: 8 bytes (16-bit) or 16 bytes (float32)
+    // 4-element vectors: 8 bytes (16-bit) or 16 bytes (float32)
     const uintptr_t align = dtype == ARTAB_F32 ? 16 : 8;
     auto bad = [&](const void *p) { return p && reinterpret_cast<uintptr_t>(p) % align != 0; };
     if (bad(x) || bad(y) || bad(bias) || bad(gamma) || bad(beta) || bad(out) || ldx % 4 || (y && ldy % 4))
         return fail(ARTAB_ERR_BAD_STRIDE, "add_layernorm operands must be aligned to 4 elements");
-    (void)per;
     AddLayerNormParams P;
     P.x = x; P.y = y; P.bias = bias; P.gamma = gamma; P.beta = beta; P.out = out;
     P.rows = rows; P.ldx = ldx; P.ldy = ldy; P.D = D; P.eps = eps;

@@ -510,7 +510,7 @@ __global__ __launch_bounds__(2 * kTrajWaves * 64) void trajectory_crews_kernel(T
     // The same in float32: the two tokens are columns 0 and 1 of four (and 2 and 3 again); 16 keys per block.
     auto attention_f32 = [&](int h, int t, auto &keys) {
         const Lane me = here();
-        const int lane = me.lane, quad = me.quad(), sub = me.sub(), tok = me.tok();
+        const int lane = me.lane, quad = me.quad(), sub = me.sub();
         u32x4 qf[2];
 #pragma unroll
         for (int x = 0; x < 2; ++x) qf[x] = *reinterpret_cast<const u32x4 *>(qs + me.row() * LD + DH * h + Ops::kStep * x + Ops::kPer * quad);
@@ -594,7 +594,6 @@ __global__ __launch_bounds__(2 * kTrajWaves * 64) void trajectory_crews_kernel(T
             Ops::finish(o_acc[db]);
             a_o[db] = o_acc[db];
         }
-        (void)tok;
     };
     auto attention = [&](int h, int t, auto &keys) {
         if constexpr (k16) attention_16(h, t, keys);

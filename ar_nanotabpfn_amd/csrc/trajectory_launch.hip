@@ -85,11 +85,13 @@ hipError_t decode(const TrajectoryParams &P, int D, int F, hipStream_t st) {
                 return;
             }
         }
-        if (P.G > 1)
+        if (P.G > 1) {
             hipLaunchKernelGGL((trajectory_decode_kernel<T, decltype(d)::value, decltype(f)::value, true>), grid, block, 0, st, P);
-        else
+            e = hipGetLastError();
+        } else if constexpr (sizeof(T) == 2) {  // (in float32 the crews take all of them)
             hipLaunchKernelGGL((trajectory_decode_kernel<T, decltype(d)::value, decltype(f)::value, false>), grid, block, 0, st, P);
-        e = hipGetLastError();
+            e = hipGetLastError();
+        }
     });
     return e;
 }
