@@ -25,7 +25,8 @@ def _f64(t):
 
 @pytest.mark.parametrize("dtype", list(BOUND), ids=["bf16", "f16", "f32"])
 @pytest.mark.parametrize("backend", ["triton_shared_context", "flex_attention"], ids=["shared", "own"])
-@pytest.mark.parametrize("D,Nc,group", [(128, 3, 1), (128, 40, 3), (256, 33, 1)])
+# (d_model 128 with 300 rows, 256 with 150 and 300: a second and a third group of keys to every wavefront of a head)
+@pytest.mark.parametrize("D,Nc,group", [(128, 3, 1), (128, 40, 3), (256, 33, 1), (128, 300, 1), (256, 150, 1), (256, 300, 1)])
 def test_whole_run_against_float64(device, monkeypatch, tuning, dtype, backend, D, Nc, group):
     from ar_nanotabpfn_amd.glue import TrajectoryDecoder
     from ar_nanotabpfn_amd.inference import ARTabPFNPredictor
