@@ -58,14 +58,14 @@ def test_loss_and_gradients(device, D, K, B, T):
     exact, exact_grads = _modules_in(torch.float64, head, z, y)
     auto, auto_grads = _modules_in(torch.float32, head, z, y, autocast=True)
     loss, grads = _kernels(head, z, y)
-    # five roundings of at most 2^-9 in raw outputs of the order of one, which enter with 1 / 0.5
-    assert abs(loss.item() - exact.item()) <= 2e-2 * max(1.0, abs(exact.item()))
-    # z, W_1, the hidden layer, W_2, the raw outputs' gradient: five roundings of at most 2^-9, times 1 / 0.5; and the
-    # modules' error, which has the same ones: both norms are those of the few rows whose y lies far out, where a
-    # component's t^2 multiplies them, one draw of the roundings each
+    # five roundings of at most 2^-9, of random sign, in raw outputs of the order of one, which enter with 1 / 0.5
+    assert abs(loss.item() - exact.item()) <= 5 * 2.0 ** -9 * max(1.0, abs(exact.item()))
+    # z, W_1, the hidden layer, W_2, the raw outputs' gradient are rounded as in the modules.  Both errors are those of the few
+    # rows whose y lies far out, where a component's t^2 multiplies them, one draw of the roundings each: some ten such rows,
+    # whose norms differ by a third from draw to draw; and a rounding where the modules happen to have none (1 or 2 rows)
     for got, ref, module in zip(grads, exact_grads, auto_grads):
         error, theirs = ((g.double() - ref).norm() for g in (got, module))
-        assert error <= theirs + 2 * 5 * 2.0 ** -9 * ref.norm() + 1e-9, (tuple(got.shape), error.item(), theirs.item())
+        assert error <= 1.5 * theirs + 2.0 ** -9 * ref.norm() + 1e-9, (tuple(got.shape), error.item(), theirs.item())
     if B * T >= 1000:  # the ordinary row is not further off than with the modules
         ours, theirs = (((g[0].double() - exact_grads[0]).norm(dim=2) / exact_grads[0].norm(dim=2)).median() for g in (grads, auto_grads))
         assert ours <= theirs
