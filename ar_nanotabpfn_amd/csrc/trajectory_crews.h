@@ -97,12 +97,8 @@ __global__ __launch_bounds__(2 * kTrajWaves * 64) void trajectory_crews_kernel(T
     // the parameter vectors of this layer and of the next; cache addresses of every layer
     __shared__ __attribute__((aligned(16))) T pbuf[2][8 * VW];
     __shared__ unsigned long long kv_s[4 * kTrajMaxLayers];
-    // what the end of every step needs: norm g and b, x and y embedding w and b, markers target and
-    // buffer; the head's biases; the position token of the coming step
-    __shared__ __attribute__((aligned(16))) T cst[8 * D + F + kTrajHeadOut + 3 * kTrajMaxMix + 1], tok_s[D];
-    T *const c_ng = cst, *const c_nb = cst + D, *const c_wx = cst + 2 * D, *const c_bx = cst + 3 * D, *const c_wy = cst + 4 * D,
-             *const c_by = cst + 5 * D, *const c_mt = cst + 6 * D, *const c_mb = cst + 7 * D, *const c_b1 = cst + 8 * D,
-             *const c_b2 = c_b1 + F, *const c_mix = c_b2 + kTrajHeadOut;
+    __shared__ __attribute__((aligned(16))) T cst[TrajConstants<T, D, F>::kElems], tok_s[D];  // and the position token of the coming step
+    const TrajConstants<T, D, F> C(cst);
 
     const int tid = threadIdx.x, warp = __builtin_amdgcn_readfirstlane(tid >> 6), wave = warp & (NW - 1), lane = tid & 63;
     const int ctid = tid & (NTC - 1);                       // within the crew
@@ -607,31 +603,14 @@ __global__ __launch_bounds__(2 * kTrajWaves * 64) void trajectory_crews_kernel(T
     if (tid < kPieces) reinterpret_cast<u32x4 *>(pbuf[0])[tid] = vec_src[tid];
     for (int i = tid; i < 4 * P.n_layers; i += NT) kv_s[i] = P.kv[i];
     const T *const xm = static_cast<const T *>(P.x_mean);
-    for (int d = tid; d < D; d += NT) {
-        c_ng[d] = static_cast<const T *>(P.norm_g)[d];
-        c_nb[d] = static_cast<const T *>(P.norm_b)[d];
-        c_wx[d] = static_cast<const T *>(P.w_x)[d];
-        c_bx[d] = static_cast<const T *>(P.b_x)[d];
-        c_wy[d] = static_cast<const T *>(P.w_y)[d];
-        c_by[d] = static_cast<const T *>(P.b_y)[d];
-        c_mt[d] = static_cast<const T *>(P.markers)[d];
-        c_mb[d] = static_cast<const T *>(P.markers)[2 * D + d];
-    }
-    for (int d = tid; d < F; d += NT) c_b1[d] = static_cast<const T *>(P.b_h1)[d];
+    C.template load<NT>(P, tid);
     if (tid == 0) {
         eps_s[0] = P.eps1;
         eps_s[1] = P.eps2;
         eps_s[2] = P.eps3;
     }
-    if (tid < kTrajHeadOut) c_b2[tid] = static_cast<const T *>(P.b_h2)[tid];
-    if (tid < 3 * P.K) c_mix[tid] = static_cast<const T *>(P.mix)[tid];
     __syncthreads();
-    for (int i = tid; i < NR * D; i += NT) {
-        const int r = i / D, d = i % D;
-        float v = 0.f;
-        if (r == 1) v = to_f32(xm[b * P.Nt]) * to_f32(c_wx[d]) + to_f32(c_bx[d]) + to_f32(c_mt[d]);
-        xs[r * LD + d] = from_f32<T>(v);
-    }
+    C.template first_rows<NT>(P, b, 1, NR, xs, LD, tid);
     __syncthreads();
 
     // ---- the run, written once for both crews: every barrier is one of both.
@@ -730,15 +709,8 @@ __global__ __launch_bounds__(2 * kTrajWaves * 64) void trajectory_crews_kernel(T
                     if constexpr (kW2Early) ask(f_2, at + S::p2, from0, integral_constant<int, w2>{});
                     // the caches: row 0 is committed at slot t - 1 (its first read is a step away); behind the last one
                     // the target row, where the caller keeps it
-                    constexpr int CPR = DH * sizeof(T) / 16, PER = H * CPR;  // 16-byte pieces of a head's row, of a row
                     auto commit = [&](int from, int slot) {
-                        const Global ck = layer_kv(l, 2), cv = layer_kv(l, 3);
-                        for (int i = ctid; i < 2 * PER; i += NTC) {
-                            const int c = i % PER, which = i / PER;
-                            const Global dst = (which ? cv : ck) + ((b * H + c / CPR) * P.own_rows + slot) * static_cast<long>(DH * sizeof(T)) + 16 * (c % CPR);
-                            *(__attribute__((address_space(1))) u32x4 *)dst =
-                                *reinterpret_cast<const u32x4 *>((which ? vn : kn) + from * LD + c * (16 / sizeof(T)));
-                        }
+                        traj_commit<T, D, NTC>(layer_kv(l, 2), layer_kv(l, 3), kn, vn, LD, b, 1, P.own_rows, from, slot, ctid);
                     };
                     if (t > 0) commit(0, P.own_base + t - 1);
                     if (P.park_target && last_step) commit(1, P.own_base + t);
@@ -830,16 +802,14 @@ __global__ __launch_bounds__(2 * kTrajWaves * 64) void trajectory_crews_kernel(T
                     for (int e = 0; e < EPL; ++e) q += (x[e] - mean) * (x[e] - mean);
                     const float rstd = rsqrtf(row_sum(lanes16_sum(q)) / D + P.eps_out);
 #pragma unroll
-                    for (int e = 0; e < EPL; ++e)
-                        ys[r * LD + lane * EPL + e] =
-                            from_f32<T>((x[e] - mean) * rstd * to_f32(c_ng[lane * EPL + e]) + to_f32(c_nb[lane * EPL + e]));
+                    for (int e = 0; e < EPL; ++e) ys[r * LD + lane * EPL + e] = C.normed(x[e], mean, rstd, lane * EPL + e);
                 }
             }
             __syncthreads();
             if constexpr (kB) {
                 f32x4 acc[S::NF];
                 product(acc, first<w1>(f_b), head_at, integral_constant<int, S::KD>{}, ys, LD);
-                gelu_store(acc, c_b1);
+                gelu_store(acc, C.b1);
             }
             __syncthreads();
             if constexpr (kA) {
@@ -848,7 +818,7 @@ __global__ __launch_bounds__(2 * kTrajWaves * 64) void trajectory_crews_kernel(T
                 const Lane ln = here();
                 if (16 * wave < kTrajHeadOut && ln.writes()) {
                     float bias[4];
-                    traj_load4<T>(c_b2 + 16 * wave + 4 * ln.sub(), bias);
+                    traj_load4<T>(C.b2 + 16 * wave + 4 * ln.sub(), bias);
 #pragma unroll
                     for (int e = 0; e < 4; ++e) raw_s[ln.row()][16 * wave + 4 * ln.sub() + e] = acc[0][e] + bias[e];
                 }
@@ -862,7 +832,7 @@ __global__ __launch_bounds__(2 * kTrajWaves * 64) void trajectory_crews_kernel(T
                 ask(f_qkv, S::pQkv, from0, integral_constant<int, kQkvEarly>{});
                 if (wave == 0) {  // a lane per component
                     const float *raw = raw_s[1];
-                    const T *const mix = c_mix;
+                    const T *const mix = C.mix;
                     const int k = min(lane, P.K - 1);
                     const float logit = raw[3 * k + 2] + to_f32(mix[2 * P.K + k]);
                     const float mx = row_max(lanes16_max(logit));
@@ -875,10 +845,7 @@ __global__ __launch_bounds__(2 * kTrajWaves * 64) void trajectory_crews_kernel(T
                     }
                     const unsigned long long past = __ballot(lane < P.K && upto > my_u * cum);
                     const int comp = past ? __builtin_ctzll(past) : P.K - 1;
-                    const float mean = raw[3 * comp] + to_f32(mix[comp]);
-                    const float sraw = raw[3 * comp + 1] + to_f32(mix[P.K + comp]);
-                    const float sp = sraw > 20.f ? sraw : log1pf(expf(sraw));
-                    const T y = from_f32<T>(mean + (fminf(sp, P.std_max) + P.std_min) * my_n);
+                    const T y = C.value(P, raw, comp, my_n);
                     if (lane == 0) {
                         static_cast<T *>(P.preds)[b * P.Nt + t] = y;
                         y_s = to_f32(y);
@@ -887,27 +854,7 @@ __global__ __launch_bounds__(2 * kTrajWaves * 64) void trajectory_crews_kernel(T
             }
             __syncthreads();
             if (last_step) break;
-            for (int i = tid; i < 2 * (D / 4); i += NT) {
-                const int d = 4 * (i % (D / 4)), r = i / (D / 4);
-                float wx[4], bx[4], m[4], o[4];
-                traj_load4<T>(c_wx + d, wx);
-                traj_load4<T>(c_bx + d, bx);
-                traj_load4<T>((r & 1 ? c_mt : c_mb) + d, m);
-                const float xv = x_s[r];
-                if (r & 1) {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) o[e] = xv * wx[e] + bx[e] + m[e];
-                } else {
-                    float wy[4], by[4], tk[4];
-                    traj_load4<T>(c_wy + d, wy);
-                    traj_load4<T>(c_by + d, by);
-                    traj_load4<T>(tok_s + d, tk);
-                    const float yv = y_s;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) o[e] = xv * wx[e] + bx[e] + yv * wy[e] + by[e] + m[e] + tk[e];
-                }
-                traj_store4<T>(xs + r * LD + d, o);
-            }
+            C.template next_rows<NT>(x_s, &y_s, tok_s, 1, xs, LD, tid);
             __syncthreads();
         }
     };

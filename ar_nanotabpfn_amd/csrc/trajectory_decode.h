@@ -191,6 +191,96 @@ __global__ void trajectory_tape_kernel(const T *w, char *tape, long tape_stride,
     *reinterpret_cast<u32x4 *>(tape + wave * tape_stride + (static_cast<long>(first) + ks * stride + offset + b) * 1024 +
                                16 * lane) = v;
 }
+// ---- what the one-crew and the two-crew kernel (trajectory_crews.h) have in common at both ends of a step
+
+// What the end of every step needs, in LDS: norm g and b, x and y embedding w and b, markers target and buffer; the
+// head's biases.
+template <typename T, int D, int F>
+struct TrajConstants {
+    static constexpr int kElems = 8 * D + F + kTrajHeadOut + 3 * kTrajMaxMix + 1;
+    T *ng, *nb, *wx, *bx, *wy, *by, *mt, *mb, *b1, *b2, *mix;
+    __device__ __forceinline__ explicit TrajConstants(T *at)
+        : ng(at), nb(at + D), wx(at + 2 * D), bx(at + 3 * D), wy(at + 4 * D), by(at + 5 * D), mt(at + 6 * D), mb(at + 7 * D),
+          b1(at + 8 * D), b2(b1 + F), mix(b2 + kTrajHeadOut) {}
+    template <int NT>
+    __device__ __forceinline__ void load(const TrajectoryParams &P, int tid) const {
+        for (int d = tid; d < D; d += NT) {
+            ng[d] = static_cast<const T *>(P.norm_g)[d];
+            nb[d] = static_cast<const T *>(P.norm_b)[d];
+            wx[d] = static_cast<const T *>(P.w_x)[d];
+            bx[d] = static_cast<const T *>(P.b_x)[d];
+            wy[d] = static_cast<const T *>(P.w_y)[d];
+            by[d] = static_cast<const T *>(P.b_y)[d];
+            mt[d] = static_cast<const T *>(P.markers)[d];
+            mb[d] = static_cast<const T *>(P.markers)[2 * D + d];
+        }
+        for (int d = tid; d < F; d += NT) b1[d] = static_cast<const T *>(P.b_h1)[d];
+        if (tid < kTrajHeadOut) b2[tid] = static_cast<const T *>(P.b_h2)[tid];
+        if (tid < 3 * P.K) mix[tid] = static_cast<const T *>(P.mix)[tid];
+    }
+    // The rows of step 0, `rows` of them from trajectory b0 on: the target rows of `valid` trajectories, zero elsewhere.
+    template <int NT>
+    __device__ __forceinline__ void first_rows(const TrajectoryParams &P, long b0, int valid, int rows, T *xs, int ld, int tid) const {
+        const T *const xm = static_cast<const T *>(P.x_mean);
+        for (int i = tid; i < rows * D; i += NT) {
+            const int r = i / D, d = i % D, g = r >> 1;
+            float v = 0.f;
+            if ((r & 1) && g < valid) v = to_f32(xm[(b0 + g) * P.Nt]) * to_f32(wx[d]) + to_f32(bx[d]) + to_f32(mt[d]);
+            xs[r * ld + d] = from_f32<T>(v);
+        }
+    }
+    // The rows of the next step: buffer row 2 g with the value just drawn and the position's token, target row 2 g + 1.
+    template <int NT>
+    __device__ __forceinline__ void next_rows(const float *x_s, const float *y_s, const T *tok_s, int valid, T *xs, int ld, int tid) const {
+        for (int i = tid; i < 2 * valid * (D / 4); i += NT) {
+            const int d = 4 * (i % (D / 4)), r = i / (D / 4);
+            float w[4], b[4], m[4], o[4];
+            traj_load4<T>(wx + d, w);
+            traj_load4<T>(bx + d, b);
+            traj_load4<T>((r & 1 ? mt : mb) + d, m);
+            const float xv = x_s[r];
+            if (r & 1) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o[e] = xv * w[e] + b[e] + m[e];
+            } else {
+                float w2[4], b2[4], tk[4];
+                traj_load4<T>(wy + d, w2);
+                traj_load4<T>(by + d, b2);
+                traj_load4<T>(tok_s + d, tk);
+                const float yv = y_s[r >> 1];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o[e] = xv * w[e] + b[e] + yv * w2[e] + b2[e] + m[e] + tk[e];
+            }
+            traj_store4<T>(xs + r * ld + d, o);
+        }
+    }
+    // The final norm of a row, its element from mean and 1 / std.
+    __device__ __forceinline__ T normed(float x, float mean, float rstd, int d) const {
+        return from_f32<T>((x - mean) * rstd * to_f32(ng[d]) + to_f32(nb[d]));
+    }
+    // The value of component `comp` of a row's raw outputs, from a standard normal variate.
+    __device__ __forceinline__ T value(const TrajectoryParams &P, const float *raw, int comp, float normal) const {
+        const float mean = raw[3 * comp] + to_f32(mix[comp]);
+        const float sraw = raw[3 * comp + 1] + to_f32(mix[P.K + comp]);
+        const float sp = sraw > 20.f ? sraw : log1pf(expf(sraw));
+        return from_f32<T>(mean + (fminf(sp, P.std_max) + P.std_min) * normal);
+    }
+};
+
+// Keys and values of token row 2 g + `from` to row `slot` of the cache of trajectory b0 + g.
+template <typename T, int D, int NT>
+__device__ __forceinline__ void traj_commit(__attribute__((address_space(1))) char *ck, __attribute__((address_space(1))) char *cv,
+                                            const T *kn, const T *vn, int ld, long b0, int valid, int own_rows, int from, int slot, int tid) {
+    constexpr int DH = 32, H = D / DH, CPR = DH * sizeof(T) / 16, PER = H * CPR;  // 16-byte pieces of a head's row, of a row
+    for (int i = tid; i < valid * 2 * PER; i += NT) {
+        const int c = i % PER, which = i / PER & 1, g = i / (2 * PER);
+        __attribute__((address_space(1))) char *const dst =
+            (which ? cv : ck) + (((b0 + g) * H + c / CPR) * own_rows + slot) * static_cast<long>(DH * sizeof(T)) + 16 * (c % CPR);
+        *(__attribute__((address_space(1))) u32x4 *)dst =
+            *reinterpret_cast<const u32x4 *>((which ? vn : kn) + (2 * g + from) * ld + c * (16 / sizeof(T)));
+    }
+}
+
 // SEVERAL: G > 1.  (One trajectory has no columns to keep apart: doing it all the same costs 3 % of a run.)
 template <typename T, int D, int F, bool SEVERAL>
 __global__ __launch_bounds__(kTrajWaves * 64) void trajectory_decode_kernel(TrajectoryParams P) {
@@ -223,12 +313,8 @@ __global__ __launch_bounds__(kTrajWaves * 64) void trajectory_decode_kernel(Traj
     // the parameter vectors of this layer and of the next; cache addresses of every layer
     __shared__ __attribute__((aligned(16))) T pbuf[2][8 * VW];
     __shared__ unsigned long long kv_s[4 * kTrajMaxLayers];
-    // what the end of every step needs: norm g and b, x and y embedding w and b, markers target and
-    // buffer; the head's biases; the position token of the coming step
-    __shared__ __attribute__((aligned(16))) T cst[8 * D + F + kTrajHeadOut + 3 * kTrajMaxMix + 1], tok_s[D];
-    T *const c_ng = cst, *const c_nb = cst + D, *const c_wx = cst + 2 * D, *const c_bx = cst + 3 * D, *const c_wy = cst + 4 * D,
-             *const c_by = cst + 5 * D, *const c_mt = cst + 6 * D, *const c_mb = cst + 7 * D, *const c_b1 = cst + 8 * D,
-             *const c_b2 = c_b1 + F, *const c_mix = c_b2 + kTrajHeadOut;
+    __shared__ __attribute__((aligned(16))) T cst[TrajConstants<T, D, F>::kElems], tok_s[D];  // and the position token of the coming step
+    const TrajConstants<T, D, F> C(cst);
 
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int tok = Ops::tok(lane), sub = Ops::sub(lane);  // output layout of the products
@@ -599,26 +685,9 @@ __global__ __launch_bounds__(kTrajWaves * 64) void trajectory_decode_kernel(Traj
     if (tid < kPieces) reinterpret_cast<u32x4 *>(pbuf[0])[tid] = vec_src[tid];
     for (int i = tid; i < 4 * P.n_layers; i += NT) kv_s[i] = P.kv[i];
     const T *const xm = static_cast<const T *>(P.x_mean);
-    for (int d = tid; d < D; d += NT) {
-        c_ng[d] = static_cast<const T *>(P.norm_g)[d];
-        c_nb[d] = static_cast<const T *>(P.norm_b)[d];
-        c_wx[d] = static_cast<const T *>(P.w_x)[d];
-        c_bx[d] = static_cast<const T *>(P.b_x)[d];
-        c_wy[d] = static_cast<const T *>(P.w_y)[d];
-        c_by[d] = static_cast<const T *>(P.b_y)[d];
-        c_mt[d] = static_cast<const T *>(P.markers)[d];
-        c_mb[d] = static_cast<const T *>(P.markers)[2 * D + d];
-    }
-    for (int d = tid; d < F; d += NT) c_b1[d] = static_cast<const T *>(P.b_h1)[d];
-    if (tid < kTrajHeadOut) c_b2[tid] = static_cast<const T *>(P.b_h2)[tid];
-    if (tid < 3 * P.K) c_mix[tid] = static_cast<const T *>(P.mix)[tid];
+    C.template load<NT>(P, tid);
     __syncthreads();
-    for (int i = tid; i < ROWS * D; i += NT) {
-        const int r = i / D, d = i % D, g = r >> 1;
-        float v = 0.f;
-        if ((r & 1) && g < valid) v = to_f32(xm[(b0 + g) * P.Nt]) * to_f32(c_wx[d]) + to_f32(c_bx[d]) + to_f32(c_mt[d]);
-        xs[r * LD + d] = from_f32<T>(v);
-    }
+    C.template first_rows<NT>(P, b0, valid, ROWS, xs, LD, tid);
     __syncthreads();
 
     using std::integral_constant;
@@ -680,19 +749,8 @@ __global__ __launch_bounds__(kTrajWaves * 64) void trajectory_decode_kernel(Traj
             }
             // the caches: row 2 g is committed at slot t - 1 of trajectory g (its first read is a step
             // away); behind the last one the target row, where the caller keeps it
-            {
-                constexpr int CPR = DH * sizeof(T) / 16, PER = H * CPR;  // 16-byte pieces of a head's row, of a row
-                auto commit = [&](int from, int slot) {
-                    for (int i = tid; i < valid * 2 * PER; i += NT) {
-                        const int c = i % PER, which = i / PER & 1, g = i / (2 * PER);
-                        const Global dst = (which ? kv[3] : kv[2]) + (((b0 + g) * H + c / CPR) * P.own_rows + slot) * static_cast<long>(DH * sizeof(T)) + 16 * (c % CPR);
-                        *(__attribute__((address_space(1))) u32x4 *)dst =
-                            *reinterpret_cast<const u32x4 *>((which ? vn : kn) + (2 * g + from) * LD + c * (16 / sizeof(T)));
-                    }
-                };
-                if (t > 0) commit(0, P.own_base + t - 1);
-                if (P.park_target && last_step) commit(1, P.own_base + t);
-            }
+            if (t > 0) traj_commit<T, D, NT>(kv[2], kv[3], kn, vn, LD, b0, valid, P.own_rows, 0, P.own_base + t - 1, tid);
+            if (P.park_target && last_step) traj_commit<T, D, NT>(kv[2], kv[3], kn, vn, LD, b0, valid, P.own_rows, 1, P.own_base + t, tid);
             attention(head0, t);
 #pragma unroll
             for (int hh = 1; hh < HPW; ++hh) {
@@ -754,16 +812,14 @@ __global__ __launch_bounds__(kTrajWaves * 64) void trajectory_decode_kernel(Traj
                 for (int e = 0; e < EPL; ++e) q += (x[e] - mean) * (x[e] - mean);
                 const float rstd = rsqrtf(wave_sum(q) / D + P.eps_out);
 #pragma unroll
-                for (int e = 0; e < EPL; ++e)
-                    ys[r * LD + lane * EPL + e] =
-                        from_f32<T>((x[e] - mean) * rstd * to_f32(c_ng[lane * EPL + e]) + to_f32(c_nb[lane * EPL + e]));
+                for (int e = 0; e < EPL; ++e) ys[r * LD + lane * EPL + e] = C.normed(x[e], mean, rstd, lane * EPL + e);
             }
             __syncthreads();
         }
         {
             f32x4 acc[S::NF];
             product(integral_constant<int, 0>{}, integral_constant<int, S::KD>{}, acc, ys, LD);
-            gelu_store(acc, c_b1);
+            gelu_store(acc, C.b1);
             __syncthreads();
         }
         {
@@ -771,7 +827,7 @@ __global__ __launch_bounds__(kTrajWaves * 64) void trajectory_decode_kernel(Traj
             product(integral_constant<int, S::kH1>{}, integral_constant<int, S::KF>{}, acc, hs, LF);
             if (16 * wave < kTrajHeadOut) {
                 float bias[4];
-                traj_load4<T>(c_b2 + 16 * wave + 4 * sub, bias);
+                traj_load4<T>(C.b2 + 16 * wave + 4 * sub, bias);
 #pragma unroll
                 for (int e = 0; e < 4; ++e) raw_s[tok][16 * wave + 4 * sub + e] = acc[0][e] + bias[e];
             }
@@ -788,7 +844,7 @@ __global__ __launch_bounds__(kTrajWaves * 64) void trajectory_decode_kernel(Traj
         }
         if (tid < valid) {
             const float *raw = raw_s[2 * tid + 1];
-            const T *const mix = c_mix;
+            const T *const mix = C.mix;
             float mx = -INFINITY;
             for (int k = 0; k < P.K; ++k) mx = fmaxf(mx, raw[3 * k + 2] + to_f32(mix[2 * P.K + k]));
             float z = 0.f;
@@ -803,39 +859,14 @@ __global__ __launch_bounds__(kTrajWaves * 64) void trajectory_decode_kernel(Traj
                     break;
                 }
             }
-            const float mean = raw[3 * comp] + to_f32(mix[comp]);
-            const float sraw = raw[3 * comp + 1] + to_f32(mix[P.K + comp]);
-            const float sp = sraw > 20.f ? sraw : log1pf(expf(sraw));
-            const T y = from_f32<T>(mean + (fminf(sp, P.std_max) + P.std_min) * my_n);
+            const T y = C.value(P, raw, comp, my_n);
             static_cast<T *>(P.preds)[(b0 + tid) * P.Nt + t] = y;
             y_s[tid] = to_f32(y);
         }
         __syncthreads();
         if (last_step) break;
-        {
-            for (int i = tid; i < 2 * valid * (D / 4); i += NT) {
-                const int d = 4 * (i % (D / 4)), r = i / (D / 4);
-                float wx[4], bx[4], m[4], o[4];
-                traj_load4<T>(c_wx + d, wx);
-                traj_load4<T>(c_bx + d, bx);
-                traj_load4<T>((r & 1 ? c_mt : c_mb) + d, m);
-                const float xv = x_s[r];
-                if (r & 1) {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) o[e] = xv * wx[e] + bx[e] + m[e];
-                } else {
-                    float wy[4], by[4], tk[4];
-                    traj_load4<T>(c_wy + d, wy);
-                    traj_load4<T>(c_by + d, by);
-                    traj_load4<T>(tok_s + d, tk);
-                    const float yv = y_s[r >> 1];
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) o[e] = xv * wx[e] + bx[e] + yv * wy[e] + by[e] + m[e] + tk[e];
-                }
-                traj_store4<T>(xs + r * LD + d, o);
-            }
-            __syncthreads();
-        }
+        C.template next_rows<NT>(x_s, y_s, tok_s, valid, xs, LD, tid);
+        __syncthreads();
     }
 }
 
