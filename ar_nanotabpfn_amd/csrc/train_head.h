@@ -17,7 +17,8 @@ namespace artab {
 constexpr int kHeadCols = 128;  // width of the raw outputs' gradient: a piece of the weight gradients
 
 struct TrainHead {
-    const float *z, *y;        // [M, D], [M]
+    const float *z, *y;        // [M, D], [M] (y: forward)
+    float *kept_y;             // [M]: written forward, read backward
     const float *w1, *b1, *w2, *b2;                    // [F, D], [F], [3 K, F], [3 K]
     const float *mean_bias, *std_bias, *weight_bias;   // [K]
     float std_min;
@@ -131,7 +132,8 @@ __global__ __launch_bounds__(kTrainWaves * 64, 3) void train_head_kernel(TrainHe
         {   // the mixture of a row: eight lanes, component k on lane k % 8
             const int tid = opaque(threadIdx.x), row = tid >> 3, j = tid & 7;
             const bool live = L.row0 + row < P.M;
-            const float y = P.y[min(L.row0 + row, P.M - 1)];
+            const float y = (BACKWARD ? P.kept_y : P.y)[min(L.row0 + row, P.M - 1)];
+            if (!BACKWARD && live && j == 0) P.kept_y[L.row0 + row] = y;
             float *const r = raw_s + row * LR;
             const auto add = [](float a, float b) { return a + b; };
             const auto larger = [](float a, float b) { return a > b || a != a ? a : b; };  // (a NaN stays)

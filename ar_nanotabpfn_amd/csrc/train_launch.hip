@@ -366,6 +366,7 @@ int head_groups(long M) {  // as many workgroups as are resident (three to a com
 int head_jobs(const artab_train_head_args &a) { return (a.F / 128) * (a.D / 128) + a.F / 128; }
 
 struct HeadSaved {
+    float *y;  // a copy: the caller's may change before the backward pass, as under modules
     bf16_t *packed;
     float *part_loss;
     size_t bytes;
@@ -373,6 +374,7 @@ struct HeadSaved {
 HeadSaved head_saved(const artab_train_head_args &a) {
     Arena s(a.saved);
     HeadSaved v;
+    v.y = s.take<float>(a.rows);
     v.packed = s.take<bf16_t>(2 * static_cast<size_t>(a.F) * (a.D + head_cols(a)));
     v.part_loss = s.take<float>(head_groups(a.rows));
     v.bytes = s.used;
@@ -400,17 +402,18 @@ HeadScratch head_scratch(const artab_train_head_args &a) {
 
 TrainHead head_params(const artab_train_head_args &a) {
     TrainHead P{};
-    P.z = a.z; P.y = a.y; P.w1 = a.w1; P.b1 = a.b1; P.w2 = a.w2; P.b2 = a.b2;
+    P.z = a.z; P.w1 = a.w1; P.b1 = a.b1; P.w2 = a.w2; P.b2 = a.b2;
     P.mean_bias = a.mean_bias; P.std_bias = a.std_bias; P.weight_bias = a.weight_bias; P.std_min = a.std_min; P.K = a.K; P.M = a.rows;
     const HeadSaved S = head_saved(a);
-    P.packed = S.packed; P.part_loss = S.part_loss;
+    P.packed = S.packed; P.part_loss = S.part_loss; P.kept_y = S.y;
     return P;
 }
 
 template <int D, int NP>
 int head_forward(const artab_train_head_args &a, hipStream_t st) {
     constexpr int F = 256;
-    const TrainHead P = head_params(a);
+    TrainHead P = head_params(a);
+    P.y = a.y;
     const int groups = head_groups(a.rows);
     hipLaunchKernelGGL((train_head_pack_kernel<D, F, NP>), dim3(static_cast<unsigned>((train_head_packed_elems<D, F, NP>() / 8 + 255) / 256)),
                        dim3(256), 0, st, P);
@@ -487,7 +490,7 @@ int artab_train_head_forward(const artab_train_head_args *a, void *stream) {
 }
 int artab_train_head_backward(const artab_train_head_args *a, void *stream) {
     if (!artab::head_supported(a)) return ARTAB_ERR_UNSUPPORTED;
-    if (!a->z || !a->y || !a->w1 || !a->b1 || !a->w2 || !a->b2 || !a->mean_bias || !a->std_bias || !a->weight_bias || !a->saved || !a->dloss ||
+    if (!a->z || !a->w1 || !a->b1 || !a->w2 || !a->b2 || !a->mean_bias || !a->std_bias || !a->weight_bias || !a->saved || !a->dloss ||
         !a->dz || !a->grads || !a->scratch)
         return ARTAB_ERR_NULL_POINTER;
     if (artab::off_16(a->z, a->w1, a->b1, a->w2, a->saved, a->dz, a->grads, a->scratch)) return ARTAB_ERR_BAD_STRIDE;

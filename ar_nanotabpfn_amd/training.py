@@ -221,16 +221,17 @@ class _HeadLoss(torch.autograd.Function):
         _head_pointers(a, z, y, params, saved)
         a.loss = loss.data_ptr()
         _lib.check(lib.artab_train_head_forward(ctypes.byref(a), _lib.current_stream(z.device)))
-        ctx.save_for_backward(z, y, saved, *params)
+        ctx.save_for_backward(z, saved, *params)
         return loss
 
     @staticmethod
     def backward(ctx, dloss):
         lib = _lib.load()
-        z, y, saved, *params = ctx.saved_tensors  # (raises if one of them was changed in place since)
+        z, saved, *params = ctx.saved_tensors  # (raises if one of them was changed in place since)
         create_graph = torch.is_grad_enabled()
         if create_graph or _transformed(dloss, z, *params):  # gradients that can be differentiated again, or many at once
             wanted = [t for t in (z, *params) if t.requires_grad]
+            y = saved[: 4 * ctx.args.rows].view(torch.float32).view(*z.shape[:2], 1)  # (the kernels' copy)
             with torch.enable_grad(), torch.autocast("cuda", torch.bfloat16):
                 loss = torch.func.functional_call(ctx.head, dict(zip(_HEAD_PARAMETERS, params)), (z, y))[0]
             grads = iter(torch.autograd.grad(loss, wanted, dloss, create_graph=create_graph))
@@ -238,11 +239,11 @@ class _HeadLoss(torch.autograd.Function):
             return (dz, None, None, *dparams)
         a = _lib.ArtabTrainHeadArgs.from_buffer_copy(ctx.args)
         D, F, K = a.D, a.F, a.K
-        if not (_f32(z.device, (z, y), (z.shape, y.shape)) and z.numel() == a.rows * D and y.numel() == a.rows
-                and saved.data_ptr() % 16 == 0 and _f32(z.device, params, _head_shapes(D, F, K))):
+        if not (_f32(z.device, (z,), (z.shape,)) and z.numel() == a.rows * D and saved.data_ptr() % 16 == 0
+                and _f32(z.device, params, _head_shapes(D, F, K))):
             raise RuntimeError("a parameter of the head has another size or type than in the forward pass")
         dloss = dloss.float().contiguous()
-        _head_pointers(a, z, y, params, saved)
+        _head_pointers(a, z, None, params, saved)
         scratch = torch.empty(lib.artab_train_head_scratch_bytes(ctypes.byref(a)), device=z.device, dtype=torch.uint8)
         dz = torch.empty_like(z)
         grads = torch.empty(F * D + 128 * F + F + 128, device=z.device, dtype=torch.float32)
@@ -267,9 +268,9 @@ def _head_shapes(D: int, F: int, K: int):
     return ((F, D), (F,), (3 * K, F), (3 * K,), (K,), (K,), (K,))
 
 
-def _head_pointers(a, z: Tensor, y: Tensor, params, saved: Tensor):
+def _head_pointers(a, z: Tensor, y, params, saved: Tensor):
     for name, t in zip(("z", "y", "w1", "b1", "w2", "b2", "mean_bias", "std_bias", "weight_bias", "saved"), (z, y, *params, saved)):
-        setattr(a, name, t.data_ptr())
+        setattr(a, name, None if t is None else t.data_ptr())
 
 
 def head_loss(head, z: Tensor, y: Tensor):

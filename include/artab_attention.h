@@ -563,7 +563,8 @@ int artab_train_embed_backward(const artab_train_embed_args *args, void *stream)
  * The mixture head behind that stack and its loss (model.py:150-246), for `rows` rows: gelu(z W_1^T + b_1) W_2^T + b_2
  * as K x (mean, deviation, weight); loss = the mean negative log-likelihood of y.  D in {128, 256}, F = 256,
  * 3 K <= 128; anything else: artab_train_head_saved_bytes returns 0.
- *   forward:  z [rows, D], y [rows] -> loss (one float); fills `saved`, kept by the caller for the backward call.
+ *   forward:  z [rows, D], y [rows] -> loss (one float); fills `saved`, kept by the caller for the backward call (it
+ *             begins with a copy of y: the backward call does not read `y`).
  *   backward: dloss (one float) -> dz [rows, D] and `grads` (float32): dW_1 [F, D], dW_2 [128, F] (zero past row 3 K),
  *             db_1 [F], db_2 [128] (entries 3 k + 0, 1, 2 are also those of the three biases of component k).
  */

@@ -46,6 +46,12 @@ def _kernels(head, z, y):
     return loss, _gradients(loss, z, head)
 
 
+def _loss_of(head_loss, head, z, y):
+    z = z.detach().requires_grad_()
+    with torch.autocast("cuda", torch.bfloat16):
+        return head_loss(head, z, y), z, head
+
+
 @pytest.mark.parametrize("D,K,B,T", [
     (128, 20, 3, 33),     # 60 raw outputs, a ragged last tile
     (128, 2, 1, 1), (256, 5, 2, 32),
@@ -167,3 +173,24 @@ def test_batched_gradients_of_head_parameters(device):
     for g, w in zip(got, want):  # (the modules' products here, the kernels' there, as above)
         assert g.shape == (3, *w.shape)
         assert float((g - scales.view(-1, *[1] * w.dim()) * w).norm()) <= 2 * 2 * 5 * 2.0 ** -9 * float((scales.norm() * w.norm()))
+
+
+def test_targets_that_lie_anywhere_and_move_on(device):
+    """The values are a table's last columns, at an odd address, and the program puts the next ones in their place before
+    the backward pass (the modules keep no reference to them)."""
+    from ar_nanotabpfn_amd.training import head_loss
+
+    head, z, y = _problem(device, 128, 5, 1, 33)
+    want = _gradients(*_loss_of(head_loss, head, z, y))
+    table = torch.cat([torch.zeros(1, 5, 1, device=device), y], dim=1)
+    mine = table[:, 5:]
+    assert mine.is_contiguous() and mine.data_ptr() % 16
+    args = _loss_of(head_loss, head, z, mine)
+    table.fill_(float("nan"))
+    for got, ref in zip(_gradients(*args), want):
+        assert torch.equal(got, ref)
+    mine.copy_(y)
+    loss, z, _ = _loss_of(head_loss, head, z, mine)
+    table.fill_(float("nan"))
+    (got,) = torch.autograd.grad(loss, z, create_graph=True)  # (the modules' route, with the kept values)
+    assert got.isfinite().all() and (got - want[0]).norm() <= 2 * 5 * 2.0 ** -9 * want[0].norm()
