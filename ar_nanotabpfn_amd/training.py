@@ -281,6 +281,7 @@ def head_loss(head, z: Tensor, y: Tensor):
     params = (one.weight, one.bias, two.weight, two.bias, head.mean_bias, head.std_bias, head.weight_bias)
     F, K = one.out_features, head.num_components
     if not (torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") == torch.bfloat16 and torch.is_grad_enabled()
+            and all(p is not None for p in params)  # (a Linear without a bias)
             and z.is_cuda and z.dtype == torch.float32 and z.dim() == 3 and tuple(y.shape) == (z.shape[0], z.shape[1], 1)
             and not y.requires_grad and head.dim_y == 1 and isinstance(K, int) and isinstance(head.std_min, float)
             and z.shape[2] in (128, 256) and F == 256 and 1 <= 3 * K <= 128 and 1 <= z.shape[0] * z.shape[1] < 2 ** 30

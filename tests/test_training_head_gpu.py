@@ -128,6 +128,8 @@ def test_what_the_kernels_are_not_for(device):
         assert head_loss(head, z, y.clone().requires_grad_()) is None
         assert head_loss(head, z[:, ::2], y[:, ::2]) is None
         assert head_loss(head, z, y.double()) is None
+        head.head[2] = torch.nn.Linear(256, 15, bias=False, device=device)
+        assert head_loss(head, z, y) is None and head(z, y)[0].isfinite()
         assert head_loss(head.half(), z, y) is None
 
 
