@@ -155,7 +155,7 @@ struct FlashPlan {
 // Over 2000 calls of 16 to 2048 keys, 16 to 2200 rows, 8 to 1024 pairs, the last fifth of them drawn when the rule stood, it is
 // above the best of the three by 0.6 % on average in bf16 (f16 1.0; head_dim 64 0.2 and 0.2), by at most 22 (a call of 8 us; 17; 11
 // and 11); by rows alone (256 while there are 512 workgroups) 6.5 % (4.9; 7.4 and 10.0), up to 58, better by 12 % at one call and by at most 7 elsewhere.
-// us: 64 x 4 pairs, 608 rows, 96 keys 22.4 -> 17.1; 616 rows, 316 keys 34 -> 25; 1544 rows, 1000 keys 108 (128 rows: 128); 64 x 8,
+// us: 64 x 4 pairs, 608 rows, 96 keys 22.4 -> 17.1; 616 rows, 316 keys 34 -> 25; 1544 rows, 1000 keys 96 (128 rows: 101); 64 x 8,
 // 516 rows, 116 keys of head_dim 64 72 -> 50; 32 x 8, 80 rows, 1040 keys 22 -> 17.
 static int unsliced_tile(long G, long pairs, int Nc, int Dh, bool bf16) {
     const auto padded = [&](int bm) { return static_cast<double>((G + bm - 1) / bm * bm); };
