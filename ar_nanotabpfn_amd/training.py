@@ -257,8 +257,10 @@ class _HeadLoss(torch.autograd.Function):
 def _transformed(*tensors) -> bool:
     """Whether a transform is at work (``vmap`` and its kin), or one of the tensors stands for many (batched gradients) or
     has a tangent."""
-    return torch._C._are_functorch_transforms_active() or any(
-        not torch._C._has_storage(t) or forward_ad.unpack_dual(t).tangent is not None for t in tensors)
+    if torch._C._are_functorch_transforms_active() or not all(map(torch._C._has_storage, tensors)):
+        return True
+    # (outside of every dual level there are no tangents)
+    return forward_ad._current_level >= 0 and any(forward_ad.unpack_dual(t).tangent is not None for t in tensors)
 
 
 _HEAD_PARAMETERS = ("head.0.weight", "head.0.bias", "head.2.weight", "head.2.bias", "mean_bias", "std_bias", "weight_bias")
