@@ -234,6 +234,9 @@ SIGNATURES = {
     "artab_trajectory_tape_bytes": (_sz, [_i, _i, _i, _i]),
     "artab_trajectory_pack": (_i, [_p, _p, _i, _i, _i, _i, _i, _i, _i, _p]),
     "artab_trajectory_decode": (_i, [ctypes.POINTER(ArtabTrajectoryArgs), _i, _p]),
+    "artab_trajectory_parts": (_i, [_i, _i, _i, _i, _i, _i, _i, _i, _i]),
+    "artab_trajectory_exchange_bytes": (_sz, [_i, _i, _i]),
+    "artab_trajectory_decode_parts": (_i, [ctypes.POINTER(ArtabTrajectoryArgs), _i, _p, _i, _p]),
     "artab_layer_post": (_i, [_p, _i64, _p, _i64, _p, _p, _p, _f, _p, _p, _p, _p, _p, _p, _f, _p, _i64, _i, _i, _i, _p]),
 }
 

@@ -43,7 +43,7 @@ static TuneSlot g_tune[kTuneCount] = {
     {"ARTAB_CTX_YIELD", false, 0},    {"ARTAB_ORDER_GATE_LAUNCH", false, 0},
     {"ARTAB_BN", false, 0},          {"ARTAB_LEAN", false, 0},         {"ARTAB_LEAN_OCC", false, 0},
     {"ARTAB_NW", false, 0},          {"ARTAB_TILE_ROWS", false, 0},    {"ARTAB_LAYER_FETCHERS", false, 0},
-    {"ARTAB_TRAJECTORY", false, 0},
+    {"ARTAB_TRAJECTORY", false, 0},  {"ARTAB_TRAJECTORY_PARTS", false, 0},
 };
 static const bool g_tune_loaded = [] {
     for (TuneSlot &t : g_tune) {
@@ -1968,6 +1968,60 @@ int artab_trajectory_group(int B, int Nc, int Nt, int H, int D, int F, int own_c
     return artab_trajectory_group_layers(B, Nc, Nt, H, D, F, 12, own_context, dtype);
 }
 
+// Several workgroups to a trajectory (trajectory_crews.h): where they fit the chip at one per compute unit.  Each has its share
+// of the heads, that is of the q/k/v weights and of all keys, and waits once per layer for the others, about 0.9 us.  us per
+// layer and step with 1 / 2 / 4 / 8 of them | step by step, 4 layers, the difference of runs of 32 and 8 steps, shared contexts:
+//   bf16, d_model 128, 64 trajectories: 300 rows 6.9 / 6.4 / 7.5 | 22.7; 4000 31.6 / 21.0 / 13.3 | 25.7; 16000 102.9 / 61.4 / 33.4 | 31.9
+//   d_model 256, 32: 300 rows 15.7 / 12.1 / 9.9 / 10.5 | 24.3; 4000 60.9 / 36.1 / 22.9 / 17.4 | 29.6; 16000 203.8 / 120.4 / 65.6 / 37.7 | 36.1
+//   d_model 512, 8: 300 rows 44.1 / 33.9 / 27.9 / 23.4 | 45.4; 4000 139.2 / 93.5 / 53.6 / 39.0 | 52.9; 16000 434.7 / 268.6 / 142.5 / 81.7 | 65.6
+//   float32, d_model 256, 32: 300 rows 40.6 / 30.5 / 26.8 / 26.9 | 136.8; 16000 589.8 / 304.7 / 160.7 / 90.0 | 155.7
+// and contexts of their own: bf16, d_model 256, 64 trajectories 600 rows 21.7 / 15.7 / 15.7, 2500 rows 72.6 / 42.6 / 35.9.  The
+// estimates below are lines through these, each at most a quarter off.  Behind half of the compute units they wait for
+// their weights together: a tenth with 4 or 8, less with 2.
+int artab_trajectory_parts(int B, int Nc, int Nt, int H, int D, int F, int n_layers, int own_context, int dtype) {
+    const TrajectoryTapeLayout layout = trajectory_layout(D, F, n_layers, dtype);
+    if (B < 1 || Nt < 1 || Nc < 1 || n_layers < 1 || H * 32 != D || layout.stride == 0) return 1;
+    const int force = tune(kTuneTrajectoryParts, 0);
+    if (force > 0) return traj_parts_built(D, force) ? force : 1;
+    if (tune(kTuneTrajectory, -1) >= 0) return 1;
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+        cus = 256;
+    // Workgroups that wait for others are on the chip together because an XCD starts them in order: at most one trajectory of a
+    // launch is there in part, seven workgroups for the 32 compute units of an XCD.  A partition with fewer XCDs could hold several
+    // in part.
+    if (cus < 256) return 1;
+    const bool f32 = dtype == ARTAB_F32;
+    static constexpr double kBase[2][3][4] = {{{5.2, 6.0, 6.8, 0.}, {13.0, 9.8, 8.8, 9.0}, {37.0, 31.0, 24.5, 22.5}},
+                                              {{12.0, 12.0, 11.5, 0.}, {30.0, 24.0, 23.0, 22.5}, {0., 0., 0., 0.}}};
+    static constexpr double kShare[4] = {1.0, 0.53, 0.28, 0.135};
+    const int width = D == 128 ? 0 : D == 256 ? 1 : 2;
+    const double rows = Nc + 0.5 * Nt, row = 2.0 * elem_size(dtype) * D, stream = row / (f32 ? 59e3 : 82.5e3);
+    const double memory = own_context ? B * row * rows / 11.2e6 : 0.;  // (half of it shows)
+    const auto run = [&](int i) {
+        const double crowd = 2L * B << i > cus ? (i == 0 ? 0. : i == 1 ? 0.03 : 0.1) : 0.;
+        return kBase[f32][width][i] * (1. + crowd) + stream * kShare[i] * rows + memory;
+    };
+    double best = run(0);
+    int parts = 1;
+    for (int i = 1; i < 4; ++i)
+        if (traj_parts_built(D, 1 << i) && static_cast<long>(B) << i <= cus && run(i) < best) best = run(i), parts = 1 << i;
+    double steps;  // the other route: as in artab_trajectory_group_layers() for own contexts, lines through the above for shared ones
+    if (own_context) {
+        const double wavefront = f32 || B == 1 ? 0.0 : row * rows / H / 6.5e3;
+        steps = std::max((f32 ? 240.0 : 100.0) + 480.0 / n_layers, 20.0 + std::max(wavefront, B * row * rows / 5e6));
+    } else if (f32) {
+        steps = (D == 128 ? 70.0 + 0.8 * B : 80.0 + 1.7 * B) + 1.5e-3 * rows;
+    } else {
+        steps = (D == 128 ? 24.0 + 0.45e-3 * rows : D == 256 ? 26.0 + 0.56e-3 * rows : 46.0 + 1.1e-3 * rows) + 8.0 * B * Nc * D / 1200e6;
+    }
+    return best < steps ? parts : 1;
+}
+
+size_t artab_trajectory_exchange_bytes(int B, int D, int dtype) {
+    return B < 1 || D < 1 ? 0 : 2 * static_cast<size_t>(B) * 8 * (dtype == ARTAB_F32 ? traj_exchange_words<float>(D) : traj_exchange_words<bf16_t>(D));
+}
+
 size_t artab_trajectory_tape_bytes(int D, int F, int n_layers, int dtype) {
     return n_layers < 1 ? 0 : static_cast<size_t>(kTrajWaves) * trajectory_layout(D, F, n_layers, dtype).stride;
 }
@@ -2009,6 +2063,10 @@ int artab_trajectory_pack(void *tape, const void *w, int which, int layer, int r
 }
 
 int artab_trajectory_decode(const artab_trajectory_args *a, int dtype, void *stream) {
+    return artab_trajectory_decode_parts(a, 1, nullptr, dtype, stream);
+}
+
+int artab_trajectory_decode_parts(const artab_trajectory_args *a, int parts, void *exchange, int dtype, void *stream) {
     if (!a) return fail(ARTAB_ERR_NULL_POINTER, "args is NULL");
     const TrajectoryTapeLayout t = trajectory_layout(a->D, a->F, a->n_layers, dtype);
     if (t.stride == 0 || a->n_layers < 1)
@@ -2028,6 +2086,15 @@ int artab_trajectory_decode(const artab_trajectory_args *a, int dtype, void *str
         return fail(ARTAB_ERR_NULL_POINTER, "trajectory_decode: no pointer may be NULL");
     if (misaligned16(a->tape) || misaligned16(a->vecs))
         return fail(ARTAB_ERR_BAD_STRIDE, "trajectory_decode: tape and vecs must be 16-byte aligned");
+    if (parts != 1) {
+        if (!traj_parts_built(a->D, parts) || a->group != 1)
+            return fail(ARTAB_ERR_UNSUPPORTED, "trajectory_decode: %d workgroups to %d trajectories at D=%d", parts, a->group, a->D);
+        // (exchanges are numbered in 32 bits)
+        if (static_cast<int64_t>(a->Nt) * a->n_layers >= (int64_t{1} << 31) || static_cast<int64_t>(a->B) * parts >= (1 << 28))
+            return fail(ARTAB_ERR_BAD_SHAPE, "trajectory_decode: bad sizes B=%d Nt=%d", a->B, a->Nt);
+        if (!exchange) return fail(ARTAB_ERR_NULL_POINTER, "trajectory_decode: exchange is NULL");
+        if (misaligned16(exchange)) return fail(ARTAB_ERR_BAD_STRIDE, "exchange must be 16-byte aligned");
+    }
     TrajectoryParams P{};
     P.tape = static_cast<const char *>(a->tape); P.tape_stride = t.stride; P.vecs = a->vecs;
     P.kv = reinterpret_cast<const unsigned long long *>(a->kv); P.n_layers = a->n_layers;
@@ -2039,10 +2106,11 @@ int artab_trajectory_decode(const artab_trajectory_args *a, int dtype, void *str
     P.rand_u = a->rand_u; P.rand_n = a->rand_n; P.rand_n_f32 = a->rand_n_f32 || dtype == ARTAB_F32; P.x_mean = a->x_mean;
     P.w_x = a->w_x; P.b_x = a->b_x; P.w_y = a->w_y; P.b_y = a->b_y; P.markers = a->markers; P.ar_tokens = a->ar_tokens; P.bs = a->bs;
     P.preds = a->preds; P.B = a->B; P.Nt = a->Nt; P.G = a->group;
+    P.exchange = static_cast<unsigned long long *>(exchange);
     hipStream_t st = static_cast<hipStream_t>(stream);
-    hipError_t e = dtype == ARTAB_BF16 ? launch_trajectory_decode_bf16(P, a->D, a->F, st)
-                   : dtype == ARTAB_F16 ? launch_trajectory_decode_f16(P, a->D, a->F, st)
-                                        : launch_trajectory_decode_f32(P, a->D, a->F, st);
+    hipError_t e = dtype == ARTAB_BF16 ? launch_trajectory_decode_bf16(P, a->D, a->F, parts, st)
+                   : dtype == ARTAB_F16 ? launch_trajectory_decode_f16(P, a->D, a->F, parts, st)
+                                        : launch_trajectory_decode_f32(P, a->D, a->F, parts, st);
     return launch_status(e, "trajectory_decode");
 }
 

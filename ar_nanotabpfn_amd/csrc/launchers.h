@@ -38,6 +38,7 @@ enum Tune : int {
     kTuneTileRows,        // ARTAB_TILE_ROWS: layer kernels with 16 or 32 token rows per workgroup; 33, 64: layer_wide.h's with 32, 64
     kTuneLayerFetchers,   // ARTAB_LAYER_FETCHERS: weight-fetching workgroups per XCD of a layer-boundary launch (0..32)
     kTuneTrajectory,      // ARTAB_TRAJECTORY: 0 keeps sampling runs off the whole-run kernel, 1..8 trajectories per workgroup
+    kTuneTrajectoryParts, // ARTAB_TRAJECTORY_PARTS: workgroups per trajectory (1, 2, 4, 8; no more than there are heads)
     kTuneCount
 };
 // The override of `key` if one is set, else `fallback` (artab_api.hip).
@@ -134,7 +135,7 @@ struct TrajectoryTapeLayout {
     hipError_t launch_trajectory_tape_##suffix(const void *w, char *tape, long stride, int N, int K,     \
                                                const TrajectoryTapeLayout::Matrix &m, int section,       \
                                                hipStream_t st);                                          \
-    hipError_t launch_trajectory_decode_##suffix(const TrajectoryParams &P, int D, int F, hipStream_t st);
+    hipError_t launch_trajectory_decode_##suffix(const TrajectoryParams &P, int D, int F, int parts, hipStream_t st);
 ARTAB_TRAJ_DECLARE(bf16)
 ARTAB_TRAJ_DECLARE(f16)
 ARTAB_TRAJ_DECLARE(f32)

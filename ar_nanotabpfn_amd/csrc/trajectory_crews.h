@@ -1,5 +1,5 @@
 // The whole-run decode of one trajectory per workgroup (trajectory_decode.h has the scheme, the weights' tapes and the
-// rounding model) with two crews of eight wavefronts.  d_model 128 or 256.
+// rounding model) with two crews of eight wavefronts.  d_model 128 or 256; with several workgroups to a trajectory 512 too.
 //
 // What bounds a run is one compute unit: its address unit, which a wavefront's 1 KiB request occupies for 16 clocks,
 // and the chain of a layer's products, norms and barriers.  A wavefront waits until its request is accepted, so whoever
@@ -23,6 +23,13 @@
 // Not kept: crew 0 taking a share of a long context's keys (its registers do not hold them beside the weights: 9.2
 // instead of 7.0 ms for 64 x 512 own rows); workgroups half a layer apart (no difference: it is not the memory they
 // wait for together, a compute unit gets 55-85 GB/s of keys whatever the others do).
+//
+// Several workgroups to a trajectory (PARTS): each has its share of the heads, which is its share of the q/k/v weights and
+// of the keys, what one compute unit needs longest for; everything behind the attention all of them compute, the same to the
+// bit.  Per layer they give each other their heads' output, 1 KiB in 16 bits at d_model 256: dealing out the other products as well
+// would take two more exchanges of about 0.9 us each and save 1.4.  64 trajectories of d_model 256 with 600 own rows, bf16, us per
+// layer and step: 21.7 with one workgroup, 15.7 with two; 32 on a shared context of 4000 rows 60.9 / 36.1 / 22.9 / 17.4 with 1 / 2 /
+// 4 / 8.  artab_trajectory_parts() says how many.
 #pragma once
 
 #include "trajectory_decode.h"
@@ -58,7 +65,7 @@ __device__ __forceinline__ float lanes16_max(float x) {
     return fmaxf(x, row_rotate<1>(x));
 }
 
-template <typename T, int D, int F>
+template <typename T, int D, int F, int PARTS>
 __global__ __launch_bounds__(2 * kTrajWaves * 64) void trajectory_crews_kernel(TrajectoryParams P) {
     typedef TrajOps<T> Ops;
     typedef TrajShape<T, D, F> S;
@@ -69,13 +76,17 @@ __global__ __launch_bounds__(2 * kTrajWaves * 64) void trajectory_crews_kernel(T
     constexpr int VW = D > F ? D : F;
     // Keys per block: one step of the second product's contraction.
     constexpr int BK = k16 ? 32 : 16;
-    static_assert(H <= NW, "a wavefront per head, or several");
-    constexpr int NP = NW / H;                      // wavefronts per head
+    constexpr int HL = H / PARTS;                   // heads of this workgroup
+    static_assert(HL <= NW && HL * PARTS == H, "a wavefront per head, or several");
+    constexpr int NP = NW / HL;                     // wavefronts per head
     constexpr int VPAD = DH + 16;
     constexpr int GB = 4;  // blocks on their way per wavefront (and, in 16 bits, of one group of score products)
     // fragments of a product that are requested ahead: as many as the registers allow
     constexpr int kMost = 16;
-    constexpr int wFo = S::kFo < kMost ? S::kFo : kMost, wQkv = S::kQkv < kMost ? S::kQkv : kMost, wO = S::kO < kMost ? S::kO : kMost,
+    // q/k/v: 16-feature blocks of this workgroup's heads in one of the three, blocks per wavefront
+    constexpr int BL = D / PARTS / 16, NQ = (3 * BL + NW - 1) / NW, kQkv = NQ * S::KD;
+    static_assert(PARTS > 1 || NQ == 3 * S::ND, "all heads: the tape's own order");
+    constexpr int wFo = S::kFo < kMost ? S::kFo : kMost, wQkv = kQkv < kMost ? kQkv : kMost, wO = S::kO < kMost ? S::kO : kMost,
                   w1 = S::k1 < kMost ? S::k1 : kMost, w2 = S::k2 < kMost ? S::k2 : kMost, wH2 = S::kH2 < w2 ? S::kH2 : w2;
     // where there is room beside others: W_2's together with W_o's, the first of q/k/v's together with W_2's, the keys
     // together with W_fo's
@@ -114,7 +125,12 @@ __global__ __launch_bounds__(2 * kTrajWaves * 64) void trajectory_crews_kernel(T
         __device__ __forceinline__ int quad() const { return lane >> 4; }
     };
     auto here = [&]() { return Lane{opaque(tid & 63)}; };
-    const long b = blockIdx.x;  // the trajectory
+    // The trajectory, and which of its workgroups this is.  Workgroups are started in order and dealt round-robin over
+    // the eight XCDs: those of one trajectory come one after the other on one XCD.
+    const int member = PARTS > 1 ? static_cast<int>(blockIdx.x >> 3) % PARTS : 0;
+    const long b = PARTS > 1 ? static_cast<long>(blockIdx.x >> 3) / PARTS * 8 + (blockIdx.x & 7) : blockIdx.x;
+    if (PARTS > 1 && b >= P.B) return;
+    __shared__ int gone_s;  // another workgroup of the trajectory was waited for in vain
 
     // Global memory by its address space: made from integers, plain pointers would be generic ones, whose loads count
     // as LDS accesses too, and every wait for LDS would wait for them.
@@ -128,13 +144,35 @@ __global__ __launch_bounds__(2 * kTrajWaves * 64) void trajectory_crews_kernel(T
         const unsigned lo = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(p)), hi = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(p >> 32));
         return *(Global16)((Global)(static_cast<unsigned long long>(hi) << 32 | lo) + lane_byte);
     };
-    // Fragments FROM .. TO - 1 of the product whose first one is at `at`.
-    auto ask = [&](auto &buf, int at, auto from_, auto to_) {
+    // Where a product's fragments are, by number: one after the other on this wavefront's tape; of q/k/v, where several
+    // workgroups share a trajectory, those of its own heads' blocks, on whichever tapes they are.
+    auto run_at = [&](int at) { return [=](int n, unsigned lane_byte) { return fragment(at + n, lane_byte); }; };
+    auto qkv_block = [&](int i) { return min(wave + NW * i, 3 * BL - 1); };  // (q's blocks, k's, v's; past the end the last one again)
+    unsigned long long qkv_tape[NQ];
+#pragma unroll
+    for (int i = 0; i < NQ; ++i) {
+        const int m = qkv_block(i), c = member * BL + m % BL;  // the block's place among all of its matrix
+        qkv_tape[i] = reinterpret_cast<unsigned long long>(P.tape) + (c % NW) * static_cast<unsigned long long>(P.tape_stride) +
+                      static_cast<unsigned long long>(S::pQkv + m / BL * S::ND + c / NW) * 1024;
+    }
+    auto qkv_at = [&](int layer_at) {
+        if constexpr (PARTS == 1) {
+            return run_at(layer_at + S::pQkv);
+        } else {
+            return [=, &qkv_tape](int n, unsigned lane_byte) {
+                const unsigned long long p = qkv_tape[n % NQ] + static_cast<long>(layer_at + n / NQ * 3 * S::ND) * 1024;
+                const unsigned lo = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(p)), hi = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(p >> 32));
+                return *(Global16)((Global)(static_cast<unsigned long long>(hi) << 32 | lo) + lane_byte);
+            };
+        }
+    };
+    // Fragments FROM .. TO - 1 of a product.
+    auto ask = [&](auto &buf, auto frag, auto from_, auto to_) {
         constexpr int FROM = decltype(from_)::value, TO = decltype(to_)::value;
         __builtin_amdgcn_sched_barrier(0);
         const unsigned lane_byte = 16 * here().lane;
 #pragma unroll
-        for (int i = FROM; i < TO; ++i) buf[i] = fragment(at + i, lane_byte);
+        for (int i = FROM; i < TO; ++i) buf[i] = frag(i, lane_byte);
         __builtin_amdgcn_sched_barrier(0);
     };
     // Values that nobody needs any more, where only one of two paths overwrites them: on the other one their registers
@@ -148,7 +186,7 @@ __global__ __launch_bounds__(2 * kTrajWaves * 64) void trajectory_crews_kernel(T
     };
     // acc[i] = W_i A^T over KS steps of NB blocks.  The buffer holds the first fragments; the others follow where there
     // is one free.
-    auto product = [&](auto &acc, auto &buf, int at, auto ks_, const T *act, int ld) {
+    auto product = [&](auto &acc, auto &buf, auto frag, auto ks_, const T *act, int ld) {
         constexpr int KS = decltype(ks_)::value, NB = sizeof(acc) / sizeof(acc[0]), W = sizeof(buf) / sizeof(buf[0]), N = KS * NB;
         constexpr int KC = KS < 4 ? KS : 4;  // activation operands are read KC steps at a time
         const Lane ln = here();
@@ -168,7 +206,7 @@ __global__ __launch_bounds__(2 * kTrajWaves * 64) void trajectory_crews_kernel(T
                     const int n = (k0 + k) * NB + i;
                     if (NB == 1 && (k & 1)) odd[i] = Ops::mma(buf[n % W], bf[k], odd[i]);
                     else acc[i] = Ops::mma(buf[n % W], bf[k], acc[i]);
-                    if (n + W < N) buf[n % W] = fragment(at + n + W, 16 * ln.lane);
+                    if (n + W < N) buf[n % W] = frag(n + W, 16 * ln.lane);
                 }
             if (N > W) __builtin_amdgcn_sched_barrier(0);
         }
@@ -244,8 +282,8 @@ __global__ __launch_bounds__(2 * kTrajWaves * 64) void trajectory_crews_kernel(T
     };
 
     // ---- attention (crew 1): committed rows, then the rows of this step
-    const int part = wave / H;
-    const int head0 = wave % H;
+    const int part = wave / HL;
+    const int head0 = member * HL + wave % HL;
     const int first_block = part;  // the wavefront's blocks: this one and every NP-th
     T *const vt = v_lds + (k16 ? wave * GB * BK * VPAD : 0);
     constexpr unsigned RB = DH * sizeof(T);  // bytes of a row
@@ -348,14 +386,49 @@ __global__ __launch_bounds__(2 * kTrajWaves * 64) void trajectory_crews_kernel(T
             for (int db = 0; db < 2; ++db) *reinterpret_cast<f32x4 *>(part_o + (wave * NR + tok) * DH + 16 * db + 4 * sub) = a_o[db];
         }
     };
-    auto attention_take = [&](int h) {
+    // ---- what the workgroups of a trajectory give each other: their heads' attention output, as 8-byte words of values and
+    // the number of the exchange, stored and read with relaxed device-wide atomics.  A word is its own signal: no fence, no
+    // counter, one trip through the memory side.  Two sets of words, in turn: who sends exchange n + 2 has every word of
+    // n + 1, and whoever sent those had all words of n.
+    constexpr int VPW = k16 ? 2 : 1, WORDS = NR * D / VPW;  // values per word, words per exchange
+    static_assert(WORDS <= NTC, "one word per thread of a crew");
+    auto words = [&](unsigned tag) { return P.exchange + (2 * b + (tag & 1)) * WORDS; };
+    auto send = [&](int row, int col, const float (&o)[4], unsigned tag) {
+        if (gone_s) return;  // (what it would send is not the trajectory's: the others are to give up too)
+        unsigned long long *const at = words(tag) + (row * D + col) / VPW;
+#pragma unroll
+        for (int i = 0; i < 4 / VPW; ++i) {
+            unsigned value;
+            if constexpr (k16) value = pack2<T>(o[2 * i], o[2 * i + 1]);
+            else value = __builtin_bit_cast(unsigned, o[i]);
+            __hip_atomic_store(at + i, static_cast<unsigned long long>(tag) << 32 | value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    };
+    auto receive = [&](unsigned tag) {
+        const int i = ctid, row = i / (WORDS / NR), col = i % (WORDS / NR) * VPW;
+        if (i >= WORDS || col / (D / PARTS) == member) return;
+        const unsigned long long *const at = words(tag) + i;
+        unsigned long long v = __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        // (every wait ends: a workgroup that is not there after some seconds is given up, and the draws become NaN)
+        for (int polls = gone_s ? kTrajMostPolls : 0; static_cast<unsigned>(v >> 32) != tag; ++polls) {
+            if (polls >= kTrajMostPolls) {
+                gone_s = 1;
+                break;
+            }
+            __builtin_amdgcn_s_sleep(1);
+            v = __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        const unsigned value = static_cast<unsigned>(v);
+        *reinterpret_cast<unsigned *>(xs + row * LD + col) = value;
+    };
+    auto attention_take = [&](int h, unsigned tag) {
         const Lane ln = here();
         const int tok = ln.tok(), sub = ln.sub();
         if ((NP == 1 || part == 0) && ln.writes()) {
             if constexpr (NP > 1) {  // the other wavefronts' keys of this head
 #pragma unroll
                 for (int p = 1; p < NP; ++p) {
-                    const int w = wave + p * H;
+                    const int w = wave + p * HL;
                     const float m2 = part_m[w * NR + tok], l2 = part_l[w * NR + tok];
                     const float m_new = fmaxf(a_m, m2);
                     const float a1 = fast_exp2(a_m - m_new), a2 = fast_exp2(m2 - m_new);
@@ -374,6 +447,7 @@ __global__ __launch_bounds__(2 * kTrajWaves * 64) void trajectory_crews_kernel(T
             for (int db = 0; db < 2; ++db) {
                 const float o[4] = {a_o[db][0] * inv, a_o[db][1] * inv, a_o[db][2] * inv, a_o[db][3] * inv};
                 traj_store4<T>(xs + tok * LD + DH * h + 16 * db + 4 * sub, o);
+                if constexpr (PARTS > 1) send(tok, DH * h + 16 * db + 4 * sub, o, tag);
             }
         }
     };
@@ -608,6 +682,7 @@ __global__ __launch_bounds__(2 * kTrajWaves * 64) void trajectory_crews_kernel(T
         eps_s[0] = P.eps1;
         eps_s[1] = P.eps2;
         eps_s[2] = P.eps3;
+        if constexpr (PARTS > 1) gone_s = 0;
     }
     __syncthreads();
     C.template first_rows<NT>(P, b, 1, NR, xs, LD, tid);
@@ -625,9 +700,9 @@ __global__ __launch_bounds__(2 * kTrajWaves * 64) void trajectory_crews_kernel(T
         constexpr integral_constant<int, 0> from0{};
         constexpr integral_constant<int, GB> all_blocks{};
         const int head_at = P.n_layers * S::kLayer;
-        if constexpr (kA) ask(f_qkv, S::pQkv, from0, integral_constant<int, kQkvEarly>{});
+        if constexpr (kA) ask(f_qkv, qkv_at(0), from0, integral_constant<int, kQkvEarly>{});
         if constexpr (kB) {
-            ask(f_b, S::pFo, from0, integral_constant<int, wFo>{});
+            ask(f_b, run_at(S::pFo), from0, integral_constant<int, wFo>{});
             prepare(head0, 0, 0);
             if constexpr (kKeysEarly) {
                 ask_keys(keys, from0, all_blocks);
@@ -670,33 +745,33 @@ __global__ __launch_bounds__(2 * kTrajWaves * 64) void trajectory_crews_kernel(T
                 if constexpr (kB) {
                     f32x4 acc[S::ND];
                     residual(xs);
-                    product(acc, first<wFo>(f_b), at + S::pFo, integral_constant<int, S::KD>{}, xs, LD);
+                    product(acc, first<wFo>(f_b), run_at(at + S::pFo), integral_constant<int, S::KD>{}, xs, LD);
                     add(acc);
                     norm_sums(v);
                 } else {
-                    ask(f_qkv, at + S::pQkv, integral_constant<int, kQkvEarly>{}, integral_constant<int, kQkvMid>{});
+                    ask(f_qkv, qkv_at(at), integral_constant<int, kQkvEarly>{}, integral_constant<int, kQkvMid>{});
                 }
                 __syncthreads();
                 if constexpr (kB) norm_store(v, vec, vec + VW, eps_s, ys);
-                else ask(f_qkv, at + S::pQkv, integral_constant<int, kQkvMid>{}, integral_constant<int, wQkv>{});
+                else ask(f_qkv, qkv_at(at), integral_constant<int, kQkvMid>{}, integral_constant<int, wQkv>{});
                 __syncthreads();
                 // q, k, v
                 if constexpr (kA) {
-                    f32x4 acc[3 * S::ND];
-                    product(acc, f_qkv, at + S::pQkv, integral_constant<int, S::KD>{}, ys, LD);
+                    f32x4 acc[NQ];
+                    product(acc, f_qkv, qkv_at(at), integral_constant<int, S::KD>{}, ys, LD);
                     const Lane ln = here();
 #pragma unroll
-                    for (int p = 0; p < 3; ++p)
+                    for (int i = 0; i < NQ; ++i) {
+                        // part of q/k/v and 16-feature block in it
+                        const int m = qkv_block(i), p = PARTS == 1 ? i / S::ND : m / BL, c = PARTS == 1 ? wave + NW * (i % S::ND) : member * BL + m % BL;
+                        float o[4];
 #pragma unroll
-                        for (int i = 0; i < S::ND; ++i) {
-                            float o[4];
-#pragma unroll
-                            for (int e = 0; e < 4; ++e) {
-                                o[e] = acc[p * S::ND + i][e];
-                                if (p == 0) o[e] = to_f32(from_f32<T>(o[e])) * P.qscale;
-                            }
-                            if (ln.writes()) traj_store4<T>(qkv + p * NR * LD + ln.row() * LD + 16 * (wave + NW * i) + 4 * ln.sub(), o);
+                        for (int e = 0; e < 4; ++e) {
+                            o[e] = acc[i][e];
+                            if (p == 0) o[e] = to_f32(from_f32<T>(o[e])) * P.qscale;
                         }
+                        if (ln.writes()) traj_store4<T>(qkv + p * NR * LD + ln.row() * LD + 16 * c + 4 * ln.sub(), o);
+                    }
                 } else {
                     if constexpr (!kKeysEarly) ask_keys(keys, from0, all_blocks);
                     ask_values(keys, integral_constant<int, kSpread ? GB / 2 : 0>{}, all_blocks);
@@ -704,52 +779,51 @@ __global__ __launch_bounds__(2 * kTrajWaves * 64) void trajectory_crews_kernel(T
                 __syncthreads();
                 u32x4 next_vec = {0u, 0u, 0u, 0u};
                 if constexpr (kA) {
-                    ask(f_o, at + S::pO, from0, integral_constant<int, wO>{});
+                    ask(f_o, run_at(at + S::pO), from0, integral_constant<int, wO>{});
                     if (ctid < kPieces) next_vec = vec_src[(last_layer ? 0 : l + 1) * kPieces + ctid];
-                    if constexpr (kW2Early) ask(f_2, at + S::p2, from0, integral_constant<int, w2>{});
+                    if constexpr (kW2Early) ask(f_2, run_at(at + S::p2), from0, integral_constant<int, w2>{});
                     // the caches: row 0 is committed at slot t - 1 (its first read is a step away); behind the last one
                     // the target row, where the caller keeps it
                     auto commit = [&](int from, int slot) {
-                        traj_commit<T, D, NTC>(layer_kv(l, 2), layer_kv(l, 3), kn, vn, LD, b, 1, P.own_rows, from, slot, ctid);
+                        traj_commit<T, D, NTC, HL>(layer_kv(l, 2), layer_kv(l, 3), kn, vn, LD, b, 1, P.own_rows, from, slot, ctid, member * HL);
                     };
                     if (t > 0) commit(0, P.own_base + t - 1);
                     if (P.park_target && last_step) commit(1, P.own_base + t);
                 } else {
                     attention(head0, t, keys);
                     if constexpr (NP > 1) attention_put();
-                    else attention_take(head0);
                 }
-                if constexpr (NP > 1) {
-                    __syncthreads();
-                    if constexpr (kB) attention_take(head0);
-                }
+                if constexpr (NP > 1) __syncthreads();
+                const unsigned tag = static_cast<unsigned>(t * P.n_layers + l) + 1u;  // of this exchange
+                if constexpr (kB) attention_take(head0, tag);
+                else if constexpr (PARTS > 1) receive(tag);
                 __syncthreads();
                 // x1 = LN2(y + attn W_o^T)
                 if constexpr (kA) {
                     f32x4 acc[S::ND];
                     residual(ys);
-                    product(acc, f_o, at + S::pO, integral_constant<int, S::KD>{}, xs, LD);
+                    product(acc, f_o, run_at(at + S::pO), integral_constant<int, S::KD>{}, xs, LD);
                     add(acc);
                     norm_sums(v);
                 } else {
                     prepare(head0, last_layer ? 0 : l + 1, last_layer ? t + 1 : t);
-                    ask(f_b, at + S::p1, from0, integral_constant<int, w1 / 2>{});
+                    ask(f_b, run_at(at + S::p1), from0, integral_constant<int, w1 / 2>{});
                 }
                 __syncthreads();
                 if constexpr (kA) norm_store(v, vec + 2 * VW, vec + 3 * VW, eps_s + 1, ys);
-                else ask(f_b, at + S::p1, integral_constant<int, w1 / 2>{}, integral_constant<int, w1>{});
+                else ask(f_b, run_at(at + S::p1), integral_constant<int, w1 / 2>{}, integral_constant<int, w1>{});
                 if constexpr (kB && kSpread) ask_keys(keys, from0, integral_constant<int, GB / 2>{});
                 __syncthreads();
                 // h = gelu(x1 W_1^T + b_1)
                 if constexpr (kB) {
                     f32x4 acc[S::NF];
-                    product(acc, first<w1>(f_b), at + S::p1, integral_constant<int, S::KD>{}, ys, LD);
+                    product(acc, first<w1>(f_b), run_at(at + S::p1), integral_constant<int, S::KD>{}, ys, LD);
                     gelu_store(acc, vec + 4 * VW);
                 } else {
                     if (ctid < kPieces) reinterpret_cast<u32x4 *>(pbuf[pp ^ 1])[ctid] = next_vec;
-                    if constexpr (!kW2Early) ask(f_2, at + S::p2, from0, integral_constant<int, w2>{});
+                    if constexpr (!kW2Early) ask(f_2, run_at(at + S::p2), from0, integral_constant<int, w2>{});
                     forget(f_qkv);
-                    if (kQkvEarly > 0 && !last_layer) ask(f_qkv, at + S::kLayer + S::pQkv, from0, integral_constant<int, kQkvEarly>{});
+                    if (kQkvEarly > 0 && !last_layer) ask(f_qkv, qkv_at(at + S::kLayer), from0, integral_constant<int, kQkvEarly>{});
                 }
                 __syncthreads();
                 // x = LN3(x1 + h W_2^T + b_2)
@@ -760,7 +834,7 @@ __global__ __launch_bounds__(2 * kTrajWaves * 64) void trajectory_crews_kernel(T
                     const Lane ln = here();
 #pragma unroll
                     for (int b = 0; b < S::ND; ++b) traj_load4<T>(vec + 7 * VW + 16 * (wave + NW * b) + 4 * ln.sub(), bias[b]);
-                    product(acc, f_2, at + S::p2, integral_constant<int, S::KF>{}, hs, LF);
+                    product(acc, f_2, run_at(at + S::p2), integral_constant<int, S::KF>{}, hs, LF);
                     add(acc);
 #pragma unroll
                     for (int b = 0; b < S::ND; ++b)
@@ -769,8 +843,8 @@ __global__ __launch_bounds__(2 * kTrajWaves * 64) void trajectory_crews_kernel(T
                     norm_sums(v);
                 } else {
                     forget(f_b);
-                    if (last_layer) ask(f_b, head_at, from0, integral_constant<int, w1>{});
-                    else ask(f_b, at + S::kLayer + S::pFo, from0, integral_constant<int, wFo>{});
+                    if (last_layer) ask(f_b, run_at(head_at), from0, integral_constant<int, w1>{});
+                    else ask(f_b, run_at(at + S::kLayer + S::pFo), from0, integral_constant<int, wFo>{});
                     if constexpr (kSpread) ask_keys(keys, integral_constant<int, GB / 2>{}, all_blocks);
                 }
                 __syncthreads();
@@ -785,7 +859,7 @@ __global__ __launch_bounds__(2 * kTrajWaves * 64) void trajectory_crews_kernel(T
             }
 
             // ---- the head on the target rows, one draw per trajectory, the rows of the next step
-            if constexpr (kA) ask(f_2, head_at + S::kH1, from0, integral_constant<int, wH2>{});
+            if constexpr (kA) ask(f_2, run_at(head_at + S::kH1), from0, integral_constant<int, wH2>{});
             {
                 constexpr int EPL = D / 64;
                 if (const int r = warp; r < NR) {
@@ -808,13 +882,13 @@ __global__ __launch_bounds__(2 * kTrajWaves * 64) void trajectory_crews_kernel(T
             __syncthreads();
             if constexpr (kB) {
                 f32x4 acc[S::NF];
-                product(acc, first<w1>(f_b), head_at, integral_constant<int, S::KD>{}, ys, LD);
+                product(acc, first<w1>(f_b), run_at(head_at), integral_constant<int, S::KD>{}, ys, LD);
                 gelu_store(acc, C.b1);
             }
             __syncthreads();
             if constexpr (kA) {
                 f32x4 acc[1];
-                product(acc, first<wH2>(f_2), head_at + S::kH1, integral_constant<int, S::KF>{}, hs, LF);
+                product(acc, first<wH2>(f_2), run_at(head_at + S::kH1), integral_constant<int, S::KF>{}, hs, LF);
                 const Lane ln = here();
                 if (16 * wave < kTrajHeadOut && ln.writes()) {
                     float bias[4];
@@ -825,11 +899,11 @@ __global__ __launch_bounds__(2 * kTrajWaves * 64) void trajectory_crews_kernel(T
                 if (ctid < 2) x_s[ctid] = to_f32(my_x);
                 if (ctid < D) tok_s[ctid] = my_tok;
             } else {
-                ask(f_b, S::pFo, from0, integral_constant<int, wFo>{});
+                ask(f_b, run_at(S::pFo), from0, integral_constant<int, wFo>{});
             }
             __syncthreads();
             if constexpr (kA) {
-                ask(f_qkv, S::pQkv, from0, integral_constant<int, kQkvEarly>{});
+                ask(f_qkv, qkv_at(0), from0, integral_constant<int, kQkvEarly>{});
                 if (wave == 0) {  // a lane per component
                     const float *raw = raw_s[1];
                     const T *const mix = C.mix;
@@ -845,9 +919,10 @@ __global__ __launch_bounds__(2 * kTrajWaves * 64) void trajectory_crews_kernel(T
                     }
                     const unsigned long long past = __ballot(lane < P.K && upto > my_u * cum);
                     const int comp = past ? __builtin_ctzll(past) : P.K - 1;
-                    const T y = C.value(P, raw, comp, my_n);
+                    T y = C.value(P, raw, comp, my_n);
+                    if (PARTS > 1 && gone_s) y = from_f32<T>(NAN);
                     if (lane == 0) {
-                        static_cast<T *>(P.preds)[b * P.Nt + t] = y;
+                        if (member == 0) static_cast<T *>(P.preds)[b * P.Nt + t] = y;  // (all of them have drawn it)
                         y_s = to_f32(y);
                     }
                 }

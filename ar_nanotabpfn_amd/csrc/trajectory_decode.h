@@ -76,7 +76,23 @@ struct TrajectoryParams {
     const void *ar_tokens; int bs;      // [bs, D]
     void *preds;             // [B, Nt]
     int B, Nt, G;
+    // several workgroups to a trajectory (trajectory_crews.h): what they give each other, zero in front of the launch
+    unsigned long long *exchange;
 };
+// A wait for another workgroup's word: about a microsecond each, some ten seconds in all.
+constexpr int kTrajMostPolls = 1 << 24;
+// Whether the two-crew kernel is built for `parts` workgroups to a trajectory: each has one head or more, a wavefront of one
+// crew or more for each of them.
+constexpr bool traj_parts_built(int D, int parts) {
+    return (parts == 2 || parts == 4 || parts == 8) && D / 32 >= parts && D / 32 / parts <= kTrajWaves;
+}
+// Words of 8 bytes in one exchange between a trajectory's workgroups: two rows of D values, four bytes of them per word.
+template <typename T>
+constexpr int traj_exchange_words(int D) { return 2 * D * static_cast<int>(sizeof(T)) / 4; }
+static __global__ __launch_bounds__(256) void trajectory_exchange_kernel(unsigned long long *words, long n) {
+    const long i = static_cast<long>(blockIdx.x) * 256 + threadIdx.x;
+    if (i < n) words[i] = 0;  // (the number of no exchange)
+}
 
 // One 1 KiB fragment per operand and product.  Both types read the A operand as row lane % 16 of a
 // 16-row block, kPer consecutive contraction elements at kPer (lane / 16).
@@ -267,13 +283,14 @@ struct TrajConstants {
     }
 };
 
-// Keys and values of token row 2 g + `from` to row `slot` of the cache of trajectory b0 + g.
-template <typename T, int D, int NT>
+// Keys and values of token row 2 g + `from`, HL heads of them from `head` on, to row `slot` of the cache of trajectory b0 + g.
+template <typename T, int D, int NT, int HL = D / 32>
 __device__ __forceinline__ void traj_commit(__attribute__((address_space(1))) char *ck, __attribute__((address_space(1))) char *cv,
-                                            const T *kn, const T *vn, int ld, long b0, int valid, int own_rows, int from, int slot, int tid) {
-    constexpr int DH = 32, H = D / DH, CPR = DH * sizeof(T) / 16, PER = H * CPR;  // 16-byte pieces of a head's row, of a row
+                                            const T *kn, const T *vn, int ld, long b0, int valid, int own_rows, int from, int slot, int tid,
+                                            int head = 0) {
+    constexpr int DH = 32, H = D / DH, CPR = DH * sizeof(T) / 16, PER = HL * CPR;  // 16-byte pieces of a head's row, of HL of them
     for (int i = tid; i < valid * 2 * PER; i += NT) {
-        const int c = i % PER, which = i / PER & 1, g = i / (2 * PER);
+        const int c = head * CPR + i % PER, which = i / PER & 1, g = i / (2 * PER);
         __attribute__((address_space(1))) char *const dst =
             (which ? cv : ck) + (((b0 + g) * H + c / CPR) * own_rows + slot) * static_cast<long>(DH * sizeof(T)) + 16 * (c % CPR);
         *(__attribute__((address_space(1))) u32x4 *)dst =

@@ -73,14 +73,33 @@ hipError_t tape_matrix(const void *w, char *tape, long stride, int N, int K, con
     return hipGetLastError();
 }
 
+// Several workgroups to a trajectory: the heads are dealt over them.
+template <typename T, int D, int F, int PARTS>
+hipError_t decode_parts(const TrajectoryParams &P, hipStream_t st) {
+    if constexpr (traj_parts_built(D, PARTS)) {
+        const long words = 2L * P.B * traj_exchange_words<T>(D);
+        hipLaunchKernelGGL(trajectory_exchange_kernel, dim3(static_cast<unsigned>((words + 255) / 256)), dim3(256), 0, st, P.exchange, words);
+        hipLaunchKernelGGL((trajectory_crews_kernel<T, D, F, PARTS>), dim3(static_cast<unsigned>((P.B + 7) / 8 * 8 * PARTS)),
+                           dim3(2 * kTrajWaves * 64), 0, st, P);
+        return hipGetLastError();
+    }
+    return hipErrorInvalidValue;
+}
+
 template <typename T>
-hipError_t decode(const TrajectoryParams &P, int D, int F, hipStream_t st) {
+hipError_t decode(const TrajectoryParams &P, int D, int F, int parts, hipStream_t st) {
     hipError_t e = hipErrorInvalidValue;
     with_shape<T>(D, F, [&](auto d, auto f) {
+        if (parts > 1) {
+            constexpr int kD = decltype(d)::value, kF = decltype(f)::value;
+            e = parts == 2 ? decode_parts<T, kD, kF, 2>(P, st) : parts == 4 ? decode_parts<T, kD, kF, 4>(P, st)
+                : parts == 8 ? decode_parts<T, kD, kF, 8>(P, st) : hipErrorInvalidValue;
+            return;
+        }
         const dim3 grid(static_cast<unsigned>((P.B + P.G - 1) / P.G)), block(kTrajWaves * 64);
         if constexpr (decltype(d)::value <= 256) {
             if (crews_serve(P, D, sizeof(T) == 4)) {
-                hipLaunchKernelGGL((trajectory_crews_kernel<T, decltype(d)::value, decltype(f)::value>), grid, dim3(2 * kTrajWaves * 64), 0, st, P);
+                hipLaunchKernelGGL((trajectory_crews_kernel<T, decltype(d)::value, decltype(f)::value, 1>), grid, dim3(2 * kTrajWaves * 64), 0, st, P);
                 e = hipGetLastError();
                 return;
             }
@@ -106,8 +125,8 @@ hipError_t decode(const TrajectoryParams &P, int D, int F, hipStream_t st) {
                                                const TrajectoryTapeLayout::Matrix &m, int section, hipStream_t st) { \
         return tape_matrix<TrajT>(w, tape, stride, N, K, m, section, st);                                             \
     }                                                                                                                 \
-    hipError_t launch_trajectory_decode_##suffix(const TrajectoryParams &P, int D, int F, hipStream_t st) {           \
-        return decode<TrajT>(P, D, F, st);                                                                            \
+    hipError_t launch_trajectory_decode_##suffix(const TrajectoryParams &P, int D, int F, int parts, hipStream_t st) { \
+        return decode<TrajT>(P, D, F, parts, st);                                                                     \
     }
 
 #if ARTAB_TRAJ_TYPE == 0

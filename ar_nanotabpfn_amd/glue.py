@@ -475,7 +475,11 @@ class TrajectoryDecoder:
         """Trajectories per workgroup, or 0 where the step-by-step launches are the faster route."""
         return _lib.load().artab_trajectory_group_layers(B, Nc, Nt, self.H, self.D, self.F, self.L, int(own_context), self.dtype_code)
 
-    def __call__(self, caches, n_ctx: int, own_base: int, x_mean: Tensor, rand_u: Tensor, rand_n: Tensor, group: int) -> Tensor:
+    def parts(self, B: int, Nc: int, Nt: int, own_context: bool) -> int:
+        """Workgroups per trajectory; 1 where ``group`` decides."""
+        return _lib.load().artab_trajectory_parts(B, Nc, Nt, self.H, self.D, self.F, self.L, int(own_context), self.dtype_code)
+
+    def __call__(self, caches, n_ctx: int, own_base: int, x_mean: Tensor, rand_u: Tensor, rand_n: Tensor, group: int, parts: int = 1) -> Tensor:
         """``caches``: per layer ``(context K, context V, trajectory K, trajectory V)``, contiguous; with
         ``n_ctx == 0`` every trajectory's own context fills the first ``own_base`` rows of its cache and
         the context tensors are not read.  ``x_mean [B,Nt]``; ``rand_u`` / ``rand_n`` ``[>=Nt,B]``.  Returns
@@ -493,5 +497,9 @@ class TrajectoryDecoder:
         a.own_rows, a.park_target = caches[0][2].shape[2], int(n_ctx == 0)
         a.rand_u, a.rand_n, a.rand_n_f32 = rand_u.data_ptr(), rand_n.data_ptr(), int(rand_n.dtype == torch.float32)
         a.x_mean, a.preds, a.B, a.Nt, a.group = x_mean.data_ptr(), preds.data_ptr(), B, Nt, group
-        _lib.check(_lib.load().artab_trajectory_decode(ctypes.byref(a), self.dtype_code, _lib.current_stream(self.device)))
+        lib = _lib.load()
+        exchange = None
+        if parts > 1:  # (of this call's own: freed for later work of this stream)
+            exchange = torch.empty(lib.artab_trajectory_exchange_bytes(B, self.D, self.dtype_code), device=self.device, dtype=torch.uint8)
+        _lib.check(lib.artab_trajectory_decode_parts(ctypes.byref(a), parts, _ptr(exchange), self.dtype_code, _lib.current_stream(self.device)))
         return preds

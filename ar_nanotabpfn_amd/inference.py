@@ -496,7 +496,10 @@ class ARTabPFNPredictor:
         run = self._trajectory[1]
         if run is not None and capturing(x_target.device) and not run.tables_made(caches):
             return None
-        group = run.group(B, n_ctx + own_base, Nt, not shared) if run is not None else 0
+        if run is None:
+            return None
+        parts = run.parts(B, n_ctx + own_base, Nt, not shared)
+        group = 1 if parts > 1 else run.group(B, n_ctx + own_base, Nt, not shared)
         if group == 0:
             return None
         device, dtype = x_target.device, x_target.dtype
@@ -509,7 +512,7 @@ class ARTabPFNPredictor:
             for u, n in zip(rand_u.unbind(0), rand_n.unbind(0)):  # as head.sample does, step by step
                 u.uniform_()
                 n.normal_()
-        values = run(caches, n_ctx, own_base, x_target.mean(dim=-1).contiguous(), rand_u, rand_n, group)
+        values = run(caches, n_ctx, own_base, x_target.mean(dim=-1).contiguous(), rand_u, rand_n, group, parts)
         if shared:
             self.buffer_len = Nt - 1
             self.seq_len = self.context_len + self.buffer_len

@@ -677,6 +677,16 @@ size_t artab_trajectory_tape_bytes(int D, int F, int n_layers, int dtype);
 int artab_trajectory_pack(void *tape, const void *w, int which, int layer, int rows, int D, int F, int n_layers,
                           int dtype, void *stream);
 int artab_trajectory_decode(const artab_trajectory_args *args, int dtype, void *stream);
+/*
+ * The same with `parts` workgroups (2, 4 or 8, no more than heads; D up to 256; args->group is 1) to a trajectory: each
+ * computes its share of the heads, what follows the attention all of them.  They wait for each other once per layer; a
+ * wait that is in vain for some ten seconds turns the trajectory's further draws into NaN.  `exchange`:
+ * artab_trajectory_exchange_bytes of device memory (16-byte aligned) of this call's own until it is done.
+ * artab_trajectory_parts says how many are fastest: 1 where artab_trajectory_group_layers decides.
+ */
+int artab_trajectory_parts(int B, int Nc, int Nt, int H, int D, int F, int n_layers, int own_context, int dtype);
+size_t artab_trajectory_exchange_bytes(int B, int D, int dtype);
+int artab_trajectory_decode_parts(const artab_trajectory_args *args, int parts, void *exchange, int dtype, void *stream);
 
 /*
  * The boundary between two decode steps in one launch: artab_layer_post (or

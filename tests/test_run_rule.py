@@ -1,6 +1,8 @@
 """Where a sampling run takes the whole-run kernel: the rule against what both routes took on an MI355X (us per layer
 and step)."""
 
+import ctypes
+
 import pytest
 
 from ar_nanotabpfn_amd import _lib
@@ -47,3 +49,43 @@ SHARED = [
 def test_shared_contexts_take_the_faster_route(dtype, D, B, Nc, run, steps):
     group = _lib.load().artab_trajectory_group_layers(B, Nc, 12, D // 32, D, 256, 4, 0, dtype)
     assert (group > 0) == (run < steps)
+
+
+# several workgroups to a trajectory: dtype, d_model, trajectories, context rows, own contexts, us per layer and step with
+# 1, 2, 4 and 8 of them, step by step (4 layers; None: not built, or not measured)
+PARTS = [
+    (BF16, 128, 64, 16000, 0, (102.9, 61.4, 33.4, None), 31.9), (BF16, 128, 32, 4000, 0, (30.7, 19.1, 13.2, None), 25.2),
+    (BF16, 128, 100, 200, 0, (10.0, 10.4, None, None), 33.1), (BF16, 128, 128, 3000, 0, (28.7, 20.5, None, None), 32.9),
+    (BF16, 256, 32, 300, 0, (15.7, 12.1, 9.9, 10.5), 24.3), (BF16, 256, 32, 16000, 0, (203.8, 120.4, 65.6, 37.7), 36.1),
+    (BF16, 256, 64, 16000, 0, (200.6, 116.7, 61.7, None), 35.1), (BF16, 256, 8, 4000, 0, (66.4, 39.1, 22.7, 16.8), 28.8),
+    (BF16, 256, 64, 600, 1, (21.7, 15.7, 15.7, None), None), (BF16, 256, 64, 2500, 1, (72.6, 42.6, 35.9, None), None),
+    (BF16, 512, 8, 300, 0, (44.1, 33.9, 27.9, 23.4), 45.4), (BF16, 512, 32, 16000, 0, (420.4, 267.5, 137.3, 80.3), 68.5),
+    (BF16, 512, 64, 2500, 1, (144.6, 106.5, 86.5, None), None), (F32, 128, 64, 32, 0, (15.7, 16.3, 16.2, None), 124.2),
+    (F32, 128, 8, 4000, 0, (84.2, 46.4, 29.3, None), 85.7), (F32, 256, 32, 300, 0, (40.6, 30.5, 26.8, 26.9), 136.8),
+    (F32, 256, 128, 16000, 0, (588.7, 304.0, None, None), 356.7), (F32, 256, 64, 2500, 1, (154.5, 103.3, 78.1, None), None)]
+
+
+@pytest.mark.parametrize("dtype,D,B,Nc,own,times,steps", PARTS)
+def test_workgroups_per_trajectory(dtype, D, B, Nc, own, times, steps):
+    lib = _lib.load()
+    parts = lib.artab_trajectory_parts(B, Nc, 24, D // 32, D, 256, 4, own, dtype)
+    assert parts * B <= 256 or parts == 1
+    taken = times[parts.bit_length() - 1]
+    if parts == 1 and not lib.artab_trajectory_group_layers(B, Nc, 24, D // 32, D, 256, 4, own, dtype):
+        taken = steps
+    assert taken <= 1.1 * min(t for t in (*times, steps) if t is not None)
+
+
+def test_workgroups_per_trajectory_are_checked():
+    lib = _lib.load()
+    a = _lib.ArtabTrajectoryArgs()
+    for name, kind in a._fields_:  # (pointers that nobody follows: the calls end in front of the launch)
+        if kind is ctypes.c_void_p:
+            setattr(a, name, 4096)
+    a.n_layers, a.n_ctx, a.ctx_rows, a.own_rows, a.K, a.bs, a.B, a.Nt, a.group, a.D, a.F = 2, 8, 8, 8, 3, 4, 4, 4, 1, 128, 256
+    call = lambda parts, exchange: lib.artab_trajectory_decode_parts(ctypes.byref(a), parts, exchange, BF16, None)  # noqa: E731
+    assert call(3, 4096) == call(8, 4096) == call(0, 4096) == call(-2, 4096) == _lib.ARTAB_ERR_UNSUPPORTED
+    assert call(2, None) == _lib.ARTAB_ERR_NULL_POINTER and call(2, 4104) == _lib.ARTAB_ERR_BAD_STRIDE
+    a.group = 2
+    assert call(2, 4096) == _lib.ARTAB_ERR_UNSUPPORTED
+    assert lib.artab_trajectory_exchange_bytes(4, 128, BF16) == 2 * 4 * 128 * 8 and lib.artab_trajectory_exchange_bytes(0, 128, BF16) == 0
