@@ -81,14 +81,21 @@ static hipError_t launch_flash_bm(const FlashParams &P, int BM, hipStream_t stre
         // the lean pass: 256 query rows as eight wavefronts of one 32-row block each, four
         // wavefronts per SIMD (kTuneLean = 0 selects the software-pipelined form)
         if (BM == 256 && tune(kTuneLean, 1) != 0) {
-            // 96 registers (five per SIMD by the register file) leave room for the streaming
-            // buffer pass beside four of these wavefronts; kTuneLeanOcc = 4 takes 128
-            if (tune(kTuneLeanOcc, 5) == 4)
-                launch_one(flash_kernel<T, DH, 1, 8, kFlashBN, true, 4>, grid, 512, stream, P);
-            else if (P.mode == kFlashContext)  // the decode launch: nothing but the context pass compiled in
+            // Beside a streaming buffer pass 96 registers (five per SIMD by the register file) leave room for its wavefront
+            // beside four of these.  Alone (kTuneLeanOcc = 4: always) teacher forcing and the row mask take 128: bf16, us, 64 x 8 pairs, 128 targets,
+            // 512 own keys 26.3 -> 23.5, 200 targets, 2000 keys 102.6 -> 95.1; 64 x 4 pairs of 1544 rows, 1000 keys 103.6 ->
+            // 92.8; prefills of bf16 do not gain (64 x 8 x 512 rows 34.9, 36.0).  f16 needs them for its reference (mfma_flash.h), and
+            // spills at 96.
+            constexpr bool f16 = !MfmaOps<T>::kWideExponent;
+            const bool beside = P.beside_rows || P.beside_n > 0 || P.yield_from > 0, four = tune(kTuneLeanOcc, 5) == 4;
+            if (P.mode == kFlashContext && !four && (beside || !f16))  // the decode launch: nothing but the context pass compiled in
                 launch_one(flash_kernel<T, DH, 1, 8, kFlashBN, true, 5, true>, grid, 512, stream, P);
-            else
+            else if (P.mode == kFlashContext && f16)
+                launch_one(flash_kernel<T, DH, 1, 8, kFlashBN, true, 4, f16>, grid, 512, stream, P);
+            else if (P.mode == kFlashPrefill && !f16 && !four)
                 launch_one(flash_kernel<T, DH, 1, 8, kFlashBN, true, 5>, grid, 512, stream, P);
+            else
+                launch_one(flash_kernel<T, DH, 1, 8, kFlashBN, true, 4>, grid, 512, stream, P);
             return hipGetLastError();
         }
     }

@@ -27,8 +27,14 @@
 // float32 holds 2^s for |s| < 126, bf16 keeps that exponent range, and the
 // accumulators are float32.  A row whose probability mass leaves [2^-100, 2^100]
 // (or any NaN/inf) makes the whole workgroup redo its tile range with the
-// classical online-softmax (running maximum, rescaled accumulators); fp16, whose
-// exponent range is too small for the fast path, always takes that robust path.
+// classical online-softmax (running maximum, rescaled accumulators).  f16, whose
+// exponent range is too small for that, takes its probabilities against one reference per row, the largest
+// score of the first 64 keys, where the pass is the lean one (256 query rows, head_dim 32), and the
+// online softmax elsewhere; a row sum that has overflowed (a later score 2^20 times the reference) makes it redo
+// its range like the others.  One multiply-add per score for scale and reference, so that the queries stay as
+// they are: error against float64 2.9e-4 where the online softmax has 3.5e-4 (64 x 8 pairs of 512 normal rows).
+// us, online softmax -> this: prefill of 64 x 8 x 512 rows 52.0 -> 41.1, 1 x 8 x 16384 533 -> 354; 1024 x 8 x 2 queries over
+// 16384 keys 90.0 -> 61.0; 64 x 4 pairs of 1544 rows, 1000 keys 144 -> 108.
 #pragma once
 
 #include <type_traits>
@@ -174,6 +180,7 @@ __device__ __forceinline__ void flash_stamp_end(const FlashParams &P) {
 // Probability mass (sum of 2^s over a row) the fast path accepts.
 constexpr float kFastMassMax = 1.2676506e30f;  // 2^100
 constexpr float kFastMassMin = 7.8886091e-31f; // 2^-100
+constexpr float kLeanAbove = 4.f;              // f16: see lean_pass
 
 // Largest / smallest teacher-forcing key limit over query rows [a, b] (inclusive).
 __host__ __device__ inline int tf_range_max(int a, int b, int Nt) {
@@ -1013,6 +1020,11 @@ void flash_kernel(const char *early_k, const char *early_v, int early_sh, int ea
             }
         };
 
+        // f16: the queries are not scaled; scale and reference of a column's scores are one operation (scaled queries with the
+        // reference as what the products start from would save it, 305 us instead of 354 at 8 x 16384 rows, for 1.04 times the
+        // online softmax's error).
+        const float f16_scale = P.qscale;
+        auto exponent = [&](int j, float s) { return Ops::kWideExponent ? s : fmaf(s, f16_scale, -m_run[j]); };
         // One 32-key block of the tile in `stage_` against this wavefront's queries.
         auto block = [&](auto stage_, int sb, auto mask_tag, int blk0, bool is_ctx, int seg_end) {
             constexpr bool MASK = decltype(mask_tag)::value;
@@ -1054,7 +1066,7 @@ void flash_kernel(const char *early_k, const char *early_v, int early_sh, int ea
                 for (int t = 0; t < 2; ++t)
 #pragma unroll
                     for (int e = 0; e < 4; ++e)
-                        pb[t][e] = pack2<T>(fast_exp2(s[8 * t + 2 * e]), fast_exp2(s[8 * t + 2 * e + 1]));
+                        pb[t][e] = pack2<T>(fast_exp2(exponent(j, s[8 * t + 2 * e])), fast_exp2(exponent(j, s[8 * t + 2 * e + 1])));
 #pragma unroll
                 for (int t = 0; t < 2; ++t) lsum[j][t] = Ops::mma16(ones_sel, __builtin_bit_cast(vec, pb[t]), lsum[j][t]);
 #pragma unroll
@@ -1169,7 +1181,37 @@ void flash_kernel(const char *early_k, const char *early_v, int early_sh, int ea
                 for (int t = 2; t < NST - 1; ++t)
                     if (n_main > t) dma_tile(t);
             }
-            scale_q(qraw, lane);
+            if constexpr (Ops::kWideExponent) {
+                scale_q(qraw, lane);
+            } else {  // (a column past the last row is the group's first row, computed for nobody)
+#pragma unroll
+                for (int j = 0; j < QB; ++j)
+#pragma unroll
+                    for (int ks = 0; ks < KS; ++ks) qreg[j][ks] = __builtin_bit_cast(vec, qraw[j][ks]);
+            }
+        }
+        if constexpr (!Ops::kWideExponent) {
+            // The reference: the column's largest score among the keys of the first tile, kLeanAbove (base 2) above it.  A probability
+            // overflows 16 bits if a later score is 20 (base 2) larger, and the row sum says so: the robust pass then.
+            __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+            __syncthreads();
+            const int seen = ctx_end - ctx_begin;
+#pragma unroll
+            for (int j = 0; j < QB; ++j) {
+                float top = -INFINITY;
+#pragma unroll
+                for (int sb = 0; sb < SB; ++sb) {
+                    f32x16 s;
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) s[v] = 0.f;
+#pragma unroll
+                    for (int ks = 0; ks < KS; ++ks)
+                        s = Ops::mma(*reinterpret_cast<const vec *>(kv_lds + lk_rd + (sb * KS + ks) * CH), qreg[j][ks], s);
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) top = fmaxf(top, 32 * sb + 8 * (v >> 2) + 4 * hb + (v & 3) < seen ? s[v] : -INFINITY);
+                }
+                m_run[j] = fmaf(fmaxf(top, __shfl_xor(top, 32, 64)), f16_scale, kLeanAbove);
+            }
         }
 
         int it = 0;
@@ -1273,7 +1315,8 @@ void flash_kernel(const char *early_k, const char *early_v, int early_sh, int ea
         }
     };
 
-    bool robust = !Ops::kWideExponent || P.force_robust;
+    // (the lean pass of f16 takes its reference from a tile of context keys)
+    bool robust = P.force_robust || (!Ops::kWideExponent && (!LEAN || ctx_tiles == 0));
     if (!robust) {
         if constexpr (LEAN)
             lean_pass();
