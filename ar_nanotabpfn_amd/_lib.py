@@ -137,6 +137,26 @@ class ArtabTrainEmbedArgs(ctypes.Structure):
     ]
 
 
+class ArtabEmbedRowsArgs(ctypes.Structure):
+    """``artab_embed_rows_args`` of include/artab_attention.h, field for field."""
+
+    _fields_ = [
+        ("x", _p), ("y", _p), *((n, ctypes.c_int64) for n in ("x_stride_b", "x_stride_n", "x_stride_c", "y_stride_b", "y_stride_n")),
+        *((n, _i) for n in ("B", "N", "C", "D", "pairs")), *((n, _p) for n in ("w_x", "b_x", "w_y", "b_y", "markers", "ar_tokens")),
+        ("bs", _i), ("out", _p),
+    ]
+
+
+class ArtabDensityArgs(ctypes.Structure):
+    """``artab_density_args`` of include/artab_attention.h, field for field."""
+
+    _fields_ = [
+        ("x", _p), ("x_stride_b", ctypes.c_int64), ("norm_gamma", _p), ("norm_beta", _p), ("eps", _f),
+        *((n, _p) for n in ("w1", "b1", "w2", "b2", "mean_bias", "std_bias", "weight_bias")), ("K", _i), ("std_min", _f), ("y", _p),
+        ("y_stride_b", ctypes.c_int64), ("y_stride_n", ctypes.c_int64), ("out", _p), *((n, _i) for n in ("B", "Nt", "D", "F")),
+    ]
+
+
 class ArtabTrainHeadArgs(ctypes.Structure):
     """``artab_train_head_args`` of include/artab_attention.h, field for field."""
 
@@ -234,6 +254,9 @@ SIGNATURES = {
     "artab_trajectory_tape_bytes": (_sz, [_i, _i, _i, _i]),
     "artab_trajectory_pack": (_i, [_p, _p, _i, _i, _i, _i, _i, _i, _i, _p]),
     "artab_trajectory_decode": (_i, [ctypes.POINTER(ArtabTrajectoryArgs), _i, _p]),
+    "artab_embed_rows": (_i, [ctypes.POINTER(ArtabEmbedRowsArgs), _i, _p]),
+    "artab_density_supported": (_i, [_i, _i, _i]),
+    "artab_density": (_i, [ctypes.POINTER(ArtabDensityArgs), _i, _p]),
     "artab_trajectory_parts": (_i, [_i, _i, _i, _i, _i, _i, _i, _i, _i]),
     "artab_trajectory_exchange_bytes": (_sz, [_i, _i, _i]),
     "artab_trajectory_decode_parts": (_i, [ctypes.POINTER(ArtabTrajectoryArgs), _i, _p, _i, _p]),

@@ -49,7 +49,8 @@ EXPORTS = "{ global: artab_*; local: *; };\n"
 # (source, extra defines, object name)
 UNITS = [("artab_api.hip", [], "artab_api.o"), ("flash_launch.hip", [], "flash_launch.o"), ("f32_launch.hip", [], "f32_launch.o"),
          ("f32_layer_launch.hip", [], "f32_layer_launch.o"),
-         ("backward_launch.hip", [], "backward_launch.o"), ("train_launch.hip", [], "train_launch.o")]
+         ("backward_launch.hip", [], "backward_launch.o"), ("train_launch.hip", [], "train_launch.o"),
+         ("density_launch.hip", [], "density_launch.o")]
 # objects that differ between the two libraries
 PRODUCT_ONLY = [("launch_observer_none.hip", [], "launch_observer_none.o")]
 BENCH_ONLY = [("bench_hooks.hip", [], "bench_hooks.o"), ("mix_bench.hip", [], "mix_bench.o")]

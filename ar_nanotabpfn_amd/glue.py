@@ -16,6 +16,7 @@ from typing import Optional
 import torch
 import torch.nn.functional as F
 from torch import Tensor, nn
+from torch.autograd import forward_ad
 
 from . import _lib
 from .live import Prepared
@@ -212,6 +213,64 @@ def layer_post_pre(attn: Tensor, y: Tensor, w_o: Tensor, norm2: nn.LayerNorm, w_
         )
     )
     return y_next, qkv_next
+
+
+def _plain(device, dtype, *tensors_and_shapes) -> bool:
+    """Tensors as a launch reads them: of this type, on this device, of these sizes, without strides, in 16-byte pieces."""
+    return all(t is not None and type(t) in (Tensor, nn.Parameter) and t.dtype == dtype and t.device == device and t.shape == s
+               and t.is_contiguous() and t.data_ptr() % 16 == 0 for t, s in zip(tensors_and_shapes[0::2], tensors_and_shapes[1::2]))
+
+
+def _values_only() -> bool:
+    """Whether a call may pass torch's operators by: nothing is recorded, cast, traced, transformed or given a tangent."""
+    return not (torch.is_grad_enabled() or torch.is_autocast_enabled("cuda") or torch.jit.is_tracing()
+                or torch._C._are_functorch_transforms_active() or forward_ad._current_level >= 0)
+
+
+def embed_context_rows(embedder, x: Tensor, y: Tensor, ar_tokens: Optional[Tensor] = None) -> Optional[Tensor]:
+    """``embedder.embed_context(x, y)`` ``[B,N,D]``, or with ``ar_tokens [bs,D]`` the rows of a teacher-forced pass
+    ``[B,2N,D]`` (buffer rows with their position tokens, then target rows), as one launch (``artab_embed_rows``); None
+    where the launch does not stand for the modules, which the caller has looked at.  ``x [B,N,C]``, ``y [B,N]`` or ``[B,N,1]``, any strides."""
+    if not (x.is_cuda and x.dtype in _lib._DTYPE_CODE and _values_only() and type(x) in (Tensor, nn.Parameter) and type(y) in (Tensor, nn.Parameter)
+            and x.dim() == 3 and y.dtype == x.dtype and y.device == x.device and (y.shape == x.shape[:2] or y.shape == (*x.shape[:2], 1)) and x.numel()):
+        return None
+    w_x, w_y, markers = embedder.x_embed.weight, embedder.y_embed.weight, embedder.marker_embed.weight
+    (B, N, C), D, pairs = x.shape, w_x.shape[0], ar_tokens is not None
+    params = (w_x, (D, 1), embedder.x_embed.bias, (D,), w_y, (D, 1), embedder.y_embed.bias, (D,), markers, (3, D))
+    if pairs:
+        params += (ar_tokens, (ar_tokens.shape[0], D))
+    if not (D % 8 == 0 and B * N < 2 ** 32 // D and _plain(x.device, x.dtype, *params) and (not pairs or len(ar_tokens))):
+        return None
+    out = torch.empty((B, 2 * N if pairs else N, D), device=x.device, dtype=x.dtype)
+    a = _lib.ArtabEmbedRowsArgs(x.data_ptr(), y.data_ptr(), *x.stride(), *y.stride()[:2], B, N, C, D, int(pairs), *(p.data_ptr() for p in params[0:10:2]),
+                                ar_tokens.data_ptr() if pairs else None, len(ar_tokens) if pairs else 0, out.data_ptr())
+    _lib.check(_lib.load().artab_embed_rows(ctypes.byref(a), _lib.dtype_code(x.dtype), _lib.current_stream(x.device)))
+    return out
+
+
+def mixture_log_density(norm: nn.LayerNorm, head, rows: Tensor, y: Tensor) -> Optional[Tensor]:
+    """``head.log_likelihood(norm(rows), y[..., None])`` ``[B,Nt]`` as one launch (``artab_density``), or None where it does not stand
+    for the modules, which the caller has looked at.  ``rows [B,Nt,D]`` with rows behind each other, ``y [B,Nt]``."""
+    if not (rows.is_cuda and rows.dtype in _lib._DTYPE_CODE and _values_only() and type(rows) is Tensor and type(y) in (Tensor, nn.Parameter)
+            and y.shape == rows.shape[:2] and y.dtype == rows.dtype and y.device == rows.device and y.numel()):
+        return None
+    one, two, (B, Nt, D) = head.head[0], head.head[2], rows.shape
+    F_, K, lib = one.out_features, head.num_components, _lib.load()
+    if not (head.dim_y == 1 and isinstance(K, int) and isinstance(head.std_min, float) and lib.artab_density_supported(D, F_, K)
+            and rows.stride(2) == 1 and (Nt == 1 or rows.stride(1) == D) and B * Nt < 2 ** 30 and norm.normalized_shape == (D,)):
+        return None
+    # (the launch reads vectors element by element: any place will do)
+    vectors = (norm.weight, (D,), norm.bias, (D,), one.bias, (F_,), two.bias, (3 * K,), head.mean_bias, (K,), head.std_bias, (K,), head.weight_bias, (K,))
+    if not (_plain(rows.device, rows.dtype, one.weight, (F_, D), two.weight, (3 * K, F_))
+            and all(t is not None and type(t) in (Tensor, nn.Parameter) and t.dtype == rows.dtype and t.device == rows.device and t.shape == s
+                    and t.is_contiguous() for t, s in zip(vectors[0::2], vectors[1::2]))):
+        return None
+    out = torch.empty((B, Nt), device=rows.device, dtype=rows.dtype)
+    v = [t.data_ptr() for t in vectors[0::2]]
+    a = _lib.ArtabDensityArgs(rows.data_ptr(), rows.stride(0), v[0], v[1], norm.eps, one.weight.data_ptr(), v[2], two.weight.data_ptr(), v[3], *v[4:],
+                              K, head.std_min, y.data_ptr(), *y.stride(), out.data_ptr(), B, Nt, D, F_)
+    _lib.check(lib.artab_density(ctypes.byref(a), _lib.dtype_code(rows.dtype), _lib.current_stream(rows.device)))
+    return out
 
 
 class SampleEmbedStep:

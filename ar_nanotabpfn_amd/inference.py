@@ -27,9 +27,10 @@ from . import attention_kernels as ak
 from .attention import DecodeMask, TeacherForcingMask
 from . import _lib
 from .live import Methods, ModelState, capturing, plain_modules
-from .model import Embedder, MixtureGaussianHead
+from .model import Embedder, MixtureGaussianHead, density_as_defined, embedder_as_defined
 from .stack import LAYER_METHODS, LayerStack
-from .glue import SampleEmbedStep, DecodeStepBoundary, TrajectoryDecoder, add_layer_norm
+from .glue import (SampleEmbedStep, DecodeStepBoundary, TrajectoryDecoder, add_layer_norm, embed_context_rows,
+                   mixture_log_density)
 
 __all__ = ["ARTabPFNPredictor"]
 
@@ -250,7 +251,12 @@ class ARTabPFNPredictor:
         if self.backend == _SHARED:
             self.prefill_context_shared(x_context, y_context)
             return
-        self._prefill_own(self.embedder.embed_context(x_context, y_context))
+        self._prefill_own(self._context_rows(x_context, y_context))
+
+    def _context_rows(self, x: Tensor, y: Tensor) -> Tensor:
+        """The embedded context rows: one launch where it stands for the embedder's methods."""
+        rows = embed_context_rows(self.embedder, x, y) if x.is_cuda and embedder_as_defined(self.embedder) else None
+        return self.embedder.embed_context(x, y) if rows is None else rows
 
     def _prefill_own(self, x_row: Tensor) -> None:
         """``prefill_context`` of embedded rows, a cache for each batch entry."""
@@ -267,7 +273,7 @@ class ARTabPFNPredictor:
     def prefill_context_shared(self, x_context: Tensor, y_context: Tensor) -> None:
         """Shared layout: only batch entry 0 is encoded — the context is taken to be the
         same for every trajectory (inference.py:180-223)."""
-        self._prefill_shared(self.embedder.embed_context(x_context[0:1], y_context[0:1]), x_context.shape[0])
+        self._prefill_shared(self._context_rows(x_context[0:1], y_context[0:1]), x_context.shape[0])
 
     def _prefill_shared(self, x_row: Tensor, batch: int) -> None:
         """``prefill_context_shared`` of embedded rows, for ``batch`` trajectories."""
@@ -828,6 +834,10 @@ class ARTabPFNPredictor:
 
     def _teacher_forcing_embedding(self, x_target: Tensor, y_target: Tensor) -> Tensor:
         Nt = x_target.shape[1]
+        if x_target.is_cuda and embedder_as_defined(self.embedder):
+            rows = embed_context_rows(self.embedder, x_target, y_target, self.ar_tokens)
+            if rows is not None:
+                return rows
         pos = torch.arange(Nt, device=x_target.device) % self.ar_tokens.shape[0]
         buffer_emb = self.embedder.embed_buffer(x_target, y_target) + self.ar_tokens[pos]
         return torch.cat([buffer_emb, self.embedder.embed_target(x_target)], dim=1)
@@ -835,10 +845,25 @@ class ARTabPFNPredictor:
     def _evaluate_joint_density_shared(self, x_context, y_context, x_target, y_target) -> Tensor:
         B, Nt = x_context.shape[0], x_target.shape[1]
         self.init_kv_cache(B, Nt, x_context.device, x_context.dtype)
-        z = self._density_pass(x_context, y_context, x_target, y_target)
-        if z is None:
+        rows = self._density_pass(x_context, y_context, x_target, y_target)
+        if rows is None:
             self.prefill_context(x_context, y_context)
-            z = self._teacher_forcing_decode_shared(self._teacher_forcing_embedding(x_target, y_target), Nt)
+            targets = self._teacher_forcing_embedding(x_target, y_target)
+            if not _DENSITY_METHODS.of(self):
+                z = self._teacher_forcing_decode_shared(targets, Nt)
+                return self.head.log_likelihood(z[:, Nt:, :], y_target.unsqueeze(-1))
+            rows = self._teacher_forcing_rows_shared(targets, Nt)
+        return self._log_density(rows, y_target)
+
+    @torch.no_grad()
+    def _log_density(self, rows: Tensor, y_target: Tensor) -> Tensor:
+        """Log-density ``[B,Nt]`` from the layer stack's rows ``[B,2Nt,D]``."""
+        Nt = rows.shape[1] // 2
+        if rows.is_cuda and density_as_defined(self.backbone.norm, self.head):
+            density = mixture_log_density(self.backbone.norm, self.head, rows[:, Nt:], y_target)
+            if density is not None:
+                return density
+        z = add_layer_norm(rows, None, None, self.backbone.norm)
         return self.head.log_likelihood(z[:, Nt:, :], y_target.unsqueeze(-1))
 
     # Rows up to which the two passes of a density share their layer boundaries: such a boundary is a launch of few
@@ -847,7 +872,7 @@ class ARTabPFNPredictor:
 
     def _density_pass(self, x_context, y_context, x_target, y_target) -> Optional[Tensor]:
         """Prefill and teacher-forced pass, side by side where the library takes them so, on caches that have just been
-        made: the second one's normed rows, or None, with nothing done, where they are not even tried so."""
+        made: the second one's rows, or None, with nothing done, where they are not even tried so."""
         (B, Nt), shared = x_target.shape[:2], self.backend == _SHARED
         if not (x_context.is_cuda and _DENSITY_METHODS.of(self) and Nt > 0 and x_context.shape[1] > 0
                 and x_context.shape[1] * (1 if shared else B) + 2 * B * Nt <= self._DENSITY_ROWS):
@@ -856,35 +881,43 @@ class ARTabPFNPredictor:
         if not (ak is _attention_module and _STACK_METHODS.of(self)
                 and self._stack.applies(layers, torch.Size((n, x_context.shape[1], self.backbone.d_model)), x_context.dtype, x_context.device)):
             return None
-        x_row = self.embedder.embed_context(x_context[:n], y_context[:n])
+        x_row = self._context_rows(x_context[:n], y_context[:n])
         caches = self._context_caches(x_row) if shared else [(l.k_cache, l.v_cache) for l in self.backbone.layers]
         targets = self._teacher_forcing_embedding(x_target, y_target)
         z = self._prefill_pass(x_row, caches, targets)
         if z is None:  # (layers or caches are not of its form: one after the other, with the rows that are embedded now)
             if shared:
                 self._prefill_shared(x_row, x_context.shape[0])
-                return self._teacher_forcing_decode_shared(targets, Nt)
+                return self._teacher_forcing_rows_shared(targets, Nt)
             self._prefill_own(x_row)
-            return self._teacher_forcing_decode(targets, Nt)
+            return self._teacher_forcing_rows(targets, Nt)
         self.seq_len = x_row.shape[1]
         if shared:
             self.context_len, self.buffer_len, self._prefill_batch_size = x_row.shape[1], 0, x_context.shape[0]
-        return add_layer_norm(z, None, None, self.backbone.norm)
+        return z
 
     def _evaluate_joint_density_flex(self, x_context, y_context, x_target, y_target) -> Tensor:
         B, Nc = x_context.shape[0], x_context.shape[1]
         Nt = x_target.shape[1]
         self.init_kv_cache(B, Nc + 2 * Nt, x_context.device, x_context.dtype)
-        z = self._density_pass(x_context, y_context, x_target, y_target)
-        if z is None:
+        rows = self._density_pass(x_context, y_context, x_target, y_target)
+        if rows is None:
             self.prefill_context(x_context, y_context)
-            z = self._teacher_forcing_decode(self._teacher_forcing_embedding(x_target, y_target), Nt)
-        return self.head.log_likelihood(z[:, Nt:, :], y_target.unsqueeze(-1))
+            targets = self._teacher_forcing_embedding(x_target, y_target)
+            if not _DENSITY_METHODS.of(self):
+                z = self._teacher_forcing_decode(targets, Nt)
+                return self.head.log_likelihood(z[:, Nt:, :], y_target.unsqueeze(-1))
+            rows = self._teacher_forcing_rows(targets, Nt)
+        return self._log_density(rows, y_target)
 
     @torch.no_grad()
     def _teacher_forcing_decode(self, embedding: Tensor, num_targets: int) -> Tensor:
         """``[buffers, targets]`` under the teacher-forcing mask on the full cache
         (inference.py:455-471)."""
+        return add_layer_norm(self._teacher_forcing_rows(embedding, num_targets), None, None, self.backbone.norm)
+
+    def _teacher_forcing_rows(self, embedding: Tensor, num_targets: int) -> Tensor:
+        """That pass in front of the final norm."""
         if embedding.shape[1] != 2 * num_targets:
             raise ValueError("Expected N == 2*num_targets for teacher forcing.")
         mask = TeacherForcingMask(num_cached=self.seq_len, num_targets=num_targets)
@@ -892,10 +925,13 @@ class ARTabPFNPredictor:
         x_row = self._stack_pass(embedding, [(l.k_cache, l.v_cache) for l in self.backbone.layers], num_targets, start)
         if x_row is None:
             x_row = self._run_layers(embedding, lambda layer, q, k, v: self._attend_with_cache(layer, q, k, v, mask, start))
-        return add_layer_norm(x_row, None, None, self.backbone.norm)
+        return x_row
 
     @torch.no_grad()
     def _teacher_forcing_decode_shared(self, embedding: Tensor, num_targets: int) -> Tensor:
+        return add_layer_norm(self._teacher_forcing_rows_shared(embedding, num_targets), None, None, self.backbone.norm)
+
+    def _teacher_forcing_rows_shared(self, embedding: Tensor, num_targets: int) -> Tensor:
         if embedding.shape[1] != 2 * num_targets:
             raise ValueError("Expected N == 2*num_targets for teacher forcing.")
         x_row = self._stack_pass(embedding, [(l.k_ctx_cache, l.v_ctx_cache) for l in self.backbone.layers], num_targets,
@@ -903,7 +939,7 @@ class ARTabPFNPredictor:
         if x_row is None:
             x_row = self._run_layers(
                 embedding, lambda layer, q, k, v: self._attend_teacher_forcing_shared(layer, q, k, v, num_targets))
-        return add_layer_norm(x_row, None, None, self.backbone.norm)
+        return x_row
 
     def _layer_teacher_forcing_shared(self, layer, x_row: Tensor, num_targets: int) -> Tensor:
         """inference.py:835-890: buffer K/V are the fresh projections of the first Nt

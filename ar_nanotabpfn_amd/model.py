@@ -428,9 +428,22 @@ def _embedder_as_defined(embedder) -> bool:
     return plain_modules(modules, (Embedder, nn.Linear, nn.Linear, nn.Embedding)) and _EMBEDDER_METHODS.of(embedder)
 
 
+_DENSITY_METHODS = Methods(MixtureGaussianHead, "log_likelihood")
+
+
 def _head_as_defined(head) -> bool:
     modules, _ = walk((head,))
     return plain_modules(modules, (MixtureGaussianHead, nn.Sequential, nn.Linear, nn.GELU, nn.Linear)) and _HEAD_METHODS.of(head)
+
+
+def embedder_as_defined(embedder) -> bool:
+    """Whether a launch may stand for the embedder's methods (``glue.embed_context_rows``)."""
+    return _embedder_as_defined(embedder)
+
+
+def density_as_defined(norm, head) -> bool:
+    """Whether a launch may stand for the final norm and ``head.log_likelihood`` (``glue.mixture_log_density``)."""
+    return plain_modules((norm,), (nn.LayerNorm,)) and _head_as_defined(head) and _DENSITY_METHODS.of(head)
 
 
 def _backbone_as_defined(backbone) -> bool:

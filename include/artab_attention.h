@@ -689,6 +689,43 @@ size_t artab_trajectory_exchange_bytes(int B, int D, int dtype);
 int artab_trajectory_decode_parts(const artab_trajectory_args *args, int parts, void *exchange, int dtype, void *stream);
 
 /*
+ * Embedded rows in one launch (model.py:23-76): mean of the features * w_x + b_x + marker, context and buffer rows with
+ * y * w_y + b_y, buffer row n with position token n % bs.  pairs 0: context rows [B, N, D]; pairs 1: the rows of a
+ * teacher-forced pass [B, 2 N, D], buffer rows and then target rows (inference.py:420-437).  Strides in elements; float32 up to the
+ * result.  D a multiple of 8; the parameters and `out` 16-byte aligned.
+ */
+typedef struct artab_embed_rows_args {
+    const void *x, *y;       /* [B, N, C], [B, N] */
+    int64_t x_stride_b, x_stride_n, x_stride_c, y_stride_b, y_stride_n;
+    int B, N, C, D, pairs;
+    const void *w_x, *b_x, *w_y, *b_y, *markers, *ar_tokens; /* [D] x 4, [3, D], [bs, D] */
+    int bs;
+    void *out;
+} artab_embed_rows_args;
+int artab_embed_rows(const artab_embed_rows_args *args, int dtype, void *stream);
+
+/*
+ * The log-density of target rows in one launch: the final norm, gelu(z W_1^T + b_1) W_2^T + b_2 and the mixture of K normals at y
+ * (model.py:150-272, inference.py:440-453).  Weights row-major as the modules have them, W_1 and W_2 16-byte aligned.
+ * D in {128, 256, 512}, F = 256, 3 K <= 128 (artab_density_supported).
+ */
+typedef struct artab_density_args {
+    const void *x;           /* row t of batch entry b at x + b * x_stride_b + t * D elements */
+    int64_t x_stride_b;
+    const void *norm_gamma, *norm_beta;
+    float eps;
+    const void *w1, *b1, *w2, *b2, *mean_bias, *std_bias, *weight_bias;
+    int K;
+    float std_min;
+    const void *y;           /* [B, Nt] */
+    int64_t y_stride_b, y_stride_n;
+    void *out;               /* [B, Nt] */
+    int B, Nt, D, F;
+} artab_density_args;
+int artab_density_supported(int D, int F, int K);
+int artab_density(const artab_density_args *args, int dtype, void *stream);
+
+/*
  * The boundary between two decode steps in one launch: artab_layer_post (or
  * artab_layer_post_from_partials when `partials` is given and holds slots; `attn`, [B, D] with
  * row stride lda, is read otherwise) of the last layer on the B target rows y (row stride ldy),
