@@ -2,10 +2,16 @@
 // attention calls: the tail of a layer (out projection, norm2, feed-forward, norm3) and the head of the next
 // (feature stage, norm1, q/k/v projections), or either part alone.
 //
-// A workgroup takes 16 rows through all products with the activations in LDS; only attention output, y and
+// A workgroup takes TR rows through all products with the activations in LDS; only attention output, y and
 // q/k/v touch memory.  Bound: the float32 matrix rate of its compute unit, 256 FLOP per clock: 16 rows of
-// d_model 256 are 14.7 MFLOP, 24 us; a launch of up to 4096 rows takes 38 to 40 us, where seven library products
-// and the norms and activation between them took 60 (1440 rows) and, from Python, 200 us of host time.  Layouts:
+// d_model 256 are 14.7 MFLOP, 24 us; a launch of up to 4096 rows takes 38 to 41 us, where seven library products
+// and the norms and activation between them took 60 (1440 rows) and, from Python, 200 us of host time.
+//
+// Few rows leave most compute units idle in tiles of 16, so there are tiles of 8 and 4, which have to do without the
+// 16x16 form: v_mfma_f32_4x4x1_16b_f32 takes four tokens to 64 weights at the same rate, the sixteen blocks of a
+// fragment being four groups of outputs times four of contraction elements, whose sums are added at the end.  Four rows
+// are 6 us of products at d_model 256, under the 12 us that 1.8 MB of weights take through the compute unit.  A layer of
+// 333 rows of 256 with its attention 46 -> 30 us, of 1773 (density of 16 x 45 targets) 71 -> 59.  Layouts:
 //   * D = W X^T: a weight row is a row of the first operand, a token a column, so that a lane holds four
 //     neighbouring outputs of one token; contraction step 4t + e takes the elements {16t + 4g + e} (g = lane / 16),
 //     so fragments of both operands are 16-byte pieces;
@@ -32,15 +38,57 @@ struct F32LayerParams {
     float eps1, eps2, eps3;
 };
 
-constexpr int kF32Rows = 16;
-
 constexpr int f32_layer_waves(int D) { return D == 128 ? 8 : 16; }
+
+// The results of a product over a tile of TR rows, and where in a wavefront they are: a lane that `holds` has outputs
+// 4 sub .. 4 sub + 3 of token tok.
+template <int TR>
+struct F32Tile {
+    static_assert(TR == 4 || TR == 8 || TR == 16, "whole sets of four rows");
+    static constexpr bool kNarrow = TR < 16;  // products of 4x4 blocks
+    static constexpr int kSets = kNarrow ? TR / 4 : 1;
+    int tok, sub;
+    bool holds;
+    __device__ __forceinline__ explicit F32Tile(int lane) {
+        if constexpr (kNarrow) {  // every row of 16 lanes has all sums: the first kSets rows hold a set of four tokens each
+            tok = 4 * (lane >> 4) + (lane & 3);
+            sub = (lane >> 2) & 3;
+            holds = lane < 16 * kSets;
+        } else {
+            tok = lane & 15;
+            sub = lane >> 4;
+            holds = true;
+        }
+    }
+    // the row of the tile that the lane reads as the second operand, of set i
+    static __device__ __forceinline__ int row(int lane, int i) { return kNarrow ? 4 * i + (lane & 3) : lane & 15; }
+    static __device__ __forceinline__ f32x4 mma(float w, float x, const f32x4 &acc) {
+        if constexpr (kNarrow) return __builtin_amdgcn_mfma_f32_4x4x1f32(w, x, acc, 0, 0, 0);
+        else return __builtin_amdgcn_mfma_f32_16x16x4f32(w, x, acc, 0, 0, 0);
+    }
+    // 4x4 blocks: lanes 16 g .. have summed the contraction elements {16 t + 4 g + e} only
+    static __device__ __forceinline__ f32x4 finish(const f32x4 (&acc)[kSets], int lane) {
+        if constexpr (kNarrow) {
+            f32x4 r;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                float x[kSets];
+#pragma unroll
+                for (int i = 0; i < kSets; ++i) x[i] = row_sum(acc[i][e]);
+                r[e] = kSets > 1 && (lane & 16) ? x[kSets - 1] : x[0];
+            }
+            return r;
+        }
+        return acc[0];
+    }
+};
 
 // Products of one wavefront: its blocks of 16 outputs against the tile.  Fragments arrive in chunks of C, one
 // chunk ahead across block boundaries; begin() requests the first, to be called in front of the barrier or
 // the norm that the product has to wait for.
-template <int K, int NB, int NW>
+template <int K, int NB, int NW, int TR>
 struct F32Product {
+    typedef F32Tile<TR> Tile;
     static constexpr int C = K > 256 ? 4 : 8, T = K / 16,  // (8 would spill at K 512)
                         N = NB * T / C;
     static_assert(T % C == 0 && N >= 1, "whole chunks");
@@ -55,14 +103,20 @@ struct F32Product {
 #pragma unroll
         for (int j = 0; j < C; ++j) ring[0][j] = p[64 * j];
     }
-    // done(block of 16 outputs, acc): acc holds outputs 4 g .. 4 g + 3 of token lane % 16
+    // done(block of 16 outputs, acc): acc as F32Tile says
     template <typename Done>
     __device__ __forceinline__ void run(const float *w, const float *tile, int ld, int wave, int lane, Done done) {
-        const float *src = tile + (lane & 15) * ld + 4 * (lane >> 4);
-        f32x4 acc;
+        constexpr int S = Tile::kSets;
+        const float *src[S];
+#pragma unroll
+        for (int s = 0; s < S; ++s) src[s] = tile + Tile::row(lane, s) * ld + 4 * (lane >> 4);
+        f32x4 acc[S];
 #pragma unroll
         for (int i = 0; i < N; ++i) {
-            if (i % (T / C) == 0) acc = f32x4{0.f, 0.f, 0.f, 0.f};
+            if (i % (T / C) == 0) {
+#pragma unroll
+                for (int s = 0; s < S; ++s) acc[s] = f32x4{0.f, 0.f, 0.f, 0.f};
+            }
             if (i + 1 < N) {
                 const f32x4 *p = at(w, i + 1, wave, lane);
 #pragma unroll
@@ -70,18 +124,22 @@ struct F32Product {
             }
 #pragma unroll
             for (int j = 0; j < C; ++j) {
-                const f32x4 v = *reinterpret_cast<const f32x4 *>(src + 16 * (i % (T / C) * C + j));
+                f32x4 v[S];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(ring[i & 1][j][e], v[e], acc, 0, 0, 0);
+                for (int s = 0; s < S; ++s) v[s] = *reinterpret_cast<const f32x4 *>(src[s] + 16 * (i % (T / C) * C + j));
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int s = 0; s < S; ++s) acc[s] = Tile::mma(ring[i & 1][j][e], v[s][e], acc[s]);
             }
             __builtin_amdgcn_sched_barrier(0);  // requests further ahead than the ring would be parked in scratch memory
-            if (i % (T / C) == T / C - 1) done(wave + NW * (i / (T / C)), acc);
+            if (i % (T / C) == T / C - 1) done(wave + NW * (i / (T / C)), Tile::finish(acc, lane));
         }
     }
 };
 
 // Rows of `tile` normalised in place, a wavefront per row; `store` (or null): rows of D written there too.
-template <int D, int NW>
+template <int D, int NW, int TR>
 __device__ __forceinline__ void f32_norm_rows(float *tile, int ld, const float *gamma, const float *beta, float eps, int wave, int lane,
                                               float *store, long row0, int valid) {
     constexpr int E = D / 64;
@@ -89,7 +147,7 @@ __device__ __forceinline__ void f32_norm_rows(float *tile, int ld, const float *
 #pragma unroll
     for (int e = 0; e < E; ++e) g[e] = gamma[64 * e + lane], b[e] = beta[64 * e + lane];
 #pragma unroll
-    for (int r = wave; r < kF32Rows; r += NW) {
+    for (int r = wave; r < TR; r += NW) {
         float *row = tile + r * ld;
         float v[E], sum = 0.f, sq = 0.f;
 #pragma unroll
@@ -107,15 +165,17 @@ __device__ __forceinline__ void f32_norm_rows(float *tile, int ld, const float *
     }
 }
 
-template <int D, int F>
+template <int D, int F, int TR>
 __global__ __launch_bounds__(f32_layer_waves(D) * 64) void f32_layer_kernel(F32LayerParams P) {
-    constexpr int NW = f32_layer_waves(D), NT = NW * 64, TR = kF32Rows;
+    constexpr int NW = f32_layer_waves(D), NT = NW * 64;
     constexpr int LD = D + 4, LF = F + 4, LM = LD > LF ? LD : LF;
     constexpr int NBD = D / 16 / NW, NBF = F / 16 / NW;
     static_assert(NBD * NW * 16 == D && NBF * NW * 16 == F, "whole blocks per wavefront");
     __shared__ __attribute__((aligned(16))) float a[TR * LM];  // attention output, hidden layer, then the layer output
     __shared__ __attribute__((aligned(16))) float s[TR * LD];  // the row sums that are normalised
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, c = lane & 15, g = lane >> 4;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const F32Tile<TR> at(lane);
+    const int c = at.tok, g = at.sub;
     const long row0 = static_cast<long>(blockIdx.x) * TR;
     const int valid = static_cast<int>(min(static_cast<long>(TR), P.rows - row0));
     // rows past the end read the last one: valid addresses, and nothing of them is stored
@@ -128,6 +188,7 @@ __global__ __launch_bounds__(f32_layer_waves(D) * 64) void f32_layer_kernel(F32L
     };
     const auto add_to = [&](float *tile, const float *bias) {  // residual rows in `tile` += outputs (+ bias)
         return [=](int nb, const f32x4 &acc) {
+            if (!at.holds) return;
             f32x4 *p = reinterpret_cast<f32x4 *>(tile + c * LD + 16 * nb + 4 * g);
             f32x4 v = *p;
             if (bias) {
@@ -142,18 +203,18 @@ __global__ __launch_bounds__(f32_layer_waves(D) * 64) void f32_layer_kernel(F32L
         };
     };
 
-    F32Product<D, NBD, NW> fo;
+    F32Product<D, NBD, NW, TR> fo;
     if (P.post) {
-        F32Product<D, NBD, NW> o;
+        F32Product<D, NBD, NW, TR> o;
         o.begin(P.w_o, wave, lane);
         load_rows(a, LD, P.attn);
         load_rows(s, LD, P.y);
         __syncthreads();
         o.run(P.w_o, a, LD, wave, lane, add_to(s, nullptr));
-        F32Product<D, NBF, NW> up;
+        F32Product<D, NBF, NW, TR> up;
         up.begin(P.w_1, wave, lane);
         __syncthreads();
-        f32_norm_rows<D, NW>(s, LD, P.gamma2, P.beta2, P.eps2, wave, lane, nullptr, 0, 0);
+        f32_norm_rows<D, NW, TR>(s, LD, P.gamma2, P.beta2, P.eps2, wave, lane, nullptr, 0, 0);
         __syncthreads();
         up.run(P.w_1, s, LD, wave, lane, [&](int nb, const f32x4 &acc) {
             const f32x4 t = *reinterpret_cast<const f32x4 *>(P.b_1 + 16 * nb + 4 * g);
@@ -163,15 +224,15 @@ __global__ __launch_bounds__(f32_layer_waves(D) * 64) void f32_layer_kernel(F32L
                 const float h = acc[e] + t[e];
                 v[e] = 0.5f * h * (1.f + erff(h * 0.70710678118654752f));
             }
-            *reinterpret_cast<f32x4 *>(a + c * LF + 16 * nb + 4 * g) = v;
+            if (at.holds) *reinterpret_cast<f32x4 *>(a + c * LF + 16 * nb + 4 * g) = v;
         });
-        F32Product<F, NBD, NW> down;
+        F32Product<F, NBD, NW, TR> down;
         down.begin(P.w_2, wave, lane);
         __syncthreads();
         down.run(P.w_2, a, LF, wave, lane, add_to(s, P.b_2));
         if (P.pre) fo.begin(P.w_fo, wave, lane);
         __syncthreads();
-        f32_norm_rows<D, NW>(s, LD, P.gamma3, P.beta3, P.eps3, wave, lane, P.pre ? nullptr : P.out, row0, valid);
+        f32_norm_rows<D, NW, TR>(s, LD, P.gamma3, P.beta3, P.eps3, wave, lane, P.pre ? nullptr : P.out, row0, valid);
         if (!P.pre) return;
     } else {
         fo.begin(P.w_fo, wave, lane);
@@ -180,19 +241,20 @@ __global__ __launch_bounds__(f32_layer_waves(D) * 64) void f32_layer_kernel(F32L
     __syncthreads();
     // y = norm1(x + x W_fo^T): every wavefront reads all of s, so the sums go to the other tile
     fo.run(P.w_fo, s, LD, wave, lane, [&](int nb, const f32x4 &acc) {
-        const int at = c * LD + 16 * nb + 4 * g;
-        f32x4 v = *reinterpret_cast<const f32x4 *>(s + at);
+        if (!at.holds) return;
+        const int to = c * LD + 16 * nb + 4 * g;
+        f32x4 v = *reinterpret_cast<const f32x4 *>(s + to);
 #pragma unroll
         for (int e = 0; e < 4; ++e) v[e] += acc[e];
-        *reinterpret_cast<f32x4 *>(a + at) = v;
+        *reinterpret_cast<f32x4 *>(a + to) = v;
     });
-    F32Product<D, 3 * NBD, NW> qkv;
+    F32Product<D, 3 * NBD, NW, TR> qkv;
     qkv.begin(P.w_qkv, wave, lane);
     __syncthreads();
-    f32_norm_rows<D, NW>(a, LD, P.gamma1, P.beta1, P.eps1, wave, lane, P.y_next, row0, valid);
+    f32_norm_rows<D, NW, TR>(a, LD, P.gamma1, P.beta1, P.eps1, wave, lane, P.y_next, row0, valid);
     __syncthreads();
     qkv.run(P.w_qkv, a, LD, wave, lane, [&](int nb, const f32x4 &acc) {
-        if (c < valid) *reinterpret_cast<f32x4 *>(P.qkv + (row0 + c) * (3 * D) + 16 * nb + 4 * g) = acc;
+        if (at.holds && c < valid) *reinterpret_cast<f32x4 *>(P.qkv + (row0 + c) * (3 * D) + 16 * nb + 4 * g) = acc;
     });
 }
 
