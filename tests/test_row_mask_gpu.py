@@ -211,14 +211,16 @@ def test_row_mask_backward_argument_errors(device):
 
 def _torch_row_attention(q, k, v, context_len, buffer_len, attending_chunks, use_triton=True):
     """Plain PyTorch statement of the same op (dense mask, float32 softmax): the reference the
-    device path's parameter gradients are compared with."""
+    device path's parameter gradients are compared with.  In float32 under autocast too: the library's
+    batched bfloat16 products with a transposed right operand have faulted the device."""
     from ar_nanotabpfn_amd.attention import RowMask
 
     R = q.shape[2]
     mask = RowMask(R, context_len, buffer_len, attending_chunks).dense(q.device)
-    s = torch.matmul(q.float(), k.float().transpose(-1, -2)) * q.shape[-1] ** -0.5
-    p = torch.softmax(s.masked_fill(~mask, float("-inf")), dim=-1)
-    return torch.matmul(p, v.float()).to(q.dtype)
+    with torch.autocast("cuda", enabled=False):
+        s = torch.matmul(q.float(), k.float().transpose(-1, -2).contiguous()) * q.shape[-1] ** -0.5
+        p = torch.softmax(s.masked_fill(~mask, float("-inf")), dim=-1)
+        return torch.matmul(p, v.float().contiguous()).to(q.dtype)
 
 
 def _training_problem(device, dtype, cfg, B, Nc, Nb, Nt, seed=1):
