@@ -229,10 +229,13 @@ class _HeadLoss(torch.autograd.Function):
         lib = _lib.load()
         z, saved, *params = ctx.saved_tensors  # (raises if one of them was changed in place since)
         create_graph = torch.is_grad_enabled()
-        if create_graph or _transformed(dloss, z, *params):  # gradients that can be differentiated again, or many at once
+        transformed = _transformed(dloss, z, *params)
+        if create_graph or transformed:  # gradients that can be differentiated again, or many at once
             wanted = [t for t in (z, *params) if t.requires_grad]
             y = saved[: 4 * ctx.args.rows].view(torch.float32).view(*z.shape[:2], 1)  # (the kernels' copy)
-            with torch.enable_grad(), torch.autocast("cuda", torch.bfloat16):
+            # (in float32 under a transform: it makes batched products of the modules' products, their right operands transposed
+            # views, and those of bfloat16 have faulted the device)
+            with torch.enable_grad(), torch.autocast("cuda", torch.bfloat16, enabled=not transformed):
                 loss = torch.func.functional_call(ctx.head, dict(zip(_HEAD_PARAMETERS, params)), (z, y))[0]
             grads = iter(torch.autograd.grad(loss, wanted, dloss, create_graph=create_graph))
             dz, *dparams = (next(grads) if t.requires_grad else None for t in (z, *params))
