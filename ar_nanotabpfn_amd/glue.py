@@ -216,9 +216,14 @@ def layer_post_pre(attn: Tensor, y: Tensor, w_o: Tensor, norm2: nn.LayerNorm, w_
 
 
 def _plain(device, dtype, *tensors_and_shapes) -> bool:
-    """Tensors as a launch reads them: of this type, on this device, of these sizes, without strides, in 16-byte pieces."""
+    """Tensors as a launch reads them: of this type, on this device, of these sizes, without strides."""
     return all(t is not None and type(t) in (Tensor, nn.Parameter) and t.dtype == dtype and t.device == device and t.shape == s
-               and t.is_contiguous() and t.data_ptr() % 16 == 0 for t, s in zip(tensors_and_shapes[0::2], tensors_and_shapes[1::2]))
+               and t.is_contiguous() for t, s in zip(tensors_and_shapes[0::2], tensors_and_shapes[1::2]))
+
+
+def _in_pieces(*tensors):
+    """The tensors, or copies of them, for a launch that reads 16-byte pieces: a model's parameters can be views into one vector."""
+    return [t if t.data_ptr() % 16 == 0 else t.clone() for t in tensors]
 
 
 def _values_only() -> bool:
@@ -242,8 +247,9 @@ def embed_context_rows(embedder, x: Tensor, y: Tensor, ar_tokens: Optional[Tenso
     if not (D % 8 == 0 and B * N < 2 ** 32 // D and _plain(x.device, x.dtype, *params) and (not pairs or len(ar_tokens))):
         return None
     out = torch.empty((B, 2 * N if pairs else N, D), device=x.device, dtype=x.dtype)
-    a = _lib.ArtabEmbedRowsArgs(x.data_ptr(), y.data_ptr(), *x.stride(), *y.stride()[:2], B, N, C, D, int(pairs), *(p.data_ptr() for p in params[0:10:2]),
-                                ar_tokens.data_ptr() if pairs else None, len(ar_tokens) if pairs else 0, out.data_ptr())
+    read = _in_pieces(*params[0::2])  # (held until the launch)
+    a = _lib.ArtabEmbedRowsArgs(x.data_ptr(), y.data_ptr(), *x.stride(), *y.stride()[:2], B, N, C, D, int(pairs), *(p.data_ptr() for p in read[:5]),
+                                read[5].data_ptr() if pairs else None, len(ar_tokens) if pairs else 0, out.data_ptr())
     _lib.check(_lib.load().artab_embed_rows(ctypes.byref(a), _lib.dtype_code(x.dtype), _lib.current_stream(x.device)))
     return out
 
@@ -261,13 +267,12 @@ def mixture_log_density(norm: nn.LayerNorm, head, rows: Tensor, y: Tensor) -> Op
         return None
     # (the launch reads vectors element by element: any place will do)
     vectors = (norm.weight, (D,), norm.bias, (D,), one.bias, (F_,), two.bias, (3 * K,), head.mean_bias, (K,), head.std_bias, (K,), head.weight_bias, (K,))
-    if not (_plain(rows.device, rows.dtype, one.weight, (F_, D), two.weight, (3 * K, F_))
-            and all(t is not None and type(t) in (Tensor, nn.Parameter) and t.dtype == rows.dtype and t.device == rows.device and t.shape == s
-                    and t.is_contiguous() for t, s in zip(vectors[0::2], vectors[1::2]))):
+    if not _plain(rows.device, rows.dtype, one.weight, (F_, D), two.weight, (3 * K, F_), *vectors):
         return None
     out = torch.empty((B, Nt), device=rows.device, dtype=rows.dtype)
     v = [t.data_ptr() for t in vectors[0::2]]
-    a = _lib.ArtabDensityArgs(rows.data_ptr(), rows.stride(0), v[0], v[1], norm.eps, one.weight.data_ptr(), v[2], two.weight.data_ptr(), v[3], *v[4:],
+    w1, w2 = _in_pieces(one.weight, two.weight)  # (held until the launch)
+    a = _lib.ArtabDensityArgs(rows.data_ptr(), rows.stride(0), v[0], v[1], norm.eps, w1.data_ptr(), v[2], w2.data_ptr(), v[3], *v[4:],
                               K, head.std_min, y.data_ptr(), *y.stride(), out.data_ptr(), B, Nt, D, F_)
     _lib.check(lib.artab_density(ctypes.byref(a), _lib.dtype_code(rows.dtype), _lib.current_stream(rows.device)))
     return out
