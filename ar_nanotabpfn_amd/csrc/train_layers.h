@@ -680,6 +680,16 @@ struct TrainFinal {
     int B, R, first;
 };
 
+// Sum over the wavefront without the LDS: a row's four sums one after the other, 19 rows to a wavefront, were most of the
+// backward kernel's time (38912 rows of 128: 24.3 us, 16.8 with this).
+__device__ __forceinline__ float train_wave_sum(float x) {
+    x += row_rotate<8>(x);
+    x += row_rotate<4>(x);
+    x += row_rotate<2>(x);
+    x += row_rotate<1>(x);
+    return row_sum(x);
+}
+
 // one wavefront per row; lane l holds elements l D/64 ..
 template <int D, bool BACKWARD>
 __global__ __launch_bounds__(256) void train_final_kernel(TrainFinal P) {
@@ -713,11 +723,11 @@ __global__ __launch_bounds__(256) void train_final_kernel(TrainFinal P) {
             x[e] = fmaf((P.r3[m * D + lane * E + e] - st.x) * st.y, g3[e], b3[e]);
             s += x[e];
         }
-        const float mean = wave_sum(s) * (1.f / D);
+        const float mean = train_wave_sum(s) * (1.f / D);
         float q = 0.f;
 #pragma unroll
         for (int e = 0; e < E; ++e) q = fmaf(x[e] - mean, x[e] - mean, q);
-        const float rstd = rsqrtf(wave_sum(q) * (1.f / D) + P.eps);
+        const float rstd = rsqrtf(train_wave_sum(q) * (1.f / D) + P.eps);
         const long zi = (b * (P.R - P.first) + (at - P.first)) * D + lane * E;
         if (!BACKWARD) {
 #pragma unroll
@@ -734,7 +744,7 @@ __global__ __launch_bounds__(256) void train_final_kernel(TrainFinal P) {
                 s1 += gy[e];
                 s2 = fmaf(gy[e], xh[e], s2);
             }
-            const float m1 = wave_sum(s1) * (1.f / D), m2 = wave_sum(s2) * (1.f / D);
+            const float m1 = train_wave_sum(s1) * (1.f / D), m2 = train_wave_sum(s2) * (1.f / D);
 #pragma unroll
             for (int e = 0; e < E; ++e) P.dx[m * D + lane * E + e] = rstd * (gy[e] - m1 - xh[e] * m2);
         }
@@ -753,25 +763,35 @@ __global__ __launch_bounds__(256) void train_final_kernel(TrainFinal P) {
 
 // ---- weight gradients: C[n][k] = sum_m P[m][n] Q[m][k] in pieces of 128 x 128, each over `slices` runs of
 // rows.  Both operands want the contraction (rows) consecutive in a lane: transposing reads of row-major LDS
-// tiles.  Eight wavefronts: two groups take half of a tile's 64 rows each, a group's four hold 64 x 64.
+// tiles.  Sixteen wavefronts: four groups take a quarter of a tile's 128 rows each, a group's four hold 64 x 64.
+//
+// Bound: the trip to memory.  A workgroup waits for one tile while it has multiplied the one before, one workgroup to
+// a compute unit (one launch fills the chip once, or its partial sums would be as many bytes as its operands), so the
+// bytes per unit and trip are what counts: tiles of 64 rows, eight wavefronts, took 40 us for the nine pieces of 38912
+// rows of 128 (140 MB), this 29.3.  Pieces of one slice read the same rows: they run on one XCD, whose L2 then has them.
 struct TrainGradJobs {
     const bf16_t *p[kTrainMaxJobs], *q[kTrainMaxJobs];
     int ldp[kTrainMaxJobs], ldq[kTrainMaxJobs];
     float *part;               // [slices][jobs][128 * 128]
-    long M, rows_per_slice;    // a multiple of 64
-    int jobs;
+    long M, rows_per_slice;    // a multiple of kTrainGradRows
+    int jobs, slices;
 };
+constexpr int kTrainGradRows = 128;
+// Workgroups are dealt round-robin over the eight XCDs: pieces in a row, slice after slice, to each of them.
+__host__ __device__ constexpr int train_grad_blocks(int jobs, int slices) { return (jobs * slices + 7) / 8 * 8; }
 
-static __global__ __launch_bounds__(512) void train_weight_grad_kernel(TrainGradJobs J) {
+static __global__ __launch_bounds__(1024) void train_weight_grad_kernel(TrainGradJobs J) {
     typedef MfmaOps<bf16_t> Ops;
-    constexpr int TR = 64, LD = 128 + 16;  // 288 bytes: 32 mod 128, what the transposing reads want
+    constexpr int TR = kTrainGradRows, LD = 128 + 16;  // 288 bytes: 32 mod 128, what the transposing reads want
     __shared__ __attribute__((aligned(16))) bf16_t lds[2][2][TR * LD];
-    const int job = blockIdx.x, slice = blockIdx.y;
+    const int piece = static_cast<int>((blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3));
+    if (piece >= J.jobs * J.slices) return;
+    const int job = piece % J.jobs, slice = piece / J.jobs;
     const bf16_t *const p = J.p[job], *const q = J.q[job];
     const int ldp = J.ldp[job], ldq = J.ldq[job];
     const long m0 = slice * J.rows_per_slice, m1 = min(J.M, m0 + J.rows_per_slice);
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-    const int half = wave >> 2, wn = wave & 1, wk = (wave >> 1) & 1;
+    const int group = wave >> 2, wn = wave & 1, wk = (wave >> 1) & 1;
     f32x16 acc[2][2];
 #pragma unroll
     for (int a = 0; a < 2; ++a)
@@ -783,7 +803,7 @@ static __global__ __launch_bounds__(512) void train_weight_grad_kernel(TrainGrad
     auto fetch = [&](long m) {
 #pragma unroll
         for (int x = 0; x < 2; ++x) {
-            const int i = tid + 512 * x, r = i / 16, c = i % 16;
+            const int i = tid + 1024 * x, r = i / 16, c = i % 16;
             const long row = min(m + r, J.M - 1);
             rp[x] = *reinterpret_cast<const u32x4 *>(p + row * ldp + 8 * c);
             rq[x] = *reinterpret_cast<const u32x4 *>(q + row * ldq + 8 * c);
@@ -792,7 +812,7 @@ static __global__ __launch_bounds__(512) void train_weight_grad_kernel(TrainGrad
     auto put = [&](int buf, long m) {
 #pragma unroll
         for (int x = 0; x < 2; ++x) {
-            const int i = tid + 512 * x, r = i / 16, c = i % 16;
+            const int i = tid + 1024 * x, r = i / 16, c = i % 16;
             const u32x4 zero = {0u, 0u, 0u, 0u};
             *reinterpret_cast<u32x4 *>(&lds[buf][0][r * LD + 8 * c]) = m + r < m1 ? rp[x] : zero;  // rows past the end: no product
             *reinterpret_cast<u32x4 *>(&lds[buf][1][r * LD + 8 * c]) = rq[x];
@@ -820,8 +840,8 @@ static __global__ __launch_bounds__(512) void train_weight_grad_kernel(TrainGrad
                 bf16x8 a[2], c[2];
 #pragma unroll
                 for (int i = 0; i < 2; ++i) {
-                    a[i] = operand(lds[buf][0], 32 * half + 16 * ks, 64 * wn + 32 * i);
-                    c[i] = operand(lds[buf][1], 32 * half + 16 * ks, 64 * wk + 32 * i);
+                    a[i] = operand(lds[buf][0], 32 * group + 16 * ks, 64 * wn + 32 * i);
+                    c[i] = operand(lds[buf][1], 32 * group + 16 * ks, 64 * wk + 32 * i);
                 }
 #pragma unroll
                 for (int i = 0; i < 2; ++i)
@@ -831,41 +851,47 @@ static __global__ __launch_bounds__(512) void train_weight_grad_kernel(TrainGrad
             if (more) put(buf ^ 1, m + TR);  // the other buffer's readers passed the barrier above
         }
     }
-    // the second group's sums through LDS (64 x 64 floats per wavefront pair would fill it: one quarter at a time)
-    float *const x = reinterpret_cast<float *>(lds);
-    float *const out = J.part + (static_cast<long>(slice) * J.jobs + job) * (128 * 128);
+    // the groups' sums through LDS, a 32 x 32 block of every wavefront at a time, added up by one group each; two areas in turn
+    float *const out = J.part + static_cast<long>(piece) * (128 * 128);
     const int c32 = lane & 31, hb = lane >> 5;
+    constexpr int AREA = 16 * 1024;  // floats: 16 of a lane, 16 wavefronts
+    static_assert(2 * AREA * sizeof(float) <= sizeof(lds), "two areas");
+    __syncthreads();
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int round = 0; round < 4; ++round) {
+        constexpr int kQuarter = AREA / 4;
+        const int i = round >> 1, j = round & 1;
+        float *const x = reinterpret_cast<float *>(lds) + (round & 1) * AREA;
+        if (group != round) {
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            __syncthreads();
-            if (half == 1) {
+            for (int v = 0; v < 16; ++v) x[group * kQuarter + (wave & 3) * 1024 + v * 64 + lane] = acc[i][j][v];
+        }
+        __syncthreads();
+        if (group == round) {
 #pragma unroll
-                for (int v = 0; v < 16; ++v) x[(wave & 3) * 1024 + v * 64 + lane] = acc[i][j][v];
-            }
-            __syncthreads();
-            if (half == 0) {
+            for (int v = 0; v < 16; ++v) {
+                const int n = 64 * wn + 32 * i + 8 * (v >> 2) + 4 * hb + (v & 3), k = 64 * wk + 32 * j + c32;
+                float sum = acc[i][j][v];
 #pragma unroll
-                for (int v = 0; v < 16; ++v) {
-                    const int n = 64 * wn + 32 * i + 8 * (v >> 2) + 4 * hb + (v & 3), k = 64 * wk + 32 * j + c32;
-                    out[n * 128 + k] = acc[i][j][v] + x[(wave & 3) * 1024 + v * 64 + lane];
-                }
+                for (int other = 1; other < 4; ++other) sum += x[((round + other) & 3) * kQuarter + (wave & 3) * 1024 + v * 64 + lane];
+                out[n * 128 + k] = sum;
             }
         }
+    }
 }
 
-// A step's reduction is 12 us with eight rows of column sums on their way, 7.7 with 32.
-//
 // Adds up the slices of the weight gradients (where each piece goes: `out`, row stride `ld`) and the workgroups'
-// column sums.
+// column sums.  Bound: trips to memory one after the other, so a thread has all it adds up on its way at once, up to 32
+// slices; a column's rows (some 700) are dealt over 16 threads, the columns over as many workgroups.  A step's reduction of
+// 28 slices of nine pieces: 7.7 us with 64 columns to a workgroup and 16 slices on their way, 6.2 with these.
+constexpr int kTrainReduceCols = 16;
 struct TrainReduce {
     const float *part; int jobs, slices;
     float *out[kTrainMaxJobs]; int ld[kTrainMaxJobs];
     struct Cols {
         const float *part;     // [groups][ld], n columns of it
         float *out;
-        int groups, ld, n;
+        int groups, ld, n;     // n: a multiple of kTrainReduceCols
     } cols[2];
     int n_cols;
 };
@@ -874,42 +900,53 @@ static __global__ __launch_bounds__(256) void train_reduce_kernel(TrainReduce P)
     const int piece_groups = P.jobs * 16;  // 16 workgroups of 1024 elements per piece
     if (static_cast<int>(blockIdx.x) < piece_groups) {
         const int job = blockIdx.x / 16, e = (blockIdx.x % 16) * 1024 + 4 * tid;
+        const long step = static_cast<long>(P.jobs) * 16384;
+        const float *const from = P.part + static_cast<long>(job) * 16384 + e;
+        constexpr int AHEAD = 32;
         f32x4 s = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 16
-        for (int i = 0; i < P.slices; ++i) s += *reinterpret_cast<const f32x4 *>(P.part + (static_cast<long>(i) * P.jobs + job) * 16384 + e);
+        for (int i = 0; i < P.slices; i += AHEAD) {
+            f32x4 v[AHEAD];
+#pragma unroll
+            for (int u = 0; u < AHEAD; ++u) v[u] = *reinterpret_cast<const f32x4 *>(from + min(i + u, P.slices - 1) * step);
+#pragma unroll
+            for (int u = 0; u < AHEAD; ++u) s += i + u < P.slices ? v[u] : f32x4{0.f, 0.f, 0.f, 0.f};
+        }
         *reinterpret_cast<f32x4 *>(P.out[job] + static_cast<long>(e / 128) * P.ld[job] + e % 128) = s;
         return;
     }
-    // 64 columns per workgroup, four wavefronts deal the rows
-    __shared__ float acc[4][64];
-    int at = (static_cast<int>(blockIdx.x) - piece_groups) * 64;
+    __shared__ float acc[256];
+    int at = (static_cast<int>(blockIdx.x) - piece_groups) * kTrainReduceCols;
     int which = 0;
     while (which + 1 < P.n_cols && at >= P.cols[which].n) {
         at -= P.cols[which].n;
         ++which;
     }
     const TrainReduce::Cols C = P.cols[which];
-    const int wave = tid >> 6, lane = tid & 63;
-    constexpr int AHEAD = 32;  // rows on their way at a time: a few workgroups walk some hundred rows each
+    constexpr int SIDE = 256 / kTrainReduceCols, AHEAD = 32;
+    const int c = tid % kTrainReduceCols, side = tid / kTrainReduceCols;
     float part[AHEAD];
 #pragma unroll
     for (int u = 0; u < AHEAD; ++u) part[u] = 0.f;
-    const float *col = C.part + at + lane;
-    for (int i = wave; i < C.groups; i += 4 * AHEAD) {
+    const float *col = C.part + at + c;
+    for (int i = side; i < C.groups; i += SIDE * AHEAD) {
         float v[AHEAD];
 #pragma unroll
-        for (int u = 0; u < AHEAD; ++u) v[u] = col[static_cast<long>(min(i + 4 * u, C.groups - 1)) * C.ld];
+        for (int u = 0; u < AHEAD; ++u) v[u] = col[static_cast<long>(min(i + SIDE * u, C.groups - 1)) * C.ld];
 #pragma unroll
-        for (int u = 0; u < AHEAD; ++u) part[u] += i + 4 * u < C.groups ? v[u] : 0.f;
+        for (int u = 0; u < AHEAD; ++u) part[u] += i + SIDE * u < C.groups ? v[u] : 0.f;
     }
 #pragma unroll
     for (int half = AHEAD / 2; half > 0; half /= 2)
 #pragma unroll
         for (int u = 0; u < half; ++u) part[u] += part[u + half];
-    const float s = part[0];
-    acc[wave][lane] = s;
+    acc[tid] = part[0];
     __syncthreads();
-    if (wave == 0) C.out[at + lane] = (acc[0][lane] + acc[1][lane]) + (acc[2][lane] + acc[3][lane]);
+    if (tid < kTrainReduceCols) {
+        float s = 0.f;
+#pragma unroll
+        for (int i = 0; i < SIDE; ++i) s += acc[i * kTrainReduceCols + tid];
+        C.out[at + tid] = s;
+    }
 }
 
 // ---- row embeddings (model.py:23-76, :323-333): x = mean(features) w_x + b_x + marker, context and buffer rows
