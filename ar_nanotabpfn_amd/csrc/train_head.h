@@ -113,8 +113,8 @@ __global__ __launch_bounds__(kTrainWaves * 64, 3) void train_head_kernel(TrainHe
         }
         __syncthreads();
         if constexpr (BACKWARD) {
-            train_unstage<D>(P.zb, D, zs, LD, L.row0, P.M);
-            train_unstage<F>(P.h, F, hs, LF, L.row0, P.M);
+            train_unstage<D>(P.zb, zs, LD, L);
+            train_unstage<F>(P.h, hs, LF, L);
         }
         {
             f32x4 raw[NR][2];
@@ -195,7 +195,7 @@ __global__ __launch_bounds__(kTrainWaves * 64, 3) void train_head_kernel(TrainHe
                 for (int row = 0; row < kTrainRows; ++row) s += raw_s[row * LR + threadIdx.x];
                 sums[F + threadIdx.x] += s;
             }
-            train_unstage<kHeadCols>(P.draw, kHeadCols, gs, LG, L.row0, P.M);
+            train_unstage<kHeadCols>(P.draw, gs, LG, L);
             f32x4 d[NF][2];
             train_product<NF, NP / 32>(d, gs, LG, w2t, 0, L);
 #pragma unroll
@@ -206,7 +206,7 @@ __global__ __launch_bounds__(kTrainWaves * 64, 3) void train_head_kernel(TrainHe
             }
             train_to_lds(hs, LF, d, L);
             __syncthreads();
-            train_unstage<F>(P.du, F, hs, LF, L.row0, P.M);
+            train_unstage<F>(P.du, hs, LF, L);
             f32x4 dz[NB][2];
             train_product<NB, F / 32>(dz, hs, LF, w1t, 0, L);
             train_store<D>(P.dz, dz, L);

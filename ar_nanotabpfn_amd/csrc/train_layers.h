@@ -21,10 +21,10 @@
 // workgroups, so that the loads of one run under the products of others: four to a compute unit forward, three backward
 // at d_model 128; three and two at 256.
 //
-// 38912 rows of 128: forward 51 us a layer (as two kernels, with r3 written and read back between them, 56; its bytes
-// at the rate of a copy 25), backward 74 us (two kernels 107; 50).  The rest is the weights, 295 and 360 KB a tile from
-// L2, and that the few tiles of a compute unit (4.75) load, multiply and store nearly in step.  Measured and not kept
-// (forward): weights requested ahead of the barriers (50), five workgroups to a compute unit (53, spills).
+// 38912 rows of 128: forward 45 us a layer (its bytes at the rate of a copy 25), backward 72 us (50).  The rest is the
+// weights, 295 and 360 KB a tile from L2 (with one cached fragment for all of them 32 and 59 us), and that the few tiles
+// of a compute unit (4.75) load, multiply and store nearly in step; with neither stores nor memory behind the loads 19 and
+// 34.  Measured and not kept (forward): five workgroups to a compute unit (spills).
 #pragma once
 
 #include "common.h"
@@ -173,18 +173,38 @@ __device__ __forceinline__ const bf16_t *train_opaque(const bf16_t *p) {
     return p;
 }
 
+// Global memory at a wavefront-uniform address and a lane's 32-bit byte offset, in global memory's own address space: a
+// pointer the compiler cannot trace would be a generic one, whose loads count as LDS accesses too, and every wait for an
+// activation in LDS would wait for the weights behind it; and the addition is the load's own, not two vector instructions
+// in front of it.
+template <typename V>
+__device__ __forceinline__ V train_get(const void *base, unsigned byte) {
+    typedef const __attribute__((address_space(1))) char *Global;
+    return *(const __attribute__((address_space(1))) V *)((Global)base + byte);
+}
+template <typename V>
+__device__ __forceinline__ void train_put(void *base, unsigned byte, const V &v) {
+    typedef __attribute__((address_space(1))) char *Global;
+    *(__attribute__((address_space(1))) V *)((Global)base + byte) = v;
+}
+
+typedef float TrainStat __attribute__((ext_vector_type(2)));  // (mean, 1/std) of a row
+
 struct TrainLane {
     int wave, lane, tok, quad;
-    long row0, M;
-    __device__ __forceinline__ TrainLane(long tile, long M_) : M(M_) {
+    long row0;
+    int last;  // of the tile's rows
+    __device__ __forceinline__ TrainLane(long tile, long M) {
         wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
         lane = opaque(threadIdx.x & 63);
         tok = lane & 15;
         quad = lane >> 4;
         row0 = tile * kTrainRows;
+        last = static_cast<int>(min(static_cast<long>(kTrainRows), M - row0)) - 1;
     }
-    __device__ __forceinline__ long row(int tb) const { return min(row0 + 16 * tb + tok, M - 1); }
-    __device__ __forceinline__ bool live(int tb) const { return row0 + 16 * tb + tok < M; }
+    // of token half tb: its row in the tile (past the end the last one again) and whether it is one
+    __device__ __forceinline__ int in(int tb) const { return min(16 * tb + tok, last); }
+    __device__ __forceinline__ bool live(int tb) const { return 16 * tb + tok <= last; }
     __device__ __forceinline__ int col(int b) const { return 16 * (wave + kTrainWaves * b) + 4 * quad; }
 };
 
@@ -193,7 +213,7 @@ __device__ __forceinline__ void train_load(f32x4 (&v)[NB][2], const float *src, 
 #pragma unroll
     for (int tb = 0; tb < 2; ++tb)
 #pragma unroll
-        for (int b = 0; b < NB; ++b) v[b][tb] = *reinterpret_cast<const f32x4 *>(src + L.row(tb) * D + L.col(b));
+        for (int b = 0; b < NB; ++b) v[b][tb] = train_get<f32x4>(src + L.row0 * D, 4u * (L.in(tb) * D + L.col(b)));
 }
 template <int D, int NB>
 __device__ __forceinline__ void train_store(float *dst, const f32x4 (&v)[NB][2], const TrainLane &L) {
@@ -201,18 +221,30 @@ __device__ __forceinline__ void train_store(float *dst, const f32x4 (&v)[NB][2],
     for (int tb = 0; tb < 2; ++tb)
         if (L.live(tb)) {
 #pragma unroll
-            for (int b = 0; b < NB; ++b) *reinterpret_cast<f32x4 *>(dst + L.row(tb) * D + L.col(b)) = v[b][tb];
+            for (int b = 0; b < NB; ++b) train_put(dst + L.row0 * D, 4u * (L.in(tb) * D + L.col(b)), v[b][tb]);
         }
 }
+// Values rounded for a store later on.
 template <int NB>
-__device__ __forceinline__ void train_store16(bf16_t *dst, long ld, int col0, const f32x4 (&v)[NB][2], const TrainLane &L) {
+struct TrainPacked {
+    u32x2 v[NB][2];
+    __device__ __forceinline__ explicit TrainPacked(const f32x4 (&x)[NB][2]) {
 #pragma unroll
-    for (int tb = 0; tb < 2; ++tb)
-        if (L.live(tb)) {
+        for (int b = 0; b < NB; ++b)
 #pragma unroll
-            for (int b = 0; b < NB; ++b) store4f<bf16_t>(dst + L.row(tb) * ld + col0 + L.col(b), v[b][tb][0], v[b][tb][1], v[b][tb][2], v[b][tb][3]);
-        }
-}
+            for (int tb = 0; tb < 2; ++tb) v[b][tb] = u32x2{pack2<bf16_t>(x[b][tb][0], x[b][tb][1]), pack2<bf16_t>(x[b][tb][2], x[b][tb][3])};
+    }
+    // (row stride LDG)
+    template <int LDG>
+    __device__ __forceinline__ void store(bf16_t *dst, int col0, const TrainLane &L) const {
+#pragma unroll
+        for (int tb = 0; tb < 2; ++tb)
+            if (L.live(tb)) {
+#pragma unroll
+                for (int b = 0; b < NB; ++b) train_put(dst + L.row0 * LDG + col0, 2u * (L.in(tb) * LDG + L.col(b)), v[b][tb]);
+            }
+    }
+};
 template <int NB>
 __device__ __forceinline__ void train_to_lds(bf16_t *tile, int ld, const f32x4 (&v)[NB][2], const TrainLane &L) {
 #pragma unroll
@@ -221,59 +253,97 @@ __device__ __forceinline__ void train_to_lds(bf16_t *tile, int ld, const f32x4 (
         for (int b = 0; b < NB; ++b)
             store4f<bf16_t>(tile + (16 * tb + L.tok) * ld + L.col(b), v[b][tb][0], v[b][tb][1], v[b][tb][2], v[b][tb][3]);
 }
-// [32, W] bf16 between global memory (row stride ld) and an LDS tile (row stride lds_ld), 16 bytes a lane
+// [32, W] bf16 between global memory (row stride W) and an LDS tile (row stride lds_ld), 16 bytes a lane
 template <int W>
-__device__ __forceinline__ void train_stage(bf16_t *tile, int lds_ld, const bf16_t *src, long ld, long row0, long M) {
+__device__ __forceinline__ void train_stage(bf16_t *tile, int lds_ld, const bf16_t *src, const TrainLane &L) {
     constexpr int CPR = W / 8;
     static_assert(kTrainRows * CPR % (kTrainWaves * 64) == 0, "whole passes");
     const int tid = opaque(threadIdx.x);
 #pragma unroll
     for (int x = 0; x < kTrainRows * CPR / (kTrainWaves * 64); ++x) {
         const int i = tid + kTrainWaves * 64 * x, r = i / CPR, c = i % CPR;
-        *reinterpret_cast<u32x4 *>(tile + r * lds_ld + 8 * c) = *reinterpret_cast<const u32x4 *>(src + min(row0 + r, M - 1) * ld + 8 * c);
+        *reinterpret_cast<u32x4 *>(tile + r * lds_ld + 8 * c) = train_get<u32x4>(src + L.row0 * W, 2u * (min(r, L.last) * W + 8 * c));
     }
 }
 template <int W>
-__device__ __forceinline__ void train_unstage(bf16_t *dst, long ld, const bf16_t *tile, int lds_ld, long row0, long M) {
+__device__ __forceinline__ void train_unstage(bf16_t *dst, const bf16_t *tile, int lds_ld, const TrainLane &L) {
     constexpr int CPR = W / 8;
     static_assert(kTrainRows * CPR % (kTrainWaves * 64) == 0, "whole passes");
     const int tid = opaque(threadIdx.x);
 #pragma unroll
     for (int x = 0; x < kTrainRows * CPR / (kTrainWaves * 64); ++x) {
         const int i = tid + kTrainWaves * 64 * x, r = i / CPR, c = i % CPR;
-        if (row0 + r < M) *reinterpret_cast<u32x4 *>(dst + (row0 + r) * ld + 8 * c) = *reinterpret_cast<const u32x4 *>(tile + r * lds_ld + 8 * c);
+        if (r <= L.last) train_put(dst + L.row0 * W, 2u * (r * W + 8 * c), *reinterpret_cast<const u32x4 *>(tile + r * lds_ld + 8 * c));
     }
 }
 
-// acc[b][tb] = sum_k W[16 (nb0 + wave + 4 b) ..][k] A[16 tb + tok][k]; a few contraction steps of the
-// weights are on their way ahead of the one being multiplied
-template <int NB, int KS>
-__device__ __forceinline__ void train_product(f32x4 (&acc)[NB][2], const bf16_t *tile, int ld, const bf16_t *w, int nb0, const TrainLane &L) {
-    typedef MfmaOps<bf16_t> Ops;
-    constexpr int PF = NB <= 2 ? (KS < 4 ? KS : 4) : 2;
-    const char *const base = reinterpret_cast<const char *>(w) + (static_cast<long>(nb0 + L.wave) * KS) * 1024 + 16 * L.lane;
-    auto frag = [&](int b, int ks) { return *reinterpret_cast<const u32x4 *>(base + (static_cast<long>(kTrainWaves) * b * KS + ks) * 1024); };
-    u32x4 ring[PF][NB];
+// acc[b][tb] = sum_k W[16 (nb0 + wave + 4 b) ..][k] A[16 tb + tok][k].  A ring of eight weight fragments is on its way ahead of
+// the one being multiplied; begin() requests the first.
+//
+// Order of requests.  A wavefront's loads and stores are counted together and in order: a wait for a load is a wait for
+// every store in front of it, and their way to memory is longer than a product.  So the next product's first fragments, and
+// the tensors it needs, are asked for before the results of the one behind are stored, and the parameter vectors lie in
+// LDS.  38912 rows of 128, stores in front of the requests / behind them: forward 50.8 / 44.8 us, the last layer's
+// backward 50.7 / 47.2, the others' 73.2 / 71.8 (without any stores 35.1, 32.4 and 50.8).
+struct TrainRing {
+    u32x4 f[8];
+    template <int NB, int KS>
+    static constexpr int ahead() { return 8 / NB < KS ? 8 / NB : KS; }  // contraction steps in the ring
+    static __device__ __forceinline__ u32x4 get(const bf16_t *w, int nb0, int b, int ks, int steps, const TrainLane &L) {
+        return train_get<u32x4>(reinterpret_cast<const char *>(w) + ((nb0 + L.wave + kTrainWaves * b) * static_cast<long>(steps) + ks) * 1024,
+                                16u * L.lane);
+    }
+    template <int NB, int KS>
+    __device__ __forceinline__ void begin(const bf16_t *w, int nb0, const TrainLane &L) {
 #pragma unroll
-    for (int p = 0; p < PF; ++p)
+        for (int p = 0; p < ahead<NB, KS>(); ++p)
 #pragma unroll
-        for (int b = 0; b < NB; ++b) ring[p][b] = frag(b, p);
+            for (int b = 0; b < NB; ++b) f[p * NB + b] = get(w, nb0, b, p, KS, L);
+    }
+    template <int NB, int KS>
+    __device__ __forceinline__ void run(f32x4 (&acc)[NB][2], const bf16_t *tile, int ld, const bf16_t *w, int nb0, const TrainLane &L) {
+        typedef MfmaOps<bf16_t> Ops;
+        constexpr int PF = ahead<NB, KS>();
 #pragma unroll
-    for (int b = 0; b < NB; ++b)
+        for (int b = 0; b < NB; ++b)
 #pragma unroll
-        for (int tb = 0; tb < 2; ++tb) acc[b][tb] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const bf16_t *const a = tile + L.tok * ld + 8 * L.quad;
+            for (int tb = 0; tb < 2; ++tb) acc[b][tb] = f32x4{0.f, 0.f, 0.f, 0.f};
+        const bf16_t *const a = tile + L.tok * ld + 8 * L.quad;
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-        const bf16x8 a0 = *reinterpret_cast<const bf16x8 *>(a + 32 * ks), a1 = *reinterpret_cast<const bf16x8 *>(a + 16 * ld + 32 * ks);
+        for (int ks = 0; ks < KS; ++ks) {
+            const bf16x8 a0 = *reinterpret_cast<const bf16x8 *>(a + 32 * ks), a1 = *reinterpret_cast<const bf16x8 *>(a + 16 * ld + 32 * ks);
 #pragma unroll
-        for (int b = 0; b < NB; ++b) {
-            const bf16x8 wv = __builtin_bit_cast(bf16x8, ring[ks % PF][b]);
-            acc[b][0] = Ops::mma16(wv, a0, acc[b][0]);
-            acc[b][1] = Ops::mma16(wv, a1, acc[b][1]);
-            if (ks + PF < KS) ring[ks % PF][b] = frag(b, ks + PF);
+            for (int b = 0; b < NB; ++b) {
+                u32x4 &slot = f[ks % PF * NB + b];
+                const bf16x8 wv = __builtin_bit_cast(bf16x8, slot);
+                acc[b][0] = Ops::mma16(wv, a0, acc[b][0]);
+                acc[b][1] = Ops::mma16(wv, a1, acc[b][1]);
+                if (ks + PF < KS) slot = get(w, nb0, b, ks + PF, KS, L);
+            }
         }
     }
+};
+template <int NB, int KS>
+__device__ __forceinline__ void train_product(f32x4 (&acc)[NB][2], const bf16_t *tile, int ld, const bf16_t *w, int nb0, const TrainLane &L) {
+    TrainRing ring;
+    ring.begin<NB, KS>(w, nb0, L);
+    ring.run<NB, KS>(acc, tile, ld, w, nb0, L);
+}
+
+// A parameter vector: in LDS where a kernel keeps it there, else in memory.  N floats by the lanes of one wavefront.
+template <bool LDS>
+struct TrainVector {
+    const float *p;
+    __device__ __forceinline__ f32x4 at(int col) const {
+        if constexpr (LDS) return *reinterpret_cast<const f32x4 *>(p + col);
+        else return train_get<f32x4>(p, 4u * col);
+    }
+};
+template <int N>
+__device__ __forceinline__ void train_keep(float *lds, const float *src, int wave) {
+    static_assert(N <= 256 && N % 4 == 0, "one request of a wavefront");
+    const int i = 4 * static_cast<int>(threadIdx.x & 63);
+    if (static_cast<int>(threadIdx.x >> 6) == wave && i < N) *reinterpret_cast<f32x4 *>(lds + i) = train_get<f32x4>(src, 4u * i);
 }
 
 // Sums of two per-row values over all features: lanes, then wavefronts.  red: [4][32] float2.
@@ -334,19 +404,23 @@ __device__ __forceinline__ void train_stats(const f32x4 (&v)[NB][2], float2 *red
             m2 += fmaf(kLocal * d, d, p[w].y);
         }
         st[tb] = make_float2(mean, rsqrtf(m2 / D + eps));
-        if (L.wave == 0 && L.quad == 0 && L.live(tb)) stats[L.row(tb)] = st[tb];
+        if (L.wave == 0 && L.quad == 0 && L.live(tb)) train_put(stats + L.row0, 8u * L.in(tb), TrainStat{st[tb].x, st[tb].y});
     }
 }
 __device__ __forceinline__ void train_get_stats(float2 (&st)[2], const float2 *stats, const TrainLane &L) {
 #pragma unroll
-    for (int tb = 0; tb < 2; ++tb) st[tb] = stats[L.row(tb)];
+    for (int tb = 0; tb < 2; ++tb) {
+        const TrainStat v = train_get<TrainStat>(stats + L.row0, 8u * L.in(tb));
+        st[tb] = make_float2(v[0], v[1]);
+    }
 }
 // x = (r - mean) / std * g + b
-template <int NB>
-__device__ __forceinline__ void train_norm(f32x4 (&x)[NB][2], const f32x4 (&r)[NB][2], const float2 (&st)[2], const float *g, const float *be, const TrainLane &L) {
+template <int NB, bool LDS>
+__device__ __forceinline__ void train_norm(f32x4 (&x)[NB][2], const f32x4 (&r)[NB][2], const float2 (&st)[2], const TrainVector<LDS> &g, const TrainVector<LDS> &be,
+                                           const TrainLane &L) {
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
-        const f32x4 gv = *reinterpret_cast<const f32x4 *>(g + L.col(b)), bv = *reinterpret_cast<const f32x4 *>(be + L.col(b));
+        const f32x4 gv = g.at(L.col(b)), bv = be.at(L.col(b));
 #pragma unroll
         for (int tb = 0; tb < 2; ++tb)
 #pragma unroll
@@ -392,35 +466,55 @@ struct TrainForward {
 };
 
 template <int D, int F, bool BACK, bool FRONT>
-__global__ __launch_bounds__(kTrainWaves * 64) void train_forward_kernel(TrainForward P) {
+__global__ __launch_bounds__(kTrainWaves * 64, D == 128 ? 4 : 3) void train_forward_kernel(TrainForward P) {
     constexpr int NB = D / 64, NF = F / 64, LD = D + 8, LF = F + 8;
     __shared__ __attribute__((aligned(16))) bf16_t as[kTrainRows * (LD > LF || !BACK ? LD : LF)], ys[kTrainRows * LD];
     __shared__ float2 red[kTrainWaves * kTrainRows];
+    __shared__ __attribute__((aligned(16))) float vecs[(BACK ? 5 * D + F : 0) + (FRONT ? 2 * D : 0)];
+    float *const vec1 = vecs + (BACK ? 5 * D + F : 0);  // of the next layer's norm
+    typedef TrainVector<true> Kept;
     const TrainLane L(blockIdx.x, P.M);
+    TrainRing ring;
     f32x4 x[NB][2], acc[NB][2];
     float2 st[2];
+    const bf16_t *const w_o = P.packed + train_matrix_at<D, F>(kTmO), *const w_1 = P.packed + train_matrix_at<D, F>(kTm1),
+                 *const w_2 = P.packed + train_matrix_at<D, F>(kTm2), *const w_fo = P.next_packed + train_matrix_at<D, F>(kTmFo),
+                 *const w_qkv = P.next_packed + train_matrix_at<D, F>(kTmQkv);
     if constexpr (BACK) {
-        train_stage<D>(as, LD, P.attn, D, L.row0, P.M);
+        ring.begin<NB, D / 32>(w_o, 0, L);
+        train_stage<D>(as, LD, P.attn, L);
         train_load<D>(x, P.r1, L);
         train_get_stats(st, P.stats1, L);
-        train_norm(x, x, st, P.g1, P.b1, L);
+        train_keep<D>(vecs, P.g2, 0);
+        train_keep<D>(vecs + D, P.b2, 1);
+        train_keep<D>(vecs + 2 * D, P.bias2, 2);
+        train_keep<F>(vecs + 5 * D, P.bias1, 3);
+        if constexpr (FRONT) {
+            train_keep<D>(vecs + 3 * D, P.g3, 0);
+            train_keep<D>(vecs + 4 * D, P.b3, 1);
+            train_keep<D>(vec1, P.next_g1, 2);
+            train_keep<D>(vec1 + D, P.next_b1, 3);
+        }
+        train_norm(x, x, st, TrainVector<false>{P.g1}, TrainVector<false>{P.b1}, L);
         __syncthreads();
-        train_product<NB, D / 32>(acc, as, LD, P.packed + train_matrix_at<D, F>(kTmO), 0, L);
+        ring.run<NB, D / 32>(acc, as, LD, w_o, 0, L);
 #pragma unroll
         for (int b = 0; b < NB; ++b)
 #pragma unroll
             for (int tb = 0; tb < 2; ++tb) x[b][tb] += acc[b][tb];
+        ring.begin<NF, D / 32>(w_1, 0, L);
         train_store<D>(P.r2, x, L);
         train_stats<D>(x, red, P.eps2, P.stats2, st, L);
-        train_norm(x, x, st, P.g2, P.b2, L);
+        train_norm(x, x, st, Kept{vecs}, Kept{vecs + D}, L);
         train_to_lds(ys, LD, x, L);
         __syncthreads();
         {
             f32x4 u[NF][2];
-            train_product<NF, D / 32>(u, ys, LD, P.packed + train_matrix_at<D, F>(kTm1), 0, L);
+            ring.run<NF, D / 32>(u, ys, LD, w_1, 0, L);
+            ring.begin<NB, F / 32>(w_2, 0, L);
 #pragma unroll
             for (int b = 0; b < NF; ++b) {
-                const f32x4 bias = *reinterpret_cast<const f32x4 *>(P.bias1 + L.col(b));
+                const f32x4 bias = Kept{vecs + 5 * D}.at(L.col(b));
 #pragma unroll
                 for (int tb = 0; tb < 2; ++tb)
 #pragma unroll
@@ -433,37 +527,43 @@ __global__ __launch_bounds__(kTrainWaves * 64) void train_forward_kernel(TrainFo
             train_to_lds(as, LF, u, L);
         }
         __syncthreads();
-        train_product<NB, F / 32>(acc, as, LF, P.packed + train_matrix_at<D, F>(kTm2), 0, L);
+        ring.run<NB, F / 32>(acc, as, LF, w_2, 0, L);
+        if constexpr (FRONT) ring.begin<NB, D / 32>(w_fo, 0, L);
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
-            const f32x4 bias = *reinterpret_cast<const f32x4 *>(P.bias2 + L.col(b));
+            const f32x4 bias = Kept{vecs + 2 * D}.at(L.col(b));
 #pragma unroll
             for (int tb = 0; tb < 2; ++tb) x[b][tb] += acc[b][tb] + bias;
         }
         train_store<D>(P.r3, x, L);
         train_stats<D>(x, red, P.eps3, P.stats3, st, L);  // (its barrier: nobody reads the tiles any more)
-        if constexpr (FRONT) train_norm(x, x, st, P.g3, P.b3, L);
+        if constexpr (FRONT) train_norm(x, x, st, Kept{vecs + 3 * D}, Kept{vecs + 4 * D}, L);
     } else {
+        ring.begin<NB, D / 32>(w_fo, 0, L);
         train_load<D>(x, P.x, L);
+        train_keep<D>(vec1, P.next_g1, 2);
+        train_keep<D>(vec1 + D, P.next_b1, 3);
     }
     if constexpr (FRONT) {
         const TrainLane L(blockIdx.x, P.M);
         train_to_lds(as, LD, x, L);
         __syncthreads();
-        train_product<NB, D / 32>(acc, as, LD, P.next_packed + train_matrix_at<D, F>(kTmFo), 0, L);
+        ring.run<NB, D / 32>(acc, as, LD, w_fo, 0, L);
 #pragma unroll
         for (int b = 0; b < NB; ++b)
 #pragma unroll
             for (int tb = 0; tb < 2; ++tb) acc[b][tb] += x[b][tb];
+        ring.begin<NB, D / 32>(w_qkv, 0, L);
         train_store<D>(P.next_r1, acc, L);
         train_stats<D>(acc, red, P.next_eps1, P.next_stats1, st, L);
-        train_norm(acc, acc, st, P.next_g1, P.next_b1, L);
+        train_norm(acc, acc, st, Kept{vec1}, Kept{vec1 + D}, L);
         train_to_lds(ys, LD, acc, L);
         __syncthreads();
 #pragma unroll
         for (int part = 0; part < 3; ++part) {
-            train_product<NB, D / 32>(acc, ys, LD, P.next_packed + train_matrix_at<D, F>(kTmQkv), part * (D / 16), L);
-            train_store16(P.next_qkv, 3 * D, part * D, acc, L);
+            ring.run<NB, D / 32>(acc, ys, LD, w_qkv, part * (D / 16), L);
+            if (part < 2) ring.begin<NB, D / 32>(w_qkv, (part + 1) * (D / 16), L);
+            TrainPacked<NB>(acc).template store<3 * D>(P.next_qkv, part * D, L);
         }
     }
 }
@@ -487,13 +587,13 @@ __device__ __forceinline__ void train_col_add(float *sums, const f32x4 &s, int c
 
 // d(sum in front of a norm) from d(its output); column sums of the parameters' gradients.  Rows past the end
 // contribute nothing.  One barrier inside.
-template <int D, int NB>
-__device__ __forceinline__ void train_norm_backward(f32x4 (&d)[NB][2], const f32x4 (&r)[NB][2], const float2 (&st)[2], const float *g,
+template <int D, int NB, bool LDS>
+__device__ __forceinline__ void train_norm_backward(f32x4 (&d)[NB][2], const f32x4 (&r)[NB][2], const float2 (&st)[2], const TrainVector<LDS> &g,
                                                     float *sum_g, float *sum_b, float2 *red, const TrainLane &L) {
     TrainPair s[2] = {{0.f, 0.f}, {0.f, 0.f}};
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
-        const f32x4 gv = *reinterpret_cast<const f32x4 *>(g + L.col(b));
+        const f32x4 gv = g.at(L.col(b));
         f32x4 cg = {0.f, 0.f, 0.f, 0.f}, cb = cg;
 #pragma unroll
         for (int tb = 0; tb < 2; ++tb) {
@@ -555,78 +655,122 @@ template <int D, int F, bool FRONT, bool BACK>
 __global__ __launch_bounds__(kTrainWaves * 64, D == 128 ? 3 : 2) void train_backward_kernel(TrainBackward P) {
     constexpr int NB = D / 64, LD = D + 8, LQ = 3 * D + 8, LF = F + 8, NS = 7 * D + F;
     constexpr int kWide = FRONT && LQ > LD + LF ? LQ : LD + LF;  // d(qkv) lies where x2 and d(u) do later
+    constexpr bool kKept = D == 128;  // the parameter vectors in LDS (256: two workgroups to a compute unit leave no room)
     __shared__ __attribute__((aligned(16))) bf16_t ds[kTrainRows * LD], wide[kTrainRows * kWide];
     __shared__ float2 red[kTrainWaves * kTrainRows];
-    __shared__ __attribute__((aligned(16))) float sums[NS];
+    __shared__ __attribute__((aligned(16))) float sums[NS], vecs[kKept ? 6 * D + F : 4];
     bf16_t *const qs = wide, *const xs = wide, *const us = wide + kTrainRows * LD;
+    typedef TrainVector<kKept> Vector;
+    const Vector g1{kKept ? vecs : P.g1}, b1{kKept ? vecs + D : P.b1}, g2{kKept ? vecs + 2 * D : P.g2}, b2{kKept ? vecs + 3 * D : P.b2},
+        g3{kKept ? vecs + 4 * D : P.g3}, b3{kKept ? vecs + 5 * D : P.b3}, bias1{kKept ? vecs + 6 * D : P.bias1};
+    const bool normed = BACK || P.stats3;  // (the input of the first layer stands for itself)
+    if constexpr (kKept) {
+        if constexpr (FRONT) {
+            train_keep<D>(vecs, P.g1, 0);
+            train_keep<D>(vecs + D, P.b1, 1);
+        }
+        if constexpr (BACK) {
+            train_keep<D>(vecs + 2 * D, P.g2, 2);
+            train_keep<D>(vecs + 3 * D, P.b2, 3);
+            train_keep<F>(vecs + 6 * D, P.bias1, 0);
+        }
+        if (normed) {
+            train_keep<D>(vecs + 4 * D, P.g3, 1);
+            train_keep<D>(vecs + 5 * D, P.b3, 2);
+        }
+    }
     for (int i = threadIdx.x; i < NS; i += kTrainWaves * 64) sums[i] = 0.f;
     __syncthreads();
     const long tiles = (P.M + kTrainRows - 1) / kTrainRows;
     for (long tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
         const TrainLane L(tile, P.M);
         const bf16_t *const packed = train_opaque(P.packed), *const back_packed = train_opaque(P.back_packed);
+        const bf16_t *const w_qkv_t = packed + train_matrix_at<D, F>(kTmQkvT), *const w_fo_t = packed + train_matrix_at<D, F>(kTmFoT),
+                     *const w_1 = back_packed + train_matrix_at<D, F>(kTm1), *const w_1_t = back_packed + train_matrix_at<D, F>(kTm1T),
+                     *const w_2_t = back_packed + train_matrix_at<D, F>(kTm2T), *const w_o_t = back_packed + train_matrix_at<D, F>(kTmOT);
+        constexpr int HF = F / 2, NH = HF / 64;  // the feed-forward in two halves of its width
+        TrainRing ring;
         f32x4 d[NB][2], r[NB][2], acc[NB][2];
         float2 st[2];
         if constexpr (FRONT) {
-            train_stage<3 * D>(qs, LQ, P.dqkv, 3 * D, L.row0, P.M);
+            ring.begin<NB, 3 * D / 32>(w_qkv_t, 0, L);
+            train_stage<3 * D>(qs, LQ, P.dqkv, L);
             train_load<D>(d, P.dr2, L);
             train_load<D>(r, P.r1, L);
             train_get_stats(st, P.stats1, L);
-            train_norm(acc, r, st, P.g1, P.b1, L);
-            train_store16(P.x1, D, 0, acc, L);
             __syncthreads();
-            train_product<NB, 3 * D / 32>(acc, qs, LQ, packed + train_matrix_at<D, F>(kTmQkvT), 0, L);
+            ring.run<NB, 3 * D / 32>(acc, qs, LQ, w_qkv_t, 0, L);
+            ring.begin<NB, D / 32>(w_fo_t, 0, L);
 #pragma unroll
             for (int b = 0; b < NB; ++b)
 #pragma unroll
                 for (int tb = 0; tb < 2; ++tb) d[b][tb] += acc[b][tb];
-            train_norm_backward<D>(d, r, st, P.g1, sums + 5 * D + F, sums + 6 * D + F, red, L);
+            train_norm(acc, r, st, g1, b1, L);
+            const TrainPacked<NB> x1(acc);
+            f32x4 r3[NB][2];
+            train_load<D>(r3, P.r3, L);
+            float2 st3[2] = {};
+            if (normed) train_get_stats(st3, P.stats3, L);
+            x1.template store<D>(P.x1, 0, L);
+            train_norm_backward<D>(d, r, st, g1, sums + 5 * D + F, sums + 6 * D + F, red, L);
             train_to_lds(ds, LD, d, L);
-            train_load<D>(r, P.r3, L);
-            if (BACK || P.stats3) {
-                train_get_stats(st, P.stats3, L);
-                train_norm(acc, r, st, P.g3, P.b3, L);
-                train_store16(P.x, D, 0, acc, L);
-            } else {
-                train_store16(P.x, D, 0, r, L);
-            }
+#pragma unroll
+            for (int b = 0; b < NB; ++b)
+#pragma unroll
+                for (int tb = 0; tb < 2; ++tb) r[b][tb] = r3[b][tb];
+            st[0] = st3[0];
+            st[1] = st3[1];
             __syncthreads();
-            train_unstage<D>(P.d1, D, ds, LD, L.row0, P.M);
-            train_product<NB, D / 32>(acc, ds, LD, packed + train_matrix_at<D, F>(kTmFoT), 0, L);
+            ring.run<NB, D / 32>(acc, ds, LD, w_fo_t, 0, L);
 #pragma unroll
             for (int b = 0; b < NB; ++b)
 #pragma unroll
                 for (int tb = 0; tb < 2; ++tb) d[b][tb] += acc[b][tb];
-            if constexpr (!BACK) train_store<D>(P.dx, d, L);
         } else {
             train_load<D>(d, P.dx, L);
             train_load<D>(r, P.r3, L);
             train_get_stats(st, P.stats3, L);
         }
-        if constexpr (BACK) {
+        if constexpr (!BACK) {
+            if (normed) train_norm(r, r, st, g3, b3, L);
+            TrainPacked<NB>(r).template store<D>(P.x, 0, L);
+            train_unstage<D>(P.d1, ds, LD, L);
+            train_store<D>(P.dx, d, L);
+        } else {
             const TrainLane L(tile, P.M);
-            train_norm_backward<D>(d, r, st, P.g3, sums, sums + D, red, L);  // (its barrier: nobody reads ds or the wide tile any more)
+            ring.begin<NH, D / 32>(w_1, 0, L);
+            f32x4 r2[NB][2];
+            float2 st2[2];
+            train_load<D>(r2, P.r2, L);
+            train_get_stats(st2, P.stats2, L);
+            if constexpr (FRONT) {
+                train_norm(acc, r, st, g3, b3, L);
+                TrainPacked<NB>(acc).template store<D>(P.x, 0, L);
+                train_unstage<D>(P.d1, ds, LD, L);
+            }
+            train_norm_backward<D>(d, r, st, g3, sums, sums + D, red, L);  // (its barrier: nobody reads ds or the wide tile any more)
 #pragma unroll
             for (int b = 0; b < NB; ++b) train_col_add(sums + 2 * D, d[b][0] + d[b][1], L.col(b), L);  // (rows past the end are zero)
             train_to_lds(ds, LD, d, L);
-            train_load<D>(r, P.r2, L);
-            train_get_stats(st, P.stats2, L);
-            train_norm(acc, r, st, P.g2, P.b2, L);
+#pragma unroll
+            for (int b = 0; b < NB; ++b)
+#pragma unroll
+                for (int tb = 0; tb < 2; ++tb) r[b][tb] = r2[b][tb];
+            st[0] = st2[0];
+            st[1] = st2[1];
+            train_norm(acc, r, st, g2, b2, L);
             train_to_lds(xs, LD, acc, L);
             __syncthreads();
-            train_unstage<D>(P.d3, D, ds, LD, L.row0, P.M);
-            train_unstage<D>(P.x2, D, xs, LD, L.row0, P.M);
-            // the feed-forward in two halves of its width
-            constexpr int HF = F / 2, NH = HF / 64;
 #pragma unroll 1
             for (int half = 0; half < 2; ++half) {
                 const int f0 = half * HF;
                 const TrainLane L(tile, P.M);
                 f32x4 u[NH][2], dh[NH][2];
-                train_product<NH, D / 32>(u, xs, LD, back_packed + train_matrix_at<D, F>(kTm1), f0 / 16, L);
+                ring.run<NH, D / 32>(u, xs, LD, w_1, f0 / 16, L);
+                ring.begin<NH, D / 32>(w_2_t, f0 / 16, L);
 #pragma unroll
                 for (int b = 0; b < NH; ++b) {
-                    const f32x4 bias = *reinterpret_cast<const f32x4 *>(P.bias1 + f0 + L.col(b));
+                    const f32x4 bias = bias1.at(f0 + L.col(b));
 #pragma unroll
                     for (int tb = 0; tb < 2; ++tb)
 #pragma unroll
@@ -637,8 +781,15 @@ __global__ __launch_bounds__(kTrainWaves * 64, D == 128 ? 3 : 2) void train_back
                             u[b][tb][e] = dv;
                         }
                 }
-                train_store16(P.h, F, f0, dh, L);
-                train_product<NH, D / 32>(dh, ds, LD, back_packed + train_matrix_at<D, F>(kTm2T), f0 / 16, L);
+                const TrainPacked<NH> h(dh);
+                ring.run<NH, D / 32>(dh, ds, LD, w_2_t, f0 / 16, L);
+                if (half == 0) ring.begin<NH, D / 32>(w_1, HF / 16, L);
+                else ring.begin<NB, F / 32>(w_1_t, 0, L);
+                h.template store<F>(P.h, f0, L);
+                if (half == 0) {
+                    train_unstage<D>(P.d3, ds, LD, L);
+                    train_unstage<D>(P.x2, xs, LD, L);
+                }
 #pragma unroll
                 for (int b = 0; b < NH; ++b) {
 #pragma unroll
@@ -648,19 +799,20 @@ __global__ __launch_bounds__(kTrainWaves * 64, D == 128 ? 3 : 2) void train_back
                 train_to_lds(us + f0, LF, u, L);
             }
             __syncthreads();
-            train_unstage<F>(P.du, F, us, LF, L.row0, P.M);
-            train_product<NB, F / 32>(acc, us, LF, back_packed + train_matrix_at<D, F>(kTm1T), 0, L);
+            ring.run<NB, F / 32>(acc, us, LF, w_1_t, 0, L);
+            ring.begin<NB, D / 32>(w_o_t, 0, L);
+            train_unstage<F>(P.du, us, LF, L);
 #pragma unroll
             for (int b = 0; b < NB; ++b)
 #pragma unroll
                 for (int tb = 0; tb < 2; ++tb) d[b][tb] += acc[b][tb];
-            train_norm_backward<D>(d, r, st, P.g2, sums + 3 * D, sums + 4 * D, red, L);
-            train_store<D>(P.dr2, d, L);
+            train_norm_backward<D>(d, r, st, g2, sums + 3 * D, sums + 4 * D, red, L);
             train_to_lds(ds, LD, d, L);  // (its readers are behind the barrier inside the norm)
             __syncthreads();
-            train_unstage<D>(P.d2, D, ds, LD, L.row0, P.M);
-            train_product<NB, D / 32>(acc, ds, LD, back_packed + train_matrix_at<D, F>(kTmOT), 0, L);
-            train_store16(P.dattn, D, 0, acc, L);
+            ring.run<NB, D / 32>(acc, ds, LD, w_o_t, 0, L);
+            train_store<D>(P.dr2, d, L);
+            train_unstage<D>(P.d2, ds, LD, L);
+            TrainPacked<NB>(acc).template store<D>(P.dattn, 0, L);
         }
         __syncthreads();
     }
