@@ -293,10 +293,13 @@ void flash_kernel(const char *early_k, const char *early_v, int early_sh, int ea
             const int i = wave + NW * r;
             if (i < NI) {
                 const unsigned m0v = lds_base + stage_ * STAGE_BYTES + i * 1024;
-                unsigned m0_saved;  // M0 (the LDS base of a direct load) is left as it was found
+                // M0 (the LDS base of a direct load) is left as it was found.  One wait state between writing it and the
+                // load that reads it: without, the load may take the old one and land elsewhere.
+                unsigned m0_saved;
                 asm volatile(
                     "s_mov_b32 %0, m0\n\t"
                     "s_mov_b32 m0, %1\n\t"
+                    "s_nop 0\n\t"
                     "global_load_lds_dwordx4 %2, %3\n\t"
                     "s_mov_b32 m0, %0"
                     : "=&s"(m0_saved)
@@ -1250,6 +1253,7 @@ void flash_kernel(const char *early_k, const char *early_v, int early_sh, int ea
                         asm volatile(
                             "s_mov_b32 %0, m0\n\t"
                             "s_mov_b32 m0, %1\n\t"
+                            "s_nop 0\n\t"
                             "global_load_lds_dwordx4 %2, %3\n\t"
                             "s_mov_b32 m0, %0"
                             : "=&s"(m0_saved)
