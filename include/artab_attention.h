@@ -678,7 +678,7 @@ int artab_trajectory_pack(void *tape, const void *w, int which, int layer, int r
                           int dtype, void *stream);
 int artab_trajectory_decode(const artab_trajectory_args *args, int dtype, void *stream);
 /*
- * The same with `parts` workgroups (2, 4 or 8, no more than heads; D up to 256; args->group is 1) to a trajectory: each
+ * The same with `parts` workgroups (2, 4 or 8, no more than heads; args->group is 1) to a trajectory: each
  * computes its share of the heads, what follows the attention all of them.  They wait for each other once per layer; a
  * wait that is in vain for some ten seconds turns the trajectory's further draws into NaN.  `exchange`:
  * artab_trajectory_exchange_bytes of device memory (16-byte aligned) of this call's own until it is done.
