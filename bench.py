@@ -761,7 +761,7 @@ def training_step(device):
     12 layers, d_model 128, 4 heads, d_ff 256, 20 mixture components; batch 64 of 64 context + 32
     buffer + 512 target rows; bf16 autocast, AdamW, gradient clipping at 1.0 as in train.py:289-310)
     with the row attention on the device kernels in both directions, and the same step with the row
-    attention as PyTorch's scaled_dot_product_attention under the dense boolean mask."""
+    attention as PyTorch's scaled_dot_product_attention in float32 under the dense boolean mask."""
     import torch.nn.functional as F
 
     import ar_nanotabpfn_amd.attention_kernels as ak
@@ -781,7 +781,10 @@ def training_step(device):
 
     def sdpa_row_attention(q, k, v, context_len, buffer_len, attending_chunks, use_triton=True):
         mask = RowMask(q.shape[2], context_len, buffer_len, attending_chunks).dense(q.device)
-        return F.scaled_dot_product_attention(q, k, v, attn_mask=mask)
+        # (in float32: torch's batched bfloat16 products with a transposed right operand, which its attention may make of
+        # the call in either direction, have faulted the device)
+        with torch.autocast("cuda", enabled=False):
+            return F.scaled_dot_product_attention(q.float(), k.float(), v.float(), attn_mask=mask).to(q.dtype)
 
     def one_step():
         opt.zero_grad(set_to_none=True)
@@ -812,7 +815,7 @@ def training_step(device):
     finally:
         ak.row_mask_attention = device_attention
     log(f"[training step] 12 layers, B={B}, rows {Nc}+{Nb}+{Nt}, bf16 autocast + AdamW: {ms_dev:.2f} ms per step with the "
-        f"device row attention, {ms_ref:.2f} ms with scaled_dot_product_attention under the dense mask")
+        f"device row attention, {ms_ref:.2f} ms with scaled_dot_product_attention in float32 under the dense mask")
     print(json.dumps({"training_step": dict(
         config="train_tabular_online.yaml", B=B, Nc=Nc, Nb=Nb, Nt=Nt, ms_per_step=round(ms_dev, 3),
         ms_per_step_sdpa_dense_mask=round(ms_ref, 3), loss_after=round(loss_dev, 4), loss_after_sdpa=round(loss_ref, 4))}))
