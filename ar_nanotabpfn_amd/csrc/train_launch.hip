@@ -1,9 +1,6 @@
 // The layer stack of a training step: buffers and launches of the kernels of train_layers.h around the row
 // attention (include/artab_attention.h, artab_train_*).
 #include "../../include/artab_attention.h"
-
-#include <algorithm>
-
 #include "launchers.h"
 #include "train_head.h"
 #include "train_layers.h"
@@ -90,21 +87,12 @@ int backward_groups(long M, int D) {
     const long resident = D == 128 ? 768 : 512, tiles = (M + kTrainRows - 1) / kTrainRows;
     return static_cast<int>(tiles < resident ? tiles : resident);
 }
-// Pieces of 128 x 128 of a layer's weight gradients: those of its front (q/k/v, feature attention) and of its back.
-int front_jobs(int D) { return 4 * D * D / (128 * 128); }
-int back_jobs(int D, int F) { return (D * D + 2 * D * F) / (128 * 128); }
-// Row slices of the weight-gradient products: as many as pieces times slices give every compute unit one workgroup (they
-// have one to a compute unit), none shorter than 256 rows.
+int grad_jobs(int D, int F) { return (5 * D * D + 2 * D * F) / (128 * 128); }
+// Row slices of the weight-gradient products: enough that pieces times slices give every compute unit a
+// workgroup, none shorter than 256 rows.
 int grad_slices(long M, int jobs) {
-    const long most = (M + 255) / 256, want = jobs < 256 ? 256 / jobs : 1;
+    const long most = (M + 255) / 256, want = (256 + jobs - 1) / jobs;
     return static_cast<int>(want < most ? want : most);
-}
-// Pieces times slices of the largest of a step's launches: of both, of either alone.
-size_t grad_pieces(long M, int D, int F) {
-    size_t most = 0;
-    for (const int jobs : {front_jobs(D) + back_jobs(D, F), front_jobs(D), back_jobs(D, F)})
-        most = std::max(most, static_cast<size_t>(grad_slices(M, jobs)) * jobs);
-    return most;
 }
 constexpr int kFinalGroups = 512;
 
@@ -115,13 +103,13 @@ struct Scratch {
 };
 Scratch scratch_layout(const artab_train_args &a) {
     const size_t M = static_cast<size_t>(a.B) * a.R, D = a.D, F = a.F;
-    const int groups = backward_groups(M, a.D);
+    const int groups = backward_groups(M, a.D), jobs = grad_jobs(a.D, a.F);
     Scratch v;
     Arena s(a.scratch);
     v.dx = s.take<float>(M * D);
     v.dr2 = s.take<float>(M * D);
     v.delta = s.take<float>(M * a.H);
-    v.part_w = s.take<float>(grad_pieces(M, a.D, a.F) * 16384);
+    v.part_w = s.take<float>(static_cast<size_t>(grad_slices(M, jobs)) * jobs * 16384);
     v.part_c = s.take<float>(groups * (7 * D + F));
     v.part_f = s.take<float>(kFinalGroups * 2 * D);
     v.d3 = s.take<bf16_t>(M * D);
@@ -219,9 +207,9 @@ int forward(const artab_train_args &a, hipStream_t st) {
 struct GradProducts {
     TrainGradJobs jobs{};
     TrainReduce reduce{};
-    GradProducts(long M, float *part) {
-        jobs.part = part; jobs.M = M;
-        reduce.part = part;
+    GradProducts(long M, int slices, float *part) {
+        jobs.part = part; jobs.M = M; jobs.rows_per_slice = ((M + slices - 1) / slices + 63) / 64 * 64;
+        reduce.part = part; reduce.slices = slices;
     }
     void add(const bf16_t *P, int ldp, const bf16_t *Q, int ldq, int N, int K, float *out) {
         for (int n = 0; n < N; n += 128)
@@ -232,13 +220,10 @@ struct GradProducts {
             }
     }
     void launch(hipStream_t st) {
-        const int slices = grad_slices(jobs.M, jobs.jobs);
-        jobs.slices = reduce.slices = slices;
-        jobs.rows_per_slice = ((jobs.M + slices - 1) / slices + kTrainGradRows - 1) / kTrainGradRows * kTrainGradRows;
         reduce.jobs = jobs.jobs;
         int columns = 0;
         for (int i = 0; i < reduce.n_cols; ++i) columns += reduce.cols[i].n;
-        hipLaunchKernelGGL(train_weight_grad_kernel, dim3(train_grad_blocks(jobs.jobs, jobs.slices)), dim3(1024), 0, st, jobs);
+        hipLaunchKernelGGL(train_weight_grad_kernel, dim3(jobs.jobs, reduce.slices), dim3(512), 0, st, jobs);
         hipLaunchKernelGGL(train_reduce_kernel, dim3(jobs.jobs * 16 + columns / kTrainReduceCols), dim3(256), 0, st, reduce);
     }
 };
@@ -249,7 +234,7 @@ int backward(const artab_train_args &a, hipStream_t st) {
     const Scratch X = scratch_layout(a);
     const GradLayout G(D, F);
     const long M = static_cast<long>(a.B) * a.R;
-    const int groups = backward_groups(M, a.D);
+    const int groups = backward_groups(M, a.D), jobs = grad_jobs(D, F), slices = grad_slices(M, jobs);
     const dim3 block(kTrainWaves * 64);
     {
         const float *const *p = a.params + static_cast<size_t>(a.n_layers - 1) * kParams;
@@ -265,7 +250,7 @@ int backward(const artab_train_args &a, hipStream_t st) {
     }
     for (int l = a.n_layers; l >= 0; --l) {  // launch l: the front of layer l, then the back of layer l - 1
         TrainBackward A{};
-        GradProducts products(M, X.part_w);
+        GradProducts products(M, slices, X.part_w);
         A.M = M; A.dr2 = X.dr2; A.part = X.part_c; A.dx = l > 0 ? X.dx : a.dx;
         if (l < a.n_layers) {
             const float *const *p = a.params + static_cast<size_t>(l) * kParams;
@@ -441,10 +426,10 @@ int head_backward(const artab_train_head_args &a, hipStream_t st) {
     constexpr int F = 256;
     TrainHead P = head_params(a);
     const HeadScratch X = head_scratch(a);
-    const int groups = head_groups(a.rows);
+    const int groups = head_groups(a.rows), jobs = head_jobs(a), slices = grad_slices(P.M, jobs);
     P.dloss = a.dloss; P.dz = a.dz; P.zb = X.zb; P.h = X.h; P.du = X.du; P.draw = X.draw; P.part = X.part;
     hipLaunchKernelGGL((train_head_kernel<D, F, NP, true>), dim3(groups), dim3(kTrainWaves * 64), 0, st, P);
-    GradProducts products(P.M, X.part_w);
+    GradProducts products(P.M, slices, X.part_w);
     products.add(X.du, F, X.zb, D, F, D, a.grads);
     products.add(X.draw, kHeadCols, X.h, F, kHeadCols, F, a.grads + static_cast<long>(F) * D);
     products.reduce.cols[products.reduce.n_cols++] = {X.part, a.grads + static_cast<long>(F) * (D + kHeadCols), groups, F + kHeadCols, F + kHeadCols};

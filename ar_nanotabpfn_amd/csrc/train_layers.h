@@ -915,35 +915,29 @@ __global__ __launch_bounds__(256) void train_final_kernel(TrainFinal P) {
 
 // ---- weight gradients: C[n][k] = sum_m P[m][n] Q[m][k] in pieces of 128 x 128, each over `slices` runs of
 // rows.  Both operands want the contraction (rows) consecutive in a lane: transposing reads of row-major LDS
-// tiles.  Sixteen wavefronts: four groups take a quarter of a tile's 128 rows each, a group's four hold 64 x 64.
+// tiles.  Eight wavefronts: two groups take half of a tile's 64 rows each, a group's four hold 64 x 64.
 //
-// Bound: the trip to memory.  A workgroup waits for one tile while it has multiplied the one before, one workgroup to
-// a compute unit (one launch fills the chip once, or its partial sums would be as many bytes as its operands), so the
-// bytes per unit and trip are what counts: tiles of 64 rows, eight wavefronts, took 40 us for the nine pieces of 38912
-// rows of 128 (140 MB), this 29.3.  Pieces of one slice read the same rows: they run on one XCD, whose L2 then has them.
+// Bound: the trip to memory; a workgroup waits for one tile while it has multiplied the one before.  38912 rows of 128, nine
+// pieces (140 MB): 40 us.  Two tiles on their way, or tiles of 128 rows on sixteen wavefronts, took 29, and both were in the
+// tree when a run of the device tests faulted; neither is to come back before the cause of that is known.
 struct TrainGradJobs {
     const bf16_t *p[kTrainMaxJobs], *q[kTrainMaxJobs];
     int ldp[kTrainMaxJobs], ldq[kTrainMaxJobs];
     float *part;               // [slices][jobs][128 * 128]
-    long M, rows_per_slice;    // a multiple of kTrainGradRows
-    int jobs, slices;
+    long M, rows_per_slice;    // a multiple of 64
+    int jobs;
 };
-constexpr int kTrainGradRows = 128;
-// Workgroups are dealt round-robin over the eight XCDs: pieces in a row, slice after slice, to each of them.
-__host__ __device__ constexpr int train_grad_blocks(int jobs, int slices) { return (jobs * slices + 7) / 8 * 8; }
 
-static __global__ __launch_bounds__(1024) void train_weight_grad_kernel(TrainGradJobs J) {
+static __global__ __launch_bounds__(512) void train_weight_grad_kernel(TrainGradJobs J) {
     typedef MfmaOps<bf16_t> Ops;
-    constexpr int TR = kTrainGradRows, LD = 128 + 16;  // 288 bytes: 32 mod 128, what the transposing reads want
+    constexpr int TR = 64, LD = 128 + 16;  // 288 bytes: 32 mod 128, what the transposing reads want
     __shared__ __attribute__((aligned(16))) bf16_t lds[2][2][TR * LD];
-    const int piece = static_cast<int>((blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3));
-    if (piece >= J.jobs * J.slices) return;
-    const int job = piece % J.jobs, slice = piece / J.jobs;
+    const int job = blockIdx.x, slice = blockIdx.y;
     const bf16_t *const p = J.p[job], *const q = J.q[job];
     const int ldp = J.ldp[job], ldq = J.ldq[job];
     const long m0 = slice * J.rows_per_slice, m1 = min(J.M, m0 + J.rows_per_slice);
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-    const int group = wave >> 2, wn = wave & 1, wk = (wave >> 1) & 1;
+    const int half = wave >> 2, wn = wave & 1, wk = (wave >> 1) & 1;
     f32x16 acc[2][2];
 #pragma unroll
     for (int a = 0; a < 2; ++a)
@@ -955,7 +949,7 @@ static __global__ __launch_bounds__(1024) void train_weight_grad_kernel(TrainGra
     auto fetch = [&](long m) {
 #pragma unroll
         for (int x = 0; x < 2; ++x) {
-            const int i = tid + 1024 * x, r = i / 16, c = i % 16;
+            const int i = tid + 512 * x, r = i / 16, c = i % 16;
             const long row = min(m + r, J.M - 1);
             rp[x] = *reinterpret_cast<const u32x4 *>(p + row * ldp + 8 * c);
             rq[x] = *reinterpret_cast<const u32x4 *>(q + row * ldq + 8 * c);
@@ -964,7 +958,7 @@ static __global__ __launch_bounds__(1024) void train_weight_grad_kernel(TrainGra
     auto put = [&](int buf, long m) {
 #pragma unroll
         for (int x = 0; x < 2; ++x) {
-            const int i = tid + 1024 * x, r = i / 16, c = i % 16;
+            const int i = tid + 512 * x, r = i / 16, c = i % 16;
             const u32x4 zero = {0u, 0u, 0u, 0u};
             *reinterpret_cast<u32x4 *>(&lds[buf][0][r * LD + 8 * c]) = m + r < m1 ? rp[x] : zero;  // rows past the end: no product
             *reinterpret_cast<u32x4 *>(&lds[buf][1][r * LD + 8 * c]) = rq[x];
@@ -992,8 +986,8 @@ static __global__ __launch_bounds__(1024) void train_weight_grad_kernel(TrainGra
                 bf16x8 a[2], c[2];
 #pragma unroll
                 for (int i = 0; i < 2; ++i) {
-                    a[i] = operand(lds[buf][0], 32 * group + 16 * ks, 64 * wn + 32 * i);
-                    c[i] = operand(lds[buf][1], 32 * group + 16 * ks, 64 * wk + 32 * i);
+                    a[i] = operand(lds[buf][0], 32 * half + 16 * ks, 64 * wn + 32 * i);
+                    c[i] = operand(lds[buf][1], 32 * half + 16 * ks, 64 * wk + 32 * i);
                 }
 #pragma unroll
                 for (int i = 0; i < 2; ++i)
@@ -1003,33 +997,28 @@ static __global__ __launch_bounds__(1024) void train_weight_grad_kernel(TrainGra
             if (more) put(buf ^ 1, m + TR);  // the other buffer's readers passed the barrier above
         }
     }
-    // the groups' sums through LDS, a 32 x 32 block of every wavefront at a time, added up by one group each; two areas in turn
-    float *const out = J.part + static_cast<long>(piece) * (128 * 128);
+    // the second group's sums through LDS (64 x 64 floats per wavefront pair would fill it: one quarter at a time)
+    float *const x = reinterpret_cast<float *>(lds);
+    float *const out = J.part + (static_cast<long>(slice) * J.jobs + job) * (128 * 128);
     const int c32 = lane & 31, hb = lane >> 5;
-    constexpr int AREA = 16 * 1024;  // floats: 16 of a lane, 16 wavefronts
-    static_assert(2 * AREA * sizeof(float) <= sizeof(lds), "two areas");
-    __syncthreads();
 #pragma unroll
-    for (int round = 0; round < 4; ++round) {
-        constexpr int kQuarter = AREA / 4;
-        const int i = round >> 1, j = round & 1;
-        float *const x = reinterpret_cast<float *>(lds) + (round & 1) * AREA;
-        if (group != round) {
+    for (int i = 0; i < 2; ++i)
 #pragma unroll
-            for (int v = 0; v < 16; ++v) x[group * kQuarter + (wave & 3) * 1024 + v * 64 + lane] = acc[i][j][v];
-        }
-        __syncthreads();
-        if (group == round) {
+        for (int j = 0; j < 2; ++j) {
+            __syncthreads();
+            if (half == 1) {
 #pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                const int n = 64 * wn + 32 * i + 8 * (v >> 2) + 4 * hb + (v & 3), k = 64 * wk + 32 * j + c32;
-                float sum = acc[i][j][v];
+                for (int v = 0; v < 16; ++v) x[(wave & 3) * 1024 + v * 64 + lane] = acc[i][j][v];
+            }
+            __syncthreads();
+            if (half == 0) {
 #pragma unroll
-                for (int other = 1; other < 4; ++other) sum += x[((round + other) & 3) * kQuarter + (wave & 3) * 1024 + v * 64 + lane];
-                out[n * 128 + k] = sum;
+                for (int v = 0; v < 16; ++v) {
+                    const int n = 64 * wn + 32 * i + 8 * (v >> 2) + 4 * hb + (v & 3), k = 64 * wk + 32 * j + c32;
+                    out[n * 128 + k] = acc[i][j][v] + x[(wave & 3) * 1024 + v * 64 + lane];
+                }
             }
         }
-    }
 }
 
 // Adds up the slices of the weight gradients (where each piece goes: `out`, row stride `ld`) and the workgroups'

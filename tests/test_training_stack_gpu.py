@@ -22,9 +22,10 @@ def only_modules(monkeypatch):
     (128, 4, 1, 1, 16, 1, 15, 1, 1), (128, 4, 2, 3, 17, 4, 12, 2, 6), (128, 2, 2, 5, 40, 8, 100, 3, 8),
     (256, 8, 2, 2, 33, 5, 61, 10, 32), (256, 4, 1, 7, 64, 16, 129, 2, 16),
     (128, 4, 1, 3, 300, 32, 64, 2, 32),
-    # a run of this file and the other training tests once left the GPU faulted, with a weight-gradient kernel that has been
-    # taken out again; which test it was is not known, and no access out of range has been found.  Of those tests these
-    # sizes (and the 515 tiles of the many-tiles test) have not run since with the attention's query tiles they take now.
+    # a run of this file and the other training tests once left the GPU faulted, and later a run of all device tests; both had
+    # a weight-gradient kernel with twice the bytes on their way, which has been taken out both times.  Which test it was is
+    # not known, and no access out of range has been found.  Of the first run's tests these sizes (and the 515 tiles of the
+    # many-tiles test) have not run since with the attention's query tiles they take now.
     pytest.param(128, 4, 1, 33, 300, 32, 512, 2, 32, marks=pytest.mark.skip(reason="part of a run that faulted, cause not shown"))])
 def test_fused_training_equals_modules(device, monkeypatch, D, H, L, B, Nc, Nb, Nt, feat, tokens):
     import ar_nanotabpfn_amd.model as model_mod
