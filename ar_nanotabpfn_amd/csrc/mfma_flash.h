@@ -30,8 +30,8 @@
 // classical online-softmax (running maximum, rescaled accumulators).  f16, whose
 // exponent range is too small for that, takes its probabilities against one reference per row, the largest
 // score of the first 64 keys, where the pass is the lean one (256 query rows, head_dim 32), and the
-// online softmax elsewhere; a row sum that has overflowed (a later score 2^20 times the reference) makes it redo
-// its range like the others.  One multiply-add per score for scale and reference, so that the queries stay as
+// online softmax elsewhere; a row sum that has overflowed (a later score 16 above the reference, base 2) makes it
+// redo its range like the others.  One multiply-add per score for scale and reference, so that the queries stay as
 // they are: error against float64 2.9e-4 where the online softmax has 3.5e-4 (64 x 8 pairs of 512 normal rows).
 // us, online softmax -> this: prefill of 64 x 8 x 512 rows 52.0 -> 41.1, 1 x 8 x 16384 533 -> 354; 1024 x 8 x 2 queries over
 // 16384 keys 90.0 -> 61.0; 64 x 4 pairs of 1544 rows, 1000 keys 144 -> 108.
@@ -180,7 +180,6 @@ __device__ __forceinline__ void flash_stamp_end(const FlashParams &P) {
 // Probability mass (sum of 2^s over a row) the fast path accepts.
 constexpr float kFastMassMax = 1.2676506e30f;  // 2^100
 constexpr float kFastMassMin = 7.8886091e-31f; // 2^-100
-constexpr float kLeanAbove = 4.f;              // f16: see lean_pass
 
 // Largest / smallest teacher-forcing key limit over query rows [a, b] (inclusive).
 __host__ __device__ inline int tf_range_max(int a, int b, int Nt) {
@@ -1194,8 +1193,9 @@ void flash_kernel(const char *early_k, const char *early_v, int early_sh, int ea
             }
         }
         if constexpr (!Ops::kWideExponent) {
-            // The reference: the column's largest score among the keys of the first tile, kLeanAbove (base 2) above it.  A probability
-            // overflows 16 bits if a later score is 20 (base 2) larger, and the row sum says so: the robust pass then.
+            // The reference: the column's largest score among the keys of the first tile.  Not above it: probabilities below
+            // 2^-14 are rounded to steps of 2^-24, and of a long tail of them behind one large score that much of the sum would be
+            // lost.  One overflows 16 bits if a later score is 16 (base 2) larger, and the row sum says so: the robust pass then.
             __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
             __syncthreads();
             const int seen = ctx_end - ctx_begin;
@@ -1213,7 +1213,7 @@ void flash_kernel(const char *early_k, const char *early_v, int early_sh, int ea
 #pragma unroll
                     for (int v = 0; v < 16; ++v) top = fmaxf(top, 32 * sb + 8 * (v >> 2) + 4 * hb + (v & 3) < seen ? s[v] : -INFINITY);
                 }
-                m_run[j] = fmaf(fmaxf(top, __shfl_xor(top, 32, 64)), f16_scale, kLeanAbove);
+                m_run[j] = fmaxf(top, __shfl_xor(top, 32, 64)) * f16_scale;
             }
         }
 

@@ -24,9 +24,9 @@ def _rel(a, b):
 
 
 # keys: one, short of, at and past the first tile of 64, several tiles; the step in the scores (natural) behind the first 64
-# keys: none, inside, at the edge of and beyond 20 powers of two, and far below
+# keys: none, inside, at the edge of and beyond 16 powers of two, and far below
 @pytest.mark.parametrize("Nc", [1, 63, 64, 65, 200, 1100])
-@pytest.mark.parametrize("step", [0.0, 12.0, 14.0, 40.0, -40.0])
+@pytest.mark.parametrize("step", [0.0, 9.0, 11.1, 12.0, 14.0, 40.0, -40.0])
 def test_context_with_a_step_in_its_scores(device, tuning, Nc, step):
     import ar_nanotabpfn_amd.attention_kernels as ak
 
@@ -43,6 +43,34 @@ def test_context_with_a_step_in_its_scores(device, tuning, Nc, step):
     want, want_lse = _reference(q, k, v)
     assert _rel(out, want) <= TOL
     assert float((lse.double() - want_lse).abs().max()) <= 2 * TOL * max(1.0, abs(step))
+
+
+# one key among the first 64 that is `up` (natural) above a long tail, all of one score or with a spread of them: 2^-11 to
+# 2^-20 of its probability each, which 16 bits hold in steps of 2^-24
+@pytest.mark.parametrize("up", [8.0, 10.0, 11.0, 12.0, 14.0])
+@pytest.mark.parametrize("spread", [0.0, 1.0])
+def test_one_early_key_above_a_long_tail(device, tuning, up, spread):
+    import ar_nanotabpfn_amd.attention_kernels as ak
+
+    tuning(ARTAB_SMALL=0, ARTAB_SPLIT=1)
+    B, H, Nc, Dh = 300, 1, 16384, 32
+    g = torch.Generator().manual_seed(int(up))
+    q = spread * torch.randn(B, H, 1, Dh, generator=g)
+    k, v = (torch.randn(H, Nc, Dh, generator=g) for _ in range(2))
+    q[..., 0] = 4.0
+    k[..., 0] = 0.0
+    k[:, 17, 0] = up * Dh ** 0.5 / 4.0
+    q, k, v = (t.to(device, torch.float16) for t in (q, k, v))
+    errors = []
+    want, want_lse = _reference(q, k, v)
+    for lean in (1, 0):  # 0: the online softmax
+        tuning(ARTAB_LEAN=lean)
+        out, lse = ak.context_attention(q, k, v)
+        errors.append((_rel(out, want), float((lse.double() - want_lse).abs().max())))
+    # the same probabilities in the same steps; beside them the output's rounding, 2^-11, a third of it on average, and the
+    # logarithm's in float32, 2^-24 of a sum in front of which up to `up` is subtracted
+    assert errors[0][0] <= 1.1 * errors[1][0] + 2.0 ** -11 / 3
+    assert errors[0][1] <= 1.1 * errors[1][1] + 4 * up * 2.0 ** -24
 
 
 def test_rows_of_no_use_for_a_reference(device, tuning):
