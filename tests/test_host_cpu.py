@@ -74,6 +74,15 @@ def test_tuning_overrides_are_explicit_and_restorable(monkeypatch):
     assert L.tuning.get("ARTAB_TILE_ROWS") is None and L.tuning.get("ARTAB_DENSE_BELOW") is None
 
 
+def test_every_override_of_the_library_is_a_key():
+    import re
+
+    L = _lib()
+    text = open(os.path.join(os.path.dirname(L.__file__), "csrc", "artab_api.hip")).read()
+    table = text[text.index("g_tune[kTuneCount]") : text.index("g_tune_loaded")]
+    assert sorted(re.findall(r'\{"(ARTAB_\w+)"', table)) == sorted(L.TUNING_KEYS)
+
+
 def test_workspace_query_is_host_only():
     lib = _lib().load()
     assert lib.artab_workspace_bytes(1024, 8, 2, 16384, 32, 0) > 0
