@@ -43,7 +43,7 @@ static TuneSlot g_tune[kTuneCount] = {
     {"ARTAB_CTX_YIELD", false, 0},    {"ARTAB_ORDER_GATE_LAUNCH", false, 0},
     {"ARTAB_BN", false, 0},          {"ARTAB_LEAN", false, 0},         {"ARTAB_LEAN_OCC", false, 0},
     {"ARTAB_NW", false, 0},          {"ARTAB_TILE_ROWS", false, 0},    {"ARTAB_LAYER_FETCHERS", false, 0},
-    {"ARTAB_TRAJECTORY", false, 0},  {"ARTAB_TRAJECTORY_PARTS", false, 0},
+    {"ARTAB_TRAJECTORY", false, 0},  {"ARTAB_TRAJECTORY_PARTS", false, 0}, {"ARTAB_TRAJECTORY_POLLS", false, 0},
 };
 static const bool g_tune_loaded = [] {
     for (TuneSlot &t : g_tune) {
@@ -1986,9 +1986,8 @@ int artab_trajectory_parts(int B, int Nc, int Nt, int H, int D, int F, int n_lay
     int dev = 0, cus = 0;
     if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
         cus = 256;
-    // Workgroups that wait for others are on the chip together because an XCD starts them in order: at most one trajectory of a
-    // launch is there in part, seven workgroups for the 32 compute units of an XCD.  A partition with fewer XCDs could hold several
-    // in part.
+    // Workgroups that wait for others have to be on the chip together (trajectory_crews.h); a partition with fewer XCDs could hold
+    // several trajectories in part, and would give them up.
     if (cus < 256) return 1;
     const bool f32 = dtype == ARTAB_F32;
     static constexpr double kBase[2][3][4] = {{{5.2, 6.0, 6.8, 0.}, {13.0, 9.8, 8.8, 9.0}, {37.0, 31.0, 24.5, 22.5}},
@@ -2105,7 +2104,8 @@ int artab_trajectory_decode_parts(const artab_trajectory_args *a, int parts, voi
     P.rand_u = a->rand_u; P.rand_n = a->rand_n; P.rand_n_f32 = a->rand_n_f32 || dtype == ARTAB_F32; P.x_mean = a->x_mean;
     P.w_x = a->w_x; P.b_x = a->b_x; P.w_y = a->w_y; P.b_y = a->b_y; P.markers = a->markers; P.ar_tokens = a->ar_tokens; P.bs = a->bs;
     P.preds = a->preds; P.B = a->B; P.Nt = a->Nt; P.G = a->group;
-    P.exchange = static_cast<unsigned long long *>(exchange);
+    P.most_polls = std::max(0, tune(kTuneTrajectoryPolls, kTrajMostPolls));
+    P.exchange = parts > 1 ? static_cast<unsigned long long *>(exchange) : nullptr;
     hipStream_t st = static_cast<hipStream_t>(stream);
     hipError_t e = dtype == ARTAB_BF16 ? launch_trajectory_decode_bf16(P, a->D, a->F, parts, st)
                    : dtype == ARTAB_F16 ? launch_trajectory_decode_f16(P, a->D, a->F, parts, st)

@@ -39,6 +39,7 @@ enum Tune : int {
     kTuneLayerFetchers,   // ARTAB_LAYER_FETCHERS: weight-fetching workgroups per XCD of a layer-boundary launch (0..32)
     kTuneTrajectory,      // ARTAB_TRAJECTORY: 0 keeps sampling runs off the whole-run kernel, 1..8 trajectories per workgroup
     kTuneTrajectoryParts, // ARTAB_TRAJECTORY_PARTS: workgroups per trajectory (1, 2, 4, 8; no more than there are heads)
+    kTuneTrajectoryPolls, // ARTAB_TRAJECTORY_POLLS: looks for another workgroup's word before the trajectory is given up (>= 0)
     kTuneCount
 };
 // The override of `key` if one is set, else `fallback` (artab_api.hip).

@@ -30,6 +30,14 @@
 // would take two more exchanges of about 0.9 us each and save 1.4.  64 trajectories of d_model 256 with 600 own rows, bf16, us per
 // layer and step: 21.7 with one workgroup, 15.7 with two; 32 on a shared context of 4000 rows 60.9 / 36.1 / 22.9 / 17.4 with 1 / 2 /
 // 4 / 8.  artab_trajectory_parts() says how many.
+//
+// Workgroups that wait for others want them on the chip.  An XCD starts those of a launch in order, so that at most one
+// trajectory of it is there in part: seven workgroups at most for the XCD's 32 compute units, and four such launches at once (the
+// queues a process has by default) have room.  More of them, a stream with a mask of few compute units, a device with fewer XCDs, or
+// kernels of others that stay for long can keep a partner away.  A wait ends after most_polls looks; the workgroup then marks its
+// own words, on which the others of the trajectory end too, and the launch behind this one computes the trajectory
+// again with one workgroup: caches, draws and variates are the trajectory's own, so nothing of the first attempt is left.
+// Where nothing was given up that launch only reads the words.
 #pragma once
 
 #include "trajectory_decode.h"
@@ -130,7 +138,10 @@ __global__ __launch_bounds__(2 * kTrajWaves * 64) void trajectory_crews_kernel(T
     const int member = PARTS > 1 ? static_cast<int>(blockIdx.x >> 3) % PARTS : 0;
     const long b = PARTS > 1 ? static_cast<long>(blockIdx.x >> 3) / PARTS * 8 + (blockIdx.x & 7) : blockIdx.x;
     if (PARTS > 1 && b >= P.B) return;
-    __shared__ int gone_s;  // another workgroup of the trajectory was waited for in vain
+    if constexpr (PARTS == 1)
+        if (P.exchange && !traj_given_up<T, D, NT>(P.exchange, b, tid)) return;
+    // looks that a wait for another workgroup may take; below zero once one was in vain, or another workgroup has given up
+    __shared__ int patience_s;
 
     // Global memory by its address space: made from integers, plain pointers would be generic ones, whose loads count
     // as LDS accesses too, and every wait for LDS would wait for them.
@@ -394,7 +405,7 @@ __global__ __launch_bounds__(2 * kTrajWaves * 64) void trajectory_crews_kernel(T
     static_assert(WORDS <= NTC, "one word per thread of a crew");
     auto words = [&](unsigned tag) { return P.exchange + (2 * b + (tag & 1)) * WORDS; };
     auto send = [&](int row, int col, const float (&o)[4], unsigned tag) {
-        if (gone_s) return;  // (what it would send is not the trajectory's: the others are to give up too)
+        if (patience_s < 0) return;  // (what it would send is not the trajectory's)
         unsigned long long *const at = words(tag) + (row * D + col) / VPW;
 #pragma unroll
         for (int i = 0; i < 4 / VPW; ++i) {
@@ -409,10 +420,10 @@ __global__ __launch_bounds__(2 * kTrajWaves * 64) void trajectory_crews_kernel(T
         if (i >= WORDS || col / (D / PARTS) == member) return;
         const unsigned long long *const at = words(tag) + i;
         unsigned long long v = __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        // (every wait ends: a workgroup that is not there after some seconds is given up, and the draws become NaN)
-        for (int polls = gone_s ? kTrajMostPolls : 0; static_cast<unsigned>(v >> 32) != tag; ++polls) {
-            if (polls >= kTrajMostPolls) {
-                gone_s = 1;
+        // (every wait ends: the step is then finished with what there is, nobody uses it)
+        for (int looks = patience_s; static_cast<unsigned>(v >> 32) != tag; --looks) {
+            if (looks <= 0 || static_cast<unsigned>(v >> 32) == kTrajGone) {
+                patience_s = -1;
                 break;
             }
             __builtin_amdgcn_s_sleep(1);
@@ -682,7 +693,7 @@ __global__ __launch_bounds__(2 * kTrajWaves * 64) void trajectory_crews_kernel(T
         eps_s[0] = P.eps1;
         eps_s[1] = P.eps2;
         eps_s[2] = P.eps3;
-        if constexpr (PARTS > 1) gone_s = 0;
+        if constexpr (PARTS > 1) patience_s = P.most_polls;
     }
     __syncthreads();
     C.template first_rows<NT>(P, b, 1, NR, xs, LD, tid);
@@ -919,8 +930,7 @@ __global__ __launch_bounds__(2 * kTrajWaves * 64) void trajectory_crews_kernel(T
                     }
                     const unsigned long long past = __ballot(lane < P.K && upto > my_u * cum);
                     const int comp = past ? __builtin_ctzll(past) : P.K - 1;
-                    T y = C.value(P, raw, comp, my_n);
-                    if (PARTS > 1 && gone_s) y = from_f32<T>(NAN);
+                    const T y = C.value(P, raw, comp, my_n);
                     if (lane == 0) {
                         if (member == 0) static_cast<T *>(P.preds)[b * P.Nt + t] = y;  // (all of them have drawn it)
                         y_s = to_f32(y);
@@ -928,13 +938,22 @@ __global__ __launch_bounds__(2 * kTrajWaves * 64) void trajectory_crews_kernel(T
                 }
             }
             __syncthreads();
-            if (last_step) break;
+            // (last written several barriers ago: all threads see the same)
+            if (last_step || (PARTS > 1 && __builtin_amdgcn_readfirstlane(patience_s) < 0)) break;
             C.template next_rows<NT>(x_s, &y_s, tok_s, 1, xs, LD, tid);
             __syncthreads();
         }
     };
     if (warp < NW) run(integral_constant<int, 0>{});
     else run(integral_constant<int, 1>{});
+    if constexpr (PARTS > 1) {
+        if (patience_s < 0) {  // given up: mark this workgroup's words of both sets
+            constexpr int MINE = D / PARTS / VPW;
+            for (int i = tid; i < 2 * NR * MINE; i += NT)
+                __hip_atomic_store(words(0) + i / MINE * (D / VPW) + member * MINE + i % MINE, static_cast<unsigned long long>(kTrajGone) << 32,
+                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
 }
 
 }  // namespace artab

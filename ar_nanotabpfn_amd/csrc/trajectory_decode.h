@@ -76,11 +76,16 @@ struct TrajectoryParams {
     const void *ar_tokens; int bs;      // [bs, D]
     void *preds;             // [B, Nt]
     int B, Nt, G;
-    // several workgroups to a trajectory (trajectory_crews.h): what they give each other, zero in front of the launch
+    // several workgroups to a trajectory (trajectory_crews.h): how often one of them looks for another's word, and what they
+    // give each other, zero in front of the launch.  One workgroup to a trajectory: null, or the words of such a launch in
+    // front of this one, which is then for the trajectories that it has given up.
+    int most_polls;
     unsigned long long *exchange;
 };
-// A wait for another workgroup's word: about a microsecond each, some ten seconds in all.
-constexpr int kTrajMostPolls = 1 << 24;
+// A look for another workgroup's word takes about a microsecond: some 60 ms in all.  The others are on the chip, or will be
+// when kernels of other streams make room; longer than that costs more than the run with one workgroup.
+constexpr int kTrajMostPolls = 1 << 16;
+constexpr unsigned kTrajGone = ~0u;  // in the place of an exchange's number: the workgroup has given its trajectory up
 // Whether the two-crew kernel is built for `parts` workgroups to a trajectory: each has one head or more, a wavefront of one
 // crew or more for each of them.
 constexpr bool traj_parts_built(int D, int parts) {
@@ -92,6 +97,17 @@ constexpr int traj_exchange_words(int D) { return 2 * D * static_cast<int>(sizeo
 static __global__ __launch_bounds__(256) void trajectory_exchange_kernel(unsigned long long *words, long n) {
     const long i = static_cast<long>(blockIdx.x) * 256 + threadIdx.x;
     if (i < n) words[i] = 0;  // (the number of no exchange)
+}
+// Whether trajectory b has been given up by a launch of several workgroups to a trajectory.  For all NT threads of a workgroup.
+template <typename T, int D, int NT>
+__device__ __forceinline__ bool traj_given_up(const unsigned long long *exchange, long b, int tid) {
+    __shared__ int found;
+    if (tid == 0) found = 0;
+    __syncthreads();
+    for (int i = tid; i < 2 * traj_exchange_words<T>(D); i += NT)
+        if (static_cast<unsigned>(exchange[b * 2 * traj_exchange_words<T>(D) + i] >> 32) == kTrajGone) found = 1;
+    __syncthreads();
+    return __builtin_amdgcn_readfirstlane(found) != 0;
 }
 
 // One 1 KiB fragment per operand and product.  Both types read the A operand as row lane % 16 of a
@@ -338,6 +354,8 @@ __global__ __launch_bounds__(kTrajWaves * 64) void trajectory_decode_kernel(Traj
     const int row16 = lane & 15, quad = lane >> 4;         // operand layout
     const long b0 = static_cast<long>(blockIdx.x) * P.G;
     const int valid = static_cast<int>(min(static_cast<long>(P.G), P.B - b0));
+    if constexpr (!SEVERAL)
+        if (P.exchange && !traj_given_up<T, D, NT>(P.exchange, b0, tid)) return;
 
     // ---- the weight tape
     u32x4 ring[S::kRing];

@@ -75,7 +75,7 @@ hipError_t tape_matrix(const void *w, char *tape, long stride, int N, int K, con
 
 // Several workgroups to a trajectory: the heads are dealt over them.
 template <typename T, int D, int F, int PARTS>
-hipError_t decode_parts(const TrajectoryParams &P, hipStream_t st) {
+hipError_t launch_parts(const TrajectoryParams &P, hipStream_t st) {
     if constexpr (traj_parts_built(D, PARTS)) {
         const long words = 2L * P.B * traj_exchange_words<T>(D);
         hipLaunchKernelGGL(trajectory_exchange_kernel, dim3(static_cast<unsigned>((words + 255) / 256)), dim3(256), 0, st, P.exchange, words);
@@ -87,15 +87,24 @@ hipError_t decode_parts(const TrajectoryParams &P, hipStream_t st) {
 }
 
 template <typename T>
-hipError_t decode(const TrajectoryParams &P, int D, int F, int parts, hipStream_t st) {
+hipError_t decode_parts(const TrajectoryParams &P, int D, int F, int parts, hipStream_t st) {
     hipError_t e = hipErrorInvalidValue;
     with_shape<T>(D, F, [&](auto d, auto f) {
-        if (parts > 1) {
-            constexpr int kD = decltype(d)::value, kF = decltype(f)::value;
-            e = parts == 2 ? decode_parts<T, kD, kF, 2>(P, st) : parts == 4 ? decode_parts<T, kD, kF, 4>(P, st)
-                : parts == 8 ? decode_parts<T, kD, kF, 8>(P, st) : hipErrorInvalidValue;
-            return;
-        }
+        constexpr int kD = decltype(d)::value, kF = decltype(f)::value;
+        e = parts == 2 ? launch_parts<T, kD, kF, 2>(P, st) : parts == 4 ? launch_parts<T, kD, kF, 4>(P, st)
+            : parts == 8 ? launch_parts<T, kD, kF, 8>(P, st) : hipErrorInvalidValue;
+    });
+    return e;
+}
+
+template <typename T>
+hipError_t decode(const TrajectoryParams &P, int D, int F, int parts, hipStream_t st) {
+    hipError_t e = hipErrorInvalidValue;
+    if (parts > 1) {  // and, behind it, one workgroup to each trajectory that has been given up
+        e = decode_parts<T>(P, D, F, parts, st);
+        if (e != hipSuccess) return e;
+    }
+    with_shape<T>(D, F, [&](auto d, auto f) {
         const dim3 grid(static_cast<unsigned>((P.B + P.G - 1) / P.G)), block(kTrajWaves * 64);
         if constexpr (decltype(d)::value <= 256) {
             if (crews_serve(P, D, sizeof(T) == 4)) {

@@ -86,8 +86,7 @@ const char *artab_last_error(void);
  * ARTAB_BM, ARTAB_SPLIT, ARTAB_SMALL, ARTAB_STREAM, ARTAB_STREAM_PER_CU, ARTAB_STREAM_PRIO,
  * ARTAB_STREAM_SHORT, ARTAB_STREAM_CALM, ARTAB_DENSE_BELOW, ARTAB_CTX_YIELD, ARTAB_ORDER_GATE_LAUNCH,
  * ARTAB_BN, ARTAB_LEAN, ARTAB_LEAN_OCC, ARTAB_NW, ARTAB_TILE_ROWS, ARTAB_LAYER_FETCHERS,
- * ARTAB_TRAJECTORY (what each
- * selects: csrc/launchers.h).
+ * ARTAB_TRAJECTORY, ARTAB_TRAJECTORY_PARTS, ARTAB_TRAJECTORY_POLLS (what each selects: csrc/launchers.h).
  *   artab_tuning_set: enable != 0 sets the override to `value`, enable == 0 removes it (the
  *                     library's own choice applies again).  Not thread-safe against running calls.
  *   artab_tuning_get: returns 1 if an override is set (its value in *value), 0 if not.
@@ -680,7 +679,8 @@ int artab_trajectory_decode(const artab_trajectory_args *args, int dtype, void *
 /*
  * The same with `parts` workgroups (2, 4 or 8, no more than heads; args->group is 1) to a trajectory: each
  * computes its share of the heads, what follows the attention all of them.  They wait for each other once per layer; a
- * wait that is in vain for some ten seconds turns the trajectory's further draws into NaN.  `exchange`:
+ * trajectory in which such a wait is in vain for some 60 ms (ARTAB_TRAJECTORY_POLLS), because other work or a mask of compute units keeps
+ * a workgroup off the chip, is computed again by one workgroup, by a launch behind the first.  `exchange`:
  * artab_trajectory_exchange_bytes of device memory (16-byte aligned) of this call's own until it is done.
  * artab_trajectory_parts says how many are fastest: 1 where artab_trajectory_group_layers decides.
  */

@@ -62,6 +62,56 @@ def test_parts_equal_one_workgroup_and_step_by_step(device, tuning, dtype, backe
             assert _rel(a, b) <= TOL[dtype]
 
 
+def _run(device, dtype, D, parts, B, Nc, Nt):
+    """A call of the whole-run kernel on a model of its own with given variates, and its caches' tensors."""
+    from ar_nanotabpfn_amd.glue import TrajectoryDecoder
+    from ar_nanotabpfn_amd.inference import ARTabPFNPredictor
+    from ar_nanotabpfn_amd.model import ARTabPFN
+
+    torch.manual_seed(D + B)
+    model = ARTabPFN(d_model=D, n_heads=D // 32, n_layers=2, d_ff=256, num_features=2, buffer_size=6, num_components=3).eval().to(device, dtype)
+    pred = ARTabPFNPredictor.from_trained_model(model, backend="triton_shared_context")
+    pred.init_kv_cache(B, Nt, torch.device(device), dtype)
+    pred.prefill_context(torch.randn(1, Nc, 2, device=device, dtype=dtype).expand(B, -1, -1), torch.randn(1, Nc, device=device, dtype=dtype).expand(B, -1))
+    run = TrajectoryDecoder(pred.embedder, pred.backbone, pred.head, pred.ar_tokens)
+    caches = [(l.k_ctx_cache, l.v_ctx_cache, l.k_buf_cache, l.v_buf_cache) for l in pred.backbone.layers]
+    x = torch.randn(B, Nt, device=device, dtype=dtype)
+    u, n = torch.rand(Nt, B, device=device), torch.randn(Nt, B, device=device)
+    return lambda k=parts: run(caches, Nc, 0, x, u, n, 1, k), [t for c in caches for t in c[2:]]
+
+
+# (d_model 512: one workgroup to a trajectory is another kernel)
+@pytest.mark.parametrize("dtype,D,parts,B,Nc,Nt", [(torch.bfloat16, 128, 4, 11, 70, 5), (torch.float16, 256, 2, 3, 33, 1), (torch.float32, 256, 8, 2, 129, 4),
+                                                   (torch.bfloat16, 512, 8, 9, 40, 3)])
+def test_trajectories_that_are_given_up(device, tuning, dtype, D, parts, B, Nc, Nt):
+    """No second look for another workgroup's word: every trajectory is given up, and is what one workgroup makes of it."""
+    call, own = _run(device, dtype, D, parts, B, Nc, Nt)
+    want = call(1)
+    rows = [t[:, :, : Nt - 1].clone() for t in own]
+    for t in own:
+        t.zero_()
+    tuning(ARTAB_TRAJECTORY_POLLS=0)
+    assert torch.equal(call(), want)
+    assert all(torch.equal(t[:, :, : Nt - 1], r) for t, r in zip(own, rows))
+    tuning(ARTAB_TRAJECTORY_POLLS=None)
+    assert torch.isfinite(call()).all() and torch.equal(call(), call())
+
+
+def test_runs_with_parts_on_two_streams(device):
+    calls = [_run(device, torch.bfloat16, 256, parts, B, 300, 12)[0] for parts, B in ((8, 13), (4, 40))]
+    want = [call() for call in calls]
+    streams = [torch.cuda.Stream(device) for _ in calls]
+    torch.cuda.synchronize()
+    got = [[], []]
+    for _ in range(4):
+        for call, stream, out in zip(calls, streams, got):
+            with torch.cuda.stream(stream):
+                out.append(call())
+    torch.cuda.synchronize()
+    for outs, w in zip(got, want):
+        assert all(torch.equal(o, w) for o in outs)
+
+
 def test_runs_with_parts_in_a_recorded_graph(device, tuning):
     """Replays, with other work and a synchronisation between them: the words are cleared by a launch that is recorded too."""
     from ar_nanotabpfn_amd.glue import TrajectoryDecoder
