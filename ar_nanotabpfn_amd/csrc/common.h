@@ -245,14 +245,6 @@ __device__ __forceinline__ float dot2_acc<f16_t>(unsigned a, unsigned b, float a
     return __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, a), __builtin_bit_cast(f16x2, b), acc, false);
 }
 
-// (The compiler does not space inline assembly from the matrix products whose results it reads: five wait states behind
-// a 4x4x4 product.  Where this is used four instructions lie between; the fifth is its own.)
-__device__ __forceinline__ float max3(float a, float b, float c) {
-    float r;
-    asm("s_nop 0\n\tv_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-    return r;
-}
-
 // Visible-key limit of teacher-forcing query row i among Nt buffer keys: buffer
 // query i (< Nt) sees keys [0, i]; target query i (>= Nt) sees keys [0, i - Nt).
 __host__ __device__ __forceinline__ int tf_limit(int i, int Nt) { return i < Nt ? i + 1 : i - Nt; }

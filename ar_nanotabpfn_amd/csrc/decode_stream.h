@@ -295,7 +295,8 @@ __device__ __forceinline__ void decode_stream_body(const DecodeParams &P, unsign
     // A lane group that has seen no valid key yet (KEYS = 16, short buffers) keeps m = -inf and
     // mq = 0: its probabilities are exp2(-inf) = 0.
     auto softmax = [&](const float (&sc)[4]) {
-        const float m_new = max3(max3(m, sc[0], sc[1]), sc[2], sc[3]);
+        // (two v_max3; as inline assembly the compiler would not space them from the products in front)
+        const float m_new = fmaxf(fmaxf(fmaxf(fmaxf(m, sc[0]), sc[1]), sc[2]), sc[3]);
         if (__builtin_amdgcn_ballot_w64(m_new > m) != 0) {
             const float alpha = m == -INFINITY ? 0.f : fast_exp2((m - m_new) * qscale);
             l *= alpha;
