@@ -818,7 +818,7 @@ def training_step(device):
         f"device row attention, {ms_ref:.2f} ms with scaled_dot_product_attention in float32 under the dense mask")
     print(json.dumps({"training_step": dict(
         config="train_tabular_online.yaml", B=B, Nc=Nc, Nb=Nb, Nt=Nt, ms_per_step=round(ms_dev, 3),
-        ms_per_step_sdpa_dense_mask=round(ms_ref, 3), loss_after=round(loss_dev, 4), loss_after_sdpa=round(loss_ref, 4))}))
+        ms_per_step_sdpa_f32_dense_mask=round(ms_ref, 3), loss_after=round(loss_dev, 4), loss_after_sdpa=round(loss_ref, 4))}))
 
 
 def main():
