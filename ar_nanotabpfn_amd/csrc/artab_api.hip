@@ -148,14 +148,17 @@ struct FlashPlan {
 // Query rows per workgroup where the keys are not split (prefill, teacher forcing, the training row mask): 256 (head_dim
 // 32: eight wavefronts), 128 or 64.
 // Head_dim 32: a tile of 256 rows takes less per row and key and longer to start, and rounding the rows up to whole
-// tiles costs what it adds: weighed as p(256) (N + 35) against p(128) N of N keys and p rows, times 1.2 up to 500 keys and
-// 1.35 from 1500 on; f16, whose smaller tiles keep a running maximum, 1.3 and 2.3.  The longer the keys, the fewer workgroups it
-// takes for that to be worth idle units: 256, down to 64 (f16 128, down to any number).
+// tiles costs what it adds: weighed as p(256) (N + 50) against p(128) N of N keys and p rows, times 1.1 up to 500 keys and
+// 1.25 from 1500 on; f16, whose smaller tiles keep a running maximum, N + 35, 1.3 and 2.3.  The longer the keys, the fewer
+// workgroups it takes for that to be worth idle units: 256, down to 64 (f16 128, down to any number).
 // Head_dim 64: 64 rows where 128 would leave the chip half empty or round the rows up.
-// Over 130 drawn calls of 16 to 2048 keys, 16 to 2100 rows, 8 to 2000 pairs, teacher forcing and the row mask, it is above the
-// best of the three by 1.1 % on average in both types, by at most 29 and 34 (a call of 8 x 121 pairs, 16 rows).  us: 64 x 4 pairs, 608
-// rows, 96 keys 22.4 -> 17.1; 616 rows, 316 keys 34 -> 25; 1544 rows, 1000 keys 141 (128 rows, f16) -> 108; 64 x 8, 516 rows,
-// 116 keys of head_dim 64 72 -> 50; 32 x 8, 80 rows, 1040 keys 22 -> 17.
+// Over 2000 calls of 16 to 2048 keys, 16 to 2200 rows, 8 to 1024 pairs, the last fifth of them drawn when the rule stood, it is
+// above the best of the three by 0.6 % on average in bf16 (head_dim 64 0.2, f16 0.2), by at most 22 (a call of 8 us; 11 and 11);
+// by rows alone (256 while there are 512 workgroups) 6.5 % (7.4 and 10.0), up to 58, better by 12 % at one call and by at most 7
+// elsewhere.  That was with 96 registers in tiles of 256 rows, which take 128 for teacher forcing and the row mask now.  f16 at
+// head_dim 32, on its present kernels: 130 drawn calls, 1.1 % above the best on average, at most 34 (8 x 121 pairs, 16 rows).
+// us: 64 x 4 pairs, 608 rows, 96 keys 22.4 -> 17.1; 616 rows, 316 keys 34 -> 25; 1544 rows, 1000 keys 96 (128 rows: 101; f16
+// 141 -> 108); 64 x 8, 516 rows, 116 keys of head_dim 64 72 -> 50; 32 x 8, 80 rows, 1040 keys 22 -> 17.
 static int unsliced_tile(long G, long pairs, int Nc, int Dh, bool bf16) {
     const auto padded = [&](int bm) { return static_cast<double>((G + bm - 1) / bm * bm); };
     const auto wgs = [&](int bm) { return (G + bm - 1) / bm * pairs; };
@@ -163,8 +166,8 @@ static int unsliced_tile(long G, long pairs, int Nc, int Dh, bool bf16) {
         return (G <= 64 && (bf16 || Nc <= 300 || pairs >= 512)) || (wgs(64) <= 256 && Nc <= (bf16 ? 500 : 256)) ||
                        (wgs(64) <= 512 && Nc <= (bf16 ? 600 : 128) && padded(64) < padded(128)) ? 64 : 128;
     const double far = Nc <= 500 ? 0. : Nc >= 1500 ? 1. : (Nc - 500) * 1e-3;
-    if (wgs(256) >= (bf16 ? 256 - 192 * far : 128 - 128 * far) &&
-        padded(256) * (Nc + 35) < padded(128) * (bf16 ? 1.2 + 0.15 * far : 1.3 + far) * Nc)
+    if (bf16 ? wgs(256) >= 256 - 192 * far && padded(256) * (Nc + 50) < padded(128) * (1.1 + 0.15 * far) * Nc
+             : wgs(256) >= 128 - 128 * far && padded(256) * (Nc + 35) < padded(128) * (1.3 + far) * Nc)
         return 256;
     return (G <= 64 && Nc <= 300) || (wgs(64) <= 256 && Nc <= 256) ? 64 : 128;
 }
