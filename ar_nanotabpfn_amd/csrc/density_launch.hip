@@ -16,7 +16,7 @@ template <typename T>
 int embed(const artab_embed_rows_args &a, hipStream_t st) {
     EmbedRowsParams P{};
     P.x = a.x; P.y = a.y; P.xb = a.x_stride_b; P.xn = a.x_stride_n; P.xc = a.x_stride_c; P.yb = a.y_stride_b; P.yn = a.y_stride_n;
-    P.B = a.B; P.N = a.N; P.C = a.C; P.D = a.D; P.pairs = a.pairs;
+    P.B = a.B; P.N = a.N; P.C = a.C; P.D = a.D; P.one_over_c = 1. / a.C; P.pairs = a.pairs;
     P.w_x = a.w_x; P.b_x = a.b_x; P.w_y = a.w_y; P.b_y = a.b_y; P.markers = a.markers; P.tokens = a.ar_tokens; P.bs = a.bs; P.out = a.out;
     const long threads = static_cast<long>(a.B) * a.N * (a.pairs ? 2 : 1) * (a.D * static_cast<long>(sizeof(T)) / 16);
     hipLaunchKernelGGL((embed_rows_kernel<T>), dim3(static_cast<unsigned>((threads + 255) / 256)), dim3(256), 0, st, P);

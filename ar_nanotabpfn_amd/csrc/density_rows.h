@@ -19,6 +19,7 @@ struct EmbedRowsParams {
     const void *x, *y;        // features [B, N, C], values [B, N], any strides (elements)
     long xb, xn, xc, yb, yn;
     int B, N, C, D;
+    double one_over_c;
     int pairs;                // 0: context rows [B, N, D]; 1: buffer rows, then target rows [B, 2 N, D]
     const void *w_x, *b_x, *w_y, *b_y;  // [D]
     const void *markers;      // [3, D]: target, context, buffer
@@ -40,10 +41,12 @@ __global__ __launch_bounds__(256) void embed_rows_kernel(EmbedRowsParams P) {
     const bool target = P.pairs && n >= P.N;
     if (target) n -= P.N;
     const T *const x = static_cast<const T *>(P.x) + b * P.xb + n * P.xn;
-    // Eight sums, added in pairs: one after the other 64 features of mean 3 and deviation 1 gave rows 1.1e-7 off in float32,
-    // where the library's reduction gives 5.8e-8 and this 6.1e-8; and eight loads are on their way at a time.
+    // Eight sums, so that eight loads are on their way at a time; of float32 features in 64 bits.  In 32 bits the rows were further off
+    // than the library's reduction leaves them (21 features of mean 3 and deviation 1: 5.9e-8 against 5.1e-8 to 5.9e-8, by its
+    // order; 4.6e-8 now, modelled on the CPU).
+    typedef std::conditional_t<sizeof(T) == 4, double, float> Sum;
     constexpr int SUMS = 8;
-    float part[SUMS] = {};
+    Sum part[SUMS] = {};
     for (int c0 = 0; c0 < P.C; c0 += SUMS) {
         float t[SUMS];
 #pragma unroll
@@ -51,31 +54,43 @@ __global__ __launch_bounds__(256) void embed_rows_kernel(EmbedRowsParams P) {
 #pragma unroll
         for (int u = 0; u < SUMS; ++u) part[u] += c0 + u < P.C ? t[u] : 0.f;
     }
-    const float mean = (((part[0] + part[1]) + (part[2] + part[3])) + ((part[4] + part[5]) + (part[6] + part[7]))) / P.C;
-    float v[PER];
-    auto vector = [&](const void *p, long at, auto use) {
+    const Sum sum = ((part[0] + part[1]) + (part[2] + part[3])) + ((part[4] + part[5]) + (part[6] + part[7]));
+    float mean;
+    if constexpr (sizeof(T) == 4) mean = static_cast<float>(sum * P.one_over_c);
+    else mean = sum / P.C;
+    auto vector = [&](float (&to)[PER], const void *p, long at, auto use) {
         const u32x4 raw = *reinterpret_cast<const u32x4 *>(static_cast<const T *>(p) + at + d);
 #pragma unroll
         for (int e = 0; e < PER; ++e) {
             if constexpr (sizeof(T) == 2) {
                 const unsigned word = raw[e / 2];
-                use(v[e], e & 1 ? unpack_hi<T>(word) : unpack_lo<T>(word));
+                use(to[e], e & 1 ? unpack_hi<T>(word) : unpack_lo<T>(word));
             } else {
                 const unsigned word = raw[e];
-                use(v[e], __builtin_bit_cast(float, word));
+                use(to[e], __builtin_bit_cast(float, word));
             }
         }
     };
+    const auto take = [](float &a, float t) { a = t; };
     const auto add = [](float &a, float t) { a += t; };
-    vector(P.w_x, 0, [&](float &a, float t) { a = mean * t; });
-    vector(P.b_x, 0, add);
+    const auto line = [&](float (&to)[PER], float at, const void *slope, const void *start) {
+        float w[PER];
+        vector(w, slope, 0, take);
+        vector(to, start, 0, take);
+#pragma unroll
+        for (int e = 0; e < PER; ++e) to[e] = fmaf(at, w[e], to[e]);
+    };
+    // in the modules' order: (mean w_x + b_x) + (y w_y + b_y) + marker + token
+    float v[PER];
+    line(v, mean, P.w_x, P.b_x);
     if (!target) {
-        const float y = to_f32(static_cast<const T *>(P.y)[b * P.yb + n * P.yn]);
-        vector(P.w_y, 0, [&](float &a, float t) { a = fmaf(y, t, a); });
-        vector(P.b_y, 0, add);
+        float u[PER];
+        line(u, to_f32(static_cast<const T *>(P.y)[b * P.yb + n * P.yn]), P.w_y, P.b_y);
+#pragma unroll
+        for (int e = 0; e < PER; ++e) v[e] += u[e];
     }
-    vector(P.markers, (target ? 0 : P.pairs ? 2 : 1) * static_cast<long>(P.D), add);
-    if (P.pairs && !target) vector(P.tokens, static_cast<long>(n % P.bs) * P.D, add);
+    vector(v, P.markers, (target ? 0 : P.pairs ? 2 : 1) * static_cast<long>(P.D), add);
+    if (P.pairs && !target) vector(v, P.tokens, static_cast<long>(n % P.bs) * P.D, add);
     u32x4 o;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {

@@ -64,8 +64,9 @@ def test_embedded_rows_of_many_features(device, C):
     g = torch.Generator().manual_seed(C)
     x, y = (torch.randn(2, 200, C, generator=g) + 3).to(device), torch.randn(2, 200, generator=g).to(device)
     want = copy.deepcopy(e).double().embed_context(x.double(), y.double())
-    # both are a few roundings of 2^-24, of random sign, in each of the same steps
-    assert _rel(embed_context_rows(e, x, y), want) <= 1.25 * _rel(e.embed_context(x, y), want)
+    # the mean is rounded once and each later step as in the modules, or not at all: their error at most, of 51200 values with some five
+    # roundings of random sign (a share of 1/sqrt(5 x 51200) of it by chance, five times that allowed)
+    assert _rel(embed_context_rows(e, x, y), want) <= 1.01 * _rel(e.embed_context(x, y), want)
     wide = torch.cat([x] * 10, dim=-1)
     assert embed_context_rows(e, wide[..., :64], y) is not None and embed_context_rows(e, wide[..., :65], y) is None
 
