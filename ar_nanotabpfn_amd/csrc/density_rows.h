@@ -7,7 +7,7 @@
 // these.  Bound: writing the rows; the launch and the chain norm, product, activation, product, mixture.
 //
 // Everything is float32 between the inputs and the results, but for the operands of the two products, which are of the
-// model's type.
+// model's type, and the sum of a row's float32 features (64 bits).
 #pragma once
 
 #include "common.h"

@@ -692,7 +692,7 @@ int artab_trajectory_decode_parts(const artab_trajectory_args *args, int parts, 
  * Embedded rows in one launch (model.py:23-76): mean of the features * w_x + b_x + marker, context and buffer rows with
  * y * w_y + b_y, buffer row n with position token n % bs.  pairs 0: context rows [B, N, D]; pairs 1: the rows of a
  * teacher-forced pass [B, 2 N, D], buffer rows and then target rows (inference.py:420-437).  Strides in elements; float32 up to the
- * result.  D a multiple of 8; the parameters and `out` 16-byte aligned.
+ * result (the sum of float32 features 64 bits).  D a multiple of 8; the parameters and `out` 16-byte aligned.
  */
 typedef struct artab_embed_rows_args {
     const void *x, *y;       /* [B, N, C], [B, N] */
